@@ -1,8 +1,8 @@
 // out[M, N] = a[M, K] . w[N, K]^T  (both operands row-major with K contiguous, the layout of
 // an activation and of a projection's weight), accumulated in 32-bit.
 //
-// Float engine: a plain tiled FMA kernel; every output element is one sequential sum over k,
-// so a row's result does not depend on the other rows of the batch.
+// Float engine: 32-bit matrix instructions, the weight streamed for few rows and tiled for many; the order of an
+// element's sum is the same everywhere, so a row's result does not depend on the other rows of the batch.
 // Bfloat16 engine, three families, each with a fixed k order for every output element (so a row's result
 // does not depend on the rows beside it): up to 64 rows the weight is streamed once straight into
 // v_mfma_f32_16x16x32_bf16 (`gemm_skinny_kernel`, optionally with the residual add and RMSNorm in front
@@ -13,58 +13,256 @@
 
 #if !MLR_BF16
 // ------------------------------------------------------------------------------ float
-#define BM 64
-#define BN 64
-#define BK 16
+// v_mfma_f32_16x16x4_f32 (32-bit products and sums), 16 k at a time: a lane holds four consecutive k of one row of
+// each operand (one 16-byte load), and the four products of a group take the k {e, 4 + e, 8 + e, 12 + e}.  The order of
+// an element's sum follows from K alone, whatever kernel and tile serve it, so that a token's result is the same to the
+// bit however a step was cut: k is cut into at most eight PARTS of `part_of(K)`, a part is summed in groups of 16 from
+// its start, and the parts are added as (p0 + p1 + ..) + (ph + ..), the second half from part (parts + 1) / 2 on.
+// Shorter chains than one sum over all of k: the error against 64 bits of a 3072-wide product is a third of that.
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 
-__global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ a,
-                                                       const float* __restrict__ w,
-                                                       float* __restrict__ out, int M, int N, int K) {
-    __shared__ float as[BK][BM + 4];
-    __shared__ float ws[BK][BN + 4];
-    const int t = threadIdx.x;
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-    const int tx = t % 16, ty = t / 16;
-    const int lrow = t / 4, lk = (t % 4) * 4;       // this thread stages row lrow, k lk..lk+3
-    float acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+static int part_of(int K) { return K <= 512 ? 64 : ((K + 7) / 8 + 15) / 16 * 16; }
 
-    for (int k0 = 0; k0 < K; k0 += BK) {
+// Four consecutive k of a row from k on, zeros from `end` on (VEC: rows start on 16 bytes and K is a multiple of four).
+template <bool VEC>
+__device__ __forceinline__ floatx4 load_k4(const float* __restrict__ row, int k, int end) {
+    floatx4 v = {0.f, 0.f, 0.f, 0.f};
+    if (VEC) {
+        if (k < end) v = *reinterpret_cast<const floatx4*>(row + k);
+    } else {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int k = k0 + lk + e;
-            const int am = m0 + lrow, wn = n0 + lrow;
-            as[lk + e][lrow] = (am < M && k < K) ? a[(size_t)am * K + k] : 0.f;
-            ws[lk + e][lrow] = (wn < N && k < K) ? w[(size_t)wn * K + k] : 0.f;
+        for (int e = 0; e < 4; ++e)
+            if (k + e < end) v[e] = row[k + e];
+    }
+    return v;
+}
+
+// Up to 32 rows: bound by the weight, which is streamed once from memory straight into the matrix cores.  A workgroup
+// owns NT strips of 16 output columns, its eight wavefronts a part of k each, so that all loads of a short part are under
+// way at once; the parts meet in LDS.
+template <int TM, int NT, bool VEC>
+__global__ __launch_bounds__(512) void gemm_f32_rows_kernel(const float* __restrict__ a, const float* __restrict__ w,
+                                                            float* __restrict__ out, int M, int N, int K, int part) {
+    constexpr int U = TM * NT <= 2 ? 8 : 4;              // groups of 16 k asked for at once
+    constexpr int W = NT * 16 + 1;
+    __shared__ float red[8][TM * 16][W];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = (lane >> 4) * 4;
+    const int n0 = blockIdx.x * (NT * 16);
+    const float* ar[TM];
+    const float* wr[NT];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) ar[i] = a + (size_t)min(i * 16 + r, M - 1) * K;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) wr[j] = w + (size_t)min(n0 + j * 16 + r, N - 1) * K;
+    floatx4 acc[TM][NT];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    int k = wave * part;
+    const int end = min(K, k + part);
+    // (whole groups without checks: loads behind a condition would wait for each other)
+    for (; VEC && k + 16 * U <= end; k += 16 * U) {
+        floatx4 wv[NT][U], av[TM][U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+            for (int j = 0; j < NT; ++j) wv[j][u] = *reinterpret_cast<const floatx4*>(wr[j] + k + u * 16 + q);
+#pragma unroll
+            for (int i = 0; i < TM; ++i) av[i][u] = *reinterpret_cast<const floatx4*>(ar[i] + k + u * 16 + q);
         }
-        __syncthreads();
 #pragma unroll
-        for (int k = 0; k < BK; ++k) {
-            float av[4], wv[4];
+        for (int u = 0; u < U; ++u)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) av[i] = as[k][ty * 4 + i];
+            for (int e = 0; e < 4; ++e)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) wv[j] = ws[k][tx * 4 + j];
+                for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+                    for (int j = 0; j < NT; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i][u][e], wv[j][u][e], acc[i][j], 0, 0, 0);
+    }
+    for (; k < end; k += 16) {
+        floatx4 wv[NT], av[TM];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(av[i], wv[j], acc[i][j]);
-        }
-        __syncthreads();
+        for (int j = 0; j < NT; ++j) wv[j] = load_k4<VEC>(wr[j], k + q, end);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) av[i] = load_k4<VEC>(ar[i], k + q, end);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i][e], wv[j][e], acc[i][j], 0, 0, 0);
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int m = m0 + ty * 4 + i;
-        if (m >= M) continue;
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int n = n0 + tx * 4 + j;
-            if (n < N) out[(size_t)m * N + n] = acc[i][j];
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) red[wave][i * 16 + q + e][j * 16 + r] = acc[i][j][e];
+    __syncthreads();
+    const int parts = (K + part - 1) / part, half = (parts + 1) / 2;
+    for (int i = threadIdx.x; i < TM * 16 * NT * 16; i += 512) {
+        const int row = i / (NT * 16), col = i % (NT * 16);
+        if (row >= M || n0 + col >= N) continue;
+        float first = red[0][row][col];
+        for (int p = 1; p < half; ++p) first += red[p][row][col];
+        if (half < parts) {
+            float second = red[half][row][col];
+            for (int p = half + 1; p < parts; ++p) second += red[p][row][col];
+            first += second;
+        }
+        out[(size_t)row * N + n0 + col] = first;
+    }
+}
+
+// More rows: bound by the matrix cores.  Two sets of WM x WN wavefronts, each with its half of the parts of k and its own
+// LDS blocks of G groups of 16 k (rows of a group 80 bytes apart: 16 lanes' 16-byte reads meet every bank once), the next
+// block's loads under way while one is multiplied -- so small tiles, whose products take no time, take long blocks.  The
+// second set's sums reach the first through LDS at the end.
+template <int WM, int WN, int TM, int TN, int G, bool VEC>
+__global__ __launch_bounds__(WM * WN * 128) void gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ w,
+                                                                      float* __restrict__ out, int M, int N, int K, int part) {
+    constexpr int BM = WM * TM * 16, BN = WN * TN * 16, SET = WM * WN * 64, STRIDE = 20, ROWS = BM + BN;
+    constexpr int ALL = ROWS * 4 * G, CHUNKS = ALL / SET;                    // 16-byte chunks of a block
+    static_assert(ALL % SET == 0, "whole chunks a thread");
+    static_assert(4 * G * ROWS * STRIDE >= BM * BN, "the second set's sums fit the blocks' place");
+    extern __shared__ __attribute__((aligned(16))) float lds[];               // [buffer][set][group][row][STRIDE]
+    const int set = threadIdx.x / SET, t = threadIdx.x % SET, lane = t & 63, wave = t >> 6;
+    const int wm = wave / WN, wn = wave % WN, r = lane & 15, q = (lane >> 4) * 4;
+    // neighbouring tiles of a weight strip to the same XCD (workgroups are dealt out to the eight in turn)
+    const int tiles_m = (M + BM - 1) / BM, tiles = tiles_m * ((N + BN - 1) / BN), each = (tiles + 7) / 8;
+    const int tile = (blockIdx.x % 8) * each + blockIdx.x / 8;
+    if (blockIdx.x / 8 >= each || tile >= tiles) return;
+    const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * BN;
+    const int parts = (K + part - 1) / part, half = (parts + 1) / 2;
+    const int begin = set * half * part, end = set ? K : min(K, half * part);
+    const int groups = (min(K, half * part) + 15) / 16, turns = (groups + G - 1) / G, per = part / 16;
+
+    floatx4 stage[CHUNKS];
+    auto load = [&](int k0) {                              // (chunk: four k of a row; a row's chunks side by side)
+#pragma unroll
+        for (int c = 0; c < CHUNKS; ++c) {
+            const int row = (t + c * SET) / (4 * G), k = k0 + (t + c * SET) % (4 * G) * 4;
+            const float* p = row < BM ? a + (size_t)min(m0 + row, M - 1) * K : w + (size_t)min(n0 + row - BM, N - 1) * K;
+            stage[c] = load_k4<VEC>(p, k, end);
+        }
+    };
+    floatx4 acc[TM][TN], sum[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = sum[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    load(begin);
+    int in_part = 0;
+    for (int turn = 0; turn < turns; ++turn) {
+        float* block = lds + ((turn & 1) * 2 + set) * (G * ROWS * STRIDE);
+#pragma unroll
+        for (int c = 0; c < CHUNKS; ++c) {
+            const int row = (t + c * SET) / (4 * G), k = (t + c * SET) % (4 * G);
+            *reinterpret_cast<floatx4*>(block + ((k >> 2) * ROWS + row) * STRIDE + (k & 3) * 4) = stage[c];
+        }
+        __syncthreads();
+        if (turn + 1 < turns) load(begin + (turn + 1) * 16 * G);
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const float* rows = block + g * ROWS * STRIDE;
+            floatx4 av[TM], wv[TN];
+#pragma unroll
+            for (int i = 0; i < TM; ++i) av[i] = *reinterpret_cast<const floatx4*>(rows + ((wm * TM + i) * 16 + r) * STRIDE + q);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) wv[j] = *reinterpret_cast<const floatx4*>(rows + (BM + (wn * TN + j) * 16 + r) * STRIDE + q);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i][e], wv[j][e], acc[i][j], 0, 0, 0);
+            // (groups beyond the set's half hold zeros and add nothing)
+            if (++in_part == per || (turn + 1 == turns && g + 1 == G)) {
+                in_part = 0;
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) {
+                        sum[i][j] += acc[i][j];
+                        acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+                    }
+            }
         }
     }
+    __syncthreads();
+    if (set == 1) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+                *reinterpret_cast<floatx4*>(lds + (((wave * TM + i) * TN + j) * 64 + lane) * 4) = sum[i][j];
+    }
+    __syncthreads();
+    if (set == 1) return;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const floatx4 second = *reinterpret_cast<const floatx4*>(lds + (((wave * TM + i) * TN + j) * 64 + lane) * 4);
+            const int n = n0 + (wn * TN + j) * 16 + r;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int m = m0 + (wm * TM + i) * 16 + q + e;
+                if (m < M && n < N) out[(size_t)m * N + n] = sum[i][j][e] + second[e];
+            }
+        }
+}
+
+template <int TM, int NT, bool VEC>
+static int launch_f32_rows(const float* a, const float* w, float* out, int M, int N, int K, hipStream_t stream) {
+    gemm_f32_rows_kernel<TM, NT, VEC><<<(N + NT * 16 - 1) / (NT * 16), 512, 0, stream>>>(a, w, out, M, N, K, part_of(K));
+    return (int)hipGetLastError();
+}
+
+template <int T, int G, bool VEC>
+static int launch_f32_tile(const float* a, const float* w, float* out, int M, int N, int K, hipStream_t stream) {
+    constexpr int B = 2 * T * 16;
+    const long long tiles = (long long)((M + B - 1) / B) * ((N + B - 1) / B);
+    if (tiles > 0x7ffffff0LL) return -2;
+    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_tile_kernel<2, 2, T, T, G, VEC>),
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, 4 * G * 2 * B * 20 * sizeof(float));
+    if (allowed != hipSuccess) return (int)allowed;
+    gemm_f32_tile_kernel<2, 2, T, T, G, VEC><<<(unsigned)((tiles + 7) / 8 * 8), 512, 4 * G * 2 * B * 20 * sizeof(float), stream>>>(
+        a, w, out, M, N, K, part_of(K));
+    return (int)hipGetLastError();
+}
+
+template <bool VEC>
+static int launch_gemm_f32(const float* a, const float* w, float* out, int M, int N, int K, hipStream_t stream) {
+    const int strips = (N + 15) / 16;
+    if (M <= 16) {
+        // Four strips a workgroup, for which the rows are read once, where that still gives two workgroups a compute unit
+        // and the rows weigh something beside the weight: 16 rows of N x K = 24576 x 4096 88.6 us for 102.0, of 151936 x
+        // 1024 126 for 158 (5 TB/s of weight); but 4 rows 85.7 for 73.1 (5.5 TB/s).  The weights of a layer of the 0.6B
+        // sizes (4096 x 1024, 1024 x 2048, 6144 x 1024, 1024 x 3072) take 8 to 11 us with 8 rows, where a 64 x 64 tile
+        // with k from end to end took 101, 196, 101 and 292.
+        return M > 8 && strips >= 1024 ? launch_f32_rows<1, 4, VEC>(a, w, out, M, N, K, stream)
+                                       : launch_f32_rows<1, 1, VEC>(a, w, out, M, N, K, stream);
+    }
+    if (M <= 32)
+        // (two strips beyond one a compute unit: 6144 x 1024 11.3 us for 13.6; up to 256 strips one: 4096 x 1024 9.1 for 11.5)
+        return strips > 256 ? launch_f32_rows<2, 2, VEC>(a, w, out, M, N, K, stream)
+                            : launch_f32_rows<2, 1, VEC>(a, w, out, M, N, K, stream);
+    // The square tile whose workgroups, one a compute unit at a time, are done first: a tile of 64 takes 1 / 3.7 of the time
+    // of one of 128, a tile of 32 0.35 of one of 64 (at 2048 rows of 4096 x 12288, 24576 x 4096 and 2048 x 2112; tiles of
+    // 128 reach 120 TFLOP/s there).  1500 rows of 6144 x 1024 take 197 us in tiles of 64 and 228 in those of 128, 64 rows
+    // of 1024 x 3072 27 in those of 32 for 66 (from 33 rows on the kernel above is no faster: 30 us here).
+    auto cost = [&](int b, double one) {
+        return one * (double)(((long long)((M + b - 1) / b) * ((N + b - 1) / b) + 255) / 256);
+    };
+    const double c32 = cost(32, 0.35), c64 = cost(64, 1.0), c128 = cost(128, 3.7);
+    if (c32 <= c64 && c32 <= c128) return launch_f32_tile<1, 4, VEC>(a, w, out, M, N, K, stream);
+    return c64 <= c128 ? launch_f32_tile<2, 2, VEC>(a, w, out, M, N, K, stream)
+                       : launch_f32_tile<4, 1, VEC>(a, w, out, M, N, K, stream);
 }
 
 extern "C" int mlr_gemm(const void* a, const void* w, void* out, int M, int N, int K, int out_float,
@@ -72,10 +270,10 @@ extern "C" int mlr_gemm(const void* a, const void* w, void* out, int M, int N, i
     (void)out_float;                                   // the float engine's outputs are float
     if (M <= 0 || N <= 0) return 0;
     if (K <= 0) return -1;
-    dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
-    if (grid.y > 65535) return -2;
-    gemm_f32_kernel<<<grid, 256, 0, stream>>>((const float*)a, (const float*)w, (float*)out, M, N, K);
-    return (int)hipGetLastError();
+    if ((M + 63) / 64 > 65535) return -2;
+    const bool aligned = K % 4 == 0 && ((uintptr_t)a | (uintptr_t)w) % 16 == 0;
+    return aligned ? launch_gemm_f32<true>((const float*)a, (const float*)w, (float*)out, M, N, K, stream)
+                   : launch_gemm_f32<false>((const float*)a, (const float*)w, (float*)out, M, N, K, stream);
 }
 
 #else

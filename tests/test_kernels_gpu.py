@@ -209,6 +209,34 @@ def test_gemm_rows_do_not_depend_on_the_batch(dtype):
         torch.testing.assert_close(small.float(), full[:64].float(), atol=0.13, rtol=1e-2)   # one bfloat16 step at |x| ~ 16
 
 
+@pytest.mark.parametrize("n,kk", [(1, 4), (15, 1), (17, 60), (33, 64), (70, 511), (64, 516), (130, 528), (16400, 96), (4112, 1030), (96, 3072),
+                                  (40, 12296)])
+def test_gemm_float_edges(n, kk):
+    """The float product at the edges of its row counts (8/9, 16/17, 32/33: another kernel or strip width), tiles and parts of
+    k, rows that start on 16 bytes and rows that do not: one order of additions, so a row's bits are those it has alone; and
+    every element within the bound of a sum in at most eight chains, (k / 8 + 16 + 9) 2^-24 sum |a w| (a part is rounded up to
+    16, at least 64; then nine additions)."""
+    k = kernels(torch.float32)
+    rows = 300 if n < 5000 else 70
+    a, w = rnd((rows, kk), torch.float32, 21), rnd((n, kk), torch.float32, 22)
+    a[3] *= 1e-20                                        # (products of row 3 below the smallest normal number)
+    w[0] *= 1e-20
+
+    def run(lo, hi):
+        out = torch.full((hi - lo, n), float("nan"), device="cuda")
+        k.gemm(a[lo:hi].contiguous(), w, out)
+        return out
+    whole = run(0, rows)
+    bound = (max(kk / 8 + 16, 64) + 9) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T) + kk * 2.0 ** -149
+    assert bool(((whole.double() - a.double() @ w.double().T).abs() <= bound).all())
+    for lo, hi in [(0, 1), (3, 4), (1, 9), (0, 9), (2, 18), (5, 22), (0, 32), (4, 37), (0, 64), (1, 66), (0, rows - 1)]:
+        assert torch.equal(run(lo, hi), whole[lo:hi]), (lo, hi)
+    shifted = torch.empty(rows * kk + 1, device="cuda")[1:].view(rows, kk).copy_(a)      # rows 4 bytes off
+    out = torch.empty((rows, n), device="cuda")
+    k.gemm(shifted, w, out)
+    assert torch.equal(out, whole)
+
+
 @pytest.mark.parametrize("shape", [0, 1, 2, 3])
 @pytest.mark.parametrize("gated", [False, True])
 @pytest.mark.parametrize("mnk", [(65, 70, 64), (300, 257, 192), (513, 1000, 128), (128, 256, 1024), (1, 5, 320)])
