@@ -236,6 +236,207 @@ __global__ __launch_bounds__(64) void attention_combine_kernel(AttnArgs a) {
     }
 }
 
+#if !MLR_BF16
+// The float engine's attention on v_mfma_f32_16x16x4_f32 (32-bit products and sums) for head sizes and pages that are
+// multiples of 16 and up to 16 query heads a kv head.  A workgroup serves 16 columns -- consecutive tokens of one request
+// times the query heads of one kv head -- which share what it reads of keys and values; the kernel above, one token a
+// workgroup, fetches every value of a channel from a cache line of its own (16 heads on 8 of 128 channels, pages of 16: 111 us for
+// eight tokens behind 400 keys, 306 behind 4000, 0.68 ms for a prompt of 400 and 16.7 for one of 2048; here 19, 63, 53 us
+// and 0.57 ms).  Groups are found by the kernel: a row leads one when it is a multiple of the tokens a group holds or does
+// not continue the row before it.
+//
+// Keys are walked in tiles of 16 at absolute multiples of 16, wavefront w the tiles t with t % 4 == w, their partial
+// results merged in the order 0..3; a tile that a column does not see changes nothing of it.  A column's sums and their
+// order follow from its own position alone, whatever stands beside it.  Per tile: scores^T = K . Q^T (a lane holds four
+// channels of a key's row and of a query's: one 16-byte load each), softmax with a running maximum, out^T += V^T . P^T,
+// whose operand P lies in the registers as the first product leaves it (a lane: keys 4 (lane / 16) + i of column
+// lane % 16) and whose V is four keys of a channel, side by side in the transposed page.
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
+
+template <int NC, bool EXACT>
+__global__ __launch_bounds__(256, NC <= 4 ? 3 : NC <= 8 ? 2 : 1) void attention_f32_kernel(AttnArgs a, int rows) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];              // [4][D][17], maxima [4][16], sums [4][16]
+    const int D = EXACT ? NC * 16 : a.head_dim, nc = EXACT ? NC : a.head_dim / 16, P = a.page_size;
+    const int g = a.q_heads / a.kv_heads, per = max(1, 16 / g);
+    // the rows that lead whatever stands before them come first, a prompt's last and longest in front, the others behind:
+    // a workgroup that has nothing to do is over soon, but not beside one that keeps its compute unit's registers
+    const int blocks = (rows + per - 1) / per;
+    const int m = (blocks - 1 - (int)blockIdx.x % blocks) * per + blockIdx.x / blocks, kvh = blockIdx.y, split = blockIdx.z;
+    if (m >= rows) return;
+    const int slot = a.slots[m], pos0 = a.positions[m];
+    if (m % per != 0 && a.slots[m - 1] == slot && a.positions[m - 1] == pos0 - 1) return;      // (the row before leads)
+    int ntok = 1;
+    while ((m + ntok) % per != 0 && m + ntok < rows && a.slots[m + ntok] == slot && a.positions[m + ntok] == pos0 + ntok) ++ntok;
+    int lo = a.window > 0 ? max(0, pos0 - a.window + 1) : 0, hi = pos0 + ntok;
+    if (a.max_splits > 1) {
+        lo = max(lo, split * a.split_keys);
+        hi = min(hi, (split + 1) * a.split_keys);
+        if (lo >= hi) return;                                                // (no token of the group reads this part)
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, b4 = (lane >> 4) * 4;
+    const int tok = min(c / g, ntok - 1), head = kvh * g + c % g, pos = pos0 + tok;
+    const int from = a.window > 0 ? max(0, pos - a.window + 1) : 0;          // this column sees keys from .. pos
+
+    floatx4 q[NC];
+    const float* qr = a.q + ((size_t)(m + tok) * a.q_heads + head) * D + b4;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) q[i] = EXACT || i < nc ? *reinterpret_cast<const floatx4*>(qr + i * 16) : floatx4{0.f, 0.f, 0.f, 0.f};
+
+    const int t_end = (hi + 15) / 16, t_first = lo / 16 + ((wave - lo / 16) & 3);
+    const int32_t* table = a.block_table + (size_t)slot * a.max_blocks;
+    int pages = -1;                                                          // lane i: page of the wavefront's tile i of 64
+    floatx4 k[NC], v[NC];
+    auto load_k = [&](int t, int page) {
+        const float* kr = a.k_pages + ((long long)max(page, 0) * a.kv_heads + kvh) * P * D + (size_t)(t * 16 % P + c) * D + b4;
+#pragma unroll
+        for (int i = 0; i < NC; ++i)
+            if (EXACT || i < nc) k[i] = *reinterpret_cast<const floatx4*>(kr + i * 16);
+    };
+    auto load_v = [&](int t, int page) {
+        const float* vr = a.v_pages + ((long long)max(page, 0) * a.kv_heads + kvh) * P * D + (size_t)c * P + t * 16 % P + b4;
+#pragma unroll
+        for (int i = 0; i < NC; ++i)
+            if (EXACT || i < nc) v[i] = *reinterpret_cast<const floatx4*>(vr + (size_t)i * 16 * P);
+    };
+    float run_max = -INFINITY, run_sum = 0.f;
+    floatx4 acc[NC];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int t0 = t_first; t0 < t_end; t0 += 256) {                          // 64 tiles of the wavefront at a time
+        const int block = (t0 + 4 * lane) * 16 / P;
+        pages = t0 + 4 * lane < t_end && block < a.max_blocks ? table[block] : -1;
+        const int n = min(64, (t_end - t0 + 3) / 4);
+        int page = __shfl(pages, 0);
+        load_k(t0, page);
+        load_v(t0, page);
+        for (int n_t = 0; n_t < n; ++n_t) {
+            const int t = t0 + 4 * n_t, key0 = t * 16 + b4, next_page = __shfl(pages, min(n_t + 1, n - 1));
+            floatx4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < NC; ++i)
+                if (EXACT || i < nc) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i][e], q[i][e], s, 0, 0, 0);
+                }
+            // (the next tile's keys are on their way from here on, its values from the end of this turn on: each into the
+            // registers that are free then)
+            if (n_t + 1 < n) load_k(t + 4, next_page);
+            float p[4], top = -INFINITY;
+            bool seen[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                seen[i] = page >= 0 && key0 + i >= from && key0 + i <= pos;
+                p[i] = seen[i] ? s[i] * a.scale : -INFINITY;
+                top = fmaxf(top, p[i]);
+            }
+            top = fmaxf(top, __shfl_xor(top, 16));
+            top = fmaxf(top, __shfl_xor(top, 32));
+            const float new_max = fmaxf(run_max, top);
+            const float corr = new_max > -INFINITY ? expf(run_max - new_max) : 1.f;
+            float sum = 0.f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                // (a score that is not a number stays one where nothing else sets the maximum: pages that nobody wrote show)
+                p[i] = seen[i] && new_max > -INFINITY ? expf(p[i] - new_max) : p[i] != p[i] ? p[i] : 0.f;
+                sum += p[i];
+            }
+            sum += __shfl_xor(sum, 16);
+            sum += __shfl_xor(sum, 32);
+            run_sum = run_sum * corr + sum;
+            run_max = new_max;
+#pragma unroll
+            for (int i = 0; i < NC; ++i) acc[i] *= corr;
+            // Every token of the group sees the whole tile, or values that a token must not see would meet its probability
+            // of zero: places that were never written are cleared, and where a value is not finite the tokens go one by one.
+            const bool inner = page >= 0 && t * 16 + 15 <= pos0 && (a.window <= 0 || t * 16 > pos0 + ntok - 1 - a.window);
+            bool odd = false;
+            if (!inner) {
+#pragma unroll
+                for (int i = 0; i < NC; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        if (page < 0 || key0 + e < lo || key0 + e >= hi) v[i][e] = 0.f;
+                        if (EXACT || i < nc) odd |= !(fabsf(v[i][e]) <= 3.402823466e38f);
+                    }
+            }
+            if (__builtin_expect(__any(odd), 0)) {
+                for (int other = 0; other < ntok; ++other) {
+                    const int own = pos0 + other, own_from = a.window > 0 ? max(0, own - a.window + 1) : 0;
+#pragma unroll
+                    for (int i = 0; i < NC; ++i) {
+                        floatx4 next = acc[i];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            next = __builtin_amdgcn_mfma_f32_16x16x4f32(key0 + e >= own_from && key0 + e <= own ? v[i][e] : 0.f, p[e], next, 0, 0, 0);
+                        if (tok == other) acc[i] = next;
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < NC; ++i)
+                    if (EXACT || i < nc) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i][e], p[e], acc[i], 0, 0, 0);
+                    }
+            }
+            if (n_t + 1 < n) load_v(t + 4, next_page);
+            page = next_page;
+        }
+    }
+    // the four wavefronts' results, in the order 0..3
+    float* maxima = lds + 4 * D * 17;
+    float* sums = maxima + 64;
+    if (lane < 16) {
+        maxima[wave * 16 + c] = run_max;
+        sums[wave * 16 + c] = run_sum;
+    }
+    __syncthreads();
+    const float gmax = fmaxf(fmaxf(maxima[c], maxima[16 + c]), fmaxf(maxima[32 + c], maxima[48 + c]));
+    const float weight = run_max > -INFINITY ? expf(run_max - gmax) : run_sum;       // (no key: 0; none but NaN: NaN)
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+        if (EXACT || i < nc) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) lds[(wave * D + i * 16 + b4 + e) * 17 + c] = weight * acc[i][e];
+        }
+    __syncthreads();
+    for (int i = threadIdx.x; i < ntok * g * D; i += 256) {
+        const int col = i / D, d = i % D;
+        float num = 0.f, den = 0.f, most = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) most = fmaxf(most, maxima[w * 16 + col]);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const float top = maxima[w * 16 + col];
+            num += lds[(w * D + d) * 17 + col];
+            den += top > -INFINITY ? expf(top - most) * sums[w * 16 + col] : sums[w * 16 + col];
+        }
+        const size_t row = (size_t)(m + col / g) * a.q_heads + kvh * g + col % g;
+        if (a.max_splits > 1) {
+            float* dst = a.partial + (row * a.max_splits + split) * (D + 2);
+            dst[d] = num;
+            if (d == 0) {
+                dst[D] = most;
+                dst[D + 1] = den;
+            }
+        } else {
+            a.out[row * D + d] = den != 0.f ? num / den : 0.f;
+        }
+    }
+}
+
+template <int NC, bool EXACT>
+static int launch_attention_f32(const AttnArgs& a, int rows, hipStream_t stream) {
+    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_f32_kernel<NC, EXACT>),
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, (4 * NC * 16 * 17 + 128) * 4);
+    if (allowed != hipSuccess) return (int)allowed;
+    const int per = max(1, 16 / (a.q_heads / a.kv_heads)), blocks = (rows + per - 1) / per;
+    attention_f32_kernel<NC, EXACT><<<dim3(blocks * per, a.kv_heads, a.max_splits), 256, (4 * a.head_dim * 17 + 128) * sizeof(float), stream>>>(
+        a, rows);
+    return (int)hipGetLastError();
+}
+#endif
+
 extern "C" int mlr_paged_attention(
     const void* q, const void* k_pages, const void* v_pages, const int32_t* block_table,
     int max_blocks, const int32_t* slots, const int32_t* positions, void* out, float* partial,
@@ -252,9 +453,21 @@ extern "C" int mlr_paged_attention(
     const int head_chunks = (group + HEADS_PER_BLOCK - 1) / HEADS_PER_BLOCK;
     const size_t lds = sizeof(float) * ((size_t)HEADS_PER_BLOCK * head_dim +
                                         TILE_KEYS * (DIM_CHUNK + 1) + HEADS_PER_BLOCK * TILE_KEYS);
-    dim3 grid(rows, kv_heads, head_chunks * a.max_splits);
-    paged_attention_kernel<<<grid, 256, lds, stream>>>(a);
-    int err = (int)hipGetLastError();
+    int err = 0;
+#if !MLR_BF16
+    const bool aligned = ((uintptr_t)q | (uintptr_t)k_pages | (uintptr_t)v_pages) % 16 == 0;
+    if (head_dim % 16 == 0 && page_size % 16 == 0 && group <= 16 && aligned)
+        err = head_dim == 64    ? launch_attention_f32<4, true>(a, rows, stream)
+              : head_dim == 128 ? launch_attention_f32<8, true>(a, rows, stream)
+              : head_dim < 128  ? launch_attention_f32<8, false>(a, rows, stream)
+                                : launch_attention_f32<16, false>(a, rows, stream);
+    else
+#endif
+    {
+        dim3 grid(rows, kv_heads, head_chunks * a.max_splits);
+        paged_attention_kernel<<<grid, 256, lds, stream>>>(a);
+        err = (int)hipGetLastError();
+    }
     if (err != 0) return err;
     if (a.max_splits > 1) {
         attention_combine_kernel<<<dim3(rows, q_heads), 64, 0, stream>>>(a);

@@ -564,6 +564,43 @@ def test_paged_attention(dtype, case):
         assert torch.isnan(out4[lengths[0]:].float()).all()
 
 
+@pytest.mark.parametrize("hq,hkv,d,page,window,split_keys", [(4, 2, 128, 16, None, 0), (4, 2, 128, 16, None, 64), (6, 2, 64, 32, 20, 0),
+                                                             (16, 1, 48, 16, None, 0), (3, 1, 256, 16, 33, 64)])
+def test_paged_attention_float_rows_alone(hq, hkv, d, page, window, split_keys):
+    """The float engine: a token's bits do not depend on the tokens that share its workgroup, nor on where a call starts; and a
+    value that is not finite reaches exactly the tokens that see it, wherever it lies in a tile of 16 keys."""
+    k = kernels(torch.float32)
+    n, scale = 150, 1 / math.sqrt(d)
+    blocks = (n + page - 1) // page
+    q = rnd((n, hq * d), torch.float32, 40)
+    k_pages, v_pages = rnd((blocks + 1, hkv, page, d), torch.float32, 41), rnd((blocks + 1, hkv, d, page), torch.float32, 42)
+    k_pages[-1], v_pages[-1] = float("nan"), float("nan")
+    tail = n - (blocks - 1) * page                       # (behind the last key: never written)
+    k_pages[blocks - 1, :, tail:], v_pages[blocks - 1, :, :, tail:] = float("nan"), float("nan")
+    table = torch.full((1, blocks + 2), -1, dtype=torch.int32, device="cuda")
+    table[0, :blocks] = torch.arange(blocks, dtype=torch.int32)
+    splits = -(-n // split_keys) if split_keys else 1
+    partial = torch.full((k.attention_partial_numel(n, hq, d, splits),), float("nan"), device="cuda") if split_keys else None
+
+    def run(rows):
+        out = torch.full((len(rows), hq * d), float("nan"), device="cuda")
+        k.paged_attention(q[rows].contiguous(), k_pages, v_pages, table, torch.zeros(len(rows), dtype=torch.int32, device="cuda"),
+                          torch.tensor(rows, dtype=torch.int32, device="cuda"), out, hq, hkv, d, page, scale, window=window,
+                          split_keys=split_keys, max_splits=splits, partial=partial)
+        return out
+    every = list(range(n))
+    whole = run(every)
+    for rows in ([0], [n - 1], [5], every[3:], every[17:60], every[::-1], every[::7]):
+        assert torch.equal(run(rows), whole[rows])
+    for bad, at in ((float("inf"), 37), (float("nan"), 64), (float("-inf"), 143)):
+        kept = v_pages[at // page, :, :, at % page].clone()
+        v_pages[at // page, :, :, at % page] = bad
+        hit = torch.tensor([p >= at and (window is None or p - at < window) for p in every])
+        got = run(every)
+        assert torch.equal(got[~hit], whole[~hit]) and not torch.isfinite(got[hit]).any()
+        v_pages[at // page, :, :, at % page] = kept
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_attention_finds_one_far_key(dtype):
     """One key among a thousand matches the query (scaled so that its score stands out): the
