@@ -61,6 +61,11 @@ class Workspace:
         self._views[(name, dtype, shape)] = view
         return view
 
+    def room(self, name, dtype):
+        """Elements that the name's buffer holds now."""
+        buf = self._buffers.get((name, dtype))
+        return 0 if buf is None else buf.numel()
+
     def bytes(self):
         return self.planned_bytes + self.unplanned_bytes()
 
@@ -127,14 +132,14 @@ class StepContext:
         self._groups = {}
         self.fixed_groups = None
 
-    def token_groups(self, tokens_per_group, big_factor=0):
+    def token_groups(self, tokens_per_group, big_factor=0, without=()):
         """The step's rows cut into groups of consecutive tokens of one request, as device int32 vectors
         (first row of each group, tokens in each group) with their number.  Returns (small, big, (rows in
         small groups, one beyond the last batch row of a small group)): small groups hold at most
         `tokens_per_group` tokens; with big_factor > 0, a request that brings more than `tokens_per_group`
         tokens is cut into big groups of at most big_factor * tokens_per_group instead (prompt portions), else
-        `big` is empty."""
-        key = (tokens_per_group, big_factor)
+        `big` is empty.  `without`: entries of the step (their numbers, ascending) whose rows are left out."""
+        key = (tokens_per_group, big_factor, without)
         hit = self._groups.get(key)
         if hit is not None:
             return hit
@@ -142,25 +147,28 @@ class StepContext:
             return self.fixed_groups[key]
         first, count, big_first, big_count = [], [], [], []
         small_rows = small_end = 0
-        for _, row, n, _ in self.segments:
+        for i, (_, row, n, _) in enumerate(self.segments):
+            if i in without:
+                continue
             if big_factor > 0 and n > tokens_per_group:
                 size = big_factor * tokens_per_group
-                for i in range(0, n, size):
-                    big_first.append(row + i)
-                    big_count.append(min(size, n - i))
+                for at in range(0, n, size):
+                    big_first.append(row + at)
+                    big_count.append(min(size, n - at))
             else:
                 small_rows += n
                 small_end = max(small_end, row + n)
-                for i in range(0, n, tokens_per_group):
-                    first.append(row + i)
-                    count.append(min(tokens_per_group, n - i))
+                for at in range(0, n, tokens_per_group):
+                    first.append(row + at)
+                    count.append(min(tokens_per_group, n - at))
         g, gb = len(first), len(big_first)
         if self.fixed_groups is not None:
             # a step that is to be captured: its groups depend on the lengths of its entries only, so they
             # get a tensor of their own once (this is the eager run before the capture) and stay there
             dev = torch.tensor(first + count + big_first + big_count + [0], dtype=torch.int32, device=self.workspace.device)
         else:
-            dev = self.workspace.get(f"token_groups_{tokens_per_group}_{big_factor}", (2 * (g + gb),), torch.int32)
+            rest = "_rest" if without else ""
+            dev = self.workspace.get(f"token_groups_{tokens_per_group}_{big_factor}{rest}", (2 * (g + gb),), torch.int32)
             if self._group_upload is None:
                 self._group_upload = Uploader(4096, dev.device)
             self._group_upload.send(first + count + big_first + big_count, dev)

@@ -84,26 +84,38 @@ class Runner:
         if _kv_dtype(kv_dtype, self.dtype) != self.dtype:
             raise ValueError(f"kv_dtype {kv_dtype}: the {self.dtype} engine's attention kernels read pages of their own "
                              "element type only")
-        if max_tokens is None:
-            # the pool takes what the budget leaves beside the scratch buffers, the metadata and the library's
-            # scratch (the weights are resident already and no longer part of the free memory)
-            other = MemoryPlan(workspace=Workspace.plan_bytes(workspace_plan), metadata=5 * 4 * self.max_batch_tokens + 8,
-                               library_scratch=LIBRARY_GEMM_WORKSPACE if uses_library else 0).to_allocate()
-            room = device_budget(device_budget_bytes or 0, self.device) - other
-            max_tokens = CacheManager.tokens_that_fit(model.cache_entry_specs, self.dtype, page_size, max_slots,
-                                                      self.max_length, room)
-            if max_tokens <= 0:
-                raise MemoryBudgetError(f"the device's budget leaves {room} bytes for the cache: not one page a group")
-            if device_budget_bytes is None:
-                device_budget_bytes = 0
-        self.max_tokens = max_tokens
-        kv, tables, state = CacheManager.plan(model.cache_entry_specs, self.dtype, page_size, max_tokens, max_slots,
-                                              self.max_length)
-        self.memory_plan = MemoryPlan(
+        plan = lambda workspace, pages: MemoryPlan(
             weights=model.arena.planned if model.arena is not None else model.weight_bytes(),
-            kv_pages=kv, block_tables=tables, state=state, workspace=Workspace.plan_bytes(workspace_plan),
+            kv_pages=pages[0], block_tables=pages[1], state=pages[2], workspace=Workspace.plan_bytes(workspace),
             metadata=5 * 4 * self.max_batch_tokens + 8, library_scratch=LIBRARY_GEMM_WORKSPACE if uses_library else 0)
-        self.memory_plan.check(device_budget_bytes, self.device)
+        auto = max_tokens is None
+        if auto and device_budget_bytes is None:
+            device_budget_bytes = 0
+        for spare in (True, False):
+            # (first with the scratch memory that some parts would like besides what they need; without it where that does
+            # not fit)
+            if not spare:
+                workspace_plan = model.workspace_plan(self.max_batch_tokens, self.max_logits_rows, dict(limits, spare=False))
+            if auto:
+                # the pool takes what the budget leaves beside the scratch buffers, the metadata and the library's
+                # scratch (the weights are resident already and no longer part of the free memory)
+                room = device_budget(device_budget_bytes, self.device) - plan(workspace_plan, (0, 0, 0)).to_allocate()
+                max_tokens = CacheManager.tokens_that_fit(model.cache_entry_specs, self.dtype, page_size, max_slots,
+                                                          self.max_length, room)
+                if max_tokens <= 0:
+                    if spare:
+                        continue
+                    raise MemoryBudgetError(f"the device's budget leaves {room} bytes for the cache: not one page a group")
+            self.max_tokens = max_tokens
+            kv, tables, state = CacheManager.plan(model.cache_entry_specs, self.dtype, page_size, max_tokens, max_slots,
+                                                  self.max_length)
+            self.memory_plan = plan(workspace_plan, (kv, tables, state))
+            try:
+                self.memory_plan.check(device_budget_bytes, self.device)
+                break
+            except MemoryBudgetError:
+                if not spare:
+                    raise
         self.cache = CacheManager(model.cache_entry_specs, self.dtype, self.device, page_size,
                                   max_tokens, max_slots, self.max_length)
         assert (self.cache.kv_bytes(), self.cache.table_bytes(), self.cache.state_bytes()) == (kv, tables, state), \

@@ -1669,6 +1669,98 @@ class Kernels:
             _p(partial if splits > 1 else None), _c_int(int(split_keys)), _c_int(int(splits)), _stream())
         _ok(code, "sink_attention_tiles")
 
+    PORTION_PAGES = 1024          # page ids of a group's keys that the portion kernel keeps
+
+    def portion_attention_supported(self, q_heads, kv_heads, key_dim, value_dim, k_row, v_row, page_size, mask=None, mask_size=0,
+                                    max_context=0, keep_first=0):
+        """Whether `portion_attention` takes these sizes: the bfloat16 engine, keys of 128 channels with as many value channels
+        or of 64 with 64 or 128, cache rows that start at multiples of 16 bytes, pages of a power of two of at least 16
+        tokens, and a group's keys on no more pages than the kernel keeps."""
+        whole = self.SINK_MASKS.get(mask, 0) == 0
+        reach = max_context if whole else mask_size + 256 + (keep_first if keep_first > 0 else 0)
+        return (self.dtype == torch.bfloat16 and (key_dim, value_dim) in ((128, 128), (64, 128), (64, 64)) and k_row % 8 == 0
+                and v_row % 8 == 0 and page_size >= 16 and page_size & (page_size - 1) == 0
+                and reach // page_size + 4 <= self.PORTION_PAGES and kv_heads * q_heads <= 65535)
+
+    @timed("attention")
+    def portion_attention(self, q, k_pages, v_pages, block_table, slots, positions, sink, out, group_first, group_count, groups,
+                          columns, head_block, q_heads, kv_heads, key_dim, value_dim, page_size, scale, mask=None, mask_size=0,
+                          max_context=0, keep_first=0, softcap=None):
+        """`sink_attention` on 32 x 32 matrix tiles for `groups` groups of consecutive tokens of one request each, at most
+        columns / head_block tokens a group (columns: 64 or 128)."""
+        _tensor(q, "q", self.dtype, ndim=2)
+        rows = q.shape[0]
+        _need(q.shape[1] == q_heads * key_dim, "q: wrong width")
+        k_row = self._sink_pages(k_pages, "k_pages", kv_heads, page_size, key_dim)
+        v_row = self._sink_pages(v_pages, "v_pages", kv_heads, page_size, value_dim)
+        _need(mask in self.SINK_MASKS, f"mask {mask!r}: one of all, window, chunk")
+        kind = self.SINK_MASKS[mask]
+        _need(kind == 0 or mask_size >= 1, "a window or chunk needs a positive size")
+        _need(self.portion_attention_supported(q_heads, kv_heads, key_dim, value_dim, k_row, v_row, page_size, mask, mask_size, max_context,
+                                               self._kept(kind, keep_first)), "portion_attention: sizes that the kernel does not take")
+        _tensor(block_table, "block_table", torch.int32, ndim=2)
+        _tensor(slots, "slots", torch.int32, (rows,))
+        _tensor(positions, "positions", torch.int32, (rows,))
+        _tensor(group_first, "group_first", torch.int32, ndim=1)
+        _tensor(group_count, "group_count", torch.int32, ndim=1)
+        _need(group_first.numel() >= groups and group_count.numel() >= groups, "group vectors too short")
+        if sink is not None:
+            _tensor(sink, "sink", torch.float32, (q_heads,))
+        _tensor(out, "out", self.dtype, (rows, q_heads * value_dim))
+        _ok(self._lib("portion_attention").mlr_portion_attention(
+            _p(q), ctypes.c_long(q.shape[1]), _p(k_pages), ctypes.c_long(k_row), _p(v_pages), ctypes.c_long(v_row), _p(block_table),
+            _c_int(block_table.shape[1]), _p(slots), _p(positions), _p(sink), _p(out), ctypes.c_long(out.shape[1]), _p(group_first),
+            _p(group_count), _c_int(groups), _c_int(columns), _c_int(head_block), _c_int(q_heads), _c_int(kv_heads), _c_int(key_dim),
+            _c_int(value_dim), _c_int(page_size), _c_int(kind), _c_int(int(mask_size)), _c_int(self._kept(kind, keep_first)),
+            _c_float(self._cap(softcap)), _c_int(int(max_context)), _c_float(scale), _stream()), "portion_attention")
+
+    def latent_portions_supported(self, head_dim, rot_dim, value_dim, rank):
+        """Whether a portion's latent attention may run on keys and values that are made for it (`portion_attention_split`)."""
+        return self.dtype == torch.bfloat16 and (head_dim, rot_dim, value_dim) == (128, 64, 128) and rank % 8 == 0
+
+    @timed("attention")
+    def latent_rows(self, pages, block_table, slots, row, key0, keys, page_size, rank, latent, shared):
+        """Rows key0 .. key0 + keys - 1 of the request of batch row `row`: latent parts [keys, rank], shared key parts
+        [keys, rot], out of its pages."""
+        rot = shared.shape[1]
+        _tensor(latent, "latent", self.dtype, (keys, rank))
+        _tensor(shared, "shared", self.dtype, (keys, rot))
+        width = self._sink_pages(pages, "pages", 1, page_size, rank + rot)
+        _tensor(block_table, "block_table", torch.int32, ndim=2)
+        _tensor(slots, "slots", torch.int32, ndim=1)
+        _need(0 <= row < slots.numel() and key0 >= 0, "latent_rows: no such row")
+        _ok(self._lib("portion_attention").mlr_latent_rows(
+            _p(pages), ctypes.c_long(width), _p(block_table), _c_int(block_table.shape[1]), _p(slots), _c_int(row), _c_int(page_size),
+            _c_int(key0), _c_int(keys), _c_int(rank), _c_int(rot), _p(latent), _p(shared), _stream()), "latent_rows")
+
+    @timed("attention")
+    def portion_attention_split(self, q_plain, q_turned, keys, shared, values, slots, positions, sink, out, row, rows, key0, columns,
+                                heads, scale, mask=None, mask_size=0):
+        """Batch rows row .. row + rows - 1, a portion of one request, over its keys from position key0 on, every head with keys
+        and values of its own: score = (q_plain . key + q_turned . shared) * scale.  q_plain [M, heads, 128] and q_turned
+        [M, heads, 64] (views with channels side by side), keys and values [K, heads, 128], shared [K, 64]."""
+        _need(q_plain.dtype == q_turned.dtype == self.dtype and q_plain.stride(2) == q_turned.stride(2) == 1, "queries: channels side by side")
+        m = q_plain.shape[0]
+        _need(tuple(q_plain.shape) == (m, heads, 128) and tuple(q_turned.shape) == (m, heads, 64), "queries: wrong sizes")
+        _need(0 <= row and rows >= 1 and row + rows <= m, "portion_attention_split: rows beyond the batch")
+        n = keys.shape[0]
+        _tensor(keys, "keys", self.dtype, (n, heads * 128))
+        _tensor(values, "values", self.dtype, (n, heads * 128))
+        _tensor(shared, "shared", self.dtype, (n, 64))
+        _need(mask in self.SINK_MASKS and (self.SINK_MASKS[mask] == 0 or mask_size >= 1), f"mask {mask!r} of size {mask_size}")
+        _tensor(slots, "slots", torch.int32, (m,))
+        _tensor(positions, "positions", torch.int32, (m,))
+        if sink is not None:
+            _tensor(sink, "sink", torch.float32, (heads,))
+        _tensor(out, "out", self.dtype, (m, heads * 128))
+        aligned = all(t.data_ptr() % 16 == 0 for t in (q_plain, q_turned, keys, shared, values))
+        _need(aligned and all(s % 8 == 0 for s in q_plain.stride()[:2] + q_turned.stride()[:2]), "queries: rows and heads at multiples of 16 bytes")
+        _ok(self._lib("portion_attention").mlr_portion_attention_split(
+            _p(q_plain), ctypes.c_long(q_plain.stride(0)), ctypes.c_long(q_plain.stride(1)), _p(q_turned), ctypes.c_long(q_turned.stride(0)),
+            ctypes.c_long(q_turned.stride(1)), _p(keys), _p(shared), _p(values), _p(slots), _p(positions), _p(sink), _p(out),
+            ctypes.c_long(out.shape[1]), _c_int(row), _c_int(rows), _c_int(key0), _c_int(columns), _c_int(heads), _c_int(128), _c_int(64),
+            _c_int(128), _c_int(self.SINK_MASKS[mask]), _c_int(int(mask_size)), _c_float(scale), _stream()), "portion_attention_split")
+
     @staticmethod
     def sink_partial_numel(groups, tokens, q_heads, value_dim, splits):
         """Floats that the shares of `splits` key ranges take for `groups` groups of up to `tokens` tokens."""

@@ -49,6 +49,32 @@ def _rope_table(position, ctx, device, rot_limit):
     return rotation.table, bool(rotation.interleaved)
 
 
+# Portions of latent attention that make keys and values of their own: from this many tokens and keys on (16 heads, rank
+# 512, a step of eight layers of which two are latent attention, made against moved: 32 tokens behind 1000 keys 1.92 ms
+# against 2.02, behind 4000 2.10 against 3.01; without context 512 tokens 3.17 against 3.09, 2048 5.4 against 6.5), and up
+# to this many keys (the scratch memory: 9.3 KB a key).
+PORTION_ROWS = 32
+PORTION_LEAST_KEYS = 768
+PORTION_KEYS = 16384
+
+
+def _portion_library(weight):
+    return ["portion_attention"] if weight is not None and weight.dtype == torch.bfloat16 else []
+
+
+def _row_ranges(segments, without):
+    """The batch rows of the step's entries but those `without`, as few ranges as there are."""
+    ranges = []
+    for i, (_, row, n, _) in enumerate(segments):
+        if i in without:
+            continue
+        if ranges and ranges[-1][1] == row:
+            ranges[-1] = (ranges[-1][0], row + n)
+        else:
+            ranges.append((row, row + n))
+    return ranges
+
+
 PARTIAL_CAP = 8 << 20         # floats that the shares of the key ranges of one launch may take at most
 RANGE_KEYS = 128              # the narrowest key range of a workgroup
 MOST_RANGES = 16              # key ranges of a group at most
@@ -57,8 +83,9 @@ MOST_RANGES = 16              # key ranges of a group at most
 def _groups_plan(rows, q_heads, kv_heads, value_dim):
     """The token-group vectors and the room for key ranges' shares that `attend` asks the step's context for."""
     from ..kernels.ops import Kernels
-    _, big_tokens, _, small_tokens = Kernels.sink_tiles_layout(q_heads, kv_heads)
-    return {(f"token_groups_{small_tokens}_{max(1, big_tokens // small_tokens)}", torch.int32): 2 * rows + 2,
+    big_heads, big_tokens, _, small_tokens = Kernels.sink_tiles_layout(q_heads, kv_heads)
+    factors = {max(1, big_tokens // small_tokens)} | {columns // min(big_heads, 32) // small_tokens for columns in (64, 128)}
+    return {**{(f"token_groups_{small_tokens}_{factor}", torch.int32): 2 * rows + 2 for factor in sorted(factors)},
             ("sink_partial", torch.float32): min(PARTIAL_CAP, Kernels.sink_partial_numel(rows, small_tokens, q_heads, value_dim, MOST_RANGES))}
 
 
@@ -82,17 +109,33 @@ def _key_ranges(ctx, groups, tokens, workgroups, q_heads, value_dim, mask, mask_
     return keys, -(-reach // keys), room
 
 
+def portion_columns(ctx, q_heads):
+    """Columns (token, head) of a portion kernel's workgroup: 128 (half the staging a column of those of 64) when the step
+    brings at least one such workgroup for every compute unit."""
+    return 128 if ctx.n_tokens * q_heads >= 128 * ctx.compute_units else 64
+
+
 def attend(ctx, q, k_pages, v_pages, view, sink, out, q_heads, kv_heads, key_dim, value_dim, scale, mask, mask_size,
-           keep_first=0, softcap=None):
-    """Every token of the step over the keys it sees.  The bfloat16 engine on the matrix cores where they take the
-    sizes (prompt portions in workgroups of 64 columns, single tokens and short portions in workgroups of 16 whose
-    wavefronts share the value channels); else, and in the float engine, one wavefront a (token, head), whose sums
-    follow from the token's position alone."""
+           keep_first=0, softcap=None, without=()):
+    """Every token of the step over the keys it sees (but those of the entries `without`).  The bfloat16 engine on the
+    matrix cores where they take the sizes (prompt portions in workgroups of 128 or 64 columns, single tokens and short
+    portions in workgroups of 16 whose wavefronts share the value channels); else, and in the float engine, one wavefront
+    a (token, head), whose sums follow from the token's position alone."""
     k = ctx.kernels
     if k.sink_tiles_supported(key_dim, value_dim, k_pages.shape[3], v_pages.shape[3], view.page_size, mask, mask_size,
                               ctx.max_positions, keep_first) and q.shape[1] % 8 == 0:
         big_heads, big_tokens, small_heads, small_tokens = k.sink_tiles_layout(q_heads, kv_heads)
-        small, big, _ = ctx.token_groups(small_tokens, max(1, big_tokens // small_tokens))
+        portions = k.portion_attention_supported(q_heads, kv_heads, key_dim, value_dim, k_pages.shape[3], v_pages.shape[3], view.page_size,
+                                                 mask, mask_size, ctx.max_positions, keep_first)
+        if portions:
+            columns, big_heads = portion_columns(ctx, q_heads), min(big_heads, 32)
+            big_tokens = columns // big_heads
+        small, big, _ = ctx.token_groups(small_tokens, max(1, big_tokens // small_tokens), without)
+        if portions and big[2] > 0:
+            k.portion_attention(q, k_pages, v_pages, view.block_table, ctx.slots, ctx.positions, sink, out, *big, columns, big_heads,
+                                q_heads, kv_heads, key_dim, value_dim, view.page_size, scale, mask, mask_size, ctx.max_positions,
+                                keep_first, softcap)
+            big = (None, None, 0)
         for (first, count, n), heads, split in ((big, big_heads, False), (small, small_heads, True)):
             if n == 0:
                 continue
@@ -164,7 +207,7 @@ class SinkAttention:
                          self.mask_size if self.mask is not None else None, keep_first=self.keep_first)
 
     def libraries(self):
-        return ["gemm", "sink_attention", "elementwise"]
+        return ["gemm", "sink_attention", "elementwise"] + _portion_library(self.o)
 
     def workspace_plan(self, rows, dtype, limits):
         s = self.spec
@@ -214,7 +257,7 @@ class LatentAttention:
         self.head_gate = getattr(s, "head_gate", None)
         if self.head_gate not in (None, "sigmoid"):
             raise PartError(f"head_gate {self.head_gate!r}: sigmoid or none")
-        self.proj = self.o = self.norm = self.uk_t = self.uv = self.sink = self.uq = self.q_norm = self.gate = None
+        self.proj = self.o = self.norm = self.uk = self.uk_t = self.uv = self.sink = self.uq = self.q_norm = self.gate = None
 
     def weight_specs(self):
         s = self.spec
@@ -245,6 +288,7 @@ class LatentAttention:
         # the key up-projection as the queries meet it: per head [rank, head_dim]
         self.uk_t = weights["uk"].view(s.heads, s.head_dim, s.rank).transpose(1, 2).contiguous()
         self.uv = weights["uv"].view(s.heads, s.value_dim, s.rank)
+        self.uk = weights["uk"]
         self.o = weights["o"]
         self.sink = weights["sink"] if s.sink else None
 
@@ -252,18 +296,66 @@ class LatentAttention:
         return PagedSpec((("latent", (1, PAGE, self.row)),), self.mask_size if self.mask is not None else None)
 
     def libraries(self):
-        return ["gemm", "grouped_gemm", "sink_attention", "elementwise"]
+        return ["gemm", "grouped_gemm", "sink_attention", "elementwise"] + _portion_library(self.o)
+
+    def _made(self, keys):
+        """Elements that a portion's made rows take: latent and shared parts, keys, values."""
+        s = self.spec
+        return keys * (self.row + s.heads * s.head_dim + self.o_width)
+
+    def _portions_planned(self, rows, dtype, limits):
+        """Elements of `latent_out` for the longest portion that makes its keys (0: none of this runner's does): its place is
+        free until the step's other rows come.  Without `limits["spare"]` no more than those other rows need."""
+        s = self.spec
+        if dtype != torch.bfloat16 or (s.head_dim, s.rot_dim, s.value_dim) != (128, 64, 128) or s.rank % 8 != 0 or not limits.get("spare", True):
+            return 0
+        most = limits["max_length"] if self.mask is None else min(limits["max_length"], self.mask_size + rows)
+        return self._made(min(most, PORTION_KEYS) + 64)
 
     def workspace_plan(self, rows, dtype, limits):
         s = self.spec
+        groups = _groups_plan(rows, s.heads, 1, s.rank)
+        rest = {(f"{name}_rest", kind): count for (name, kind), count in groups.items() if name.startswith("token_groups")}
         first = self.q_width if s.q_rank is None else s.q_rank
         more = {} if s.q_rank is None else {("latent_cq", dtype): rows * s.q_rank, ("latent_queries", dtype): rows * self.q_width}
         if self.head_gate is not None:
             more[("latent_gate", dtype)] = rows * s.heads
         return {("latent_proj", dtype): rows * (first + self.row + (s.heads if self.head_gate is not None else 0)),
                 ("latent_q", dtype): rows * s.heads * self.row,
-                ("latent_out", dtype): rows * s.heads * s.rank, ("attn", dtype): rows * self.o_width,
-                (self.out_name, dtype): rows * s.hidden, **more, **_groups_plan(rows, s.heads, 1, s.rank)}
+                ("latent_out", dtype): max(rows * s.heads * s.rank, self._portions_planned(rows, dtype, limits)), ("attn", dtype): rows * self.o_width,
+                (self.out_name, dtype): rows * s.hidden, **more, **rest, **groups}
+
+    def _portions(self, ctx):
+        """The step's entries whose keys and values are made for them: (entry, first batch row, tokens, first key, keys).
+        For a token the up-projections on the queries' side cost nothing, but then a pair (query, key) is rank + rot + rank
+        products a head; with keys and values made once for a portion it is head_dim + rot + value_dim, 1088 against 320 at
+        rank 512, for rank * (head_dim + value_dim) products a key and head.  Not in a step that is to be captured: first
+        key and number of keys would be fixed in the graph."""
+        s = self.spec
+        if ctx.fixed_groups is not None or not ctx.kernels.latent_portions_supported(s.head_dim, s.rot_dim, s.value_dim, s.rank):
+            return []
+        out, room = [], ctx.workspace.room("latent_out", torch.bfloat16)
+        for i, (_, row, n, p0) in enumerate(ctx.segments):
+            if n < PORTION_ROWS:
+                continue
+            first = 0 if self.mask is None else max(0, p0 - self.mask_size + 1) if self.mask == "window" else p0 // self.mask_size * self.mask_size
+            first = first // 64 * 64                     # (the kernel's blocks of keys start there)
+            if PORTION_LEAST_KEYS <= p0 + n - first <= PORTION_KEYS + 64 and self._made(p0 + n - first) <= room:
+                out.append((i, row, n, first, p0 + n - first))
+        return out
+
+    def _attend_portion(self, ctx, queries, q, pages, view, attn, row, n, first, keys):
+        s, k = self.spec, ctx.kernels
+        made, at, parts = ctx.workspace.get("latent_out", (self._made(keys),), attn.dtype), 0, []
+        for width in (s.rank, s.rot_dim, s.heads * s.head_dim, self.o_width):
+            parts.append(made[at:at + keys * width].view(keys, width))
+            at += keys * width
+        latent, shared, made_k, made_v = parts
+        k.latent_rows(pages, view.block_table, ctx.slots, row, first, keys, view.page_size, s.rank, latent, shared)
+        k.gemm(latent, self.uk, made_k)
+        k.gemm(latent, self.uv.view(self.o_width, s.rank), made_v)
+        k.portion_attention_split(queries, q, made_k, shared, made_v, ctx.slots, ctx.positions, self.sink, attn, row, n, first,
+                                  128 if n * s.heads >= 128 * ctx.compute_units else 64, s.heads, float(s.scale), self.mask, self.mask_size)
 
     def forward(self, ctx, x, cache_id, write_cache=True):
         s = self.spec
@@ -295,14 +387,22 @@ class LatentAttention:
             k.latent_prep(proj[:, s.q_rank:s.q_rank + self.row], q, pages, view.block_table, ctx.slots, ctx.positions, self.norm, float(s.eps),
                           rope, s.heads, s.head_dim, s.rot_dim, s.rank, view.page_size, write_cache, q_src=queries,
                           interleaved=interleaved)
-        # the plain query channels through the key up-projection, head by head, into the first `rank` channels
-        k.heads_gemm(torch.as_strided(queries, (m, s.heads, s.head_dim), (q_ld, s.head_dim + s.rot_dim, 1)), self.uk_t,
-                     torch.as_strided(q, (m, s.heads, s.rank), (s.heads * self.row, self.row, 1)))
-        lat = ctx.workspace.get("latent_out", (m, s.heads * s.rank), x.dtype)
-        attend(ctx, q, pages, pages, view, self.sink, lat, s.heads, 1, self.row, s.rank, float(s.scale), self.mask,
-               self.mask_size)
+        plain = torch.as_strided(queries, (m, s.heads, s.head_dim), (q_ld, s.head_dim + s.rot_dim, 1), queries.storage_offset())
         attn = ctx.workspace.get("attn", (m, self.o_width), x.dtype)
-        k.heads_gemm(lat.view(m, s.heads, s.rank), self.uv, attn.view(m, s.heads, s.value_dim))
+        portions = self._portions(ctx)
+        for _, row, n, first, keys in portions:
+            self._attend_portion(ctx, plain, q.view(m, s.heads, self.row)[:, :, s.rank:], pages, view, attn, row, n, first, keys)
+        rest = _row_ranges(ctx.segments, tuple(p[0] for p in portions)) if portions else [(0, m)]
+        # the others' plain query channels through the key up-projection, head by head, into the first `rank` channels
+        moved = torch.as_strided(q, (m, s.heads, s.rank), (s.heads * self.row, self.row, 1), q.storage_offset())
+        for r0, r1 in rest:
+            k.heads_gemm(plain[r0:r1], self.uk_t, moved[r0:r1])
+        if rest:
+            lat = ctx.workspace.get("latent_out", (m, s.heads * s.rank), x.dtype)
+            attend(ctx, q, pages, pages, view, self.sink, lat, s.heads, 1, self.row, s.rank, float(s.scale), self.mask,
+                   self.mask_size, without=tuple(p[0] for p in portions))
+        for r0, r1 in rest:
+            k.heads_gemm(lat.view(m, s.heads, s.rank)[r0:r1], self.uv, attn.view(m, s.heads, s.value_dim)[r0:r1])
         if gate is not None:
             k.head_gate_mul(attn, gate, attn, s.heads)
         out = ctx.workspace.get(self.out_name, (m, s.hidden), x.dtype)

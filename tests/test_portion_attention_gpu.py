@@ -1,0 +1,157 @@
+"""The attention of prompt portions with a mask rule on the 32 x 32 matrix tiles, and latent attention whose portions make
+keys and values of their own, against the same formulas in 64 bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+BF16 = torch.bfloat16
+
+
+def attended(q, keys, values, positions, mask, size, keep, sink, scale, cap):
+    """q [M, H, D] at `positions` over keys [T, G, D], values [T, G, V]: float64 [M, H, V]."""
+    q, keys, values = q.double(), keys.double(), values.double()
+    H, G, T = q.shape[1], keys.shape[1], keys.shape[0]
+    p, j = positions[:, None].cpu(), torch.arange(T)[None]
+    seen = j <= p
+    if mask == "window":
+        seen &= (p - j < size) | (j < keep)
+    elif mask == "chunk":
+        seen &= (j // size == p // size) | (j < keep)
+    out = []
+    for h in range(H):
+        s = (q[:, h] @ keys[:, h // (H // G)].T) * scale
+        s = s if cap is None else cap * torch.tanh(s / cap)
+        s = s.masked_fill(~seen, -torch.inf)
+        if sink is not None:
+            s = torch.cat([s, sink[h].double().expand(s.shape[0], 1)], 1)
+        out.append(torch.softmax(s, 1)[:, :T] @ values[:, h // (H // G)])
+    return torch.stack(out, 1)
+
+
+def rounded(g, *shape, scale=1.0):
+    return (torch.randn(shape, generator=g) * scale).to(BF16)
+
+
+def ints(values):
+    return torch.tensor(values, dtype=torch.int32, device="cuda")
+
+
+@pytest.mark.parametrize("mask,size,keep", [(None, 0, 0), ("window", 37, 0), ("window", 90, 70), ("window", 64, 5), ("window", 1, 0),
+                                            ("chunk", 24, 0), ("chunk", 64, 0)])
+@pytest.mark.parametrize("heads,kv,dim,vdim,page,cap,with_sink", [(8, 2, 128, 128, 16, None, True), (3, 3, 64, 64, 32, 20.0, False),
+                                                                  (20, 1, 64, 128, 128, None, False), (5, 1, 128, 128, 64, 6.0, True)])
+def test_portions_with_a_mask(mask, size, keep, heads, kv, dim, vdim, page, cap, with_sink):
+    """A portion that starts a prompt and one from the middle of another in one launch, whose lengths fill no group, block or
+    page; unwritten places and pages that a window has given back hold NaN."""
+    from mini_llm_runtime_amd.kernels import Kernels
+    k = Kernels(BF16)
+    g = torch.Generator().manual_seed(heads * 100 + size)
+    lengths, begins = [91, 333], [0, 201]
+    keys, values = [rounded(g, n, kv, dim, scale=0.5) for n in lengths], [rounded(g, n, kv, vdim) for n in lengths]
+    blocks = [-(-n // page) for n in lengths]
+    order = torch.randperm(sum(blocks) + 1, generator=g).tolist()
+    k_pages = torch.full((sum(blocks) + 1, kv, page, dim), float("nan"), dtype=BF16)
+    v_pages = torch.full((sum(blocks) + 1, kv, page, vdim), float("nan"), dtype=BF16)
+    table = torch.full((2, max(blocks) + 1), -1, dtype=torch.int32)
+    for r in range(2):
+        first_seen = begins[r] - size + 1 if mask == "window" else begins[r] // size * size if mask else 0
+        for b in range(blocks[r]):
+            if (b + 1) * page <= first_seen and b * page >= keep:
+                continue                                       # (given back)
+            page_id = order.pop()
+            table[r, b] = page_id
+            part = slice(b * page, min((b + 1) * page, lengths[r]))
+            k_pages[page_id, :, :part.stop - part.start] = keys[r][part].transpose(0, 1)
+            v_pages[page_id, :, :part.stop - part.start] = values[r][part].transpose(0, 1)
+    positions = torch.cat([torch.arange(b, n) for b, n in zip(begins, lengths)])
+    rows = [n - b for b, n in zip(begins, lengths)]
+    slots = [0] * rows[0] + [1] * rows[1]
+    q = rounded(g, sum(rows), heads, dim, scale=0.5)
+    sink = torch.randn(heads, generator=g) if with_sink else None
+    want = torch.cat([attended(q[:rows[0]], keys[0], values[0], positions[:rows[0]], mask, size, keep, sink, 0.25, cap),
+                      attended(q[rows[0]:], keys[1], values[1], positions[rows[0]:], mask, size, keep, sink, 0.25, cap)])
+    per = heads // kv
+    head_block = 1
+    while head_block < per:
+        head_block *= 2
+    for columns in (64, 128):
+        tokens = columns // head_block
+        first = [at for r, base in ((0, 0), (1, rows[0])) for at in range(base, base + rows[r], tokens)]
+        count = [min(tokens, (rows[0] if at < rows[0] else sum(rows)) - at) for at in first]
+        out = torch.full((sum(rows), heads * vdim), float("nan"), dtype=BF16, device="cuda")
+        assert k.portion_attention_supported(heads, kv, dim, vdim, dim, vdim, page, mask, size, 400, keep)
+        k.portion_attention(q.reshape(sum(rows), -1).cuda(), k_pages.cuda(), v_pages.cuda(), table.cuda(), ints(slots), positions.int().cuda(),
+                            None if sink is None else sink.cuda(), out, ints(first), ints(count), len(first), columns, head_block, heads,
+                            kv, dim, vdim, page, 0.25, mask, size, 400, keep, cap)
+        # probabilities and the result are rounded to 2^-9 each, of values of size 1
+        torch.testing.assert_close(out.double().cpu().view(want.shape), want, atol=1.5e-2, rtol=1e-2)
+
+
+@pytest.mark.parametrize("mask,size", [(None, 0), ("window", 100), ("window", 7), ("chunk", 64)])
+@pytest.mark.parametrize("heads,begin,rows", [(3, 0, 250), (1, 130, 120), (2, 257, 65)])
+def test_portions_with_keys_in_two_parts(mask, size, heads, begin, rows):
+    from mini_llm_runtime_amd.kernels import Kernels
+    k = Kernels(BF16)
+    g = torch.Generator().manual_seed(heads + begin + size)
+    total = begin + rows
+    plain, turned, values = rounded(g, total, heads, 128, scale=0.4), rounded(g, total, 64, scale=0.4), rounded(g, total, heads, 128)
+    q = rounded(g, rows + 3, heads, 192, scale=0.4)            # (the portion stands behind three other rows)
+    sink = torch.randn(heads, generator=g)
+    positions = torch.cat([torch.zeros(3, dtype=torch.long), torch.arange(begin, total)])
+    want = attended(q[3:], torch.cat([plain, turned[:, None].expand(total, heads, 64)], 2), values, positions[3:], mask, size, 0, sink, 0.2, None)
+    first = 0 if mask is None else max(0, begin - size + 1) if mask == "window" else begin // size * size
+    first = first // 64 * 64
+    on_gpu = q.cuda()
+    for columns in (64, 128):
+        out = torch.full((rows + 3, heads * 128), float("nan"), dtype=BF16, device="cuda")
+        k.portion_attention_split(on_gpu[:, :, :128], on_gpu[:, :, 128:], plain[first:].reshape(-1, heads * 128).cuda(), turned[first:].cuda(),
+                                  values[first:].reshape(-1, heads * 128).cuda(), torch.zeros(rows + 3, dtype=torch.int32, device="cuda"),
+                                  positions.int().cuda(), sink.cuda(), out, 3, rows, first, columns, heads, 0.2, mask, size)
+        assert torch.isnan(out[:3].float()).all()
+        torch.testing.assert_close(out[3:].double().cpu().view(want.shape), want, atol=1.5e-2, rtol=1e-2)
+
+
+@pytest.mark.parametrize("window", [70, 1000])
+def test_latent_portions_of_a_model(tmp_path, window, monkeypatch):
+    """A model whose latent attention has the sizes of that path, in every way of cutting: portions that make their keys (64
+    tokens and more, from the start and from the middle, beside single tokens and short portions), against the plain
+    implementation."""
+    from helpers import compare, make_requests, plain_logits, portions, run_steps, whole
+    from plain import pamunex_plain as P
+    from mini_llm_runtime_amd.config import config_from_dict
+    from mini_llm_runtime_amd.engine import Runner
+    from mini_llm_runtime_amd.kernels import Kernels
+    from mini_llm_runtime_amd.parts import DecoderModel
+    from mini_llm_runtime_amd.weights import write_random_model
+    latent = dict(type="latent_attention", mlp=None, mixer=dict(heads=2, dim=128, rot_dim=64, vdim=128, kv_rank=48, scale=192 ** -0.5,
+                                                                rot=dict(dims=64, base=10000.0), mask=dict(size=window)))
+    cfg = dict(architecture="Pamunex", vocab=97, width=64, norm=dict(eps=1e-5), logit_scale=1.0, layers=[latent, latent])
+    folder = str(tmp_path / "model")
+    write_random_model(folder, config_from_dict(cfg), seed=3, matrix_std=0.12, norm_std=0.2)
+    requests = make_requests(97, [150, 64, 201, 9], seed=2)
+    want = plain_logits(P.PlainPamunex(folder), requests)
+    part = lambda rid, lo, hi: dict(id=rid, tokens=requests[rid][lo:hi], want=list(range(hi - lo)))
+    beside = [dict(step=0, entries=[part("r0", 0, 70), part("r3", 0, 5)], end=[]),
+              dict(step=1, entries=[part("r3", 5, 6), part("r0", 70, 71), part("r2", 0, 130), part("r1", 0, 64)], end=["r1"]),
+              dict(step=2, entries=[part("r3", 6, 9), part("r2", 130, 201), part("r0", 71, 150)], end=["r0", "r2", "r3"])]
+    monkeypatch.setattr("mini_llm_runtime_amd.parts.sink_attention.PORTION_LEAST_KEYS", 0)
+    calls = []
+    original = Kernels.portion_attention_split
+    monkeypatch.setattr(Kernels, "portion_attention_split", lambda self, *a, **kw: calls.append(a) or original(self, *a, **kw))
+    model = DecoderModel.load(folder, BF16)
+    for cut in (whole(requests), portions(requests, (100, 65, 64, 7)), beside):
+        calls.clear()
+        runner = Runner(model, max_tokens=640, max_slots=4, max_length=256, max_batch_tokens=512, page_size=16)
+        compare(run_steps(runner, cut), want, "bfloat16")
+        assert calls, "no portion made its keys"
+        assert runner.workspace.unplanned_bytes() == 0
+    # a budget without room for the scratch memory of long portions: the runner is built all the same, and a portion too long
+    # for the room there is goes the other way
+    options = dict(max_tokens=4096, max_slots=2, max_length=4000, max_batch_tokens=256, page_size=16)
+    amply = Runner(model, device_budget_bytes=0, **options)
+    tight = Runner(model, device_budget_bytes=amply.memory_plan.to_allocate() - 1, **options)
+    assert tight.memory_plan.workspace < amply.memory_plan.workspace
+    for runner in (amply, tight):
+        calls.clear()
+        compare(run_steps(runner, whole(requests)), want, "bfloat16")
+        assert bool(calls) == (runner is amply) or runner.workspace.room("latent_out", BF16) >= 64 * (48 + 64 + 512)
