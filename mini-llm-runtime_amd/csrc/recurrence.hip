@@ -397,11 +397,17 @@ __global__ __launch_bounds__(64) void delta_rule_kernel(DeltaArgs a) {
 // and beta alone.  The first kernel (one workgroup per chunk and head, all side by side) leaves in scratch memory
 //     W = T (beta Khat) [DC, N],  Y = T (beta V) [DC, V],  B[t, s] = sum_i q_t[i] k_s[i] e^{c_t[i] - c_s[i]} (s <= t),
 //     Qhat[t] = q_t e^{c_t},  Kbar[s] = k_s e^{c_last - c_s},  G = e^{c_last};
-// the second (one workgroup per request, head and 16 or 32 value channels) walks a request's chunks in
-// their order with the state in LDS:  U = Y - W S0;  O = Qhat S0 + B U;  S <- diag(G) S0 + Kbar^T U.
+// the second (one workgroup per request, head and 16 value channels) walks a request's chunks in
+// their order with the state in registers:  U = Y - W S0;  O = Qhat S0 + B U;  S <- diag(G) S0 + Kbar^T U.
 // Every exponent is a difference c_t - c_s with s <= t or c_t itself, so nothing overflows however strong a decay
 // is.  The result differs from the token-by-token kernel's by 32-bit rounding.
+//
+// Both kernels multiply with v_mfma_f32_16x16x4_f32 (32-bit products and sums; lane = 16 b + c: A row c, B column c, k-slot
+// b; C column c, rows 4 b + i).  Product i of four takes the k {i, 4 + i, 8 + i, 12 + i}: A is four neighbouring k of a row,
+// and what a product leaves in C is the next one's B as it lies -- the state, 16 key channels a tile, and U never leave the
+// registers but to be added across wavefronts.
 #define DELTA_CHUNK 32
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 
 struct DeltaChunkArgs {
     DeltaArgs d;
@@ -409,37 +415,52 @@ struct DeltaChunkArgs {
     float* scratch;                                              // [chunks][heads][delta_chunk_floats(N, V)]
 };
 
+// W [DC][Np], Qhat [DC][Np], Kbar^T [Np][DC], Y [DC][V], B [DC][DC], G [Np]; Np: N up to a multiple of 16, zeros there
+__host__ __device__ inline int delta_padded(int N) { return (N + 15) / 16 * 16; }
 __host__ __device__ inline size_t delta_chunk_floats(int N, int V) {
-    return (size_t)DELTA_CHUNK * (3 * N + V + DELTA_CHUNK) + N;
+    return (size_t)DELTA_CHUNK * (3 * delta_padded(N) + V + DELTA_CHUNK) + delta_padded(N);
 }
 
+__device__ __forceinline__ floatx4 mma4(const floatx4& a, const floatx4& b, floatx4 c) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], c, 0, 0, 0);
+    return c;
+}
+
+// One workgroup a chunk and head.  The pairs (t, s) of one half of the chunk need an exponential a key channel each, so a
+// thread takes one pair (120 a half); between the halves e^{c_t - c_s} = e^{c_t - c_15} e^{c_15 - c_s}, neither above 1, and
+// the sums are a matrix product.  T = (I + A)^-1 by halves too: two triangles of 16 a lane column by column, and
+// -T22 A21 T11 between them.  A thread for each of 1024 pairs, half of them idle, T row by row over 32 rows, and the two
+// products with T one element a thread took 199 us for 2048 tokens of 16 heads of 128 x 128 channels; this one 98, of
+// which the exponentials are the most.
 __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(DeltaChunkArgs g) {
-    constexpr int C = DELTA_CHUNK, CS = DELTA_CHUNK + 1;
+    constexpr int C = DELTA_CHUNK, CS = DELTA_CHUNK + 4;
     const DeltaArgs& a = g.d;
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    const int N = a.N, V = a.V, NS = N + 1;
+    const int N = a.N, V = a.V, Np = delta_padded(N), NS = Np + 4;
     float* q_l = lds;                    // [C][NS]
     float* k_l = q_l + C * NS;
     float* c_l = k_l + C * NS;
     float* A_l = c_l + C * NS;           // [C][CS]
     float* B_l = A_l + C * CS;
     float* T_l = B_l + C * CS;
-    float* beta_l = T_l + C * CS;        // [C]
+    float* part_l = T_l + C * CS;        // [4][2][256]: the wavefronts' shares of the block between the halves
+    float* beta_l = part_l + 4 * 2 * 256;        // [C]
     const int chunk = blockIdx.x, head = blockIdx.y;
     const int r0 = g.chunk_first[chunk], n = g.chunk_count[chunk];
     const int qk_head = head / a.heads_per_group;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, b4 = (lane >> 4) * 4;
     float* base = g.scratch + ((size_t)chunk * a.heads + head) * delta_chunk_floats(N, V);
     float* W = base;
-    float* Qh = W + (size_t)C * N;
-    float* Kb = Qh + (size_t)C * N;
-    float* Y = Kb + (size_t)C * N;
+    float* Qh = W + (size_t)C * Np;
+    float* Kt = Qh + (size_t)C * Np;
+    float* Y = Kt + (size_t)C * Np;
     float* B = Y + (size_t)C * V;
     float* G = B + C * C;
-    for (int idx = tid; idx < C * N; idx += 256) {
-        const int t = idx / N, i = idx % N;
+    for (int idx = tid; idx < C * Np; idx += 256) {
+        const int t = idx / Np, i = idx % Np;
         float dq = 0.f, dk = 0.f, dc = 0.f;
-        if (t < n) {
+        if (t < n && i < N) {
             const size_t row = (size_t)(r0 + t);
             dq = to_float(a.q[row * a.q_stride + qk_head * N + i]);
             dk = to_float(a.k[row * a.k_stride + qk_head * N + i]);
@@ -447,6 +468,7 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(DeltaChunkArgs
         }
         q_l[t * NS + i] = dq; k_l[t * NS + i] = dk; c_l[t * NS + i] = dc;
     }
+    for (int p = tid; p < C * CS; p += 256) A_l[p] = B_l[p] = T_l[p] = 0.f;
     __syncthreads();
     for (int t = wave; t < C; t += 4) {                     // unit vectors, q scaled; beta
         float qq = 0.f, kk = 0.f;
@@ -463,199 +485,290 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(DeltaChunkArgs
         for (int i = lane; i < N; i += 64) { q_l[t * NS + i] *= fq; k_l[t * NS + i] *= fk; }
         if (lane == 0) beta_l[t] = t < n ? sigmoid_f(a.beta_raw[(size_t)(r0 + t) * a.beta_stride + head]) : 0.f;
     }
-    for (int i = tid; i < N; i += 256) {                    // c_t: the running sum of the log decays (rows past n add 0)
+    for (int i = tid; i < Np; i += 256) {                   // c_t: the running sum of the log decays (rows past n add 0)
         float sum = 0.f;
+#pragma unroll
         for (int t = 0; t < C; ++t) { sum += c_l[t * NS + i]; c_l[t * NS + i] = sum; }
     }
     __syncthreads();
-    for (int p = tid; p < C * C; p += 256) {
-        const int t = p / C, s = p % C;
-        float sa = 0.f, sb = 0.f;
-        if (s <= t && t < n) {
-            const float* ct = c_l + t * NS; const float* cs = c_l + s * NS;
-            const float* kt = k_l + t * NS; const float* ks = k_l + s * NS; const float* qt = q_l + t * NS;
-            for (int i = 0; i < N; ++i) {
-                const float x = ks[i] * expf(ct[i] - cs[i]);
-                sa += kt[i] * x;
-                sb += qt[i] * x;
+    auto four = [](const float* p) { return *reinterpret_cast<const floatx4*>(p); };
+    if (tid < 240) {                                        // the pairs s < t of both halves
+        const int p = tid % 120, h0 = tid / 120 * 16;
+        int t = (int)((1.0f + sqrtf(1.0f + 8.0f * (float)p)) * 0.5f);
+        t -= t * (t - 1) / 2 > p ? 1 : 0;
+        t += t * (t + 1) / 2 <= p ? 1 : 0;
+        const int s = p - t * (t - 1) / 2;
+        const float* ct = c_l + (h0 + t) * NS; const float* cs = c_l + (h0 + s) * NS;
+        const float* kt = k_l + (h0 + t) * NS; const float* ks = k_l + (h0 + s) * NS; const float* qt = q_l + (h0 + t) * NS;
+        floatx4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < Np; i += 4) {
+            const floatx4 d = four(ct + i) - four(cs + i), k4 = four(ks + i), kt4 = four(kt + i), qt4 = four(qt + i);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float x = k4[e] * expf(d[e]);
+                sa[e] += kt4[e] * x;
+                sb[e] += qt4[e] * x;
             }
         }
-        A_l[t * CS + s] = s < t ? beta_l[t] * sa : 0.f;
-        B_l[t * CS + s] = sb;
-        B[t * C + s] = sb;
-    }
-    for (int idx = tid; idx < C * N; idx += 256) {          // Qhat, Kbar, G (they read what the loop above reads)
-        const int t = idx / N, i = idx % N;
-        const float ct = c_l[t * NS + i], last = c_l[(C - 1) * NS + i];
-        Qh[idx] = q_l[t * NS + i] * expf(ct);
-        Kb[idx] = k_l[t * NS + i] * expf(last - ct);
-        if (t == 0) G[i] = expf(last);
-    }
-    __syncthreads();
-    if (tid < C) {                                          // T = (I + A)^-1, a column a lane, row after row
-        const int j = tid;
-        for (int t = 0; t < C; ++t) {
-            float x = t == j ? 1.f : 0.f;
-            for (int s = 0; s < t; ++s) x -= A_l[t * CS + s] * T_l[s * CS + j];
-            T_l[t * CS + j] = x;
+        A_l[(h0 + t) * CS + h0 + s] = beta_l[h0 + t] * ((sa[0] + sa[1]) + (sa[2] + sa[3]));
+        B_l[(h0 + t) * CS + h0 + s] = (sb[0] + sb[1]) + (sb[2] + sb[3]);
+    } else {                                                // the pairs s = t, of B
+        for (int t = tid - 240; t < C; t += 16) {
+            floatx4 sb = {0.f, 0.f, 0.f, 0.f};
+            for (int i = 0; i < Np; i += 4) sb += four(q_l + t * NS + i) * four(k_l + t * NS + i);
+            B_l[t * CS + t] = (sb[0] + sb[1]) + (sb[2] + sb[3]);
         }
     }
-    for (int idx = tid; idx < C * N; idx += 256) {          // beta Khat in q's place
-        const int t = idx / N, i = idx % N;
-        q_l[t * NS + i] = beta_l[t] * k_l[t * NS + i] * expf(c_l[t * NS + i]);
+    {                                                       // rows 16 .. 31 against columns 0 .. 15: a share of the channels a wavefront
+        floatx4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
+        for (int i0 = wave * 16; i0 < Np; i0 += 64) {
+            const int i = i0 + b4;
+            const floatx4 mid = four(c_l + 15 * NS + i), dt = four(c_l + (16 + c) * NS + i) - mid, ds = mid - four(c_l + c * NS + i);
+            floatx4 kt = four(k_l + (16 + c) * NS + i), qt = four(q_l + (16 + c) * NS + i), ks = four(k_l + c * NS + i);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float f = expf(dt[e]);
+                kt[e] *= f;
+                qt[e] *= f;
+                ks[e] *= expf(ds[e]);
+            }
+            sa = mma4(kt, ks, sa);
+            sb = mma4(qt, ks, sb);
+        }
+        *reinterpret_cast<floatx4*>(part_l + (wave * 2) * 256 + lane * 4) = sa;
+        *reinterpret_cast<floatx4*>(part_l + (wave * 2 + 1) * 256 + lane * 4) = sb;
+    }
+    for (int idx = tid; idx < C * Np; idx += 256) {         // Qhat and G (they read what the loops above read)
+        const int t = idx / Np, i = idx % Np;
+        Qh[idx] = q_l[t * NS + i] * expf(c_l[t * NS + i]);
+        if (t == 0) G[i] = expf(c_l[(C - 1) * NS + i]);
+    }
+    for (int idx = tid; idx < C * Np; idx += 256) {         // Kbar, a channel's tokens side by side
+        const int i = idx / C, t = idx % C;
+        Kt[idx] = k_l[t * NS + i] * expf(c_l[(C - 1) * NS + i] - c_l[t * NS + i]);
     }
     __syncthreads();
-    for (int idx = tid; idx < C * N; idx += 256) {
-        const int t = idx / N, i = idx % N;
-        float acc = 0.f;
-        for (int s = 0; s <= t; ++s) acc += T_l[t * CS + s] * q_l[s * NS + i];
-        W[idx] = acc;
+    {
+        const int e = tid & 3, l = tid >> 2, t = 16 + (l >> 4) * 4 + e, s = l & 15;      // element e of lane l
+        float sa = 0.f, sb = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            sa += part_l[(w * 2) * 256 + tid];
+            sb += part_l[(w * 2 + 1) * 256 + tid];
+        }
+        A_l[t * CS + s] = beta_l[t] * sa;
+        B_l[t * CS + s] = sb;
     }
-    for (int idx = tid; idx < C * V; idx += 256) {
-        const int t = idx / V, j = idx % V;
-        float acc = 0.f;
-        const int last = min(t, n - 1);
-        for (int s = 0; s <= last; ++s)
-            acc += T_l[t * CS + s] * beta_l[s] * to_float(a.v[(size_t)(r0 + s) * a.v_stride + head * V + j]);
-        Y[idx] = acc;
+    for (int idx = tid; idx < C * Np; idx += 256) {         // beta Khat in q's place
+        const int t = idx / Np, i = idx % Np;
+        q_l[t * NS + i] = beta_l[t] * k_l[t * NS + i] * expf(c_l[t * NS + i]);
+    }
+    if (tid < 32) {                                         // the inverses of the two triangles, a column a lane, row after row
+        const int j = tid & 15, h0 = tid & 16;
+        float x[16];
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            x[t] = t == j ? 1.f : 0.f;
+#pragma unroll
+            for (int s = 0; s < t; ++s) x[t] -= A_l[(h0 + t) * CS + h0 + s] * x[s];
+        }
+#pragma unroll
+        for (int t = 0; t < 16; ++t) T_l[(h0 + t) * CS + h0 + j] = x[t];
+    }
+    __syncthreads();
+    if (wave == 0) {                                        // T21 = -T22 (A21 T11)
+        floatx4 t11, p = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) t11[i] = T_l[(b4 + i) * CS + c];
+        p = mma4(four(A_l + (16 + c) * CS + b4), t11, p);
+        p = mma4(four(T_l + (16 + c) * CS + 16 + b4), p, floatx4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+        for (int i = 0; i < 4; ++i) T_l[(16 + b4 + i) * CS + c] = -p[i];
+    }
+    for (int p = tid; p < C * C; p += 256) B[p] = B_l[(p / C) * CS + p % C];
+    __syncthreads();
+    floatx4 tf[2][2];                                       // T's rows 16 rt + c, columns 16 st + b4 ..
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+        for (int st = 0; st < 2; ++st) tf[rt][st] = four(T_l + (16 * rt + c) * CS + 16 * st + b4);
+    auto product = [&](const floatx4 (&x)[2], float* dst, int width, int col, bool ok) {      // T x, 16 columns
+        floatx4 top = mma4(tf[0][0], x[0], floatx4{0.f, 0.f, 0.f, 0.f});
+        floatx4 low = mma4(tf[1][1], x[1], mma4(tf[1][0], x[0], floatx4{0.f, 0.f, 0.f, 0.f}));
+        if (!ok) return;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            dst[(size_t)(b4 + i) * width + col] = top[i];
+            dst[(size_t)(16 + b4 + i) * width + col] = low[i];
+        }
+    };
+    for (int i0 = wave * 16; i0 < Np; i0 += 64) {
+        floatx4 x[2];
+#pragma unroll
+        for (int st = 0; st < 2; ++st)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[st][i] = q_l[(16 * st + b4 + i) * NS + i0 + c];
+        product(x, W, Np, i0 + c, true);
+    }
+    for (int j0 = wave * 16; j0 < V; j0 += 64) {
+        const int j = j0 + c;
+        floatx4 x[2];
+#pragma unroll
+        for (int st = 0; st < 2; ++st)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int t = 16 * st + b4 + i;
+                x[st][i] = t < n && j < V ? beta_l[t] * to_float(a.v[(size_t)(r0 + t) * a.v_stride + head * V + j]) : 0.f;
+            }
+        product(x, Y, V, j, j < V);
     }
 }
 
-template <int VEC> struct alignas(4 * VEC) DeltaVec { float v[VEC]; };
-
-// VEC value channels a thread, 8 * VEC a workgroup: the narrower form fills the GPU when heads and value channels are few.
-template <int VEC>
-__global__ __launch_bounds__(256) void delta_chunk_scan_kernel(DeltaChunkArgs g) {
-    constexpr int C = DELTA_CHUNK, CS = DELTA_CHUNK + 1, COLS = 8 * VEC;
-    constexpr int PER = DELTA_CHUNK * 128 / 256;           // elements of a [C][N] tile a thread moves, N <= 128
-    constexpr int PER_B = DELTA_CHUNK * DELTA_CHUNK / 256;
-    typedef DeltaVec<VEC> vec_t;
+// One workgroup per request, head and 16 value channels; a wavefront owns the key channels of the tiles wave, wave + 4 (of 16)
+// and keeps their part of the state in registers.  A chunk: every wavefront's share of W S0 goes through LDS (the one barrier
+// a chunk), all add them up to U, and update their part of the state; the shares of O meet in LDS likewise and are added a
+// chunk later.  A chunk's operands are on their way while the chunk before is worked on.  Scalar sums out of tiles staged in
+// LDS took 598 us for 2048 tokens of 16 heads of 128 x 128 channels (64 chunks, 128 workgroups); this one 153, 2.4 us a
+// chunk, of which 0.7 are its 52 matrix instructions a wavefront and the rest the chain between them: it is bound by the
+// walk's length, not by memory (with one chunk of operands under way instead of two 166 us).
+template <int NT>
+__global__ __launch_bounds__(256, 1) void delta_chunk_scan_kernel(DeltaChunkArgs g) {
+    constexpr int C = DELTA_CHUNK;
     const DeltaArgs& a = g.d;
-    extern __shared__ __attribute__((aligned(16))) float lds[];
-    const int N = a.N, V = a.V, NS = N + 1;
-    float* S_l = lds;                    // [N][COLS]
-    float* U_l = S_l + N * COLS;         // [C][COLS]
-    float* W_l = U_l + C * COLS;         // [C][NS]: W, then Kbar
-    float* Q_l = W_l + C * NS;           // [C][NS]: Qhat
-    float* B_l = Q_l + C * NS;           // [C][CS]
-    float* G_l = B_l + C * CS;           // [N]
-    const int seg = blockIdx.x, head = blockIdx.y, col0 = blockIdx.z * COLS;
+    __shared__ __attribute__((aligned(16))) float u_l[2][4][2][256], o_l[2][4][2][256];      // [buffer][wavefront][row tile][lane, element]
+    const int N = a.N, V = a.V, Np = delta_padded(N);
+    const int seg = blockIdx.x, head = blockIdx.y;
     const int r0 = a.seg_first[seg], n = a.seg_count[seg];
     const int slot = a.slots[r0];
-    const int tid = threadIdx.x, t = tid >> 3, jq = (tid & 7) * VEC;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, b4 = (lane >> 4) * 4;
+    const int col = blockIdx.z * 16 + c;
+    const bool col_ok = col < V;
     int chunk0 = 0;
     for (int s = 0; s < seg; ++s) chunk0 += (a.seg_count[s] + C - 1) / C;
-    const size_t per = delta_chunk_floats(N, V);
+    const size_t step = (size_t)a.heads * delta_chunk_floats(N, V);
     const size_t state_at = (size_t)slot * a.state_stride + (size_t)head * N * V;
-    const int tile = C * N;
-    int at_lds[PER];                                        // where this thread's tile elements go in LDS
+    const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+    floatx4 S[NT];
+    bool mine[NT];
 #pragma unroll
-    for (int r = 0; r < PER; ++r) {
-        const int idx = tid + 256 * r;
-        at_lds[r] = (idx / N) * NS + idx % N;
-    }
-    for (int idx = tid; idx < N * COLS; idx += 256) {
-        const int i = idx / COLS, c = col0 + idx % COLS;
-        S_l[idx] = c < V ? a.live[state_at + (size_t)i * V + c] : 0.f;
-    }
-    // a chunk's W, Qhat, B, G and Y are on their way into registers while the chunk before is worked on; Kbar while
-    // the chunk's own first products run
-    float w_next[PER], q_next[PER], k_next[PER], b_next[PER_B], y_next[VEC], g_next;
-    const float* base = g.scratch + ((size_t)chunk0 * a.heads + head) * per;
-    auto fetch = [&](const float* from) {
+    for (int j = 0; j < NT; ++j) {
+        const int n0 = (wave + 4 * j) * 16;
+        mine[j] = n0 < Np;
 #pragma unroll
-        for (int r = 0; r < PER; ++r) {
-            const int idx = tid + 256 * r;
-            w_next[r] = idx < tile ? from[idx] : 0.f;
-            q_next[r] = idx < tile ? from[tile + idx] : 0.f;
+        for (int i = 0; i < 4; ++i) {
+            const int ch = n0 + b4 + i;
+            S[j][i] = ch < N && col_ok ? a.live[state_at + (size_t)ch * V + col] : 0.f;
         }
-        const float* Y = from + 3 * (size_t)tile;
-        const float* B = Y + (size_t)C * V;
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) y_next[e] = col0 + jq + e < V ? Y[(size_t)t * V + col0 + jq + e] : 0.f;
-#pragma unroll
-        for (int r = 0; r < PER_B; ++r) b_next[r] = B[tid + 256 * r];
-        g_next = tid < N ? B[C * C + tid] : 0.f;
+    }
+    struct Chunk {
+        floatx4 w[2][NT], q[2][NT], k[NT][2], gate[NT], b, y[2];
     };
-    fetch(base);
-    for (int c0 = 0; c0 < n; c0 += C) {
-        const int nt = min(C, n - c0);
-        const float* Kb = base + 2 * (size_t)tile;
-        __syncthreads();                                    // the state is whole, the tiles of the chunk before are read
+    const int b_row = wave & 1, b_col = wave >> 1;          // this wavefront's quarter of B (the one above the diagonal is zero)
+    auto fetch = [&](const float* from, Chunk& x) {
+        const float* Qh = from + (size_t)C * Np;
+        const float* Kt = Qh + (size_t)C * Np;
+        const float* Y = Kt + (size_t)C * Np;
+        const float* B = Y + (size_t)C * V;
+        const float* G = B + C * C;
 #pragma unroll
-        for (int r = 0; r < PER; ++r)
-            if (tid + 256 * r < tile) { W_l[at_lds[r]] = w_next[r]; Q_l[at_lds[r]] = q_next[r]; }
+        for (int j = 0; j < NT; ++j) {
+            const int n0 = mine[j] ? (wave + 4 * j) * 16 : 0;                  // (for a tile that is not there: its state stays zero)
 #pragma unroll
-        for (int r = 0; r < PER_B; ++r) B_l[((tid + 256 * r) / C) * CS + (tid + 256 * r) % C] = b_next[r];
-        if (tid < N) G_l[tid] = g_next;
-        float u[VEC], o[VEC];
+            for (int rt = 0; rt < 2; ++rt) {
+                x.w[rt][j] = *reinterpret_cast<const floatx4*>(from + (16 * rt + c) * Np + n0 + b4);
+                x.q[rt][j] = *reinterpret_cast<const floatx4*>(Qh + (16 * rt + c) * Np + n0 + b4);
+                x.k[j][rt] = *reinterpret_cast<const floatx4*>(Kt + (n0 + c) * C + 16 * rt + b4);
+            }
+            x.gate[j] = *reinterpret_cast<const floatx4*>(G + n0 + b4);
+        }
+        x.b = *reinterpret_cast<const floatx4*>(B + (16 * b_row + c) * C + 16 * b_col + b4);
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) { u[e] = y_next[e]; o[e] = 0.f; }
+        for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
-        for (int r = 0; r < PER; ++r) k_next[r] = tid + 256 * r < tile ? Kb[tid + 256 * r] : 0.f;
+            for (int i = 0; i < 4; ++i) x.y[rt][i] = Y[(size_t)(16 * rt + b4 + i) * V + (col_ok ? col : 0)];
+    };
+    auto put_out = [&](int buf, int c0) {                   // the shares of a chunk's O, added up: two of a lane's elements a thread
+        const int rt = wave >> 1, e0 = (wave & 1) * 2;
+#pragma unroll
+        for (int e = e0; e < e0 + 2; ++e) {
+            const int t = 16 * rt + b4 + e;
+            const float o = ((o_l[buf][0][rt][lane * 4 + e] + o_l[buf][1][rt][lane * 4 + e]) + o_l[buf][2][rt][lane * 4 + e]) +
+                            o_l[buf][3][rt][lane * 4 + e];
+            if (c0 + t < n && col_ok) a.out[(size_t)(r0 + c0 + t) * ((size_t)a.heads * V) + head * V + col] = o;
+        }
+    };
+    const float* base = g.scratch + (size_t)chunk0 * step + (size_t)head * delta_chunk_floats(N, V);
+    Chunk ring[3];                                          // the chunk at work and the two behind it
+    const float* last = base + (size_t)((n - 1) / C) * step;
+    fetch(base, ring[0]);
+    fetch(base + step <= last ? base + step : last, ring[1]);
+    auto turn = [&](const Chunk& now, Chunk& ahead, int c0, int buf) {
+        fetch(base + 2 * step <= last ? base + 2 * step : last, ahead);        // (never behind a branch)
+        base += step;
+        floatx4 part[2] = {zero, zero}, o[2] = {zero, zero};
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int rt = 0; rt < 2; ++rt) part[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.w[rt][j][i], S[j][i], part[rt], 0, 0, 0);
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt) *reinterpret_cast<floatx4*>(&u_l[buf][wave][rt][lane * 4]) = part[rt];
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int rt = 0; rt < 2; ++rt) o[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.q[rt][j][i], S[j][i], o[rt], 0, 0, 0);
         __syncthreads();
-        {
-            const float* wt = W_l + t * NS;
-            const float* qt = Q_l + t * NS;
-#pragma unroll 8
-            for (int i = 0; i < N; ++i) {
-                const float w = wt[i], qv = qt[i];
-                const vec_t s4 = *reinterpret_cast<const vec_t*>(S_l + i * COLS + jq);
+        floatx4 u[2];
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) { u[e] -= w * s4.v[e]; o[e] += qv * s4.v[e]; }
-            }
+        for (int rt = 0; rt < 2; ++rt) {
+            floatx4 sum = *reinterpret_cast<const floatx4*>(&u_l[buf][0][rt][lane * 4]);
+#pragma unroll
+            for (int w = 1; w < 4; ++w) sum += *reinterpret_cast<const floatx4*>(&u_l[buf][w][rt][lane * 4]);
+            u[rt] = now.y[rt] - sum;
         }
-        {
-            vec_t u4;
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) u4.v[e] = u[e];
-            *reinterpret_cast<vec_t*>(U_l + t * COLS + jq) = u4;
+        for (int j = 0; j < NT; ++j) S[j] *= now.gate[j];
+#pragma unroll
+        for (int st = 0; st < 2; ++st)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.k[j][st][i], u[st][i], S[j], 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+            if (!mine[j]) S[j] = zero;                      // (the same in every lane)
+        if (b_row >= b_col) {
+            if (b_row == 0) o[0] = mma4(now.b, u[0], o[0]);
+            else o[1] = mma4(now.b, b_col == 0 ? u[0] : u[1], o[1]);
         }
-        __syncthreads();                                    // U is whole; W's tile has been read
+        if (c0 > 0) put_out(buf ^ 1, c0 - C);               // (written before the barrier above)
 #pragma unroll
-        for (int r = 0; r < PER; ++r)
-            if (tid + 256 * r < tile) W_l[at_lds[r]] = k_next[r];
-        if (c0 + C < n) {
-            base += (size_t)a.heads * per;
-            fetch(base);
-        }
-        {
-            const float* bt = B_l + t * CS;
-#pragma unroll 4
-            for (int s = 0; s <= t; ++s) {
-                const float w = bt[s];
-                const vec_t u4 = *reinterpret_cast<const vec_t*>(U_l + s * COLS + jq);
-#pragma unroll
-                for (int e = 0; e < VEC; ++e) o[e] += w * u4.v[e];
-            }
-        }
-        if (t < nt) {
-#pragma unroll
-            for (int e = 0; e < VEC; ++e)
-                if (col0 + jq + e < V) a.out[(size_t)(r0 + c0 + t) * ((size_t)a.heads * V) + head * V + col0 + jq + e] = o[e];
-        }
-        __syncthreads();                                    // Kbar is in W's place
-        for (int i = t; i < N; i += C) {                   // (a thread's own elements of S: no other thread reads them now)
-            vec_t s4 = *reinterpret_cast<const vec_t*>(S_l + i * COLS + jq);
-            const float gi = G_l[i];
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) s4.v[e] *= gi;
-#pragma unroll 8
-            for (int s = 0; s < C; ++s) {
-                const float w = W_l[s * NS + i];
-                const vec_t u4 = *reinterpret_cast<const vec_t*>(U_l + s * COLS + jq);
-#pragma unroll
-                for (int e = 0; e < VEC; ++e) s4.v[e] += w * u4.v[e];
-            }
-            *reinterpret_cast<vec_t*>(S_l + i * COLS + jq) = s4;
-        }
+        for (int rt = 0; rt < 2; ++rt) *reinterpret_cast<floatx4*>(&o_l[buf][wave][rt][lane * 4]) = o[rt];
+    };
+    int buf = 0;
+    for (int c0 = 0; c0 < n; c0 += 3 * C) {
+        turn(ring[0], ring[2], c0, buf);
+        buf ^= 1;
+        if (c0 + C >= n) break;
+        turn(ring[1], ring[0], c0 + C, buf);
+        buf ^= 1;
+        if (c0 + 2 * C >= n) break;
+        turn(ring[2], ring[1], c0 + 2 * C, buf);
+        buf ^= 1;
     }
     __syncthreads();
-    if (a.write_state)
-        for (int idx = tid; idx < N * COLS; idx += 256) {
-            const int i = idx / COLS, c = col0 + idx % COLS;
-            if (c < V) a.stage[state_at + (size_t)i * V + c] = S_l[idx];
-        }
+    put_out(buf ^ 1, (n - 1) / C * C);
+    if (a.write_state && col_ok)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int ch = (wave + 4 * j) * 16 + b4 + i;
+                if (ch < N) a.stage[state_at + (size_t)ch * V + col] = S[j][i];
+            }
 }
 
 template <int NR, int PARTS>
@@ -803,18 +916,18 @@ int mlr_delta_rule_chunked(const void* q, long q_stride, const void* k, long k_s
                       beta_stride, out, live, stage, state_stride, seg_first, seg_count, slots, heads, heads_per_group, n_keys,
                       n_values, write_state, unit_norm, q_scale, unit_eps, decay_per_head},
                      chunk_first, chunk_count, scratch};
-    const int C = DELTA_CHUNK, NS = n_keys + 1;
-    const size_t lds1 = sizeof(float) * ((size_t)3 * C * NS + (size_t)3 * C * (C + 1) + C);
-    delta_chunk_prepare_kernel<<<dim3(chunks, heads), 256, lds1, stream>>>(g);
+    if ((reinterpret_cast<uintptr_t>(scratch) & 15) != 0) return -1;
+    const int C = DELTA_CHUNK, Np = delta_padded(n_keys);
+    const size_t lds = sizeof(float) * ((size_t)3 * C * (Np + 4) + (size_t)3 * C * (C + 4) + 4 * 2 * 256 + C);
+    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_chunk_prepare_kernel),
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
+    if (allowed != hipSuccess) return (int)allowed;
+    delta_chunk_prepare_kernel<<<dim3(chunks, heads), 256, lds, stream>>>(g);
     int err = (int)hipGetLastError();
     if (err != 0) return err;
-    // 32 value channels a workgroup where that fills the GPU, else 16
-    const bool wide = (long)segments * heads * ((n_values + 31) / 32) >= 256;
-    const int cols = wide ? 32 : 16;
-    const size_t lds2 = sizeof(float) * ((size_t)n_keys * cols + (size_t)C * cols + (size_t)2 * C * NS + (size_t)C * (C + 1) + n_keys);
-    const dim3 grid(segments, heads, (n_values + cols - 1) / cols);
-    if (wide) delta_chunk_scan_kernel<4><<<grid, 256, lds2, stream>>>(g);
-    else delta_chunk_scan_kernel<2><<<grid, 256, lds2, stream>>>(g);
+    const dim3 grid(segments, heads, (n_values + 15) / 16);
+    if (Np <= 64) delta_chunk_scan_kernel<1><<<grid, 256, 0, stream>>>(g);
+    else delta_chunk_scan_kernel<2><<<grid, 256, 0, stream>>>(g);
     return (int)hipGetLastError();
 }
 
