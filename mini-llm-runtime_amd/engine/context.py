@@ -104,6 +104,14 @@ class Uploader:
         self._busy = True
 
 
+# Single tokens that fill the GPU without a split, one workgroup a token and kv head: the longest context of the batch would
+# keep its workgroup walking when the others are done, so no workgroup walks more than this many keys.  Measured with 64
+# requests of 129 to 3001 tokens: a step of the 0.6B sizes 3.69 ms instead of 4.25 (ranges of 1024: 3.79), of four layers of the
+# 8B sizes 1.30 instead of 1.41; with 64 requests of 3900 tokens each, where a split only adds partial results, 6.90 instead of
+# 6.87 and 1.71 instead of 1.69.
+LONG_RANGE = 2048
+
+
 class StepContext:
     """One step's view for the parts: the tokens with their positions and slots (device int32
     vectors of equal length), the segments they form (host), the cache, the kernels and the
@@ -191,7 +199,7 @@ class StepContext:
         forced = longest is not None and self.max_context > longest
         if rows > self.split_max_tokens and not forced:
             return 0, 1, None
-        return self._split(max(1, rows * kv_heads), self.target_workgroups, batch_rows, q_heads, head_dim, longest)
+        return self._split(max(1, rows * kv_heads), self.target_workgroups, batch_rows, q_heads, head_dim, longest, LONG_RANGE)
 
     def group_split(self, groups, batch_rows, kv_heads, q_heads, head_dim, longest=None):
         """As `attention_split` for `groups` groups of many tokens each (prompt portions), which give
@@ -228,8 +236,8 @@ class StepContext:
             keys *= 2
         return -(-max_length // keys)
 
-    def _split(self, units, enough, batch_rows, q_heads, head_dim, longest=None):
-        """`units` workgroups without a split; no split when they are `enough`.  The partial results never take
+    def _split(self, units, enough, batch_rows, q_heads, head_dim, longest=None, widest=None):
+        """`units` workgroups without a split; no split when they are `enough`, but for contexts beyond `widest` keys.  The partial results never take
         more than `partial_budget` floats (when one is set: the runner's memory plan): key ranges are doubled
         until they fit, which a forced split allows up to `longest`."""
         base = self.split_keys
@@ -243,7 +251,12 @@ class StepContext:
             while keys > base and keys > longest:
                 keys //= 2
         elif units >= enough:
-            return 0, 1, None
+            if widest is None or self.max_context <= widest:
+                return 0, 1, None
+            while keys < widest:
+                keys *= 2
+            while keys > base and keys > widest:
+                keys //= 2
         budget = self.partial_budget
         numel = lambda k: self.kernels.attention_partial_numel(batch_rows, q_heads, head_dim, -(-self.max_context // k))
         while budget is not None and numel(keys) > budget and (not forced or keys * 2 <= longest):

@@ -44,6 +44,11 @@ def test_small_batches_over_long_contexts_are_split_and_short_ones_not():
     assert splits > 1 and keys * splits >= 4096
     assert context(200).attention_split(1, 1, 8, 16, 128, longest=65504)[1] == 1
     assert context(4096, split_keys=0).attention_split(1, 1, 8, 16, 128, longest=65504)[1] == 1
+    # workgroups enough without a split: none walks more than 2048 keys, and shorter contexts stay whole
+    assert context(2048).attention_split(64, 64, 8, 16, 128, longest=65504)[1] == 1
+    assert context(2049).attention_split(64, 64, 8, 16, 128, longest=65504)[:2] == (2048, 2)
+    assert context(8192).attention_split(64, 64, 8, 16, 128, longest=65504)[:2] == (2048, 4)
+    assert context(8192, split_keys=4096).attention_split(64, 64, 8, 16, 128, longest=65504)[:2] == (4096, 2)
 
 
 def attention_part(head_dim=128):
