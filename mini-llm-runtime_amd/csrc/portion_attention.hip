@@ -345,13 +345,17 @@ __global__ __launch_bounds__(256) void latent_rows_kernel(const __bf16* __restri
                                                           int max_blocks, const int32_t* __restrict__ slots, int m, int page_size,
                                                           int key0, int keys, int rank, int rot, __bf16* __restrict__ latent,
                                                           __bf16* __restrict__ shared) {
-    const int chunks = (rank + rot) / 8, at = blockIdx.x * 256 + threadIdx.x, i = at / chunks, d = at % chunks * 8;
+    // (a wavefront a row, which looks its page up once: 1777 rows of 576 values 3.7 us; 17 with a lookup for every 16 bytes)
+    const int i = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (i >= keys) return;
     const int block = (key0 + i) / page_size;
     const int page = block < max_blocks ? block_table[(size_t)slots[m] * max_blocks + block] : -1;
-    vec16 x = {{0, 0, 0, 0}};
-    if (page >= 0) x = *reinterpret_cast<const vec16*>(pages + ((long long)page * page_size + (key0 + i) % page_size) * row + d);
-    *reinterpret_cast<vec16*>(d < rank ? latent + (size_t)i * rank + d : shared + (size_t)i * rot + d - rank) = x;
+    const __bf16* src = pages + ((long long)max(page, 0) * page_size + (key0 + i) % page_size) * row;
+    for (int d = lane * 8; d < rank + rot; d += 512) {
+        vec16 x = *reinterpret_cast<const vec16*>(src + d);
+        if (page < 0) x = {{0, 0, 0, 0}};
+        *reinterpret_cast<vec16*>(d < rank ? latent + (size_t)i * rank + d : shared + (size_t)i * rot + d - rank) = x;
+    }
 }
 
 extern "C" {
@@ -389,8 +393,7 @@ int mlr_latent_rows(const void* pages, long row, const int32_t* block_table, int
                     int key0, int keys, int rank, int rot, void* latent, void* shared, hipStream_t stream) {
     if (keys <= 0) return 0;
     if (rank % 8 != 0 || rot % 8 != 0 || row % 8 != 0 || key0 < 0) return -1;
-    const long total = (long)keys * ((rank + rot) / 8);
-    latent_rows_kernel<<<(unsigned)((total + 255) / 256), 256, 0, stream>>>((const __bf16*)pages, row, block_table, max_blocks, slots, m, page_size,
+    latent_rows_kernel<<<(unsigned)((keys + 3) / 4), 256, 0, stream>>>((const __bf16*)pages, row, block_table, max_blocks, slots, m, page_size,
                                                                           key0, keys, rank, rot, (__bf16*)latent, (__bf16*)shared);
     return (int)hipGetLastError();
 }

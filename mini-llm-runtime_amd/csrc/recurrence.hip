@@ -69,6 +69,56 @@ __global__ __launch_bounds__(256) void causal_conv_kernel(ConvArgs a) {
     }
 }
 
+#if MLR_BF16
+// Many rows: eight channels a thread (16-byte accesses) and CONV_ROWS rows, for which its weights stay in registers.  Bound by
+// memory; one value a thread took 62 us for 2048 rows of 4096 channels, this 22.
+#define CONV_ROWS 4
+template <int TAPS>
+__global__ __launch_bounds__(256) void causal_conv_rows_kernel(ConvArgs a) {
+    const int c = (blockIdx.y * 256 + threadIdx.x) * 8;
+    if (c >= a.channels) return;
+    float w[8 * TAPS], b[8];
+#pragma unroll
+    for (int e = 0; e < 8 * TAPS; e += 4) *reinterpret_cast<float4*>(w + e) = *reinterpret_cast<const float4*>(a.w + (size_t)c * TAPS + e);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) b[e] = a.b ? a.b[c + e] : 0.f;
+    constexpr int before = TAPS - 1;
+    for (int r = blockIdx.x * CONV_ROWS; r < min(a.rows, ((int)blockIdx.x + 1) * CONV_ROWS); ++r) {
+        const int slot = a.slots[r], pos = a.positions[r];
+        int have = 0;
+        while (have < before && r - have - 1 >= 0 && a.slots[r - have - 1] == slot && a.positions[r - have - 1] == pos - have - 1) ++have;
+        const bool last = r + 1 >= a.rows || a.slots[r + 1] != slot || a.positions[r + 1] != pos + 1;
+        float in[TAPS][8];
+#pragma unroll
+        for (int d = 0; d < TAPS; ++d) {
+            if (d <= have) {
+                load_vec(a.x + (size_t)(r - d) * a.x_stride + c, in[d]);
+            } else {
+                const float* from = a.live + (size_t)slot * a.state_stride + (size_t)(before - d + have) * a.channels + c;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) in[d][e] = from[e];
+            }
+        }
+        float acc[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            acc[e] = b[e];
+#pragma unroll
+            for (int d = before; d >= 0; --d) acc[e] += w[e * TAPS + before - d] * in[d][e];
+            if (a.silu) acc[e] = acc[e] / (1.0f + expf(-acc[e]));
+        }
+        store_vec(a.out + (size_t)r * a.out_stride + c, acc);
+        if (last && a.write_state) {
+#pragma unroll
+            for (int d = 0; d < before; ++d)
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    a.stage[(size_t)slot * a.state_stride + (size_t)(before - 1 - d) * a.channels + c + e] = in[d][e];
+        }
+    }
+}
+#endif
+
 // ---- decays ---------------------------------------------------------------------------------------------
 // Gated linear attention: the logarithm of alpha = sigmoid(z + b)^(1 / tau), that is -softplus(-(z + b)) / tau.
 __global__ void gla_log_decay_kernel(const elem_t* __restrict__ z, const float* __restrict__ bias, float* __restrict__ out,
@@ -258,14 +308,16 @@ __global__ void piece_states_kernel(ScanArgs a, int pieces) {
 // ---- the delta rule ----------------------------------------------------------------------------------------
 // Decays of the key channels from a step size per channel: log g = -exp(A_log[head]) * softplus(z + bias), z the
 // 32-bit output of a low-rank pair of projections laid out [heads][N].
-__global__ void channel_log_decay_kernel(const float* __restrict__ z, const float* __restrict__ bias,
-                                         const float* __restrict__ a_log, float* __restrict__ out, size_t rows, int width,
-                                         int per_head) {
-    const size_t total = rows * width;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
-        const int c = (int)(i % width);
-        out[i] = -expf(a_log[c / per_head]) * softplus_f(z[i] + (bias ? bias[c] : 0.f));
-    }
+// A thread stays in its column and takes the rate and the bias once (`stride` is a multiple of the width): 19 us for 2048 rows of
+// 2048 channels, 23 where every element divides its place and takes its own rate.  The logarithms bound it.
+__global__ __launch_bounds__(256) void channel_log_decay_kernel(const float* __restrict__ z, const float* __restrict__ bias,
+                                                                const float* __restrict__ a_log, float* __restrict__ out, size_t total,
+                                                                size_t stride, int width, int per_head) {
+    const size_t first = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (first >= stride) return;
+    const int c = (int)(first % width);
+    const float rate = -expf(a_log[c / per_head]), add = bias ? bias[c] : 0.f;
+    for (size_t i = first; i < total; i += stride) out[i] = rate * softplus_f(z[i] + add);
 }
 
 struct DeltaArgs {
@@ -811,6 +863,14 @@ int mlr_causal_conv(const void* x, long x_stride, const float* w, const float* b
     if (taps < 1 || taps > CONV_MAX_TAPS) return -1;
     ConvArgs a{(const elem_t*)x, x_stride, w, b, (elem_t*)out, out_stride, live, stage, state_stride, slots, positions,
                rows, channels, taps, silu, write_state};
+#if MLR_BF16
+    const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    // (64 rows: below that the walk of CONV_ROWS rows is longer than what the wider accesses save)
+    if (rows >= 64 && taps == 4 && channels % 8 == 0 && x_stride % 8 == 0 && out_stride % 8 == 0 && aligned(x) && aligned(out) && aligned(w)) {
+        causal_conv_rows_kernel<4><<<dim3((rows + CONV_ROWS - 1) / CONV_ROWS, (channels / 8 + 255) / 256), 256, 0, stream>>>(a);
+        return (int)hipGetLastError();
+    }
+#endif
     causal_conv_kernel<<<dim3(rows, (channels + 255) / 256), 256, 0, stream>>>(a);
     return (int)hipGetLastError();
 }
@@ -858,8 +918,10 @@ int mlr_channel_log_decay(const float* z, const float* bias, const float* a_log,
                           hipStream_t stream) {
     if (rows <= 0) return 0;
     if (heads < 1 || n_keys < 1) return -1;
-    channel_log_decay_kernel<<<grid_for((size_t)rows * heads * n_keys, 256), 256, 0, stream>>>(z, bias, a_log, out, (size_t)rows,
-                                                                                            heads * n_keys, n_keys);
+    const size_t width = (size_t)heads * n_keys, total = (size_t)rows * width;
+    const size_t across = width >= 262144 ? 1 : 262144 / width;               // rows side by side: a quarter of a million threads
+    const size_t stride = (across < (size_t)rows ? across : (size_t)rows) * width;
+    channel_log_decay_kernel<<<(unsigned)((stride + 255) / 256), 256, 0, stream>>>(z, bias, a_log, out, total, stride, (int)width, n_keys);
     return (int)hipGetLastError();
 }
 
