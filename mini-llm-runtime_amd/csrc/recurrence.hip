@@ -347,15 +347,15 @@ __device__ __forceinline__ size_t decay_at(const DeltaArgs& a, size_t row, int h
 // exponentiated, beta = sigmoid(raw), k . q of every token.  A token then costs one pass over the lane's rows for
 // (g S)^T k and (g S)^T q, an exchange between the parts, and one pass for the write; the read-out after the write is
 // o = (g S)^T q + (k . q) u.  Every sum's order follows from the head's sizes alone.
-template <int NR, int PARTS>
+template <int NR, int PARTS, int TILE>
 __global__ __launch_bounds__(64) void delta_rule_kernel(DeltaArgs a) {
     constexpr int COLS = 64 / PARTS;
     constexpr int NPAD = NR * PARTS;
-    __shared__ __attribute__((aligned(16))) float g_lds[DELTA_TILE * NPAD];
-    __shared__ __attribute__((aligned(16))) float k_lds[DELTA_TILE * NPAD];
-    __shared__ __attribute__((aligned(16))) float q_lds[DELTA_TILE * NPAD];
-    __shared__ float v_lds[DELTA_TILE * COLS];
-    __shared__ float beta_lds[DELTA_TILE], kq_lds[DELTA_TILE];
+    __shared__ __attribute__((aligned(16))) float g_lds[TILE * NPAD];
+    __shared__ __attribute__((aligned(16))) float k_lds[TILE * NPAD];
+    __shared__ __attribute__((aligned(16))) float q_lds[TILE * NPAD];
+    __shared__ float v_lds[TILE * COLS];
+    __shared__ float beta_lds[TILE], kq_lds[TILE];
     const int seg = blockIdx.x, head = blockIdx.y, col0 = blockIdx.z * COLS;
     const int r0 = a.seg_first[seg], n = a.seg_count[seg];
     const int slot = a.slots[r0];
@@ -370,8 +370,8 @@ __global__ __launch_bounds__(64) void delta_rule_kernel(DeltaArgs a) {
         const int i = part * NR + r;
         S[r] = i < N && col < V ? a.live[state_at + (size_t)i * V + col] : 0.f;
     }
-    for (int t0 = 0; t0 < n; t0 += DELTA_TILE) {
-        const int nt = min(DELTA_TILE, n - t0);
+    for (int t0 = 0; t0 < n; t0 += TILE) {
+        const int nt = min(TILE, n - t0);
         __syncthreads();                                  // the tile before has been read
         for (int t = 0; t < nt; ++t) {
             const size_t row = (size_t)(r0 + t0 + t);
@@ -823,19 +823,26 @@ __global__ __launch_bounds__(256, 1) void delta_chunk_scan_kernel(DeltaChunkArgs
             }
 }
 
+// (requests of one token each: room for one in LDS, as in launch_scan; 48 requests of 32 heads of 128 x 128 69.8 us, now 54.6)
 template <int NR, int PARTS>
-static int launch_delta(const DeltaArgs& a, int segments, hipStream_t stream) {
+static int launch_delta(const DeltaArgs& a, int segments, bool singles, hipStream_t stream) {
     constexpr int COLS = 64 / PARTS;
-    delta_rule_kernel<NR, PARTS><<<dim3(segments, a.heads, (a.V + COLS - 1) / COLS), 64, 0, stream>>>(a);
+    const dim3 grid(segments, a.heads, (a.V + COLS - 1) / COLS);
+    if (singles) delta_rule_kernel<NR, PARTS, 1><<<grid, 64, 0, stream>>>(a);
+    else delta_rule_kernel<NR, PARTS, DELTA_TILE><<<grid, 64, 0, stream>>>(a);
     return (int)hipGetLastError();
 }
 
+// Requests of one token each (`singles`) stage one at a time: the step is bound by reading and writing the states, and with
+// the LDS of 16 tokens only three workgroups fit a compute unit (48 requests of 16 heads of 128 x 128: 25.2 us, with room
+// for one token 20.3; one request 8.6 and 5.9).
 template <int NR, int TILE>
-static int launch_scan(const ScanArgs& a, int segments, hipStream_t stream) {
-    const size_t lds = sizeof(float) * ((size_t)3 * TILE * NR * SCAN_PARTS + (size_t)TILE * SCAN_COLS * (1 + SCAN_PARTS));
+static int launch_scan(const ScanArgs& a, int segments, bool singles, hipStream_t stream) {
+    const size_t lds_token = sizeof(float) * ((size_t)3 * NR * SCAN_PARTS + (size_t)SCAN_COLS * (1 + SCAN_PARTS)), lds = TILE * lds_token;
     dim3 grid(segments, a.heads, (a.V + SCAN_COLS - 1) / SCAN_COLS);
     if (a.piece_state == nullptr) {
-        linear_recurrence_kernel<NR, TILE, 0><<<grid, 256, lds, stream>>>(a);
+        if (singles) linear_recurrence_kernel<NR, 1, 0><<<grid, 256, lds_token, stream>>>(a);
+        else linear_recurrence_kernel<NR, TILE, 0><<<grid, 256, lds, stream>>>(a);
         return (int)hipGetLastError();
     }
     linear_recurrence_kernel<NR, TILE, 1><<<grid, 256, lds, stream>>>(a);
@@ -894,7 +901,7 @@ int mlr_linear_recurrence(const void* q, long q_stride, const void* k, long k_st
                           const float* log_decay, long decay_stride, int decay_per_channel, const float* v_scale,
                           long v_scale_stride, const float* skip, float q_scale, float* out, const float* live, float* stage,
                           long state_stride, const int32_t* seg_first, const int32_t* seg_count, const int32_t* slots,
-                          int segments, int heads, int heads_per_group, int n_keys, int n_values, int write_state,
+                          int rows, int segments, int heads, int heads_per_group, int n_keys, int n_values, int write_state,
                           float* piece_state, float* piece_decay, int silu, const float* rope, const int32_t* positions,
                           int rot_dim, hipStream_t stream) {
     // piece_state, piece_decay given: `seg_first`/`seg_count` name pieces of requests (a request's pieces one after
@@ -908,10 +915,10 @@ int mlr_linear_recurrence(const void* q, long q_stride, const void* k, long k_st
                piece_decay};
     if ((piece_state == nullptr) != (piece_decay == nullptr)) return -2;
     const int nr = (n_keys + SCAN_PARTS - 1) / SCAN_PARTS;
-    if (nr <= 8) return launch_scan<8, 16>(a, segments, stream);
-    if (nr <= 16) return launch_scan<16, 16>(a, segments, stream);
-    if (nr <= 32) return launch_scan<32, 16>(a, segments, stream);
-    return launch_scan<64, 8>(a, segments, stream);
+    if (nr <= 8) return launch_scan<8, 16>(a, segments, rows == segments, stream);
+    if (nr <= 16) return launch_scan<16, 16>(a, segments, rows == segments, stream);
+    if (nr <= 32) return launch_scan<32, 16>(a, segments, rows == segments, stream);
+    return launch_scan<64, 8>(a, segments, rows == segments, stream);
 }
 
 int mlr_channel_log_decay(const float* z, const float* bias, const float* a_log, float* out, int rows, int heads, int n_keys,
@@ -930,8 +937,8 @@ int mlr_channel_log_decay(const float* z, const float* bias, const float* a_log,
 // one, up to 256 four; heads of few value channels use the narrower layouts too, so that their lanes are not idle.
 int mlr_delta_rule(const void* q, long q_stride, const void* k, long k_stride, const void* v, long v_stride,
                    const float* log_decay, const float* beta_raw, long beta_stride, float* out, const float* live, float* stage,
-                   long state_stride, const int32_t* seg_first, const int32_t* seg_count, const int32_t* slots, int segments,
-                   int heads, int heads_per_group, int n_keys, int n_values, int write_state, int unit_norm, float q_scale,
+                   long state_stride, const int32_t* seg_first, const int32_t* seg_count, const int32_t* slots, int rows,
+                   int segments, int heads, int heads_per_group, int n_keys, int n_values, int write_state, int unit_norm, float q_scale,
                    float unit_eps, int decay_per_head, hipStream_t stream) {
     if (segments <= 0) return 0;
     if (n_keys < 1 || n_keys > 256 || n_values < 1 || heads < 1 || heads > 65535 || heads_per_group < 1 ||
@@ -946,10 +953,10 @@ int mlr_delta_rule(const void* q, long q_stride, const void* k, long k_stride, c
     const int nr = (n_keys + parts - 1) / parts;
 #define MLR_DELTA(PARTS)                                                        \
     if (parts == PARTS) {                                                       \
-        if (nr <= 8) return launch_delta<8, PARTS>(a, segments, stream);        \
-        if (nr <= 16) return launch_delta<16, PARTS>(a, segments, stream);      \
-        if (nr <= 32) return launch_delta<32, PARTS>(a, segments, stream);      \
-        return launch_delta<64, PARTS>(a, segments, stream);                    \
+        if (nr <= 8) return launch_delta<8, PARTS>(a, segments, rows == segments, stream);        \
+        if (nr <= 16) return launch_delta<16, PARTS>(a, segments, rows == segments, stream);      \
+        if (nr <= 32) return launch_delta<32, PARTS>(a, segments, rows == segments, stream);      \
+        return launch_delta<64, PARTS>(a, segments, rows == segments, stream);                    \
     }
     MLR_DELTA(1)
     MLR_DELTA(2)

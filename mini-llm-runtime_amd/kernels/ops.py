@@ -992,7 +992,7 @@ class Kernels:
                ctypes.c_long(decay_stride), _c_int(1 if per_channel else 0), _p(v_scale),
                ctypes.c_long(heads if v_scale is not None else 0), _p(skip), _c_float(q_scale), _p(out),
                _ptr(live.data_ptr() + at), _ptr(stage.data_ptr() + at), ctypes.c_long(live.stride(0)), _p(seg_first),
-               _p(seg_count), _p(slots), _c_int(segments), _c_int(heads), _c_int(heads_per_group), _c_int(n_keys),
+               _p(seg_count), _p(slots), _c_int(rows), _c_int(segments), _c_int(heads), _c_int(heads_per_group), _c_int(n_keys),
                _c_int(n_values), _c_int(1 if write_state else 0), _p(piece_state), _p(piece_decay),
                _c_int(1 if activation == "silu" else 0), _p(rope), _p(positions if rope is not None else None), _c_int(rot),
                _stream()), "linear_recurrence")
@@ -1098,7 +1098,7 @@ class Kernels:
         _ok(self._lib("recurrence").mlr_delta_rule(
             _p(q), ctypes.c_long(qs), _p(k), ctypes.c_long(ks), _p(v), ctypes.c_long(vs), _p(log_decay), _p(beta_raw),
             ctypes.c_long(bs), _p(out), _ptr(live.data_ptr() + at), _ptr(stage.data_ptr() + at), ctypes.c_long(live.stride(0)),
-            _p(seg_first), _p(seg_count), _p(slots), _c_int(segments), _c_int(heads), _c_int(heads_per_group), _c_int(n_keys),
+            _p(seg_first), _p(seg_count), _p(slots), _c_int(rows), _c_int(segments), _c_int(heads), _c_int(heads_per_group), _c_int(n_keys),
             _c_int(n_values), _c_int(1 if write_state else 0), _c_int(1 if unit_norm else 0), _c_float(q_scale),
             _c_float(unit_eps), _c_int(1 if decay_per_head else 0), _stream()), "delta_rule")
 

@@ -675,3 +675,32 @@ def test_configurations_drawn_at_random(tmp_path, seed):
         if dtype_name == "float32":
             assert max_difference(results["whole"], results["portions"]) == 0.0, cfg
             assert max_difference(results["whole"], results["mixed"]) == 0.0, cfg
+
+
+@pytest.mark.parametrize("dtype_name", DTYPES)
+@pytest.mark.parametrize("keys,values", [(1, 3), (30, 64), (64, 70), (128, 128), (250, 17)])
+def test_requests_of_one_token_get_what_they_get_beside_longer_ones(dtype_name, keys, values):
+    """A step of single tokens keeps less in LDS; the arithmetic, and so every bit, is that of any other step."""
+    from mini_llm_runtime_amd.kernels import Kernels
+    dtype = DTYPES[dtype_name]
+    k = Kernels(dtype)
+    gen = torch.Generator("cuda").manual_seed(keys)
+    heads, singles, state = 3, 5, 3 * keys * values
+    rows = singles + 2                                       # the last request brings two tokens where it takes part
+    q, key, v = (torch.randn(rows, heads * n, generator=gen, device="cuda").to(dtype) for n in (keys, keys, values))
+    decay = -torch.rand(rows, heads * keys, generator=gen, device="cuda")
+    beta = torch.randn(rows, heads, generator=gen, device="cuda")
+    live = torch.randn(singles + 2, state, generator=gen, device="cuda")
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    slots = ints([4, 0, 2, 5, 1, 3, 3])
+    for rule in ("decayed", "delta"):
+        got = []
+        for m, segments in ((singles, singles), (rows, singles + 1)):
+            out, stage = torch.empty(m, heads * values, device="cuda"), live.clone()
+            where = (out, live, stage, 0, ints(list(range(segments))), ints([1] * singles + [2])[:segments], segments, slots[:m])
+            if rule == "decayed":
+                k.linear_recurrence(q[:m], key[:m], v[:m], decay[:m], *where, heads, keys, values)
+            else:
+                k.delta_rule(q[:m], key[:m], v[:m], decay[:m], beta[:m], *where, heads, keys, values)
+            got.append((out[:singles], stage[slots[:singles].long()]))
+        assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]), rule
