@@ -713,36 +713,51 @@ __global__ __launch_bounds__(256) void sink_attention_tiles_kernel(SinkArgs a, c
 }
 
 // The merge of the key ranges' shares (maxima and sums in the base-2 domain, as the kernel above leaves them), the
-// sink and the division: one wavefront per (token of a group, head).
+// sink and the division: one wavefront per (token of a group, head), NC values a lane.  Bound by its chain of loads: the
+// values are asked for AHEAD ranges at a time, the first before the ranges' maxima are known (48 tokens of 16 heads of 128
+// values in 6 ranges: 8.7 us range by range, now 5.1).
+template <int NC>
 __global__ __launch_bounds__(64) void sink_tiles_combine_kernel(SinkArgs a, const int32_t* __restrict__ group_first,
                                                                 const int32_t* __restrict__ group_count) {
+    constexpr int AHEAD = NC <= 2 ? 8 : 16 / NC;
     const int group = blockIdx.x, ti = blockIdx.z, head = blockIdx.y, lane = threadIdx.x;
     if (ti >= group_count[group]) return;
     const int m = group_first[group] + ti, V = a.value_dim;
     const float* base = a.partial + (((size_t)group * a.group_tokens + ti) * a.q_heads + head) * a.splits * (V + 4);
-    float top = a.sink != nullptr ? a.sink[head] * 1.4426950408889634f : -INFINITY;
-    const float sink2 = top;
-    for (int z = 0; z < a.splits; ++z) top = fmaxf(top, base[(size_t)z * (V + 4) + V]);
+    float part[AHEAD][NC];
+    auto fetch = [&](int z0) {
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u)
+#pragma unroll
+            for (int i = 0; i < NC; ++i) part[u][i] = base[(size_t)min(z0 + u, a.splits - 1) * (V + 4) + min(lane + 64 * i, V - 1)];
+    };
+    fetch(0);
+    const float sink2 = a.sink != nullptr ? a.sink[head] * 1.4426950408889634f : -INFINITY;
+    float top = sink2;
+    for (int z = lane; z < a.splits; z += 64) top = fmaxf(top, base[(size_t)z * (V + 4) + V]);
+    top = wave_max(top);
     float den = a.sink != nullptr ? exp2f(sink2 - top) : 0.f;
-    float num[8];
+    float num[NC];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) num[i] = 0.f;
-    for (int z = 0; z < a.splits; ++z) {
-        const float* p = base + (size_t)z * (V + 4);
-        const float zmax = p[V];
-        if (!(zmax > -INFINITY)) continue;     // (a range beyond the token's keys)
-        const float w = exp2f(zmax - top);
-        den += w * p[V + 1];
+    for (int i = 0; i < NC; ++i) num[i] = 0.f;
+    for (int z0 = 0; z0 < a.splits; z0 += AHEAD) {
+        if (z0 > 0) fetch(z0);
+        const float* mine = base + (size_t)min(z0 + lane % AHEAD, a.splits - 1) * (V + 4) + V;     // (lane u: range z0 + u)
+        const float maxima = mine[0], sums = mine[1];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int c = lane + 64 * i;
-            if (c < V) num[i] += w * p[c];
+        for (int u = 0; u < AHEAD; ++u) {
+            const float zmax = __shfl(maxima, u, MLR_WAVE);
+            if (z0 + u >= a.splits || !(zmax > -INFINITY)) continue;      // (a range beyond the token's keys)
+            const float w = exp2f(zmax - top);
+            den += w * __shfl(sums, u, MLR_WAVE);
+#pragma unroll
+            for (int i = 0; i < NC; ++i) num[i] += w * part[u][i];
         }
     }
     const float inv = den > 0.f ? 1.0f / den : 0.f;
     __bf16* dst = a.out + (size_t)m * a.out_stride + (size_t)head * V;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < NC; ++i) {
         const int c = lane + 64 * i;
         if (c < V) dst[c] = (__bf16)(num[i] * inv);
     }
@@ -762,8 +777,10 @@ static int launch_sink_tiles(const SinkArgs& a, const int32_t* first, const int3
     }
     sink_attention_tiles_kernel<NKF, NVT, SPLITV><<<dim3(groups, a.kv_heads * head_blocks, a.partial ? a.splits : 1), 256, lds,
                                                    stream>>>(a, first, count, head_block, head_blocks);
-    if (a.partial != nullptr)
-        sink_tiles_combine_kernel<<<dim3(groups, a.q_heads, a.group_tokens), 64, 0, stream>>>(a, first, count);
+    if (a.partial != nullptr) {
+        constexpr int NC = (NVT * 16 + 63) / 64;
+        sink_tiles_combine_kernel<NC><<<dim3(groups, a.q_heads, a.group_tokens), 64, 0, stream>>>(a, first, count);
+    }
     return (int)hipGetLastError();
 }
 #endif

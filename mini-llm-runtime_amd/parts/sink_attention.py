@@ -92,14 +92,17 @@ def _groups_plan(rows, q_heads, kv_heads, value_dim):
 def _key_ranges(ctx, groups, tokens, workgroups, q_heads, value_dim, mask, mask_size, keep_first=0):
     """(keys a range, ranges, room for their shares) for a launch over `groups` groups of single tokens or short portions
     that has `workgroups` workgroups without ranges: where those do not fill the GPU, a group's keys (its window or
-    chunk; without a mask the step's longest context) are dealt out to several workgroups, as many as reach
-    `target_workgroups`, none narrower than RANGE_KEYS, and no more than their shares have room for."""
+    chunk; without a mask the step's longest context) are dealt out to several workgroups, as many as reach twice
+    `target_workgroups` (four a compute unit), none narrower than RANGE_KEYS, and no more than their shares have room for.
+    Single tokens of requests of 100 to 1200 keys, Sagopel's sizes: 48 of them 1741 us a step for 1762 with half as many
+    workgroups, 128 2699 for 2790; Pamunex's latent attention 1393 for 1420 and 1946 for 2064; three times as many: 1755,
+    2681, 1387, 1894.  Batches of 16 or less, which RANGE_KEYS and MOST_RANGES bound, take the same."""
     k = ctx.kernels
     reach = (mask_size if mask == "chunk" else mask_size + tokens - 1) if mask is not None else ctx.max_context
     if mask is not None and keep_first > 0:
         reach += -(-keep_first // 32) * 32
     reach = min(reach, ctx.max_context + 31) + 31             # (ranges start at the first tile, which may start earlier)
-    most = max(1, min(MOST_RANGES, -(-reach // RANGE_KEYS), -(-ctx.target_workgroups // max(1, workgroups))))
+    most = max(1, min(MOST_RANGES, -(-reach // RANGE_KEYS), -(-2 * ctx.target_workgroups // max(1, workgroups))))
     room = ctx.workspace.get("sink_partial", (min(PARTIAL_CAP, k.sink_partial_numel(groups, tokens, q_heads, value_dim, most)),),
                              torch.float32)
     most = min(most, room.numel() // k.sink_partial_numel(groups, tokens, q_heads, value_dim, 1))

@@ -907,3 +907,25 @@ def test_configurations_drawn_at_random(tmp_path, seed):
         if dtype_name == "float32":
             assert max_difference(results["whole"], results["portions"]) == 0.0, cfg
             assert max_difference(results["whole"], results["mixed"]) == 0.0, cfg
+
+
+@pytest.mark.parametrize("T,ranges", [(250, 32), (257, 32), (600, 32), (2100, 32), (2100, 1056)])
+@pytest.mark.parametrize("dim,vdim", [(64, 48), (128, 128), (128, 144), (576, 512)])
+def test_a_lone_tokens_keys_in_many_ranges(T, ranges, dim, vdim):
+    """The merge asks for several ranges at a time: numbers of ranges around those and around a wavefront's 64 lanes."""
+    from mini_llm_runtime_amd.kernels import Kernels
+    dtype, heads, kv, page = torch.bfloat16, 4, 2, 16
+    k = Kernels(dtype)
+    rng = np.random.default_rng(T + dim)
+    keys, values = (back(rounded(rng.normal(size=(T, kv, d)), dtype)) for d in (dim, vdim))
+    q = back(rounded(rng.normal(size=(1, heads, dim)), dtype))
+    want = P.attend(q, keys, values, dim ** -0.5, 50.0, np.ones((1, T), dtype=bool))
+    (k_pages, table), (v_pages, _) = paged(keys, page, dtype, seed=1), paged(values, page, dtype, seed=1)
+    _, _, small_heads, small_tokens = k.sink_tiles_layout(heads, kv)
+    splits = -(-(T + 31) // ranges)
+    out = torch.full((1, heads * vdim), float("nan"), dtype=dtype, device="cuda")
+    partial = torch.full((k.sink_partial_numel(1, small_tokens, heads, vdim, splits),), float("nan"), device="cuda")
+    k.sink_attention_tiles(rounded(q.reshape(1, -1), dtype), k_pages, v_pages, table, ints([0]), ints([T - 1]), None, out, ints([0]),
+                           ints([1]), 1, small_heads, True, heads, kv, dim, vdim, page, dim ** -0.5, None, 0, T, partial=partial,
+                           split_keys=ranges, splits=splits, softcap=50.0)
+    np.testing.assert_allclose(back(out), want, **tolerance("bfloat16"))
