@@ -70,7 +70,7 @@ __global__ __launch_bounds__(256) void causal_conv_kernel(ConvArgs a) {
 }
 
 #if MLR_BF16
-// Many rows: eight channels a thread (16-byte accesses) and CONV_ROWS rows, for which its weights stay in registers.  Bound by
+// Many values: eight channels a thread (16-byte accesses) and CONV_ROWS rows, for which its weights stay in registers.  Bound by
 // memory; one value a thread took 62 us for 2048 rows of 4096 channels, this 22.
 #define CONV_ROWS 4
 template <int TAPS>
@@ -872,8 +872,10 @@ int mlr_causal_conv(const void* x, long x_stride, const float* w, const float* b
                rows, channels, taps, silu, write_state};
 #if MLR_BF16
     const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-    // (64 rows: below that the walk of CONV_ROWS rows is longer than what the wider accesses save)
-    if (rows >= 64 && taps == 4 && channels % 8 == 0 && x_stride % 8 == 0 && out_stride % 8 == 0 && aligned(x) && aligned(out) && aligned(w)) {
+    // A walk of CONV_ROWS rows takes 11 us however few they are.  The line lies where one value a thread takes as long: 256
+    // rows of 6144 channels 12.2 us and 11.3 here, 384 of 4352 12.5 and 12.0; but 512 of 2048 9.2 and 11.0, 128 of 4352 6.7 and 10.9.
+    const bool many = (long)rows * channels >= 3L << 19;
+    if (many && taps == 4 && channels % 8 == 0 && x_stride % 8 == 0 && out_stride % 8 == 0 && aligned(x) && aligned(out) && aligned(w)) {
         causal_conv_rows_kernel<4><<<dim3((rows + CONV_ROWS - 1) / CONV_ROWS, (channels / 8 + 255) / 256), 256, 0, stream>>>(a);
         return (int)hipGetLastError();
     }

@@ -23,8 +23,7 @@ def ints(x):
     return torch.tensor(x, dtype=torch.int32, device="cuda")
 
 
-@pytest.mark.parametrize("channels", [8, 264, 2056])
-@pytest.mark.parametrize("rows", [64, 67])
+@pytest.mark.parametrize("rows,channels", [(768, 2048), (767, 2056), (769, 2048), (5959, 264), (153, 10288)])
 def test_causal_conv_of_many_rows(rows, channels):
     k = kernels(torch.bfloat16)
     gen = torch.Generator("cuda").manual_seed(rows + channels)
