@@ -1,8 +1,8 @@
 // out[M, N] = a[M, K] . w[N, K]^T  (both operands row-major with K contiguous, the layout of
 // an activation and of a projection's weight), accumulated in 32-bit.
 //
-// Float engine: 32-bit matrix instructions, the weight streamed for few rows and tiled for many; the order of an
-// element's sum is the same everywhere, so a row's result does not depend on the other rows of the batch.
+// Float engine: 32-bit matrix instructions, a wavefront a strip of columns for few rows and tiles for many; every element is
+// one chain of fmaf over k from 0 up, so a row's result does not depend on the other rows of the batch.
 // Bfloat16 engine, three families, each with a fixed k order for every output element (so a row's result
 // does not depend on the rows beside it): up to 64 rows the weight is streamed once straight into
 // v_mfma_f32_16x16x32_bf16 (`gemm_skinny_kernel`, optionally with the residual add and RMSNorm in front
@@ -13,213 +13,200 @@
 
 #if !MLR_BF16
 // ------------------------------------------------------------------------------ float
-// v_mfma_f32_16x16x4_f32 (32-bit products and sums), 16 k at a time: a lane holds four consecutive k of one row of
-// each operand (one 16-byte load), and the four products of a group take the k {e, 4 + e, 8 + e, 12 + e}.  The order of
-// an element's sum follows from K alone, whatever kernel and tile serve it, so that a token's result is the same to the
-// bit however a step was cut: k is cut into at most eight PARTS of `part_of(K)`, a part is summed in groups of 16 from
-// its start, and the parts are added as (p0 + p1 + ..) + (ph + ..), the second half from part (parts + 1) / 2 on.
-// Shorter chains than one sum over all of k: the error against 64 bits of a 3072-wide product is a third of that.
+// v_mfma_f32_16x16x4_f32 rounds as four fmaf one behind the other in the order of its k-slots, so an element is ONE chain of
+// fmaf over k from 0 up, whatever kernel and tile serve it: its bits hang neither on the rows beside it nor on how a step was
+// cut, and a plain loop over k gives the same.  A matrix instruction wants k-slot b from lanes 16 b ..; a 16-byte load gives a
+// lane four neighbouring k of one row, so four lane blocks exchange: `turned` makes register i of block b what register b of
+// block i was, and product i of a group of 16 then takes k = 4 i + b.
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 
-static int part_of(int K) { return K <= 512 ? 64 : ((K + 7) / 8 + 15) / 16 * 16; }
+__device__ __forceinline__ floatx4 turned(const floatx4& v) {
+    unsigned r[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = __float_as_uint(v[i]);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const auto x = __builtin_amdgcn_permlane32_swap(r[i], r[i + 2], false, false);
+        r[i] = x[0];
+        r[i + 2] = x[1];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i += 2) {
+        const auto x = __builtin_amdgcn_permlane16_swap(r[i], r[i + 1], false, false);
+        r[i] = x[0];
+        r[i + 1] = x[1];
+    }
+    return floatx4{__uint_as_float(r[0]), __uint_as_float(r[1]), __uint_as_float(r[2]), __uint_as_float(r[3])};
+}
 
-// Four consecutive k of a row from k on, zeros from `end` on (VEC: rows start on 16 bytes and K is a multiple of four).
+// Four consecutive k of a row from k on, zeros from K on (VEC: rows start on 16 bytes and K is a multiple of four).
 template <bool VEC>
-__device__ __forceinline__ floatx4 load_k4(const float* __restrict__ row, int k, int end) {
+__device__ __forceinline__ floatx4 load_k4(const float* __restrict__ row, int k, int K) {
     floatx4 v = {0.f, 0.f, 0.f, 0.f};
     if (VEC) {
-        if (k < end) v = *reinterpret_cast<const floatx4*>(row + k);
+        if (k < K) v = *reinterpret_cast<const floatx4*>(row + k);
     } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-            if (k + e < end) v[e] = row[k + e];
+            if (k + e < K) v[e] = row[k + e];
     }
     return v;
 }
 
-// Up to 32 rows: bound by the weight, which is streamed once from memory straight into the matrix cores.  A workgroup
-// owns NT strips of 16 output columns, its eight wavefronts a part of k each, so that all loads of a short part are under
-// way at once; the parts meet in LDS.
-template <int TM, int NT, bool VEC>
-__global__ __launch_bounds__(512) void gemm_f32_rows_kernel(const float* __restrict__ a, const float* __restrict__ w,
-                                                            float* __restrict__ out, int M, int N, int K, int part) {
-    constexpr int U = TM * NT <= 2 ? 8 : 4;              // groups of 16 k asked for at once
-    constexpr int W = NT * 16 + 1;
-    __shared__ float red[8][TM * 16][W];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = (lane >> 4) * 4;
-    const int n0 = blockIdx.x * (NT * 16);
-    const float* ar[TM];
-    const float* wr[NT];
+// Few tiles of 16 x 16: a wavefront owns 16 rows and NT strips of 16 columns and walks all of k alone.  The chain of products is
+// the bound (32 clocks for every four k), so nothing else may stand in its way: the exchange between lane blocks is left to LDS
+// (16-byte stores of what a lane has loaded, 4-byte reads of what it needs, both free of bank conflicts; no other wavefront
+// takes part), blocks of U groups of 16 k are stored one block and loaded two blocks ahead, and a group is read one group ahead.
+template <int NT, int U>
+__global__ __launch_bounds__(64) void gemm_f32_strip_kernel(const float* __restrict__ a, const float* __restrict__ w,
+                                                            float* __restrict__ out, int M, int N, int K) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];               // [2][U][1 + NT][256]
+    constexpr int P = 1 + NT;
+    const int lane = threadIdx.x, r = lane & 15, b = lane >> 4, m0 = blockIdx.y * 16, n0 = blockIdx.x * (NT * 16);
+    const float* from[P];                                  // the lane's row of a and of every strip
+    from[0] = a + (size_t)min(m0 + r, M - 1) * K + b * 4;
 #pragma unroll
-    for (int i = 0; i < TM; ++i) ar[i] = a + (size_t)min(i * 16 + r, M - 1) * K;
+    for (int j = 0; j < NT; ++j) from[1 + j] = w + (size_t)min(n0 + j * 16 + r, N - 1) * K + b * 4;
+    floatx4 acc[NT], x[U][P];
 #pragma unroll
-    for (int j = 0; j < NT; ++j) wr[j] = w + (size_t)min(n0 + j * 16 + r, N - 1) * K;
-    floatx4 acc[TM][NT];
+    for (int j = 0; j < NT; ++j) acc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const int blocks = (K + 16 * U - 1) / (16 * U);
+    auto fetch = [&](int t, int u, bool whole) {           // (never behind a condition of its own; K is a multiple of four)
+        const int at = whole ? t * U * 16 : min((t * U + u) * 16, K - 4 - b * 4) - u * 16;
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+        for (int j = 0; j < P; ++j) x[u][j] = *reinterpret_cast<const floatx4*>(from[j] + at + u * 16);
+    };
+    auto stash = [&](int t, int u, bool whole) {
 #pragma unroll
-        for (int j = 0; j < NT; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-    int k = wave * part;
-    const int end = min(K, k + part);
-    // (whole groups without checks: loads behind a condition would wait for each other)
-    for (; VEC && k + 16 * U <= end; k += 16 * U) {
-        floatx4 wv[NT][U], av[TM][U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-#pragma unroll
-            for (int j = 0; j < NT; ++j) wv[j][u] = *reinterpret_cast<const floatx4*>(wr[j] + k + u * 16 + q);
-#pragma unroll
-            for (int i = 0; i < TM; ++i) av[i][u] = *reinterpret_cast<const floatx4*>(ar[i] + k + u * 16 + q);
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int j = 0; j < NT; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i][u][e], wv[j][u][e], acc[i][j], 0, 0, 0);
-    }
-    for (; k < end; k += 16) {
-        floatx4 wv[NT], av[TM];
-#pragma unroll
-        for (int j = 0; j < NT; ++j) wv[j] = load_k4<VEC>(wr[j], k + q, end);
-#pragma unroll
-        for (int i = 0; i < TM; ++i) av[i] = load_k4<VEC>(ar[i], k + q, end);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < NT; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i][e], wv[j][e], acc[i][j], 0, 0, 0);
-    }
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) red[wave][i * 16 + q + e][j * 16 + r] = acc[i][j][e];
-    __syncthreads();
-    const int parts = (K + part - 1) / part, half = (parts + 1) / 2;
-    for (int i = threadIdx.x; i < TM * 16 * NT * 16; i += 512) {
-        const int row = i / (NT * 16), col = i % (NT * 16);
-        if (row >= M || n0 + col >= N) continue;
-        float first = red[0][row][col];
-        for (int p = 1; p < half; ++p) first += red[p][row][col];
-        if (half < parts) {
-            float second = red[half][row][col];
-            for (int p = half + 1; p < parts; ++p) second += red[p][row][col];
-            first += second;
-        }
-        out[(size_t)row * N + n0 + col] = first;
-    }
-}
-
-// More rows: bound by the matrix cores.  Two sets of WM x WN wavefronts, each with its half of the parts of k and its own
-// LDS blocks of G groups of 16 k (rows of a group 80 bytes apart: 16 lanes' 16-byte reads meet every bank once), the next
-// block's loads under way while one is multiplied -- so small tiles, whose products take no time, take long blocks.  The
-// second set's sums reach the first through LDS at the end.
-template <int WM, int WN, int TM, int TN, int G, bool VEC>
-__global__ __launch_bounds__(WM * WN * 128) void gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ w,
-                                                                      float* __restrict__ out, int M, int N, int K, int part) {
-    constexpr int BM = WM * TM * 16, BN = WN * TN * 16, SET = WM * WN * 64, STRIDE = 20, ROWS = BM + BN;
-    constexpr int ALL = ROWS * 4 * G, CHUNKS = ALL / SET;                    // 16-byte chunks of a block
-    static_assert(ALL % SET == 0, "whole chunks a thread");
-    static_assert(4 * G * ROWS * STRIDE >= BM * BN, "the second set's sums fit the blocks' place");
-    extern __shared__ __attribute__((aligned(16))) float lds[];               // [buffer][set][group][row][STRIDE]
-    const int set = threadIdx.x / SET, t = threadIdx.x % SET, lane = t & 63, wave = t >> 6;
-    const int wm = wave / WN, wn = wave % WN, r = lane & 15, q = (lane >> 4) * 4;
-    // neighbouring tiles of a weight strip to the same XCD (workgroups are dealt out to the eight in turn)
-    const int tiles_m = (M + BM - 1) / BM, tiles = tiles_m * ((N + BN - 1) / BN), each = (tiles + 7) / 8;
-    const int tile = (blockIdx.x % 8) * each + blockIdx.x / 8;
-    if (blockIdx.x / 8 >= each || tile >= tiles) return;
-    const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * BN;
-    const int parts = (K + part - 1) / part, half = (parts + 1) / 2;
-    const int begin = set * half * part, end = set ? K : min(K, half * part);
-    const int groups = (min(K, half * part) + 15) / 16, turns = (groups + G - 1) / G, per = part / 16;
-
-    floatx4 stage[CHUNKS];
-    auto load = [&](int k0) {                              // (chunk: four k of a row; a row's chunks side by side)
-#pragma unroll
-        for (int c = 0; c < CHUNKS; ++c) {
-            const int row = (t + c * SET) / (4 * G), k = k0 + (t + c * SET) % (4 * G) * 4;
-            const float* p = row < BM ? a + (size_t)min(m0 + row, M - 1) * K : w + (size_t)min(n0 + row - BM, N - 1) * K;
-            stage[c] = load_k4<VEC>(p, k, end);
+        for (int j = 0; j < P; ++j) {
+            floatx4 v = x[u][j];
+            if (!whole && (t * U + u) * 16 + b * 4 >= K) v = floatx4{0.f, 0.f, 0.f, 0.f};
+            *reinterpret_cast<floatx4*>(lds + (((t & 1) * U + u) * P + j) * 256 + lane * 4) = v;
         }
     };
-    floatx4 acc[TM][TN], sum[TM][TN];
+    auto whole = [&](int t) { return (t + 1) * U * 16 <= K; };
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int u = 0; u < U; ++u) fetch(0, u, false);
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = sum[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-    load(begin);
-    int in_part = 0;
-    for (int turn = 0; turn < turns; ++turn) {
-        float* block = lds + ((turn & 1) * 2 + set) * (G * ROWS * STRIDE);
+    for (int u = 0; u < U; ++u) stash(0, u, false);
 #pragma unroll
-        for (int c = 0; c < CHUNKS; ++c) {
-            const int row = (t + c * SET) / (4 * G), k = (t + c * SET) % (4 * G);
-            *reinterpret_cast<floatx4*>(block + ((k >> 2) * ROWS + row) * STRIDE + (k & 3) * 4) = stage[c];
+    for (int u = 0; u < U; ++u) fetch(min(1, blocks - 1), u, false);
+    auto turn = [&](int t, bool all) {                     // all: the two blocks behind t are whole
+        const float* at = lds + (t & 1) * (U * P * 256) + r * 4 + b;
+        floatx4 now[P], next[P];
+        auto read = [&](int u, floatx4 (&v)[P]) {          // element i: k = 4 i + b of the group
+#pragma unroll
+            for (int j = 0; j < P; ++j)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[j][i] = at[(u * P + j) * 256 + i * 64];
+        };
+        read(0, now);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (u + 1 < U) read(u + 1, next);
+            stash(t + 1, u, all);
+            fetch(all ? t + 2 : min(t + 2, blocks - 1), u, all);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now[0][i], now[1 + j][i], acc[j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);             // (left alone, the compiler moves a load to where its value is used)
+#pragma unroll
+            for (int j = 0; j < P; ++j) now[j] = next[j];
         }
+    };
+    int t = 0;
+    for (; t + 2 < blocks && whole(t + 2); ++t) turn(t, true);
+    for (; t < blocks; ++t) turn(t, false);                // (behind the last block zeros are stored that nothing reads)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int m = m0 + b * 4 + e, n = n0 + j * 16 + r;
+            if (m < M && n < N) out[(size_t)m * N + n] = acc[j][e];
+        }
+}
+
+// More rows: bound by the matrix cores.  Four wavefronts of T x T tiles of 16 x 16; blocks of G groups of 16 k go through LDS as
+// the products want them (rows of a group 80 bytes apart: 16 lanes' 16-byte accesses meet every bank once), the next block's
+// loads under way while one is multiplied -- so small tiles, whose products take no time, take long blocks.
+template <int T, int G, bool VEC>
+__global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ w,
+                                                            float* __restrict__ out, int M, int N, int K) {
+    constexpr int B = 2 * T * 16, STRIDE = 20, ROWS = 2 * B, UNITS = ROWS / 16, EACH = UNITS * G / 4;     // units: 16 rows x 16 k
+    static_assert(UNITS * G % 4 == 0, "as many units for every wavefront");
+    extern __shared__ __attribute__((aligned(16))) float lds[];               // [buffer][group][row][STRIDE]
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = (lane >> 4) * 4;
+    const int wm = wave / 2, wn = wave % 2;
+    // neighbouring tiles of a weight strip to the same XCD (workgroups are dealt out to the eight in turn)
+    const int tiles_m = (M + B - 1) / B, tiles = tiles_m * ((N + B - 1) / B), each = (tiles + 7) / 8;
+    const int tile = (blockIdx.x % 8) * each + blockIdx.x / 8;
+    if (blockIdx.x / 8 >= each || tile >= tiles) return;
+    const int m0 = (tile % tiles_m) * B, n0 = (tile / tiles_m) * B;
+    const int turns = (K + 16 * G - 1) / (16 * G);
+
+    floatx4 stage[EACH];
+    auto load = [&](int k0) {
+#pragma unroll
+        for (int c = 0; c < EACH; ++c) {
+            const int unit = wave + 4 * c, row = unit % UNITS * 16 + r;
+            const float* p = row < B ? a + (size_t)min(m0 + row, M - 1) * K : w + (size_t)min(n0 + row - B, N - 1) * K;
+            stage[c] = load_k4<VEC>(p, k0 + unit / UNITS * 16 + q, K);
+        }
+    };
+    floatx4 acc[T][T];
+#pragma unroll
+    for (int i = 0; i < T; ++i)
+#pragma unroll
+        for (int j = 0; j < T; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    load(0);
+    for (int turn = 0; turn < turns; ++turn) {
+        float* block = lds + (turn & 1) * (G * ROWS * STRIDE);
+#pragma unroll
+        for (int c = 0; c < EACH; ++c) {
+            const int unit = wave + 4 * c;
+            *reinterpret_cast<floatx4*>(block + (unit / UNITS * ROWS + unit % UNITS * 16 + r) * STRIDE + q) = turned(stage[c]);
+        }
+        // (one barrier a turn: a buffer is written again behind the barrier that follows every wavefront's reads of it)
         __syncthreads();
-        if (turn + 1 < turns) load(begin + (turn + 1) * 16 * G);
+        if (turn + 1 < turns) load((turn + 1) * 16 * G);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int g = 0; g < G; ++g) {
             const float* rows = block + g * ROWS * STRIDE;
-            floatx4 av[TM], wv[TN];
+            floatx4 av[T], wv[T];
 #pragma unroll
-            for (int i = 0; i < TM; ++i) av[i] = *reinterpret_cast<const floatx4*>(rows + ((wm * TM + i) * 16 + r) * STRIDE + q);
+            for (int i = 0; i < T; ++i) av[i] = *reinterpret_cast<const floatx4*>(rows + ((wm * T + i) * 16 + r) * STRIDE + q);
 #pragma unroll
-            for (int j = 0; j < TN; ++j) wv[j] = *reinterpret_cast<const floatx4*>(rows + (BM + (wn * TN + j) * 16 + r) * STRIDE + q);
+            for (int j = 0; j < T; ++j) wv[j] = *reinterpret_cast<const floatx4*>(rows + (B + (wn * T + j) * 16 + r) * STRIDE + q);
 #pragma unroll
             for (int e = 0; e < 4; ++e)
 #pragma unroll
-                for (int i = 0; i < TM; ++i)
+                for (int i = 0; i < T; ++i)
 #pragma unroll
-                    for (int j = 0; j < TN; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i][e], wv[j][e], acc[i][j], 0, 0, 0);
-            // (groups beyond the set's half hold zeros and add nothing)
-            if (++in_part == per || (turn + 1 == turns && g + 1 == G)) {
-                in_part = 0;
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int j = 0; j < TN; ++j) {
-                        sum[i][j] += acc[i][j];
-                        acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-                    }
-            }
+                    for (int j = 0; j < T; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i][e], wv[j][e], acc[i][j], 0, 0, 0);
         }
     }
-    __syncthreads();
-    if (set == 1) {
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < T; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j)
-                *reinterpret_cast<floatx4*>(lds + (((wave * TM + i) * TN + j) * 64 + lane) * 4) = sum[i][j];
-    }
-    __syncthreads();
-    if (set == 1) return;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const floatx4 second = *reinterpret_cast<const floatx4*>(lds + (((wave * TM + i) * TN + j) * 64 + lane) * 4);
-            const int n = n0 + (wn * TN + j) * 16 + r;
+        for (int j = 0; j < T; ++j) {
+            const int n = n0 + (wn * T + j) * 16 + r;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int m = m0 + (wm * TM + i) * 16 + q + e;
-                if (m < M && n < N) out[(size_t)m * N + n] = sum[i][j][e] + second[e];
+                const int m = m0 + (wm * T + i) * 16 + q + e;
+                if (m < M && n < N) out[(size_t)m * N + n] = acc[i][j][e];
             }
         }
 }
 
-template <int TM, int NT, bool VEC>
-static int launch_f32_rows(const float* a, const float* w, float* out, int M, int N, int K, hipStream_t stream) {
-    gemm_f32_rows_kernel<TM, NT, VEC><<<(N + NT * 16 - 1) / (NT * 16), 512, 0, stream>>>(a, w, out, M, N, K, part_of(K));
+template <int NT, int U>
+static int launch_f32_strip(const float* a, const float* w, float* out, int M, int N, int K, hipStream_t stream) {
+    constexpr size_t lds = 2 * U * (1 + NT) * 256 * sizeof(float);
+    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_strip_kernel<NT, U>),
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (allowed != hipSuccess) return (int)allowed;
+    gemm_f32_strip_kernel<NT, U><<<dim3((N + NT * 16 - 1) / (NT * 16), (M + 15) / 16), 64, lds, stream>>>(a, w, out, M, N, K);
     return (int)hipGetLastError();
 }
 
@@ -228,39 +215,37 @@ static int launch_f32_tile(const float* a, const float* w, float* out, int M, in
     constexpr int B = 2 * T * 16;
     const long long tiles = (long long)((M + B - 1) / B) * ((N + B - 1) / B);
     if (tiles > 0x7ffffff0LL) return -2;
-    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_tile_kernel<2, 2, T, T, G, VEC>),
-                                                          hipFuncAttributeMaxDynamicSharedMemorySize, 4 * G * 2 * B * 20 * sizeof(float));
+    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_tile_kernel<T, G, VEC>),
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, 2 * G * 2 * B * 20 * sizeof(float));
     if (allowed != hipSuccess) return (int)allowed;
-    gemm_f32_tile_kernel<2, 2, T, T, G, VEC><<<(unsigned)((tiles + 7) / 8 * 8), 512, 4 * G * 2 * B * 20 * sizeof(float), stream>>>(
-        a, w, out, M, N, K, part_of(K));
+    gemm_f32_tile_kernel<T, G, VEC><<<(unsigned)((tiles + 7) / 8 * 8), 256, 2 * G * 2 * B * 20 * sizeof(float), stream>>>(a, w, out, M, N, K);
     return (int)hipGetLastError();
 }
 
 template <bool VEC>
 static int launch_gemm_f32(const float* a, const float* w, float* out, int M, int N, int K, hipStream_t stream) {
-    const int strips = (N + 15) / 16;
-    if (M <= 16) {
-        // Four strips a workgroup, for which the rows are read once, where that still gives two workgroups a compute unit
-        // and the rows weigh something beside the weight: 16 rows of N x K = 24576 x 4096 88.6 us for 102.0, of 151936 x
-        // 1024 126 for 158 (5 TB/s of weight); but 4 rows 85.7 for 73.1 (5.5 TB/s).  The weights of a layer of the 0.6B
-        // sizes (4096 x 1024, 1024 x 2048, 6144 x 1024, 1024 x 3072) take 8 to 11 us with 8 rows, where a 64 x 64 tile
-        // with k from end to end took 101, 196, 101 and 292.
-        return M > 8 && strips >= 1024 ? launch_f32_rows<1, 4, VEC>(a, w, out, M, N, K, stream)
-                                       : launch_f32_rows<1, 1, VEC>(a, w, out, M, N, K, stream);
+    // A wavefront a tile of 16 x 16 while those are few: 8 rows of 4096 x 1024, 1024 x 2048, 6144 x 1024 and 1024 x 3072 take 9.3,
+    // 14.0, 10.8 and 19.3 us (tiles of 32 14.3, 23.7, 15.8 and 34.3), 64 rows of 1024 x 3072 19.4 (40), 32 of 6144 x 1024 (768
+    // tiles) 16.0 (17.6).  Two strips a wavefront beyond that, while the rows are few or up to 1024 tiles: 64 rows of 4096 x 1024
+    // 14.9 (one strip 19.9, tiles of 32 16.7), 8 of 24576 x 4096 96 and of 151936 x 1024 158 (130 and 184; the weight alone
+    // takes 84 and 130); 64 rows of 6144 x 1024 (1536 tiles) 22.1 and in tiles of 32 21.3.
+    const long long units = (long long)((M + 15) / 16) * ((N + 15) / 16);
+    if (VEC && (M + 15) / 16 <= 65535) {
+        if (units <= 768) return launch_f32_strip<1, 8>(a, w, out, M, N, K, stream);
+        if (M <= 16 || units <= 1024) return launch_f32_strip<2, 4>(a, w, out, M, N, K, stream);
     }
-    if (M <= 32)
-        // (two strips beyond one a compute unit: 6144 x 1024 11.3 us for 13.6; up to 256 strips one: 4096 x 1024 9.1 for 11.5)
-        return strips > 256 ? launch_f32_rows<2, 2, VEC>(a, w, out, M, N, K, stream)
-                            : launch_f32_rows<2, 1, VEC>(a, w, out, M, N, K, stream);
     // The square tile whose workgroups, one a compute unit at a time, are done first: a tile of 64 takes 1 / 3.7 of the time
-    // of one of 128, a tile of 32 0.35 of one of 64 (at 2048 rows of 4096 x 12288, 24576 x 4096 and 2048 x 2112; tiles of
-    // 128 reach 120 TFLOP/s there).  1500 rows of 6144 x 1024 take 197 us in tiles of 64 and 228 in those of 128, 64 rows
-    // of 1024 x 3072 27 in those of 32 for 66 (from 33 rows on the kernel above is no faster: 30 us here).
+    // of one of 128, a tile of 32 0.35 of one of 64 (at 2048 rows of 4096 x 4096; tiles of 128 reach 120 TFLOP/s there).  1500
+    // rows of 6144 x 1024 take 198 us in tiles of 64 and 230 in those of 128, 2048 rows 257 and 231, 400 rows of 1024 x 3072 57
+    // in those of 32 and 96 in those of 64.
     auto cost = [&](int b, double one) {
         return one * (double)(((long long)((M + b - 1) / b) * ((N + b - 1) / b) + 255) / 256);
     };
     const double c32 = cost(32, 0.35), c64 = cost(64, 1.0), c128 = cost(128, 3.7);
-    if (c32 <= c64 && c32 <= c128) return launch_f32_tile<1, 4, VEC>(a, w, out, M, N, K, stream);
+    if (c32 <= c64 && c32 <= c128)
+        // (blocks of 8 groups leave room for one workgroup a compute unit, of 4 for three: 128 rows of 4096 x 1024, 512 tiles, 24.3
+        // and 26.0 us, of 6144 x 1024, 768 tiles, 36.7 and 30.0)
+        return c32 <= 0.7 ? launch_f32_tile<1, 8, VEC>(a, w, out, M, N, K, stream) : launch_f32_tile<1, 4, VEC>(a, w, out, M, N, K, stream);
     return c64 <= c128 ? launch_f32_tile<2, 2, VEC>(a, w, out, M, N, K, stream)
                        : launch_f32_tile<4, 1, VEC>(a, w, out, M, N, K, stream);
 }

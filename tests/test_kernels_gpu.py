@@ -212,10 +212,9 @@ def test_gemm_rows_do_not_depend_on_the_batch(dtype):
 @pytest.mark.parametrize("n,kk", [(1, 4), (15, 1), (17, 60), (33, 64), (70, 511), (64, 516), (130, 528), (16400, 96), (4112, 1030), (96, 3072),
                                   (40, 12296)])
 def test_gemm_float_edges(n, kk):
-    """The float product at the edges of its row counts (8/9, 16/17, 32/33: another kernel or strip width), tiles and parts of
-    k, rows that start on 16 bytes and rows that do not: one order of additions, so a row's bits are those it has alone; and
-    every element within the bound of a sum in at most eight chains, (k / 8 + 16 + 9) 2^-24 sum |a w| (a part is rounded up to
-    16, at least 64; then nine additions)."""
+    """The float product at the edges of its row counts, strips, tiles and groups of k, rows that start on 16 bytes and rows that
+    do not: one order of additions, so a row's bits are those it has alone; and every element well within the worst case of a
+    chain over k, k 2^-24 sum |a w| (the roundings of a long chain go both ways: an eighth of that from k = 600 on)."""
     k = kernels(torch.float32)
     rows = 300 if n < 5000 else 70
     a, w = rnd((rows, kk), torch.float32, 21), rnd((n, kk), torch.float32, 22)
@@ -235,6 +234,30 @@ def test_gemm_float_edges(n, kk):
     out = torch.empty((rows, n), device="cuda")
     k.gemm(shifted, w, out)
     assert torch.equal(out, whole)
+
+
+@pytest.mark.parametrize("m,n,kk", [(1, 16, 4), (1, 1, 1), (5, 40, 1028), (16, 33, 127), (9, 12400, 260), (33, 5200, 132), (70, 3300, 516),
+                                    (32, 20000, 68), (130, 5000, 132), (2048, 4096, 36), (2048, 4090, 31)])
+def test_gemm_float_is_one_chain_over_k(m, n, kk):
+    """Every element of the float product is fmaf after fmaf from k = 0 up, to the bit, in every kernel and tile (a sampled token
+    lies within the last bits of a product now and then, so the order is part of the result).  Factors are whole numbers below
+    128 times 2^-3 .. 2^3: products and their sums up to 2^21 (k below 2^11) are whole multiples of 2^-6 and exact in 64 bits, so
+    that rounding such a sum to 32 bits is what fmaf does."""
+    k = kernels(torch.float32)
+    g = torch.Generator("cuda").manual_seed(m + n + kk)
+
+    def coarse(*shape):
+        return torch.randint(-127, 128, shape, generator=g, device="cuda").float() * 2.0 ** torch.randint(-3, 4, shape, generator=g, device="cuda")
+    a, w = coarse(m, kk), coarse(n, kk)
+    want = torch.zeros((m, n), device="cuda")
+    for i in range(kk):
+        want = (want.double() + a[:, i, None].double() * w[None, :, i].double()).float()
+    assert kk < 64 or not torch.equal(want, (a.double() @ w.double().T).float())      # (the chain's roundings are to be seen)
+    shifted = torch.empty(m * kk + 1, device="cuda")[1:].view(m, kk).copy_(a)      # rows 4 bytes off
+    for rows in (a, shifted):
+        out = torch.full((m, n), float("nan"), device="cuda")
+        k.gemm(rows, w, out)
+        assert torch.equal(out, want)
 
 
 @pytest.mark.parametrize("shape", [0, 1, 2, 3])
