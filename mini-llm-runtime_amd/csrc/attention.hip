@@ -237,25 +237,27 @@ __global__ __launch_bounds__(64) void attention_combine_kernel(AttnArgs a) {
 }
 
 #if !MLR_BF16
-// The float engine's attention on v_mfma_f32_16x16x4_f32 (32-bit products and sums) for head sizes and pages that are
-// multiples of 16 and up to 16 query heads a kv head.  A workgroup serves 16 columns -- consecutive tokens of one request
-// times the query heads of one kv head -- which share what it reads of keys and values; the kernel above, one token a
-// workgroup, fetches every value of a channel from a cache line of its own (16 heads on 8 of 128 channels, pages of 16: 111 us for
-// eight tokens behind 400 keys, 306 behind 4000, 0.68 ms for a prompt of 400 and 16.7 for one of 2048; here 19, 63, 53 us
-// and 0.57 ms).  Groups are found by the kernel: a row leads one when it is a multiple of the tokens a group holds or does
-// not continue the row before it.
+// The float engine's attention on v_mfma_f32_16x16x4_f32 (which rounds as four fmaf one behind the other in the order of its
+// k-slots) for head sizes and pages that are multiples of 16 and up to 16 query heads a kv head: every sum of the kernel above
+// in its order, so the same bits.  A workgroup serves 16 columns -- consecutive tokens of one request times the query heads of
+// one kv head -- which share what it reads of keys and values; the kernel above, one token a workgroup, fetches every value of a
+// channel from a cache line of its own (16 heads on 8 of 128 channels, pages of 16: 111 us for eight tokens behind 400 keys, 306
+// behind 4000, 0.68 ms for a prompt of 400 and 16.7 for one of 2048; here 27, 76, 62 us and 0.69 ms, and with tiles of 16 keys,
+// whose sums are other ones, 17, 62, 53 us and 0.59 ms).  Groups are found by the kernel: a row leads one when it is a multiple
+// of the tokens a group holds or does not continue the row before it.
 //
-// Keys are walked in tiles of 16 at absolute multiples of 16, wavefront w the tiles t with t % 4 == w, their partial
-// results merged in the order 0..3; a tile that a column does not see changes nothing of it.  A column's sums and their
-// order follow from its own position alone, whatever stands beside it.  Per tile: scores^T = K . Q^T (a lane holds four
-// channels of a key's row and of a query's: one 16-byte load each), softmax with a running maximum, out^T += V^T . P^T,
-// whose operand P lies in the registers as the first product leaves it (a lane: keys 4 (lane / 16) + i of column
-// lane % 16) and whose V is four keys of a channel, side by side in the transposed page.
+// Keys are walked in tiles of 64 at absolute multiples of 64.  Per tile: wavefront w takes the scores of keys 16 w ..,
+// scores^T = K . Q^T, a chain over up to 128 channels a time; they meet in LDS, where 16 threads a column take the running
+// maximum and sum (a sum over keys is a tree: keys 32 apart, 16, 8, 4, 2, 1); then wavefront w takes the 16-channel blocks w,
+// w + 4, ..: out^T += V^T . P^T, a chain over the 64 keys.  A tile that a column does not see changes nothing of it.
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 
+#define F32_PITCH 68           // floats between columns of the scores in LDS: 64 lanes' reads meet every bank once
+
 template <int NC, bool EXACT>
-__global__ __launch_bounds__(256, NC <= 4 ? 3 : NC <= 8 ? 2 : 1) void attention_f32_kernel(AttnArgs a, int rows) {
-    extern __shared__ __attribute__((aligned(16))) float lds[];              // [4][D][17], maxima [4][16], sums [4][16]
+__global__ __launch_bounds__(256, NC <= 8 ? 2 : 1) void attention_f32_kernel(AttnArgs a, int rows) {
+    __shared__ __attribute__((aligned(16))) float p_lds[2][16 * F32_PITCH];
+    __shared__ float corr_lds[2][16], sum_lds[16];
     const int D = EXACT ? NC * 16 : a.head_dim, nc = EXACT ? NC : a.head_dim / 16, P = a.page_size;
     const int g = a.q_heads / a.kv_heads, per = max(1, 16 / g);
     // the rows that lead whatever stands before them come first, a prompt's last and longest in front, the others behind:
@@ -274,165 +276,183 @@ __global__ __launch_bounds__(256, NC <= 4 ? 3 : NC <= 8 ? 2 : 1) void attention_
         if (lo >= hi) return;                                                // (no token of the group reads this part)
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, b4 = (lane >> 4) * 4;
-    const int tok = min(c / g, ntok - 1), head = kvh * g + c % g, pos = pos0 + tok;
-    const int from = a.window > 0 ? max(0, pos - a.window + 1) : 0;          // this column sees keys from .. pos
+    const int tok = min(c / g, ntok - 1), head = kvh * g + c % g;
+    // the column and the places of a tile (j, j + 16, j + 32, j + 48) that this thread takes part in the softmax with
+    const int col = threadIdx.x >> 4, j = threadIdx.x & 15, pos = pos0 + min(col / g, ntok - 1);
+    const int from = max(lo, a.window > 0 ? pos - a.window + 1 : 0), until = min(hi, pos + 1);       // it sees keys from .. until - 1
 
     floatx4 q[NC];
     const float* qr = a.q + ((size_t)(m + tok) * a.q_heads + head) * D + b4;
 #pragma unroll
-    for (int i = 0; i < NC; ++i) q[i] = EXACT || i < nc ? *reinterpret_cast<const floatx4*>(qr + i * 16) : floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < NC; ++i) q[i] = EXACT || i < nc ? turned(*reinterpret_cast<const floatx4*>(qr + i * 16)) : floatx4{0.f, 0.f, 0.f, 0.f};
 
-    const int t_end = (hi + 15) / 16, t_first = lo / 16 + ((wave - lo / 16) & 3);
+    constexpr int NV = (NC + 3) / 4;                                         // blocks of 16 channels of a wavefront
+    const int t_first = lo / 64, t_end = (hi + 63) / 64;
     const int32_t* table = a.block_table + (size_t)slot * a.max_blocks;
-    int pages = -1;                                                          // lane i: page of the wavefront's tile i of 64
-    floatx4 k[NC], v[NC];
-    auto load_k = [&](int t, int page) {
-        const float* kr = a.k_pages + ((long long)max(page, 0) * a.kv_heads + kvh) * P * D + (size_t)(t * 16 % P + c) * D + b4;
+    int pages = -1;                                                          // lane i: page of the i-th 16 keys of the next 16 tiles
+    auto load_pages = [&](int t) {
+        const int block = (t * 64 + lane * 16) / P;
+        pages = t * 64 + lane * 16 < hi && block < a.max_blocks ? table[block] : -1;
+    };
+    floatx4 k[NC], v[NV][4];
+    auto load_k = [&](int t) {
+        const int page = __shfl(pages, ((t - t_first) & 15) * 4 + wave), at = (t * 64 + wave * 16) % P;
+        const float* kr = a.k_pages + ((long long)max(page, 0) * a.kv_heads + kvh) * P * D + (size_t)(at + c) * D + b4;
 #pragma unroll
         for (int i = 0; i < NC; ++i)
             if (EXACT || i < nc) k[i] = *reinterpret_cast<const floatx4*>(kr + i * 16);
     };
-    auto load_v = [&](int t, int page) {
-        const float* vr = a.v_pages + ((long long)max(page, 0) * a.kv_heads + kvh) * P * D + (size_t)c * P + t * 16 % P + b4;
+    auto load_v = [&](int t) {
 #pragma unroll
-        for (int i = 0; i < NC; ++i)
-            if (EXACT || i < nc) v[i] = *reinterpret_cast<const floatx4*>(vr + (size_t)i * 16 * P);
+        for (int s = 0; s < 4; ++s) {
+            const int page = __shfl(pages, ((t - t_first) & 15) * 4 + s), at = (t * 64 + s * 16) % P;
+            const float* vr = a.v_pages + ((long long)max(page, 0) * a.kv_heads + kvh) * P * D + (size_t)c * P + at + b4;
+#pragma unroll
+            for (int i = 0; i < NV; ++i)
+                if (wave + 4 * i < nc) v[i][s] = *reinterpret_cast<const floatx4*>(vr + (size_t)(wave + 4 * i) * 16 * P);
+        }
     };
     float run_max = -INFINITY, run_sum = 0.f;
-    floatx4 acc[NC];
+    floatx4 acc[NV];
 #pragma unroll
-    for (int i = 0; i < NC; ++i) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
-    for (int t0 = t_first; t0 < t_end; t0 += 256) {                          // 64 tiles of the wavefront at a time
-        const int block = (t0 + 4 * lane) * 16 / P;
-        pages = t0 + 4 * lane < t_end && block < a.max_blocks ? table[block] : -1;
-        const int n = min(64, (t_end - t0 + 3) / 4);
-        int page = __shfl(pages, 0);
-        load_k(t0, page);
-        load_v(t0, page);
-        for (int n_t = 0; n_t < n; ++n_t) {
-            const int t = t0 + 4 * n_t, key0 = t * 16 + b4, next_page = __shfl(pages, min(n_t + 1, n - 1));
+    for (int i = 0; i < NV; ++i) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    load_pages(t_first);
+    load_k(t_first);
+    load_v(t_first);
+    for (int t = t_first; t < t_end; ++t) {
+        const int buf = t & 1, nth = ((t - t_first) & 15) * 4;
+        floatx4 score = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i0 = 0; i0 < NC; i0 += DIM_CHUNK / 16) {
             floatx4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int i = 0; i < NC; ++i)
+            for (int i = i0; i < NC && i < i0 + DIM_CHUNK / 16; ++i)
                 if (EXACT || i < nc) {
+                    const floatx4 kt = turned(k[i]);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i][e], q[i][e], s, 0, 0, 0);
+                    for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(kt[e], q[i][e], s, 0, 0, 0);
                 }
-            // (the next tile's keys are on their way from here on, its values from the end of this turn on: each into the
-            // registers that are free then)
-            if (n_t + 1 < n) load_k(t + 4, next_page);
-            float p[4], top = -INFINITY;
-            bool seen[4];
+            if (i0 == 0) score = s;
+            else if (EXACT || i0 < nc) score += s;
+        }
+        *reinterpret_cast<floatx4*>(&p_lds[buf][c * F32_PITCH + wave * 16 + b4]) = score;
+        int seen_page[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                seen[i] = page >= 0 && key0 + i >= from && key0 + i <= pos;
-                p[i] = seen[i] ? s[i] * a.scale : -INFINITY;
-                top = fmaxf(top, p[i]);
-            }
-            top = fmaxf(top, __shfl_xor(top, 16));
-            top = fmaxf(top, __shfl_xor(top, 32));
-            const float new_max = fmaxf(run_max, top);
-            const float corr = new_max > -INFINITY ? expf(run_max - new_max) : 1.f;
-            float sum = 0.f;
+        for (int i = 0; i < 4; ++i) seen_page[i] = __shfl(pages, nth + i);
+        // (the next tile's keys are on their way from here on, its values from the end of this turn on: each into the
+        // registers that are free then)
+        const bool more = t + 1 < t_end;
+        if (more && nth == 60) load_pages(t + 1);
+        if (more) load_k(t + 1);
+        __syncthreads();
+        float p[4], top = -INFINITY;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                // (a score that is not a number stays one where nothing else sets the maximum: pages that nobody wrote show)
-                p[i] = seen[i] && new_max > -INFINITY ? expf(p[i] - new_max) : p[i] != p[i] ? p[i] : 0.f;
-                sum += p[i];
-            }
-            sum += __shfl_xor(sum, 16);
-            sum += __shfl_xor(sum, 32);
-            run_sum = run_sum * corr + sum;
-            run_max = new_max;
+        for (int i = 0; i < 4; ++i) {
+            const int key = t * 64 + 16 * i + j;
+            const bool seen = seen_page[i] >= 0 && key >= from && key < until;
+            p[i] = seen ? p_lds[buf][col * F32_PITCH + 16 * i + j] * a.scale : -INFINITY;
+            top = fmaxf(top, p[i]);
+        }
 #pragma unroll
-            for (int i = 0; i < NC; ++i) acc[i] *= corr;
-            // Every token of the group sees the whole tile, or values that a token must not see would meet its probability
-            // of zero: places that were never written are cleared, and where a value is not finite the tokens go one by one.
-            const bool inner = page >= 0 && t * 16 + 15 <= pos0 && (a.window <= 0 || t * 16 > pos0 + ntok - 1 - a.window);
-            bool odd = false;
-            if (!inner) {
+        for (int d = 8; d > 0; d >>= 1) top = fmaxf(top, __shfl_xor(top, d));
+        const float new_max = fmaxf(run_max, top);
+        const float corr = new_max > -INFINITY ? expf(run_max - new_max) : 1.f;
 #pragma unroll
-                for (int i = 0; i < NC; ++i)
+        for (int i = 0; i < 4; ++i)
+            // (a score that is not a number stays one where nothing else sets the maximum: pages that nobody wrote show)
+            p[i] = p[i] != p[i] ? p[i] : new_max > -INFINITY ? expf(p[i] - new_max) : 0.f;
+        float sum = (p[0] + p[2]) + (p[1] + p[3]);
+#pragma unroll
+        for (int d = 8; d > 0; d >>= 1) sum += __shfl_xor(sum, d);
+        run_sum = run_sum * corr + sum;
+        run_max = new_max;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) p_lds[buf][col * F32_PITCH + 16 * i + j] = p[i];
+        if (j == 0) corr_lds[buf][col] = corr;
+        __syncthreads();
+        // Every token of the group sees the whole tile, or values that a token must not see would meet its probability
+        // of zero: places that were never written are cleared, and where a value is not finite the tokens go one by one.
+        const float scale_by = corr_lds[buf][c];
+        bool mapped = true;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) mapped = mapped && seen_page[s] >= 0;
+        const bool inner = mapped && t * 64 >= lo && t * 64 + 63 <= pos0 && (a.window <= 0 || t * 64 > pos0 + ntok - 1 - a.window);
+        bool odd = false;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            acc[i] *= scale_by;
+            if (wave + 4 * i >= nc) continue;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                if (!inner) {
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        if (page < 0 || key0 + e < lo || key0 + e >= hi) v[i][e] = 0.f;
-                        if (EXACT || i < nc) odd |= !(fabsf(v[i][e]) <= 3.402823466e38f);
-                    }
-            }
-            if (__builtin_expect(__any(odd), 0)) {
-                for (int other = 0; other < ntok; ++other) {
-                    const int own = pos0 + other, own_from = a.window > 0 ? max(0, own - a.window + 1) : 0;
-#pragma unroll
-                    for (int i = 0; i < NC; ++i) {
-                        floatx4 next = acc[i];
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            next = __builtin_amdgcn_mfma_f32_16x16x4f32(key0 + e >= own_from && key0 + e <= own ? v[i][e] : 0.f, p[e], next, 0, 0, 0);
-                        if (tok == other) acc[i] = next;
+                        const int key = t * 64 + s * 16 + b4 + e;
+                        if (seen_page[s] < 0 || key < lo || key >= hi) v[i][s][e] = 0.f;
+                        odd |= !(fabsf(v[i][s][e]) <= 3.402823466e38f);
                     }
                 }
-            } else {
-#pragma unroll
-                for (int i = 0; i < NC; ++i)
-                    if (EXACT || i < nc) {
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i][e], p[e], acc[i], 0, 0, 0);
-                    }
+                v[i][s] = turned(v[i][s]);                                   // element e: the key 16 s + 4 e + lane / 16
             }
-            if (n_t + 1 < n) load_v(t + 4, next_page);
-            page = next_page;
         }
-    }
-    // the four wavefronts' results, in the order 0..3
-    float* maxima = lds + 4 * D * 17;
-    float* sums = maxima + 64;
-    if (lane < 16) {
-        maxima[wave * 16 + c] = run_max;
-        sums[wave * 16 + c] = run_sum;
-    }
-    __syncthreads();
-    const float gmax = fmaxf(fmaxf(maxima[c], maxima[16 + c]), fmaxf(maxima[32 + c], maxima[48 + c]));
-    const float weight = run_max > -INFINITY ? expf(run_max - gmax) : run_sum;       // (no key: 0; none but NaN: NaN)
+        const float* pr = &p_lds[buf][c * F32_PITCH + (lane >> 4)];
+        if (__builtin_expect(__any(odd), 0)) {
+            for (int other = 0; other < ntok; ++other) {
+                const int own = pos0 + other, own_from = a.window > 0 ? max(0, own - a.window + 1) : 0;
 #pragma unroll
-    for (int i = 0; i < NC; ++i)
-        if (EXACT || i < nc) {
+                for (int i = 0; i < NV; ++i) {
+                    if (wave + 4 * i >= nc) continue;
+                    floatx4 next = acc[i];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) lds[(wave * D + i * 16 + b4 + e) * 17 + c] = weight * acc[i][e];
-        }
-    __syncthreads();
-    for (int i = threadIdx.x; i < ntok * g * D; i += 256) {
-        const int col = i / D, d = i % D;
-        float num = 0.f, den = 0.f, most = -INFINITY;
+                    for (int s = 0; s < 4; ++s)
 #pragma unroll
-        for (int w = 0; w < 4; ++w) most = fmaxf(most, maxima[w * 16 + col]);
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const float top = maxima[w * 16 + col];
-            num += lds[(w * D + d) * 17 + col];
-            den += top > -INFINITY ? expf(top - most) * sums[w * 16 + col] : sums[w * 16 + col];
-        }
-        const size_t row = (size_t)(m + col / g) * a.q_heads + kvh * g + col % g;
-        if (a.max_splits > 1) {
-            float* dst = a.partial + (row * a.max_splits + split) * (D + 2);
-            dst[d] = num;
-            if (d == 0) {
-                dst[D] = most;
-                dst[D + 1] = den;
+                        for (int e = 0; e < 4; ++e) {
+                            const int key = t * 64 + 16 * s + 4 * e + (lane >> 4);
+                            next = __builtin_amdgcn_mfma_f32_16x16x4f32(key >= own_from && key <= own ? v[i][s][e] : 0.f, pr[16 * s + 4 * e], next, 0, 0, 0);
+                        }
+                    if (tok == other) acc[i] = next;
+                }
             }
         } else {
-            a.out[row * D + d] = den != 0.f ? num / den : 0.f;
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float prob = pr[16 * s + 4 * e];
+#pragma unroll
+                    for (int i = 0; i < NV; ++i)
+                        if (wave + 4 * i < nc) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i][s][e], prob, acc[i], 0, 0, 0);
+                }
+        }
+        if (more) load_v(t + 1);
+    }
+    if (j == 0) sum_lds[col] = run_sum;
+    const bool split_up = a.max_splits > 1;
+    if (split_up && j == 0 && col < ntok * g) {
+        float* dst = a.partial + (((size_t)(m + col / g) * a.q_heads + kvh * g + col % g) * a.max_splits + split) * (D + 2);
+        dst[D] = run_max;
+        dst[D + 1] = run_sum;
+    }
+    __syncthreads();
+    if (c >= ntok * g) return;
+    const size_t row = (size_t)(m + tok) * a.q_heads + head;
+    const float den = sum_lds[c];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        if (wave + 4 * i >= nc) continue;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int d = (wave + 4 * i) * 16 + b4 + e;
+            if (split_up) a.partial[(row * a.max_splits + split) * (D + 2) + d] = acc[i][e];
+            else a.out[row * D + d] = den != 0.f ? acc[i][e] / den : 0.f;
         }
     }
 }
 
 template <int NC, bool EXACT>
 static int launch_attention_f32(const AttnArgs& a, int rows, hipStream_t stream) {
-    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_f32_kernel<NC, EXACT>),
-                                                          hipFuncAttributeMaxDynamicSharedMemorySize, (4 * NC * 16 * 17 + 128) * 4);
-    if (allowed != hipSuccess) return (int)allowed;
     const int per = max(1, 16 / (a.q_heads / a.kv_heads)), blocks = (rows + per - 1) / per;
-    attention_f32_kernel<NC, EXACT><<<dim3(blocks * per, a.kv_heads, a.max_splits), 256, (4 * a.head_dim * 17 + 128) * sizeof(float), stream>>>(
-        a, rows);
+    attention_f32_kernel<NC, EXACT><<<dim3(blocks * per, a.kv_heads, a.max_splits), 256, 0, stream>>>(a, rows);
     return (int)hipGetLastError();
 }
 #endif

@@ -63,6 +63,27 @@ __device__ __forceinline__ float turn_y(float a, float b, float c, float s) { re
 // a^2 + b^2, to be added to a running sum
 __device__ __forceinline__ float squares(float a, float b) { return opaque(__builtin_fmaf(a, a, opaque(b * b))); }
 
+// Four floats a lane: register i of lane block b (lanes 16 b ..) becomes what register b of block i was, so that four
+// neighbouring places of a row become the places 4 i + b, which is what a 16x16x4 matrix instruction wants.
+template <typename V> __device__ __forceinline__ V turned(const V& v) {
+    unsigned r[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = __float_as_uint(v[i]);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const auto x = __builtin_amdgcn_permlane32_swap(r[i], r[i + 2], false, false);
+        r[i] = x[0];
+        r[i + 2] = x[1];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i += 2) {
+        const auto x = __builtin_amdgcn_permlane16_swap(r[i], r[i + 1], false, false);
+        r[i] = x[0];
+        r[i + 1] = x[1];
+    }
+    return V{__uint_as_float(r[0]), __uint_as_float(r[1]), __uint_as_float(r[2]), __uint_as_float(r[3])};
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, MLR_WAVE);

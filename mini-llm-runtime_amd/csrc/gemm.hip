@@ -16,28 +16,8 @@
 // v_mfma_f32_16x16x4_f32 rounds as four fmaf one behind the other in the order of its k-slots, so an element is ONE chain of
 // fmaf over k from 0 up, whatever kernel and tile serve it: its bits hang neither on the rows beside it nor on how a step was
 // cut, and a plain loop over k gives the same.  A matrix instruction wants k-slot b from lanes 16 b ..; a 16-byte load gives a
-// lane four neighbouring k of one row, so four lane blocks exchange: `turned` makes register i of block b what register b of
-// block i was, and product i of a group of 16 then takes k = 4 i + b.
+// lane four neighbouring k of one row, so four lane blocks exchange (`turned`): product i of a group of 16 takes k = 4 i + b.
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
-
-__device__ __forceinline__ floatx4 turned(const floatx4& v) {
-    unsigned r[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) r[i] = __float_as_uint(v[i]);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const auto x = __builtin_amdgcn_permlane32_swap(r[i], r[i + 2], false, false);
-        r[i] = x[0];
-        r[i + 2] = x[1];
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i += 2) {
-        const auto x = __builtin_amdgcn_permlane16_swap(r[i], r[i + 1], false, false);
-        r[i] = x[0];
-        r[i + 1] = x[1];
-    }
-    return floatx4{__uint_as_float(r[0]), __uint_as_float(r[1]), __uint_as_float(r[2]), __uint_as_float(r[3])};
-}
 
 // Four consecutive k of a row from k on, zeros from K on (VEC: rows start on 16 bytes and K is a multiple of four).
 template <bool VEC>

@@ -624,6 +624,37 @@ def test_paged_attention_float_rows_alone(hq, hkv, d, page, window, split_keys):
         v_pages[at // page, :, :, at % page] = kept
 
 
+@pytest.mark.parametrize("hq,hkv,d,page,window,split_keys", [(16, 8, 128, 16, None, 256), (16, 1, 128, 32, 100, 64), (7, 1, 16, 16, None, 0),
+                                                             (10, 2, 80, 48, 20, 128), (3, 3, 144, 16, None, 64), (6, 2, 256, 128, 300, 0),
+                                                             (5, 1, 192, 64, 1, 64), (8, 2, 64, 16, None, 0)])
+def test_paged_attention_float_has_the_general_kernels_bits(hq, hkv, d, page, window, split_keys):
+    """Tokens that share a workgroup on the matrix instructions get, to the bit, what the kernel of one token a workgroup gives them
+    (reached by queries that do not start on 16 bytes): prompts, single tokens and portions of several requests, in and out of
+    order, with pages that end inside a tile."""
+    k = kernels(torch.float32)
+    lengths, portions = [1, 63, 200, 517, 385], [1, 63, 1, 130, 17]
+    blocks = [-(-n // page) for n in lengths]
+    order = torch.randperm(sum(blocks), generator=torch.Generator().manual_seed(d)).int()
+    k_pages, v_pages = rnd((sum(blocks), hkv, page, d), torch.float32, 50), rnd((sum(blocks), hkv, d, page), torch.float32, 51)
+    table = torch.full((len(lengths), max(blocks) + 1), -1, dtype=torch.int32)
+    for i, n in enumerate(blocks):
+        table[i, :n] = order[sum(blocks[:i]):sum(blocks[:i]) + n]
+    rows = [(i, p) for i, (n, m) in enumerate(zip(lengths, portions)) for p in range(n - m, n)]
+    splits = -(-max(lengths) // split_keys) if split_keys else 1
+    q = rnd((len(rows), hq * d), torch.float32, 52) * 2
+    for picked in (list(range(len(rows))), list(range(len(rows)))[::-1], list(range(0, len(rows), 3))):
+        partial = torch.full((k.attention_partial_numel(len(picked), hq, d, splits),), float("nan"), device="cuda") if split_keys else None
+        got = []
+        for spare in (0, 1):
+            queries = torch.empty(len(picked) * hq * d + spare, device="cuda")[spare:].view(len(picked), hq * d).copy_(q[picked])
+            out = torch.full_like(queries, float("nan"))
+            k.paged_attention(queries, k_pages, v_pages, table.cuda(), torch.tensor([rows[i][0] for i in picked], dtype=torch.int32, device="cuda"),
+                              torch.tensor([rows[i][1] for i in picked], dtype=torch.int32, device="cuda"), out, hq, hkv, d, page,
+                              d ** -0.5, window=window, split_keys=split_keys, max_splits=splits, partial=partial)
+            got.append(out)
+        assert torch.equal(got[0], got[1])
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_attention_finds_one_far_key(dtype):
     """One key among a thousand matches the query (scaled so that its score stands out): the
