@@ -839,9 +839,11 @@ template <int VEC> __device__ __forceinline__ void store_elems(elem_t* p, const 
 //   acc != null: acc[src] += y (the float residual stream takes a sublayer's normed output), and with
 //     cast != null also cast[src] = T(acc[src]): the stream as the next sublayer's input;
 //   else out[r] = T(y).
-// One workgroup a row, VEC values an access; the row is read once and kept in registers where it fits (4096 values), else
-// read again.  1777 rows of 2048 values: 17 us one value at a time, 9.8 with four.
-#define LN_REGS 16
+// One workgroup a row, VEC values an access.  Thread t adds up the values t, t + 256, .. of the row, however it was read: a
+// router behind the norm turns on the last bits of it, so the order of the sum is part of the result.  A row of up to LN_ROW
+// values is read once, with VEC 4 through LDS; a longer one is read again for each sum, a value at a time.  1777 rows of 2048
+// values: 12.0 us one value at a time, 9.7 with four.
+#define LN_ROW 4096
 template <int VEC>
 __global__ __launch_bounds__(256) void layernorm_kernel(const elem_t* __restrict__ xe, const float* __restrict__ xf,
                                                         const float* __restrict__ weight, const float* __restrict__ bias,
@@ -849,43 +851,58 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const elem_t* __restrict
                                                         elem_t* __restrict__ cast, elem_t* __restrict__ out, int width,
                                                         float eps, float out_scale) {
     __shared__ float scratch[16];
+    __shared__ __attribute__((aligned(16))) float row[VEC > 1 ? LN_ROW : 1];
+    constexpr int HELD = LN_ROW / 256;
     const int r = blockIdx.x;
     const size_t src = rows ? (size_t)rows[r] : (size_t)r;
-    const bool kept = width <= LN_REGS * 256;
-    float x[LN_REGS / VEC][VEC];
+    const bool kept = width <= LN_ROW;
+    float x[HELD / VEC][VEC];                              // the thread's places as it reads and writes them
     auto read = [&](int c, float* v) {
         if (xe) load_elems<VEC>(xe + src * width + c, v);
         else load_floats<VEC>(xf + src * width + c, v);
     };
-    // `each` for every place of the row that this thread holds
-    auto walk = [&](auto each) {
-        if (kept) {
+    if (kept) {
 #pragma unroll
-            for (int j = 0; j < LN_REGS / VEC; ++j) {
-                const int c = (threadIdx.x + j * 256) * VEC;
-                if (c < width) each(c, x[j]);
-            }
-        } else {
-            for (int c = threadIdx.x * VEC; c < width; c += 256 * VEC) {
-                read(c, x[0]);
-                each(c, x[0]);
-            }
+        for (int j = 0; j < HELD / VEC; ++j) {
+            const int c = (threadIdx.x + j * 256) * VEC;
+            if (c < width) read(c, x[j]);
         }
-    };
-    float sum = 0.f;
-    if (kept) walk([&](int c, float* v) { read(c, v); });
-    walk([&](int, const float* v) {
+        if (VEC > 1) {
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) sum += v[e];
-    });
+            for (int j = 0; j < HELD / VEC; ++j) {
+                const int c = (threadIdx.x + j * 256) * VEC;
+                if (c < width) store_floats<VEC>(row + c, x[j]);
+            }
+            __syncthreads();
+        }
+    }
+    auto value = [&](int c) { return xe ? to_float(xe[src * width + c]) : xf[src * width + c]; };
+    float mine[HELD], sum = 0.f, dev = 0.f;                // the values that the thread adds up
+    if (kept) {
+#pragma unroll
+        for (int j = 0; j < HELD; ++j) {
+            const int c = threadIdx.x + j * 256;
+            mine[j] = c < width ? (VEC > 1 ? row[c] : x[j][0]) : 0.f;
+            sum += mine[j];
+        }
+    } else {
+        for (int c = threadIdx.x; c < width; c += 256) sum += value(c);
+    }
     const float mean = block_sum(sum, scratch) / (float)width;
-    float dev = 0.f;
-    walk([&](int, const float* v) {
+    if (kept) {
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) dev += (v[e] - mean) * (v[e] - mean);
-    });
+        for (int j = 0; j < HELD; ++j) mine[j] = threadIdx.x + j * 256 < width ? mine[j] - mean : 0.f;
+        dev = squares(mine[0], mine[1]);
+#pragma unroll
+        for (int j = 2; j < HELD; ++j) dev = __builtin_fmaf(mine[j], mine[j], dev);
+    } else {
+        for (int c = threadIdx.x; c < width; c += 256) {
+            const float d = value(c) - mean;
+            dev = __builtin_fmaf(d, d, dev);
+        }
+    }
     const float inv = 1.0f / sqrtf(block_sum(dev, scratch) / (float)width + eps);
-    walk([&](int c, const float* v) {
+    auto finish = [&](int c, const float* v) {
         float y[VEC], w[VEC], b[VEC];
         load_floats<VEC>(weight + c, w);
         if (bias) load_floats<VEC>(bias + c, b);
@@ -901,7 +918,19 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const elem_t* __restrict
         for (int e = 0; e < VEC; ++e) h[e] += y[e];
         store_floats<VEC>(acc + src * width + c, h);
         if (cast != nullptr) store_elems<VEC>(cast + src * width + c, h);
-    });
+    };
+    if (kept) {
+#pragma unroll
+        for (int j = 0; j < HELD / VEC; ++j) {
+            const int c = (threadIdx.x + j * 256) * VEC;
+            if (c < width) finish(c, x[j]);
+        }
+    } else {
+        for (int c = threadIdx.x * VEC; c < width; c += 256 * VEC) {
+            read(c, x[0]);
+            finish(c, x[0]);
+        }
+    }
 }
 
 // The activation of a feed-forward without a gate, element by element (32-bit): ACT 0 relu(x)^2; ACT 1 the exact gelu,
@@ -1368,7 +1397,7 @@ int mlr_layernorm(const void* xe, const float* xf, const float* weight, const fl
     if (n_out <= 0) return 0;
     if ((xe == nullptr) == (xf == nullptr) || (acc == nullptr && out == nullptr) || (acc != nullptr && rows != nullptr))
         return -1;
-    if (width % 4 == 0 && aligned16(xe, xf, weight, bias, acc, cast, out))
+    if (width % 4 == 0 && width <= LN_ROW && aligned16(xe, xf, weight, bias, acc, cast, out))
         layernorm_kernel<4><<<n_out, 256, 0, stream>>>((const elem_t*)xe, xf, weight, bias, rows, acc, (elem_t*)cast,
                                                        (elem_t*)out, width, eps, out_scale);
     else

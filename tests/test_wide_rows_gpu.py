@@ -88,6 +88,28 @@ def test_layer_norm_of_wide_rows(dtype, width):
         assert torch.equal(cast, h.to(dtype))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("width", [4, 260, 1000, 1028, 2048, 4096, 4100])
+def test_layer_norm_of_wide_rows_adds_up_in_the_same_order(dtype, width):
+    """A router behind the norm turns on its last bits: four values an access and one give the same ones, added to the float
+    stream, cast beside it, and as the final norm's rows."""
+    k = kernels(dtype)
+    gen = torch.Generator("cuda").manual_seed(width)
+    rows = 70
+    x = (torch.randn(rows, width, generator=gen, device="cuda") * 3 + 1).to(dtype)
+    h0 = torch.randn(rows, width, generator=gen, device="cuda")
+    w, b = (torch.randn(width, generator=gen, device="cuda") for _ in range(2))
+    picked = ints([5, 0, 69, 33])
+    for bias in (b, None):
+        got = []
+        for weight in (w, moved(w)):
+            h, cast, out = h0.clone(), torch.empty_like(x), torch.empty(4, width, dtype=dtype, device="cuda")
+            k.layernorm_add(x, weight, bias, h, cast=cast, eps=1e-5)
+            k.layernorm_rows(h0, weight, bias, out, 1e-5, rows=picked)
+            got.append((h, cast, out))
+        assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
 @pytest.mark.parametrize("rows,heads,keys", [(1, 3, 7), (300, 8, 128), (2, 1100, 256)])
 def test_decay_per_channel(rows, heads, keys):
     k = kernels(torch.bfloat16)
