@@ -135,6 +135,7 @@ class StepContext:
         self.fixed_groups = None      # a captured step's groups: {key: token_groups' result}, in tensors of their own
         self.status = None            # device int32 [2] when the hidden state is to be checked after every layer
         self.partial_budget = None    # floats that split attention's partial results may take (the memory plan's)
+        self.routed = False           # the model chooses among experts (`DecoderModel.routes`)
 
     def begin_step(self):
         self._groups = {}

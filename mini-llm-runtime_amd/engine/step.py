@@ -132,6 +132,7 @@ class Runner:
         self.ctx = StepContext(self.kernels, self.cache, self.workspace, self.dtype, self.max_length,
                                split_keys, split_max_tokens)
         self.ctx.target_workgroups = target_workgroups
+        self.ctx.routed = model.routes()
         # split attention keeps its partial results within what was planned for them
         self.ctx.partial_budget = workspace_plan.get(("attn_partial", torch.float32))
         self.ctx.status = self._status if self.check_finite else None

@@ -142,6 +142,7 @@ class DecoderModel:
         at most `logits_rows` wanted places asks for: the final norm's rows here, the rest from the parts that
         state theirs (the ends: `workspace_plan(rows, logits_rows, dtype, limits)`; blocks and their parts:
         `workspace_plan(rows, dtype, limits)`; a part without one gets its buffers on demand)."""
+        limits = dict(limits, routed=self.routes())
         plan = {("final", self.dtype): logits_rows * self.spec.hidden}
         if any(run.add_embedding for run in self.spec.schedule):
             plan[("embedding_copy", torch.float32)] = rows * self.spec.hidden
@@ -163,6 +164,11 @@ class DecoderModel:
         return all(getattr(part, "graph_safe", False) for block in self.blocks
                    for part in [block, *block.parts().values()]) and all(getattr(part, "graph_safe", False)
                                                                          for part in self._ends())
+
+    def routes(self):
+        """True when a layer chooses among experts.  Such a choice is no continuous function of what comes before it: where
+        two experts lie within rounding, sums in another order pick the other one, and the token's row changes by percents."""
+        return any(getattr(part, "routes", False) for block in self.blocks for part in block.parts().values())
 
     def weight_bytes(self):
         """Bytes of the tensors the model uses (each once; without the padding between them)."""

@@ -27,6 +27,7 @@ from .registry import PartError, build_part, register_part
 @register_part("ffn", "routed_mlp")
 class RoutedMlp:
     graph_safe = True
+    routes = True                 # (see `DecoderModel.routes`)
 
     def __init__(self, spec):
         s = self.spec = spec

@@ -49,6 +49,14 @@ def _rope_table(position, ctx, device, rot_limit):
     return rotation.table, bool(rotation.interleaved)
 
 
+# Prompt portions of a model with a router keep the 64-column kernel and, in latent attention, the queries moved into the
+# latent space, in both of which the sums of a row are rounded as they always were.  The portion kernel and made keys are no
+# less precise (against 64 bits the median row of 640 is off by 0.26 % either way) but round elsewhere, and then other tokens
+# are the ones whose choice of experts lies within rounding: of 640 scored rows of 1777-token prompts 6 had another choice than
+# 64 bits, with portions 8, with either of the two alone 5 and 6, and only some of them the same.  Such a row's logits differ
+# by a third, so a prompt would be scored otherwise than before.  (That prompt in 8 layers of 2048 channels: 3.82 ms, with
+# portions 2.47.)
+#
 # Portions of latent attention that make keys and values of their own: from this many tokens and keys on (16 heads, rank
 # 512, a step of eight layers of which two are latent attention, made against moved: 32 tokens behind 1000 keys 1.92 ms
 # against 2.02, behind 4000 2.10 against 3.01; without context 512 tokens 3.17 against 3.09, 2048 5.4 against 6.5), and up
@@ -128,8 +136,8 @@ def attend(ctx, q, k_pages, v_pages, view, sink, out, q_heads, kv_heads, key_dim
     if k.sink_tiles_supported(key_dim, value_dim, k_pages.shape[3], v_pages.shape[3], view.page_size, mask, mask_size,
                               ctx.max_positions, keep_first) and q.shape[1] % 8 == 0:
         big_heads, big_tokens, small_heads, small_tokens = k.sink_tiles_layout(q_heads, kv_heads)
-        portions = k.portion_attention_supported(q_heads, kv_heads, key_dim, value_dim, k_pages.shape[3], v_pages.shape[3], view.page_size,
-                                                 mask, mask_size, ctx.max_positions, keep_first)
+        portions = not ctx.routed and k.portion_attention_supported(q_heads, kv_heads, key_dim, value_dim, k_pages.shape[3], v_pages.shape[3], view.page_size,
+                                                                    mask, mask_size, ctx.max_positions, keep_first)
         if portions:
             columns, big_heads = portion_columns(ctx, q_heads), min(big_heads, 32)
             big_tokens = columns // big_heads
@@ -310,7 +318,8 @@ class LatentAttention:
         """Elements of `latent_out` for the longest portion that makes its keys (0: none of this runner's does): its place is
         free until the step's other rows come.  Without `limits["spare"]` no more than those other rows need."""
         s = self.spec
-        if dtype != torch.bfloat16 or (s.head_dim, s.rot_dim, s.value_dim) != (128, 64, 128) or s.rank % 8 != 0 or not limits.get("spare", True):
+        if dtype != torch.bfloat16 or (s.head_dim, s.rot_dim, s.value_dim) != (128, 64, 128) or s.rank % 8 != 0 or \
+                limits.get("routed", False) or not limits.get("spare", True):
             return 0
         most = limits["max_length"] if self.mask is None else min(limits["max_length"], self.mask_size + rows)
         return self._made(min(most, PORTION_KEYS) + 64)
@@ -335,7 +344,7 @@ class LatentAttention:
         rank 512, for rank * (head_dim + value_dim) products a key and head.  Not in a step that is to be captured: first
         key and number of keys would be fixed in the graph."""
         s = self.spec
-        if ctx.fixed_groups is not None or not ctx.kernels.latent_portions_supported(s.head_dim, s.rot_dim, s.value_dim, s.rank):
+        if ctx.routed or ctx.fixed_groups is not None or not ctx.kernels.latent_portions_supported(s.head_dim, s.rot_dim, s.value_dim, s.rank):
             return []
         out, room = [], ctx.workspace.room("latent_out", torch.bfloat16)
         for i, (_, row, n, p0) in enumerate(ctx.segments):

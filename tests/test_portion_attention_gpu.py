@@ -155,3 +155,37 @@ def test_latent_portions_of_a_model(tmp_path, window, monkeypatch):
         calls.clear()
         compare(run_steps(runner, whole(requests)), want, "bfloat16")
         assert bool(calls) == (runner is amply) or runner.workspace.room("latent_out", BF16) >= 64 * (48 + 64 + 512)
+
+
+def test_a_model_with_a_router_keeps_its_sums(tmp_path, monkeypatch):
+    """A choice of experts turns on the last bits where two lie within rounding: prompt portions of a model that makes such
+    choices keep the kernels whose order of rounding its results have always had, those of one that does not take the others."""
+    from helpers import compare, make_requests, plain_logits, run_steps, whole
+    from plain import pamunex_plain as P
+    from mini_llm_runtime_amd.config import config_from_dict
+    from mini_llm_runtime_amd.engine import Runner
+    from mini_llm_runtime_amd.kernels import Kernels
+    from mini_llm_runtime_amd.parts import DecoderModel
+    from mini_llm_runtime_amd.weights import write_random_model
+    monkeypatch.setattr("mini_llm_runtime_amd.parts.sink_attention.PORTION_LEAST_KEYS", 0)
+    calls = set()
+    for name in ("portion_attention", "portion_attention_split"):
+        original = getattr(Kernels, name)
+        monkeypatch.setattr(Kernels, name, lambda self, *a, name=name, original=original, **kw: calls.add(name) or original(self, *a, **kw))
+    requests = make_requests(97, [150, 64, 201], seed=2)
+    for routed in (False, True):
+        mlp = dict(kind="moe", expert=dict(ff=32), router=dict(experts=4, top=2)) if routed else dict(kind="dense", ff=64)
+        layers = [dict(type="latent_attention", mlp=None, mixer=dict(heads=2, dim=128, rot_dim=64, vdim=128, kv_rank=48, scale=192 ** -0.5,
+                                                                     rot=dict(dims=64, base=10000.0), mask=dict(size=100))),
+                  dict(type="attention", mlp=mlp, mixer=dict(heads=4, kv_heads=2, dim=128, vdim=128, scale=128 ** -0.5,
+                                                             rot=dict(dims=64, base=10000.0), mask=dict(size=100)))]
+        cfg = dict(architecture="Pamunex", vocab=97, width=64, norm=dict(eps=1e-5), logit_scale=1.0, layers=layers)
+        folder = str(tmp_path / f"model{routed}")
+        write_random_model(folder, config_from_dict(cfg), seed=3, matrix_std=0.12, norm_std=0.2)
+        runner = Runner(DecoderModel.load(folder, BF16), max_tokens=640, max_slots=4, max_length=256, max_batch_tokens=512, page_size=16)
+        calls.clear()
+        got = run_steps(runner, whole(requests))
+        assert calls == (set() if routed else {"portion_attention", "portion_attention_split"})
+        assert runner.workspace.unplanned_bytes() == 0
+        if not routed:
+            compare(got, plain_logits(P.PlainPamunex(folder), requests), "bfloat16")
