@@ -131,6 +131,7 @@ class StepContext:
         self.single_tokens = False    # every segment brings exactly one token (a decoding step)
         self.max_context = 0          # largest position + 1 among the step's tokens
         self._groups = {}
+        self._left_out = {}           # buffer of token groups without some entries -> the sets of entries it was asked without
         self._group_upload = None
         self.fixed_groups = None      # a captured step's groups: {key: token_groups' result}, in tensors of their own
         self.status = None            # device int32 [2] when the hidden state is to be checked after every layer
@@ -138,16 +139,18 @@ class StepContext:
         self.routed = False           # the model chooses among experts (`DecoderModel.routes`)
 
     def begin_step(self):
-        self._groups = {}
+        self._groups, self._left_out = {}, {}
         self.fixed_groups = None
 
-    def token_groups(self, tokens_per_group, big_factor=0, without=()):
+    def token_groups(self, tokens_per_group, big_factor=0, without=(), rest="rest"):
         """The step's rows cut into groups of consecutive tokens of one request, as device int32 vectors
         (first row of each group, tokens in each group) with their number.  Returns (small, big, (rows in
         small groups, one beyond the last batch row of a small group)): small groups hold at most
         `tokens_per_group` tokens; with big_factor > 0, a request that brings more than `tokens_per_group`
         tokens is cut into big groups of at most big_factor * tokens_per_group instead (prompt portions), else
-        `big` is empty.  `without`: entries of the step (their numbers, ascending) whose rows are left out."""
+        `big` is empty.  `without`: entries of the step (their numbers, ascending) whose rows are left out; `rest` then
+        ends the name of the buffer, for callers that leave out different entries of one step (a buffer asked again without
+        other entries gets another one beside it: what was handed out before stays as it is)."""
         key = (tokens_per_group, big_factor, without)
         hit = self._groups.get(key)
         if hit is not None:
@@ -176,8 +179,15 @@ class StepContext:
             # get a tensor of their own once (this is the eager run before the capture) and stay there
             dev = torch.tensor(first + count + big_first + big_count + [0], dtype=torch.int32, device=self.workspace.device)
         else:
-            rest = "_rest" if without else ""
-            dev = self.workspace.get(f"token_groups_{tokens_per_group}_{big_factor}{rest}", (2 * (g + gb),), torch.int32)
+            name = f"token_groups_{tokens_per_group}_{big_factor}"
+            if without:
+                name = f"{name}_{rest}"
+                sets = self._left_out.setdefault(name, [])
+                if without not in sets:
+                    sets.append(without)
+                if sets.index(without) > 0:
+                    name = f"{name}_{sets.index(without)}"
+            dev = self.workspace.get(name, (2 * (g + gb),), torch.int32)
             if self._group_upload is None:
                 self._group_upload = Uploader(4096, dev.device)
             self._group_upload.send(first + count + big_first + big_count, dev)

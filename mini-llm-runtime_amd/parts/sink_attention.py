@@ -127,8 +127,8 @@ def portion_columns(ctx, q_heads):
 
 
 def attend(ctx, q, k_pages, v_pages, view, sink, out, q_heads, kv_heads, key_dim, value_dim, scale, mask, mask_size,
-           keep_first=0, softcap=None, without=()):
-    """Every token of the step over the keys it sees (but those of the entries `without`).  The bfloat16 engine on the
+           keep_first=0, softcap=None, without=(), rest="rest"):
+    """Every token of the step over the keys it sees (but those of the entries `without`, see `token_groups`).  The bfloat16 engine on the
     matrix cores where they take the sizes (prompt portions in workgroups of 128 or 64 columns, single tokens and short
     portions in workgroups of 16 whose wavefronts share the value channels); else, and in the float engine, one wavefront
     a (token, head), whose sums follow from the token's position alone."""
@@ -141,7 +141,7 @@ def attend(ctx, q, k_pages, v_pages, view, sink, out, q_heads, kv_heads, key_dim
         if portions:
             columns, big_heads = portion_columns(ctx, q_heads), min(big_heads, 32)
             big_tokens = columns // big_heads
-        small, big, _ = ctx.token_groups(small_tokens, max(1, big_tokens // small_tokens), without)
+        small, big, _ = ctx.token_groups(small_tokens, max(1, big_tokens // small_tokens), without, rest)
         if portions and big[2] > 0:
             k.portion_attention(q, k_pages, v_pages, view.block_table, ctx.slots, ctx.positions, sink, out, *big, columns, big_heads,
                                 q_heads, kv_heads, key_dim, value_dim, view.page_size, scale, mask, mask_size, ctx.max_positions,
@@ -265,6 +265,8 @@ class LatentAttention:
         self.row = s.rank + s.rot_dim                    # a token's cache row, and a query head after the move
         self.o_width = s.heads * s.value_dim
         self.out_name = "mixer_out"
+        # what the choice of a step's entries that make their keys hangs on besides the step (see `_portions`)
+        self.rest = f"rest_{self.mask}_{self.mask_size}_{self._made(1)}"
         self.head_gate = getattr(s, "head_gate", None)
         if self.head_gate not in (None, "sigmoid"):
             raise PartError(f"head_gate {self.head_gate!r}: sigmoid or none")
@@ -327,7 +329,8 @@ class LatentAttention:
     def workspace_plan(self, rows, dtype, limits):
         s = self.spec
         groups = _groups_plan(rows, s.heads, 1, s.rank)
-        rest = {(f"{name}_rest", kind): count for (name, kind), count in groups.items() if name.startswith("token_groups")}
+        rest = {(f"{name}_{self.rest}", kind): count for (name, kind), count in groups.items()
+                if name.startswith("token_groups") and self._portions_planned(rows, dtype, limits) > 0}
         first = self.q_width if s.q_rank is None else s.q_rank
         more = {} if s.q_rank is None else {("latent_cq", dtype): rows * s.q_rank, ("latent_queries", dtype): rows * self.q_width}
         if self.head_gate is not None:
@@ -412,7 +415,7 @@ class LatentAttention:
         if rest:
             lat = ctx.workspace.get("latent_out", (m, s.heads * s.rank), x.dtype)
             attend(ctx, q, pages, pages, view, self.sink, lat, s.heads, 1, self.row, s.rank, float(s.scale), self.mask,
-                   self.mask_size, without=tuple(p[0] for p in portions))
+                   self.mask_size, without=tuple(p[0] for p in portions), rest=self.rest)
         for r0, r1 in rest:
             k.heads_gemm(lat.view(m, s.heads, s.rank)[r0:r1], self.uv, attn.view(m, s.heads, s.value_dim)[r0:r1])
         if gate is not None:

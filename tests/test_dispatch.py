@@ -51,6 +51,74 @@ def test_small_batches_over_long_contexts_are_split_and_short_ones_not():
     assert context(8192, split_keys=4096).attention_split(64, 64, 8, 16, 128, longest=65504)[:2] == (4096, 2)
 
 
+class HostUpload:
+    """`Uploader` without a GPU."""
+
+    def send(self, values, dst):
+        dst[:len(values)] = torch.tensor(values, dtype=torch.int32)
+
+
+def spelled(hit):
+    return [[v[:n].tolist() for v in (first, count)] for first, count, n in hit[:2]] + [hit[2]]
+
+
+def test_token_groups_that_leave_out_entries_keep_to_themselves():
+    """Layers that leave out different entries of one step: what one was handed is not overwritten by the other, and the first
+    one's is still there when a third layer leaves out what the first did."""
+    ctx = context(4096)
+    ctx.workspace.reserve({(f"token_groups_1_{factor}{rest}", torch.int32): 4000 for factor in (0, 4) for rest in ("", "_rest")})
+    ctx._group_upload = HostUpload()
+    ctx.segments = [(0, 0, 1, 900), (1, 1, 800, 2000), (2, 801, 400, 600), (3, 1201, 150, 0)]
+    want = lambda out: [row for i, (_, row, n, _) in enumerate(ctx.segments) if i not in out for row in range(row, row + n)]  # noqa: E731
+    covered = lambda hit: sorted(r for first, count, n in hit[:2] for f, c in zip(first[:n].tolist(), count[:n].tolist())  # noqa: E731
+                                 for r in range(f, f + c))
+    for factor in (0, 4):
+        handed = {}
+        for out in ((1, 2), (1,), (1, 2), (), (2, 3), (1,)):
+            hit = ctx.token_groups(1, factor, out)
+            assert covered(hit) == want(out)
+            assert handed.setdefault(out, spelled(hit)) == spelled(hit)
+        for out in handed:
+            assert spelled(ctx.token_groups(1, factor, out)) == handed[out]
+    ctx.begin_step()
+    ctx.segments = [(0, 0, 40, 0), (1, 40, 3, 5)]
+    assert covered(ctx.token_groups(1, 4, (0,))) == [40, 41, 42]
+
+
+def latent_part(window):
+    from mini_llm_runtime_amd.config import config_from_dict
+    layer = dict(type="latent_attention", mlp=None, mixer=dict(heads=16, dim=128, rot_dim=64, vdim=128, kv_rank=512, scale=192 ** -0.5,
+                                                               rot=dict(dims=64, base=10000.0), mask=dict(size=window)))
+    spec = config_from_dict(dict(architecture="Pamunex", vocab=97, width=64, norm=dict(eps=1e-5), logit_scale=1.0, layers=[layer])).model_spec()
+    return build_part("mixer", spec.layers[0].mixer)
+
+
+def test_latent_layers_of_different_windows_in_one_step():
+    """Windows 1024, 256 and 1024 leave other entries of a step to the attention behind the moved queries: every layer's groups
+    cover exactly the rows it leaves, out of planned memory, whatever came between."""
+    parts = [latent_part(window) for window in (1024, 256, 1024)]
+    rows, limits = 1351, dict(max_length=4096, page_size=16, split_keys=256, split_max_tokens=256, target_workgroups=512, max_slots=4)
+    ctx = context(4096)
+    ctx._group_upload = HostUpload()
+    plan = {}
+    for part in parts:
+        for key, count in part.workspace_plan(rows, torch.bfloat16, limits).items():
+            plan[key] = max(plan.get(key, 0), count)
+    # (of the large buffers only the room is asked here)
+    sizes = {key: count for key, count in plan.items() if key[0].startswith("token_groups")}
+    ctx.workspace.reserve(sizes)
+    ctx.workspace.room = lambda name, dtype: plan[name, dtype]
+    ctx.segments = [(0, 0, 1, 900), (1, 1, 800, 2000), (2, 801, 400, 600), (3, 1201, 150, 0)]
+    left = [tuple(p[0] for p in part._portions(ctx)) for part in parts]
+    assert left[0] == left[2] != left[1]
+    hits = [ctx.token_groups(1, 4, out, part.rest) for part, out in zip(parts, left)]
+    for (small, big, _), out in zip(hits, left):
+        got = [(f, c) for first, count, n in (small, big) for f, c in zip(first[:n].tolist(), count[:n].tolist())]
+        assert sorted(r for f, c in got for r in range(f, f + c)) == \
+            [r for i, (_, row, n, _) in enumerate(ctx.segments) if i not in out for r in range(row, row + n)]
+    assert ctx.workspace.unplanned_bytes() == 0
+
+
 def attention_part(head_dim=128):
     norm = NormSpec("rmsnorm", head_dim, 1e-6)
     return build_part("mixer", AttentionSpec("gqa_attention", 1024, 16, 8, head_dim, head_dim ** -0.5, norm,

@@ -157,6 +157,38 @@ def test_latent_portions_of_a_model(tmp_path, window, monkeypatch):
         assert bool(calls) == (runner is amply) or runner.workspace.room("latent_out", BF16) >= 64 * (48 + 64 + 512)
 
 
+def test_latent_layers_of_different_windows_in_one_step(tmp_path, monkeypatch):
+    """Layers of windows 1000, 30 and 1000 whose portions make their keys for other entries of a step each: the rest of the rows
+    must be every layer's own, against the plain implementation."""
+    from helpers import compare, make_requests, plain_logits, run_steps
+    from plain import pamunex_plain as P
+    from mini_llm_runtime_amd.config import config_from_dict
+    from mini_llm_runtime_amd.engine import Runner
+    from mini_llm_runtime_amd.engine.context import StepContext
+    from mini_llm_runtime_amd.parts import DecoderModel
+    from mini_llm_runtime_amd.weights import write_random_model
+    latent = lambda size: dict(type="latent_attention", mlp=None,  # noqa: E731
+                               mixer=dict(heads=2, dim=128, rot_dim=64, vdim=128, kv_rank=48, scale=192 ** -0.5,
+                                          rot=dict(dims=64, base=10000.0), mask=dict(size=size)))
+    cfg = dict(architecture="Pamunex", vocab=97, width=64, norm=dict(eps=1e-5), logit_scale=1.0, layers=[latent(1000), latent(30), latent(1000)])
+    folder = str(tmp_path / "model")
+    write_random_model(folder, config_from_dict(cfg), seed=3, matrix_std=0.12, norm_std=0.2)
+    requests = make_requests(97, [250, 240, 70, 9], seed=2)
+    part = lambda rid, lo, hi: dict(id=rid, tokens=requests[rid][lo:hi], want=list(range(hi - lo)))  # noqa: E731
+    steps = [dict(step=0, entries=[part("r0", 0, 201), part("r3", 0, 5), part("r1", 0, 64)], end=[]),
+             dict(step=1, entries=[part("r3", 5, 6), part("r0", 201, 241), part("r1", 64, 240), part("r2", 0, 50)], end=["r1"]),
+             dict(step=2, entries=[part("r3", 6, 9), part("r0", 241, 250), part("r2", 50, 70)], end=["r0", "r2", "r3"])]
+    monkeypatch.setattr("mini_llm_runtime_amd.parts.sink_attention.PORTION_LEAST_KEYS", 120)
+    asked = []
+    original = StepContext.token_groups
+    monkeypatch.setattr(StepContext, "token_groups", lambda self, *a: asked.append(a[2] if len(a) > 2 else ()) or original(self, *a))
+    runner = Runner(DecoderModel.load(folder, BF16), max_tokens=640, max_slots=4, max_length=256, max_batch_tokens=512, page_size=16)
+    got = run_steps(runner, steps)
+    assert asked[3:6] == [(1, 2), (2,), (1, 2)]                      # (the second step's three layers)
+    assert runner.workspace.unplanned_bytes() == 0
+    compare(got, plain_logits(P.PlainPamunex(folder), requests), "bfloat16")
+
+
 def test_a_model_with_a_router_keeps_its_sums(tmp_path, monkeypatch):
     """A choice of experts turns on the last bits where two lie within rounding: prompt portions of a model that makes such
     choices keep the kernels whose order of rounding its results have always had, those of one that does not take the others."""
