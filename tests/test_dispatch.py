@@ -12,7 +12,7 @@ from mini_llm_runtime_amd.parts.registry import PartError, build_part
 
 def kernels_without_gpu(dtype=torch.bfloat16):
     k = Kernels.__new__(Kernels)              # the size questions need no device
-    k.dtype, k.library_gemm = dtype, True
+    k.dtype, k.library_gemm, k._libs = dtype, True, {}
     return k
 
 
@@ -117,6 +117,22 @@ def test_latent_layers_of_different_windows_in_one_step():
         assert sorted(r for f, c in got for r in range(f, f + c)) == \
             [r for i, (_, row, n, _) in enumerate(ctx.segments) if i not in out for r in range(row, row + n)]
     assert ctx.workspace.unplanned_bytes() == 0
+
+
+@pytest.mark.parametrize("head_dim,value_dim", [(16, 16), (20, 24), (24, 24), (40, 64), (72, 128), (120, 48), (128, 128)])
+def test_the_delta_rules_chunks_are_planned_as_the_kernels_lay_them_out(head_dim, value_dim):
+    """A step that fills its tokens with one portion, and one of as many portions as there are slots, stay inside the plan."""
+    from mini_llm_runtime_amd.config import config_from_dict
+    layer = dict(type="channel_delta", mlp=dict(kind="dense", ff=64),
+                 mixer=dict(heads=4, kv_heads=2, dim=head_dim, vdim=value_dim, conv=4, decay_rank=16, gate_rank=16))
+    spec = config_from_dict(dict(architecture="Tigelorn", vocab=97, width=64, norm=dict(eps=1e-5), layers=[layer],
+                                 embedding=dict(bigram=dict(buckets=31, mul_prev=7, mul_cur=29)))).model_spec()
+    part, k = build_part("mixer", spec.layers[0].mixer), kernels_without_gpu()
+    for rows, slots in ((512, 1), (2048, 1), (2048, 7)):
+        plan = part.workspace_plan(rows, torch.bfloat16, dict(max_slots=slots))
+        lengths = [rows - 33 * (slots - 1)] + [33] * (slots - 1)
+        chunks = sum(-(-n // k.delta_chunk_tokens()) for n in lengths)
+        assert plan["delta_chunks", torch.float32] >= k.delta_chunk_floats(chunks, 4, head_dim, value_dim)
 
 
 def attention_part(head_dim=128):
