@@ -79,7 +79,6 @@ class Runner:
         # the memory plan, and the budget gate before anything of it is allocated
         limits = dict(max_length=self.max_length, page_size=page_size, split_keys=split_keys,
                       split_max_tokens=split_max_tokens, target_workgroups=target_workgroups, max_slots=max_slots)
-        workspace_plan = model.workspace_plan(self.max_batch_tokens, self.max_logits_rows, limits)
         uses_library = library_gemm and self.dtype == torch.bfloat16
         if _kv_dtype(kv_dtype, self.dtype) != self.dtype:
             raise ValueError(f"kv_dtype {kv_dtype}: the {self.dtype} engine's attention kernels read pages of their own "
@@ -91,31 +90,34 @@ class Runner:
         auto = max_tokens is None
         if auto and device_budget_bytes is None:
             device_budget_bytes = 0
-        for spare in (True, False):
-            # (first with the scratch memory that some parts would like besides what they need; without it where that does
-            # not fit)
-            if not spare:
-                workspace_plan = model.workspace_plan(self.max_batch_tokens, self.max_logits_rows, dict(limits, spare=False))
+
+        def planned(spare):
+            """(scratch buffers, tokens in the pool, its bytes, the memory plan), checked against the budget; `spare`: with the
+            scratch memory that some parts would like besides what they need."""
+            workspace = model.workspace_plan(self.max_batch_tokens, self.max_logits_rows, dict(limits, spare=spare))
+            tokens = max_tokens
             if auto:
                 # the pool takes what the budget leaves beside the scratch buffers, the metadata and the library's
                 # scratch (the weights are resident already and no longer part of the free memory)
-                room = device_budget(device_budget_bytes, self.device) - plan(workspace_plan, (0, 0, 0)).to_allocate()
-                max_tokens = CacheManager.tokens_that_fit(model.cache_entry_specs, self.dtype, page_size, max_slots,
-                                                          self.max_length, room)
-                if max_tokens <= 0:
-                    if spare:
-                        continue
+                room = device_budget(device_budget_bytes, self.device) - plan(workspace, (0, 0, 0)).to_allocate()
+                tokens = CacheManager.tokens_that_fit(model.cache_entry_specs, self.dtype, page_size, max_slots,
+                                                      self.max_length, room)
+                if tokens <= 0:
                     raise MemoryBudgetError(f"the device's budget leaves {room} bytes for the cache: not one page a group")
-            self.max_tokens = max_tokens
-            kv, tables, state = CacheManager.plan(model.cache_entry_specs, self.dtype, page_size, max_tokens, max_slots,
-                                                  self.max_length)
-            self.memory_plan = plan(workspace_plan, (kv, tables, state))
-            try:
-                self.memory_plan.check(device_budget_bytes, self.device)
-                break
-            except MemoryBudgetError:
-                if not spare:
-                    raise
+            pages = CacheManager.plan(model.cache_entry_specs, self.dtype, page_size, tokens, max_slots, self.max_length)
+            memory = plan(workspace, pages)
+            memory.check(device_budget_bytes, self.device)
+            return workspace, tokens, pages, memory
+
+        workspace_plan, max_tokens, (kv, tables, state), self.memory_plan = needed = planned(False)
+        try:
+            # spare scratch memory only where the pool holds as much beside it
+            wished = planned(True)
+            if wished[1] >= needed[1]:
+                workspace_plan, max_tokens, (kv, tables, state), self.memory_plan = wished
+        except MemoryBudgetError:
+            pass
+        self.max_tokens = max_tokens
         self.cache = CacheManager(model.cache_entry_specs, self.dtype, self.device, page_size,
                                   max_tokens, max_slots, self.max_length)
         assert (self.cache.kv_bytes(), self.cache.table_bytes(), self.cache.state_bytes()) == (kv, tables, state), \

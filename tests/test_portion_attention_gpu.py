@@ -157,6 +157,36 @@ def test_latent_portions_of_a_model(tmp_path, window, monkeypatch):
         assert bool(calls) == (runner is amply) or runner.workspace.room("latent_out", BF16) >= 64 * (48 + 64 + 512)
 
 
+def test_the_page_pool_goes_before_spare_scratch_memory(tmp_path):
+    """A pool sized by the budget holds what it would hold without the scratch memory that made keys would like, down to a
+    budget that leaves a few pages."""
+    from mini_llm_runtime_amd.config import config_from_dict
+    from mini_llm_runtime_amd.engine import MemoryBudgetError, Runner
+    from mini_llm_runtime_amd.parts import DecoderModel
+    from mini_llm_runtime_amd.weights import write_random_model
+    latent = dict(type="latent_attention", mlp=None, mixer=dict(heads=2, dim=128, rot_dim=64, vdim=128, kv_rank=48, scale=192 ** -0.5,
+                                                                rot=dict(dims=64, base=10000.0), mask=dict(size=4000)))
+    cfg = dict(architecture="Pamunex", vocab=97, width=64, norm=dict(eps=1e-5), logit_scale=1.0, layers=[latent, latent])
+    folder = str(tmp_path / "model")
+    write_random_model(folder, config_from_dict(cfg), seed=3, matrix_std=0.12, norm_std=0.2)
+    model = DecoderModel.load(folder, BF16)
+    runner = lambda budget: Runner(model, max_slots=3, max_length=4000, max_batch_tokens=256, page_size=16,  # noqa: E731
+                                   device_budget_bytes=budget)
+    ample = runner(0)
+    whole = ample.memory_plan.to_allocate()
+    assert ample.max_tokens >= 3 * 4000
+    bare = runner(whole - 1)
+    assert bare.max_tokens == ample.max_tokens and bare.memory_plan.workspace < ample.memory_plan.workspace
+    least = whole - ample.memory_plan.workspace - ample.memory_plan.kv_pages + bare.memory_plan.workspace      # without a page
+    page = -(-ample.memory_plan.kv_pages // (ample.max_tokens // 16))
+    spare = ample.memory_plan.workspace - bare.memory_plan.workspace
+    for pages in (8, spare // page - 1, spare // page + 8):
+        tight = runner(least + pages * page)
+        assert abs(tight.max_tokens - 16 * pages) <= 16 * 2 and tight.memory_plan.workspace == bare.memory_plan.workspace
+    with pytest.raises(MemoryBudgetError):
+        runner(least - 1)
+
+
 def test_latent_layers_of_different_windows_in_one_step(tmp_path, monkeypatch):
     """Layers of windows 1000, 30 and 1000 whose portions make their keys for other entries of a step each: the rest of the rows
     must be every layer's own, against the plain implementation."""
