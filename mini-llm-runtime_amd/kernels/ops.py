@@ -322,8 +322,9 @@ class Kernels:
 
     # -- projections -------------------------------------------------------------------------
     @timed("gemm", _gemm_work)
-    def gemm(self, a, w, out):
-        """out[M, N] = a[M, K] . w[N, K]^T; out has the element type or is float32."""
+    def gemm(self, a, w, out, library=True):
+        """out[M, N] = a[M, K] . w[N, K]^T; out has the element type or is float32.  `library=False`: never the vendor
+        library's, which looks a plan up for every new number of rows."""
         _tensor(a, "a", self.dtype, ndim=2)
         _tensor(w, "w", self.dtype, ndim=2)
         m, k = a.shape
@@ -331,7 +332,7 @@ class Kernels:
         _need(k == k2, lambda: f"gemm: inner sizes differ ({k} and {k2})")
         _need(out.dtype in (self.dtype, torch.float32), lambda: f"gemm: output type {out.dtype} not supported")
         _tensor(out, "out", out.dtype, (m, n))
-        if self.library_gemm and self.dtype == torch.bfloat16 and m > LIBRARY_GEMM_MIN_ROWS and \
+        if library and self.library_gemm and self.dtype == torch.bfloat16 and m > LIBRARY_GEMM_MIN_ROWS and \
                 (out.dtype == torch.float32 or not self.streams_weight(m, k)):
             # many rows: a plain matrix product, handed to the vendor library (hipBLASLt), as the reference
             # hands its projections to cuBLAS (src/minillm/cuda/matrix.cpp:11-37).  (Float outputs are

@@ -367,8 +367,11 @@ class LatentAttention:
             at += keys * width
         latent, shared, made_k, made_v = parts
         k.latent_rows(pages, view.block_table, ctx.slots, row, first, keys, view.page_size, s.rank, latent, shared)
-        k.gemm(latent, self.uk, made_k)
-        k.gemm(latent, self.uv.view(self.o_width, s.rank), made_v)
+        # (their number of rows is that of the keys, another one for nearly every portion: on the wide kernel, which needs no
+        # plan.  The first prompt of a length, 1000 to 1740 tokens in eight layers of 2048 channels of which two are latent
+        # attention: 6.0 ms, with the library's plans for these two products 6.4; one more prompt of that length 3.6 either way)
+        k.gemm(latent, self.uk, made_k, library=False)
+        k.gemm(latent, self.uv.view(self.o_width, s.rank), made_v, library=False)
         k.portion_attention_split(queries, q, made_k, shared, made_v, ctx.slots, ctx.positions, self.sink, attn, row, n, first,
                                   128 if n * s.heads >= 128 * ctx.compute_units else 64, s.heads, float(s.scale), self.mask, self.mask_size)
 

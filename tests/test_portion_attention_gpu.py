@@ -157,6 +157,40 @@ def test_latent_portions_of_a_model(tmp_path, window, monkeypatch):
         assert bool(calls) == (runner is amply) or runner.workspace.room("latent_out", BF16) >= 64 * (48 + 64 + 512)
 
 
+def test_made_keys_ask_for_no_plan_of_the_library(tmp_path, monkeypatch):
+    """The vendor library looks a plan up for every new number of rows; of portions' keys there is another one nearly every time."""
+    from helpers import make_requests
+    from mini_llm_runtime_amd.config import config_from_dict
+    from mini_llm_runtime_amd.engine import Entry, Runner
+    from mini_llm_runtime_amd.kernels import Kernels
+    from mini_llm_runtime_amd.parts import DecoderModel
+    from mini_llm_runtime_amd.weights import write_random_model
+    latent = dict(type="latent_attention", mlp=None, mixer=dict(heads=2, dim=128, rot_dim=64, vdim=128, kv_rank=64, scale=192 ** -0.5,
+                                                                rot=dict(dims=64, base=10000.0), mask=dict(size=4000)))
+    cfg = dict(architecture="Pamunex", vocab=97, width=64, norm=dict(eps=1e-5), logit_scale=1.0, layers=[latent])
+    folder = str(tmp_path / "model")
+    write_random_model(folder, config_from_dict(cfg), seed=3, matrix_std=0.12, norm_std=0.2)
+    monkeypatch.setattr("mini_llm_runtime_amd.parts.sink_attention.PORTION_LEAST_KEYS", 0)
+    runner = Runner(DecoderModel.load(folder, BF16), max_tokens=640, max_slots=4, max_length=512, max_batch_tokens=256, page_size=16)
+    rows, made = set(), set()
+    library, original = runner.kernels._lib("library_gemm"), Kernels.gemm
+
+    def gemm(self, a, w, out, library=True):
+        made.add(a.shape[0]) if not library else None
+        return original(self, a, w, out, library)
+
+    class Spied:
+        def mlr_library_gemm(self, a, w, out, m, *rest):
+            rows.add(m.value)
+            return library.mlr_library_gemm(a, w, out, m, *rest)
+    monkeypatch.setattr(Kernels, "gemm", gemm)
+    monkeypatch.setitem(runner.kernels._libs, "library_gemm", Spied())
+    slot, tokens = runner.open_request(), make_requests(97, [260], seed=4)["r0"]
+    for lo, hi in ((0, 90), (90, 173), (173, 260)):
+        runner.step([Entry(slot, tokens[lo:hi], [hi - lo - 1])])
+    assert rows <= {90, 83, 87} and made == {90, 173, 260}
+
+
 def test_the_page_pool_goes_before_spare_scratch_memory(tmp_path):
     """A pool sized by the budget holds what it would hold without the scratch memory that made keys would like, down to a
     budget that leaves a few pages."""
