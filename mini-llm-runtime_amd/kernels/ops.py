@@ -1673,13 +1673,14 @@ class Kernels:
     PORTION_PAGES = 1024          # page ids of a group's keys that the portion kernel keeps
 
     def portion_attention_supported(self, q_heads, kv_heads, key_dim, value_dim, k_row, v_row, page_size, mask=None, mask_size=0,
-                                    max_context=0, keep_first=0):
+                                    max_context=0, keep_first=0, scale=1.0):
         """Whether `portion_attention` takes these sizes: the bfloat16 engine, keys of 128 channels with as many value channels
         or of 64 with 64 or 128, cache rows that start at multiples of 16 bytes, pages of a power of two of at least 16
-        tokens, and a group's keys on no more pages than the kernel keeps."""
+        tokens, a group's keys on no more pages than the kernel keeps, and a positive factor on the scores (the kernel takes
+        a tile's maximum before it multiplies)."""
         whole = self.SINK_MASKS.get(mask, 0) == 0
         reach = max_context if whole else mask_size + 256 + (keep_first if keep_first > 0 else 0)
-        return (self.dtype == torch.bfloat16 and (key_dim, value_dim) in ((128, 128), (64, 128), (64, 64)) and k_row % 8 == 0
+        return (self.dtype == torch.bfloat16 and scale > 0 and (key_dim, value_dim) in ((128, 128), (64, 128), (64, 64)) and k_row % 8 == 0
                 and v_row % 8 == 0 and page_size >= 16 and page_size & (page_size - 1) == 0
                 and reach // page_size + 4 <= self.PORTION_PAGES and kv_heads * q_heads <= 65535)
 
@@ -1698,7 +1699,7 @@ class Kernels:
         kind = self.SINK_MASKS[mask]
         _need(kind == 0 or mask_size >= 1, "a window or chunk needs a positive size")
         _need(self.portion_attention_supported(q_heads, kv_heads, key_dim, value_dim, k_row, v_row, page_size, mask, mask_size, max_context,
-                                               self._kept(kind, keep_first)), "portion_attention: sizes that the kernel does not take")
+                                               self._kept(kind, keep_first), scale), "portion_attention: sizes that the kernel does not take")
         _tensor(block_table, "block_table", torch.int32, ndim=2)
         _tensor(slots, "slots", torch.int32, (rows,))
         _tensor(positions, "positions", torch.int32, (rows,))
@@ -1715,9 +1716,9 @@ class Kernels:
             _c_int(value_dim), _c_int(page_size), _c_int(kind), _c_int(int(mask_size)), _c_int(self._kept(kind, keep_first)),
             _c_float(self._cap(softcap)), _c_int(int(max_context)), _c_float(scale), _stream()), "portion_attention")
 
-    def latent_portions_supported(self, head_dim, rot_dim, value_dim, rank):
+    def latent_portions_supported(self, head_dim, rot_dim, value_dim, rank, scale=1.0):
         """Whether a portion's latent attention may run on keys and values that are made for it (`portion_attention_split`)."""
-        return self.dtype == torch.bfloat16 and (head_dim, rot_dim, value_dim) == (128, 64, 128) and rank % 8 == 0
+        return self.dtype == torch.bfloat16 and scale > 0 and (head_dim, rot_dim, value_dim) == (128, 64, 128) and rank % 8 == 0
 
     @timed("attention")
     def latent_rows(self, pages, block_table, slots, row, key0, keys, page_size, rank, latent, shared):
@@ -1749,6 +1750,7 @@ class Kernels:
         _tensor(values, "values", self.dtype, (n, heads * 128))
         _tensor(shared, "shared", self.dtype, (n, 64))
         _need(mask in self.SINK_MASKS and (self.SINK_MASKS[mask] == 0 or mask_size >= 1), f"mask {mask!r} of size {mask_size}")
+        _need(scale > 0, "portion_attention_split: a positive factor on the scores")
         _tensor(slots, "slots", torch.int32, (m,))
         _tensor(positions, "positions", torch.int32, (m,))
         if sink is not None:

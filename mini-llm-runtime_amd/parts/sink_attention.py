@@ -136,8 +136,8 @@ def attend(ctx, q, k_pages, v_pages, view, sink, out, q_heads, kv_heads, key_dim
     if k.sink_tiles_supported(key_dim, value_dim, k_pages.shape[3], v_pages.shape[3], view.page_size, mask, mask_size,
                               ctx.max_positions, keep_first) and q.shape[1] % 8 == 0:
         big_heads, big_tokens, small_heads, small_tokens = k.sink_tiles_layout(q_heads, kv_heads)
-        portions = not ctx.routed and k.portion_attention_supported(q_heads, kv_heads, key_dim, value_dim, k_pages.shape[3], v_pages.shape[3], view.page_size,
-                                                                    mask, mask_size, ctx.max_positions, keep_first)
+        portions = not ctx.routed and k.portion_attention_supported(q_heads, kv_heads, key_dim, value_dim, k_pages.shape[3], v_pages.shape[3],
+                                                                    view.page_size, mask, mask_size, ctx.max_positions, keep_first, scale)
         if portions:
             columns, big_heads = portion_columns(ctx, q_heads), min(big_heads, 32)
             big_tokens = columns // big_heads
@@ -320,7 +320,7 @@ class LatentAttention:
         """Elements of `latent_out` for the longest portion that makes its keys (0: none of this runner's does): its place is
         free until the step's other rows come.  Without `limits["spare"]` no more than those other rows need."""
         s = self.spec
-        if dtype != torch.bfloat16 or (s.head_dim, s.rot_dim, s.value_dim) != (128, 64, 128) or s.rank % 8 != 0 or \
+        if dtype != torch.bfloat16 or not s.scale > 0 or (s.head_dim, s.rot_dim, s.value_dim) != (128, 64, 128) or s.rank % 8 != 0 or \
                 limits.get("routed", False) or not limits.get("spare", True):
             return 0
         most = limits["max_length"] if self.mask is None else min(limits["max_length"], self.mask_size + rows)
@@ -347,7 +347,8 @@ class LatentAttention:
         rank 512, for rank * (head_dim + value_dim) products a key and head.  Not in a step that is to be captured: first
         key and number of keys would be fixed in the graph."""
         s = self.spec
-        if ctx.routed or ctx.fixed_groups is not None or not ctx.kernels.latent_portions_supported(s.head_dim, s.rot_dim, s.value_dim, s.rank):
+        if ctx.routed or ctx.fixed_groups is not None or \
+                not ctx.kernels.latent_portions_supported(s.head_dim, s.rot_dim, s.value_dim, s.rank, float(s.scale)):
             return []
         out, room = [], ctx.workspace.room("latent_out", torch.bfloat16)
         for i, (_, row, n, p0) in enumerate(ctx.segments):

@@ -157,6 +157,30 @@ def test_latent_portions_of_a_model(tmp_path, window, monkeypatch):
         assert bool(calls) == (runner is amply) or runner.workspace.room("latent_out", BF16) >= 64 * (48 + 64 + 512)
 
 
+@pytest.mark.parametrize("scale", [-0.1, 0.0])
+def test_factors_on_the_scores_that_are_not_positive(tmp_path, monkeypatch, scale):
+    """The portion kernel takes a tile's maximum before the factor, so such a layer's portions go the other way."""
+    from helpers import compare, make_requests, plain_logits, portions, run_steps, whole
+    from plain import pamunex_plain as P
+    from mini_llm_runtime_amd.config import config_from_dict
+    from mini_llm_runtime_amd.engine import Runner
+    from mini_llm_runtime_amd.parts import DecoderModel
+    from mini_llm_runtime_amd.weights import write_random_model
+    monkeypatch.setattr("mini_llm_runtime_amd.parts.sink_attention.PORTION_LEAST_KEYS", 0)
+    rot, mask = dict(dims=64, base=10000.0), dict(size=100)
+    layers = [dict(type="latent_attention", mlp=None, mixer=dict(heads=2, dim=128, rot_dim=64, vdim=128, kv_rank=48, scale=scale, rot=rot, mask=mask)),
+              dict(type="attention", mlp=dict(kind="dense", ff=64),
+                   mixer=dict(heads=4, kv_heads=2, dim=128, vdim=128, scale=scale, rot=rot, mask=mask))]
+    folder = str(tmp_path / "model")
+    write_random_model(folder, config_from_dict(dict(architecture="Pamunex", vocab=97, width=64, norm=dict(eps=1e-5), logit_scale=1.0,
+                                                     layers=layers)), seed=3, matrix_std=0.12, norm_std=0.2)
+    requests = make_requests(97, [150, 64, 201], seed=2)
+    want, model = plain_logits(P.PlainPamunex(folder), requests), DecoderModel.load(folder, BF16)
+    for cut in (whole(requests), portions(requests, (100, 65, 7))):
+        runner = Runner(model, max_tokens=640, max_slots=4, max_length=256, max_batch_tokens=512, page_size=16)
+        compare(run_steps(runner, cut), want, "bfloat16")
+
+
 def test_made_keys_ask_for_no_plan_of_the_library(tmp_path, monkeypatch):
     """The vendor library looks a plan up for every new number of rows; of portions' keys there is another one nearly every time."""
     from helpers import make_requests
