@@ -479,6 +479,27 @@ __device__ __forceinline__ floatx4 mma4(const floatx4& a, const floatx4& b, floa
     return c;
 }
 
+// The same for a lower triangular A (zeros above): row t takes B's rows 0 .. t.  A zero does not keep a later row out that is
+// not finite -- a token must not see what comes after it --, so then every row is taken by itself with the later ones cleared.
+__device__ __forceinline__ floatx4 mma4_lower(const floatx4& a, const floatx4& b, const floatx4& c) {
+    bool odd = false;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) odd |= !(fabsf(b[i]) <= 3.402823466e38f);
+    if (__builtin_expect(!__any(odd), 1)) return mma4(a, b, c);
+    const int first = ((threadIdx.x & 63) >> 4) * 4;
+    floatx4 out = c;
+    for (int t = 0; t < 16; ++t) {
+        floatx4 seen;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) seen[i] = first + i <= t ? b[i] : 0.f;
+        const floatx4 row = mma4(a, seen, c);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (first + i == t) out[i] = row[i];
+    }
+    return out;
+}
+
 // One workgroup a chunk and head.  The pairs (t, s) of one half of the chunk need an exponential a key channel each, so a
 // thread takes one pair (120 a half); between the halves e^{c_t - c_s} = e^{c_t - c_15} e^{c_15 - c_s}, neither above 1, and
 // the sums are a matrix product.  T = (I + A)^-1 by halves too: two triangles of 16 a lane column by column, and
@@ -633,7 +654,7 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(DeltaChunkArgs
 #pragma unroll
         for (int i = 0; i < 4; ++i) t11[i] = T_l[(b4 + i) * CS + c];
         p = mma4(four(A_l + (16 + c) * CS + b4), t11, p);
-        p = mma4(four(T_l + (16 + c) * CS + 16 + b4), p, floatx4{0.f, 0.f, 0.f, 0.f});
+        p = mma4_lower(four(T_l + (16 + c) * CS + 16 + b4), p, floatx4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
         for (int i = 0; i < 4; ++i) T_l[(16 + b4 + i) * CS + c] = -p[i];
     }
@@ -645,8 +666,8 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(DeltaChunkArgs
 #pragma unroll
         for (int st = 0; st < 2; ++st) tf[rt][st] = four(T_l + (16 * rt + c) * CS + 16 * st + b4);
     auto product = [&](const floatx4 (&x)[2], float* dst, int width, int col, bool ok) {      // T x, 16 columns
-        floatx4 top = mma4(tf[0][0], x[0], floatx4{0.f, 0.f, 0.f, 0.f});
-        floatx4 low = mma4(tf[1][1], x[1], mma4(tf[1][0], x[0], floatx4{0.f, 0.f, 0.f, 0.f}));
+        floatx4 top = mma4_lower(tf[0][0], x[0], floatx4{0.f, 0.f, 0.f, 0.f});
+        floatx4 low = mma4_lower(tf[1][1], x[1], mma4(tf[1][0], x[0], floatx4{0.f, 0.f, 0.f, 0.f}));
         if (!ok) return;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -793,8 +814,8 @@ __global__ __launch_bounds__(256, 1) void delta_chunk_scan_kernel(DeltaChunkArgs
         for (int j = 0; j < NT; ++j)
             if (!mine[j]) S[j] = zero;                      // (the same in every lane)
         if (b_row >= b_col) {
-            if (b_row == 0) o[0] = mma4(now.b, u[0], o[0]);
-            else o[1] = mma4(now.b, b_col == 0 ? u[0] : u[1], o[1]);
+            if (b_row == 0) o[0] = mma4_lower(now.b, u[0], o[0]);
+            else o[1] = b_col == 0 ? mma4(now.b, u[0], o[1]) : mma4_lower(now.b, u[1], o[1]);
         }
         if (c0 > 0) put_out(buf ^ 1, c0 - C);               // (written before the barrier above)
 #pragma unroll

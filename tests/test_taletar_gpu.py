@@ -677,6 +677,38 @@ def test_configurations_drawn_at_random(tmp_path, seed):
             assert max_difference(results["whole"], results["mixed"]) == 0.0, cfg
 
 
+@pytest.mark.parametrize("keys,values", [(20, 24), (128, 128)])
+@pytest.mark.parametrize("at", [3, 20, 47])
+def test_delta_rule_in_chunks_a_token_that_is_not_finite_does_not_reach_those_before_it(keys, values, at):
+    """Any operand of one token, first and second half of a chunk: every bit of the tokens before it and of the other request
+    stays, and the token itself shows it."""
+    from mini_llm_runtime_amd.kernels import Kernels
+    k = Kernels(torch.bfloat16)
+    gen = torch.Generator("cuda").manual_seed(keys + at)
+    heads, lengths = 2, [70, 40]
+    n, size = sum(lengths), k.delta_chunk_tokens()
+    rnd = lambda *shape: torch.randn(shape, generator=gen, device="cuda")  # noqa: E731
+    operands = [rnd(n, heads * keys).bfloat16(), rnd(n, heads * keys).bfloat16(), rnd(n, heads * values).bfloat16(),
+                -torch.rand(n, heads * keys, generator=gen, device="cuda"), rnd(n, heads)]
+    live = rnd(3, heads * keys * values)
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    pieces = [(first + a, min(size, length - a)) for first, length in ((0, 70), (70, 40)) for a in range(0, length, size)]
+
+    def run(q, kk, v, decay, beta):
+        out, stage = torch.empty(n, heads * values, device="cuda"), live.clone()
+        scratch = torch.empty(k.delta_chunk_floats(len(pieces), heads, keys, values), device="cuda")
+        k.delta_rule_chunked(q, kk, v, decay, beta, out, live, stage, 0, ints([0, 70]), ints(lengths), 2, ints([2] * 70 + [0] * 40),
+                             ints([p[0] for p in pieces]), ints([p[1] for p in pieces]), len(pieces), scratch, heads, keys, values)
+        return out, stage
+    clean, state = run(*operands)
+    for which, bad in ((0, "nan"), (1, "nan"), (2, "nan"), (2, "inf"), (3, "nan"), (4, "nan")):
+        hurt = [x.clone() for x in operands]
+        hurt[which][at] = float(bad)
+        out, stage = run(*hurt)
+        assert torch.equal(out[:at], clean[:at]) and torch.equal(out[70:], clean[70:]), (which, bad)
+        assert torch.equal(stage[:2], state[:2]) and not torch.isfinite(out[at]).any(), (which, bad)
+
+
 @pytest.mark.parametrize("dtype_name", DTYPES)
 @pytest.mark.parametrize("keys,values", [(1, 3), (30, 64), (64, 70), (128, 128), (250, 17)])
 def test_requests_of_one_token_get_what_they_get_beside_longer_ones(dtype_name, keys, values):
