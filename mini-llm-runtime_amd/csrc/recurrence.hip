@@ -703,9 +703,10 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(DeltaChunkArgs
 // chunk later.  A chunk's operands are on their way while the chunk before is worked on.  Scalar sums out of tiles staged in
 // LDS took 598 us for 2048 tokens of 16 heads of 128 x 128 channels (64 chunks, 128 workgroups); this one 153, 2.4 us a
 // chunk, of which 0.7 are its 52 matrix instructions a wavefront and the rest the chain between them: it is bound by the
-// walk's length, not by memory (with one chunk of operands under way instead of two 166 us).
-template <int NT>
-__global__ __launch_bounds__(256, 1) void delta_chunk_scan_kernel(DeltaChunkArgs g) {
+// walk's length, not by memory (with one chunk of operands under way instead of two 166 us).  Without AHEAD, for more workgroups
+// than compute units, a chunk's operands are asked for as it begins, and three workgroups share a unit.
+template <int NT, bool AHEAD>
+__global__ __launch_bounds__(256, AHEAD ? 1 : 3) void delta_chunk_scan_kernel(DeltaChunkArgs g) {
     constexpr int C = DELTA_CHUNK;
     const DeltaArgs& a = g.d;
     __shared__ __attribute__((aligned(16))) float u_l[2][4][2][256], o_l[2][4][2][256];      // [buffer][wavefront][row tile][lane, element]
@@ -771,13 +772,7 @@ __global__ __launch_bounds__(256, 1) void delta_chunk_scan_kernel(DeltaChunkArgs
         }
     };
     const float* base = g.scratch + (size_t)chunk0 * step + (size_t)head * delta_chunk_floats(N, V);
-    Chunk ring[3];                                          // the chunk at work and the two behind it
-    const float* last = base + (size_t)((n - 1) / C) * step;
-    fetch(base, ring[0]);
-    fetch(base + step <= last ? base + step : last, ring[1]);
-    auto turn = [&](const Chunk& now, Chunk& ahead, int c0, int buf) {
-        fetch(base + 2 * step <= last ? base + 2 * step : last, ahead);        // (never behind a branch)
-        base += step;
+    auto work = [&](const Chunk& now, int c0, int buf) {
         floatx4 part[2] = {zero, zero}, o[2] = {zero, zero};
 #pragma unroll
         for (int j = 0; j < NT; ++j)
@@ -822,15 +817,32 @@ __global__ __launch_bounds__(256, 1) void delta_chunk_scan_kernel(DeltaChunkArgs
         for (int rt = 0; rt < 2; ++rt) *reinterpret_cast<floatx4*>(&o_l[buf][wave][rt][lane * 4]) = o[rt];
     };
     int buf = 0;
-    for (int c0 = 0; c0 < n; c0 += 3 * C) {
-        turn(ring[0], ring[2], c0, buf);
-        buf ^= 1;
-        if (c0 + C >= n) break;
-        turn(ring[1], ring[0], c0 + C, buf);
-        buf ^= 1;
-        if (c0 + 2 * C >= n) break;
-        turn(ring[2], ring[1], c0 + 2 * C, buf);
-        buf ^= 1;
+    if (AHEAD) {
+        Chunk ring[3];                                      // the chunk at work and the two behind it
+        const float* last = base + (size_t)((n - 1) / C) * step;
+        fetch(base, ring[0]);
+        fetch(base + step <= last ? base + step : last, ring[1]);
+        auto turn = [&](const Chunk& now, Chunk& ahead, int c0) {
+            fetch(base + 2 * step <= last ? base + 2 * step : last, ahead);    // (never behind a branch)
+            base += step;
+            work(now, c0, buf);
+            buf ^= 1;
+        };
+        for (int c0 = 0; c0 < n; c0 += 3 * C) {
+            turn(ring[0], ring[2], c0);
+            if (c0 + C >= n) break;
+            turn(ring[1], ring[0], c0 + C);
+            if (c0 + 2 * C >= n) break;
+            turn(ring[2], ring[1], c0 + 2 * C);
+        }
+    } else {
+        for (int c0 = 0; c0 < n; c0 += C) {
+            Chunk now;
+            fetch(base, now);
+            base += step;
+            work(now, c0, buf);
+            buf ^= 1;
+        }
     }
     __syncthreads();
     put_out(buf ^ 1, (n - 1) / C * C);
@@ -1018,8 +1030,17 @@ int mlr_delta_rule_chunked(const void* q, long q_stride, const void* k, long k_s
     int err = (int)hipGetLastError();
     if (err != 0) return err;
     const dim3 grid(segments, heads, (n_values + 15) / 16);
-    if (Np <= 64) delta_chunk_scan_kernel<1><<<grid, 256, 0, stream>>>(g);
-    else delta_chunk_scan_kernel<2><<<grid, 256, 0, stream>>>(g);
+    // (two chunks of operands on their way while one is at work while no compute unit has a second workgroup, which the registers
+    // would keep out: one request of 2048 tokens of 16 heads of 128 x 128 244 us, without 271; but four of 512 181 and 158, 64 of
+    // 32 404 and 218, 64 of 9 380 and 194)
+    const bool ahead = (long)segments * heads * ((n_values + 15) / 16) <= 256;
+    if (Np <= 64) {
+        if (ahead) delta_chunk_scan_kernel<1, true><<<grid, 256, 0, stream>>>(g);
+        else delta_chunk_scan_kernel<1, false><<<grid, 256, 0, stream>>>(g);
+    } else {
+        if (ahead) delta_chunk_scan_kernel<2, true><<<grid, 256, 0, stream>>>(g);
+        else delta_chunk_scan_kernel<2, false><<<grid, 256, 0, stream>>>(g);
+    }
     return (int)hipGetLastError();
 }
 

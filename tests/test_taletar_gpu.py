@@ -677,6 +677,41 @@ def test_configurations_drawn_at_random(tmp_path, seed):
             assert max_difference(results["whole"], results["mixed"]) == 0.0, cfg
 
 
+@pytest.mark.parametrize("keys,values", [(33, 16), (64, 30), (128, 16)])
+def test_delta_rule_in_chunks_one_request_alone_and_among_many(keys, values):
+    """Few workgroups ask two chunks ahead, many do not: the arithmetic, and so every bit, is the same.  Lengths around the three
+    chunks that the former turns through."""
+    from mini_llm_runtime_amd.kernels import Kernels
+    k = Kernels(torch.bfloat16)
+    gen = torch.Generator("cuda").manual_seed(keys)
+    heads, lengths = 16, [150, 32, 33, 64, 65, 96, 97, 1, 128, 129, 31, 9, 40, 64, 100, 70, 5, 20]
+    n, size = sum(lengths), k.delta_chunk_tokens()
+    assert heads * len(lengths) * (-(-values // 16)) > 256
+    rnd = lambda *shape: torch.randn(shape, generator=gen, device="cuda")  # noqa: E731
+    operands = [rnd(n, heads * keys).bfloat16(), rnd(n, heads * keys).bfloat16(), rnd(n, heads * values).bfloat16(),
+                -torch.rand(n, heads * keys, generator=gen, device="cuda"), rnd(n, heads)]
+    live = rnd(len(lengths), heads * keys * values)
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+
+    def run(requests):
+        rows = [r for i in requests for r in range(sum(lengths[:i]), sum(lengths[:i + 1]))]
+        first, at, pieces = [], 0, []
+        for i in requests:
+            first.append(at)
+            pieces += [(at + a, min(size, lengths[i] - a)) for a in range(0, lengths[i], size)]
+            at += lengths[i]
+        out, stage = torch.empty(at, heads * values, device="cuda"), live.clone()
+        scratch = torch.empty(k.delta_chunk_floats(len(pieces), heads, keys, values), device="cuda")
+        k.delta_rule_chunked(*(x[rows].contiguous() for x in operands), out, live, stage, 0, ints(first), ints([lengths[i] for i in requests]),
+                             len(requests), ints([i for i in requests for _ in range(lengths[i])]), ints([p[0] for p in pieces]),
+                             ints([p[1] for p in pieces]), len(pieces), scratch, heads, keys, values)
+        return out, stage
+    everything, states = run(list(range(len(lengths))))
+    for i, length in enumerate(lengths):
+        out, stage = run([i])
+        assert torch.equal(out, everything[sum(lengths[:i]):sum(lengths[:i]) + length]) and torch.equal(stage[i], states[i]), i
+
+
 @pytest.mark.parametrize("keys,values", [(20, 24), (128, 128)])
 @pytest.mark.parametrize("at", [3, 20, 47])
 def test_delta_rule_in_chunks_a_token_that_is_not_finite_does_not_reach_those_before_it(keys, values, at):
