@@ -316,12 +316,15 @@ class LatentAttention:
         s = self.spec
         return keys * (self.row + s.heads * s.head_dim + self.o_width)
 
+    def _portions_possible(self, dtype, limits):
+        s = self.spec
+        return dtype == torch.bfloat16 and s.scale > 0 and (s.head_dim, s.rot_dim, s.value_dim) == (128, 64, 128) and s.rank % 8 == 0 and \
+            not limits.get("routed", False)
+
     def _portions_planned(self, rows, dtype, limits):
         """Elements of `latent_out` for the longest portion that makes its keys (0: none of this runner's does): its place is
         free until the step's other rows come.  Without `limits["spare"]` no more than those other rows need."""
-        s = self.spec
-        if dtype != torch.bfloat16 or not s.scale > 0 or (s.head_dim, s.rot_dim, s.value_dim) != (128, 64, 128) or s.rank % 8 != 0 or \
-                limits.get("routed", False) or not limits.get("spare", True):
+        if not self._portions_possible(dtype, limits) or not limits.get("spare", True):
             return 0
         most = limits["max_length"] if self.mask is None else min(limits["max_length"], self.mask_size + rows)
         return self._made(min(most, PORTION_KEYS) + 64)
@@ -330,7 +333,7 @@ class LatentAttention:
         s = self.spec
         groups = _groups_plan(rows, s.heads, 1, s.rank)
         rest = {(f"{name}_{self.rest}", kind): count for (name, kind), count in groups.items()
-                if name.startswith("token_groups") and self._portions_planned(rows, dtype, limits) > 0}
+                if name.startswith("token_groups") and self._portions_possible(dtype, limits)}
         first = self.q_width if s.q_rank is None else s.q_rank
         more = {} if s.q_rank is None else {("latent_cq", dtype): rows * s.q_rank, ("latent_queries", dtype): rows * self.q_width}
         if self.head_gate is not None:

@@ -215,11 +215,12 @@ def test_made_keys_ask_for_no_plan_of_the_library(tmp_path, monkeypatch):
     assert rows <= {90, 83, 87} and made == {90, 173, 260}
 
 
-def test_the_page_pool_goes_before_spare_scratch_memory(tmp_path):
+def test_the_page_pool_goes_before_spare_scratch_memory(tmp_path, monkeypatch):
     """A pool sized by the budget holds what it would hold without the scratch memory that made keys would like, down to a
-    budget that leaves a few pages."""
+    budget that leaves a few pages; and short portions, whose keys find room all the same, stay inside the plan."""
     from mini_llm_runtime_amd.config import config_from_dict
-    from mini_llm_runtime_amd.engine import MemoryBudgetError, Runner
+    from mini_llm_runtime_amd.engine import Entry, MemoryBudgetError, Runner
+    from mini_llm_runtime_amd.kernels import Kernels
     from mini_llm_runtime_amd.parts import DecoderModel
     from mini_llm_runtime_amd.weights import write_random_model
     latent = dict(type="latent_attention", mlp=None, mixer=dict(heads=2, dim=128, rot_dim=64, vdim=128, kv_rank=48, scale=192 ** -0.5,
@@ -235,6 +236,12 @@ def test_the_page_pool_goes_before_spare_scratch_memory(tmp_path):
     assert ample.max_tokens >= 3 * 4000
     bare = runner(whole - 1)
     assert bare.max_tokens == ample.max_tokens and bare.memory_plan.workspace < ample.memory_plan.workspace
+    monkeypatch.setattr("mini_llm_runtime_amd.parts.sink_attention.PORTION_LEAST_KEYS", 0)
+    made, original = [], Kernels.portion_attention_split
+    monkeypatch.setattr(Kernels, "portion_attention_split", lambda self, *a, **kw: made.append(a) or original(self, *a, **kw))
+    slots = [bare.open_request(), bare.open_request()]
+    bare.step([Entry(slots[0], list(range(35)), [34]), Entry(slots[1], [5], [0])])
+    assert len(made) == 2 and bare.workspace.unplanned_bytes() == 0
     least = whole - ample.memory_plan.workspace - ample.memory_plan.kv_pages + bare.memory_plan.workspace      # without a page
     page = -(-ample.memory_plan.kv_pages // (ample.max_tokens // 16))
     spare = ample.memory_plan.workspace - bare.memory_plan.workspace
