@@ -236,8 +236,8 @@ __global__ __launch_bounds__(64) void diff_attention_partial_kernel(DiffArgs a) 
 // Two wavefronts per (token, head), a map each, merged over their key ranges, then the head's epilogue by the first.  Bound by
 // its chain of loads: a range's values are asked for eight ranges at a time, the first eight before the weights are known
 // (8 tokens of 16 heads in 11 ranges: 13.8 us with one wavefront, range by range, now 5.5).
-#define AHEAD 8
 __global__ __launch_bounds__(128) void diff_attention_combine_kernel(DiffArgs a) {
+    constexpr int AHEAD = 8;
     __shared__ float w_lds[2][COMBINE_MAX_SPLITS];
     __shared__ float l_lds[2][COMBINE_MAX_SPLITS];
     __shared__ float second[64 * MAX_V_REGS];

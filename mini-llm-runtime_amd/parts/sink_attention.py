@@ -60,7 +60,11 @@ def _rope_table(position, ctx, device, rot_limit):
 # Portions of latent attention that make keys and values of their own: from this many tokens and keys on (16 heads, rank
 # 512, a step of eight layers of which two are latent attention, made against moved: 32 tokens behind 1000 keys 1.92 ms
 # against 2.02, behind 4000 2.10 against 3.01; without context 512 tokens 3.17 against 3.09, 2048 5.4 against 6.5), and up
-# to this many keys (the scratch memory: 9.3 KB a key).
+# to this many keys (the scratch memory: 9.3 KB a key).  The line holds for other ranks and heads too, though a small rank
+# spares products either way: eight latent layers, 32 tokens behind 768, 128 behind 872 and a prompt of 2048, made against
+# moved, at rank 64 with 16 heads 0.98 and 0.98, 1.10 and 1.15, 1.30 and 1.98 ms; at rank 128 0.90 and 1.09, 1.04 and 1.26,
+# 1.27 and 3.20; at rank 128 with 4 heads 0.93 and 1.03, 1.09 and 1.23, 1.18 and 2.07.  A step that is replayed as a graph
+# keeps the moved queries (see `_portions`).
 PORTION_ROWS = 32
 PORTION_LEAST_KEYS = 768
 PORTION_KEYS = 16384

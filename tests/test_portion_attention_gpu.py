@@ -154,7 +154,9 @@ def test_latent_portions_of_a_model(tmp_path, window, monkeypatch):
     for runner in (amply, tight):
         calls.clear()
         compare(run_steps(runner, whole(requests)), want, "bfloat16")
-        assert bool(calls) == (runner is amply) or runner.workspace.room("latent_out", BF16) >= 64 * (48 + 64 + 512)
+        room = runner.workspace.room("latent_out", BF16)                 # (a key's latent and shared part, two heads' keys and values)
+        assert len(calls) == 2 * sum(n * (48 + 64 + 2 * 128 + 2 * 128) <= room for n in (150, 64, 201))
+        assert runner is tight or len(calls) == 2 * 3
 
 
 @pytest.mark.parametrize("scale", [-0.1, 0.0])
