@@ -72,6 +72,9 @@ __global__ __launch_bounds__(64) void gemm_f32_strip_kernel(const float* __restr
 #pragma unroll
     for (int u = 0; u < U; ++u) fetch(min(1, blocks - 1), u, false);
     auto turn = [&](int t, bool all) {                     // all: the two blocks behind t are whole
+        // (other lanes read what a lane has stored: a wavefront's LDS instructions run in their order, and the compiler keeps it)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
         const float* at = lds + (t & 1) * (U * P * 256) + r * 4 + b;
         floatx4 now[P], next[P];
         auto read = [&](int u, floatx4 (&v)[P]) {          // element i: k = 4 i + b of the group
