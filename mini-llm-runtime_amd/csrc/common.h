@@ -108,3 +108,24 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
     for (int i = 0; i < waves; ++i) total += scratch[i];
     return total;
 }
+
+// The activation of a gated feed-forward's gate: ACT 0 silu(g) = g / (1 + exp(-g)); ACT 1 the tanh form of gelu,
+// 0.5 g (1 + tanh(sqrt(2 / pi) (g + 0.044715 g^3))); ACT 2 max(g, 0).  32-bit.
+template <int ACT>
+__device__ __forceinline__ float gate_act(float g) {
+    if (ACT == 2) return fmaxf(g, 0.f);
+    if (ACT == 1) return 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g)));
+    return g / (1.0f + expf(-g));
+}
+// The activation of a feed-forward without a gate: ACT 0 relu(x)^2; ACT 1 the exact gelu, x Phi(x) with the normal
+// distribution's function.  32-bit.
+template <int ACT> __device__ __forceinline__ float plain_act(float x) {
+    if (ACT == 1) return 0.5f * x * (1.0f + erff(x * 0.70710678118654752440f));
+    const float r = fmaxf(x, 0.f);
+    return r * r;
+}
+// The gate whose branches are clamped: g * sigmoid(slope * g) * (u + 1), g = min(gate, limit), u = clamp(up, -limit, limit).
+__device__ __forceinline__ float clamped_glu(float gate, float up, float limit, float slope) {
+    const float g = fminf(gate, limit), u = fminf(fmaxf(up, -limit), limit);
+    return (g / (1.0f + expf(-slope * g))) * (u + 1.0f);
+}

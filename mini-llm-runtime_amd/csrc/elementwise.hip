@@ -260,16 +260,7 @@ __global__ void residual_add_kernel(float* __restrict__ h, const RowAddend adden
     }
 }
 
-// The activation of a gated feed-forward's gate: ACT 0 silu(g) = g / (1 + exp(-g)); ACT 1 the tanh form of gelu,
-// 0.5 g (1 + tanh(sqrt(2 / pi) (g + 0.044715 g^3))); ACT 2 max(g, 0).  32-bit.
-template <int ACT>
-__device__ __forceinline__ float gate_act(float g) {
-    if (ACT == 2) return fmaxf(g, 0.f);
-    if (ACT == 1) return 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g)));
-    return g / (1.0f + expf(-g));
-}
-
-// The same, 16 bytes per lane and access, for inter % MLR_VEC == 0.
+// act[m, f] = act(gate_up[m, f]) * gate_up[m, inter + f], 16 bytes per lane and access, for inter % MLR_VEC == 0.
 template <int ACT>
 __global__ void silu_mul_vec_kernel(const elem_t* __restrict__ gate_up, elem_t* __restrict__ act, int rows, int inter) {
     const int per_row = inter / MLR_VEC;
@@ -285,7 +276,7 @@ __global__ void silu_mul_vec_kernel(const elem_t* __restrict__ gate_up, elem_t* 
     }
 }
 
-// act[m, f] = act(gate_up[m, f]) * gate_up[m, inter + f].
+// The same, one value an access.
 template <int ACT>
 __global__ void silu_mul_kernel(const elem_t* __restrict__ gate_up, elem_t* __restrict__ act,
                                 int rows, int inter) {
@@ -550,16 +541,13 @@ __global__ void residual_add2_kernel(float* __restrict__ h, const elem_t* __rest
     }
 }
 
-// act[m, f] = g * sigmoid(slope * g) * (u + 1) with g = min(gate, limit), u = clamp(up, -limit, limit);
-// gate = gate_up[m, f], up = gate_up[m, inter + f].
+// act[m, f] = clamped_glu(gate_up[m, f], gate_up[m, inter + f]).
 __global__ void clamped_glu_kernel(const elem_t* __restrict__ gate_up, elem_t* __restrict__ act, int rows, int inter,
                                    float limit, float slope) {
     const size_t total = (size_t)rows * inter;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
         const size_t m = i / inter, f = i % inter;
-        const float g = fminf(to_float(gate_up[m * 2 * inter + f]), limit);
-        const float u = fminf(fmaxf(to_float(gate_up[m * 2 * inter + inter + f]), -limit), limit);
-        act[i] = from_float<elem_t>((g / (1.0f + expf(-slope * g))) * (u + 1.0f));
+        act[i] = from_float<elem_t>(clamped_glu(to_float(gate_up[m * 2 * inter + f]), to_float(gate_up[m * 2 * inter + inter + f]), limit, slope));
     }
 }
 
@@ -663,10 +651,7 @@ __global__ void clamped_glu_vec_kernel(const elem_t* __restrict__ gate_up, elem_
         load_vec(gate_up + m * 2 * inter + f, g);
         load_vec(gate_up + m * 2 * inter + inter + f, u);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const float gg = fminf(g[e], limit), uu = fminf(fmaxf(u[e], -limit), limit);
-            y[e] = (gg / (1.0f + expf(-slope * gg))) * (uu + 1.0f);
-        }
+        for (int e = 0; e < 8; ++e) y[e] = clamped_glu(g[e], u[e], limit, slope);
         store_vec(act + m * inter + f, y);
     }
 }
@@ -933,13 +918,7 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const elem_t* __restrict
     }
 }
 
-// The activation of a feed-forward without a gate, element by element (32-bit): ACT 0 relu(x)^2; ACT 1 the exact gelu,
-// x Phi(x) with the normal distribution's function.  VEC: MLR_VEC values in one access, or 1.
-template <int ACT> __device__ __forceinline__ float plain_act(float x) {
-    if (ACT == 1) return 0.5f * x * (1.0f + erff(x * 0.70710678118654752440f));
-    const float r = fmaxf(x, 0.f);
-    return r * r;
-}
+// `plain_act` element by element.  VEC: MLR_VEC values in one access, or 1.
 template <int ACT, int VEC>
 __global__ void plain_act_kernel(const elem_t* __restrict__ x, elem_t* __restrict__ out, size_t count) {
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (size_t)gridDim.x * blockDim.x) {

@@ -6,8 +6,8 @@
 // Bfloat16 engine, three families, each with a fixed k order for every output element (so a row's result
 // does not depend on the rows beside it): up to 64 rows the weight is streamed once straight into
 // v_mfma_f32_16x16x32_bf16 (`gemm_skinny_kernel`, optionally with the residual add and RMSNorm in front
-// or silu(gate) * up behind); more rows with k a multiple of 64 go to `gemm_wide_kernel` (32x32 tiles
-// out of double-buffered LDS blocks); any other k to the plain 16x16-tile kernel `gemm_bf16_kernel`.
+// or silu(gate) * up behind); more rows with k a multiple of 64 go to `gemm_wide_kernel` (tiles out of
+// blocks of LDS that loads fill without passing through registers); any other k to the plain 16x16-tile kernel `gemm_bf16_kernel`.
 #include "common.h"
 #include <type_traits>
 
@@ -818,308 +818,428 @@ static int launch_skinny(const void* a, const void* w, void* out, int M, int N, 
     return launch_skinny_as<MT, GATED, 4, false, EPI>(a, w, out, M, N, K, out_float, 0, epi, stream);
 }
 
-// Many rows (prompt portions), K a multiple of 64: 32x32 tiles of v_mfma_f32_32x32x16_bf16, the operands
-// staged through LDS in blocks of 64 k, double-buffered: the loads of block i + 1 are asked for before the
-// products of block i and written to the other buffer after them, one barrier per block.
-// A workgroup has WM x WN wavefronts, each TM x TN tiles: it owns BM = 32 WM TM rows and BN = 32 WN TN
-// columns of the output.  The weight is the A operand of the instruction (its rows are output columns),
-// the activation the B operand, so a lane ends up with four consecutive columns n of one row m, as in the
-// kernels above (lane = 32 h + i: A holds row i, k slots 8 h .. 8 h + 7, B column i, the same k slots,
-// C column i, rows 8 j + 4 h + r in register 4 j + r).
-// Rows of a staged block lie 144 bytes apart (128 of data): the eight lanes that the LDS serves in one
-// cycle of a 16-byte read then hit different banks.  Every output element is one sum over k in ascending
-// order whatever M is.  GATED: w = [gate; up] of N rows each; a wavefront's weight tiles alternate between
-// the two, and silu(gate) * up is written (N columns).
-typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
+// Many rows (prompt portions, mixed steps), K a multiple of 64: 16x16 tiles of v_mfma_f32_16x16x32_bf16, the operands brought
+// to LDS in blocks of 64 k by loads that do not pass through registers (`buffer_load_dwordx4 .. lds`).  A workgroup has
+// WM x WN wavefronts of TM x TN tiles each: BM = 16 WM TM rows and BN = 16 WN TN columns of the output, and STAGES blocks of LDS:
+// while one block is multiplied the others are on their way.  The weight is the A operand of the instruction (its rows are
+// output columns), the activation the B operand, so a lane ends up with four consecutive columns n of one row m
+// (lane = 16 g + i: A holds row i, k slots 8 g .. 8 g + 7, B column i, the same k slots, C column i, rows 4 g + r in register r).
+//
+// What bounds it: at 2048 x 1024 x 2048 and the like a compute unit has one tile, and what counts is how many bytes of operands
+// it has under way (a block staged through registers, as this kernel's predecessor did it, gave two); on large products it is
+// the matrix cores at the clock that the card's power leaves them (counters on 2048 x 24576 x 4096: 69 % of the cycles' matrix
+// work at 1.73 GHz, bank conflicts 3 % of the LDS cycles).  Measured inside a graph, weights cold, against the predecessor (32x32
+// tiles, two blocks through registers) and the vendor library: 2048 x 1024 x 2048 12.2 us (library 16.3), 2048 x 1024 x 3072
+// 17.0 (21.1), 2048 x 4096 x 1024 19.6 (21.3), with gate and activation 2048 x 2 * 3072 x 1024 25.8 (predecessor 37.6),
+// 732 x 2048 x 2048 10.5 (13.1), 1533 x 4096 x 4096 47.9 (51.5), 2048 x 24576 x 4096 309-331 (278-352).
+//
+// A row of a block is 128 bytes, eight pieces of 16; a load writes 64 lanes' pieces side by side (eight rows), so rows cannot be
+// padded apart.  Instead piece p of row r lies at place p ^ (r & 7) -- the lane that fetches it is chosen accordingly --, and
+// the eight lanes that the LDS serves together read eight different banks.
+// Every output element is one sum over k in ascending order, 32 k an instruction, whatever M and the shape are.
+// GATED: w = [gate; up] of N rows each; a wavefront's weight tiles alternate between the two.
 #define WIDE_BK 64
-#define WIDE_PITCH (WIDE_BK + 8)
 
-template <int WM, int WN, int TM, int TN>
+template <int WM, int WN, int TM, int TN, int NS>
 struct WideShape {
-    static constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN, THREADS = 64 * WM * WN;
+    static constexpr int BM = 16 * WM * TM, BN = 16 * WN * TN, WAVES = WM * WN;
     static constexpr int ROWS = BM + BN;                          // staged rows per block: weight, then activation
-    static constexpr int PER_THREAD = ROWS * (WIDE_BK / 8) / THREADS;      // 16-byte pieces a thread stages
-    static constexpr size_t lds_bytes = 2 * (size_t)ROWS * WIDE_PITCH * sizeof(__bf16);
-    static_assert(ROWS * (WIDE_BK / 8) % THREADS == 0, "the staged pieces must divide among the threads");
+    static constexpr int LOADS = ROWS / 8 / WAVES;                // loads of a wavefront per block, eight rows each
+    static constexpr int STAGE = ROWS * WIDE_BK;                  // elements of a block
+    static constexpr size_t lds_bytes = (size_t)NS * STAGE * sizeof(__bf16);
+    static_assert(ROWS % (8 * WAVES) == 0, "a block's rows must divide among the wavefronts");
+    static_assert(lds_bytes <= 160 * 1024, "the blocks must fit the LDS");
+    static_assert(LOADS * (NS - 1) <= 63, "the counter of loads in flight has six bits");
 };
 
-template <int WM, int WN, int TM, int TN, bool OUT_FLOAT, bool GATED>
-__global__ __launch_bounds__(64 * WM * WN) void gemm_wide_kernel(const __bf16* __restrict__ a,
-                                                                 const __bf16* __restrict__ w,
-                                                                 void* __restrict__ out_raw, int M, int N, int K,
-                                                                 int tiles_m, int tiles_n) {
-    using S = WideShape<WM, WN, TM, TN>;
-    constexpr int BM = S::BM, BN = S::BN, THREADS = S::THREADS, ROWS = S::ROWS, PT = S::PER_THREAD;
+// This wavefront's loads but the last LEFT and all its LDS reads are done, and so are every other wavefront's: behind it the
+// block that those loads filled may be read and the block that those reads took from may be filled again.  The compiler does
+// not follow loads that go to LDS, so both waits are written out.
+template <int LEFT> __device__ __forceinline__ void wide_arrive() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LEFT) : "memory");
+}
+
+// What the epilogue does with the finished sums.  The activations after WIDE_SILU are those of the separate kernels, taken of the
+// products as those read them, rounded to bfloat16: the same bits as the two launches one after the other.
+enum { WIDE_PLAIN = 0, WIDE_SILU = 1, WIDE_SILU_ROUNDED = 2, WIDE_GELU_TANH = 3, WIDE_RELU = 4, WIDE_CLAMPED = 5,
+       WIDE_RELU_SQUARED = 6, WIDE_GELU_ERF = 7 };
+
+struct WideArgs {
+    const __bf16* a;
+    const __bf16* w;
+    void* out;
+    int M, N, K, tiles_m, tiles_n;
+    int act;              // WIDE_*
+    float limit, slope;   // of WIDE_CLAMPED
+    int vector_out;       // rows of the output start on 16 bytes
+};
+
+template <int WM, int WN, int TM, int TN, int NS, bool OUT_FLOAT, bool GATED>
+__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const WideArgs args) {
+    using S = WideShape<WM, WN, TM, TN, NS>;
+    constexpr int BM = S::BM, BN = S::BN, LOADS = S::LOADS;
     static_assert(!GATED || TN % 2 == 0, "gate and up tiles come in pairs");
     extern __shared__ __attribute__((aligned(16))) __bf16 wide_lds[];
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int li = lane & 31, h = lane >> 5;
+    const int M = args.M, N = args.N, K = args.K;
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int li = lane & 15, g = lane >> 4;
     const int wm = wave / WN, wn = wave % WN;
-    // Workgroups go to the 8 XCDs in turn; each XCD gets a contiguous range of tiles, and within it
-    // consecutive tiles share their columns, so a strip of the weight is fetched into one L2 once.
-    const int total = tiles_m * tiles_n;
-    int tile = blockIdx.x;
-    if (total % 8 == 0) tile = (tile % 8) * (total / 8) + tile / 8;
-    const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * BN;
-    // In the gated case a workgroup's BN staged weight rows are BN / 2 gate rows and BN / 2 up rows of the
-    // same output columns: staged row 32 j + i of wavefront column wn is gate (j even) or up (j odd).
-    constexpr int NOUT = GATED ? BN / 2 : BN;                     // output columns of the workgroup
-    const int c0 = GATED ? (tile / tiles_m) * NOUT : n0;
-
-    // What a thread stages per block: pieces t, t + THREADS, ... of 16 bytes; piece c is row c / 8 of the
-    // staged block (weight rows first), k 8 (c % 8) ..  The first PW pieces of a thread are weight, the
-    // others activation; their places are kept as 32-bit element offsets from the matrices' bases (the host
-    // refuses matrices of 2^31 elements and more), which keeps the loads' addresses out of the registers.
-    constexpr int STEP = THREADS / 8;                             // staged rows between a thread's pieces
-    static_assert(BN % STEP == 0, "a thread's pieces must not straddle weight and activation");
-    constexpr int PW = BN / STEP;
-    uint32_t src[PT];
-    const int dst0 = (t >> 3) * WIDE_PITCH + (t & 7) * 8;
-#pragma unroll
-    for (int i = 0; i < PT; ++i) {
-        const int row = (t >> 3) + STEP * i, kc = (t & 7) * 8;
-        if (i < PW) {
-            int n;
-            if (GATED) {
-                // staged weight row -> (wavefront column, tile j, row in tile); tile pairs (2 p, 2 p + 1) are
-                // gate and up of output columns c0 + wn_ * (TN / 2) * 32 + p * 32 ..
-                const int wn_ = row / (32 * TN), j = (row / 32) % TN, r = row % 32;
-                const int col = c0 + (wn_ * (TN / 2) + j / 2) * 32 + r;
-                n = min(col, N - 1) + (j & 1) * N;
-            } else {
-                n = min(n0 + row, N - 1);
-            }
-            src[i] = (uint32_t)n * (uint32_t)K + kc;
-        } else {
-            src[i] = (uint32_t)min(m0 + row - BN, M - 1) * (uint32_t)K + kc;
-        }
+    // Workgroups go to the 8 XCDs in turn; each XCD gets a contiguous range of tiles, and in it eight tiles of rows beside
+    // each other for every tile of columns, so that an L2 holds what its tiles share.
+    constexpr int GROUP = 8;
+    int tm, tn;
+    {
+        const int total = args.tiles_m * args.tiles_n, xcd = blockIdx.x % 8;
+        const int tile = xcd * (total / 8) + min(xcd, total % 8) + blockIdx.x / 8;
+        const int per = GROUP * args.tiles_n, first = tile / per * GROUP, rows = min(GROUP, args.tiles_m - first);
+        tm = first + tile % per % rows;
+        tn = tile % per / rows;
     }
-    // Two blocks are in flight from memory while a third is multiplied: with one, a compute unit has 64 KB
-    // on its way at any time, and the latency of the loads bounds the whole GPU at about 7 TB/s of operands.
-    bf16x8 stage0[PT], stage1[PT];
-    const int blocks = K / WIDE_BK;
-    auto fetch = [&](int kb, auto which) {                    // (blocks past the end fetch the last one again)
-        const __bf16* wk = w + (size_t)min(kb, blocks - 1) * WIDE_BK;
-        const __bf16* ak = a + (size_t)min(kb, blocks - 1) * WIDE_BK;
-#pragma unroll
-        for (int i = 0; i < PT; ++i) {
-            const bf16x8 v = *reinterpret_cast<const bf16x8*>((i < PW ? wk : ak) + src[i]);
-            if constexpr (decltype(which)::value == 0) stage0[i] = v; else stage1[i] = v;
-        }
-    };
-    auto stash = [&](int buf, auto which) {
-        __bf16* base = wide_lds + (size_t)buf * ROWS * WIDE_PITCH;
-#pragma unroll
-        for (int i = 0; i < PT; ++i) {
-            if constexpr (decltype(which)::value == 0) *reinterpret_cast<bf16x8*>(base + dst0 + i * STEP * WIDE_PITCH) = stage0[i];
-            else *reinterpret_cast<bf16x8*>(base + dst0 + i * STEP * WIDE_PITCH) = stage1[i];
-        }
-    };
-    constexpr std::integral_constant<int, 0> S0{};
-    constexpr std::integral_constant<int, 1> S1{};
+    constexpr int NOUT = GATED ? BN / 2 : BN;                     // output columns of the workgroup
+    const int m0 = tm * BM, n0 = tn * NOUT;
 
-    floatx16 acc[TN][TM];
+    // Load i of a wavefront brings rows 8 (wave LOADS + i) .. of the block (weight rows first, then rows of the activation; rows
+    // beyond a matrix are its last one again).  Places are 32-bit byte offsets from the matrices' bases (the host refuses
+    // matrices of 2^31 elements and more).
+    uint32_t src[LOADS];
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[j][i][e] = 0.f;
+    for (int i = 0; i < LOADS; ++i) {
+        const int row = (wave * LOADS + i) * 8 + (lane >> 3), piece = ((lane & 7) ^ (row & 7)) * 8;
+        int r;
+        if (row < BN) {
+            if (GATED) {
+                // staged weight row -> (wavefront column, tile j, row in tile); tile pairs (2 p, 2 p + 1) are gate and up
+                // of output columns n0 + wn_ * (TN / 2) * 16 + p * 16 ..
+                const int wn_ = row / (16 * TN), j = (row / 16) % TN;
+                r = min(n0 + (wn_ * (TN / 2) + j / 2) * 16 + row % 16, N - 1) + (j & 1) * N;
+            } else {
+                r = min(n0 + row, N - 1);
+            }
+        } else {
+            r = min(m0 + row - BN, M - 1);
+        }
+        src[i] = ((uint32_t)r * (uint32_t)K + piece) * 2u;
+    }
+    const auto w_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)args.w, 0, (int)((uint32_t)N * (GATED ? 2u : 1u) * (uint32_t)K * 2u), 0x00027000);
+    const auto a_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)args.a, 0, (int)((uint32_t)M * (uint32_t)K * 2u), 0x00027000);
+    auto load = [&](int i, int kb, int stage) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds((wave * LOADS + i) * 8 < BN ? w_rsrc : a_rsrc,
+                                                 (__attribute__((address_space(3))) void*)(wide_lds + stage * S::STAGE + (wave * LOADS + i) * 512),
+                                                 16, (int)src[i], kb * (WIDE_BK * 2), 0, 0);
+    };
 
-    auto products = [&](int buf) {
-        const __bf16* base = wide_lds + (size_t)buf * ROWS * WIDE_PITCH;
-        const __bf16* wb = base + (wn * TN * 32 + li) * WIDE_PITCH + 8 * h;
-        const __bf16* ab = base + (BN + wm * TM * 32 + li) * WIDE_PITCH + 8 * h;
-        // the operands of k step ks + 1 are asked for before the products of step ks
-        bf16x8 wf[2][TN], af[2][TM];
-        auto operands = [&](int ks, int set) {
+    floatx4 acc[TM][TN];
 #pragma unroll
-            for (int j = 0; j < TN; ++j) wf[set][j] = *reinterpret_cast<const bf16x8*>(wb + j * 32 * WIDE_PITCH + 16 * ks);
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int i = 0; i < TM; ++i) af[set][i] = *reinterpret_cast<const bf16x8*>(ab + i * 32 * WIDE_PITCH + 16 * ks);
-        };
-        operands(0, 0);
+        for (int j = 0; j < TN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    // The operands of one half of a block (32 k); the other half's are read while these are multiplied.
+    bf16x8 wf[2][TN], af[2][TM];
+    const int place[2] = {(g ^ (li & 7)) * 8, ((4 + g) ^ (li & 7)) * 8};
+    auto read = [&](int r, auto set_, int stage) {                // operand r of the half `set`
+        constexpr int set = decltype(set_)::value;
+        const __bf16* base = wide_lds + stage * S::STAGE + li * WIDE_BK + place[set];
+        if (r < TN) wf[set][r] = *reinterpret_cast<const bf16x8*>(base + (wn * TN + r) * 16 * WIDE_BK);
+        else af[set][r - TN] = *reinterpret_cast<const bf16x8*>(base + (BN + (wm * TM + r - TN) * 16) * WIDE_BK);
+    };
+    constexpr std::integral_constant<int, 0> H0{};
+    constexpr std::integral_constant<int, 1> H1{};
+    auto read_all = [&](auto set_, int stage) {
 #pragma unroll
-        for (int ks = 0; ks < WIDE_BK / 16; ++ks) {
-            if (ks + 1 < WIDE_BK / 16) operands(ks + 1, (ks + 1) & 1);
+        for (int r = 0; r < TM + TN; ++r) read(r, set_, stage);
+    };
+    // The products of half `set`; between them, when READ, the reads of the other half out of `from` (all but the last row of
+    // tiles are behind them, so that they are there when their turn comes) and, when LOAD, the loads of block kb into `into`.
+    // The scheduling barriers keep it so: on its own the compiler asks for everything first and multiplies then.
+    auto products = [&](auto set_, auto read_, int from, auto load_, int kb, int into) {
+        constexpr int set = decltype(set_)::value;
+        constexpr int OPERANDS = TM + TN, ROWS = TM > 1 ? TM - 1 : 1, PER_ROW = (OPERANDS + ROWS - 1) / ROWS;
+        constexpr int LOADS_ROW = (LOADS + TM - 1) / TM;
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            if constexpr (decltype(read_)::value) {
+#pragma unroll
+                for (int r = i * PER_ROW; r < (i + 1) * PER_ROW && r < OPERANDS; ++r) read(r, std::integral_constant<int, set ^ 1>{}, from);
+            }
+            if constexpr (decltype(load_)::value) {
+#pragma unroll
+                for (int l = i * LOADS_ROW; l < (i + 1) * LOADS_ROW && l < LOADS; ++l) load(l, kb, into);
+            }
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int j = 0; j < TN; ++j)
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-                    acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[ks & 1][j], af[ks & 1][i], acc[j][i], 0, 0, 0);
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[set][j], af[set][i], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
+        __builtin_amdgcn_s_setprio(0);
     };
 
-    fetch(0, S0);
-    fetch(1, S1);
-    stash(0, S0);
-    fetch(2, S0);
-    __syncthreads();
-    // block kb is multiplied out of buffer kb % 2; block kb + 1 goes from stage[(kb + 1) % 2] into the other
-    // buffer, whose readers passed the last barrier; block kb + 3 takes its place in the registers
-    // (two blocks per turn of the loop and no branch inside: the register stages keep their names, and
-    // the compiler counts the loads in flight exactly; with a branch it waits for all of them)
-    int kb = 0;
-#pragma unroll 1
-    for (; kb + 2 <= blocks; kb += 2) {
-        products(0);
-        stash(1, S1);
-        fetch(kb + 3, S1);
-        __syncthreads();
-        products(1);
-        stash(0, S0);
-        fetch(kb + 4, S0);
-        __syncthreads();
-    }
-    if (kb < blocks) products(0);
-
-    constexpr int TNO = GATED ? TN / 2 : TN;              // 32-column tiles of output per wavefront
-    // this lane's results for tile (i, j), rows 8 q + 4 h .. + 3 of the instruction's C (output columns)
-    auto result = [&](int i, int j, int q, float* y) {
+    const int blocks = K / WIDE_BK;
+    if (blocks >= NS) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            if (GATED) {
-                const float gate = acc[2 * j][i][4 * q + r], up = acc[2 * j + 1][i][4 * q + r];
-                // silu(g) = g / (1 + 2^(-g log2 e)), with the hardware's exponential and reciprocal (both good
-                // to an ulp or so of 32 bits; the result is rounded to bfloat16): a full division costs ten
-                // instructions, and a lane has 16 TM TN / 2 of these
-                y[r] = gate * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896340736f * gate)) * up;
-            } else {
-                y[r] = acc[j][i][4 * q + r];
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i) load(i, s, s);
+        wide_arrive<LOADS * (NS - 1)>();
+        read_all(H0, 0);
+        int stage = 0;
+        // A turn: the first half's products beside the second half's reads; the block is read out then and, once everyone is
+        // there, is filled again with block kb + NS beside the second half's products, while the next block's operands arrive.
+#pragma unroll 1
+        for (int kb = 0; kb < blocks - NS; ++kb) {
+            const int next = stage + 1 == NS ? 0 : stage + 1;
+            products(H0, std::true_type{}, stage, std::false_type{}, 0, 0);
+            wide_arrive<LOADS * (NS - 2)>();
+            products(H1, std::true_type{}, next, std::true_type{}, kb + NS, stage);
+            stage = next;
+        }
+        auto tail = [&](auto self, auto left_) {                  // the last NS blocks: nothing more to ask for
+            constexpr int LEFT = decltype(left_)::value;
+            if constexpr (LEFT > 0) {
+                const int next = stage + 1 == NS ? 0 : stage + 1;
+                products(H0, std::true_type{}, stage, std::false_type{}, 0, 0);
+                if constexpr (LEFT > 1) {
+                    wide_arrive<LOADS * (LEFT > 1 ? LEFT - 2 : 0)>();
+                    products(H1, std::true_type{}, next, std::false_type{}, 0, 0);
+                } else {
+                    products(H1, std::false_type{}, 0, std::false_type{}, 0, 0);
+                }
+                stage = next;
+                self(self, std::integral_constant<int, LEFT - 1>{});
+            }
+        };
+        tail(tail, std::integral_constant<int, NS>{});
+    } else {                                                      // fewer blocks than the LDS holds: all at once
+        for (int s = 0; s < blocks; ++s)
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i) load(i, s, s);
+        wide_arrive<0>();
+        for (int s = 0; s < blocks; ++s) {
+            read_all(H0, s);
+            read_all(H1, s);
+            products(H0, std::false_type{}, 0, std::false_type{}, 0, 0);
+            products(H1, std::false_type{}, 0, std::false_type{}, 0, 0);
+        }
+    }
+
+    if constexpr (OUT_FLOAT) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            const int m = m0 + (wm * TM + i) * 16 + li;
+            if (m >= M) continue;
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const int n = n0 + (wn * TN + j) * 16 + 4 * g;
+                float* o = (float*)args.out + (size_t)m * N + n;
+                if (args.vector_out && n + 3 < N) *reinterpret_cast<floatx4*>(o) = acc[i][j];
+                else
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) if (n + r < N) o[r] = acc[i][j][r];
             }
         }
-    };
-    const int wave_m0 = m0 + wm * TM * 32, wave_n0 = (GATED ? c0 : n0) + wn * TNO * 32;
-    if constexpr (!OUT_FLOAT) {
-        // bfloat16 results leave through LDS: a lane holds four columns of one row, which would be stores of
-        // 8 bytes to 64 different rows; a piece of LDS of the wavefront's own turns them into rows of 16-byte
-        // pieces, eight lanes a 128-byte line (measured on 2048 x 4096 x 1024: the stores took 8 of 28 us).
-        constexpr int COLS = TNO * 32, OPITCH = COLS + 8, ROWS_W = TM * 32;
-        static_assert((size_t)WM * WN * ROWS_W * OPITCH * sizeof(__bf16) <= S::lds_bytes, "the output tiles must fit the LDS");
-        __syncthreads();                                   // every wavefront has read its last operands
-        __bf16* mine = wide_lds + (size_t)wave * ROWS_W * OPITCH;
-        typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4_t;
+        return;
+    }
+    // bfloat16 results leave through LDS: a lane holds four columns of one row, which would be stores of 8 bytes to 64 different
+    // rows; a piece of LDS of the wavefront's own turns them into rows of 16-byte pieces (measured on 2048 x 4096 x 1024 with
+    // this kernel's predecessor: the stores took 8 of 28 us).  A wavefront's tiles take the LDS one half after the other
+    // where all of them do not fit.
+    constexpr int TNO = GATED ? TN / 2 : TN, COLS = TNO * 16, PITCH = TN * 16 + 8, PIECES = COLS / 8;
+    constexpr int TC = (size_t)S::WAVES * TM * 16 * PITCH * sizeof(__bf16) <= S::lds_bytes ? TM : TM / 2, HALF = TC * 16;
+    static_assert(TM % TC == 0 && (size_t)S::WAVES * HALF * PITCH * sizeof(__bf16) <= S::lds_bytes, "the output tiles must fit the LDS");
+    wide_arrive<0>();                                             // every wavefront has read its last operands
+    __bf16* mine = wide_lds + wave * HALF * PITCH;
+    const bool fused = GATED && args.act == WIDE_SILU;            // (its gate never leaves the registers)
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+    for (int i0 = 0; i0 < TM; i0 += TC) {
+        auto put = [&](int i, int j, float y0, float y1, float y2, float y3) {
+            typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4_t;
+            *reinterpret_cast<bf16x4_t*>(mine + (i * 16 + li) * PITCH + j * 16 + 4 * g) = bf16x4_t{(__bf16)y0, (__bf16)y1, (__bf16)y2, (__bf16)y3};
+        };
+        if (fused) {
 #pragma unroll
-            for (int j = 0; j < TNO; ++j)
+            for (int i = 0; i < TC; ++i)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
+                for (int j = 0; j < TN / 2; ++j) {
                     float y[4];
-                    result(i, j, q, y);
-                    *reinterpret_cast<bf16x4_t*>(mine + (i * 32 + li) * OPITCH + j * 32 + 8 * q + 4 * h) =
-                        bf16x4_t{(__bf16)y[0], (__bf16)y[1], (__bf16)y[2], (__bf16)y[3]};
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        // silu(g) = g / (1 + 2^(-g log2 e)), with the hardware's exponential and reciprocal (both good to an
+                        // ulp or so of 32 bits; the result is rounded to bfloat16): a full division costs ten instructions,
+                        // and a lane has 2 TM TN of these
+                        const float gate = acc[i0 + i][2 * j][r];
+                        y[r] = gate * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896340736f * gate)) * acc[i0 + i][(2 * j + 1) % TN][r];
+                    }
+                    put(i, j, y[0], y[1], y[2], y[3]);
                 }
+        } else {
+#pragma unroll
+            for (int i = 0; i < TC; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) put(i, j, acc[i0 + i][j][0], acc[i0 + i][j][1], acc[i0 + i][j][2], acc[i0 + i][j][3]);
+        }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        constexpr int PIECES = COLS / 8;                   // 16-byte pieces in a row of the wavefront's tile
-        const bool whole_n = (N & 7) == 0;
-#pragma unroll
-        for (int t0 = 0; t0 < ROWS_W * PIECES; t0 += 64) {
-            const int c = t0 + lane, row = c / PIECES, piece = c % PIECES;
-            const int m = wave_m0 + row, n = wave_n0 + 8 * piece;
+#pragma unroll 2
+        for (int c = lane; c < HALF * PIECES; c += 64) {
+            const int row = c / PIECES, piece = c % PIECES;
+            const int m = m0 + (wm * TM + i0) * 16 + row, n = n0 + wn * COLS + 8 * piece;
             if (m >= M || n >= N) continue;
-            const bf16x8 v = *reinterpret_cast<const bf16x8*>(mine + row * OPITCH + 8 * piece);
-            __bf16* o = (__bf16*)out_raw + (size_t)m * N + n;
-            if (whole_n && n + 8 <= N) {
+            const __bf16* from = mine + row * PITCH;
+            bf16x8 v;
+            if (!GATED || fused) {
+                v = *reinterpret_cast<const bf16x8*>(from + 8 * piece);
+                if (!GATED && args.act != WIDE_PLAIN) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        v[e] = (__bf16)(args.act == WIDE_RELU_SQUARED ? plain_act<0>((float)v[e]) : plain_act<1>((float)v[e]));
+                }
+            } else {                                              // gate and up lie in neighbouring tiles
+                from += (piece >> 1) * 32 + (piece & 1) * 8;
+                const bf16x8 gate = *reinterpret_cast<const bf16x8*>(from), up = *reinterpret_cast<const bf16x8*>(from + 16);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float x = (float)gate[e], u = (float)up[e];
+                    v[e] = (__bf16)(args.act == WIDE_CLAMPED ? clamped_glu(x, u, args.limit, args.slope)
+                                    : (args.act == WIDE_GELU_TANH ? gate_act<1>(x) : args.act == WIDE_RELU ? gate_act<2>(x) : gate_act<0>(x)) * u);
+                }
+            }
+            __bf16* o = (__bf16*)args.out + (size_t)m * N + n;
+            if (args.vector_out && n + 8 <= N) {
                 *reinterpret_cast<bf16x8*>(o) = v;
             } else {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) if (n + e < N) o[e] = v[e];
             }
         }
-    } else {
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-            const int m = wave_m0 + i * 32 + li;
-            if (m >= M) continue;
-#pragma unroll
-            for (int j = 0; j < TNO; ++j)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int n = wave_n0 + j * 32 + 8 * q + 4 * h;
-                    float y[4];
-                    result(i, j, q, y);
-                    float* o = (float*)out_raw + (size_t)m * N + n;
-                    if (n + 3 < N && (N & 3) == 0) *reinterpret_cast<float4*>(o) = float4{y[0], y[1], y[2], y[3]};
-                    else
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) if (n + r < N) o[r] = y[r];
-                }
+        if (TC < TM) {                                            // the second half's tiles overwrite what was just read
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
     }
 }
 
-template <int WM, int WN, int TM, int TN, bool GATED>
-static int launch_wide(const void* a, const void* w, void* out, int M, int N, int K, int out_float,
-                       hipStream_t stream) {
-    using S = WideShape<WM, WN, TM, TN>;
-    const int tiles_m = (M + S::BM - 1) / S::BM;
-    const int tiles_n = GATED ? (N + S::BN / 2 - 1) / (S::BN / 2) : (N + S::BN - 1) / S::BN;
-    if ((long long)tiles_m * tiles_n > 0x7fffffffLL) return -2;
-    if ((unsigned long long)M * K >= (1ull << 31) || (unsigned long long)N * (GATED ? 2 : 1) * K >= (1ull << 31)) return -3;
-#define MLR_WIDE_LAUNCH(OF)                                                                                   \
-    {                                                                                                         \
-        auto* kernel = gemm_wide_kernel<WM, WN, TM, TN, OF, GATED>;                                           \
-        static const hipError_t allowed = hipFuncSetAttribute(                                                \
-            reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds_bytes); \
-        if (allowed != hipSuccess) return (int)allowed;                                                       \
-        kernel<<<dim3(tiles_m * tiles_n), S::THREADS, S::lds_bytes, stream>>>(                                \
-            (const __bf16*)a, (const __bf16*)w, out, M, N, K, tiles_m, tiles_n);                              \
-    }
-    if (out_float) MLR_WIDE_LAUNCH(true) else MLR_WIDE_LAUNCH(false)
-#undef MLR_WIDE_LAUNCH
+template <int WM, int WN, int TM, int TN, int NS, bool OUT_FLOAT, bool GATED>
+static int launch_wide_as(WideArgs& args, hipStream_t stream) {
+    using S = WideShape<WM, WN, TM, TN, NS>;
+    constexpr int NOUT = GATED ? S::BN / 2 : S::BN;
+    args.tiles_m = (args.M + S::BM - 1) / S::BM;
+    args.tiles_n = (args.N + NOUT - 1) / NOUT;
+    if ((long long)args.tiles_m * args.tiles_n > 0x7fffffffLL / 8) return -2;
+    auto* kernel = gemm_wide_kernel<WM, WN, TM, TN, NS, OUT_FLOAT, GATED>;
+    static const hipError_t allowed = hipFuncSetAttribute(
+        reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds_bytes);
+    if (allowed != hipSuccess) return (int)allowed;
+    kernel<<<dim3(args.tiles_m * args.tiles_n), 64 * S::WAVES, S::lds_bytes, stream>>>(args);
     return (int)hipGetLastError();
 }
+// (the gated form where its tiles must come in pairs and the plain one's do not: the same workgroup tile, other wavefronts)
+template <int WM, int WN, int TM, int TN, int NS, int GWM = WM, int GWN = WN, int GTM = TM, int GTN = TN>
+static int launch_wide(WideArgs& args, bool out_float, bool gated, hipStream_t stream) {
+    static_assert(WM * TM == GWM * GTM && WN * TN == GWN * GTN, "one tile for both forms");
+    if (gated) return launch_wide_as<GWM, GWN, GTM, GTN, NS, false, true>(args, stream);
+    if (out_float) return launch_wide_as<WM, WN, TM, TN, NS, true, false>(args, stream);
+    return launch_wide_as<WM, WN, TM, TN, NS, false, false>(args, stream);
+}
 
-// The wide kernel's shapes, largest first: 256 x 256 (8 wavefronts), 128 x 256, 128 x 128 (two workgroups
-// a compute unit), 128 x 64 (rows x columns of the output; 64 x 64 in the gated case, whose last shape stages
-// 64 gate and 64 up rows).  The largest shape that still gives about a workgroup per compute unit wins:
-// measured at 2048 rows, 1.05 PFLOP/s on 24576 x 4096 with the first, 0.93-0.96 on 4096 x 4096 and
-// 4096 x 12288 with the second, 0.48-0.53 on 1024 x 2048 and 1024 x 3072 with the last (the vendor library:
-// 1.44, 1.18 and 0.56-0.64).
-#define WIDE_SHAPES 4
-template <bool GATED>
-static int launch_wide_shape(int shape, const void* a, const void* w, void* out, int M, int N, int K, int out_float,
-                             hipStream_t stream) {
+// The kernel's shapes: rows and columns of a workgroup's tile (gated: half as many output columns), workgroups that a compute
+// unit holds at once, and what 1024 k of a tile cost in microseconds, alone on its compute unit or beside a second one, with
+// what a launch costs besides: fitted to 168 products of 33 to 2048 rows and fourteen inner and outer sizes between 1024 and
+// 25600 (rms 9 to 13 % a shape; the shape with the least predicted time is then within 1 % of the best one on average).
+struct WideCost { int bm, bn, per_unit; float fixed, one, all; };
+#define WIDE_SHAPES 10
+static const WideCost WIDE_COSTS[WIDE_SHAPES] = {
+    {64, 32, 2, 1.2f, 2.9f, 4.9f},     {64, 64, 2, 1.0f, 3.9f, 6.9f},     {96, 64, 2, 0.6f, 4.6f, 8.8f},    {128, 64, 1, 0.3f, 0.f, 5.7f},
+    {128, 128, 1, -0.1f, 0.f, 8.1f},   {192, 128, 1, 1.2f, 0.f, 9.8f},    {128, 192, 1, 0.6f, 0.f, 10.4f},  {256, 128, 1, 1.9f, 0.f, 11.9f},
+    {256, 192, 1, -2.2f, 0.f, 19.4f},  {256, 256, 1, -1.1f, 0.f, 21.8f}};
+
+static int launch_wide_shape(int shape, WideArgs& args, bool out_float, bool gated, hipStream_t stream) {
     switch (shape) {
-        case 0: return launch_wide<2, 4, 4, 2, GATED>(a, w, out, M, N, K, out_float, stream);
-        case 1: return launch_wide<2, 4, 2, 2, GATED>(a, w, out, M, N, K, out_float, stream);
-        case 2: return launch_wide<2, 2, 2, 2, GATED>(a, w, out, M, N, K, out_float, stream);
-        case 3:
-            if constexpr (GATED) return launch_wide<2, 2, 1, 2, true>(a, w, out, M, N, K, out_float, stream);
-            else return launch_wide<2, 2, 2, 1, false>(a, w, out, M, N, K, out_float, stream);
+        case 0: return launch_wide<2, 2, 2, 1, 6, 4, 1, 1, 2>(args, out_float, gated, stream);
+        case 1: return launch_wide<2, 2, 2, 2, 5>(args, out_float, gated, stream);
+        case 2: return launch_wide<2, 2, 3, 2, 4>(args, out_float, gated, stream);
+        case 3: return launch_wide<4, 2, 2, 2, 6>(args, out_float, gated, stream);
+        case 4: return launch_wide<2, 4, 4, 2, 4>(args, out_float, gated, stream);
+        case 5: return launch_wide<4, 2, 3, 4, 3>(args, out_float, gated, stream);
+        case 6: return launch_wide<2, 4, 4, 3, 3, 4, 2, 2, 6>(args, out_float, gated, stream);
+        case 7: return launch_wide<4, 2, 4, 4, 3>(args, out_float, gated, stream);
+        case 8: return launch_wide<4, 2, 4, 6, 2>(args, out_float, gated, stream);
+        case 9: return launch_wide<2, 4, 8, 4, 2>(args, out_float, gated, stream);
         default: return -1;
     }
 }
 
-static int wide_shape_for(int M, int N, bool gated) {
-    static const int rows[WIDE_SHAPES] = {256, 128, 128, 128}, cols[WIDE_SHAPES] = {256, 256, 128, 64};
-    static int units = 0;
-    if (units == 0) {
-        int dev = 0;
-        hipDeviceProp_t prop;
-        units = (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess)
-                    ? prop.multiProcessorCount : 256;
-    }
+// The shape with the least predicted time, and that time in microseconds.
+static int wide_shape_for(int M, int N, int K, bool gated, float* time) {
+    const int units = compute_units() > 0 ? compute_units() : 256;
+    int best = 0;
     for (int s = 0; s < WIDE_SHAPES; ++s) {
-        const int bm = (gated && s == 3) ? 64 : rows[s], bn = gated ? (s == 3 ? 64 : cols[s] / 2) : cols[s];
-        const long long tiles = (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-        if (tiles * 10 >= (long long)units * 7) return s;
+        const WideCost& c = WIDE_COSTS[s];
+        const int bn = gated ? c.bn / 2 : c.bn;
+        const long long tiles = (long long)((M + c.bm - 1) / c.bm) * ((N + bn - 1) / bn), slots = (long long)units * c.per_unit;
+        const long long left = tiles % slots;
+        const bool alone = c.per_unit == 2 && left > 0 && left <= units;      // the last tiles have a compute unit each
+        const float rounds = (float)(tiles / slots + (left > 0 && !alone ? 1 : 0));
+        const float us = c.fixed + (rounds * c.all + (alone ? c.one : 0.f)) * (float)K * (1.0f / 1024.0f);
+        if (s == 0 || us < *time) {
+            best = s;
+            *time = us;
+        }
     }
-    return WIDE_SHAPES - 1;
+    return best;
 }
 
-// For tests and measurements: the wide kernel in a given shape (0 .. WIDE_SHAPES - 1; -1: the shape that
-// `mlr_gemm` would take), plain or gated.
+// Whether the kernel takes these operands at all: whole blocks of k, 32-bit offsets, rows that start on 16 bytes.
+static bool wide_takes(const void* a, const void* w, int M, int N, int K, bool gated) {
+    return K % WIDE_BK == 0 && (unsigned long long)M * K < (1ull << 31) && (unsigned long long)N * (gated ? 2 : 1) * K < (1ull << 31) &&
+           ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(w)) & 15) == 0;
+}
+
+static int run_wide(int shape, const void* a, const void* w, void* out, int M, int N, int K, bool out_float, int act, float limit,
+                    float slope, hipStream_t stream) {
+    const bool gated = act >= WIDE_SILU && act <= WIDE_CLAMPED;
+    WideArgs args{(const __bf16*)a, (const __bf16*)w, out, M, N, K, 0, 0, act, limit, slope, 0};
+    const uintptr_t row_bytes = (uintptr_t)N * (out_float ? 4 : 2);
+    args.vector_out = ((reinterpret_cast<uintptr_t>(out) | row_bytes) & 15) == 0 ? 1 : 0;
+    float time = 0.f;
+    return launch_wide_shape(shape < 0 ? wide_shape_for(M, N, K, gated, &time) : shape, args, out_float, gated, stream);
+}
+
+// For tests and measurements: the kernel in a given shape (0 .. WIDE_SHAPES - 1; -1: the shape that `mlr_gemm` would take),
+// plain or with gate and silu.
 extern "C" int mlr_gemm_wide(const void* a, const void* w, void* out, int M, int N, int K, int out_float,
                              int shape, int gated, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
-    if (K <= 0 || K % WIDE_BK != 0 || (gated && out_float)) return -1;
-    if (shape < 0) shape = wide_shape_for(M, N, gated != 0);
-    if (gated) return launch_wide_shape<true>(shape, a, w, out, M, N, K, 0, stream);
-    return launch_wide_shape<false>(shape, a, w, out, M, N, K, out_float, stream);
+    if (K <= 0 || (gated && out_float) || !wide_takes(a, w, M, N, K, gated != 0)) return -1;
+    return run_wide(shape, a, w, out, M, N, K, out_float != 0, gated ? WIDE_SILU : WIDE_PLAIN, 0.f, 0.f, stream);
+}
+
+// Whether more than 64 rows are this kernel's beside the vendor library (act: WIDE_*).  The library has the faster way on large
+// products (60 GFLOP and more) on which this kernel's tiles do not come out evenly: below a predicted 1.2 PFLOP/s.  (154
+// products of 97 to 2048 rows: 12 % less time than the library alone, geometric mean, where the better of both would be 14 %;
+// 0.53 to 1.18 of the library's time on the products that this takes.  2048 x 5120 x 25600: 525 us for the library's 427;
+// 1533 x 5120 x 25600: 345 for 513.)  An activation that would otherwise be a launch of its own, which reads the products and
+// writes its results at 4.5 TB/s, counts for the kernel.
+extern "C" int mlr_gemm_wide_wins(int M, int N, int K, int act) {
+    const bool gated = act >= WIDE_SILU && act <= WIDE_CLAMPED;
+    if (M <= 64 || N <= 0 || K <= 0 || !wide_takes(nullptr, nullptr, M, N, K, gated)) return 0;
+    float time = 0.f;
+    wide_shape_for(M, N, K, gated, &time);
+    const float gflop = 2e-9f * (float)M * (float)N * (float)K * (gated ? 2.f : 1.f);
+    const float launch = act == WIDE_PLAIN ? 0.f : 3.0f + 1e-6f * (float)M * (float)N * (gated ? 6.f : 4.f) / 4.5f;
+    return gflop < 60.f || time <= gflop / 1.2f + launch ? 1 : 0;
+}
+
+// out[M, N] = act of the products, act one of WIDE_SILU_ROUNDED .. (gated: w is [2N, K] = [gate; up]; limit and slope are
+// WIDE_CLAMPED's): the bits of the product followed by the activation's own kernel.
+extern "C" int mlr_gemm_activated(const void* a, const void* w, void* out, int M, int N, int K, int act, float limit, float slope,
+                                  hipStream_t stream) {
+    if (M <= 0 || N <= 0) return 0;
+    if (K <= 0 || act < WIDE_SILU_ROUNDED || act > WIDE_GELU_ERF || (act == WIDE_CLAMPED && !(limit > 0.f))) return -1;
+    if (!wide_takes(a, w, M, N, K, act <= WIDE_CLAMPED)) return -2;
+    return run_wide(-1, a, w, out, M, N, K, false, act, limit, slope, stream);
 }
 
 template <int WM, int WN, int TM, int TN>
@@ -1146,8 +1266,7 @@ extern "C" int mlr_gemm(const void* a, const void* w, void* out, int M, int N, i
     if (M <= 64 && N >= 16384) return launch<2, 2, 2, 2>(a, w, out, M, N, K, out_float, stream);
     if (M <= 32) return launch_skinny<2, false>(a, w, out, M, N, K, out_float, stream);
     if (M <= 64) return launch_skinny<4, false>(a, w, out, M, N, K, out_float, stream);
-    if (K % WIDE_BK == 0 && (unsigned long long)M * K < (1ull << 31) && (unsigned long long)N * K < (1ull << 31))
-        return launch_wide_shape<false>(wide_shape_for(M, N, false), a, w, out, M, N, K, out_float, stream);
+    if (wide_takes(a, w, M, N, K, false)) return run_wide(-1, a, w, out, M, N, K, out_float != 0, WIDE_PLAIN, 0.f, 0.f, stream);
     if (M <= 128) return launch<2, 2, 2, 2>(a, w, out, M, N, K, out_float, stream);  // 64 x 64
     return launch<2, 2, 4, 4>(a, w, out, M, N, K, out_float, stream);                // 128 x 128
 }
@@ -1162,8 +1281,7 @@ extern "C" int mlr_gemm_gated_silu(const void* a, const void* w, void* out, int 
     if (M <= 16) return launch_skinny<1, true>(a, w, out, M, N, K, 0, stream);
     if (M <= 32) return launch_skinny<2, true>(a, w, out, M, N, K, 0, stream);
     if (M <= 64) return launch_skinny<4, true>(a, w, out, M, N, K, 0, stream);
-    if (K % WIDE_BK == 0 && (unsigned long long)M * K < (1ull << 31) && 2ull * N * K < (1ull << 31))
-        return launch_wide_shape<true>(wide_shape_for(M, N, true), a, w, out, M, N, K, 0, stream);
+    if (wide_takes(a, w, M, N, K, true)) return run_wide(-1, a, w, out, M, N, K, false, WIDE_SILU, 0.f, 0.f, stream);
     return 1;
 }
 

@@ -22,7 +22,8 @@ _ptr = ctypes.c_void_p
 
 MAX_HEAD_DIM = 256          # the attention and rotation kernels keep head_dim / 64 values per lane
 ATTENTION_TILE_KEYS = 64
-LIBRARY_GEMM_MIN_ROWS = 16    # above this many rows the bfloat16 engine's projections go to the library
+LIBRARY_GEMM_MIN_ROWS = 16    # above this many rows the bfloat16 engine's projections may go to the library
+WIDE_CHOICES_KEPT = 4096      # products whose way (our kernel or the library) is remembered
 LIBRARY_GEMM_WORKSPACE = 128 << 20   # bytes of scratch memory that the library may use
 PREFILL_MAX_PAGES = 2048      # page ids of one group that the prompt-portion attention kernel keeps in LDS
 TILES_MAX_HEAD_DIM = 128      # the 32x32-tile kernel for prompt portions keeps two sets of accumulators per lane
@@ -83,6 +84,15 @@ def _ok(code, what):
         raise KernelError(f"{what}: launch failed with code {code}")
 
 
+def _on16(*tensors):
+    return all(t.data_ptr() % 16 == 0 for t in tensors)
+
+
+def _start16(t):
+    """t, or a copy of it where it does not start on 16 bytes (a view into a wider buffer)."""
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def _size(t):
     return 0 if t is None else t.numel() * t.element_size()
 
@@ -133,6 +143,7 @@ class Kernels:
         self.dtype = dtype
         self.library_gemm = library_gemm
         self._library_workspace = None      # scratch memory of the vendor library's products, allocated once
+        self._wide_choices = {}             # (rows, columns, inner size, activation) -> `wide_product`
         self._libs = {}
         self.profiler = None                # a `Profiler`: every launch is then bracketed by events
 
@@ -333,10 +344,10 @@ class Kernels:
         _need(out.dtype in (self.dtype, torch.float32), lambda: f"gemm: output type {out.dtype} not supported")
         _tensor(out, "out", out.dtype, (m, n))
         if library and self.library_gemm and self.dtype == torch.bfloat16 and m > LIBRARY_GEMM_MIN_ROWS and \
-                (out.dtype == torch.float32 or not self.streams_weight(m, k)):
-            # many rows: a plain matrix product, handed to the vendor library (hipBLASLt), as the reference
-            # hands its projections to cuBLAS (src/minillm/cuda/matrix.cpp:11-37).  (Float outputs are
-            # logits, a vocabulary wide: there the library wins from 17 rows on at any inner size.)
+                (out.dtype == torch.float32 or not (self.streams_weight(m, k) or (self.wide_product(m, n, k) and _on16(a, w)))):
+            # a plain matrix product, handed to the vendor library (hipBLASLt), as the reference hands its projections to
+            # cuBLAS (src/minillm/cuda/matrix.cpp:11-37), where neither the kernels for few rows nor the one for many take
+            # it.  (Float outputs are logits, a vocabulary wide: there the library wins from 17 rows on at any inner size.)
             ws = self.reserve_library_workspace(a.device)
             _ok(self._lib("library_gemm").mlr_library_gemm(_p(a), _p(w), _p(out), _c_int(m), _c_int(n), _c_int(k),
                                                            _c_int(1 if out.dtype == torch.float32 else 0),
@@ -366,14 +377,55 @@ class Kernels:
             return rows <= 64
         return rows <= LIBRARY_GEMM_MIN_ROWS or (rows <= 64 and k * ((rows + 15) // 16) <= 4096)
 
+    def wide_product(self, rows, columns, k, act=None):
+        """Whether the kernel for many rows (more than 64) takes a product of these sizes and not the vendor library;
+        `act`: with that activation in its epilogue, of `columns` gates beside as many ups or of the product itself."""
+        if self.dtype != torch.bfloat16 or rows <= 64:
+            return False
+        key = (rows, columns, k, act)
+        wins = self._wide_choices.get(key)
+        if wins is None:
+            kind = self.WIDE_ACTS[act]
+            wins = bool(self._lib("gemm").mlr_gemm_wide_wins(_c_int(rows), _c_int(columns), _c_int(k), _c_int(kind)))
+            if not self.library_gemm:
+                weight_rows = columns * (2 if 1 <= kind <= 5 else 1)
+                wins = k % 64 == 0 and rows * k < 2 ** 31 and weight_rows * k < 2 ** 31
+            if len(self._wide_choices) >= WIDE_CHOICES_KEPT:
+                self._wide_choices.clear()
+            self._wide_choices[key] = wins
+        return wins
+
+    # the epilogues of `gemm_activated` (csrc/gemm.hip, WIDE_*)
+    WIDE_ACTS = {None: 0, "silu": 2, "gelu_tanh": 3, "relu": 4, "clamped": 5, "relu_squared": 6, "gelu_erf": 7}
+
+    @timed("gemm", _gemm_work)
+    def gemm_activated(self, a, w, out, kind, limit=0.0, slope=0.0):
+        """The product and its activation in one launch, for the sizes of `wide_product`; the bits of `gemm` followed by
+        `silu_mul`, `gated_act_mul` or `clamped_glu` (w = [gate; up] stacked) or by `plain_act`."""
+        _need(self.dtype == torch.bfloat16, "gemm_activated: bfloat16 only")
+        _need(kind is not None and kind in self.WIDE_ACTS, f"gemm_activated: activation {kind!r}")
+        _tensor(a, "a", self.dtype, ndim=2)
+        _tensor(w, "w", self.dtype, ndim=2)
+        m, k = a.shape
+        n, k2 = w.shape
+        gated = kind not in ("relu_squared", "gelu_erf")
+        _need(k == k2 and (not gated or n % 2 == 0), "gemm_activated: sizes do not fit")
+        _need(k % 64 == 0 and a.numel() < 2 ** 31 and w.numel() < 2 ** 31,
+              "gemm_activated: the inner size must be a multiple of 64, matrices below 2^31 elements")
+        _need(kind != "clamped" or limit > 0, "gemm_activated: the clamp's limit must be positive")
+        n = n // 2 if gated else n
+        _tensor(out, "out", self.dtype, (m, n))
+        a, w = _start16(a), _start16(w)
+        _ok(self._lib("gemm").mlr_gemm_activated(_p(a), _p(w), _p(out), _c_int(m), _c_int(n), _c_int(k), _c_int(self.WIDE_ACTS[kind]),
+                                                 _c_float(limit), _c_float(slope), _stream()), "gemm_activated")
+
     def gated_silu_fused(self, rows, k=None):
         """Whether `gemm_gated_silu` is the path for this many rows and inner size: the bfloat16 engine, where
-        `streams_weight` says so (elsewhere the library's product and a separate activation are faster), and
-        without the library any number of rows when the inner size is a multiple of 64."""
+        `streams_weight` says so, and without the library any number of rows when the inner size is a multiple of 64."""
         if self.dtype == torch.bfloat16 and rows > 64 and k is not None and k % 64 == 0 and rows * k < 2 ** 31:
-            # many rows: the wide kernel's gated form.  Beside the library it is the faster way while the inner
-            # size is short (measured against the library's product followed by the activation kernel, at 128
-            # to 2048 rows: 0.58-0.95 of their time at k = 1024, 0.84-1.07 at k = 2048, 1.01-1.40 beyond)
+            # Many rows: the gate taken of the unrounded products.  Beside the library only where it has always been (short
+            # inner sizes); elsewhere `gemm_activated`, which takes it of the rounded ones as the library's product and
+            # the activation's kernel do: a router behind it must not see other values.
             return not self.library_gemm or k <= 1024 or (k <= 2048 and rows <= 256)
         return self.streams_weight(rows, k if k is not None else 1 << 30)
 
@@ -391,6 +443,8 @@ class Kernels:
         two_n, k2 = w.shape
         _need(k == k2 and two_n % 2 == 0, "gemm_gated_silu: sizes do not fit")
         _tensor(out, "out", self.dtype, (m, two_n // 2))
+        if m > 64:
+            a, w = _start16(a), _start16(w)
         fn = self._lib("gemm").mlr_gemm_gated_silu
         _ok(fn(_p(a), _p(w), _p(out), _c_int(m), _c_int(two_n // 2), _c_int(k), _stream()), "gemm_gated_silu")
 

@@ -65,6 +65,8 @@ class SwiGluMlp:
             ctx.kernels.gemm_gated_silu(x, self.gate_up, act)      # few rows: the activation rides on the projection
         elif s.activation != "silu" and m <= 64 and ctx.kernels.streams_weight(m, s.hidden):
             ctx.kernels.gemm_gated_act(x, self.gate_up, act, s.activation)
+        elif ctx.kernels.wide_product(m, s.intermediate, s.hidden, s.activation):
+            ctx.kernels.gemm_activated(x, self.gate_up, act, s.activation)
         else:
             gate_up = ctx.workspace.get("gate_up", (m, 2 * s.intermediate), x.dtype)
             ctx.kernels.gemm(x, self.gate_up, gate_up)
@@ -116,6 +118,8 @@ class ClampedGluMlp:
         act = ctx.workspace.get("act", (m, s.intermediate), x.dtype)
         if k.streams_weight(m, s.hidden):             # few rows: the activation rides on the projection
             k.gemm_gated_clamped(x, self.gate_up, act, float(s.limit), float(s.slope))
+        elif k.wide_product(m, s.intermediate, s.hidden, "clamped"):
+            k.gemm_activated(x, self.gate_up, act, "clamped", float(s.limit), float(s.slope))
         else:
             gate_up = ctx.workspace.get("gate_up", (m, 2 * s.intermediate), x.dtype)
             k.gemm(x, self.gate_up, gate_up)
@@ -160,6 +164,8 @@ class PlainMlp:
         act = ctx.workspace.get("act", (m, s.intermediate), x.dtype)
         if m <= 64 and k.streams_weight(m, s.hidden):      # few rows: the activation rides on the projection
             k.gemm_act(x, self.up, act, s.activation)
+        elif k.wide_product(m, s.intermediate, s.hidden, s.activation):
+            k.gemm_activated(x, self.up, act, s.activation)
         else:
             k.gemm(x, self.up, act)
             k.plain_act(act, act, s.activation)

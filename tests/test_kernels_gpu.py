@@ -293,6 +293,54 @@ def test_gemm_wide_every_shape(shape, gated, mnk):
     assert torch.equal(out, run(-1, torch.bfloat16))
 
 
+@pytest.mark.parametrize("mnk", [(1, 8, 64), (65, 36, 128), (97, 193, 320), (257, 385, 448), (300, 1001, 832), (513, 520, 1024)])
+def test_gemm_wide_tiles_and_epilogues(mnk):
+    """Every tile of the many-row kernel at sizes around its edges, from fewer blocks of k than the LDS holds to several
+    rounds of it: the plain product within the rounding of its 32-bit sums and of bfloat16, the same bits from every tile,
+    and every activation in the epilogue with the bits of the product and the activation's own launch."""
+    from mini_llm_runtime_amd.kernels.ops import _c_int, _p, _stream
+    m, n, kk = mnk
+    k = kernels(torch.bfloat16)
+    lib = k._lib("gemm")
+    a = rnd((m, kk), torch.bfloat16, 66)
+    w = rnd((2 * n, kk), torch.bfloat16, 67, 0.3)
+
+    def run(shape, gated=0):
+        out = torch.full((m, n if gated else 2 * n), float("nan"), dtype=torch.bfloat16, device="cuda")
+        assert lib.mlr_gemm_wide(_p(a), _p(w), _p(out), _c_int(m), _c_int(out.shape[1]), _c_int(kk), _c_int(0), _c_int(shape), _c_int(gated), _stream()) == 0
+        return out
+    product, silu = run(-1), run(-1, 1)
+    want = a.double() @ w.double().T
+    # a sum of kk products in 32 bits is off by at most kk roundings of 2^-24 of the sum of their sizes; bfloat16 adds 2^-9
+    bound = kk * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T) + 2.0 ** -8 * want.abs()
+    assert bool(((product.double() - want).abs() <= bound).all())
+    for shape in range(10):
+        assert torch.equal(run(shape), product) and torch.equal(run(shape, 1), silu), shape
+    two, one = torch.empty((m, n), dtype=torch.bfloat16, device="cuda"), torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    for kind in ("silu", "gelu_tanh", "relu", "clamped"):
+        if kind == "silu":
+            k.silu_mul(product, two)
+        elif kind == "clamped":
+            k.clamped_glu(product, two, 0.7, 1.702)
+        else:
+            k.gated_act_mul(product, two, kind)
+        k.gemm_activated(a, w, one, kind, 0.7, 1.702)
+        assert torch.equal(one, two), kind
+    for kind in ("relu_squared", "gelu_erf"):
+        whole = torch.empty_like(product)
+        k.plain_act(product, whole, kind)
+        got = torch.full_like(product, float("nan"))
+        k.gemm_activated(a, w, got, kind)
+        assert torch.equal(got, whole), kind
+    shifted = torch.empty(m * kk + 1, dtype=torch.bfloat16, device="cuda")[1:].view(m, kk).copy_(a)      # rows 2 bytes off
+    k.gemm_activated(shifted, w, one, "relu")
+    k.gated_act_mul(product, two, "relu")
+    assert torch.equal(one, two)
+    out = torch.full((m, 2 * n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    k.gemm(shifted, w, out)
+    assert bool(((out.double() - want).abs() <= bound).all())
+
+
 def test_gemm_wide_rows_do_not_depend_on_the_batch():
     """More than 64 rows with an inner size that is a multiple of 64: the tile shape follows the number of
     rows, a row's bits do not."""
