@@ -2,24 +2,24 @@
 //
 // A workgroup serves one group: consecutive tokens of one request for one kv head, as 32 NQ columns (token,
 // head): 32 NQ / g tokens, g = query heads per kv head, NQ = 4 or 2 (the smaller workgroup is for batches
-// that would not fill the GPU otherwise).  Its 2 NQ wavefronts are NQ column quarters (32 columns each)
-// times two key parities: keys are walked in blocks of 64 at absolute multiples of 64, staged once per
-// workgroup through LDS (two buffers, the loads of the next block in flight in registers), and of every
-// block the wavefronts of parity 0 take keys 0..31 and those of parity 1 keys 32..63.  The two parities of
-// a column are merged through LDS at the end.
+// that would not fill the GPU otherwise).  Keys are walked in blocks of 64 at absolute multiples of 64, brought to LDS once per
+// workgroup (two buffers: one multiplied, one on its way); a wavefront owns 32 columns and takes a block's keys 0..31 or 32..63
+// (two key parities, merged through LDS at the end) or, head size 128 and NQ = 4, both halves.
 //
-// What a tile costs (measured): about 2 000 cycles of its SIMD, whether one wavefront or two share the SIMD: the
-// last group of a 2 048-token prompt alone on the GPU (one wavefront a SIMD) takes 36.6 us for its 32 blocks, the
-// whole prompt 42-44 (two a SIMD most of the time), a prompt of 8 192 tokens 0.95 us a tile and SIMD; and a
-// workgroup of eight wavefronts that shares blocks of 128 keys between four key parities (half as many turns
-// for a group) takes as long as this one.  Counted per tile at long contexts: 128 vector instructions (a
-// dependent one issues every 9 cycles, independent ones every 6, an exponential every 10-13), 16 matrix
-// instructions (512 cycles), 47 scalar ones, 16 reads and 8 writes of 16 bytes a lane through the LDS (24 KB;
-// a wavefront's read takes 31 cycles) -- which add up rather than overlap (taking the softmax, the matrix
-// instructions or the staging out of the kernel shortens it by each one's own time).  So the loop counts its
-// instructions: offsets that do not change are computed once, a thread stages 32 contiguous bytes per page
-// lookup, blocks whose keys are all written are staged without checks, the maximum of a tile is taken three
-// values at a time.
+// Head size 128 (four wavefronts, two workgroups a compute unit): the blocks go to LDS by loads that do not pass registers, and
+// the loop over the blocks that a wavefront sees whole has nothing to check.  What bounds it is what a SIMD can issue for a tile
+// and how long a tile's chain is (first product, softmax, second product), not memory: per tile 16 matrix instructions (512
+// cycles), 58 vector and some 25 scalar ones; counters at 10 000 keys of context (kernel of 237 us): matrix cores 42 % of the
+// cycles, LDS 22 %, no bank conflicts.  Measured (16 query heads over 8, pages of 16; the kernel that staged through registers,
+// eight wavefronts of 128 columns, in brackets): 2048 tokens 32.7 us with 64 columns (42.5), behind 10 240 keys 201 (232);
+// 32 query heads over 8, 2048 tokens behind 8192 keys 292 us with 128 columns (332), 64 over 8, 1501 tokens 56.5 (77); 4096 tokens
+// of 16 heads behind 8192 keys 333-351 (448).  A softmax's wavefront goes before the others of its SIMD (`s_setprio`, 3 %): its
+// chain is the longer one.  Measured and taken out: wavefronts of the two parities half a turn apart, a barrier at every half, so
+// that one multiplies while the other is in its softmax (250 us for 232); four blocks of LDS, three on their way, in
+// one workgroup of eight wavefronts (237).
+//
+// Other head sizes: 4 NQ / 2 wavefronts, staged through registers: a thread stages 32 contiguous bytes per page lookup, blocks
+// whose keys are all written are staged without checks.
 //
 // Per tile of 32 keys, with v_mfma_f32_32x32x16_bf16:
 //   S^T[key][column]  = K[key][d] . Q^T[d][column]         A = 32 keys x 16 channels from LDS, B = Q (registers)
@@ -28,9 +28,10 @@
 //                                                           sit in B's register layout already
 // Register layouts of that instruction, lane = 32 h + n: A holds row n, k-slots 8 h .. 8 h + 7; B holds
 // column n, the same k-slots; C holds column n, rows 8 j + 4 h + r for j, r in 0..3 (register 4 j + r).
-// So registers 8 m .. 8 m + 7 of S^T are the keys 16 m + 8 a + 4 h + r (a = 0, 1) of the tile: the values
-// are laid out in LDS with those keys side by side (position 16 m + 8 h + 4 a + r), and one 16-byte read
-// gives the matching A operand.
+// So registers 8 m .. 8 m + 7 of S^T are the rows 16 m + 8 a + 4 h + r (a = 0, 1) of the tile.  Staged through registers, row =
+// key, and the values are laid out in LDS with those keys side by side (position 16 m + 8 h + 4 a + r); head size 128, the row
+// is the key with bits 2 and 3 swapped, and the registers are neighbouring keys.  Either way one 16-byte read gives the
+// matching A operand.
 //
 // Softmax in the base-2 domain, 32-bit.  A column's reference maximum is only raised when a tile's maximum
 // exceeds it by more than 2^8 (probabilities then stay below 256, far from overflow; the quotient at the
@@ -49,6 +50,8 @@
 // of two, groups whose keys span more than PAGE_IDS pages.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
@@ -78,14 +81,19 @@ struct TileArgs {
     int single;                  // host: the caller's `pairing`; kernel: 1 every workgroup takes one group, 0 two (group i and group groups - 1 - i)
 };
 
+// DIRECT (head size 128): blocks go straight from memory to LDS (see `tile_group`).
 template <int ND, int NQ>
 struct TileShape {
+    static constexpr bool DIRECT = ND == 8;
+    static constexpr int TILES = DIRECT && NQ == 4 ? 2 : 1;   // tiles of a block that a wavefront takes
+    static constexpr int PARITIES = 2 / TILES;
     static constexpr int D = 16 * ND;
     static constexpr int DB = (ND + 1) / 2;               // blocks of 32 channels
-    static constexpr int THREADS = 128 * NQ;
-    static constexpr int KPITCH = D + 8;                  // elements per key row of a staged block of keys
+    static constexpr int THREADS = 64 * NQ * PARITIES;
+    static constexpr int KPITCH = DIRECT ? D : D + 8;     // elements per key row of a staged block of keys
     static constexpr int KBUF = BLOCK_KEYS * KPITCH;      // elements
-    static constexpr int VBUF = 32 * DB * VPITCH;
+    static constexpr int VBUF = DIRECT ? BLOCK_KEYS * D : 32 * DB * VPITCH;
+    static constexpr int LOADS = 16 / (THREADS / 64);           // DIRECT: a wavefront's loads of 1 KB for a block's keys, and as many for its values
     static constexpr int KSTEP = THREADS / ND;            // keys that the workgroup stages per pass
     static constexpr int VSTEP = THREADS / D;             // 16-key groups of values per pass
     static constexpr int K_PASSES = (BLOCK_KEYS + KSTEP - 1) / KSTEP;
@@ -104,6 +112,10 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
     return r;
 }
 
+// This wavefront's loads to LDS and its LDS reads are done, and so are every other wavefront's (the compiler does not follow
+// loads that go to LDS).
+__device__ __forceinline__ void tile_arrive() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 template <int ND, int NQ>
 __device__ __forceinline__ void tile_group(const TileArgs& a, int grp, int kvh, int split, unsigned char* lds_raw) {
     using S = TileShape<ND, NQ>;
@@ -115,7 +127,7 @@ __device__ __forceinline__ void tile_group(const TileArgs& a, int grp, int kvh, 
 
     const int P = a.page_size, pshift = a.page_shift;
     const int g = a.q_heads / a.kv_heads, cap = (32 * NQ) / g;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 31, h = lane >> 5;
     const int cq = wave % NQ, kp = wave / NQ;                  // column quarter, key parity
     const int row0 = a.group_row0[grp], ntok = min(a.group_ntok[grp], cap);
@@ -154,6 +166,8 @@ __device__ __forceinline__ void tile_group(const TileArgs& a, int grp, int kvh, 
         }
     }
     float m_ref = -INFINITY, l_run = 0.f;
+    float m_use = -1e30f, raise_at = -INFINITY;      // m_ref as it is subtracted (a column with no key yet: exp2(-inf - finite) = 0, not NaN);
+                                                     // the score above which it is raised
     floatx16 o[DB];
 #pragma unroll
     for (int db = 0; db < DB; ++db)
@@ -177,137 +191,39 @@ __device__ __forceinline__ void tile_group(const TileArgs& a, int grp, int kvh, 
         all_mapped = __syncthreads_and(mine_mapped) != 0;
     }
 
-    // What a thread stages per block and pass: 32 bytes of the keys (16 channels of one key) and 32 bytes of
-    // the values (16 keys of one channel; a page's values of one kv head are contiguous in the order
-    // (channel, key)), so one page id and one address serve two 16-byte loads each.
-    constexpr int KSTEP = S::KSTEP, VSTEP = S::VSTEP, KN = S::K_PASSES, VN = S::V_PASSES;
-    const int k_key0 = threadIdx.x / ND, k_c16 = threadIdx.x % ND;
-    const bool k_thread = (int)threadIdx.x < KSTEP * ND;
-    const int v_m0 = threadIdx.x / D, v_d = threadIdx.x % D;
-    const bool v_thread = (int)threadIdx.x < VSTEP * D;
-    const bool big_page = P > BLOCK_KEYS;                   // a block lies within one page
-    const uint32_t page_stride = (uint32_t)a.kv_heads * P * D;      // elements; the host keeps offsets within 32 bits
-    int k_key[KN], k_pageadd[KN], v_m16[VN], v_pageadd[VN];
-    uint32_t k_off0[KN], v_off0[VN];
-#pragma unroll
-    for (int i = 0; i < KN; ++i) {
-        k_key[i] = min(k_key0 + KSTEP * i, BLOCK_KEYS - 1);
-        k_pageadd[i] = big_page ? 0 : k_key[i] >> pshift;
-        k_off0[i] = (uint32_t)kvh * P * D + (big_page ? k_key[i] : (k_key[i] & (P - 1))) * D + 16 * k_c16;
-    }
-#pragma unroll
-    for (int i = 0; i < VN; ++i) {
-        v_m16[i] = min(v_m0 + VSTEP * i, BLOCK_KEYS / 16 - 1);
-        v_pageadd[i] = big_page ? 0 : (16 * v_m16[i]) >> pshift;
-        v_off0[i] = (uint32_t)kvh * P * D + v_d * P + (big_page ? 16 * v_m16[i] : ((16 * v_m16[i]) & (P - 1)));
-    }
-    struct Staged {
-        bf16x8 k[KN][2], v[VN][2];
-        int tb;
-        unsigned v_ok;               // bit i: pass i's page is mapped and its first key written
-        bool whole;                  // every key of the block is written and mapped: nothing to check or zero
-    };
-    // global -> registers.  No branch around a load (a load behind a branch makes the compiler wait for
-    // every load in flight): addresses are clamped to valid memory, and what must read as zero is zeroed
-    // when the registers go to LDS.  Only the pages of written keys were looked up: anything later counts
-    // as not mapped.
-    auto fetch = [&](int blk, Staged& st) {
-        const int tb = blk * BLOCK_KEYS;
-        st.tb = tb;
-        const int pidx = (tb >> pshift) - first_page;
-        const uint32_t inpage = big_page ? (tb & (P - 1)) : 0;
-        // (all blocks but a group's last, unless a window has given pages back: the same for every thread)
-        st.whole = all_mapped && a.window <= 0 && tb + BLOCK_KEYS <= ke;
-        if (st.whole) {
-#pragma unroll
-            for (int i = 0; i < KN; ++i) {
-                const int pg = page_lds[pidx + k_pageadd[i]];
-                const __bf16* kptr = a.k_pages + (__umul24(pg, page_stride) + inpage * D + k_off0[i]);
-                st.k[i][0] = *reinterpret_cast<const bf16x8*>(kptr);
-                st.k[i][1] = *reinterpret_cast<const bf16x8*>(kptr + 8);
-            }
-#pragma unroll
-            for (int i = 0; i < VN; ++i) {
-                const int pg = page_lds[pidx + v_pageadd[i]];
-                const __bf16* vptr = a.v_pages + (__umul24(pg, page_stride) + inpage + v_off0[i]);
-                st.v[i][0] = *reinterpret_cast<const bf16x8*>(vptr);
-                st.v[i][1] = *reinterpret_cast<const bf16x8*>(vptr + 8);
-            }
-            st.v_ok = ~0u;
-            return;
-        }
-        unsigned ok = 0;
-#pragma unroll
-        for (int i = 0; i < KN; ++i) {
-            const int raw = page_lds[min(pidx + k_pageadd[i], PAGE_IDS - 1)];
-            const int pg = tb + k_key[i] < ke ? raw : 0;
-            const __bf16* kptr = a.k_pages + (__umul24(max(pg, 0), page_stride) + inpage * D + k_off0[i]);
-            st.k[i][0] = *reinterpret_cast<const bf16x8*>(kptr);
-            st.k[i][1] = *reinterpret_cast<const bf16x8*>(kptr + 8);
-        }
-#pragma unroll
-        for (int i = 0; i < VN; ++i) {
-            const int raw = page_lds[min(pidx + v_pageadd[i], PAGE_IDS - 1)];
-            const int pg = tb + 16 * v_m16[i] < ke ? raw : -1;
-            ok |= (pg >= 0 ? 1u : 0u) << i;
-            const __bf16* vptr = a.v_pages + (__umul24(max(pg, 0), page_stride) + inpage + v_off0[i]);
-            st.v[i][0] = *reinterpret_cast<const bf16x8*>(vptr);
-            st.v[i][1] = *reinterpret_cast<const bf16x8*>(vptr + 8);
-        }
-        st.v_ok = ok;
-    };
-    auto stash = [&](int buf, const Staged& st) {      // registers -> LDS
-        if (k_thread) {
-            __bf16* kb = k_lds + buf * S::KBUF + k_key0 * KPITCH + 16 * k_c16;
-#pragma unroll
-            for (int i = 0; i < KN; ++i) {
-                if (KN * KSTEP > BLOCK_KEYS && k_key0 + KSTEP * i >= BLOCK_KEYS) continue;
-                *reinterpret_cast<bf16x8*>(kb + KSTEP * i * KPITCH) = st.k[i][0];
-                *reinterpret_cast<bf16x8*>(kb + KSTEP * i * KPITCH + 8) = st.k[i][1];
-            }
-        }
-        if (v_thread) {
-            __bf16* vb = v_lds + buf * S::VBUF + v_d * VPITCH + 16 * v_m0;
-#pragma unroll
-            for (int i = 0; i < VN; ++i) {
-                if (VN * VSTEP > BLOCK_KEYS / 16 && v_m0 + VSTEP * i >= BLOCK_KEYS / 16) continue;
-                bf16x8 v0 = st.v[i][0], v1 = st.v[i][1];
-                const int key0 = st.tb + 16 * (v_m0 + VSTEP * i);
-                const bool ok = (st.v_ok >> i) & 1;
-                if (!st.whole && !(ok && key0 + 16 <= ke)) {
-                    // values of keys that are not written yet, or of a page that was given back (behind a
-                    // window), count as zero: their probability is zero, but zero times whatever the
-                    // memory holds need not be
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        if (!ok || key0 + e >= ke) v0[e] = (__bf16)0.f;
-                        if (!ok || key0 + 8 + e >= ke) v1[e] = (__bf16)0.f;
-                    }
-                }
-                // keys 8 a + 4 h + r of the 16 go to position 8 h + 4 a + r
-                *reinterpret_cast<bf16x8*>(vb + 16 * VSTEP * i) =
-                    bf16x8{v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
-                *reinterpret_cast<bf16x8*>(vb + 16 * VSTEP * i + 8) =
-                    bf16x8{v0[4], v0[5], v0[6], v0[7], v1[4], v1[5], v1[6], v1[7]};
-            }
-        }
-    };
-
     const float c2 = a.scale * 1.44269504088896340736f;     // scores in the base-2 domain: one v_exp_f32 each
     // a tile's scores -> probabilities (as B operands), updating the column's reference, sum and accumulators
-    auto softmax = [&](floatx16& sc, int tb, bool interior, bf16x8* pf) {
+    auto softmax = [&](auto& sc, int tb, bool interior, auto& pf) {
+        constexpr int T = sizeof(sc) / sizeof(sc[0]);         // tiles, one behind the other
         if (!interior) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int key = tb + 8 * (i >> 2) + 4 * h + (i & 3);
-                sc[i] = (key >= kbegin_c && key < kend_c) ? sc[i] : -INFINITY;
+            for (int t = 0; t < T; ++t)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const int key = tb + 32 * t + (S::DIRECT ? 16 * (i >> 3) + 8 * h + (i & 7) : 8 * (i >> 2) + 4 * h + (i & 3));
+                    sc[t][i] = (key >= kbegin_c && key < kend_c) ? sc[t][i] : -INFINITY;
+                }
+        }
+        // (the compiler does not count an asm among the readers of a matrix instruction's result, which must wait: eight passes,
+        // twelve slots; behind the mask it has seen to it)
+        if (interior) {
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                if (t == 0) asm volatile("s_nop 11" : "+v"(sc[t]));
+                else asm volatile("" : "+v"(sc[t]));
             }
         }
-        float mx = max3(max3(sc[0], sc[1], sc[2]), max3(sc[3], sc[4], sc[5]), max3(sc[6], sc[7], sc[8]));
-        mx = max3(mx, max3(sc[9], sc[10], sc[11]), max3(sc[12], sc[13], sc[14]));
-        mx = fmaxf(mx, sc[15]) * c2;                    // c2 > 0
-        if (__builtin_amdgcn_ballot_w64(mx > m_ref + RAISE_BY) != 0) {
-            const float full = fmaxf(mx, __shfl_xor(mx, 32, 64));     // the column's maximum in this tile
+        float mx = max3(sc[0][0], sc[0][1], sc[0][2]);
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+#pragma unroll
+            for (int i = t == 0 ? 3 : 0; i + 6 <= (t == 0 ? 15 : 12); i += 6)
+                mx = max3(mx, max3(sc[t][i], sc[t][i + 1], sc[t][i + 2]), max3(sc[t][i + 3], sc[t][i + 4], sc[t][i + 5]));
+            if (t == 0) mx = max3(mx, sc[t][15], sc[t][15]);
+            else mx = max3(mx, max3(sc[t][12], sc[t][13], sc[t][14]), sc[t][15]);
+        }
+        if (__builtin_amdgcn_ballot_w64(mx > raise_at) != 0) {
+            const float full = fmaxf(mx, __shfl_xor(mx, 32, 64)) * c2;     // the column's maximum in this tile (c2 > 0)
             if (full > m_ref + RAISE_BY) {                             // the same in both lanes of a column
                 const float corr = __builtin_amdgcn_exp2f(m_ref - full);      // -inf - finite: 0
                 l_run *= corr;
@@ -316,21 +232,24 @@ __device__ __forceinline__ void tile_group(const TileArgs& a, int grp, int kvh, 
 #pragma unroll
                     for (int i = 0; i < 16; ++i) o[db][i] *= corr;
                 m_ref = full;
+                m_use = fmaxf(full, -1e30f);
+                raise_at = (full + RAISE_BY) / c2;
             }
         }
-        const float m_use = fmaxf(m_ref, -1e30f);       // a column with no key yet: exp2(-inf - finite) = 0, not NaN
         // (the sum is taken over the probabilities as the second product sees them, rounded to bfloat16, two
         // at a time: v_dot2c_f32_bf16 with a pair of ones, half the instructions of single additions)
         const bf16x2 ones = {(__bf16)1.0f, (__bf16)1.0f};
         float psum = 0.f;
 #pragma unroll
-        for (int m = 0; m < 2; ++m) {
+        for (int t = 0; t < T; ++t)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) pf[m][e] = (__bf16)__builtin_amdgcn_exp2f(fmaf(sc[8 * m + e], c2, -m_use));
+            for (int m = 0; m < 2; ++m) {
 #pragma unroll
-            for (int e = 0; e < 8; e += 2)
-                psum = __builtin_amdgcn_fdot2_f32_bf16(bf16x2{pf[m][e], pf[m][e + 1]}, ones, psum, false);
-        }
+                for (int e = 0; e < 8; ++e) pf[t][m][e] = (__bf16)__builtin_amdgcn_exp2f(fmaf(sc[t][8 * m + e], c2, -m_use));
+#pragma unroll
+                for (int e = 0; e < 8; e += 2)
+                    psum = __builtin_amdgcn_fdot2_f32_bf16(bf16x2{pf[t][m][e], pf[t][m][e + 1]}, ones, psum, false);
+            }
         l_run += psum;
     };
 
@@ -345,11 +264,11 @@ __device__ __forceinline__ void tile_group(const TileArgs& a, int grp, int kvh, 
 #pragma unroll
         for (int st = 0; st < ND; ++st) kf[st] = *reinterpret_cast<const bf16x8*>(kb + 16 * st);
         __builtin_amdgcn_sched_barrier(0);
-        floatx16 sc;
+        floatx16 sc[1];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) sc[i] = 0.f;
+        for (int i = 0; i < 16; ++i) sc[0][i] = 0.f;
 #pragma unroll
-        for (int st = 0; st < ND; ++st) sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[st], qf[st], sc, 0, 0, 0);
+        for (int st = 0; st < ND; ++st) sc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[st], qf[st], sc[0], 0, 0, 0);
         bf16x8 vf[DB][2];
 #pragma unroll
         for (int db = 0; db < DB; ++db)
@@ -358,36 +277,301 @@ __device__ __forceinline__ void tile_group(const TileArgs& a, int grp, int kvh, 
         __builtin_amdgcn_sched_barrier(0);
         // a tile that every token of this wavefront sees whole needs no mask (all but the last few)
         const bool interior = tb + TILE_KEYS <= wave_first_kend && tb >= wave_last_kbegin;
-        bf16x8 pf[2];
+        bf16x8 pf[1][2];
         softmax(sc, tb, interior, pf);
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
             for (int m = 0; m < 2; ++m)
-                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[db][m], pf[m], o[db], 0, 0, 0);
+                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[db][m], pf[0][m], o[db], 0, 0, 0);
     };
 
-    // Two blocks are under way at any time: one being multiplied out of LDS, the next in flight from memory
-    // into registers.  One barrier per block suffices with two LDS buffers: a wavefront can only reach the
-    // second write of a buffer after the barrier that follows every wavefront's read of it.  Fetches are
-    // unconditional, clamped to the last block.
-    {
-        Staged st;
-        const int last = blk_end - 1;
-        fetch(blk_begin, st);
-        int buf = 0;
-        for (int blk = blk_begin; blk < blk_end; ++blk) {
-            stash(buf, st);
-            fetch(min(blk + 1, last), st);
-            __syncthreads();
-            compute(blk, buf);
-            buf ^= 1;
+    if constexpr (S::DIRECT) {
+        // A block of 64 keys is 16 KB of keys and 16 KB of values, 32 loads of 1 KB that go from memory to LDS without passing
+        // registers (`buffer_load_dwordx4 .. lds`: a lane's 16 bytes from an address of its own, the 64 lanes' side by side in
+        // LDS); a wavefront's share is one run of 16 keys, so lies in one page.  What is permuted is which lane asks for what:
+        // row r of the block (row r of a tile of the first product) is the key with bits 2 and 3 of r swapped, so that a
+        // lane's probabilities are eight neighbouring keys and the values can stay as the cache holds them, and 16-byte
+        // piece p of row r lies at place p ^ (r & 15); of a channel's two pieces of eight keys the first lies second
+        // where bits 2 and 3 of the channel differ.  Lanes that the LDS serves together then read different banks.
+        // While one block is multiplied the next is on its way; the loop's two turns have a buffer each, so that an operand's
+        // address is a register that does not change and a constant.
+        constexpr int LOADS = S::LOADS, BLOCK = S::KBUF + S::VBUF, T = S::TILES;
+        uint32_t k_at[LOADS], v_at[LOADS];
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            const int r = 4 * i + (lane >> 4), d = 32 * i + (lane >> 1);        // of the run
+            const int key = (r & 3) | (r & 4) << 1 | (r & 8) >> 1;
+            k_at[i] = (uint32_t)(key * D + 8 * ((lane & 15) ^ r)) * 2u;
+            v_at[i] = (uint32_t)(d * P + 8 * ((lane & 1) ^ ((d >> 2 ^ d >> 3) & 1))) * 2u;
+        }
+        const uint32_t head_bytes = (uint32_t)P * D * 2, page_bytes = head_bytes * a.kv_heads;   // (page strides below 2^24 elements)
+        const unsigned char* k_head = reinterpret_cast<const unsigned char*>(a.k_pages) + (size_t)kvh * head_bytes;
+        const unsigned char* v_head = reinterpret_cast<const unsigned char*>(a.v_pages) + (size_t)kvh * head_bytes;
+        auto page_of = [&](int blk) {                     // (behind the range, or a page that is not there: page 0, cleared below)
+            const int key0 = blk * BLOCK_KEYS + 16 * wave;
+            return __builtin_amdgcn_readfirstlane(key0 < ke ? max(page_lds[min((key0 >> pshift) - first_page, PAGE_IDS - 1)], 0) : 0);
+        };
+        auto ask = [&](int blk, int page, int buf) {
+            const int in_page = (blk * BLOCK_KEYS + 16 * wave) & (P - 1);
+            const uint64_t at = (uint64_t)(uint32_t)page * page_bytes;
+            const auto kr = __builtin_amdgcn_make_buffer_rsrc((void*)(k_head + at), 0, (int)head_bytes, 0x00027000);
+            const auto vr = __builtin_amdgcn_make_buffer_rsrc((void*)(v_head + at), 0, (int)head_bytes, 0x00027000);
+            __bf16* to = k_lds + buf * BLOCK + wave * LOADS * 512;
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(kr, (__attribute__((address_space(3))) void*)(to + i * 512), 16, (int)k_at[i], in_page * (D * 2), 0, 0);
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(vr, (__attribute__((address_space(3))) void*)(to + S::KBUF + i * 512), 16, (int)v_at[i], in_page * 2, 0, 0);
+        };
+        // Values of keys that are not written yet, or of a page that was given back (behind a window), count as zero: their
+        // probability is zero, but zero times whatever the memory holds need not be.
+        auto clear_values = [&](int blk, int buf) {
+            __bf16* vb = k_lds + buf * BLOCK + S::KBUF;
+            for (int piece = threadIdx.x; piece < S::VBUF / 8; piece += THREADS) {
+                const int m = piece / (2 * D), d = piece / 2 % D, half = (piece & 1) ^ ((d >> 2 ^ d >> 3) & 1);
+                const int key0 = blk * BLOCK_KEYS + 16 * m;
+                const bool there = key0 < ke && page_lds[min((key0 >> pshift) - first_page, PAGE_IDS - 1)] >= 0;
+                if (there && key0 + 8 * half + 8 <= ke) continue;
+                bf16x8 v = *reinterpret_cast<const bf16x8*>(vb + piece * 8);
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if (!there || key0 + 8 * half + e >= ke) v[e] = (__bf16)0.f;
+                *reinterpret_cast<bf16x8*>(vb + piece * 8) = v;
+            }
+        };
+        // (kept in registers: left to itself the compiler adds them up again for every tile)
+        uint32_t k_row[ND], v_row;
+#pragma unroll
+        for (int st = 0; st < ND; ++st) {
+            k_row[st] = (uint32_t)(((TILE_KEYS * kp + n) * D + 8 * ((2 * st + h) ^ (n & 15))) * 2);
+            asm volatile("" : "+v"(k_row[st]));
+        }
+        v_row = (uint32_t)((S::KBUF + TILE_KEYS * kp * D + n * 16 + 8 * (h ^ ((n >> 2 ^ n >> 3) & 1))) * 2);
+        asm volatile("" : "+v"(v_row));
+        typedef __attribute__((address_space(3))) unsigned char lds_byte;
+        lds_byte* const kv_lds = (lds_byte*)k_lds;
+        auto operand = [&](uint32_t at, int plus) { return *reinterpret_cast<__attribute__((address_space(3))) const bf16x8*>(kv_lds + at + plus); };
+        auto tile = [&](int tb, bool interior, auto buf_) {
+            constexpr int buf = decltype(buf_)::value;
+            // all operands of a product are asked for before its first instruction, and the values before the softmax; the
+            // products of two tiles are chains of their own, side by side
+            bf16x8 kf[T][ND], vf[T][DB][2], pf[T][2];
+#pragma unroll
+            for (int st = 0; st < ND; ++st)
+#pragma unroll
+                for (int t = 0; t < T; ++t) kf[t][st] = operand(k_row[st], buf * BLOCK * 2 + t * TILE_KEYS * D * 2);
+            __builtin_amdgcn_sched_barrier(0);
+            floatx16 sc[T];
+#pragma unroll
+            for (int t = 0; t < T; ++t)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) sc[t][i] = 0.f;
+#pragma unroll
+            for (int st = 0; st < ND; ++st)
+#pragma unroll
+                for (int t = 0; t < T; ++t) sc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[t][st], qf[st], sc[t], 0, 0, 0);
+            auto values = [&](int t) {
+#pragma unroll
+                for (int m = 0; m < 2; ++m)
+#pragma unroll
+                    for (int db = 0; db < DB; ++db) vf[t][db][m] = operand(v_row, buf * BLOCK * 2 + ((2 * t + m) * 16 * D + 32 * 16 * db) * 2);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            values(0);
+            __builtin_amdgcn_s_setprio(1);
+            softmax(sc, tb, interior, pf);
+            __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                if (t + 1 < T) values(t + 1);             // (not before: both tiles' values beside the scores are too many registers)
+#pragma unroll
+                for (int m = 0; m < 2; ++m)
+#pragma unroll
+                    for (int db = 0; db < DB; ++db) o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[t][db][m], pf[t][m], o[db], 0, 0, 0);
+            }
+        };
+        const bool whole_range = all_mapped && a.window <= 0;
+        ask(blk_begin, page_of(blk_begin), 0);
+        int page = page_of(blk_begin + 1);
+        // The blocks that this wavefront sees whole, in pairs, as long as three more follow (the page of the block after next is
+        // looked up, and all keys of every block but the last are there): nothing to check.
+        int blk = blk_begin;
+        if (whole_range && wave_active) {
+            const int fast_end = min(blk_end - 3, wave_first_kend / BLOCK_KEYS);
+            int key2 = (blk_begin + 2) * BLOCK_KEYS + 16 * wave;                // this wavefront's run of the block after next
+            auto fast = [&](auto buf_) {
+                tile_arrive();
+                ask(blk + 1, page, decltype(buf_)::value ^ 1);
+                const int after = page_lds[(key2 >> pshift) - first_page];
+                tile(0, true, buf_);
+                page = __builtin_amdgcn_readfirstlane(after);
+                key2 += BLOCK_KEYS;
+                ++blk;
+            };
+            while (blk + 2 <= fast_end) {
+                fast(std::integral_constant<int, 0>{});
+                fast(std::integral_constant<int, 1>{});
+            }
+        }
+        auto turn = [&](auto buf_) {
+            constexpr int buf = decltype(buf_)::value;
+            tile_arrive();                                // the block is there, and everyone is done with the one before
+            if (blk + 1 < blk_end) ask(blk + 1, page, buf ^ 1);
+            page = page_of(blk + 2);
+            const int tb0 = blk * BLOCK_KEYS, tb = tb0 + TILE_KEYS * kp;
+            if (!whole_range || tb0 + BLOCK_KEYS > ke) {
+                clear_values(blk, buf);
+                __syncthreads();
+            }
+            ++blk;
+            if (wave_active && tb < wave_hi && tb + T * TILE_KEYS > wave_lo)    // (else: nothing for this wavefront)
+                tile(tb, tb + T * TILE_KEYS <= wave_first_kend && tb >= wave_last_kbegin, buf_);
+        };
+        while (blk < blk_end) {
+            turn(std::integral_constant<int, 0>{});
+            if (blk < blk_end) turn(std::integral_constant<int, 1>{});
+        }
+    } else {
+        // What a thread stages per block and pass: 32 bytes of the keys (16 channels of one key) and 32 bytes of
+        // the values (16 keys of one channel; a page's values of one kv head are contiguous in the order
+        // (channel, key)), so one page id and one address serve two 16-byte loads each.
+        constexpr int KSTEP = S::KSTEP, VSTEP = S::VSTEP, KN = S::K_PASSES, VN = S::V_PASSES;
+        const int k_key0 = threadIdx.x / ND, k_c16 = threadIdx.x % ND;
+        const bool k_thread = (int)threadIdx.x < KSTEP * ND;
+        const int v_m0 = threadIdx.x / D, v_d = threadIdx.x % D;
+        const bool v_thread = (int)threadIdx.x < VSTEP * D;
+        const bool big_page = P > BLOCK_KEYS;                   // a block lies within one page
+        const uint32_t page_stride = (uint32_t)a.kv_heads * P * D;      // elements; the host keeps offsets within 32 bits
+        int k_key[KN], k_pageadd[KN], v_m16[VN], v_pageadd[VN];
+        uint32_t k_off0[KN], v_off0[VN];
+#pragma unroll
+        for (int i = 0; i < KN; ++i) {
+            k_key[i] = min(k_key0 + KSTEP * i, BLOCK_KEYS - 1);
+            k_pageadd[i] = big_page ? 0 : k_key[i] >> pshift;
+            k_off0[i] = (uint32_t)kvh * P * D + (big_page ? k_key[i] : (k_key[i] & (P - 1))) * D + 16 * k_c16;
+        }
+#pragma unroll
+        for (int i = 0; i < VN; ++i) {
+            v_m16[i] = min(v_m0 + VSTEP * i, BLOCK_KEYS / 16 - 1);
+            v_pageadd[i] = big_page ? 0 : (16 * v_m16[i]) >> pshift;
+            v_off0[i] = (uint32_t)kvh * P * D + v_d * P + (big_page ? 16 * v_m16[i] : ((16 * v_m16[i]) & (P - 1)));
+        }
+        struct Staged {
+            bf16x8 k[KN][2], v[VN][2];
+            int tb;
+            unsigned v_ok;               // bit i: pass i's page is mapped and its first key written
+            bool whole;                  // every key of the block is written and mapped: nothing to check or zero
+        };
+        // global -> registers.  No branch around a load (a load behind a branch makes the compiler wait for
+        // every load in flight): addresses are clamped to valid memory, and what must read as zero is zeroed
+        // when the registers go to LDS.  Only the pages of written keys were looked up: anything later counts
+        // as not mapped.
+        auto fetch = [&](int blk, Staged& st) {
+            const int tb = blk * BLOCK_KEYS;
+            st.tb = tb;
+            const int pidx = (tb >> pshift) - first_page;
+            const uint32_t inpage = big_page ? (tb & (P - 1)) : 0;
+            // (all blocks but a group's last, unless a window has given pages back: the same for every thread)
+            st.whole = all_mapped && a.window <= 0 && tb + BLOCK_KEYS <= ke;
+            if (st.whole) {
+#pragma unroll
+                for (int i = 0; i < KN; ++i) {
+                    const int pg = page_lds[pidx + k_pageadd[i]];
+                    const __bf16* kptr = a.k_pages + (__umul24(pg, page_stride) + inpage * D + k_off0[i]);
+                    st.k[i][0] = *reinterpret_cast<const bf16x8*>(kptr);
+                    st.k[i][1] = *reinterpret_cast<const bf16x8*>(kptr + 8);
+                }
+#pragma unroll
+                for (int i = 0; i < VN; ++i) {
+                    const int pg = page_lds[pidx + v_pageadd[i]];
+                    const __bf16* vptr = a.v_pages + (__umul24(pg, page_stride) + inpage + v_off0[i]);
+                    st.v[i][0] = *reinterpret_cast<const bf16x8*>(vptr);
+                    st.v[i][1] = *reinterpret_cast<const bf16x8*>(vptr + 8);
+                }
+                st.v_ok = ~0u;
+                return;
+            }
+            unsigned ok = 0;
+#pragma unroll
+            for (int i = 0; i < KN; ++i) {
+                const int raw = page_lds[min(pidx + k_pageadd[i], PAGE_IDS - 1)];
+                const int pg = tb + k_key[i] < ke ? raw : 0;
+                const __bf16* kptr = a.k_pages + (__umul24(max(pg, 0), page_stride) + inpage * D + k_off0[i]);
+                st.k[i][0] = *reinterpret_cast<const bf16x8*>(kptr);
+                st.k[i][1] = *reinterpret_cast<const bf16x8*>(kptr + 8);
+            }
+#pragma unroll
+            for (int i = 0; i < VN; ++i) {
+                const int raw = page_lds[min(pidx + v_pageadd[i], PAGE_IDS - 1)];
+                const int pg = tb + 16 * v_m16[i] < ke ? raw : -1;
+                ok |= (pg >= 0 ? 1u : 0u) << i;
+                const __bf16* vptr = a.v_pages + (__umul24(max(pg, 0), page_stride) + inpage + v_off0[i]);
+                st.v[i][0] = *reinterpret_cast<const bf16x8*>(vptr);
+                st.v[i][1] = *reinterpret_cast<const bf16x8*>(vptr + 8);
+            }
+            st.v_ok = ok;
+        };
+        auto stash = [&](int buf, const Staged& st) {      // registers -> LDS
+            if (k_thread) {
+                __bf16* kb = k_lds + buf * S::KBUF + k_key0 * KPITCH + 16 * k_c16;
+#pragma unroll
+                for (int i = 0; i < KN; ++i) {
+                    if (KN * KSTEP > BLOCK_KEYS && k_key0 + KSTEP * i >= BLOCK_KEYS) continue;
+                    *reinterpret_cast<bf16x8*>(kb + KSTEP * i * KPITCH) = st.k[i][0];
+                    *reinterpret_cast<bf16x8*>(kb + KSTEP * i * KPITCH + 8) = st.k[i][1];
+                }
+            }
+            if (v_thread) {
+                __bf16* vb = v_lds + buf * S::VBUF + v_d * VPITCH + 16 * v_m0;
+#pragma unroll
+                for (int i = 0; i < VN; ++i) {
+                    if (VN * VSTEP > BLOCK_KEYS / 16 && v_m0 + VSTEP * i >= BLOCK_KEYS / 16) continue;
+                    bf16x8 v0 = st.v[i][0], v1 = st.v[i][1];
+                    const int key0 = st.tb + 16 * (v_m0 + VSTEP * i);
+                    const bool ok = (st.v_ok >> i) & 1;
+                    if (!st.whole && !(ok && key0 + 16 <= ke)) {
+                        // values of keys that are not written yet, or of a page that was given back (behind a
+                        // window), count as zero: their probability is zero, but zero times whatever the
+                        // memory holds need not be
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) {
+                            if (!ok || key0 + e >= ke) v0[e] = (__bf16)0.f;
+                            if (!ok || key0 + 8 + e >= ke) v1[e] = (__bf16)0.f;
+                        }
+                    }
+                    // keys 8 a + 4 h + r of the 16 go to position 8 h + 4 a + r
+                    *reinterpret_cast<bf16x8*>(vb + 16 * VSTEP * i) =
+                        bf16x8{v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
+                    *reinterpret_cast<bf16x8*>(vb + 16 * VSTEP * i + 8) =
+                        bf16x8{v0[4], v0[5], v0[6], v0[7], v1[4], v1[5], v1[6], v1[7]};
+                }
+            }
+        };
+
+        // Two blocks are under way at any time: one being multiplied out of LDS, the next in flight from memory
+        // into registers.  One barrier per block suffices with two LDS buffers: a wavefront can only reach the
+        // second write of a buffer after the barrier that follows every wavefront's read of it.  Fetches are
+        // unconditional, clamped to the last block.
+        {
+            Staged st;
+            const int last = blk_end - 1;
+            fetch(blk_begin, st);
+            int buf = 0;
+            for (int blk = blk_begin; blk < blk_end; ++blk) {
+                stash(buf, st);
+                fetch(min(blk + 1, last), st);
+                __syncthreads();
+                compute(blk, buf);
+                buf ^= 1;
+            }
         }
     }
 
     // merge of the two key parities: parity 1 hands over its state, parity 0 finishes the columns
     l_run += __shfl_xor(l_run, 32, 64);
-    __syncthreads();                                     // the staged blocks are not read any more
+    if (S::PARITIES > 1) __syncthreads();                // the staged blocks are not read any more
     float* mine = merge_lds + (size_t)cq * S::NO * 64 + lane;
     if (kp == 1) {
 #pragma unroll
@@ -397,9 +581,10 @@ __device__ __forceinline__ void tile_group(const TileArgs& a, int grp, int kvh, 
         mine[(DB * 16) * 64] = m_ref;
         mine[(DB * 16 + 1) * 64] = l_run;
     }
-    __syncthreads();
+    if (S::PARITIES > 1) __syncthreads();
+    auto theirs = [&](int i) { return S::PARITIES > 1 ? mine[i * 64] : 0.f; };
     if (kp == 0 && col_valid) {
-        const float m1 = mine[(DB * 16) * 64], l1 = mine[(DB * 16 + 1) * 64];
+        const float m1 = S::PARITIES > 1 ? theirs(DB * 16) : -INFINITY, l1 = theirs(DB * 16 + 1);
         const float m = fmaxf(m_ref, m1);
         const float w0 = m_ref > -INFINITY ? __builtin_amdgcn_exp2f(m_ref - m) : 0.f;
         const float w1 = m1 > -INFINITY ? __builtin_amdgcn_exp2f(m1 - m) : 0.f;
@@ -417,10 +602,10 @@ __device__ __forceinline__ void tile_group(const TileArgs& a, int grp, int kvh, 
                     const int d0 = 32 * db + 8 * j + 4 * h;
                     if (d0 >= D) continue;
                     float4 v;                           // (D + 4 floats a split: 16-byte stores)
-                    v.x = o[db][4 * j] * w0 + mine[(db * 16 + 4 * j) * 64] * w1;
-                    v.y = o[db][4 * j + 1] * w0 + mine[(db * 16 + 4 * j + 1) * 64] * w1;
-                    v.z = o[db][4 * j + 2] * w0 + mine[(db * 16 + 4 * j + 2) * 64] * w1;
-                    v.w = o[db][4 * j + 3] * w0 + mine[(db * 16 + 4 * j + 3) * 64] * w1;
+                    v.x = o[db][4 * j] * w0 + theirs(db * 16 + 4 * j) * w1;
+                    v.y = o[db][4 * j + 1] * w0 + theirs(db * 16 + 4 * j + 1) * w1;
+                    v.z = o[db][4 * j + 2] * w0 + theirs(db * 16 + 4 * j + 2) * w1;
+                    v.w = o[db][4 * j + 3] * w0 + theirs(db * 16 + 4 * j + 3) * w1;
                     *reinterpret_cast<float4*>(dst + d0) = v;
                 }
             if (h == 0) {
@@ -440,7 +625,7 @@ __device__ __forceinline__ void tile_group(const TileArgs& a, int grp, int kvh, 
                 bf16x4 w4;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float other = mine[(db * 16 + 4 * j + r) * 64];
+                    const float other = theirs(db * 16 + 4 * j + r);
                     w4[r] = (__bf16)((o[db][4 * j + r] * w0 + other * w1) * inv);
                 }
                 *reinterpret_cast<bf16x4*>(dst + d0) = w4;
@@ -482,11 +667,10 @@ __global__ __launch_bounds__(256) void tiles_combine_kernel(TileArgs a) {
     if (lane + 64 < D) dst[lane + 64] = (__bf16)(n1 * inv);
 }
 
-// Workgroups of 128 columns take two groups, one after the other: group i and group (groups - 1 - i).
-// Within a long prompt the groups' key ranges grow with their position, so every workgroup gets about the
+// Workgroups of eight wavefronts (128 columns, other head sizes than 128) take two groups, one after the other: group i and group
+// (groups - 1 - i).  Within a long prompt the groups' key ranges grow with their position, so every workgroup gets about the
 // same work -- unless the pairs would be fewer than the compute units: then every group gets a workgroup of
-// its own (a 2 048-token portion of the 0.6B sizes behind 30 000 tokens of context: 20.4 ms for 23.7 with
-// workgroups of 64 columns, which load and stage every key twice as often a column).  Workgroups of 64 columns take one group each, the later (longer) groups first, and two of
+// its own.  Workgroups of four wavefronts take one group each, the later (longer) groups first, and two of
 // them share a compute unit.  When all of them fit the GPU at once, the order is: the later half of the
 // groups, longest first, then the earlier half, shortest first, so that the longest group shares its compute
 // unit with the shortest (measured at 2 048 tokens: 42.4 us for 44.1; with more workgroups than places the
@@ -494,26 +678,30 @@ __global__ __launch_bounds__(256) void tiles_combine_kernel(TileArgs a) {
 // index is remapped so that the workgroups of one kv head, which read the same keys and values, share an
 // XCD and its L2.
 template <int ND, int NQ>
-__global__ __launch_bounds__(128 * NQ, NQ == 2 ? 2 : 1) void attention_tiles_kernel(TileArgs a) {
+__global__ __launch_bounds__((TileShape<ND, NQ>::THREADS), (NQ == 2 || ND == 8 ? 2 : 1)) void attention_tiles_kernel(TileArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
     const int per_head = gridDim.x, total = gridDim.x * gridDim.y;
     int lin = blockIdx.x + per_head * blockIdx.y;
     if (total % 8 == 0) lin = (lin % 8) * (total / 8) + lin / 8;
     const int first = lin % per_head, kvh = lin / per_head;
     const int second = a.groups - 1 - first;
+    int todo[2] = {first, -1};
     if (a.single) {                                     // one group a workgroup, the later ones first
         // (with splits: split by split, so that the workgroups under way at a time walk the same keys.
         // Measured at 2048 tokens in two splits: 53 us; a group's splits side by side: 60; no split: 44)
         const int half = (a.groups + 1) / 2;
-        const int grp = a.max_splits > 1 || !a.all_resident ? second : (first < half ? second : first - half);
-        tile_group<ND, NQ>(a, grp, kvh, blockIdx.z, lds_raw);
-        return;
+        todo[0] = a.max_splits > 1 || !a.all_resident ? second : (first < half ? second : first - half);
+    } else if (second > first) {
+        todo[0] = second;
+        todo[1] = first;
     }
-    if (second > first) {
-        tile_group<ND, NQ>(a, second, kvh, 0, lds_raw);
-        __syncthreads();
+#pragma unroll 1
+    for (int i = 0; i < 2; ++i) {                       // (one copy of the code for both)
+        const int grp = i == 0 ? todo[0] : todo[1];
+        if (grp < 0) return;
+        if (i > 0) __syncthreads();
+        tile_group<ND, NQ>(a, grp, kvh, a.single ? blockIdx.z : 0, lds_raw);
     }
-    tile_group<ND, NQ>(a, first, kvh, 0, lds_raw);
 }
 
 template <int ND, int NQ>
@@ -535,12 +723,13 @@ static int launch_tiles(const TileArgs& a, hipStream_t stream) {
     }
     // (pairs that would leave compute units idle are no gain: then every group gets a workgroup of its own)
     const bool few_pairs = (long)((a.groups + 1) / 2) * a.kv_heads < compute_units;
-    const bool single = NQ == 2 || a.max_splits > 1 || a.single == 1 || (a.single == 0 && few_pairs);
+    const bool two = TileShape<ND, NQ>::THREADS == 256;         // two workgroups a compute unit
+    const bool single = NQ == 2 || a.max_splits > 1 || a.single == 1 || (a.single == 0 && (two || few_pairs));
     dim3 grid(single ? a.groups : (a.groups + 1) / 2, a.kv_heads, a.max_splits);
     TileArgs b = a;
     b.single = single ? 1 : 0;
-    b.all_resident = NQ == 2 && compute_units > 0 && (long)a.groups * a.kv_heads * a.max_splits <= 2L * compute_units;
-    attention_tiles_kernel<ND, NQ><<<grid, 128 * NQ, lds, stream>>>(b);
+    b.all_resident = two && compute_units > 0 && (long)a.groups * a.kv_heads * a.max_splits <= 2L * compute_units;
+    attention_tiles_kernel<ND, NQ><<<grid, TileShape<ND, NQ>::THREADS, lds, stream>>>(b);
     int err = (int)hipGetLastError();
     if (err != 0 || a.max_splits <= 1) return err;
     tiles_combine_kernel<<<dim3(a.groups, a.q_heads, ((32 * NQ) / (a.q_heads / a.kv_heads) + 3) / 4), 256, 0, stream>>>(a);
@@ -565,8 +754,8 @@ static int launch_tiles_dim(const TileArgs& a, hipStream_t stream) {
 // request, at most columns / (q_heads / kv_heads); columns = 128 or 64).  A group's keys must span at most
 // PAGE_IDS pages (per key split, with splits).  The cache of num_pages pages must hold fewer than 2^32 elements.
 // With max_splits > 1, `partial` holds M * q_heads * max_splits * (head_dim + 4) floats, 16-byte aligned, M the batch's rows.
-// `pairing` (workgroups of 128 columns without splits): 0 two groups a workgroup unless that would leave compute
-// units idle, 1 always one group a workgroup, 2 always two.  Returns 0, a HIP error
+// `pairing` (workgroups of 128 columns without splits): 0 two groups a workgroup where it has eight wavefronts, unless that would
+// leave compute units idle, 1 always one group a workgroup, 2 always two.  Returns 0, a HIP error
 // code, or a negative number for sizes this kernel does not take.
 extern "C" int mlr_attention_tiles(
     const void* q, const void* k_pages, const void* v_pages, const int32_t* block_table, int max_blocks,

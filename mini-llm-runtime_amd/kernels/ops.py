@@ -813,8 +813,8 @@ class Kernels:
         workgroups); keys and values of a group are staged once through LDS in blocks of 64.  With
         max_splits > 1 a group's keys are split over workgroups in ranges of split_keys (a multiple of 64)
         and merged through `partial`.  `pairing`: whether a workgroup of 128 columns (without splits) takes two
-        groups, an early and a late one of a prompt, which evens out their key ranges: "auto" unless that would
-        leave compute units idle, "single" never, "pairs" always.  The caller vouches for the groups (consecutive rows of one request,
+        groups, an early and a late one of a prompt, which evens out their key ranges: "auto" where it has a compute unit to
+        itself (not with head size 128) unless that would leave units idle, "single" never, "pairs" always.  The caller vouches for the groups (consecutive rows of one request,
         no more tokens than `tiles_group_tokens`)."""
         _need(columns in TILES_COLUMNS, lambda: f"attention_tiles: columns must be one of {TILES_COLUMNS}")
         _need(pairing in TILES_PAIRING, lambda: f"attention_tiles: pairing must be one of {sorted(TILES_PAIRING)}")

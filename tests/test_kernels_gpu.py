@@ -635,6 +635,57 @@ def test_paged_attention(dtype, case):
         assert torch.isnan(out4[lengths[0]:].float()).all()
 
 
+@pytest.mark.parametrize("hq,hkv,page,before,n,window,split", [
+    (2, 1, 16, 0, 1, None, 0), (16, 8, 16, 0, 300, None, 0), (16, 8, 16, 63, 65, None, 0), (8, 1, 16, 255, 130, None, 0),
+    (4, 4, 32, 320, 193, None, 0), (4, 2, 64, 511, 129, None, 0), (4, 2, 256, 700, 200, None, 0), (16, 1, 128, 449, 33, None, 0),
+    (4, 2, 16, 500, 150, 200, 0), (4, 2, 64, 600, 97, 70, 0), (4, 2, 16, 900, 70, None, 256), (2, 1, 32, 1000, 64, 500, 128)])
+def test_prompt_portions_of_head_size_128(hq, hkv, page, before, n, window, split):
+    """The prompt portions' kernel whose blocks go to LDS past the registers, at portions that start and end beside the edges
+    of blocks and pages, with pages smaller and larger than a block, behind a window whose pages were given back, in key
+    ranges; keys not written yet hold NaN, and so does every page that is not the request's.  The same bits every time."""
+    k = kernels(torch.bfloat16)
+    d, ctx, scale = 128, before + n, 128 ** -0.5
+    blocks = (ctx + page - 1) // page
+    keys, values = rnd((ctx, hkv, d), torch.bfloat16, 90), rnd((ctx, hkv, d), torch.bfloat16, 91)
+    q = rnd((n, hq * d), torch.bfloat16, 92, 2.0)
+    ids = torch.randperm(blocks + 2, generator=torch.Generator().manual_seed(93))[:blocks].cuda()
+    k_pages = torch.full((blocks + 2, hkv, page, d), float("nan"), dtype=torch.bfloat16, device="cuda")
+    v_pages = torch.full((blocks + 2, hkv, d, page), float("nan"), dtype=torch.bfloat16, device="cuda")
+    at = torch.arange(ctx, device="cuda")
+    k_pages[ids[at // page], :, at % page] = keys
+    v_pages[ids[at // page], :, :, at % page] = values
+    table = torch.full((1, blocks + 1), -1, dtype=torch.int32, device="cuda")
+    table[0, :blocks] = ids.int()
+    if window is not None:
+        gone = max(0, before + 1 - window) // page
+        k_pages[ids[:gone]], v_pages[ids[:gone]], table[0, :gone] = float("nan"), float("nan"), -1
+    slots, pos = torch.zeros(n, dtype=torch.int32, device="cuda"), torch.arange(before, ctx, dtype=torch.int32, device="cuda")
+    g = hq // hkv
+    seen = at[None] <= pos[:, None]
+    if window is not None:
+        seen &= at[None] > pos[:, None] - window
+    want, size = torch.empty((n, hq, d), dtype=torch.float64, device="cuda"), torch.empty((n, hq, d), dtype=torch.float64, device="cuda")
+    for head in range(hq):
+        w = torch.softmax((q.view(n, hq, d)[:, head].double() @ keys[:, head // g].double().T * scale).masked_fill(~seen, -math.inf), -1)
+        want[:, head], size[:, head] = w @ values[:, head // g].double(), w @ values[:, head // g].double().abs()
+    # a probability is rounded to bfloat16 (2^-9 of itself, in numerator and denominator) and its score is a 32-bit sum; so is the result
+    bound = (2.0 ** -8 + 1e-4) * size + 2.0 ** -8 * want.abs()
+    for columns in (128, 64):
+        for cap in {columns // g, max(1, columns // g - 3)}:
+            first = list(range(0, n, cap))
+            splits = -(-ctx // split) if split else 1
+            part = torch.full((k.attention_partial_numel(n, hq, d, splits),), float("nan"), device="cuda") if split else None
+            before_out = None
+            for _ in range(3):
+                out = torch.full((n, hq * d), float("nan"), dtype=torch.bfloat16, device="cuda")
+                k.attention_tiles(q, k_pages, v_pages, table, slots, pos, out, torch.tensor(first, dtype=torch.int32, device="cuda"),
+                                  torch.tensor([min(cap, n - r) for r in first], dtype=torch.int32, device="cuda"), len(first), hq, hkv, d, page,
+                                  scale, window=window, columns=columns, split_keys=split, max_splits=splits, partial=part)
+                assert bool(((out.double().view(n, hq, d) - want).abs() <= bound).all()), (columns, cap)
+                assert before_out is None or torch.equal(out, before_out), (columns, cap)
+                before_out = out
+
+
 @pytest.mark.parametrize("hq,hkv,d,page,window,split_keys", [(4, 2, 128, 16, None, 0), (4, 2, 128, 16, None, 64), (6, 2, 64, 32, 20, 0),
                                                              (16, 1, 48, 16, None, 0), (3, 1, 256, 16, 33, 64)])
 def test_paged_attention_float_rows_alone(hq, hkv, d, page, window, split_keys):
