@@ -166,7 +166,7 @@ __device__ __forceinline__ void tile_group(const TileArgs& a, int grp, int kvh, 
         }
     }
     float m_ref = -INFINITY, l_run = 0.f;
-    float m_use = -1e30f, raise_at = -INFINITY;      // m_ref as it is subtracted (a column with no key yet: exp2(-inf - finite) = 0, not NaN);
+    float m_neg = 1e30f, raise_at = -INFINITY;       // -m_ref as it is added (a column with no key yet: exp2(-inf + finite) = 0, not NaN);
                                                      // the score above which it is raised
     floatx16 o[DB];
 #pragma unroll
@@ -232,7 +232,7 @@ __device__ __forceinline__ void tile_group(const TileArgs& a, int grp, int kvh, 
 #pragma unroll
                     for (int i = 0; i < 16; ++i) o[db][i] *= corr;
                 m_ref = full;
-                m_use = fmaxf(full, -1e30f);
+                m_neg = -fmaxf(full, -1e30f);
                 raise_at = (full + RAISE_BY) / c2;
             }
         }
@@ -245,7 +245,7 @@ __device__ __forceinline__ void tile_group(const TileArgs& a, int grp, int kvh, 
 #pragma unroll
             for (int m = 0; m < 2; ++m) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) pf[t][m][e] = (__bf16)__builtin_amdgcn_exp2f(fmaf(sc[t][8 * m + e], c2, -m_use));
+                for (int e = 0; e < 8; ++e) pf[t][m][e] = (__bf16)__builtin_amdgcn_exp2f(fmaf(sc[t][8 * m + e], c2, m_neg));
 #pragma unroll
                 for (int e = 0; e < 8; e += 2)
                     psum = __builtin_amdgcn_fdot2_f32_bf16(bf16x2{pf[t][m][e], pf[t][m][e + 1]}, ones, psum, false);
@@ -342,17 +342,16 @@ __device__ __forceinline__ void tile_group(const TileArgs& a, int grp, int kvh, 
             }
         };
         // (kept in registers: left to itself the compiler adds them up again for every tile)
+        const uint32_t kv_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)k_lds;      // (a byte of LDS)
         uint32_t k_row[ND], v_row;
 #pragma unroll
         for (int st = 0; st < ND; ++st) {
-            k_row[st] = (uint32_t)(((TILE_KEYS * kp + n) * D + 8 * ((2 * st + h) ^ (n & 15))) * 2);
+            k_row[st] = kv_base + (uint32_t)(((TILE_KEYS * kp + n) * D + 8 * ((2 * st + h) ^ (n & 15))) * 2);
             asm volatile("" : "+v"(k_row[st]));
         }
-        v_row = (uint32_t)((S::KBUF + TILE_KEYS * kp * D + n * 16 + 8 * (h ^ ((n >> 2 ^ n >> 3) & 1))) * 2);
+        v_row = kv_base + (uint32_t)((S::KBUF + TILE_KEYS * kp * D + n * 16 + 8 * (h ^ ((n >> 2 ^ n >> 3) & 1))) * 2);
         asm volatile("" : "+v"(v_row));
-        typedef __attribute__((address_space(3))) unsigned char lds_byte;
-        lds_byte* const kv_lds = (lds_byte*)k_lds;
-        auto operand = [&](uint32_t at, int plus) { return *reinterpret_cast<__attribute__((address_space(3))) const bf16x8*>(kv_lds + at + plus); };
+        auto operand = [&](uint32_t at, int plus) { return *(__attribute__((address_space(3))) const bf16x8*)(uintptr_t)(at + (uint32_t)plus); };
         auto tile = [&](int tb, bool interior, auto buf_) {
             constexpr int buf = decltype(buf_)::value;
             // all operands of a product are asked for before its first instruction, and the values before the softmax; the
