@@ -34,73 +34,103 @@ __device__ __forceinline__ floatx4 load_k4(const float* __restrict__ row, int k,
 }
 
 // Few tiles of 16 x 16: a wavefront owns 16 rows and NT strips of 16 columns and walks all of k alone.  The chain of products is
-// the bound (32 clocks for every four k), so nothing else may stand in its way: the exchange between lane blocks is left to LDS
-// (16-byte stores of what a lane has loaded, 4-byte reads of what it needs, both free of bank conflicts; no other wavefront
-// takes part), blocks of U groups of 16 k are stored one block and loaded two blocks ahead, and a group is read one group ahead.
-template <int NT, int U>
+// the bound (measured alone 13.6 ns, 32.5 clocks, for every four k), so nothing else may stand in its way.  A wavefront cannot
+// wait for memory inside it, so it has up to STAGES - 1 stages of 64 k under way, 448 k or 1.5 us of products: loads that go to
+// LDS without passing registers (`buffer_load_dwordx4 .. lds`, a lane's 16 bytes at 16 bytes of its own), for which the registers
+// would not do -- with blocks of 128 k in registers, one under way, every block waited for memory and four k took 20 ns.  The
+// exchange between lane blocks is left to LDS (4-byte reads of what a lane needs, free of bank conflicts; no other wavefront
+// takes part); a group of 16 k is read one ahead, a share of it behind each product.
+// 8 rows of 4096 x 1024, 1024 x 2048, 6144 x 1024, 1024 x 3072, weights cold: 7.6, 11.5, 10.2 and 15.6 us (9.6, 14.2, 11.9,
+// 19.5 with blocks in registers).
+template <int LEFT> __device__ __forceinline__ void strip_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LEFT) : "memory"); }
+
+template <int NT, int STAGES>
 __global__ __launch_bounds__(64) void gemm_f32_strip_kernel(const float* __restrict__ a, const float* __restrict__ w,
                                                             float* __restrict__ out, int M, int N, int K) {
-    extern __shared__ __attribute__((aligned(16))) float lds[];               // [2][U][1 + NT][256]
-    constexpr int P = 1 + NT;
+    extern __shared__ __attribute__((aligned(16))) float lds[];               // [STAGES][G][1 + NT][256]
+    constexpr int P = 1 + NT, G = 4, LOADS = G * P, STAGE = LOADS * 256;
+    static_assert(STAGES >= 3 && STAGES <= 8 && P <= 4 && LOADS * (STAGES - 1) <= 63, "the counter of loads in flight has six bits");
     const int lane = threadIdx.x, r = lane & 15, b = lane >> 4, m0 = blockIdx.y * 16, n0 = blockIdx.x * (NT * 16);
-    const float* from[P];                                  // the lane's row of a and of every strip
-    from[0] = a + (size_t)min(m0 + r, M - 1) * K + b * 4;
+    uint32_t row[P];                                       // the lane's row of a and of every strip, in bytes from the first
+    row[0] = (uint32_t)(min(m0 + r, M - 1) - m0) * (uint32_t)K * 4u;
 #pragma unroll
-    for (int j = 0; j < NT; ++j) from[1 + j] = w + (size_t)min(n0 + j * 16 + r, N - 1) * K + b * 4;
-    floatx4 acc[NT], x[U][P];
+    for (int j = 0; j < NT; ++j) row[1 + j] = (uint32_t)(min(n0 + j * 16 + r, N - 1) - n0) * (uint32_t)K * 4u;
+    const auto ar = __builtin_amdgcn_make_buffer_rsrc((void*)(a + (size_t)m0 * K), 0, (int)((uint32_t)K * 64u), 0x00027000);
+    const auto wr = __builtin_amdgcn_make_buffer_rsrc((void*)(w + (size_t)n0 * K), 0, (int)((uint32_t)K * (64u * NT)), 0x00027000);
+    const int stages = (K + 16 * G - 1) / (16 * G), full = K / (16 * G);
+    constexpr std::true_type yes{};
+    constexpr std::false_type no{};
+    // (whole: every place lies before K; otherwise places behind it are the row's last ones again, and what is read there counts as zero)
+    auto load = [&](int t, int u, int j, int slot, bool whole) {
+        const int k0 = (t * G + u) * 16;
+        uint32_t at = row[j];
+        if (!whole) at += (uint32_t)min(k0 + b * 4, K - 4) * 4u;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(j == 0 ? ar : wr, (__attribute__((address_space(3))) void*)(lds + slot * STAGE + (u * P + j) * 256), 16,
+                                                 (int)at, whole ? k0 * 4 : 0, 0, 0);
+    };
+    auto wait_for = [&](int behind) {                      // all but the last `behind` stages that were asked for are there
+        if (behind >= STAGES - 2) strip_wait<LOADS * (STAGES - 2)>();
+        else if (behind == 1) strip_wait<LOADS>();
+        else if (behind == 2) strip_wait<2 * LOADS>();
+        else if (behind == 3) strip_wait<3 * LOADS>();
+        else if (behind == 4) strip_wait<4 * LOADS>();
+        else if (behind == 5) strip_wait<5 * LOADS>();
+        else strip_wait<0>();
+    };
+    floatx4 acc[NT], now[P], next[P];
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
-    const int blocks = (K + 16 * U - 1) / (16 * U);
-    auto fetch = [&](int t, int u, bool whole) {           // (never behind a condition of its own; K is a multiple of four)
-        const int at = whole ? t * U * 16 : min((t * U + u) * 16, K - 4 - b * 4) - u * 16;
-#pragma unroll
-        for (int j = 0; j < P; ++j) x[u][j] = *reinterpret_cast<const floatx4*>(from[j] + at + u * 16);
-    };
-    auto stash = [&](int t, int u, bool whole) {
+    const float* mine = lds + r * 4 + b;
+    auto read = [&](int t, int u, int i, int slot, floatx4 (&v)[P], bool whole) {      // element i: k = 4 i + b of the group
 #pragma unroll
         for (int j = 0; j < P; ++j) {
-            floatx4 v = x[u][j];
-            if (!whole && (t * U + u) * 16 + b * 4 >= K) v = floatx4{0.f, 0.f, 0.f, 0.f};
-            *reinterpret_cast<floatx4*>(lds + (((t & 1) * U + u) * P + j) * 256 + lane * 4) = v;
+            v[j][i] = mine[slot * STAGE + (u * P + j) * 256 + i * 64];
+            if (!whole && (t * G + u) * 16 + 4 * i + b >= K) v[j][i] = 0.f;
         }
     };
-    auto whole = [&](int t) { return (t + 1) * U * 16 <= K; };
+    for (int t = 0; t < STAGES - 1 && t < stages; ++t)
 #pragma unroll
-    for (int u = 0; u < U; ++u) fetch(0, u, false);
+        for (int c = 0; c < LOADS; ++c) load(t, c / P, c % P, t, false);
 #pragma unroll
-    for (int u = 0; u < U; ++u) stash(0, u, false);
+    for (int j = 0; j < P; ++j) row[j] += (uint32_t)b * 16u;                  // (from here on: whole loads, and those of the last stage)
+    wait_for(min(STAGES - 1, stages) - 1);
 #pragma unroll
-    for (int u = 0; u < U; ++u) fetch(min(1, blocks - 1), u, false);
-    auto turn = [&](int t, bool all) {                     // all: the two blocks behind t are whole
-        // (other lanes read what a lane has stored: a wavefront's LDS instructions run in their order, and the compiler keeps it)
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        const float* at = lds + (t & 1) * (U * P * 256) + r * 4 + b;
-        floatx4 now[P], next[P];
-        auto read = [&](int u, floatx4 (&v)[P]) {          // element i: k = 4 i + b of the group
+    for (int i = 0; i < 4; ++i) read(0, 0, i, 0, now, false);
+    int slot = 0;
+    // more: a further stage is asked for, into the place of the last one read; whole: it lies before K; clean: what is read does
+    auto turn = [&](int t, auto more, bool whole, bool clean) {
+        const int ahead = slot + 1 == STAGES ? 0 : slot + 1, behind = slot == 0 ? STAGES - 1 : slot - 1;
 #pragma unroll
-            for (int j = 0; j < P; ++j)
+        for (int u = 0; u < G; ++u) {
+            if (u == G - 1) {                              // the next stage is read from here on
+                if constexpr (decltype(more)::value) strip_wait<LOADS * (STAGES - 3) + (G - 1) * P>();
+                else wait_for(stages - 2 - t);
+            }
 #pragma unroll
-                for (int i = 0; i < 4; ++i) v[j][i] = at[(u * P + j) * 256 + i * 64];
-        };
-        read(0, now);
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (u + 1 < U) read(u + 1, next);
-            stash(t + 1, u, all);
-            fetch(all ? t + 2 : min(t + 2, blocks - 1), u, all);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < 4; ++i) {
 #pragma unroll
                 for (int j = 0; j < NT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now[0][i], now[1 + j][i], acc[j], 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);             // (left alone, the compiler moves a load to where its value is used)
+                __builtin_amdgcn_sched_barrier(0);         // (left alone, the compiler moves a load to where its value is used)
+                if (u + 1 < G) read(t, u + 1, i, slot, next, clean);
+                else read(t + 1, 0, i, ahead, next, clean);
+                if (decltype(more)::value && i < P) load(t + STAGES - 1, u, i, behind, whole);
+                __builtin_amdgcn_sched_barrier(0);
+            }
 #pragma unroll
             for (int j = 0; j < P; ++j) now[j] = next[j];
         }
+        slot = ahead;
     };
     int t = 0;
-    for (; t + 2 < blocks && whole(t + 2); ++t) turn(t, true);
-    for (; t < blocks; ++t) turn(t, false);                // (behind the last block zeros are stored that nothing reads)
+    for (; t + STAGES - 1 < full; ++t) turn(t, yes, true, true);
+    if (stages == full) {
+        for (; t < stages; ++t) turn(t, no, true, true);     // (behind the last stage nothing is made of what is read)
+    } else {
+#pragma unroll
+        for (int j = 0; j < P; ++j) row[j] -= (uint32_t)b * 16u;
+        if (t + STAGES - 1 < stages) turn(t, yes, false, true), ++t;
+        for (; t < stages; ++t) turn(t, no, false, false);
+    }
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
@@ -183,13 +213,13 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
         }
 }
 
-template <int NT, int U>
+template <int NT, int STAGES>
 static int launch_f32_strip(const float* a, const float* w, float* out, int M, int N, int K, hipStream_t stream) {
-    constexpr size_t lds = 2 * U * (1 + NT) * 256 * sizeof(float);
-    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_strip_kernel<NT, U>),
+    constexpr size_t lds = STAGES * 4 * (1 + NT) * 256 * sizeof(float);
+    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_strip_kernel<NT, STAGES>),
                                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (allowed != hipSuccess) return (int)allowed;
-    gemm_f32_strip_kernel<NT, U><<<dim3((N + NT * 16 - 1) / (NT * 16), (M + 15) / 16), 64, lds, stream>>>(a, w, out, M, N, K);
+    gemm_f32_strip_kernel<NT, STAGES><<<dim3((N + NT * 16 - 1) / (NT * 16), (M + 15) / 16), 64, lds, stream>>>(a, w, out, M, N, K);
     return (int)hipGetLastError();
 }
 
@@ -207,14 +237,14 @@ static int launch_f32_tile(const float* a, const float* w, float* out, int M, in
 
 template <bool VEC>
 static int launch_gemm_f32(const float* a, const float* w, float* out, int M, int N, int K, hipStream_t stream) {
-    // A wavefront a tile of 16 x 16 while those are few: 8 rows of 4096 x 1024, 1024 x 2048, 6144 x 1024 and 1024 x 3072 take 9.3,
-    // 14.0, 10.8 and 19.3 us (tiles of 32 14.3, 23.7, 15.8 and 34.3), 64 rows of 1024 x 3072 19.4 (40), 32 of 6144 x 1024 (768
-    // tiles) 16.0 (17.6).  Two strips a wavefront beyond that, while the rows are few or up to 1024 tiles: 64 rows of 4096 x 1024
-    // 14.9 (one strip 19.9, tiles of 32 16.7), 8 of 24576 x 4096 96 and of 151936 x 1024 158 (130 and 184; the weight alone
-    // takes 84 and 130); 64 rows of 6144 x 1024 (1536 tiles) 22.1 and in tiles of 32 21.3.
+    // A wavefront a tile of 16 x 16 while those are few: 8 rows of 4096 x 1024, 1024 x 2048, 6144 x 1024 and 1024 x 3072 take 7.6,
+    // 11.5, 10.2 and 15.6 us (tiles of 32 14.3, 23.7, 15.8 and 34.3), 64 rows of 1024 x 3072 16.1 (40); up to 512 tiles, two a
+    // compute unit, with eight stages of LDS, up to 768 with five (three a unit; 40 rows of 6144 x 1024, 1152 tiles, do not come
+    // here).  Two strips a wavefront beyond that, while the rows are few or up to 1024 tiles: 64 rows of 4096 x 1024 14.1 (tiles
+    // of 32 16.7), 8 of 151936 x 1024 144 (the weight alone takes 130); 64 rows of 6144 x 1024 (1536 tiles) in tiles of 32 21.3.
     const long long units = (long long)((M + 15) / 16) * ((N + 15) / 16);
     if (VEC && (M + 15) / 16 <= 65535) {
-        if (units <= 768) return launch_f32_strip<1, 8>(a, w, out, M, N, K, stream);
+        if (units <= 768) return units <= 512 ? launch_f32_strip<1, 8>(a, w, out, M, N, K, stream) : launch_f32_strip<1, 5>(a, w, out, M, N, K, stream);
         if (M <= 16 || units <= 1024) return launch_f32_strip<2, 4>(a, w, out, M, N, K, stream);
     }
     // The square tile whose workgroups, one a compute unit at a time, are done first: a tile of 64 takes 1 / 3.7 of the time
