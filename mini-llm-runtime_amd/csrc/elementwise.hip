@@ -97,24 +97,56 @@ __device__ void norm_row_rescaled(const float* hrow, const RowAddend more, const
 
 // For output row r: src = rows ? rows[r] : r;  x = h[src] + what is still to be added to it;
 // if write_h: h[src] = x;  out[r] = (x * rsqrt(mean(x^2) + eps)) * weight.
-// One workgroup per row; the sum of squares is taken over the row in a fixed order.
-__global__ void add_rmsnorm_kernel(float* __restrict__ h, const RowAddend addend,
-                                   const float* __restrict__ weight, elem_t* __restrict__ out,
-                                   const int32_t* __restrict__ rows, int width, float eps,
-                                   int write_h) {
+// One workgroup per row; the sum of squares is taken over the row in a fixed order: a thread adds the squares of its values
+// (every 256th) in ascending order, then `block_sum`.  REGS > 0: rows of at most 256 REGS values, a thread's share asked for
+// at once and kept in registers; a value at a time, each behind the store of the one before, every value was a trip to the
+// cache of its own, and the second pass another (8 rows of 1024 in a decoding step: 5.7 -> 4.5 us; the sums' order, so their bits, are the same).
+template <int REGS>
+__global__ __launch_bounds__(256) void add_rmsnorm_kernel(float* __restrict__ h, const RowAddend addend,
+                                                          const float* __restrict__ weight, elem_t* __restrict__ out,
+                                                          const int32_t* __restrict__ rows, int width, float eps,
+                                                          int write_h) {
     __shared__ float scratch[16];
     const int r = blockIdx.x;
     const size_t src = rows ? (size_t)rows[r] : (size_t)r;
     float* hrow = h + src * width;
     const RowAddend more = addend.of_row(src, width);
+    constexpr int KEPT = REGS > 0 ? REGS : 1;
+    float x[KEPT], w[KEPT];
     float sum = 0.f;
-    for (int i = threadIdx.x; i < width; i += blockDim.x) {
-        float x = hrow[i];
-        if (more.any()) {
-            x = more.to(x, i);
-            if (write_h) hrow[i] = x;
+    if (REGS > 0) {
+        float d[KEPT], v[KEPT];
+        auto all = [&](const float* from, float* to) {         // (no load behind a condition: places behind the row are its last one)
+#pragma unroll
+            for (int i = 0; i < KEPT; ++i) to[i] = from[min((int)threadIdx.x + 256 * i, width - 1)];
+        };
+        all(hrow, x);
+        all(weight, w);
+        if (more.delta) {
+#pragma unroll
+            for (int i = 0; i < KEPT; ++i) d[i] = to_float(more.delta[min((int)threadIdx.x + 256 * i, width - 1)]);
         }
-        sum += x * x;
+        if (more.vector) all(more.vector, v);
+#pragma unroll
+        for (int i = 0; i < KEPT; ++i) {
+            if (more.delta) x[i] = fmaf(more.factor, d[i], x[i]);
+            if (more.vector) x[i] += v[i];
+            if ((int)threadIdx.x + 256 * i < width) sum += x[i] * x[i];
+        }
+        if (write_h && more.any()) {
+#pragma unroll
+            for (int i = 0; i < KEPT; ++i)
+                if ((int)threadIdx.x + 256 * i < width) hrow[threadIdx.x + 256 * i] = x[i];
+        }
+    } else {
+        for (int i = threadIdx.x; i < width; i += blockDim.x) {
+            float y = hrow[i];
+            if (more.any()) {
+                y = more.to(y, i);
+                if (write_h) hrow[i] = y;
+            }
+            sum += y * y;
+        }
     }
     sum = block_sum(sum, scratch);
     elem_t* orow = out + (size_t)r * width;
@@ -123,10 +155,16 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ h, const RowAddend addend
         return;
     }
     const float scale = 1.0f / sqrtf(sum / (float)width + eps);
+    if (REGS > 0) {
+#pragma unroll
+        for (int i = 0; i < KEPT; ++i)
+            if ((int)threadIdx.x + 256 * i < width) orow[threadIdx.x + 256 * i] = from_float<elem_t>((x[i] * scale) * w[i]);
+        return;
+    }
     for (int i = threadIdx.x; i < width; i += blockDim.x) {
-        float x = hrow[i];
-        if (!write_h) x = more.to(x, i);
-        orow[i] = from_float<elem_t>((x * scale) * weight[i]);
+        float y = hrow[i];
+        if (!write_h) y = more.to(y, i);
+        orow[i] = from_float<elem_t>((y * scale) * weight[i]);
     }
 }
 
@@ -1190,8 +1228,9 @@ int mlr_add_rmsnorm(float* h, const void* delta, float factor, const float* vect
                                                               width, eps, write_h);
         return (int)hipGetLastError();
     }
-    add_rmsnorm_kernel<<<n_out, 256, 0, stream>>>(h, addend, weight, (elem_t*)out, rows,
-                                                  width, eps, write_h);
+    if (width <= 256 * 4) add_rmsnorm_kernel<4><<<n_out, 256, 0, stream>>>(h, addend, weight, (elem_t*)out, rows, width, eps, write_h);
+    else if (width <= 256 * 20) add_rmsnorm_kernel<20><<<n_out, 256, 0, stream>>>(h, addend, weight, (elem_t*)out, rows, width, eps, write_h);
+    else add_rmsnorm_kernel<0><<<n_out, 256, 0, stream>>>(h, addend, weight, (elem_t*)out, rows, width, eps, write_h);
     return (int)hipGetLastError();
 }
 

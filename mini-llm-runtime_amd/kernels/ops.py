@@ -429,12 +429,17 @@ class Kernels:
             return not self.library_gemm or k <= 1024 or (k <= 2048 and rows <= 256)
         return self.streams_weight(rows, k if k is not None else 1 << 30)
 
+    def gated_strips(self, rows, columns, k):
+        """Whether `gemm_gated_silu` is the float engine's way for `rows` times `columns` gates: tiles of 16 x 16 that are few."""
+        return self.dtype == torch.float32 and k % 4 == 0 and -(-rows // 16) * -(-columns // 16) <= 512
+
     @timed("gemm", _gemm_work)
     def gemm_gated_silu(self, a, w, out):
         """out[M, N] = silu(a . w[:N]^T) * (a . w[N:]^T), w = [gate; up] stacked: up to 64 rows, or any number
-        when the inner size is a multiple of 64 (the wide kernel's gated form)."""
-        _need(self.dtype == torch.bfloat16, "gemm_gated_silu: bfloat16 only")
-        _need(a.shape[0] <= 64 or (a.shape[1] % 64 == 0 and a.numel() < 2 ** 31 and w.numel() < 2 ** 31),
+        when the inner size is a multiple of 64 (the wide kernel's gated form); float32: the sizes of `gated_strips`."""
+        strips = self.dtype == torch.float32
+        _need(not strips or self.gated_strips(a.shape[0], w.shape[0] // 2, a.shape[1]), "gemm_gated_silu: too many rows and columns in float32")
+        _need(strips or a.shape[0] <= 64 or (a.shape[1] % 64 == 0 and a.numel() < 2 ** 31 and w.numel() < 2 ** 31),
               "gemm_gated_silu: more than 64 rows need an inner size that is a multiple of 64 (and matrices "
               "below 2^31 elements)")
         _tensor(a, "a", self.dtype, ndim=2)
@@ -443,7 +448,7 @@ class Kernels:
         two_n, k2 = w.shape
         _need(k == k2 and two_n % 2 == 0, "gemm_gated_silu: sizes do not fit")
         _tensor(out, "out", self.dtype, (m, two_n // 2))
-        if m > 64:
+        if m > 64 or strips:
             a, w = _start16(a), _start16(w)
         fn = self._lib("gemm").mlr_gemm_gated_silu
         _ok(fn(_p(a), _p(w), _p(out), _c_int(m), _c_int(two_n // 2), _c_int(k), _stream()), "gemm_gated_silu")

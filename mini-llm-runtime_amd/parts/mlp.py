@@ -61,7 +61,7 @@ class SwiGluMlp:
         s = self.spec
         m = x.shape[0]
         act = ctx.workspace.get("act", (m, s.intermediate), x.dtype)
-        if s.activation == "silu" and ctx.kernels.gated_silu_fused(m, s.hidden):
+        if s.activation == "silu" and (ctx.kernels.gated_silu_fused(m, s.hidden) or ctx.kernels.gated_strips(m, s.intermediate, s.hidden)):
             ctx.kernels.gemm_gated_silu(x, self.gate_up, act)      # few rows: the activation rides on the projection
         elif s.activation != "silu" and m <= 64 and ctx.kernels.streams_weight(m, s.hidden):
             ctx.kernels.gemm_gated_act(x, self.gate_up, act, s.activation)

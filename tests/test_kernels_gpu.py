@@ -260,6 +260,44 @@ def test_gemm_float_is_one_chain_over_k(m, n, kk):
         assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("m,n,kk", [(1, 5, 4), (8, 3072, 1024), (16, 33, 60), (17, 100, 68), (5, 8192, 260), (40, 1500, 448), (33, 2600, 516)])
+def test_gemm_gated_silu_float(m, n, kk):
+    """The float engine's gate beside its up: the bits of the stacked product and the activation's own launch, from fewer
+    values of k than a stage holds to more than all stages do, with both numbers of stages."""
+    k = kernels(torch.float32)
+    a, w = rnd((m, kk), torch.float32, 70), rnd((2 * n, kk), torch.float32, 71, 0.3)
+    both, want = torch.empty((m, 2 * n), device="cuda"), torch.empty((m, n), device="cuda")
+    k.gemm(a, w, both)
+    k.silu_mul(both, want)
+    shifted = torch.empty(m * kk + 1, device="cuda")[1:].view(m, kk).copy_(a)      # rows 4 bytes off
+    assert k.gated_strips(m, n, kk) and not k.gated_strips(1024, 4096, 64)
+    for rows in (a, shifted):
+        out = torch.full((m, n), float("nan"), device="cuda")
+        k.gemm_gated_silu(rows, w, out)
+        assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("rows,width", [(3, 5), (8, 1024), (2, 1023), (5, 1025), (4, 5120), (2, 5121), (1, 8200)])
+def test_add_rmsnorm_float_widths(rows, width):
+    """The float engine's norm at widths around those whose rows stay in registers, with the residual written back and without:
+    a thread adds the squares of every 256th value in ascending order."""
+    k = kernels(torch.float32)
+    h, delta, w = rnd((rows, width), torch.float32, 72), rnd((rows, width), torch.float32, 73), rnd((width,), torch.float32, 74)
+    want_h = torch.addcmul(h, delta, torch.ones_like(delta))
+    squares = torch.nn.functional.pad(want_h, (0, -width % 256)).view(rows, -1, 256).double()
+    total = torch.zeros((rows, 256), dtype=torch.float64, device="cuda")
+    for i in range(squares.shape[1]):
+        total = (total + squares[:, i] * squares[:, i]).float().double()      # (fmaf: one rounding of a sum that 64 bits hold nearly exactly)
+    mean = total.sum(1) / width
+    for write in (True, False):
+        x, out = h.clone(), torch.full((rows, width), float("nan"), device="cuda")
+        k.add_rmsnorm(x, delta, w, out, 1e-6, write_h=write)
+        assert torch.equal(x, want_h if write else h)
+        # 256 partial sums are added in 32 bits over nine levels; then a division, a square root, a division and two products
+        assert bool(((out.double() - want_h.double() * torch.rsqrt(mean + 1e-6)[:, None] * w.double()).abs()
+                     <= 16 * 2.0 ** -24 * out.double().abs() + 1e-30).all())
+
+
 @pytest.mark.parametrize("shape", [0, 1, 2, 3])
 @pytest.mark.parametrize("gated", [False, True])
 @pytest.mark.parametrize("mnk", [(65, 70, 64), (300, 257, 192), (513, 1000, 128), (128, 256, 1024), (1, 5, 320)])
