@@ -469,6 +469,61 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 #define VT_PITCH 40             // elements between the channels of the transposed values (80 bytes)
 #define TILES_MAX_BLOCKS 2048   // page ids of a workgroup's key range that it keeps in LDS
 
+// A lane's column: the softmax over its keys in base 2, tile by tile; the four lanes of a column agree.
+struct SinkColumn {
+    float run_max = -INFINITY, run_sum = 0.f, scale2, cap2, cap_slope;
+    bool capped, ok;
+    int lo, pos;
+    __device__ __forceinline__ SinkColumn(const SinkArgs& a, bool col_ok, int qlo, int qpos)
+        : scale2(a.scale * 1.4426950408889634f), cap2(a.softcap * 1.4426950408889634f), capped(a.softcap > 0.f), ok(col_ok), lo(qlo), pos(qpos) {
+        cap_slope = capped ? 2.0f * scale2 / a.softcap : 0.f;
+    }
+    // The scores of the eight keys from key0 on -> probabilities pf; returns the factor on the sums so far.
+    __device__ __forceinline__ float tile(const floatx4& s0, const floatx4& s1, int key0, bool whole, int keep_first, bf16x8& pf) {
+        float sc[8];
+        float tile_max = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int kp = key0 + e;
+            const float raw = e < 4 ? s0[e] : s1[e - 4];
+            const bool seen = ok && (whole || ((kp >= lo || kp < keep_first) && kp <= pos));
+            // (capped: c tanh(s / c) = c - 2 c / (1 + e^(2 s / c)), here in base 2; an exponent beyond 32 bits gives c)
+            const float s2 = capped ? cap2 - 2.0f * cap2 * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(raw * cap_slope))
+                                    : raw * scale2;
+            sc[e] = seen ? s2 : -INFINITY;
+            tile_max = fmaxf(tile_max, sc[e]);
+        }
+        tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16, MLR_WAVE));
+        tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, MLR_WAVE));
+        const float new_max = fmaxf(run_max, tile_max);
+        // (the raw exponential instruction: its arguments are at most 0, and what underflows may be 0)
+        const float corr = new_max > -INFINITY ? __builtin_amdgcn_exp2f(run_max - new_max) : 1.f;
+        float part = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float p = new_max > -INFINITY ? __builtin_amdgcn_exp2f(sc[e] - new_max) : 0.f;
+            part += p;
+            pf[e] = (__bf16)p;
+        }
+        part += __shfl_xor(part, 16, MLR_WAVE);
+        part += __shfl_xor(part, 32, MLR_WAVE);
+        run_sum = run_sum * corr + part;
+        run_max = new_max;
+        return corr;
+    }
+    // The factor that turns the column's sums into its result: the sink, and the division.
+    __device__ __forceinline__ float end(const float* sink, int head) const {
+        float top = run_max, den = run_sum, f = 1.f;
+        if (sink != nullptr) {
+            const float sk = sink[head] * 1.4426950408889634f;
+            top = fmaxf(run_max, sk);
+            f = run_max > -INFINITY ? exp2f(run_max - top) : 0.f;
+            den = run_sum * f + exp2f(sk - top);
+        }
+        return den > 0.f ? f / den : 0.f;
+    }
+};
+
 template <int NKF, int NVT, bool SPLITV>
 __global__ __launch_bounds__(256) void sink_attention_tiles_kernel(SinkArgs a, const int32_t* __restrict__ group_first,
                                                                    const int32_t* __restrict__ group_count,
@@ -520,10 +575,7 @@ __global__ __launch_bounds__(256) void sink_attention_tiles_kernel(SinkArgs a, c
     floatx4 acc[NACC];
 #pragma unroll
     for (int j = 0; j < NACC; ++j) acc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
-    float run_max = -INFINITY, run_sum = 0.f;
-    const float scale2 = a.scale * 1.4426950408889634f;
-    const bool capped = a.softcap > 0.f;
-    const float cap2 = a.softcap * 1.4426950408889634f, cap_slope = capped ? 2.0f * scale2 / a.softcap : 0.f;
+    SinkColumn column(a, col_ok, qlo, qpos);
 
     // the page ids of the workgroup's keys, once: those of its kept tiles, behind them those of its others
     const int lead_end = min(i_end, kept) * TK;                                   // its kept keys end here
@@ -618,38 +670,10 @@ __global__ __launch_bounds__(256) void sink_attention_tiles_kernel(SinkArgs a, c
             s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, qf[kf], s0, 0, 0, 0);
             s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, qf[kf], s1, 0, 0, 0);
         }
-        float sc[8];
-        float tile_max = -INFINITY;
         // a tile that every token of the group sees whole needs no comparisons (the same in every thread)
         const bool whole = (t0 >= last_lo || t0 + TK <= a.keep_first) && t0 + TK - 1 <= p0;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int kp = t0 + 8 * b + e;
-            const float raw = e < 4 ? s0[e] : s1[e - 4];
-            const bool seen = col_ok && (whole || ((kp >= qlo || kp < a.keep_first) && kp <= qpos));
-            // (capped: c tanh(s / c) = c - 2 c / (1 + e^(2 s / c)), here in base 2; an exponent beyond 32 bits gives c)
-            const float s2 = capped ? cap2 - 2.0f * cap2 * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(raw * cap_slope))
-                                    : raw * scale2;
-            sc[e] = seen ? s2 : -INFINITY;
-            tile_max = fmaxf(tile_max, sc[e]);
-        }
-        tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16, MLR_WAVE));
-        tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, MLR_WAVE));
-        const float new_max = fmaxf(run_max, tile_max);
-        // (the raw exponential instruction: its arguments are at most 0, and what underflows may be 0)
-        const float corr = new_max > -INFINITY ? __builtin_amdgcn_exp2f(run_max - new_max) : 1.f;
-        float part = 0.f;
         bf16x8 pf;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const float p = new_max > -INFINITY ? __builtin_amdgcn_exp2f(sc[e] - new_max) : 0.f;
-            part += p;
-            pf[e] = (__bf16)p;
-        }
-        part += __shfl_xor(part, 16, MLR_WAVE);
-        part += __shfl_xor(part, 32, MLR_WAVE);
-        run_sum = run_sum * corr + part;
-        run_max = new_max;
+        const float corr = column.tile(s0, s1, t0 + 8 * b, whole, a.keep_first, pf);
         // the sums so far are only scaled where some column's maximum rose (the same in every lane of the wavefront)
         const bool rose = __builtin_amdgcn_ballot_w64(corr != 1.f) != 0;
 #pragma unroll
@@ -683,20 +707,12 @@ __global__ __launch_bounds__(256) void sink_attention_tiles_kernel(SinkArgs a, c
             if (vt * 16 < V) *reinterpret_cast<float4*>(dst + vt * 16 + 4 * b) = make_float4(acc[j][0], acc[j][1], acc[j][2], acc[j][3]);
         }
         if (b == 0 && (!SPLITV || wave == 0)) {
-            dst[V] = run_max;
-            dst[V + 1] = run_sum;
+            dst[V] = column.run_max;
+            dst[V + 1] = column.run_sum;
         }
         return;
     }
-    // the sink, and the division
-    float top = run_max, den = run_sum, f = 1.f;
-    if (a.sink != nullptr) {
-        const float sk = a.sink[head] * 1.4426950408889634f;
-        top = fmaxf(run_max, sk);
-        f = run_max > -INFINITY ? exp2f(run_max - top) : 0.f;
-        den = run_sum * f + exp2f(sk - top);
-    }
-    f = den > 0.f ? f / den : 0.f;
+    const float f = column.end(a.sink, head);
     if (!col_ok) return;
     __bf16* dst = a.out + (size_t)m * a.out_stride + (size_t)head * V;
 #pragma unroll
@@ -709,6 +725,204 @@ __global__ __launch_bounds__(256) void sink_attention_tiles_kernel(SinkArgs a, c
             for (int r = 0; r < 4; ++r) four[r] = (__bf16)(acc[j][r] * f);
             *reinterpret_cast<uint2*>(dst + vt * 16 + 4 * b) = *reinterpret_cast<const uint2*>(four);
         }
+    }
+}
+
+// The same for prompt portions whose rows fill the instruction's sizes (keys of KD = 32 NKF channels, values of 16 NVT, pages of
+// whole runs of 16 keys): every column's arithmetic, and so every bit, is the kernel's above; what differs is the way of the data.
+// Eight wavefronts, 128 columns; STAGES tiles of 32 key rows (and value rows, where those are not the key rows) in LDS,
+// all but one of them on their way: loads that go to LDS without passing registers (`buffer_load_dwordx4 .. lds`), a wavefront's
+// share in one run of 16 keys, so in one page.  The values are not transposed on the way in: `ds_read_b64_tr_b16` reads the
+// second product's operand (eight keys of one channel) out of the rows as they lie -- of 16 lanes, lane q gives the place of
+// four channels of row q / 4 and gets channel q of four rows.  16-byte piece p of row r lies at place p ^ f(r) of its eight (f: bits
+// 0, 1 and 3 of r, bit 4 added to the lowest), so that lanes that the LDS serves together read different banks.
+// What bounds it: the LDS (every wavefront reads a tile's rows twice, 68 KB a tile with 576 channels) beside 68 matrix
+// instructions a tile; the kernel above staged a tile, waited, multiplied and waited, one workgroup a compute unit, four wavefronts.
+// Pamunex's latent attention (1777 tokens, 16 heads, window 1024, 576 and 512 channels) @@ us for 320, its attention over
+// blocks (128 channels) @@ for 89.
+template <int NKF, int NVT, bool SHARED, int STAGES> struct SinkRows {
+    static constexpr int KD = NKF * 32, V = NVT * 16, WAVES = 8;
+    static constexpr int K_SHARE = 16 * (KD / 8) / (WAVES / 2), V_SHARE = SHARED ? 0 : 16 * (V / 8) / (WAVES / 2);      // pieces of a wavefront
+    static constexpr int K_LOADS = (K_SHARE + 63) / 64, V_LOADS = (V_SHARE + 63) / 64, LOADS = K_LOADS + V_LOADS;
+    static constexpr int STAGE = TK * (KD + (SHARED ? 0 : V));         // elements
+    static constexpr size_t lds_bytes = (size_t)STAGES * STAGE * sizeof(__bf16) + TILES_MAX_BLOCKS * sizeof(int32_t);
+    static_assert(KD % 64 == 0 && V % 64 == 0 && lds_bytes <= 160 * 1024 && LOADS * (STAGES - 1) <= 63, "eight pieces a swap, the LDS, the counter");
+};
+template <int LEFT> __device__ __forceinline__ void sink_arrive() {      // (the compiler does not follow loads that go to LDS)
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LEFT) : "memory");
+}
+
+template <int NKF, int NVT, bool SHARED, int STAGES>
+__global__ __launch_bounds__(512, 2) void sink_attention_rows_kernel(SinkArgs a, const int32_t* __restrict__ group_first,
+                                                                     const int32_t* __restrict__ group_count, int head_block, int head_blocks) {
+    using S = SinkRows<NKF, NVT, SHARED, STAGES>;
+    constexpr int KD = S::KD, V = S::V;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+    __bf16* rows_lds = reinterpret_cast<__bf16*>(lds_raw);             // [STAGES][keys: TK][KD], then, not SHARED, [values: TK][V]
+    int32_t* page_lds = reinterpret_cast<int32_t*>(rows_lds + STAGES * S::STAGE);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int group = blockIdx.x, kvh = blockIdx.y / head_blocks, hb = blockIdx.y % head_blocks;
+    const int first = group_first[group], count = group_count[group];
+    const int hg = a.q_heads / a.kv_heads;
+    const int p0 = a.positions[first], slot = a.slots[first];
+    const int kbegin = first_seen(p0, a.mask_kind, a.mask_size), kend = p0 + count;
+    // (tiles are numbered as in the kernel above)
+    int kept = (min(a.keep_first, kend) + TK - 1) / TK;
+    const int gap = max(0, kbegin / TK - kept);
+    if (gap == 0) kept = 0;
+    // The first tile that a token sees may lie behind tile 0 (window, chunk): without kept keys the gap makes it number 0.
+    const int i_end = (kend + TK - 1) / TK - gap;
+    const int32_t* table = a.block_table + (size_t)slot * a.max_blocks;
+
+    const int q4 = lane & 15, b = lane >> 4, col = wave * 16 + q4;
+    const int ti = col / head_block, hi = hb * head_block + col % head_block;
+    const bool col_ok = ti < count && hi < hg;
+    const int head = kvh * hg + (hi < hg ? hi : 0);
+    const int m = first + (ti < count ? ti : 0);
+    const int qpos = p0 + ti;
+    const int last_lo = first_seen(p0 + count - 1, a.mask_kind, a.mask_size);
+    bf16x8 qf[NKF];
+    const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int kf = 0; kf < NKF; ++kf)
+        qf[kf] = col_ok ? *reinterpret_cast<const bf16x8*>(a.q + (size_t)m * a.q_stride + (size_t)head * KD + kf * 32 + b * 8) : zero8;
+    floatx4 acc[NVT];
+#pragma unroll
+    for (int j = 0; j < NVT; ++j) acc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    SinkColumn column(a, col_ok, first_seen(qpos, a.mask_kind, a.mask_size), qpos);
+
+    const int lead_end = min(i_end, kept) * TK;
+    const int n_lead = lead_end > 0 ? (lead_end - 1) / a.page_size + 1 : 0;
+    const int main_first = max((kept + gap) * TK, a.keep_first > 0 ? 0 : kbegin);
+    const int main_end = min(kend, (i_end + gap) * TK);
+    const int block0 = main_first / a.page_size;
+    const int n_main = main_end > main_first ? (main_end - 1) / a.page_size - block0 + 1 : 0;
+    const int n_blocks = min(n_lead + n_main, TILES_MAX_BLOCKS);
+    int mine_mapped = 1;
+    for (int i = tid; i < n_blocks; i += 512) {
+        const int blk = i < n_lead ? i : block0 + i - n_lead, page = blk < a.max_blocks ? table[blk] : -1;
+        page_lds[i] = page;
+        mine_mapped &= page >= 0 ? 1 : 0;
+    }
+    const bool mapped = __syncthreads_and(mine_mapped) != 0;
+
+    const auto tile_at = [&](int i) { return (i < kept ? i : i + gap) * TK; };
+    // The page of the 16 keys from key0 on, -1 where there is none (beyond the range, or not mapped).
+    auto page_of = [&](int key0) {
+        const bool lead = key0 < lead_end;
+        const int rel = key0 / a.page_size - (lead ? 0 : block0), blk = lead ? rel : n_lead + rel;
+        return __builtin_amdgcn_readfirstlane(rel >= 0 && blk < n_blocks ? page_lds[blk] : -1);
+    };
+    auto swap = [](int r) { return ((r & 3) | (r & 8) >> 1) ^ (r >> 4 & 1); };
+    // what this lane asks for: piece by piece of its wavefront's quarter of a run, bytes from the run's first row
+    const int run = wave >> 2, quarter = wave & 3;
+    uint32_t k_at[S::K_LOADS], v_at[SHARED ? 1 : S::V_LOADS];
+    auto places = [&](uint32_t (&at)[S::K_LOADS], int share, int width, long stride) {
+#pragma unroll
+        for (int i = 0; i < S::K_LOADS; ++i) {
+            const int piece = quarter * share + i * 64 + lane, r = piece / (width / 8), place = piece % (width / 8);
+            at[i] = (uint32_t)(r * (int)stride + ((place & ~7) | ((place & 7) ^ swap(16 * run + r))) * 8) * 2u;
+        }
+    };
+    places(k_at, S::K_SHARE, KD, a.k_row);
+    if constexpr (!SHARED) {
+        static_assert(SHARED || S::K_LOADS == S::V_LOADS, "one loop for both");
+        places(v_at, S::V_SHARE, V, a.v_row);
+    }
+    const uint32_t k_run = (uint32_t)a.k_row * 32u, v_run = (uint32_t)a.v_row * 32u;      // bytes of a run of 16 rows
+    auto ask = [&](int i, int stage) {
+        const int key0 = tile_at(i) + 16 * run;
+        const long long row = ((long long)max(page_of(key0), 0) * a.kv_heads + kvh) * a.page_size + key0 % a.page_size;
+        __bf16* to = rows_lds + stage * S::STAGE;
+        auto some = [&](const __bf16* from, uint32_t bytes, const uint32_t (&at)[S::K_LOADS], int share, __bf16* dst) {
+            const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)from, 0, (int)bytes, 0x00027000);
+#pragma unroll
+            for (int l = 0; l < S::K_LOADS; ++l)
+                if ((l + 1) * 64 <= share || l * 64 + lane < share)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)(dst + (run * 4 * share + quarter * share + l * 64) * 8), 16,
+                                                             (int)at[l], 0, 0, 0);
+        };
+        some(a.k_pages + row * a.k_row, k_run, k_at, S::K_SHARE, to);
+        if constexpr (!SHARED) some(a.v_pages + row * a.v_row, v_run, v_at, S::V_SHARE, to + TK * KD);
+    };
+    // Rows outside the range, or without a page, count as zeros.
+    auto clear = [&](int i, int stage) {
+        const int t0 = tile_at(i);
+        const bool lead = t0 < lead_end;
+        const int end = lead ? lead_end : main_end;
+        if (mapped && (t0 >= kbegin || t0 + TK <= a.keep_first) && t0 + TK <= end) return;     // (the same in every thread)
+        const bool here[2] = {page_of(t0) >= 0, page_of(t0 + 16) >= 0};
+        constexpr int WIDTH = S::STAGE / TK / 8;                        // pieces of a key's rows
+        for (int c = tid; c < TK * WIDTH; c += 512) {
+            const int r = c < TK * (KD / 8) ? c / (KD / 8) : (c - TK * (KD / 8)) / (V / 8), kp = t0 + r;
+            if ((r < 16 ? here[0] : here[1]) && (kp >= kbegin || kp < a.keep_first) && kp < end) continue;
+            *reinterpret_cast<bf16x8*>(rows_lds + stage * S::STAGE + c * 8) = zero8;
+        }
+        __syncthreads();
+    };
+    // places of the operands in a stage, in bytes: the first product's for even and odd groups of 32 channels (the second half of its
+    // rows lies four rows on, which is no other place), the second's for every one of four neighbouring blocks of 16
+    uint32_t k_place[2], v_place[4];
+    {
+        const int r = 8 * (q4 >> 2) + (q4 & 3), tr = 8 * b + (q4 >> 2);
+#pragma unroll
+        for (int odd = 0; odd < 2; ++odd) k_place[odd] = (uint32_t)((r * KD + 8 * ((4 * odd + b) ^ swap(r))) * 2);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            v_place[j] = (uint32_t)(((SHARED ? tr * KD : TK * KD + tr * V) + 8 * ((2 * j + (q4 >> 1 & 1)) ^ swap(tr)) + 4 * (q4 & 1)) * 2);
+    }
+    constexpr int V_PITCH = SHARED ? KD : V;
+    const uint32_t rows_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)rows_lds;
+    typedef __attribute__((__vector_size__(4 * sizeof(short)))) short short4_t;
+    auto tile = [&](int t0, int stage) {
+        const uint32_t base = rows_base + (uint32_t)stage * (uint32_t)(S::STAGE * 2);
+        const uint32_t k_base[2] = {base + k_place[0], base + k_place[1]};
+        floatx4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kf = 0; kf < NKF; ++kf) {
+            const uint32_t at = k_base[kf & 1] + (kf >> 1) * 128;
+            const bf16x8 a0 = *(__attribute__((address_space(3))) const bf16x8*)(uintptr_t)at;
+            const bf16x8 a1 = *(__attribute__((address_space(3))) const bf16x8*)(uintptr_t)(at + 4 * KD * 2);
+            s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, qf[kf], s0, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, qf[kf], s1, 0, 0, 0);
+        }
+        const bool whole = (t0 >= last_lo || t0 + TK <= a.keep_first) && t0 + TK - 1 <= p0;
+        bf16x8 pf;
+        const float corr = column.tile(s0, s1, t0 + 8 * b, whole, a.keep_first, pf);
+        const bool rose = __builtin_amdgcn_ballot_w64(corr != 1.f) != 0;
+        const uint32_t v_base[4] = {base + v_place[0], base + v_place[1], base + v_place[2], base + v_place[3]};
+#pragma unroll
+        for (int j = 0; j < NVT; ++j) {
+            if (rose) acc[j] *= corr;
+            const uint32_t at = v_base[j & 3] + (j >> 2) * 128;
+            const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)(uintptr_t)at);
+            const short4_t up = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)(uintptr_t)(at + 4 * V_PITCH * 2));
+            const bf16x8 av = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7));
+            acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, pf, acc[j], 0, 0, 0);
+        }
+    };
+#pragma unroll
+    for (int s = 0; s < STAGES - 1; ++s)
+        if (s < i_end) ask(s, s);
+    int stage = 0;
+    for (int i = 0; i < i_end; ++i) {
+        // this wavefront's part of the tile is there, and behind the barrier everyone's; everyone is done with the tile before
+        if (i + STAGES - 2 < i_end) sink_arrive<S::LOADS * (STAGES - 2)>();
+        else sink_arrive<0>();
+        if (i + STAGES - 1 < i_end) ask(i + STAGES - 1, stage == 0 ? STAGES - 1 : stage - 1);
+        clear(i, stage);
+        if (wave * 16 < count * head_block) tile(tile_at(i), stage);      // (a wavefront without columns only brings rows)
+        stage = stage + 1 == STAGES ? 0 : stage + 1;
+    }
+    const float f = column.end(a.sink, head);
+    if (!col_ok) return;
+    __bf16* dst = a.out + (size_t)m * a.out_stride + (size_t)head * V;
+#pragma unroll
+    for (int j = 0; j < NVT; ++j) {
+        alignas(8) __bf16 four[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) four[r] = (__bf16)(acc[j][r] * f);
+        *reinterpret_cast<uint2*>(dst + j * 16 + 4 * b) = *reinterpret_cast<const uint2*>(four);
     }
 }
 
@@ -781,6 +995,17 @@ static int launch_sink_tiles(const SinkArgs& a, const int32_t* first, const int3
         constexpr int NC = (NVT * 16 + 63) / 64;
         sink_tiles_combine_kernel<NC><<<dim3(groups, a.q_heads, a.group_tokens), 64, 0, stream>>>(a, first, count);
     }
+    return (int)hipGetLastError();
+}
+
+template <int NKF, int NVT, bool SHARED, int STAGES>
+static int launch_sink_rows(const SinkArgs& a, const int32_t* first, const int32_t* count, int groups, int head_block, int head_blocks,
+                            hipStream_t stream) {
+    using S = SinkRows<NKF, NVT, SHARED, STAGES>;
+    auto* kernel = sink_attention_rows_kernel<NKF, NVT, SHARED, STAGES>;
+    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds_bytes);
+    if (allowed != hipSuccess) return (int)allowed;
+    kernel<<<dim3(groups, a.kv_heads * head_blocks), 512, S::lds_bytes, stream>>>(a, first, count, head_block, head_blocks);
     return (int)hipGetLastError();
 }
 #endif
@@ -906,6 +1131,38 @@ int mlr_sink_attention_tiles(const void* q, long q_stride, const void* k_pages, 
 #else
     return 1;
 #endif
+}
+
+// The rows' kernel over groups of at most 128 / head_block tokens, without key ranges: keys of 128 channels beside values of 128,
+// or latent rows of 576 channels whose first 512 are the values.  Returns 1 for other sizes.  Every result has the bits of the kernel above.
+int mlr_sink_attention_rows(const void* q, long q_stride, const void* k_pages, long k_row, const void* v_pages, long v_row,
+                            const int32_t* block_table, int max_blocks, const int32_t* slots, const int32_t* positions,
+                            const float* sink, void* out, long out_stride, const int32_t* group_first, const int32_t* group_count,
+                            int groups, int head_block, int q_heads, int kv_heads, int key_dim, int value_dim, int page_size,
+                            int mask_kind, int mask_size, int keep_first, float softcap, int max_context, float scale,
+                            hipStream_t stream) {
+#if MLR_BF16
+    if (groups <= 0) return 0;
+    const long reach = mask_kind == MASK_ALL ? (long)max_context : (long)mask_size + 128 + (keep_first > 0 ? keep_first + 96 : 0);
+    if (page_size < 16 || page_size % 16 != 0 || reach / page_size + (keep_first > 0 ? 4 : 2) > TILES_MAX_BLOCKS) return 1;
+    if (k_row % 8 != 0 || v_row % 8 != 0 || k_row < key_dim || v_row < value_dim || k_row >= (1 << 24) || v_row >= (1 << 24) || q_stride % 8 != 0 ||
+        out_stride % 4 != 0 || kv_heads <= 0 || q_heads % kv_heads != 0 ||
+        (((uintptr_t)q | (uintptr_t)k_pages | (uintptr_t)v_pages) & 15) != 0 || ((uintptr_t)out & 7) != 0)
+        return 1;
+    if (head_block < 1 || head_block > 128 || (head_block & (head_block - 1)) != 0 || (mask_kind != MASK_ALL && mask_size <= 0) ||
+        keep_first < 0 || !(softcap >= 0.f))
+        return -1;
+    const int hg = q_heads / kv_heads, head_blocks = (hg + head_block - 1) / head_block;
+    if ((long)kv_heads * head_blocks > 65535) return -2;
+    SinkArgs a{(const elem_t*)q, q_stride, (const elem_t*)k_pages, k_row, (const elem_t*)v_pages, v_row, block_table,
+               slots, positions, sink, (elem_t*)out, out_stride, max_blocks, q_heads, kv_heads, key_dim, value_dim,
+               page_size, mask_kind, mask_size, keep_first, scale, softcap, nullptr, 0, 1, 128 / head_block};
+    if (key_dim == 576 && value_dim == 512 && k_pages == v_pages && k_row == v_row)
+        return launch_sink_rows<18, 32, true, 4>(a, group_first, group_count, groups, head_block, head_blocks, stream);
+    if (key_dim == 128 && value_dim == 128 && k_pages != v_pages)
+        return launch_sink_rows<4, 8, false, 3>(a, group_first, group_count, groups, head_block, head_blocks, stream);
+#endif
+    return 1;
 }
 
 }  // extern "C"

@@ -1729,6 +1729,49 @@ class Kernels:
             _p(partial if splits > 1 else None), _c_int(int(split_keys)), _c_int(int(splits)), _stream())
         _ok(code, "sink_attention_tiles")
 
+    def sink_rows_supported(self, key_dim, value_dim, k_pages, v_pages, page_size, mask=None, mask_size=0, max_context=0, keep_first=0):
+        """The sizes of `sink_attention_rows`: keys and values of 128 channels, or latent rows of 576 channels whose first 512
+        are the values, in pages of whole runs of 16, and page ids of a workgroup's keys that fit what it keeps of them."""
+        whole = self.SINK_MASKS.get(mask, 0) == 0
+        kept = not whole and keep_first > 0
+        reach = max_context if whole else mask_size + 128 + (keep_first + 96 if kept else 0)
+        return (self.dtype == torch.bfloat16 and page_size % 16 == 0 and reach // page_size + (4 if kept else 2) <= self.SINK_TILES_BLOCKS and _on16(k_pages, v_pages) and k_pages.shape[3] < 2 ** 24
+                and ((key_dim, value_dim) == (128, 128) and k_pages.data_ptr() != v_pages.data_ptr()
+                     or (key_dim, value_dim) == (576, 512) and k_pages.data_ptr() == v_pages.data_ptr() and k_pages.shape[3] == v_pages.shape[3]))
+
+    @timed("attention")
+    def sink_attention_rows(self, q, k_pages, v_pages, block_table, slots, positions, sink, out, group_first, group_count,
+                            groups, head_block, q_heads, kv_heads, key_dim, value_dim, page_size, scale, mask=None, mask_size=0,
+                            max_context=0, keep_first=0, softcap=None):
+        """`sink_attention_tiles` for prompt portions of the sizes of `sink_rows_supported`, bit by bit, with at most 128 /
+        head_block tokens a group."""
+        _tensor(q, "q", self.dtype, ndim=2)
+        rows = q.shape[0]
+        _need(q.shape[1] == q_heads * key_dim, "q: wrong width")
+        k_row = self._sink_pages(k_pages, "k_pages", kv_heads, page_size, key_dim)
+        v_row = self._sink_pages(v_pages, "v_pages", kv_heads, page_size, value_dim)
+        _need(mask in self.SINK_MASKS, f"mask {mask!r}: one of all, window, chunk")
+        _need(self.sink_rows_supported(key_dim, value_dim, k_pages, v_pages, page_size, mask, mask_size, max_context, keep_first) and _on16(q, out),
+              "sink_attention_rows: sizes not supported")
+        kind = self.SINK_MASKS[mask]
+        _need(kind == 0 or mask_size >= 1, "a window or chunk needs a positive size")
+        _tensor(block_table, "block_table", torch.int32, ndim=2)
+        _tensor(slots, "slots", torch.int32, (rows,))
+        _tensor(positions, "positions", torch.int32, (rows,))
+        _tensor(group_first, "group_first", torch.int32, ndim=1)
+        _tensor(group_count, "group_count", torch.int32, ndim=1)
+        _need(group_first.numel() >= groups and group_count.numel() >= groups, "group vectors too short")
+        if sink is not None:
+            _tensor(sink, "sink", torch.float32, (q_heads,))
+        _tensor(out, "out", self.dtype, (rows, q_heads * value_dim))
+        code = self._lib("sink_attention").mlr_sink_attention_rows(
+            _p(q), ctypes.c_long(q.shape[1]), _p(k_pages), ctypes.c_long(k_row), _p(v_pages), ctypes.c_long(v_row),
+            _p(block_table), _c_int(block_table.shape[1]), _p(slots), _p(positions), _p(sink), _p(out),
+            ctypes.c_long(out.shape[1]), _p(group_first), _p(group_count), _c_int(groups), _c_int(head_block), _c_int(q_heads),
+            _c_int(kv_heads), _c_int(key_dim), _c_int(value_dim), _c_int(page_size), _c_int(kind), _c_int(int(mask_size)),
+            _c_int(self._kept(kind, keep_first)), _c_float(self._cap(softcap)), _c_int(int(max_context)), _c_float(scale), _stream())
+        _ok(code, "sink_attention_rows")
+
     PORTION_PAGES = 1024          # page ids of a group's keys that the portion kernel keeps
 
     def portion_attention_supported(self, q_heads, kv_heads, key_dim, value_dim, k_row, v_row, page_size, mask=None, mask_size=0,

@@ -124,10 +124,11 @@ def _key_ranges(ctx, groups, tokens, workgroups, q_heads, value_dim, mask, mask_
     return keys, -(-reach // keys), room
 
 
-def portion_columns(ctx, q_heads):
+def portion_columns(ctx, q_heads, least=128):
     """Columns (token, head) of a portion kernel's workgroup: 128 (half the staging a column of those of 64) when the step
-    brings at least one such workgroup for every compute unit."""
-    return 128 if ctx.n_tokens * q_heads >= 128 * ctx.compute_units else 64
+    brings at least `least` columns for every compute unit: one such workgroup each, or, where a workgroup has its compute unit
+    to itself and workgroups of 64 would take their turns, every second."""
+    return 128 if ctx.n_tokens * q_heads >= least * ctx.compute_units else 64
 
 
 def attend(ctx, q, k_pages, v_pages, view, sink, out, q_heads, kv_heads, key_dim, value_dim, scale, mask, mask_size,
@@ -142,14 +143,21 @@ def attend(ctx, q, k_pages, v_pages, view, sink, out, q_heads, kv_heads, key_dim
         big_heads, big_tokens, small_heads, small_tokens = k.sink_tiles_layout(q_heads, kv_heads)
         portions = not ctx.routed and k.portion_attention_supported(q_heads, kv_heads, key_dim, value_dim, k_pages.shape[3], v_pages.shape[3],
                                                                     view.page_size, mask, mask_size, ctx.max_positions, keep_first, scale)
-        if portions:
-            columns, big_heads = portion_columns(ctx, q_heads), min(big_heads, 32)
+        rows = not portions and k.sink_rows_supported(key_dim, value_dim, k_pages, v_pages, view.page_size, mask, mask_size,
+                                                      ctx.max_positions, keep_first)
+        if portions or rows:
+            columns, big_heads = portion_columns(ctx, q_heads, 64 if rows else 128), min(big_heads, 32)
             big_tokens = columns // big_heads
         small, big, _ = ctx.token_groups(small_tokens, max(1, big_tokens // small_tokens), without, rest)
         if portions and big[2] > 0:
             k.portion_attention(q, k_pages, v_pages, view.block_table, ctx.slots, ctx.positions, sink, out, *big, columns, big_heads,
                                 q_heads, kv_heads, key_dim, value_dim, view.page_size, scale, mask, mask_size, ctx.max_positions,
                                 keep_first, softcap)
+            big = (None, None, 0)
+        if rows and big[2] > 0:
+            k.sink_attention_rows(q, k_pages, v_pages, view.block_table, ctx.slots, ctx.positions, sink, out, *big, big_heads, q_heads,
+                                  kv_heads, key_dim, value_dim, view.page_size, scale, mask, mask_size, ctx.max_positions, keep_first,
+                                  softcap)
             big = (None, None, 0)
         for (first, count, n), heads, split in ((big, big_heads, False), (small, small_heads, True)):
             if n == 0:

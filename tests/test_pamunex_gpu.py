@@ -275,6 +275,46 @@ def test_matrix_core_attention_in_groups_of_tokens_and_of_single_tokens(kind, si
         np.testing.assert_allclose(got, want, rtol=3e-2, atol=2e-2, err_msg=str((head_block, tokens, split, ranges)))
 
 
+@pytest.mark.parametrize("kind,size,keep", [("all", 0, 0), ("window", 37, 0), ("chunk", 24, 0), ("window", 1, 0), ("window", 100, 45), ("chunk", 64, 5)])
+@pytest.mark.parametrize("heads,kv,shared,page,before", [(16, 1, True, 16, 0), (5, 1, True, 64, 70), (40, 1, True, 16, 33), (16, 4, False, 16, 0),
+                                                         (3, 3, False, 32, 100), (32, 1, False, 16, 61)])
+def test_attention_of_prompt_portions_by_rows(kind, size, keep, heads, kv, shared, page, before):
+    """Prompt portions of the sizes whose rows fill the matrix instructions: the bits of the kernel that stages and transposes, in
+    groups of 128 columns, of 64 and of a few, behind masks whose pages were given back, with keys that nobody wrote; and close
+    to the plain softmax."""
+    from mini_llm_runtime_amd.kernels import Kernels
+    k = Kernels(torch.bfloat16)
+    dim, vdim = (576, 512) if shared else (128, 128)
+    T, n = before + 150, 150
+    rng = np.random.default_rng(14)
+    rows = as_rounded(rng.normal(size=(T, kv, dim)) * 0.5, torch.bfloat16)
+    values = rows[:, :, :vdim] if shared else as_rounded(rng.normal(size=(T, kv, vdim)), torch.bfloat16)
+    k_pages, table = paged(rows, page, torch.bfloat16, seed=3)
+    v_pages = k_pages if shared else paged(values, page, torch.bfloat16, seed=3)[0]
+    ids = table[0].long()
+    for pages in {id(p): p for p in (k_pages, v_pages)}.values():
+        pages[ids[(T - 1) // page], :, (T - 1) % page + 1:] = float("nan")             # (never written)
+    if kind == "window" and size < before:                                            # pages that no token sees any more are gone
+        for i in range(-(-keep // page), (before + 1 - size) // page):
+            k_pages[ids[i]], v_pages[ids[i]], table[0, i] = float("nan"), float("nan"), -1
+    q = on_gpu(as_rounded(rng.normal(size=(n, heads, dim)) * 0.5, torch.bfloat16).reshape(n, -1), torch.bfloat16)
+    sink = on_gpu(rng.normal(size=heads), torch.float32) if heads != 5 else None
+    cap = 20.0 if heads == 3 else None
+    zeros, positions = torch.zeros(n, dtype=torch.int32, device="cuda"), torch.arange(before, T, dtype=torch.int32, device="cuda")
+    mask = None if kind == "all" else kind
+    big_heads, big_tokens, _, _ = k.sink_tiles_layout(heads, kv)
+    want = torch.full((n, heads * vdim), float("nan"), dtype=torch.bfloat16, device="cuda")
+    k.sink_attention_tiles(q, k_pages, v_pages, table, zeros, positions, sink, want, *groups_of(n, big_tokens), big_heads, False, heads, kv, dim, vdim,
+                           page, 0.25, mask, size, T, keep_first=keep, softcap=cap)
+    assert bool(torch.isfinite(want.float()).all())
+    block = min(big_heads, 32)
+    for tokens in (128 // block, 64 // block, max(1, 128 // block - 1), 1):
+        out = torch.full_like(want, float("nan"))
+        k.sink_attention_rows(q, k_pages, v_pages, table, zeros, positions, sink, out, *groups_of(n, tokens), block, heads, kv, dim, vdim, page, 0.25,
+                              mask, size, T, keep_first=keep, softcap=cap)
+        assert torch.equal(out, want), tokens
+
+
 @pytest.mark.parametrize("dtype_name", DTYPES)
 def test_sink_attention_without_a_sink_and_with_values_inside_the_key_rows(dtype_name):
     """sink None is the usual softmax; values may be the first channels of the key rows themselves."""
