@@ -481,18 +481,25 @@ struct SinkColumn {
     // The scores of the eight keys from key0 on -> probabilities pf; returns the factor on the sums so far.
     __device__ __forceinline__ float tile(const floatx4& s0, const floatx4& s1, int key0, bool whole, int keep_first, bf16x8& pf) {
         float sc[8];
-        float tile_max = -INFINITY;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const int kp = key0 + e;
             const float raw = e < 4 ? s0[e] : s1[e - 4];
-            const bool seen = ok && (whole || ((kp >= lo || kp < keep_first) && kp <= pos));
             // (capped: c tanh(s / c) = c - 2 c / (1 + e^(2 s / c)), here in base 2; an exponent beyond 32 bits gives c)
-            const float s2 = capped ? cap2 - 2.0f * cap2 * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(raw * cap_slope))
-                                    : raw * scale2;
-            sc[e] = seen ? s2 : -INFINITY;
-            tile_max = fmaxf(tile_max, sc[e]);
+            sc[e] = capped ? cap2 - 2.0f * cap2 * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(raw * cap_slope)) : raw * scale2;
         }
+        if (whole) {                                   // (the same in every lane: a branch, not eight comparisons)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sc[e] = ok ? sc[e] : -INFINITY;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int kp = key0 + e;
+                sc[e] = ok && (kp >= lo || kp < keep_first) && kp <= pos ? sc[e] : -INFINITY;
+            }
+        }
+        float tile_max = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) tile_max = fmaxf(tile_max, sc[e]);
         tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16, MLR_WAVE));
         tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, MLR_WAVE));
         const float new_max = fmaxf(run_max, tile_max);
@@ -738,8 +745,8 @@ __global__ __launch_bounds__(256) void sink_attention_tiles_kernel(SinkArgs a, c
 // 0, 1 and 3 of r, bit 4 added to the lowest), so that lanes that the LDS serves together read different banks.
 // What bounds it: the LDS (every wavefront reads a tile's rows twice, 68 KB a tile with 576 channels) beside 68 matrix
 // instructions a tile; the kernel above staged a tile, waited, multiplied and waited, one workgroup a compute unit, four wavefronts.
-// Pamunex's latent attention (1777 tokens, 16 heads, window 1024, 576 and 512 channels) @@ us for 320, its attention over
-// blocks (128 channels) @@ for 89.
+// Pamunex's latent attention (1777 tokens, 16 heads, window 1024, 576 and 512 channels) 107 us for 320, its attention over
+// blocks (128 channels) 51 for 89.
 template <int NKF, int NVT, bool SHARED, int STAGES> struct SinkRows {
     static constexpr int KD = NKF * 32, V = NVT * 16, WAVES = 8;
     static constexpr int K_SHARE = 16 * (KD / 8) / (WAVES / 2), V_SHARE = SHARED ? 0 : 16 * (V / 8) / (WAVES / 2);      // pieces of a wavefront
@@ -748,6 +755,14 @@ template <int NKF, int NVT, bool SHARED, int STAGES> struct SinkRows {
     static constexpr size_t lds_bytes = (size_t)STAGES * STAGE * sizeof(__bf16) + TILES_MAX_BLOCKS * sizeof(int32_t);
     static_assert(KD % 64 == 0 && V % 64 == 0 && lds_bytes <= 160 * 1024 && LOADS * (STAGES - 1) <= 63, "eight pieces a swap, the LDS, the counter");
 };
+// 16 bytes a lane from its place in the buffer to 16 bytes a lane from `to` on.  (No output register, so nothing that the compiler
+// could use before the load is done; of the builtin it knows that it writes LDS and, before every transposing read, waits for all
+// loads in flight.)
+typedef __attribute__((__vector_size__(4 * sizeof(int)))) int intx4;
+__device__ __forceinline__ void load_to_lds(intx4 rsrc, uint32_t at, const __bf16* to) {
+    const uint32_t lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)to);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(at), "s"(rsrc) : "memory", "m0");
+}
 template <int LEFT> __device__ __forceinline__ void sink_arrive() {      // (the compiler does not follow loads that go to LDS)
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LEFT) : "memory");
 }
@@ -814,36 +829,28 @@ __global__ __launch_bounds__(512, 2) void sink_attention_rows_kernel(SinkArgs a,
         return __builtin_amdgcn_readfirstlane(rel >= 0 && blk < n_blocks ? page_lds[blk] : -1);
     };
     auto swap = [](int r) { return ((r & 3) | (r & 8) >> 1) ^ (r >> 4 & 1); };
-    // what this lane asks for: piece by piece of its wavefront's quarter of a run, bytes from the run's first row
     const int run = wave >> 2, quarter = wave & 3;
-    uint32_t k_at[S::K_LOADS], v_at[SHARED ? 1 : S::V_LOADS];
-    auto places = [&](uint32_t (&at)[S::K_LOADS], int share, int width, long stride) {
-#pragma unroll
-        for (int i = 0; i < S::K_LOADS; ++i) {
-            const int piece = quarter * share + i * 64 + lane, r = piece / (width / 8), place = piece % (width / 8);
-            at[i] = (uint32_t)(r * (int)stride + ((place & ~7) | ((place & 7) ^ swap(16 * run + r))) * 8) * 2u;
-        }
-    };
-    places(k_at, S::K_SHARE, KD, a.k_row);
-    if constexpr (!SHARED) {
-        static_assert(SHARED || S::K_LOADS == S::V_LOADS, "one loop for both");
-        places(v_at, S::V_SHARE, V, a.v_row);
-    }
     const uint32_t k_run = (uint32_t)a.k_row * 32u, v_run = (uint32_t)a.v_row * 32u;      // bytes of a run of 16 rows
     auto ask = [&](int i, int stage) {
         const int key0 = tile_at(i) + 16 * run;
         const long long row = ((long long)max(page_of(key0), 0) * a.kv_heads + kvh) * a.page_size + key0 % a.page_size;
         __bf16* to = rows_lds + stage * S::STAGE;
-        auto some = [&](const __bf16* from, uint32_t bytes, const uint32_t (&at)[S::K_LOADS], int share, __bf16* dst) {
-            const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)from, 0, (int)bytes, 0x00027000);
+        // piece by piece of the wavefront's quarter of a run (bytes from the run's first row; worked out each time: kept, they are
+        // registers that the 576-channel kernel does not have)
+        auto some = [&](const __bf16* from, uint32_t bytes, int share, int width, int stride, __bf16* dst) {
+            const uint64_t start = (uint64_t)(uintptr_t)from;
+            const intx4 rsrc = {__builtin_amdgcn_readfirstlane((int)(uint32_t)start), __builtin_amdgcn_readfirstlane((int)(uint32_t)(start >> 32) & 0xffff), (int)bytes, 0x00027000};
+            int at = lane;
+            asm volatile("" : "+v"(at));
 #pragma unroll
-            for (int l = 0; l < S::K_LOADS; ++l)
-                if ((l + 1) * 64 <= share || l * 64 + lane < share)
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)(dst + (run * 4 * share + quarter * share + l * 64) * 8), 16,
-                                                             (int)at[l], 0, 0, 0);
+            for (int l = 0; l < (share + 63) / 64; ++l) {
+                const uint32_t piece = quarter * share + l * 64 + at, r = piece / (uint32_t)(width / 8), place = piece % (uint32_t)(width / 8);
+                const uint32_t bytes_at = (r * (uint32_t)stride + ((place & ~7u) | ((place & 7u) ^ swap(16 * run + r))) * 8u) * 2u;
+                if ((l + 1) * 64 <= share || l * 64 + lane < share) load_to_lds(rsrc, bytes_at, dst + (run * 4 * share + quarter * share + l * 64) * 8);
+            }
         };
-        some(a.k_pages + row * a.k_row, k_run, k_at, S::K_SHARE, to);
-        if constexpr (!SHARED) some(a.v_pages + row * a.v_row, v_run, v_at, S::V_SHARE, to + TK * KD);
+        some(a.k_pages + row * a.k_row, k_run, S::K_SHARE, KD, (int)a.k_row, to);
+        if constexpr (!SHARED) some(a.v_pages + row * a.v_row, v_run, S::V_SHARE, V, (int)a.v_row, to + TK * KD);
     };
     // Rows outside the range, or without a page, count as zeros.
     auto clear = [&](int i, int stage) {
@@ -862,45 +869,69 @@ __global__ __launch_bounds__(512, 2) void sink_attention_rows_kernel(SinkArgs a,
     };
     // places of the operands in a stage, in bytes: the first product's for even and odd groups of 32 channels (the second half of its
     // rows lies four rows on, which is no other place), the second's for every one of four neighbouring blocks of 16
-    uint32_t k_place[2], v_place[4];
+    // (a piece's number is swapped bit by bit, so the odd group's place is the even one's with 4 pieces' bit flipped, block j's the
+    // first one's with 2 j pieces')
+    uint32_t k_place, v_place;
     {
         const int r = 8 * (q4 >> 2) + (q4 & 3), tr = 8 * b + (q4 >> 2);
-#pragma unroll
-        for (int odd = 0; odd < 2; ++odd) k_place[odd] = (uint32_t)((r * KD + 8 * ((4 * odd + b) ^ swap(r))) * 2);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            v_place[j] = (uint32_t)(((SHARED ? tr * KD : TK * KD + tr * V) + 8 * ((2 * j + (q4 >> 1 & 1)) ^ swap(tr)) + 4 * (q4 & 1)) * 2);
+        k_place = (uint32_t)((r * KD + 8 * (b ^ swap(r))) * 2);
+        v_place = (uint32_t)(((SHARED ? tr * KD : TK * KD + tr * V) + 8 * ((q4 >> 1 & 1) ^ swap(tr)) + 4 * (q4 & 1)) * 2);
     }
     constexpr int V_PITCH = SHARED ? KD : V;
     const uint32_t rows_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)rows_lds;
     typedef __attribute__((__vector_size__(4 * sizeof(short)))) short short4_t;
     auto tile = [&](int t0, int stage) {
         const uint32_t base = rows_base + (uint32_t)stage * (uint32_t)(S::STAGE * 2);
-        const uint32_t k_base[2] = {base + k_place[0], base + k_place[1]};
+        const uint32_t k_base[2] = {base + k_place, base + (k_place ^ 64u)};
         floatx4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+        // (operands are read AHEAD products before their turn, in both products: with the registers nearly full the compiler
+        // would read each just before it)
+        constexpr int AHEAD = 2;
+        bf16x8 ring[AHEAD + 1][2];
+        auto read_keys = [&](int kf) {
+            const uint32_t at = k_base[kf & 1] + (kf >> 1) * 128;
+            ring[kf % (AHEAD + 1)][0] = *(__attribute__((address_space(3))) const bf16x8*)(uintptr_t)at;
+            ring[kf % (AHEAD + 1)][1] = *(__attribute__((address_space(3))) const bf16x8*)(uintptr_t)(at + 4 * KD * 2);
+        };
+#pragma unroll
+        for (int kf = 0; kf < AHEAD; ++kf) read_keys(kf);
 #pragma unroll
         for (int kf = 0; kf < NKF; ++kf) {
-            const uint32_t at = k_base[kf & 1] + (kf >> 1) * 128;
-            const bf16x8 a0 = *(__attribute__((address_space(3))) const bf16x8*)(uintptr_t)at;
-            const bf16x8 a1 = *(__attribute__((address_space(3))) const bf16x8*)(uintptr_t)(at + 4 * KD * 2);
-            s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, qf[kf], s0, 0, 0, 0);
-            s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, qf[kf], s1, 0, 0, 0);
+            if (kf + AHEAD < NKF) read_keys(kf + AHEAD);
+            __builtin_amdgcn_sched_barrier(0);
+            s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ring[kf % (AHEAD + 1)][0], qf[kf], s0, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ring[kf % (AHEAD + 1)][1], qf[kf], s1, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        const bool whole = (t0 >= last_lo || t0 + TK <= a.keep_first) && t0 + TK - 1 <= p0;
-        bf16x8 pf;
-        const float corr = column.tile(s0, s1, t0 + 8 * b, whole, a.keep_first, pf);
-        const bool rose = __builtin_amdgcn_ballot_w64(corr != 1.f) != 0;
-        const uint32_t v_base[4] = {base + v_place[0], base + v_place[1], base + v_place[2], base + v_place[3]};
-#pragma unroll
-        for (int j = 0; j < NVT; ++j) {
-            if (rose) acc[j] *= corr;
+        const uint32_t v_base[4] = {base + v_place, base + (v_place ^ 32u), base + (v_place ^ 64u), base + (v_place ^ 96u)};
+        constexpr int AHEAD_V = 3;
+        bf16x8 values[AHEAD_V + 1];
+        auto read_values = [&](int j) {
             const uint32_t at = v_base[j & 3] + (j >> 2) * 128;
             const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)(uintptr_t)at);
             const short4_t up = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)(uintptr_t)(at + 4 * V_PITCH * 2));
-            const bf16x8 av = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7));
-            acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, pf, acc[j], 0, 0, 0);
+            values[j % (AHEAD_V + 1)] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7));
+        };
+        const bool whole = (t0 >= last_lo || t0 + TK <= a.keep_first) && t0 + TK - 1 <= p0;
+        bf16x8 pf;
+        const float corr = column.tile(s0, s1, t0 + 8 * b, whole, a.keep_first, pf);
+        if (__builtin_amdgcn_ballot_w64(corr != 1.f) != 0) {           // (the same in every lane; beside the products it became 256 selects)
+#pragma unroll
+            for (int j = 0; j < NVT; ++j) acc[j] *= corr;
+        }
+#pragma unroll
+        for (int j = 0; j < AHEAD_V; ++j) read_values(j);
+#pragma unroll
+        for (int j = 0; j < NVT; ++j) {
+            if (j + AHEAD_V < NVT) read_values(j + AHEAD_V);
+            __builtin_amdgcn_sched_barrier(0);
+            acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(values[j % (AHEAD_V + 1)], pf, acc[j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
+    // (the queries are here before the first loads to LDS: waited for inside the loop, they would hold up every turn)
+#pragma unroll
+    for (int kf = 0; kf < NKF; ++kf) asm volatile("" : "+v"(qf[kf]));
 #pragma unroll
     for (int s = 0; s < STAGES - 1; ++s)
         if (s < i_end) ask(s, s);
