@@ -129,3 +129,20 @@ __device__ __forceinline__ float clamped_glu(float gate, float up, float limit, 
     const float g = fminf(gate, limit), u = fminf(fmaxf(up, -limit), limit);
     return (g / (1.0f + expf(-slope * g))) * (u + 1.0f);
 }
+// This wavefront's loads but the last LEFT and all its LDS reads are done, and so are every other wavefront's: behind it the
+// block that those loads filled may be read and the block that those reads took from may be filled again.  The compiler does
+// not follow loads that go to LDS, so both waits are written out.
+template <int LEFT> __device__ __forceinline__ void wide_arrive() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LEFT) : "memory");
+}
+// Compute units of the current device, asked for once; -1 when the device does not say.
+inline int compute_units() {
+    static int units = 0;
+    if (units == 0) {
+        int device = 0;
+        if (hipGetDevice(&device) != hipSuccess ||
+            hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || units <= 0)
+            units = -1;
+    }
+    return units;
+}

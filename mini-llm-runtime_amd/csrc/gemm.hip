@@ -818,18 +818,6 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const __
 
 // Columns of a workgroup when two strips side by side deal the work out more evenly than strips of 16 do, else 0.
 // Only where the weight is long enough for the memory's rate to count (k from 2048).
-// Compute units of the current device, asked for once; -1 when the device does not say.
-static int compute_units() {
-    static int units = 0;
-    if (units == 0) {
-        int device = 0;
-        if (hipGetDevice(&device) != hipSuccess ||
-            hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || units <= 0)
-            units = -1;
-    }
-    return units;
-}
-
 static int skinny_pair_columns(int N, int K) {
     const int units = compute_units();
     if (units < 0 || K < 2048 || N % 4 != 0) return 0;
@@ -935,13 +923,6 @@ struct WideShape {
     static_assert(lds_bytes <= 160 * 1024, "the blocks must fit the LDS");
     static_assert(LOADS * (NS - 1) <= 63, "the counter of loads in flight has six bits");
 };
-
-// This wavefront's loads but the last LEFT and all its LDS reads are done, and so are every other wavefront's: behind it the
-// block that those loads filled may be read and the block that those reads took from may be filled again.  The compiler does
-// not follow loads that go to LDS, so both waits are written out.
-template <int LEFT> __device__ __forceinline__ void wide_arrive() {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LEFT) : "memory");
-}
 
 // What the epilogue does with the finished sums.  The activations after WIDE_SILU are those of the separate kernels, taken of the
 // products as those read them, rounded to bfloat16: the same bits as the two launches one after the other.

@@ -16,6 +16,7 @@
 // `route_combine_kernel` (a token's output: the weighted sum of its experts' rows, in the order of its choices, and what
 // a shared expert gave).
 #include "common.h"
+#include <type_traits>
 
 #define ACT_NONE 0
 #define ACT_RELU2 1
@@ -266,24 +267,24 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(GroupedArgs g) {
 }
 
 // Experts with many rows each (inner sizes in multiples of 64): 32 x 32 tiles of v_mfma_f32_32x32x16_bf16 out of LDS blocks
-// of 64 k, double-buffered, two further blocks on their way from memory in registers.  A workgroup of WM x WN wavefronts,
-// each TM x TN tiles, owns 32 WM TM sorted rows of one expert and 32 WN TN of its weight's rows.  The weight is the
-// instruction's first operand, so a lane ends up with four consecutive columns of one row (lane = 32 h + i: row i of either
-// operand, k slots 8 h .. 8 h + 7; result column i, rows 8 q + 4 h + r in register 4 q + r); with gate and up rows in turn,
-// 16 and 16, a gate and its up projection lie in one lane, eight registers apart.
+// of 64 k, NS of them, brought by loads that do not pass through registers (`buffer_load_dwordx4 .. lds`).  A workgroup of
+// WM x WN wavefronts, each TM x TN tiles, owns 32 WM TM sorted rows of one expert and 32 WN TN of its weight's rows.  The weight
+// is the instruction's first operand, so a lane ends up with four consecutive columns of one row (lane = 32 h + i: row i of
+// either operand, k slots 8 h .. 8 h + 7; result column i, rows 8 q + 4 h + r in register 4 q + r); with gate and up rows in
+// turn, 16 and 16, a gate and its up projection lie in one lane, eight registers apart.
+// A row of a block is eight pieces of 16 bytes; a load writes eight rows side by side, so rows cannot be padded apart: piece p
+// of row r lies at place p ^ (r & 7), and the eight lanes that the LDS serves together read eight different banks.
 // The workgroups' tiles are counted expert by expert, within one a strip of the weight for all of the expert's rows first;
 // every XCD takes a contiguous range of those there are, so a strip is fetched into one L2.
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 #define EB_K 64
-#define EB_PITCH (EB_K + 8)
 
-template <int WM, int WN, int TM, int TN>
-__global__ __launch_bounds__(64 * WM * WN) void experts_wide_kernel(GroupedArgs g) {
-    constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN, THREADS = 64 * WM * WN, ROWS = BM + BN;
-    constexpr int STEP = THREADS / 8, PT = ROWS / STEP, PW = BN / STEP;      // 16-byte pieces a thread stages, of them weight
-    static_assert(ROWS % STEP == 0 && BN % STEP == 0, "the staged pieces must divide among the threads");
+template <int WM, int WN, int TM, int TN, int NS>
+__global__ __launch_bounds__(64 * WM * WN, 2) void experts_wide_kernel(GroupedArgs g) {
+    constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN, ROWS = BM + BN, LOADS = ROWS / 8 / (WM * WN), STAGE = ROWS * EB_K;
+    static_assert(ROWS % (8 * WM * WN) == 0, "a block's rows must divide among the wavefronts");
     extern __shared__ __attribute__((aligned(16))) __bf16 eb_lds[];
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int li = lane & 31, h = lane >> 5, wm = wave / WN, wn = wave % WN;
     // which tile: every wavefront counts the experts' tiles, a lane an expert, 64 experts at a time
     const int cols = (g.N + BN - 1) / BN;
@@ -323,29 +324,25 @@ __global__ __launch_bounds__(64 * WM * WN) void experts_wide_kernel(GroupedArgs 
     group = __builtin_amdgcn_readfirstlane(group);
     if (group < 0) return;
     const int n0 = col * BN, K = g.K, blocks = K / EB_K;
-    const __bf16* w = g.w + (size_t)group * g.w_group;
-    uint32_t src[PT];
-    const int dst0 = (t >> 3) * EB_PITCH + (t & 7) * 8;
+    // Load i of a wavefront brings rows 8 (wave LOADS + i) .. of the block (weight rows first, then the expert's rows; rows beyond
+    // either are its last one again), at 32-bit byte offsets from the bases
+    uint32_t src[LOADS];
 #pragma unroll
-    for (int i = 0; i < PT; ++i) {
-        const int row = (t >> 3) + STEP * i, kc = (t & 7) * 8;
-        if (i < PW) {
-            src[i] = (uint32_t)min(n0 + row, g.N - 1) * (uint32_t)K + kc;
+    for (int i = 0; i < LOADS; ++i) {
+        const int row = (wave * LOADS + i) * 8 + (lane >> 3), piece = ((lane & 7) ^ (row & 7)) * 8;
+        if (row < BN) {
+            src[i] = ((uint32_t)min(n0 + row, g.N - 1) * (uint32_t)K + piece) * 2u;
         } else {
             const int m = min(row0 + row - BN, row_end - 1);
-            src[i] = (uint32_t)(g.gather ? g.gather[m] : m) * (uint32_t)g.lda + kc;
+            src[i] = ((uint32_t)(g.gather ? g.gather[m] : m) * (uint32_t)g.lda + piece) * 2u;
         }
     }
-    bf16x8 stage0[PT], stage1[PT];
-    auto fetch = [&](int kb, bf16x8 (&stage)[PT]) {                           // (blocks past the end fetch the last one again)
-        const size_t k = (size_t)min(kb, blocks - 1) * EB_K;
-#pragma unroll
-        for (int i = 0; i < PT; ++i) stage[i] = *reinterpret_cast<const bf16x8*>((i < PW ? w : g.a) + k + src[i]);
-    };
-    auto stash = [&](int buf, const bf16x8 (&stage)[PT]) {
-        __bf16* base = eb_lds + (size_t)buf * ROWS * EB_PITCH;
-#pragma unroll
-        for (int i = 0; i < PT; ++i) *reinterpret_cast<bf16x8*>(base + dst0 + i * STEP * EB_PITCH) = stage[i];
+    const auto w_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(g.w + (size_t)group * g.w_group), 0, (int)((uint32_t)g.N * (uint32_t)K * 2u), 0x00027000);
+    const auto a_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)g.a, 0, -1, 0x00027000);        // (the gathered rows are the caller's)
+    auto load = [&](int i, int kb, int stage) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds((wave * LOADS + i) * 8 < BN ? w_rsrc : a_rsrc,
+                                                 (__attribute__((address_space(3))) void*)(eb_lds + stage * STAGE + (wave * LOADS + i) * 512),
+                                                 16, (int)src[i], kb * (EB_K * 2), 0, 0);
     };
     floatx16 acc[TN][TM];
 #pragma unroll
@@ -354,51 +351,89 @@ __global__ __launch_bounds__(64 * WM * WN) void experts_wide_kernel(GroupedArgs 
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[j][i][e] = 0.f;
-    auto products = [&](int buf) {
-        const __bf16* base = eb_lds + (size_t)buf * ROWS * EB_PITCH;
-        const __bf16* wb = base + (wn * TN * 32 + li) * EB_PITCH + 8 * h;
-        const __bf16* ab = base + (BN + wm * TM * 32 + li) * EB_PITCH + 8 * h;
-        bf16x8 wf[2][TN], af[2][TM];                                          // the next k step's operands are asked for first
-        auto operands = [&](int ks, int set) {
-#pragma unroll
-            for (int j = 0; j < TN; ++j) wf[set][j] = *reinterpret_cast<const bf16x8*>(wb + j * 32 * EB_PITCH + 16 * ks);
-#pragma unroll
-            for (int i = 0; i < TM; ++i) af[set][i] = *reinterpret_cast<const bf16x8*>(ab + i * 32 * EB_PITCH + 16 * ks);
-        };
-        operands(0, 0);
-#pragma unroll
-        for (int ks = 0; ks < EB_K / 16; ++ks) {
-            if (ks + 1 < EB_K / 16) operands(ks + 1, (ks + 1) & 1);
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-                    acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[ks & 1][j], af[ks & 1][i], acc[j][i], 0, 0, 0);
-        }
+    bf16x8 wf[2][TN], af[2][TM];                                              // the next k step's operands are asked for first
+    auto read = [&](int r, int ks, int stage) {
+        const __bf16* base = eb_lds + stage * STAGE + li * EB_K + ((2 * ks + h) ^ (li & 7)) * 8;
+        if (r < TN) wf[ks & 1][r] = *reinterpret_cast<const bf16x8*>(base + (wn * TN + r) * 32 * EB_K);
+        else af[ks & 1][r - TN] = *reinterpret_cast<const bf16x8*>(base + (BN + (wm * TM + r - TN) * 32) * EB_K);
     };
-    fetch(0, stage0);
-    fetch(1, stage1);
-    stash(0, stage0);
-    fetch(2, stage0);
-    __syncthreads();
-    int kb = 0;
+    // The products of k step ks; between them, when READ, the reads of the next step out of block `from` and, when LOAD, the loads
+    // of block kb into `into`.  The scheduling barriers keep it so.
+    auto products = [&](int ks, bool do_read, int from, bool do_load, int kb, int into) {
+        constexpr int OPERANDS = TM + TN, STEPS = TN * TM, PER = (OPERANDS + STEPS - 2) / (STEPS - 1), PER_L = (LOADS + STEPS - 1) / STEPS;
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+            if (do_read) {
+#pragma unroll
+                for (int r = s * PER; r < (s + 1) * PER && r < OPERANDS; ++r) read(r, (ks + 1) % (EB_K / 16), from);
+            }
+            if (do_load) {
+#pragma unroll
+                for (int l = s * PER_L; l < (s + 1) * PER_L && l < LOADS; ++l) load(l, kb, into);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            acc[s / TM][s % TM] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[ks & 1][s / TM], af[ks & 1][s % TM], acc[s / TM][s % TM], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __builtin_amdgcn_s_setprio(0);
+    };
+    auto read_first = [&](int stage) {
+#pragma unroll
+        for (int r = 0; r < TM + TN; ++r) read(r, 0, stage);
+    };
+    if (blocks >= NS) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i) load(i, s, s);
+        wide_arrive<LOADS * (NS - 1)>();
+        read_first(0);
+        int stage = 0;
+        // A turn: three k steps' products, each beside the next one's reads; the block is read out then and, once everyone is there,
+        // is filled again with block kb + NS beside the last step's products, while the next block's first operands arrive.
 #pragma unroll 1
-    for (; kb + 2 <= blocks; kb += 2) {                                       // two blocks a turn: the stages keep their names
-        products(0);
-        stash(1, stage1);
-        fetch(kb + 3, stage1);
-        __syncthreads();
-        products(1);
-        stash(0, stage0);
-        fetch(kb + 4, stage0);
-        __syncthreads();
+        for (int kb = 0; kb < blocks - NS; ++kb) {
+            const int next = stage + 1 == NS ? 0 : stage + 1;
+            products(0, true, stage, false, 0, 0);
+            products(1, true, stage, false, 0, 0);
+            products(2, true, stage, false, 0, 0);
+            wide_arrive<LOADS * (NS - 2)>();
+            products(3, true, next, true, kb + NS, stage);
+            stage = next;
+        }
+        auto tail = [&](auto self, auto left_) {                              // the last NS blocks: nothing more to ask for
+            constexpr int LEFT = decltype(left_)::value;
+            if constexpr (LEFT > 0) {
+                const int next = stage + 1 == NS ? 0 : stage + 1;
+                products(0, true, stage, false, 0, 0);
+                products(1, true, stage, false, 0, 0);
+                products(2, true, stage, false, 0, 0);
+                if constexpr (LEFT > 1) wide_arrive<LOADS * (LEFT > 1 ? LEFT - 2 : 0)>();
+                products(3, LEFT > 1, next, false, 0, 0);
+                stage = next;
+                self(self, std::integral_constant<int, LEFT - 1>{});
+            }
+        };
+        tail(tail, std::integral_constant<int, NS>{});
+    } else {                                                                  // fewer blocks than the LDS holds: all at once
+        for (int s = 0; s < blocks; ++s)
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i) load(i, s, s);
+        wide_arrive<0>();
+        for (int s = 0; s < blocks; ++s) {
+            read_first(s);
+            products(0, true, s, false, 0, 0);
+            products(1, true, s, false, 0, 0);
+            products(2, true, s, false, 0, 0);
+            products(3, false, 0, false, 0, 0);
+        }
     }
-    if (kb < blocks) products(0);
     // results leave through a piece of LDS of the wavefront's own, as rows of 16-byte pieces
     const bool halves = gated_form(g.act);
     constexpr int OPITCH = TN * 32 + 8, ROWS_W = TM * 32;
-    static_assert((size_t)WM * WN * ROWS_W * OPITCH <= 2 * (size_t)ROWS * EB_PITCH, "the output tiles must fit the LDS");
-    __syncthreads();                                                          // every wavefront has read its last operands
+    static_assert((size_t)WM * WN * ROWS_W * OPITCH <= (size_t)NS * STAGE, "the output tiles must fit the LDS");
+    wide_arrive<0>();                                                         // every wavefront has read its last operands
     __bf16* mine = eb_lds + (size_t)wave * ROWS_W * OPITCH;
     typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 #pragma unroll
@@ -439,17 +474,63 @@ __global__ __launch_bounds__(64 * WM * WN) void experts_wide_kernel(GroupedArgs 
     }
 }
 
-template <int WM, int WN, int TM, int TN>
+template <int WM, int WN, int TM, int TN, int NS>
 static int launch_experts_wide(const GroupedArgs& g, hipStream_t stream) {
     constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
-    constexpr size_t lds = 2 * (size_t)(BM + BN) * EB_PITCH * sizeof(__bf16);
-    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&experts_wide_kernel<WM, WN, TM, TN>),
+    constexpr size_t lds = (size_t)NS * (BM + BN) * EB_K * sizeof(__bf16);
+    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&experts_wide_kernel<WM, WN, TM, TN, NS>),
                                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (allowed != hipSuccess) return (int)allowed;
     const long tiles = ((long)(g.M + BM - 1) / BM + g.groups) * ((g.N + BN - 1) / BN) + 8;      // (at most, and a multiple of 8)
     if (tiles > 0x7ffffff0L) return -2;
-    experts_wide_kernel<WM, WN, TM, TN><<<(unsigned)((tiles + 7) / 8 * 8), 64 * WM * WN, lds, stream>>>(g);
+    experts_wide_kernel<WM, WN, TM, TN, NS><<<(unsigned)((tiles + 7) / 8 * 8), 64 * WM * WN, lds, stream>>>(g);
     return (int)hipGetLastError();
+}
+
+// The kernel's shapes: rows and columns of a workgroup's tile (one on a compute unit at a time), and what a round of tiles takes
+// in microseconds: `round` for its first operands and its results, `all` for each 1024 k.  Fitted to 56 products of 4 to 32
+// experts with uneven numbers of rows (1088 to 17000 together, 704 to 4096 k, weights out of memory; rms 7 % a shape).
+// The shape with the least predicted time took 13 % less than this kernel's predecessor (128 x 128, two blocks staged through
+// registers), geometric mean, 0.65 to 1.02 of it, and so would the best of the four.  What bounds it is how evenly the tiles come
+// out over the compute units: full rounds of 128 x 256 run at 1.1 PFLOP/s.  Two smaller tiles beside each other on a unit hide less
+// of the weight's way from memory (1462 x 2048 x 1408: 29 us, one tile with five blocks under way 22).  In all: 3554 x 2112 x 2048
+// of 8 experts 71 -> 54 us, 3554 x 2048 x 2112 52 -> 41, 1462 x 2816 x 2048 with a clamped gate 48 -> 37, 4096 x 12288 x 4096
+// gated 542 -> 470.
+struct ExpertsCost { int bm, bn; float round, all; };
+static const ExpertsCost EXPERTS_COSTS[] = {{128, 128, 5.32f, 9.03f}, {128, 192, 6.74f, 12.02f}, {128, 256, 7.25f, 14.68f}, {192, 256, 9.80f, 21.20f}};
+
+static int experts_shape_for(int M, int N, int K, int groups) {
+    const int units = compute_units() > 0 ? compute_units() : 256;
+    int best = 0;
+    float least = 0.f;
+    for (int s = 0; s < 4; ++s) {
+        const ExpertsCost& c = EXPERTS_COSTS[s];
+        const float rows = (float)groups * fmaxf((float)M / (float)groups / (float)c.bm + 0.5f, 1.f);      // an expert's last tile is half full
+        const float us = ceilf(rows * (float)((N + c.bn - 1) / c.bn) / (float)units) * (c.round + c.all * (float)K * (1.0f / 1024.0f));
+        if (s == 0 || us < least) {
+            best = s;
+            least = us;
+        }
+    }
+    return best;
+}
+
+// Whether the kernel takes these operands at all: rows by expert, whole blocks of k, 32-bit byte offsets, rows that start on 16
+// bytes.
+static bool experts_wide_takes(const GroupedArgs& g, long a_rows) {
+    return g.offsets != nullptr && g.N >= 128 && g.K % EB_K == 0 && g.lda % 8 == 0 && g.w_group % 8 == 0 && !g.out_float &&
+           ((reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.w) | reinterpret_cast<uintptr_t>(g.out)) & 15) == 0 &&
+           (unsigned long long)a_rows * g.lda < (1ull << 31) && (unsigned long long)g.N * g.K < (1ull << 31);
+}
+
+static int run_experts_wide(int shape, const GroupedArgs& g, hipStream_t stream) {
+    switch (shape) {
+        case 0: return launch_experts_wide<4, 2, 1, 2, 5>(g, stream);
+        case 1: return launch_experts_wide<4, 2, 1, 3, 3>(g, stream);
+        case 2: return launch_experts_wide<2, 4, 2, 2, 3>(g, stream);
+        case 3: return launch_experts_wide<2, 4, 3, 2, 2>(g, stream);
+        default: return -1;
+    }
 }
 #endif
 
@@ -655,7 +736,7 @@ extern "C" {
 
 int mlr_grouped_gemm(const void* a, long lda, long a_group, const void* w, long w_group, void* out, long ldo,
                      long out_group, const int32_t* offsets, const int32_t* gather, int M, int N, int K, int groups,
-                     int act, int out_float, float limit, float slope, hipStream_t stream) {
+                     int act, int out_float, float limit, float slope, long a_rows, hipStream_t stream) {
     if (M <= 0 || N <= 0 || groups <= 0) return 0;
     if (K <= 0 || act < ACT_NONE || act > ACT_GELU_ERF || (act == ACT_GATED_CLAMPED && !(limit > 0.f))) return -1;
 #if !MLR_BF16
@@ -667,12 +748,9 @@ int mlr_grouped_gemm(const void* a, long lda, long a_group, const void* w, long 
     GroupedArgs g{(const elem_t*)a, lda, a_group, (const elem_t*)w, w_group, out, ldo, out_group, offsets, gather,
                   M, N, K, groups, act, out_float, limit, slope};
 #if MLR_BF16
-    // experts with many rows each: the large tile (310 -> 340 TFLOP/s at 2048 tokens of width 2048, 390 -> 420 at width
-    // 4096; the products a head, with inner sizes of 128 to 512, are faster on the small one)
-    const bool aligned = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
-    if (offsets != nullptr && (long)M >= 128L * groups && N >= 128 && K % EB_K == 0 && lda % 8 == 0 && w_group % 8 == 0 && aligned &&
-        !out_float && (unsigned long long)M * lda < (1ull << 32) && (unsigned long long)N * K < (1ull << 32))
-        return launch_experts_wide<2, 2, 2, 2>(g, stream);
+    // experts with many rows each: the large tiles (below 128 rows an expert most of a tile would be padding; the products a
+    // head, with inner sizes of 128 to 512, are faster on the small one)
+    if ((long)M >= 128L * groups && experts_wide_takes(g, a_rows)) return run_experts_wide(experts_shape_for(M, N, K, groups), g, stream);
     if (offsets != nullptr && (long)M >= 256L * groups && N >= 128) {
         const int row_tiles = (M + 127) / 128 + (offsets ? groups : 0);
         if (row_tiles > 65535 || groups > 65535) return -2;
@@ -689,6 +767,20 @@ int mlr_grouped_gemm(const void* a, long lda, long a_group, const void* w, long 
     grouped_gemm_kernel<<<grid, 256, 0, stream>>>(g);
 #endif
     return (int)hipGetLastError();
+}
+
+// For tests and measurements: the products of experts with many rows in a given shape (0 .. 3).
+int mlr_experts_wide(const void* a, const void* w, void* out, const int32_t* offsets, const int32_t* gather, int M, int N, int K,
+                     int groups, int act, int shape, long a_rows, hipStream_t stream) {
+#if MLR_BF16
+    if (M <= 0 || N <= 0 || groups <= 0 || K <= 0 || act < ACT_NONE || act > ACT_GELU_ERF || act == ACT_GATED_CLAMPED) return -1;
+    GroupedArgs g{(const elem_t*)a, K, 0, (const elem_t*)w, (long)N * K, out, gated_form(act) ? N / 2 : N, 0, offsets, gather,
+                  M, N, K, groups, act, 0, 0.f, 0.f};
+    if ((gated_form(act) && N % 32 != 0) || !experts_wide_takes(g, a_rows)) return -1;
+    return run_experts_wide(shape, g, stream);
+#else
+    return -3;
+#endif
 }
 
 int mlr_router_topk(const float* z, long ld, int32_t* ids, float* weights, int rows, int experts, int top, int group_count,

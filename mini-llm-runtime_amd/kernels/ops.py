@@ -2004,7 +2004,7 @@ class Kernels:
         _ok(self._lib("grouped_gemm").mlr_grouped_gemm(
             _p(a), ctypes.c_long(a.stride(0)), ctypes.c_long(a.stride(1)), _p(w), ctypes.c_long(n * k), _p(out),
             ctypes.c_long(out.stride(0)), ctypes.c_long(out.stride(1)), _ptr(0), _ptr(0), _c_int(rows), _c_int(n), _c_int(k),
-            _c_int(groups), _c_int(self.GROUPED_ACTS[act]), _c_int(0), _c_float(0.0), _c_float(0.0), _stream()), "heads_gemm")
+            _c_int(groups), _c_int(self.GROUPED_ACTS[act]), _c_int(0), _c_float(0.0), _c_float(0.0), ctypes.c_long(rows), _stream()), "heads_gemm")
 
     @timed("gemm")
     def experts_gemm(self, a, w, out, offsets, gather=None, act=None, limit=0.0, slope=0.0):
@@ -2030,7 +2030,7 @@ class Kernels:
         _ok(self._lib("grouped_gemm").mlr_grouped_gemm(
             _p(a), ctypes.c_long(k), ctypes.c_long(0), _p(w), ctypes.c_long(n * k), _p(out), ctypes.c_long(out.shape[1]),
             ctypes.c_long(0), _p(offsets), _p(gather), _c_int(rows), _c_int(n), _c_int(k), _c_int(experts),
-            _c_int(self.GROUPED_ACTS[act]), _c_int(0), _c_float(limit), _c_float(slope), _stream()), "experts_gemm")
+            _c_int(self.GROUPED_ACTS[act]), _c_int(0), _c_float(limit), _c_float(slope), ctypes.c_long(a.shape[0]), _stream()), "experts_gemm")
 
     ROUTER_SCORES = {"sigmoid": 0, "softmax": 1}
     ROUTER_GROUPS = {"best_two": 0, "best": 1}

@@ -568,6 +568,34 @@ def test_products_of_experts_with_many_rows(counts, K, N):
             assert torch.isnan(out[rows:].float()).all()
 
 
+@pytest.mark.parametrize("shape", range(4))
+@pytest.mark.parametrize("K,N", [(64, 128), (128, 352), (192, 130), (256, 192), (704, 288)])
+def test_every_tile_of_the_products_of_experts(shape, K, N):
+    """The tile shapes at their edges (one block of k to several turns of the LDS, remainders of rows and columns, empty experts):
+    on whole numbers, whose sums are below 2^24, every order of summation gives the same result, so the output is exact."""
+    import ctypes
+    from mini_llm_runtime_amd.kernels import Kernels
+    lib = Kernels(torch.bfloat16)._lib("grouped_gemm")
+    counts = [300, 0, 1, 128, 127, 129, 31]
+    rows, tokens = sum(counts), 211
+    g = torch.Generator(device="cuda").manual_seed(K + N + shape)
+    whole = lambda *size: torch.randint(-4, 5, size, generator=g, device="cuda").to(torch.bfloat16)
+    x, w = whole(tokens, K), whole(len(counts), N, K)
+    gather = torch.randint(0, tokens, (rows,), generator=g, device="cuda", dtype=torch.int32)
+    offsets = ints(np.concatenate([[0], np.cumsum(counts)]).tolist())
+    expert = torch.repeat_interleave(torch.arange(len(counts)), torch.tensor(counts))
+    want = torch.stack([w[e].float().cpu() @ r for e, r in zip(expert.tolist(), x.float().cpu()[gather.long().cpu()])])
+    p, i, far = (lambda t: ctypes.c_void_p(t.data_ptr())), ctypes.c_int, ctypes.c_long
+    for act, y in ((0, want), (1, torch.relu(want) ** 2)):
+        out = torch.full((rows + 3, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+        assert lib.mlr_experts_wide(p(x), p(w), p(out), p(offsets), p(gather), i(rows), i(N), i(K), i(len(counts)), i(act), i(shape),
+                                    far(tokens), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+        assert torch.equal(out[:rows].cpu(), y.to(torch.bfloat16))
+        assert torch.isnan(out[rows:].float()).all()
+    assert lib.mlr_experts_wide(p(x), p(w), p(out), p(offsets), p(gather), i(rows), i(N), i(K - 8), i(len(counts)), i(0), i(shape),
+                                far(tokens), ctypes.c_void_p(0)) == -1                           # (not whole blocks of k: refused)
+
+
 @pytest.mark.parametrize("shapes", [[(5,)], [(3, 8), (4096,), (7,), (4100,)], [(1,), (9000,)]])
 def test_staged_states_become_live_in_one_launch(shapes):
     from mini_llm_runtime_amd.cache import CacheManager, StateSpec
