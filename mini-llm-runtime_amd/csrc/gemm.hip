@@ -937,9 +937,12 @@ struct WideArgs {
     int act;              // WIDE_*
     float limit, slope;   // of WIDE_CLAMPED
     int vector_out;       // rows of the output start on 16 bytes
+    int lda, ldo, a_head, out_head;       // of the form with a product a head: row pitches of activation and output, and from head to head
 };
 
-template <int WM, int WN, int TM, int TN, int NS, bool OUT_FLOAT, bool GATED>
+// HEADS: head h multiplies its columns of wider rows by a weight of its own, out[m][h] = a[m][h] . w[h]^T; the tiles are counted
+// head by head.
+template <int WM, int WN, int TM, int TN, int NS, bool OUT_FLOAT, bool GATED, bool HEADS = false>
 __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const WideArgs args) {
     using S = WideShape<WM, WN, TM, TN, NS>;
     constexpr int BM = S::BM, BN = S::BN, LOADS = S::LOADS;
@@ -952,10 +955,14 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const WideAr
     // Workgroups go to the 8 XCDs in turn; each XCD gets a contiguous range of tiles, and in it eight tiles of rows beside
     // each other for every tile of columns, so that an L2 holds what its tiles share.
     constexpr int GROUP = 8;
-    int tm, tn;
+    int tm, tn, head = 0;
     {
-        const int total = args.tiles_m * args.tiles_n, xcd = blockIdx.x % 8;
-        const int tile = xcd * (total / 8) + min(xcd, total % 8) + blockIdx.x / 8;
+        const int one = args.tiles_m * args.tiles_n, total = HEADS ? (int)gridDim.x : one, xcd = blockIdx.x % 8;
+        int tile = xcd * (total / 8) + min(xcd, total % 8) + blockIdx.x / 8;
+        if (HEADS) {
+            head = tile / one;
+            tile -= head * one;
+        }
         const int per = GROUP * args.tiles_n, first = tile / per * GROUP, rows = min(GROUP, args.tiles_m - first);
         tm = first + tile % per % rows;
         tn = tile % per / rows;
@@ -983,10 +990,12 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const WideAr
         } else {
             r = min(m0 + row - BN, M - 1);
         }
-        src[i] = ((uint32_t)r * (uint32_t)K + piece) * 2u;
+        src[i] = ((uint32_t)r * (uint32_t)(HEADS && row >= BN ? args.lda : K) + piece) * 2u;
     }
-    const auto w_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)args.w, 0, (int)((uint32_t)N * (GATED ? 2u : 1u) * (uint32_t)K * 2u), 0x00027000);
-    const auto a_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)args.a, 0, (int)((uint32_t)M * (uint32_t)K * 2u), 0x00027000);
+    const auto w_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(args.w + (HEADS ? (size_t)head * N * K : 0)), 0,
+                                                          (int)((uint32_t)N * (GATED ? 2u : 1u) * (uint32_t)K * 2u), 0x00027000);
+    const auto a_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(args.a + (HEADS ? (size_t)head * args.a_head : 0)), 0,
+                                                          (int)((HEADS ? (uint32_t)(M - 1) * (uint32_t)args.lda + (uint32_t)K : (uint32_t)M * (uint32_t)K) * 2u), 0x00027000);
     auto load = [&](int i, int kb, int stage) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds((wave * LOADS + i) * 8 < BN ? w_rsrc : a_rsrc,
                                                  (__attribute__((address_space(3))) void*)(wide_lds + stage * S::STAGE + (wave * LOADS + i) * 512),
@@ -1170,7 +1179,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const WideAr
                                     : (args.act == WIDE_GELU_TANH ? gate_act<1>(x) : args.act == WIDE_RELU ? gate_act<2>(x) : gate_act<0>(x)) * u);
                 }
             }
-            __bf16* o = (__bf16*)args.out + (size_t)m * N + n;
+            __bf16* o = (__bf16*)args.out + (HEADS ? (size_t)m * args.ldo + (size_t)head * args.out_head : (size_t)m * N) + n;
             if (args.vector_out && n + 8 <= N) {
                 *reinterpret_cast<bf16x8*>(o) = v;
             } else {
@@ -1265,7 +1274,7 @@ static bool wide_takes(const void* a, const void* w, int M, int N, int K, bool g
 static int run_wide(int shape, const void* a, const void* w, void* out, int M, int N, int K, bool out_float, int act, float limit,
                     float slope, hipStream_t stream) {
     const bool gated = act >= WIDE_SILU && act <= WIDE_CLAMPED;
-    WideArgs args{(const __bf16*)a, (const __bf16*)w, out, M, N, K, 0, 0, act, limit, slope, 0};
+    WideArgs args{(const __bf16*)a, (const __bf16*)w, out, M, N, K, 0, 0, act, limit, slope, 0, 0, 0, 0, 0};
     const uintptr_t row_bytes = (uintptr_t)N * (out_float ? 4 : 2);
     args.vector_out = ((reinterpret_cast<uintptr_t>(out) | row_bytes) & 15) == 0 ? 1 : 0;
     float time = 0.f;
@@ -1279,6 +1288,33 @@ extern "C" int mlr_gemm_wide(const void* a, const void* w, void* out, int M, int
     if (M <= 0 || N <= 0) return 0;
     if (K <= 0 || (gated && out_float) || !wide_takes(a, w, M, N, K, gated != 0)) return -1;
     return run_wide(shape, a, w, out, M, N, K, out_float != 0, gated ? WIDE_SILU : WIDE_PLAIN, 0.f, 0.f, stream);
+}
+
+// out[m][h] = a[m][h] . w[h]^T of many rows: out and a with rows of `ldo` and `lda` elements, heads `out_head` and `a_head` apart,
+// w [heads, N, K].  128 x 64 tiles of two blocks of LDS, three workgroups on a compute unit: the inner sizes are 128 to 512, two to
+// eight blocks, and what a tile waits for another one hides.  Against tiles of 64 x 64 staged through registers (`mlr_grouped_gemm`,
+// same sums, same bits): 1777 rows of 16 heads, 512 x 128 21.6 -> 11.9 us, 128 x 512 17.1 -> 9.0 (36 MB each: 8 us as a copy);
+// 2048 of 32, 51.8 -> 29.4 and 39.8 -> 26.2; 333 of 16, 8.3 -> 7.9 and 9.1 -> 7.6.  Other tiles, at 1777 rows: 64 x 64 12.7 and 9.4,
+// 128 x 128 11.2 and 9.5, with four blocks of LDS, one on a unit, 15.9 and 8.8, 256 x 128 12.5 and 11.5.
+// -3: not this kernel's (up to 64 rows, operands that it does not take), nothing was launched.
+extern "C" int mlr_gemm_heads(const void* a, long lda, long a_head, const void* w, void* out, long ldo, long out_head, int M, int N,
+                              int K, int heads, hipStream_t stream) {
+    using S = WideShape<4, 2, 2, 2, 2>;
+    if (M <= 64 || N <= 0 || heads <= 0 || K <= 0 || lda < 0 || a_head < 0 || ldo < 0 || out_head < 0 || lda % 8 != 0 || a_head % 8 != 0 ||
+        !wide_takes(a, w, M, N, K, false) || (unsigned long long)M * lda >= (1ull << 31) ||
+        (unsigned long long)(a_head | ldo | out_head) >= (1ull << 31))
+        return -3;
+    const int tiles_m = (M + S::BM - 1) / S::BM, tiles_n = (N + S::BN - 1) / S::BN;
+    if ((long long)tiles_m * tiles_n * heads > 0x7fffffffLL / 8) return -3;
+    const int vector_out = (reinterpret_cast<uintptr_t>(out) & 15) == 0 && ldo % 8 == 0 && out_head % 8 == 0 ? 1 : 0;
+    const WideArgs args{(const __bf16*)a, (const __bf16*)w, out, M, N, K, tiles_m, tiles_n, WIDE_PLAIN, 0.f, 0.f, vector_out,
+                        (int)lda, (int)ldo, (int)a_head, (int)out_head};
+    auto* kernel = gemm_wide_kernel<4, 2, 2, 2, 2, false, false, true>;
+    static const hipError_t allowed = hipFuncSetAttribute(
+        reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds_bytes);
+    if (allowed != hipSuccess) return (int)allowed;
+    kernel<<<dim3(tiles_m * tiles_n * heads), 64 * S::WAVES, S::lds_bytes, stream>>>(args);
+    return (int)hipGetLastError();
 }
 
 // Whether more than 64 rows are this kernel's beside the vendor library (act: WIDE_*).  The library has the faster way on large

@@ -2001,6 +2001,12 @@ class Kernels:
               "heads_gemm: shapes do not fit")
         _need(act in self.GROUPED_ACTS and act not in self.GROUPED_GATED, f"heads_gemm: activation {act!r}")
         n = w.shape[1]
+        if self.dtype == torch.bfloat16 and act is None:
+            rc = self._lib("gemm").mlr_gemm_heads(
+                _p(a), ctypes.c_long(a.stride(0)), ctypes.c_long(a.stride(1)), _p(w), _p(out), ctypes.c_long(out.stride(0)),
+                ctypes.c_long(out.stride(1)), _c_int(rows), _c_int(n), _c_int(k), _c_int(groups), _stream())
+            if rc != -3:                                        # (-3: few rows, or operands that the kernel does not take)
+                return _ok(rc, "heads_gemm")
         _ok(self._lib("grouped_gemm").mlr_grouped_gemm(
             _p(a), ctypes.c_long(a.stride(0)), ctypes.c_long(a.stride(1)), _p(w), ctypes.c_long(n * k), _p(out),
             ctypes.c_long(out.stride(0)), ctypes.c_long(out.stride(1)), _ptr(0), _ptr(0), _c_int(rows), _c_int(n), _c_int(k),

@@ -531,6 +531,33 @@ def test_one_product_a_head_on_slices_of_wider_rows(dtype_name):
     assert np.abs(got[..., :outer] - want).max() <= (2e-5 if dtype_name == "float32" else 1.5e-2) * scale
 
 
+@pytest.mark.parametrize("rows", [64, 65, 128, 129, 300])
+@pytest.mark.parametrize("heads,K,N,a_extra,o_extra", [(3, 128, 512, 64, 64), (4, 512, 128, 0, 0), (2, 64, 72, 8, 3), (5, 192, 33, 0, 5),
+                                                       (1, 128, 65, 5, 0), (3, 72, 40, 0, 0)])
+def test_one_product_a_head_of_many_rows(rows, heads, K, N, a_extra, o_extra):
+    """The kernel for many rows and what it leaves to the general one (pitches that are no multiple of 16 bytes, inner sizes that
+    are none of 64): every form gives the general kernel's bits, and nothing beside the heads' columns is written."""
+    import ctypes
+    from mini_llm_runtime_amd.kernels import Kernels
+    k = Kernels(torch.bfloat16)
+    g = torch.Generator(device="cuda").manual_seed(rows + K + N)
+    draw = lambda *size: torch.randn(size, generator=g, device="cuda").to(torch.bfloat16)
+    a, w = draw(rows, heads, K + a_extra)[:, :, :K], draw(heads, N, K)
+    outs = [torch.full((rows + 1, heads, N + o_extra), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    got, want = (o[:rows, :, :N] for o in outs)
+    k.heads_gemm(a, w, got)
+    p, i, far, none = (lambda t: ctypes.c_void_p(t.data_ptr())), ctypes.c_int, ctypes.c_long, ctypes.c_void_p(0)
+    assert k._lib("grouped_gemm").mlr_grouped_gemm(
+        p(a), far(a.stride(0)), far(a.stride(1)), p(w), far(N * K), p(want), far(want.stride(0)), far(want.stride(1)), none, none, i(rows),
+        i(N), i(K), i(heads), i(0), i(0), ctypes.c_float(0.0), ctypes.c_float(0.0), far(rows),
+        ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    assert torch.equal(outs[0], outs[1])
+    exact = torch.einsum("mhk,hnk->mhn", a.cpu().double(), w.cpu().double())
+    # (32-bit sums of K products, then one rounding to eight bits: half a unit of 2^-8 and K 2^-24 of the sum of magnitudes)
+    size = torch.einsum("mhk,hnk->mhn", a.cpu().double().abs(), w.cpu().double().abs())
+    assert ((got.cpu().double() - exact).abs() <= 2.0 ** -8 * exact.abs() + (K + 1) * 2.0 ** -24 * size).all()
+
+
 # ---- models ------------------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("dtype_name", DTYPES)
 @pytest.mark.parametrize("name", CONFIGS)
