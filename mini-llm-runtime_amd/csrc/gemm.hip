@@ -4,9 +4,9 @@
 // Float engine: 32-bit matrix instructions, a wavefront a strip of columns for few rows and tiles for many; every element is
 // one chain of fmaf over k from 0 up, so a row's result does not depend on the other rows of the batch.
 // Bfloat16 engine, three families, each with a fixed k order for every output element (so a row's result
-// does not depend on the rows beside it): up to 64 rows the weight is streamed once straight into
-// v_mfma_f32_16x16x32_bf16 (`gemm_skinny_kernel`, optionally with the residual add and RMSNorm in front
-// or silu(gate) * up behind); more rows with k a multiple of 64 go to `gemm_wide_kernel` (tiles out of
+// does not depend on the rows beside it): up to 16 rows, and to 64 where `few_wins` does not say otherwise, the weight is
+// streamed once straight into v_mfma_f32_16x16x32_bf16 (`gemm_skinny_kernel`, optionally with the residual add and RMSNorm in
+// front or silu(gate) * up behind); more rows with k a multiple of 64 go to `gemm_wide_kernel` (tiles out of
 // blocks of LDS that loads fill without passing through registers); any other k to the plain 16x16-tile kernel `gemm_bf16_kernel`.
 #include "common.h"
 #include <type_traits>
@@ -1213,7 +1213,10 @@ static int launch_wide_as(WideArgs& args, hipStream_t stream) {
 template <int WM, int WN, int TM, int TN, int NS, int GWM = WM, int GWN = WN, int GTM = TM, int GTN = TN>
 static int launch_wide(WideArgs& args, bool out_float, bool gated, hipStream_t stream) {
     static_assert(WM * TM == GWM * GTM && WN * TN == GWN * GTN, "one tile for both forms");
-    if (gated) return launch_wide_as<GWM, GWN, GTM, GTN, NS, false, true>(args, stream);
+    if constexpr (GTN % 2 == 0) {
+        if (gated) return launch_wide_as<GWM, GWN, GTM, GTN, NS, false, true>(args, stream);
+    }
+    if (gated) return -1;
     if (out_float) return launch_wide_as<WM, WN, TM, TN, NS, true, false>(args, stream);
     return launch_wide_as<WM, WN, TM, TN, NS, false, false>(args, stream);
 }
@@ -1229,6 +1232,35 @@ static const WideCost WIDE_COSTS[WIDE_SHAPES] = {
     {128, 128, 1, -0.1f, 0.f, 8.1f},   {192, 128, 1, 1.2f, 0.f, 9.8f},    {128, 192, 1, 0.6f, 0.f, 10.4f},  {256, 128, 1, 1.9f, 0.f, 11.9f},
     {256, 192, 1, -2.2f, 0.f, 19.4f},  {256, 256, 1, -1.1f, 0.f, 21.8f}};
 
+
+// The same for 17 to 64 rows, where a workgroup reads its weight once and what counts is the bytes of weight under way: narrow tiles
+// with up to 19 blocks on their way.  `row`: what 16 more rows add to a round.  Fitted to 240 products of 17, 24, 32, 40, 48 and 64
+// rows, inner sizes of 1024 to 5632 and 512 to 33792 rows of weight, weights cold (rms 10 to 20 % a shape; the predicted shape is
+// then 2 % behind the best one on average).  Strips of 16 columns have no gated form.
+struct FewCost { int shape, bm, bn, per_unit; float fixed, one, all, row; };
+static const FewCost FEW_COSTS[] = {
+    {0, 64, 32, 2, 2.0f, 2.0f, 5.5f, 0.62f},  {1, 64, 64, 2, 1.8f, 3.1f, 9.7f, 0.73f}, {10, 64, 16, 1, 1.7f, 0.f, 2.3f, 0.18f},
+    {11, 64, 96, 1, 2.2f, 0.f, 4.2f, 0.51f},  {12, 32, 16, 1, 2.05f, 0.f, 2.23f, 0.f}, {13, 32, 32, 1, 1.35f, 0.f, 3.1f, 0.f},
+    {14, 32, 64, 1, 1.2f, 0.f, 4.3f, 0.f}};
+
+static int few_shape_for(int M, int N, int K, bool gated) {
+    const int units = compute_units() > 0 ? compute_units() : 256, row_tiles = (M + 15) / 16;
+    int best = -1;
+    float time = 0.f;
+    for (const FewCost& c : FEW_COSTS) {
+        if (M > c.bm || (gated && c.bn == 16)) continue;
+        const int bn = gated ? c.bn / 2 : c.bn, tiles = (N + bn - 1) / bn, slots = units * c.per_unit, left = tiles % slots;
+        const bool alone = c.per_unit == 2 && left > 0 && left <= units;
+        const float rounds = (float)(tiles / slots + (left > 0 && !alone ? 1 : 0)), more = c.row * (float)row_tiles;
+        const float us = c.fixed + (rounds * (c.all + more) + (alone ? c.one + 0.6f * more : 0.f)) * (float)K * (1.0f / 1024.0f);
+        if (best < 0 || us < time) {
+            best = c.shape;
+            time = us;
+        }
+    }
+    return best;
+}
+
 static int launch_wide_shape(int shape, WideArgs& args, bool out_float, bool gated, hipStream_t stream) {
     switch (shape) {
         case 0: return launch_wide<2, 2, 2, 1, 6, 4, 1, 1, 2>(args, out_float, gated, stream);
@@ -1241,6 +1273,11 @@ static int launch_wide_shape(int shape, WideArgs& args, bool out_float, bool gat
         case 7: return launch_wide<4, 2, 4, 4, 3>(args, out_float, gated, stream);
         case 8: return launch_wide<4, 2, 4, 6, 2>(args, out_float, gated, stream);
         case 9: return launch_wide<2, 4, 8, 4, 2>(args, out_float, gated, stream);
+        case 10: return launch_wide<2, 1, 2, 1, 12>(args, out_float, gated, stream);
+        case 11: return launch_wide<2, 2, 2, 3, 7, 4, 1, 1, 6>(args, out_float, gated, stream);
+        case 12: return launch_wide<2, 1, 1, 1, 20>(args, out_float, gated, stream);
+        case 13: return launch_wide<2, 1, 1, 2, 15>(args, out_float, gated, stream);
+        case 14: return launch_wide<2, 2, 1, 2, 12>(args, out_float, gated, stream);
         default: return -1;
     }
 }
@@ -1265,6 +1302,21 @@ static int wide_shape_for(int M, int N, int K, bool gated, float* time) {
     return best;
 }
 
+// Whether 17 to 64 rows are the many-row kernel's, instead of the skinny kernels' (which take 64 rows up to k = 1024, 32 up to 2048)
+// and of the vendor library's beyond.  Its turns of 64 k wait for a barrier each, 0.14 to 0.2 us, so it loses where few workgroups
+// walk a long k and nothing else is under way: beside the library at k above 2048, or with more than 32 rows above 1024, plain
+// products need columns enough (4096 x 1024: 8.2 us for the library, 10.2 here; 4096 x 2112 10.9, 10.3), and beyond k = 4096 it is
+// behind (64 x 4096 x 12288: 34.8 for 40.4).  221 products that this takes: 0.75 of the former time (geometric mean, 0.43 to
+// 1.06): 24 x 6144 x 1024 8.0 -> 5.5 us, 32 x 6144 x 2048 16.1 -> 8.7, 64 x 6144 x 2048 13.2 -> 10.2, with gate and silu
+// 64 x 2 * 3072 x 1024 11.5 -> 6.4, 64 x 2 * 5632 x 2048 18.2 -> 14.3, 64 x 2 * 12288 x 4096 46.5 -> 40.6 (the library's product
+// and its activation's launch before).  Above 34000 rows of weight the library streams it faster (64 x 2 * 25600 x 5120: 108, 121).
+static bool few_wins(int M, int N, int K, bool gated) {
+    if (M <= 16 || M > 64 || K > 4096 || (long long)N * (gated ? 2 : 1) > 34000) return false;
+    if (K <= 1024 || (M <= 32 && K <= 2048)) return true;
+    if (K <= 2816) return gated || N > 1024;
+    return gated ? N > 1024 && N <= 12288 : N >= 6144;
+}
+
 // Whether the kernel takes these operands at all: whole blocks of k, 32-bit offsets, rows that start on 16 bytes.
 static bool wide_takes(const void* a, const void* w, int M, int N, int K, bool gated) {
     return K % WIDE_BK == 0 && (unsigned long long)M * K < (1ull << 31) && (unsigned long long)N * (gated ? 2 : 1) * K < (1ull << 31) &&
@@ -1278,10 +1330,11 @@ static int run_wide(int shape, const void* a, const void* w, void* out, int M, i
     const uintptr_t row_bytes = (uintptr_t)N * (out_float ? 4 : 2);
     args.vector_out = ((reinterpret_cast<uintptr_t>(out) | row_bytes) & 15) == 0 ? 1 : 0;
     float time = 0.f;
-    return launch_wide_shape(shape < 0 ? wide_shape_for(M, N, K, gated, &time) : shape, args, out_float, gated, stream);
+    if (shape < 0) shape = M <= 64 ? few_shape_for(M, N, K, gated) : wide_shape_for(M, N, K, gated, &time);
+    return launch_wide_shape(shape, args, out_float, gated, stream);
 }
 
-// For tests and measurements: the kernel in a given shape (0 .. WIDE_SHAPES - 1; -1: the shape that `mlr_gemm` would take),
+// For tests and measurements: the kernel in a given shape (0 .. 14; -1: the shape that `mlr_gemm` would take),
 // plain or with gate and silu.
 extern "C" int mlr_gemm_wide(const void* a, const void* w, void* out, int M, int N, int K, int out_float,
                              int shape, int gated, hipStream_t stream) {
@@ -1317,15 +1370,16 @@ extern "C" int mlr_gemm_heads(const void* a, long lda, long a_head, const void* 
     return (int)hipGetLastError();
 }
 
-// Whether more than 64 rows are this kernel's beside the vendor library (act: WIDE_*).  The library has the faster way on large
-// products (60 GFLOP and more) on which this kernel's tiles do not come out evenly: below a predicted 1.2 PFLOP/s.  (154
-// products of 97 to 2048 rows: 12 % less time than the library alone, geometric mean, where the better of both would be 14 %;
-// 0.53 to 1.18 of the library's time on the products that this takes.  2048 x 5120 x 25600: 525 us for the library's 427;
-// 1533 x 5120 x 25600: 345 for 513.)  An activation that would otherwise be a launch of its own, which reads the products and
-// writes its results at 4.5 TB/s, counts for the kernel.
+// Whether 17 rows and more are this kernel's beside the vendor library (act: WIDE_*): up to 64 rows as `few_wins` says.  Beyond, the
+// library has the faster way on large products (60 GFLOP and more) on which this kernel's tiles do not come out evenly: below a
+// predicted 1.2 PFLOP/s.  (154 products of 97 to 2048 rows: 12 % less time than the library alone, geometric mean, where the better
+// of both would be 14 %; 0.53 to 1.18 of the library's time on the products that this takes.  2048 x 5120 x 25600: 525 us for the
+// library's 427; 1533 x 5120 x 25600: 345 for 513.)  An activation that would otherwise be a launch of its own, which reads the
+// products and writes its results at 4.5 TB/s, counts for the kernel.
 extern "C" int mlr_gemm_wide_wins(int M, int N, int K, int act) {
     const bool gated = act >= WIDE_SILU && act <= WIDE_CLAMPED;
-    if (M <= 64 || N <= 0 || K <= 0 || !wide_takes(nullptr, nullptr, M, N, K, gated)) return 0;
+    if (M <= 16 || N <= 0 || K <= 0 || !wide_takes(nullptr, nullptr, M, N, K, gated)) return 0;
+    if (M <= 64) return few_wins(M, N, K, gated) ? 1 : 0;
     float time = 0.f;
     wide_shape_for(M, N, K, gated, &time);
     const float gflop = 2e-9f * (float)M * (float)N * (float)K * (gated ? 2.f : 1.f);
@@ -1364,6 +1418,8 @@ extern "C" int mlr_gemm(const void* a, const void* w, void* out, int M, int N, i
     if (K <= 0) return -1;
     if (M <= 16) return launch_skinny<1, false>(a, w, out, M, N, K, out_float, stream);
     // 17..64 rows against many columns (the output projection): tiles through LDS re-read the rows less often
+    if (!out_float && few_wins(M, N, K, false) && wide_takes(a, w, M, N, K, false))
+        return run_wide(-1, a, w, out, M, N, K, false, WIDE_PLAIN, 0.f, 0.f, stream);
     if (M <= 64 && N >= 16384) return launch<2, 2, 2, 2>(a, w, out, M, N, K, out_float, stream);
     if (M <= 32) return launch_skinny<2, false>(a, w, out, M, N, K, out_float, stream);
     if (M <= 64) return launch_skinny<4, false>(a, w, out, M, N, K, out_float, stream);
@@ -1380,6 +1436,7 @@ extern "C" int mlr_gemm_gated_silu(const void* a, const void* w, void* out, int 
     if (M <= 0 || N <= 0) return 0;
     if (K <= 0) return -1;
     if (M <= 16) return launch_skinny<1, true>(a, w, out, M, N, K, 0, stream);
+    if (few_wins(M, N, K, true) && wide_takes(a, w, M, N, K, true)) return run_wide(-1, a, w, out, M, N, K, false, WIDE_SILU, 0.f, 0.f, stream);
     if (M <= 32) return launch_skinny<2, true>(a, w, out, M, N, K, 0, stream);
     if (M <= 64) return launch_skinny<4, true>(a, w, out, M, N, K, 0, stream);
     if (wide_takes(a, w, M, N, K, true)) return run_wide(-1, a, w, out, M, N, K, false, WIDE_SILU, 0.f, 0.f, stream);

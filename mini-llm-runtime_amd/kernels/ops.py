@@ -378,16 +378,16 @@ class Kernels:
         return rows <= LIBRARY_GEMM_MIN_ROWS or (rows <= 64 and k * ((rows + 15) // 16) <= 4096)
 
     def wide_product(self, rows, columns, k, act=None):
-        """Whether the kernel for many rows (more than 64) takes a product of these sizes and not the vendor library;
+        """Whether the kernel for many rows (from 17 on) takes a product of these sizes and not the vendor library;
         `act`: with that activation in its epilogue, of `columns` gates beside as many ups or of the product itself."""
-        if self.dtype != torch.bfloat16 or rows <= 64:
+        if self.dtype != torch.bfloat16 or rows <= LIBRARY_GEMM_MIN_ROWS:
             return False
         key = (rows, columns, k, act)
         wins = self._wide_choices.get(key)
         if wins is None:
             kind = self.WIDE_ACTS[act]
             wins = bool(self._lib("gemm").mlr_gemm_wide_wins(_c_int(rows), _c_int(columns), _c_int(k), _c_int(kind)))
-            if not self.library_gemm:
+            if not self.library_gemm and rows > 64:
                 weight_rows = columns * (2 if 1 <= kind <= 5 else 1)
                 wins = k % 64 == 0 and rows * k < 2 ** 31 and weight_rows * k < 2 ** 31
             if len(self._wide_choices) >= WIDE_CHOICES_KEPT:

@@ -331,6 +331,41 @@ def test_gemm_wide_every_shape(shape, gated, mnk):
     assert torch.equal(out, run(-1, torch.bfloat16))
 
 
+@pytest.mark.parametrize("mnk", [(17, 40, 64), (31, 257, 1216), (32, 1041, 1280), (33, 96, 1344), (48, 704, 1024), (63, 1127, 2048), (64, 1152, 2816)])
+def test_gemm_few_rows_narrow_tiles(mnk):
+    """17 to 64 rows on the narrow tiles, from fewer blocks of k than the LDS holds (20 at most) to several rounds of it: the bits
+    of the many-row kernel's other tiles from each of them, from the entry points that choose among them, and with an activation;
+    no gated form of strips of 16 columns."""
+    from mini_llm_runtime_amd.kernels.ops import _c_int, _p, _stream
+    m, n, kk = mnk
+    k = kernels(torch.bfloat16)
+    lib = k._lib("gemm")
+    a = rnd((m, kk), torch.bfloat16, 68)
+    w = rnd((2 * n, kk), torch.bfloat16, 69, 0.3)
+
+    def run(shape, gated=0):
+        out = torch.full((m, n if gated else 2 * n), float("nan"), dtype=torch.bfloat16, device="cuda")
+        rc = lib.mlr_gemm_wide(_p(a), _p(w), _p(out), _c_int(m), _c_int(out.shape[1]), _c_int(kk), _c_int(0), _c_int(shape), _c_int(gated), _stream())
+        assert rc == (-1 if gated and shape in (10, 12) else 0)
+        return out
+    product, silu = run(0), run(0, 1)
+    want = a.double() @ w.double().T
+    # (kk roundings of 2^-24 of the sum of the sizes, and bfloat16's 2^-9)
+    assert bool(((product.double() - want).abs() <= kk * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T) + 2.0 ** -8 * want.abs()).all())
+    for shape in (10, 11, 12, 13, 14, -1):
+        assert torch.equal(run(shape), product), shape
+        assert shape in (10, 12) or torch.equal(run(shape, 1), silu), shape
+    out, two, one = torch.empty_like(product), torch.empty_like(silu), torch.empty_like(silu)
+    if kk <= 2816 and (n > 512 or kk <= 1024):
+        k.gemm(a, w, out, library=False)
+        assert torch.equal(out, product)
+        k.gemm_gated_silu(a, w, two)
+        assert torch.equal(two, silu)
+    k.silu_mul(product, two)
+    k.gemm_activated(a, w, one, "silu")
+    assert torch.equal(one, two)
+
+
 @pytest.mark.parametrize("mnk", [(1, 8, 64), (65, 36, 128), (97, 193, 320), (257, 385, 448), (300, 1001, 832), (513, 520, 1024)])
 def test_gemm_wide_tiles_and_epilogues(mnk):
     """Every tile of the many-row kernel at sizes around its edges, from fewer blocks of k than the LDS holds to several
