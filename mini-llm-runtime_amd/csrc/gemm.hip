@@ -942,7 +942,9 @@ struct WideArgs {
 
 // HEADS: head h multiplies its columns of wider rows by a weight of its own, out[m][h] = a[m][h] . w[h]^T; the tiles are counted
 // head by head.
-template <int WM, int WN, int TM, int TN, int NS, bool OUT_FLOAT, bool GATED, bool HEADS = false>
+// PAIRED: a turn is two blocks, and its operands are in registers before it begins: a small tile has few products a block, and
+// what its turns cost is the wait for the LDS and for the other wavefronts.
+template <int WM, int WN, int TM, int TN, int NS, bool OUT_FLOAT, bool GATED, bool HEADS = false, bool PAIRED = false>
 __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const WideArgs args) {
     using S = WideShape<WM, WN, TM, TN, NS>;
     constexpr int BM = S::BM, BN = S::BN, LOADS = S::LOADS;
@@ -1050,7 +1052,94 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const WideAr
     };
 
     const int blocks = K / WIDE_BK;
-    if (blocks >= NS) {
+    if constexpr (PAIRED) {
+        constexpr int PAIRS = NS / 2, LOADS_PAIR = 2 * LOADS;
+        static_assert(NS % 2 == 0 && PAIRS >= 2, "whole pairs of blocks");
+        bf16x8 pw[2][4][TN], pa[2][4][TM];                        // two sets of a pair's four halves
+        // (an odd count's last pair holds its last block twice and multiplies it once)
+        auto load_pair = [&](int turn, int pair) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int i = 0; i < LOADS; ++i) load(i, min(2 * turn + h, blocks - 1), 2 * pair + h);
+        };
+        auto read_pair = [&](auto set_, int pair) {
+            constexpr int set = decltype(set_)::value;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const __bf16* base = wide_lds + (2 * pair + q / 2) * S::STAGE + li * WIDE_BK + place[q & 1];
+#pragma unroll
+                for (int j = 0; j < TN; ++j) pw[set][q][j] = *reinterpret_cast<const bf16x8*>(base + (wn * TN + j) * 16 * WIDE_BK);
+#pragma unroll
+                for (int i = 0; i < TM; ++i) pa[set][q][i] = *reinterpret_cast<const bf16x8*>(base + (BN + (wm * TM + i) * 16) * WIDE_BK);
+            }
+        };
+        auto multiply = [&](auto set_, int halves) {
+            constexpr int set = decltype(set_)::value;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if (q == 2 && halves == 2) break;
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pw[set][q][j], pa[set][q][i], acc[i][j], 0, 0, 0);
+            }
+        };
+        const int turns = (blocks + 1) / 2, last = blocks % 2 ? 2 : 4;
+        if (turns >= PAIRS) {
+#pragma unroll
+            for (int t = 0; t < PAIRS; ++t) load_pair(t, t);
+            wide_arrive<LOADS_PAIR * (PAIRS - 1)>();
+            read_pair(H0, 0);
+            int pair = 0;
+            // A turn: behind the barrier everyone has read its pair, which is filled again, and the next one is there: it is
+            // read into the other set while this one is multiplied.
+            auto turn = [&](auto set_, int t) {
+                constexpr int set = decltype(set_)::value;
+                const int next = pair + 1 == PAIRS ? 0 : pair + 1;
+                wide_arrive<LOADS_PAIR * (PAIRS - 2)>();
+                read_pair(std::integral_constant<int, set ^ 1>{}, next);
+                load_pair(t + PAIRS, pair);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(set_, 4);
+                pair = next;
+            };
+            auto tail = [&](auto self, auto set_, auto left_) {   // the last PAIRS turns: nothing more to ask for
+                constexpr int set = decltype(set_)::value, LEFT = decltype(left_)::value;
+                if constexpr (LEFT > 1) {
+                    const int next = pair + 1 == PAIRS ? 0 : pair + 1;
+                    wide_arrive<LOADS_PAIR * (LEFT > 1 ? LEFT - 2 : 0)>();
+                    read_pair(std::integral_constant<int, set ^ 1>{}, next);
+                    __builtin_amdgcn_sched_barrier(0);
+                    multiply(set_, 4);
+                    pair = next;
+                    self(self, std::integral_constant<int, set ^ 1>{}, std::integral_constant<int, LEFT - 1>{});
+                } else {
+                    multiply(set_, last);
+                }
+            };
+            int t = 0;
+#pragma unroll 1
+            for (; t + 1 < turns - PAIRS; t += 2) {
+                turn(H0, t);
+                turn(H1, t + 1);
+            }
+            constexpr std::integral_constant<int, PAIRS> ALL{};
+            if (t < turns - PAIRS) {
+                turn(H0, t);
+                tail(tail, H1, ALL);
+            } else {
+                tail(tail, H0, ALL);
+            }
+        } else {                                                  // fewer pairs than the LDS holds: all at once
+            for (int t = 0; t < turns; ++t) load_pair(t, t);
+            wide_arrive<0>();
+            for (int t = 0; t < turns; ++t) {
+                read_pair(H0, t);
+                multiply(H0, t + 1 < turns ? 4 : last);
+            }
+        }
+    } else if (blocks >= NS) {
 #pragma unroll
         for (int s = 0; s < NS; ++s)
 #pragma unroll
@@ -1195,14 +1284,14 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const WideAr
     }
 }
 
-template <int WM, int WN, int TM, int TN, int NS, bool OUT_FLOAT, bool GATED>
+template <int WM, int WN, int TM, int TN, int NS, bool OUT_FLOAT, bool GATED, bool PAIRED = false>
 static int launch_wide_as(WideArgs& args, hipStream_t stream) {
     using S = WideShape<WM, WN, TM, TN, NS>;
     constexpr int NOUT = GATED ? S::BN / 2 : S::BN;
     args.tiles_m = (args.M + S::BM - 1) / S::BM;
     args.tiles_n = (args.N + NOUT - 1) / NOUT;
     if ((long long)args.tiles_m * args.tiles_n > 0x7fffffffLL / 8) return -2;
-    auto* kernel = gemm_wide_kernel<WM, WN, TM, TN, NS, OUT_FLOAT, GATED>;
+    auto* kernel = gemm_wide_kernel<WM, WN, TM, TN, NS, OUT_FLOAT, GATED, false, PAIRED>;
     static const hipError_t allowed = hipFuncSetAttribute(
         reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds_bytes);
     if (allowed != hipSuccess) return (int)allowed;
@@ -1233,15 +1322,17 @@ static const WideCost WIDE_COSTS[WIDE_SHAPES] = {
     {256, 192, 1, -2.2f, 0.f, 19.4f},  {256, 256, 1, -1.1f, 0.f, 21.8f}};
 
 
-// The same for 17 to 64 rows, where a workgroup reads its weight once and what counts is the bytes of weight under way: narrow tiles
-// with up to 19 blocks on their way.  `row`: what 16 more rows add to a round.  Fitted to 240 products of 17, 24, 32, 40, 48 and 64
-// rows, inner sizes of 1024 to 5632 and 512 to 33792 rows of weight, weights cold (rms 10 to 20 % a shape; the predicted shape is
-// then 2 % behind the best one on average).  Strips of 16 columns have no gated form.
+// The same for 17 to 64 rows, where a workgroup reads its weight once and what counts is the bytes of weight under way and what a
+// turn waits: narrow tiles with up to 19 blocks on their way, two of them a turn.  `row`: what 16 more rows add to a round.  Fitted to
+// 200 products of 17, 32, 40 and 64 rows, inner sizes of 1024 to 8192 and 512 to 51200 rows of weight, weights cold (the predicted
+// tile is 1 % behind the best one on average).  Strips of 16 columns have no gated form.  With one block a turn, a turn of the tiles
+// of 32 x 16 to 64 x 16 took 0.14 to 0.2 us: 32 x 4096 x 1024 5.2 -> 4.7 us, 32 x 2112 x 4096 10.3 -> 9.3, 17 x 2 * 704 x 2048 6.8 ->
+// 5.1; tiles of 64 x 32 and 64 x 64, which two workgroups of a compute unit share, gain nothing by it.
 struct FewCost { int shape, bm, bn, per_unit; float fixed, one, all, row; };
 static const FewCost FEW_COSTS[] = {
-    {0, 64, 32, 2, 2.0f, 2.0f, 5.5f, 0.62f},  {1, 64, 64, 2, 1.8f, 3.1f, 9.7f, 0.73f}, {10, 64, 16, 1, 1.7f, 0.f, 2.3f, 0.18f},
-    {11, 64, 96, 1, 2.2f, 0.f, 4.2f, 0.51f},  {12, 32, 16, 1, 2.05f, 0.f, 2.23f, 0.f}, {13, 32, 32, 1, 1.35f, 0.f, 3.1f, 0.f},
-    {14, 32, 64, 1, 1.2f, 0.f, 4.3f, 0.f}};
+    {0, 64, 32, 2, 1.94f, 2.07f, 5.72f, 0.59f}, {1, 64, 64, 2, 1.87f, 3.1f, 10.4f, 0.67f}, {10, 64, 16, 1, 1.38f, 0.f, 1.76f, 0.28f},
+    {11, 64, 96, 1, 2.15f, 0.f, 4.17f, 0.48f},  {12, 32, 16, 1, 2.1f, 0.f, 1.81f, 0.f},    {13, 32, 32, 1, 0.83f, 0.f, 3.04f, 0.f},
+    {14, 32, 64, 1, 0.97f, 0.f, 4.1f, 0.f}};
 
 static int few_shape_for(int M, int N, int K, bool gated) {
     const int units = compute_units() > 0 ? compute_units() : 256, row_tiles = (M + 15) / 16;
@@ -1261,6 +1352,16 @@ static int few_shape_for(int M, int N, int K, bool gated) {
     return best;
 }
 
+// The tiles for up to 64 rows, two blocks a turn (never with 32-bit results: those are the library's).
+template <int WM, int WN, int TM, int TN, int NS, int GWM = WM, int GWN = WN, int GTM = TM, int GTN = TN>
+static int launch_paired(WideArgs& args, bool out_float, bool gated, hipStream_t stream) {
+    static_assert(WM * TM == GWM * GTM && WN * TN == GWN * GTN, "one tile for both forms");
+    if (out_float) return -1;
+    if (!gated) return launch_wide_as<WM, WN, TM, TN, NS, false, false, true>(args, stream);
+    if constexpr (GTN % 2 == 0) return launch_wide_as<GWM, GWN, GTM, GTN, NS, false, true, true>(args, stream);
+    return -1;
+}
+
 static int launch_wide_shape(int shape, WideArgs& args, bool out_float, bool gated, hipStream_t stream) {
     switch (shape) {
         case 0: return launch_wide<2, 2, 2, 1, 6, 4, 1, 1, 2>(args, out_float, gated, stream);
@@ -1273,11 +1374,11 @@ static int launch_wide_shape(int shape, WideArgs& args, bool out_float, bool gat
         case 7: return launch_wide<4, 2, 4, 4, 3>(args, out_float, gated, stream);
         case 8: return launch_wide<4, 2, 4, 6, 2>(args, out_float, gated, stream);
         case 9: return launch_wide<2, 4, 8, 4, 2>(args, out_float, gated, stream);
-        case 10: return launch_wide<2, 1, 2, 1, 12>(args, out_float, gated, stream);
+        case 10: return launch_paired<2, 1, 2, 1, 12>(args, out_float, gated, stream);
         case 11: return launch_wide<2, 2, 2, 3, 7, 4, 1, 1, 6>(args, out_float, gated, stream);
-        case 12: return launch_wide<2, 1, 1, 1, 20>(args, out_float, gated, stream);
-        case 13: return launch_wide<2, 1, 1, 2, 15>(args, out_float, gated, stream);
-        case 14: return launch_wide<2, 2, 1, 2, 12>(args, out_float, gated, stream);
+        case 12: return launch_paired<2, 1, 1, 1, 20>(args, out_float, gated, stream);
+        case 13: return launch_paired<2, 1, 1, 2, 14>(args, out_float, gated, stream);
+        case 14: return launch_paired<2, 2, 1, 2, 12>(args, out_float, gated, stream);
         default: return -1;
     }
 }
@@ -1303,18 +1404,20 @@ static int wide_shape_for(int M, int N, int K, bool gated, float* time) {
 }
 
 // Whether 17 to 64 rows are the many-row kernel's, instead of the skinny kernels' (which take 64 rows up to k = 1024, 32 up to 2048)
-// and of the vendor library's beyond.  Its turns of 64 k wait for a barrier each, 0.14 to 0.2 us, so it loses where few workgroups
-// walk a long k and nothing else is under way: beside the library at k above 2048, or with more than 32 rows above 1024, plain
-// products need columns enough (4096 x 1024: 8.2 us for the library, 10.2 here; 4096 x 2112 10.9, 10.3), and beyond k = 4096 it is
-// behind (64 x 4096 x 12288: 34.8 for 40.4).  221 products that this takes: 0.75 of the former time (geometric mean, 0.43 to
-// 1.06): 24 x 6144 x 1024 8.0 -> 5.5 us, 32 x 6144 x 2048 16.1 -> 8.7, 64 x 6144 x 2048 13.2 -> 10.2, with gate and silu
+// and of the vendor library's beyond.  It loses where few workgroups walk a long k -- a turn of 128 k waits for a barrier, 0.14 us
+// and more -- and where the activation's rows, which every strip of columns reads again, outweigh its weight: 1024 columns at
+// k = 4096 (8.0 us of the library for 8.7, 64 rows 9.8 for 12.4), 64 x 4096 x 12288 (34.7 for 40.1), 64 x 2048 x 5632 (13.4 for
+// 18.2); up to 32 rows it holds on to k = 8192 (32 x 4096 x 5632 17.5 -> 15.8, 32 x 5120 x 8192 26.9 -> 26.0).
+// Against those: 24 x 6144 x 1024 8.0 -> 5.5 us, 32 x 6144 x 2048 16.1 -> 8.4, 64 x 6144 x 2048 13.2 -> 10.2, with gate and silu
 // 64 x 2 * 3072 x 1024 11.5 -> 6.4, 64 x 2 * 5632 x 2048 18.2 -> 14.3, 64 x 2 * 12288 x 4096 46.5 -> 40.6 (the library's product
-// and its activation's launch before).  Above 34000 rows of weight the library streams it faster (64 x 2 * 25600 x 5120: 108, 121).
+// and its activation's launch before); over 250 products 0.73 of the time (geometric mean, 0.43 to 1.06).  Above 34000 rows of
+// weight the library streams it faster (64 x 2 * 25600 x 5120: 106, 121).
 static bool few_wins(int M, int N, int K, bool gated) {
-    if (M <= 16 || M > 64 || K > 4096 || (long long)N * (gated ? 2 : 1) > 34000) return false;
-    if (K <= 1024 || (M <= 32 && K <= 2048)) return true;
-    if (K <= 2816) return gated || N > 1024;
-    return gated ? N > 1024 && N <= 12288 : N >= 6144;
+    const long long weight = (long long)N * (gated ? 2 : 1);
+    if (M <= 16 || M > 64 || weight > 34000) return false;
+    if (M <= 32) return K <= 2816 || (N > 1024 && (K <= 4096 || (K <= 8192 && weight <= 8192)));
+    if (K <= 2816) return K <= 2048 || gated || N > 1024;
+    return K <= 4096 && (gated ? N > 1024 && N <= 12288 : N >= 4096);
 }
 
 // Whether the kernel takes these operands at all: whole blocks of k, 32-bit offsets, rows that start on 16 bytes.
@@ -1330,7 +1433,7 @@ static int run_wide(int shape, const void* a, const void* w, void* out, int M, i
     const uintptr_t row_bytes = (uintptr_t)N * (out_float ? 4 : 2);
     args.vector_out = ((reinterpret_cast<uintptr_t>(out) | row_bytes) & 15) == 0 ? 1 : 0;
     float time = 0.f;
-    if (shape < 0) shape = M <= 64 ? few_shape_for(M, N, K, gated) : wide_shape_for(M, N, K, gated, &time);
+    if (shape < 0) shape = M <= 64 && !out_float ? few_shape_for(M, N, K, gated) : wide_shape_for(M, N, K, gated, &time);
     return launch_wide_shape(shape, args, out_float, gated, stream);
 }
 
