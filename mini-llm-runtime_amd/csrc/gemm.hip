@@ -1437,8 +1437,8 @@ static int run_wide(int shape, const void* a, const void* w, void* out, int M, i
     return launch_wide_shape(shape, args, out_float, gated, stream);
 }
 
-// For tests and measurements: the kernel in a given shape (0 .. 14; -1: the shape that `mlr_gemm` would take),
-// plain or with gate and silu.
+// The kernel in a given shape (0 .. 14, for tests and measurements) or, -1, in the one with the least predicted time, plain or with
+// gate and silu.
 extern "C" int mlr_gemm_wide(const void* a, const void* w, void* out, int M, int N, int K, int out_float,
                              int shape, int gated, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
@@ -1521,8 +1521,6 @@ extern "C" int mlr_gemm(const void* a, const void* w, void* out, int M, int N, i
     if (K <= 0) return -1;
     if (M <= 16) return launch_skinny<1, false>(a, w, out, M, N, K, out_float, stream);
     // 17..64 rows against many columns (the output projection): tiles through LDS re-read the rows less often
-    if (!out_float && few_wins(M, N, K, false) && wide_takes(a, w, M, N, K, false))
-        return run_wide(-1, a, w, out, M, N, K, false, WIDE_PLAIN, 0.f, 0.f, stream);
     if (M <= 64 && N >= 16384) return launch<2, 2, 2, 2>(a, w, out, M, N, K, out_float, stream);
     if (M <= 32) return launch_skinny<2, false>(a, w, out, M, N, K, out_float, stream);
     if (M <= 64) return launch_skinny<4, false>(a, w, out, M, N, K, out_float, stream);
@@ -1539,7 +1537,6 @@ extern "C" int mlr_gemm_gated_silu(const void* a, const void* w, void* out, int 
     if (M <= 0 || N <= 0) return 0;
     if (K <= 0) return -1;
     if (M <= 16) return launch_skinny<1, true>(a, w, out, M, N, K, 0, stream);
-    if (few_wins(M, N, K, true) && wide_takes(a, w, M, N, K, true)) return run_wide(-1, a, w, out, M, N, K, false, WIDE_SILU, 0.f, 0.f, stream);
     if (M <= 32) return launch_skinny<2, true>(a, w, out, M, N, K, 0, stream);
     if (M <= 64) return launch_skinny<4, true>(a, w, out, M, N, K, 0, stream);
     if (wide_takes(a, w, M, N, K, true)) return run_wide(-1, a, w, out, M, N, K, false, WIDE_SILU, 0.f, 0.f, stream);

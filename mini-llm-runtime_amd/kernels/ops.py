@@ -136,6 +136,8 @@ def _tensors_work(*names):
 
 
 class Kernels:
+    routed = False                          # the model chooses among experts: sums keep their order (`wide_product`)
+
     def __init__(self, dtype, library_gemm=True):
         _need(dtype in (torch.float32, torch.bfloat16), f"no kernels for element type {dtype}")
         if not torch.cuda.is_available():
@@ -343,6 +345,10 @@ class Kernels:
         _need(k == k2, lambda: f"gemm: inner sizes differ ({k} and {k2})")
         _need(out.dtype in (self.dtype, torch.float32), lambda: f"gemm: output type {out.dtype} not supported")
         _tensor(out, "out", out.dtype, (m, n))
+        if m <= 64 and out.dtype == torch.bfloat16 and self.wide_product(m, n, k) and _on16(a, w):
+            _ok(self._lib("gemm").mlr_gemm_wide(_p(a), _p(w), _p(out), _c_int(m), _c_int(n), _c_int(k), _c_int(0), _c_int(-1), _c_int(0),
+                                                _stream()), "gemm")
+            return
         if library and self.library_gemm and self.dtype == torch.bfloat16 and m > LIBRARY_GEMM_MIN_ROWS and \
                 (out.dtype == torch.float32 or not (self.streams_weight(m, k) or (self.wide_product(m, n, k) and _on16(a, w)))):
             # a plain matrix product, handed to the vendor library (hipBLASLt), as the reference hands its projections to
@@ -381,6 +387,11 @@ class Kernels:
         """Whether the kernel for many rows (from 17 on) takes a product of these sizes and not the vendor library;
         `act`: with that activation in its epilogue, of `columns` gates beside as many ups or of the product itself."""
         if self.dtype != torch.bfloat16 or rows <= LIBRARY_GEMM_MIN_ROWS:
+            return False
+        # A choice among experts turns on the last bit.  The library adds in this kernel's order, bit by bit, but where it cuts k
+        # into parts: few outputs or a long k (of 8 row counts and 21 sizes, compared: none of at least 2^19 outputs with k up to
+        # 8448 differs; 333 x 768 x 2048, every 64 x n x 2048 of few columns, 1777 x 4096 x 18432 do, in one output of 2000).
+        if self.routed and (rows <= 64 or (self.library_gemm and (rows * columns < 1 << 19 or k > 8448))):
             return False
         key = (rows, columns, k, act)
         wins = self._wide_choices.get(key)
@@ -450,6 +461,10 @@ class Kernels:
         _tensor(out, "out", self.dtype, (m, two_n // 2))
         if m > 64 or strips:
             a, w = _start16(a), _start16(w)
+        if m <= 64 and self.wide_product(m, two_n // 2, k, "silu") and _on16(a, w):
+            _ok(self._lib("gemm").mlr_gemm_wide(_p(a), _p(w), _p(out), _c_int(m), _c_int(two_n // 2), _c_int(k), _c_int(0), _c_int(-1),
+                                                _c_int(1), _stream()), "gemm_gated_silu")
+            return
         fn = self._lib("gemm").mlr_gemm_gated_silu
         _ok(fn(_p(a), _p(w), _p(out), _c_int(m), _c_int(two_n // 2), _c_int(k), _stream()), "gemm_gated_silu")
 

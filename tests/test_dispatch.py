@@ -231,3 +231,16 @@ def test_key_ranges_of_one_width_whatever_the_batch():
     ctx = context_with_budget(300000, None)
     keys, splits, chunk, _ = ctx.fixed_split(3, 16, 128)
     assert keys == 512 and splits == -(-300000 // 512) <= MAX_KEY_SPLITS and chunk == 3
+
+
+@pytest.mark.parametrize("sizes", [(17, 6144, 2048), (64, 12288, 1024), (333, 768, 2048), (1777, 4096, 18432)])
+def test_products_of_a_model_with_a_router_keep_the_order_of_their_sums(sizes):
+    """Where the vendor library may add in another order than the many-row kernel, a model that chooses among experts stays with
+    it (asked without a GPU: the answer must not need the kernels' library); other models ask the kernels' own rule."""
+    k = kernels_without_gpu()
+    k._wide_choices = {sizes + (None,): True, sizes + ("silu",): True}
+    assert k.wide_product(*sizes) and k.wide_product(*sizes, "silu")
+    k.routed = True
+    assert not k.wide_product(*sizes) and not k.wide_product(*sizes, "silu")
+    k._wide_choices[(1777, 6144, 4096, None)] = True
+    assert k.wide_product(1777, 6144, 4096)
