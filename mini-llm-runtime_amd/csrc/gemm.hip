@@ -7,7 +7,8 @@
 // does not depend on the rows beside it): up to 16 rows, and to 64 where `few_wins` does not say otherwise, the weight is
 // streamed once straight into v_mfma_f32_16x16x32_bf16 (`gemm_skinny_kernel`, optionally with the residual add and RMSNorm in
 // front or silu(gate) * up behind); more rows with k a multiple of 64 go to `gemm_wide_kernel` (tiles out of
-// blocks of LDS that loads fill without passing through registers); any other k to the plain 16x16-tile kernel `gemm_bf16_kernel`.
+// blocks of LDS that loads fill without passing through registers), and so do the rows that `few_wins` names, in a form with the
+// first kernel's order; any other k to the plain 16x16-tile kernel `gemm_bf16_kernel`.
 #include "common.h"
 #include <type_traits>
 
@@ -907,8 +908,9 @@ static int launch_skinny(const void* a, const void* w, void* out, int M, int N, 
 //
 // A row of a block is 128 bytes, eight pieces of 16; a load writes 64 lanes' pieces side by side (eight rows), so rows cannot be
 // padded apart.  Instead piece p of row r lies at place p ^ (r & 7) -- the lane that fetches it is chosen accordingly --, and
-// the eight lanes that the LDS serves together read eight different banks.
-// Every output element is one sum over k in ascending order, 32 k an instruction, whatever M and the shape are.
+// the eight lanes that the LDS serves together read eight different banks.  (FEW: a row's even pieces first, then its odd ones.)
+// Every output element is one sum over k in ascending order, 32 k an instruction, whatever M and the shape are (the forms for 17 to
+// 64 rows: eight sums, see FEW).
 // GATED: w = [gate; up] of N rows each; a wavefront's weight tiles alternate between the two.
 #define WIDE_BK 64
 
@@ -942,13 +944,20 @@ struct WideArgs {
 
 // HEADS: head h multiplies its columns of wider rows by a weight of its own, out[m][h] = a[m][h] . w[h]^T; the tiles are counted
 // head by head.
+// FEW (17 to 64 rows): the sums of `gemm_skinny_kernel`, bit by bit, so that a row's results do not turn on whether 16 rows or 64
+// are computed with it: eight parts of k, of whole blocks, each one sum and added in ascending order, and 16 consecutive bytes of
+// every 32 of a row an instruction.  (The parts are also the more exact sum: worked out with normal operands, a
+// rounding an instruction, its rms error is 0.63, 0.54 and 0.45 of one chain's at k = 1024, 2048 and 4096.)
+// Beside one chain and a gate of hardware approximations it takes 6 % more of a product's time (108 products, geometric mean; 0.2 us
+// for closing the parts, 0.4 for a gate), and 0.69 of the time of the kernels that took these rows before.
 // PAIRED: a turn is two blocks, and its operands are in registers before it begins: a small tile has few products a block, and
 // what its turns cost is the wait for the LDS and for the other wavefronts.
-template <int WM, int WN, int TM, int TN, int NS, bool OUT_FLOAT, bool GATED, bool HEADS = false, bool PAIRED = false>
+template <int WM, int WN, int TM, int TN, int NS, bool OUT_FLOAT, bool GATED, bool HEADS = false, bool FEW = false, bool PAIRED = false>
 __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const WideArgs args) {
     using S = WideShape<WM, WN, TM, TN, NS>;
     constexpr int BM = S::BM, BN = S::BN, LOADS = S::LOADS;
     static_assert(!GATED || TN % 2 == 0, "gate and up tiles come in pairs");
+    static_assert((!PAIRED || FEW) && (!FEW || !HEADS), "forms for 17 to 64 rows");
     extern __shared__ __attribute__((aligned(16))) __bf16 wide_lds[];
     const int M = args.M, N = args.N, K = args.K;
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -978,7 +987,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const WideAr
     uint32_t src[LOADS];
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
-        const int row = (wave * LOADS + i) * 8 + (lane >> 3), piece = ((lane & 7) ^ (row & 7)) * 8;
+        const int row = (wave * LOADS + i) * 8 + (lane >> 3), at = (lane & 7) ^ (row & 7), piece = (FEW ? (at & 3) * 2 + (at >> 2) : at) * 8;
         int r;
         if (row < BN) {
             if (GATED) {
@@ -1009,6 +1018,33 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const WideAr
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const int blocks = K / WIDE_BK, part_blocks = (blocks + SKINNY_WAVES - 1) / SKINNY_WAVES;
+    floatx4 sum[FEW ? TM : 1][FEW ? TN : 1];                      // FEW: the parts of k that are done
+    int part_left = part_blocks;
+    if constexpr (FEW) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) sum[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+    auto close_part = [&]() {
+        if constexpr (FEW) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    sum[i][j] += acc[i][j];
+                    acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+                }
+        }
+    };
+    auto block_done = [&]() {
+        if (FEW && --part_left == 0) {                            // (eight times a product, the same in every lane)
+            asm volatile("");                                     // (a branch: as selects, every block's products would be waited for)
+            close_part();
+            part_left = part_blocks;
+        }
+    };
     // The operands of one half of a block (32 k); the other half's are read while these are multiplied.
     bf16x8 wf[2][TN], af[2][TM];
     const int place[2] = {(g ^ (li & 7)) * 8, ((4 + g) ^ (li & 7)) * 8};
@@ -1051,7 +1087,6 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const WideAr
         __builtin_amdgcn_s_setprio(0);
     };
 
-    const int blocks = K / WIDE_BK;
     if constexpr (PAIRED) {
         constexpr int PAIRS = NS / 2, LOADS_PAIR = 2 * LOADS;
         static_assert(NS % 2 == 0 && PAIRS >= 2, "whole pairs of blocks");
@@ -1083,6 +1118,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const WideAr
                 for (int i = 0; i < TM; ++i)
 #pragma unroll
                     for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pw[set][q][j], pa[set][q][i], acc[i][j], 0, 0, 0);
+                if (q % 2 == 1) block_done();
             }
         };
         const int turns = (blocks + 1) / 2, last = blocks % 2 ? 2 : 4;
@@ -1155,6 +1191,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const WideAr
             products(H0, std::true_type{}, stage, std::false_type{}, 0, 0);
             wide_arrive<LOADS * (NS - 2)>();
             products(H1, std::true_type{}, next, std::true_type{}, kb + NS, stage);
+            block_done();
             stage = next;
         }
         auto tail = [&](auto self, auto left_) {                  // the last NS blocks: nothing more to ask for
@@ -1168,6 +1205,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const WideAr
                 } else {
                     products(H1, std::false_type{}, 0, std::false_type{}, 0, 0);
                 }
+                block_done();
                 stage = next;
                 self(self, std::integral_constant<int, LEFT - 1>{});
             }
@@ -1183,7 +1221,15 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const WideAr
             read_all(H1, s);
             products(H0, std::false_type{}, 0, std::false_type{}, 0, 0);
             products(H1, std::false_type{}, 0, std::false_type{}, 0, 0);
+            block_done();
         }
+    }
+    if constexpr (FEW) {
+        close_part();                                             // (the last part, where it is a shorter one)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = sum[i][j];
     }
 
     if constexpr (OUT_FLOAT) {
@@ -1227,11 +1273,12 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const WideAr
                     float y[4];
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        // silu(g) = g / (1 + 2^(-g log2 e)), with the hardware's exponential and reciprocal (both good to an
-                        // ulp or so of 32 bits; the result is rounded to bfloat16): a full division costs ten instructions,
-                        // and a lane has 2 TM TN of these
-                        const float gate = acc[i0 + i][2 * j][r];
-                        y[r] = gate * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896340736f * gate)) * acc[i0 + i][(2 * j + 1) % TN][r];
+                        // silu(g) = g / (1 + 2^(-g log2 e)).  Many rows: with the hardware's exponential and reciprocal (both good
+                        // to an ulp or so of 32 bits; the result is rounded to bfloat16): a full division costs ten instructions,
+                        // and a lane has 2 TM TN of these.  Few rows have few, and what `gemm_skinny_kernel` makes of them.
+                        const float gate = acc[i0 + i][2 * j][r], up = acc[i0 + i][(2 * j + 1) % TN][r];
+                        y[r] = FEW ? gate_act<0>(gate) * up
+                                   : gate * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896340736f * gate)) * up;
                     }
                     put(i, j, y[0], y[1], y[2], y[3]);
                 }
@@ -1284,14 +1331,14 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const WideAr
     }
 }
 
-template <int WM, int WN, int TM, int TN, int NS, bool OUT_FLOAT, bool GATED, bool PAIRED = false>
+template <int WM, int WN, int TM, int TN, int NS, bool OUT_FLOAT, bool GATED, bool FEW = false, bool PAIRED = false>
 static int launch_wide_as(WideArgs& args, hipStream_t stream) {
     using S = WideShape<WM, WN, TM, TN, NS>;
     constexpr int NOUT = GATED ? S::BN / 2 : S::BN;
     args.tiles_m = (args.M + S::BM - 1) / S::BM;
     args.tiles_n = (args.N + NOUT - 1) / NOUT;
     if ((long long)args.tiles_m * args.tiles_n > 0x7fffffffLL / 8) return -2;
-    auto* kernel = gemm_wide_kernel<WM, WN, TM, TN, NS, OUT_FLOAT, GATED, false, PAIRED>;
+    auto* kernel = gemm_wide_kernel<WM, WN, TM, TN, NS, OUT_FLOAT, GATED, false, FEW, PAIRED>;
     static const hipError_t allowed = hipFuncSetAttribute(
         reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds_bytes);
     if (allowed != hipSuccess) return (int)allowed;
@@ -1330,7 +1377,7 @@ static const WideCost WIDE_COSTS[WIDE_SHAPES] = {
 // 5.1; tiles of 64 x 32 and 64 x 64, which two workgroups of a compute unit share, gain nothing by it.
 struct FewCost { int shape, bm, bn, per_unit; float fixed, one, all, row; };
 static const FewCost FEW_COSTS[] = {
-    {0, 64, 32, 2, 1.94f, 2.07f, 5.72f, 0.59f}, {1, 64, 64, 2, 1.87f, 3.1f, 10.4f, 0.67f}, {10, 64, 16, 1, 1.38f, 0.f, 1.76f, 0.28f},
+    {15, 64, 32, 2, 1.94f, 2.07f, 5.72f, 0.59f}, {16, 64, 64, 2, 1.87f, 3.1f, 10.4f, 0.67f}, {10, 64, 16, 1, 1.38f, 0.f, 1.76f, 0.28f},
     {11, 64, 96, 1, 2.15f, 0.f, 4.17f, 0.48f},  {12, 32, 16, 1, 2.1f, 0.f, 1.81f, 0.f},    {13, 32, 32, 1, 0.83f, 0.f, 3.04f, 0.f},
     {14, 32, 64, 1, 0.97f, 0.f, 4.1f, 0.f}};
 
@@ -1352,13 +1399,13 @@ static int few_shape_for(int M, int N, int K, bool gated) {
     return best;
 }
 
-// The tiles for up to 64 rows, two blocks a turn (never with 32-bit results: those are the library's).
-template <int WM, int WN, int TM, int TN, int NS, int GWM = WM, int GWN = WN, int GTM = TM, int GTN = TN>
-static int launch_paired(WideArgs& args, bool out_float, bool gated, hipStream_t stream) {
+// The tiles for up to 64 rows (never with 32-bit results: those are the library's).
+template <bool PAIRED, int WM, int WN, int TM, int TN, int NS, int GWM = WM, int GWN = WN, int GTM = TM, int GTN = TN>
+static int launch_few(WideArgs& args, bool out_float, bool gated, hipStream_t stream) {
     static_assert(WM * TM == GWM * GTM && WN * TN == GWN * GTN, "one tile for both forms");
     if (out_float) return -1;
-    if (!gated) return launch_wide_as<WM, WN, TM, TN, NS, false, false, true>(args, stream);
-    if constexpr (GTN % 2 == 0) return launch_wide_as<GWM, GWN, GTM, GTN, NS, false, true, true>(args, stream);
+    if (!gated) return launch_wide_as<WM, WN, TM, TN, NS, false, false, true, PAIRED>(args, stream);
+    if constexpr (GTN % 2 == 0) return launch_wide_as<GWM, GWN, GTM, GTN, NS, false, true, true, PAIRED>(args, stream);
     return -1;
 }
 
@@ -1374,11 +1421,13 @@ static int launch_wide_shape(int shape, WideArgs& args, bool out_float, bool gat
         case 7: return launch_wide<4, 2, 4, 4, 3>(args, out_float, gated, stream);
         case 8: return launch_wide<4, 2, 4, 6, 2>(args, out_float, gated, stream);
         case 9: return launch_wide<2, 4, 8, 4, 2>(args, out_float, gated, stream);
-        case 10: return launch_paired<2, 1, 2, 1, 12>(args, out_float, gated, stream);
-        case 11: return launch_wide<2, 2, 2, 3, 7, 4, 1, 1, 6>(args, out_float, gated, stream);
-        case 12: return launch_paired<2, 1, 1, 1, 20>(args, out_float, gated, stream);
-        case 13: return launch_paired<2, 1, 1, 2, 14>(args, out_float, gated, stream);
-        case 14: return launch_paired<2, 2, 1, 2, 12>(args, out_float, gated, stream);
+        case 10: return launch_few<true, 2, 1, 2, 1, 12>(args, out_float, gated, stream);
+        case 11: return launch_few<false, 2, 2, 2, 3, 7, 4, 1, 1, 6>(args, out_float, gated, stream);
+        case 12: return launch_few<true, 2, 1, 1, 1, 20>(args, out_float, gated, stream);
+        case 13: return launch_few<true, 2, 1, 1, 2, 14>(args, out_float, gated, stream);
+        case 14: return launch_few<true, 2, 2, 1, 2, 12>(args, out_float, gated, stream);
+        case 15: return launch_few<false, 2, 2, 2, 1, 6, 4, 1, 1, 2>(args, out_float, gated, stream);
+        case 16: return launch_few<false, 2, 2, 2, 2, 5>(args, out_float, gated, stream);
         default: return -1;
     }
 }
@@ -1426,6 +1475,7 @@ static bool wide_takes(const void* a, const void* w, int M, int N, int K, bool g
            ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(w)) & 15) == 0;
 }
 
+enum { WIDE_MANY = -1, WIDE_FEW = -2 };      // the tile with the least predicted time, of one sum over k or of the forms for 17 to 64 rows
 static int run_wide(int shape, const void* a, const void* w, void* out, int M, int N, int K, bool out_float, int act, float limit,
                     float slope, hipStream_t stream) {
     const bool gated = act >= WIDE_SILU && act <= WIDE_CLAMPED;
@@ -1433,12 +1483,13 @@ static int run_wide(int shape, const void* a, const void* w, void* out, int M, i
     const uintptr_t row_bytes = (uintptr_t)N * (out_float ? 4 : 2);
     args.vector_out = ((reinterpret_cast<uintptr_t>(out) | row_bytes) & 15) == 0 ? 1 : 0;
     float time = 0.f;
-    if (shape < 0) shape = M <= 64 && !out_float ? few_shape_for(M, N, K, gated) : wide_shape_for(M, N, K, gated, &time);
+    if (shape == WIDE_FEW) shape = few_shape_for(M, N, K, gated);             // (-1, refused below, beyond 64 rows)
+    else if (shape == WIDE_MANY) shape = wide_shape_for(M, N, K, gated, &time);
     return launch_wide_shape(shape, args, out_float, gated, stream);
 }
 
-// The kernel in a given shape (0 .. 14, for tests and measurements) or, -1, in the one with the least predicted time, plain or with
-// gate and silu.
+// The kernel in a given shape (0 .. 16, for tests and measurements) or in the one with the least predicted time (-1: of one sum over
+// k; -2: of the forms for 17 to 64 rows, whose sums are those of up to 16 rows), plain or with gate and silu.
 extern "C" int mlr_gemm_wide(const void* a, const void* w, void* out, int M, int N, int K, int out_float,
                              int shape, int gated, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
@@ -1497,7 +1548,7 @@ extern "C" int mlr_gemm_activated(const void* a, const void* w, void* out, int M
     if (M <= 0 || N <= 0) return 0;
     if (K <= 0 || act < WIDE_SILU_ROUNDED || act > WIDE_GELU_ERF || (act == WIDE_CLAMPED && !(limit > 0.f))) return -1;
     if (!wide_takes(a, w, M, N, K, act <= WIDE_CLAMPED)) return -2;
-    return run_wide(-1, a, w, out, M, N, K, false, act, limit, slope, stream);
+    return run_wide(M <= 64 ? WIDE_FEW : WIDE_MANY, a, w, out, M, N, K, false, act, limit, slope, stream);
 }
 
 template <int WM, int WN, int TM, int TN>
@@ -1524,7 +1575,7 @@ extern "C" int mlr_gemm(const void* a, const void* w, void* out, int M, int N, i
     if (M <= 64 && N >= 16384) return launch<2, 2, 2, 2>(a, w, out, M, N, K, out_float, stream);
     if (M <= 32) return launch_skinny<2, false>(a, w, out, M, N, K, out_float, stream);
     if (M <= 64) return launch_skinny<4, false>(a, w, out, M, N, K, out_float, stream);
-    if (wide_takes(a, w, M, N, K, false)) return run_wide(-1, a, w, out, M, N, K, out_float != 0, WIDE_PLAIN, 0.f, 0.f, stream);
+    if (wide_takes(a, w, M, N, K, false)) return run_wide(WIDE_MANY, a, w, out, M, N, K, out_float != 0, WIDE_PLAIN, 0.f, 0.f, stream);
     if (M <= 128) return launch<2, 2, 2, 2>(a, w, out, M, N, K, out_float, stream);  // 64 x 64
     return launch<2, 2, 4, 4>(a, w, out, M, N, K, out_float, stream);                // 128 x 128
 }
@@ -1539,7 +1590,7 @@ extern "C" int mlr_gemm_gated_silu(const void* a, const void* w, void* out, int 
     if (M <= 16) return launch_skinny<1, true>(a, w, out, M, N, K, 0, stream);
     if (M <= 32) return launch_skinny<2, true>(a, w, out, M, N, K, 0, stream);
     if (M <= 64) return launch_skinny<4, true>(a, w, out, M, N, K, 0, stream);
-    if (wide_takes(a, w, M, N, K, true)) return run_wide(-1, a, w, out, M, N, K, false, WIDE_SILU, 0.f, 0.f, stream);
+    if (wide_takes(a, w, M, N, K, true)) return run_wide(WIDE_MANY, a, w, out, M, N, K, false, WIDE_SILU, 0.f, 0.f, stream);
     return 1;
 }
 

@@ -346,7 +346,7 @@ class Kernels:
         _need(out.dtype in (self.dtype, torch.float32), lambda: f"gemm: output type {out.dtype} not supported")
         _tensor(out, "out", out.dtype, (m, n))
         if m <= 64 and out.dtype == torch.bfloat16 and self.wide_product(m, n, k) and _on16(a, w):
-            _ok(self._lib("gemm").mlr_gemm_wide(_p(a), _p(w), _p(out), _c_int(m), _c_int(n), _c_int(k), _c_int(0), _c_int(-1), _c_int(0),
+            _ok(self._lib("gemm").mlr_gemm_wide(_p(a), _p(w), _p(out), _c_int(m), _c_int(n), _c_int(k), _c_int(0), _c_int(-2), _c_int(0),
                                                 _stream()), "gemm")
             return
         if library and self.library_gemm and self.dtype == torch.bfloat16 and m > LIBRARY_GEMM_MIN_ROWS and \
@@ -462,7 +462,7 @@ class Kernels:
         if m > 64 or strips:
             a, w = _start16(a), _start16(w)
         if m <= 64 and self.wide_product(m, two_n // 2, k, "silu") and _on16(a, w):
-            _ok(self._lib("gemm").mlr_gemm_wide(_p(a), _p(w), _p(out), _c_int(m), _c_int(two_n // 2), _c_int(k), _c_int(0), _c_int(-1),
+            _ok(self._lib("gemm").mlr_gemm_wide(_p(a), _p(w), _p(out), _c_int(m), _c_int(two_n // 2), _c_int(k), _c_int(0), _c_int(-2),
                                                 _c_int(1), _stream()), "gemm_gated_silu")
             return
         fn = self._lib("gemm").mlr_gemm_gated_silu

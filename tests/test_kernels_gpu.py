@@ -185,9 +185,9 @@ def test_gemm_two_strips_a_workgroup(mnk):
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_gemm_rows_do_not_depend_on_the_batch(dtype):
     """A row's result is the same bits whatever rows stand beside it.  The float kernel has one order of
-    additions for every M; the bfloat16 engine has two kernels (up to 64 rows the weight is streamed with k
-    split over four wavefronts, above that it is tiled), each with a fixed order, so bits agree within a
-    kernel and differ by rounding across the two."""
+    additions for every M; the bfloat16 engine has two (up to 64 rows k is cut into eight parts, above that it is one
+    chain), so bits agree up to 64 rows and above, and differ by rounding across the two.  (k no multiple of 64: the next
+    test has those.)"""
     from mini_llm_runtime_amd.kernels import Kernels
     k = Kernels(dtype, library_gemm=False)
     a = rnd((200, 264), dtype, 9)
@@ -207,6 +207,24 @@ def test_gemm_rows_do_not_depend_on_the_batch(dtype):
         assert torch.equal(small, full[:64])
     else:
         torch.testing.assert_close(small.float(), full[:64].float(), atol=0.13, rtol=1e-2)   # one bfloat16 step at |x| ~ 16
+
+
+@pytest.mark.parametrize("n,kk", [(150, 64), (96, 256), (1127, 1088), (3072, 1024), (704, 2048), (2112, 2816), (5000, 576), (1040, 4096)])
+def test_gemm_rows_up_to_64_have_one_order_of_sums(n, kk):
+    """Whole blocks of k: up to 16 rows are the few-row kernel's, 17 to 64 those of tiles that read their operands out of LDS where
+    they are faster.  A row has the same bits alone and among any of them, plain and with gate and silu."""
+    from mini_llm_runtime_amd.kernels import Kernels
+    k = Kernels(torch.bfloat16, library_gemm=False)
+    a, w = rnd((64, kk), torch.bfloat16, 94), rnd((2 * n, kk), torch.bfloat16, 95, 0.3)
+
+    def run(lo, hi, gated):
+        out = torch.full((hi - lo, n if gated else 2 * n), float("nan"), dtype=torch.bfloat16, device="cuda")
+        (k.gemm_gated_silu if gated else k.gemm)(a[lo:hi].contiguous(), w, out)
+        return out
+    for gated in (False, True):
+        alone = torch.cat([run(i, i + 1, gated) for i in range(64)])
+        for lo, hi in [(0, 16), (48, 64), (0, 17), (20, 52), (7, 40), (0, 64)]:
+            assert torch.equal(run(lo, hi, gated), alone[lo:hi]), (lo, hi, gated)
 
 
 @pytest.mark.parametrize("n,kk", [(1, 4), (15, 1), (17, 60), (33, 64), (70, 511), (64, 516), (130, 528), (16400, 96), (4112, 1030), (96, 3072),
@@ -333,9 +351,9 @@ def test_gemm_wide_every_shape(shape, gated, mnk):
 
 @pytest.mark.parametrize("mnk", [(17, 40, 64), (31, 257, 1216), (32, 1041, 1280), (33, 96, 1344), (48, 704, 1024), (63, 1127, 2048), (64, 1152, 2816), (32, 2050, 4032), (29, 520, 576)])
 def test_gemm_few_rows_narrow_tiles(mnk):
-    """17 to 64 rows on the narrow tiles, from fewer blocks of k than the LDS holds (20 at most) to several rounds of it, in
-    whole pairs and not: the bits of the many-row kernel's other tiles from each of them, from the entry points that choose among them, and with an activation;
-    no gated form of strips of 16 columns."""
+    """17 to 64 rows on the tiles made for them, from fewer blocks of k than the LDS holds (20 at most) to several rounds of it, in
+    whole pairs and not, with parts of k that end within a pair: the bits of the few-row kernel from each of them, from the entry points
+    that choose among them, and with an activation; no gated form of strips of 16 columns, none beyond 64 rows."""
     from mini_llm_runtime_amd.kernels.ops import _c_int, _p, _stream
     m, n, kk = mnk
     k = kernels(torch.bfloat16)
@@ -343,18 +361,21 @@ def test_gemm_few_rows_narrow_tiles(mnk):
     a = rnd((m, kk), torch.bfloat16, 68)
     w = rnd((2 * n, kk), torch.bfloat16, 69, 0.3)
 
-    def run(shape, gated=0):
+    def run(shape, gated=0, rows=m):
         out = torch.full((m, n if gated else 2 * n), float("nan"), dtype=torch.bfloat16, device="cuda")
-        rc = lib.mlr_gemm_wide(_p(a), _p(w), _p(out), _c_int(m), _c_int(out.shape[1]), _c_int(kk), _c_int(0), _c_int(shape), _c_int(gated), _stream())
-        assert rc == (-1 if gated and shape in (10, 12) else 0)
+        rc = lib.mlr_gemm_wide(_p(a), _p(w), _p(out), _c_int(rows), _c_int(out.shape[1]), _c_int(kk), _c_int(0), _c_int(shape), _c_int(gated), _stream())
+        assert rc == (-1 if rows > 64 or gated and shape in (10, 12) else 0)
         return out
-    product, silu = run(0), run(0, 1)
+    product, silu = torch.empty((m, 2 * n), dtype=torch.bfloat16, device="cuda"), torch.empty((m, n), dtype=torch.bfloat16, device="cuda")
+    assert lib.mlr_gemm(_p(a), _p(w), _p(product), _c_int(m), _c_int(2 * n), _c_int(kk), _c_int(0), _stream()) == 0
+    assert lib.mlr_gemm_gated_silu(_p(a), _p(w), _p(silu), _c_int(m), _c_int(n), _c_int(kk), _stream()) == 0
     want = a.double() @ w.double().T
     # (kk roundings of 2^-24 of the sum of the sizes, and bfloat16's 2^-9)
     assert bool(((product.double() - want).abs() <= kk * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T) + 2.0 ** -8 * want.abs()).all())
-    for shape in (10, 11, 12, 13, 14, -1):
+    for shape in (10, 11, 12, 13, 14, 15, 16, -2):
         assert torch.equal(run(shape), product), shape
         assert shape in (10, 12) or torch.equal(run(shape, 1), silu), shape
+    run(-2, rows=65)                                       # (refused before anything is launched)
     out, two, one = torch.empty_like(product), torch.empty_like(silu), torch.empty_like(silu)
     if kk <= 2816:
         k.gemm(a, w, out, library=False)
@@ -383,12 +404,15 @@ def test_gemm_wide_tiles_and_epilogues(mnk):
         assert lib.mlr_gemm_wide(_p(a), _p(w), _p(out), _c_int(m), _c_int(out.shape[1]), _c_int(kk), _c_int(0), _c_int(shape), _c_int(gated), _stream()) == 0
         return out
     product, silu = run(-1), run(-1, 1)
+    chain = product
     want = a.double() @ w.double().T
     # a sum of kk products in 32 bits is off by at most kk roundings of 2^-24 of the sum of their sizes; bfloat16 adds 2^-9
     bound = kk * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T) + 2.0 ** -8 * want.abs()
     assert bool(((product.double() - want).abs() <= bound).all())
     for shape in range(10):
-        assert torch.equal(run(shape), product) and torch.equal(run(shape, 1), silu), shape
+        assert torch.equal(run(shape), chain) and torch.equal(run(shape, 1), silu), shape
+    if m <= 64:
+        product = run(-2)                                  # (the activations' products are then those of few rows)
     two, one = torch.empty((m, n), dtype=torch.bfloat16, device="cuda"), torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
     for kind in ("silu", "gelu_tanh", "relu", "clamped"):
         if kind == "silu":
