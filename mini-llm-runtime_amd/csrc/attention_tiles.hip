@@ -223,8 +223,10 @@ __device__ __forceinline__ void tile_group(const TileArgs& a, int grp, int kvh, 
             else mx = max3(mx, max3(sc[t][12], sc[t][13], sc[t][14]), sc[t][15]);
         }
         if (__builtin_amdgcn_ballot_w64(mx > raise_at) != 0) {
-            const float full = fmaxf(mx, __shfl_xor(mx, 32, 64)) * c2;     // the column's maximum in this tile (c2 > 0)
-            if (full > m_ref + RAISE_BY) {                             // the same in both lanes of a column
+            const float both = fmaxf(mx, __shfl_xor(mx, 32, 64)), full = both * c2;      // the column's maximum in this tile (c2 > 0)
+            // (the same in both lanes of a column, and the vote's own comparison: a column is raised by its own scores, not where a
+            // neighbour's vote lets a comparison that rounds otherwise pass; full alone may be -inf)
+            if (both > raise_at && full > m_ref) {
                 const float corr = __builtin_amdgcn_exp2f(m_ref - full);      // -inf - finite: 0
                 l_run *= corr;
 #pragma unroll

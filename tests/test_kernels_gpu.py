@@ -783,6 +783,60 @@ def test_prompt_portions_of_head_size_128(hq, hkv, page, before, n, window, spli
                 before_out = out
 
 
+@pytest.mark.parametrize("d", [128, 64])
+def test_prompt_portions_columns_do_not_depend_on_their_neighbours(d):
+    """A column's reference is raised by its own scores alone.  The second block's maximum is the rounded threshold itself, which
+    times the scale exceeds reference + 8 by a rounding: with neighbours that raise theirs in the same tile and with ones that
+    do not, the column's results are the same bits.  (Scores are sums of three factors of eight bits: exact.  The other keys of
+    the block lie at the edges of a probability's rounding to bfloat16, each with a channel of its own, so a raised reference shows.)"""
+    k = kernels(torch.bfloat16)
+    f32, scale, page = np.float32, d ** -0.5, 64
+    c2 = f32(scale) * f32(1.44269504088896340736)
+    edges = []
+    for s0 in np.arange(20, 110, 2.0 ** -5).astype(f32):
+        m0 = f32(s0 * c2)
+        s1 = f32(f32(m0 + f32(8)) / c2)
+        if f32(s1 * c2) > f32(m0 + f32(8)) and 64 <= s1 < 128:
+            edges.append((s0, m0, s1))
+    edges = edges[:4]
+    assert len(edges) == 4
+    keys, values = np.zeros((160, 4, d), f32), np.zeros((160, 4, d), f32)
+    for head, (s0, m0, s1) in enumerate(edges):
+        scores = np.zeros(128, f32)
+        scores[[0, 32]] = s0                                 # (both halves of a block: either may have a reference of its own)
+        for half in (64, 96):
+            scores[half] = s1
+            for i in range(1, 32):
+                middle = (2 * ((i - 1) // 7) + 1) * 2.0 ** -8 + 1         # between two neighbours in bfloat16, times 2^4
+                x = f32((float(m0) + 4 + math.log2(middle)) / float(c2))
+                scores[half + i] = x + f32((i - 1) % 7 - 3) * np.spacing(x)
+        rest = scores.copy()
+        for part in range(3):                                # eight bits each
+            digit = torch.tensor(rest).view(torch.int32).bitwise_and(-65536).view(torch.float32).numpy()
+            keys[:128, head, part] = digit
+            rest = rest - digit
+        assert not rest.any()
+        values[np.arange(64, 128), head, np.arange(64) % d] = 1
+    k_pages = torch.tensor(keys[:128]).view(2, page, 4, d).transpose(1, 2)
+    v_pages = torch.tensor(values[:128]).view(2, page, 4, d).permute(0, 2, 3, 1)
+    pad = torch.zeros((1, 4, page, d))
+    k_pages = torch.cat([k_pages, pad]).to(torch.bfloat16).contiguous().cuda()
+    v_pages = torch.cat([v_pages, pad.transpose(2, 3)]).to(torch.bfloat16).contiguous().cuda()
+    table = torch.tensor([[0, 1, 2]], dtype=torch.int32, device="cuda")
+    slots, pos = torch.zeros(32, dtype=torch.int32, device="cuda"), torch.arange(128, 160, dtype=torch.int32, device="cuda")
+    first, count = torch.tensor([0], dtype=torch.int32, device="cuda"), torch.tensor([32], dtype=torch.int32, device="cuda")
+    for columns in (64, 128):
+        got = []
+        for neighbours in (0.0, 2.0):
+            q = torch.zeros((32, 4, d))
+            q[0, :, :3], q[1:, :, :3] = 1, neighbours
+            out = torch.full((32, 4 * d), float("nan"), dtype=torch.bfloat16, device="cuda")
+            k.attention_tiles(q.view(32, -1).to(torch.bfloat16).cuda(), k_pages, v_pages, table, slots, pos, out, first, count, 1, 4, 4, d, page, scale,
+                              columns=columns)
+            got.append(out[0])
+        assert bool((got[0].view(4, d)[:, 1:32] > 0).all()) and torch.equal(got[0], got[1]), columns
+
+
 @pytest.mark.parametrize("hq,hkv,d,page,window,split_keys", [(4, 2, 128, 16, None, 0), (4, 2, 128, 16, None, 64), (6, 2, 64, 32, 20, 0),
                                                              (16, 1, 48, 16, None, 0), (3, 1, 256, 16, 33, 64)])
 def test_paged_attention_float_rows_alone(hq, hkv, d, page, window, split_keys):
