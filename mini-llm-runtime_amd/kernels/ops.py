@@ -1744,13 +1744,14 @@ class Kernels:
             _p(partial if splits > 1 else None), _c_int(int(split_keys)), _c_int(int(splits)), _stream())
         _ok(code, "sink_attention_tiles")
 
-    def sink_rows_supported(self, key_dim, value_dim, k_pages, v_pages, page_size, mask=None, mask_size=0, max_context=0, keep_first=0):
+    def sink_rows_supported(self, key_dim, value_dim, k_pages, v_pages, page_size, mask=None, mask_size=0, max_context=0, keep_first=0, rows=()):
         """The sizes of `sink_attention_rows`: keys and values of 128 channels, or latent rows of 576 channels whose first 512
-        are the values, in pages of whole runs of 16, and page ids of a workgroup's keys that fit what it keeps of them."""
+        are the values, in pages of whole runs of 16, and page ids of a workgroup's keys that fit what it keeps of them.  `rows`: the
+        queries and results, which start on 16 bytes like the pages (`sink_attention_tiles` takes them anywhere)."""
         whole = self.SINK_MASKS.get(mask, 0) == 0
         kept = not whole and keep_first > 0
         reach = max_context if whole else mask_size + 128 + (keep_first + 96 if kept else 0)
-        return (self.dtype == torch.bfloat16 and page_size % 16 == 0 and reach // page_size + (4 if kept else 2) <= self.SINK_TILES_BLOCKS and _on16(k_pages, v_pages) and k_pages.shape[3] < 2 ** 24
+        return (self.dtype == torch.bfloat16 and page_size % 16 == 0 and reach // page_size + (4 if kept else 2) <= self.SINK_TILES_BLOCKS and _on16(k_pages, v_pages, *rows) and k_pages.shape[3] < 2 ** 24
                 and ((key_dim, value_dim) == (128, 128) and k_pages.data_ptr() != v_pages.data_ptr()
                      or (key_dim, value_dim) == (576, 512) and k_pages.data_ptr() == v_pages.data_ptr() and k_pages.shape[3] == v_pages.shape[3]))
 
@@ -1766,7 +1767,7 @@ class Kernels:
         k_row = self._sink_pages(k_pages, "k_pages", kv_heads, page_size, key_dim)
         v_row = self._sink_pages(v_pages, "v_pages", kv_heads, page_size, value_dim)
         _need(mask in self.SINK_MASKS, f"mask {mask!r}: one of all, window, chunk")
-        _need(self.sink_rows_supported(key_dim, value_dim, k_pages, v_pages, page_size, mask, mask_size, max_context, keep_first) and _on16(q, out),
+        _need(self.sink_rows_supported(key_dim, value_dim, k_pages, v_pages, page_size, mask, mask_size, max_context, keep_first, (q, out)),
               "sink_attention_rows: sizes not supported")
         kind = self.SINK_MASKS[mask]
         _need(kind == 0 or mask_size >= 1, "a window or chunk needs a positive size")

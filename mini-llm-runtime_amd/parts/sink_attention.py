@@ -144,7 +144,7 @@ def attend(ctx, q, k_pages, v_pages, view, sink, out, q_heads, kv_heads, key_dim
         portions = not ctx.routed and k.portion_attention_supported(q_heads, kv_heads, key_dim, value_dim, k_pages.shape[3], v_pages.shape[3],
                                                                     view.page_size, mask, mask_size, ctx.max_positions, keep_first, scale)
         rows = not portions and k.sink_rows_supported(key_dim, value_dim, k_pages, v_pages, view.page_size, mask, mask_size,
-                                                      ctx.max_positions, keep_first)
+                                                      ctx.max_positions, keep_first, (q, out))
         if portions or rows:
             columns, big_heads = portion_columns(ctx, q_heads, 64 if rows else 128), min(big_heads, 32)
             big_tokens = columns // big_heads

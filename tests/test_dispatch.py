@@ -244,3 +244,26 @@ def test_products_of_a_model_with_a_router_keep_the_order_of_their_sums(sizes):
     assert not k.wide_product(*sizes) and not k.wide_product(*sizes, "silu")
     k._wide_choices[(1777, 6144, 4096, None)] = True
     assert k.wide_product(1777, 6144, 4096)
+
+
+@pytest.mark.parametrize("shift_q,shift_out", [(0, 0), (1, 0), (0, 1)])
+def test_rows_that_do_not_start_on_16_bytes_keep_the_attention_that_takes_them(shift_q, shift_out):
+    """Queries or results that are views off 16 bytes: the prompt portions' kernel for whole rows does not take them, the general one
+    does, and nothing is refused."""
+    from mini_llm_runtime_amd.parts.sink_attention import attend
+    ctx = context(1000)
+    ctx.workspace.reserve({("token_groups_1_8", torch.int32): 4000})
+    ctx._group_upload, ctx.segments, ctx.n_tokens, ctx.routed = HostUpload(), [(0, 0, 300, 0)], 300, True
+    ctx.slots = ctx.positions = torch.zeros(300, dtype=torch.int32)
+    ctx.max_positions, ctx.compute_units = 1000, 256
+    taken = []
+    k = ctx.kernels
+    k.sink_attention_rows = lambda *a, **kw: taken.append("rows")
+    k.sink_attention_tiles = lambda *a, **kw: taken.append("tiles")
+
+    def rows(width, shift):
+        return torch.empty(300 * width + shift, dtype=torch.bfloat16)[shift:].view(300, width)
+    k_pages, v_pages = (torch.empty((70, 1, 16, 128), dtype=torch.bfloat16) for _ in range(2))
+    view = type("View", (), dict(page_size=16, block_table=None))
+    attend(ctx, rows(16 * 128, shift_q), k_pages, v_pages, view, None, rows(16 * 128, shift_out), 16, 1, 128, 128, 0.1, None, 0)
+    assert taken[0] == ("tiles" if shift_q or shift_out else "rows")
