@@ -383,10 +383,11 @@ class Kernels:
             return rows <= 64
         return rows <= LIBRARY_GEMM_MIN_ROWS or (rows <= 64 and k * ((rows + 15) // 16) <= 4096)
 
-    def wide_product(self, rows, columns, k, act=None):
+    def wide_product(self, rows, columns, k, act=None, w=None):
         """Whether the kernel for many rows (from 17 on) takes a product of these sizes and not the vendor library;
-        `act`: with that activation in its epilogue, of `columns` gates beside as many ups or of the product itself."""
-        if self.dtype != torch.bfloat16 or rows <= LIBRARY_GEMM_MIN_ROWS:
+        `act`: with that activation in its epilogue, of `columns` gates beside as many ups or of the product itself; `w`: the
+        weight, which must start on 16 bytes."""
+        if self.dtype != torch.bfloat16 or rows <= LIBRARY_GEMM_MIN_ROWS or (w is not None and not _on16(w)):
             return False
         # A choice among experts turns on the last bit.  The library adds in this kernel's order, bit by bit, but where it cuts k
         # into parts: few outputs or a long k (of 8 row counts and 21 sizes, compared: none of at least 2^19 outputs with k up to
@@ -409,10 +410,10 @@ class Kernels:
     # the epilogues of `gemm_activated` (csrc/gemm.hip, WIDE_*)
     WIDE_ACTS = {None: 0, "silu": 2, "gelu_tanh": 3, "relu": 4, "clamped": 5, "relu_squared": 6, "gelu_erf": 7}
 
-    @timed("gemm", _gemm_work)
     def gemm_activated(self, a, w, out, kind, limit=0.0, slope=0.0):
         """The product and its activation in one launch, for the sizes of `wide_product`; the bits of `gemm` followed by
-        `silu_mul`, `gated_act_mul` or `clamped_glu` (w = [gate; up] stacked) or by `plain_act`."""
+        `silu_mul`, `gated_act_mul` or `clamped_glu` (w = [gate; up] stacked) or by `plain_act`, and those launches themselves
+        where the weight does not start on 16 bytes."""
         _need(self.dtype == torch.bfloat16, "gemm_activated: bfloat16 only")
         _need(kind is not None and kind in self.WIDE_ACTS, f"gemm_activated: activation {kind!r}")
         _tensor(a, "a", self.dtype, ndim=2)
@@ -424,30 +425,53 @@ class Kernels:
         _need(k % 64 == 0 and a.numel() < 2 ** 31 and w.numel() < 2 ** 31,
               "gemm_activated: the inner size must be a multiple of 64, matrices below 2^31 elements")
         _need(kind != "clamped" or limit > 0, "gemm_activated: the clamp's limit must be positive")
-        n = n // 2 if gated else n
-        _tensor(out, "out", self.dtype, (m, n))
-        a, w = _start16(a), _start16(w)
+        _tensor(out, "out", self.dtype, (m, n // 2 if gated else n))
+        if _on16(w):
+            self._gemm_activated(_start16(a), w, out, kind, limit, slope)
+        else:
+            self._product_then_activation(a, w, out, kind, limit, slope)
+
+    def _product_then_activation(self, a, w, out, kind, limit=0.0, slope=0.0):
+        """(the weight's copy on 16 bytes would be made again on every call, and in every replay of a captured one)"""
+        if kind in self.PLAIN_ACTS:
+            self.gemm(a, w, out)
+            self.plain_act(out, out, kind)
+            return
+        both = torch.empty((a.shape[0], w.shape[0]), dtype=self.dtype, device=a.device)
+        self.gemm(a, w, both)
+        if kind == "clamped":
+            self.clamped_glu(both, out, limit, slope)
+        elif kind == "silu":
+            self.silu_mul(both, out)
+        else:
+            self.gated_act_mul(both, out, kind)
+
+    @timed("gemm", _gemm_work)
+    def _gemm_activated(self, a, w, out, kind, limit, slope):
+        (m, k), n = a.shape, out.shape[1]
         _ok(self._lib("gemm").mlr_gemm_activated(_p(a), _p(w), _p(out), _c_int(m), _c_int(n), _c_int(k), _c_int(self.WIDE_ACTS[kind]),
                                                  _c_float(limit), _c_float(slope), _stream()), "gemm_activated")
 
-    def gated_silu_fused(self, rows, k=None):
+    def gated_silu_fused(self, rows, k=None, w=None):
         """Whether `gemm_gated_silu` is the path for this many rows and inner size: the bfloat16 engine, where
-        `streams_weight` says so, and without the library any number of rows when the inner size is a multiple of 64."""
-        if self.dtype == torch.bfloat16 and rows > 64 and k is not None and k % 64 == 0 and rows * k < 2 ** 31:
+        `streams_weight` says so, and without the library any number of rows when the inner size is a multiple of 64 (and the weight
+        `w`, where it is given, starts on 16 bytes)."""
+        if self.dtype == torch.bfloat16 and rows > 64 and k is not None and k % 64 == 0 and rows * k < 2 ** 31 and (w is None or _on16(w)):
             # Many rows: the gate taken of the unrounded products.  Beside the library only where it has always been (short
             # inner sizes); elsewhere `gemm_activated`, which takes it of the rounded ones as the library's product and
             # the activation's kernel do: a router behind it must not see other values.
             return not self.library_gemm or k <= 1024 or (k <= 2048 and rows <= 256)
         return self.streams_weight(rows, k if k is not None else 1 << 30)
 
-    def gated_strips(self, rows, columns, k):
-        """Whether `gemm_gated_silu` is the float engine's way for `rows` times `columns` gates: tiles of 16 x 16 that are few."""
-        return self.dtype == torch.float32 and k % 4 == 0 and -(-rows // 16) * -(-columns // 16) <= 512
+    def gated_strips(self, rows, columns, k, w=None):
+        """Whether `gemm_gated_silu` is the float engine's way for `rows` times `columns` gates: tiles of 16 x 16 that are few (and
+        the weight `w`, where it is given, starts on 16 bytes)."""
+        return self.dtype == torch.float32 and k % 4 == 0 and -(-rows // 16) * -(-columns // 16) <= 512 and (w is None or _on16(w))
 
-    @timed("gemm", _gemm_work)
     def gemm_gated_silu(self, a, w, out):
         """out[M, N] = silu(a . w[:N]^T) * (a . w[N:]^T), w = [gate; up] stacked: up to 64 rows, or any number
-        when the inner size is a multiple of 64 (the wide kernel's gated form); float32: the sizes of `gated_strips`."""
+        when the inner size is a multiple of 64 (the wide kernel's gated form); float32: the sizes of `gated_strips`.  More than 64
+        rows, and float32, of a weight off 16 bytes: the product and `silu_mul`."""
         strips = self.dtype == torch.float32
         _need(not strips or self.gated_strips(a.shape[0], w.shape[0] // 2, a.shape[1]), "gemm_gated_silu: too many rows and columns in float32")
         _need(strips or a.shape[0] <= 64 or (a.shape[1] % 64 == 0 and a.numel() < 2 ** 31 and w.numel() < 2 ** 31),
@@ -459,8 +483,14 @@ class Kernels:
         two_n, k2 = w.shape
         _need(k == k2 and two_n % 2 == 0, "gemm_gated_silu: sizes do not fit")
         _tensor(out, "out", self.dtype, (m, two_n // 2))
-        if m > 64 or strips:
-            a, w = _start16(a), _start16(w)
+        if (m > 64 or strips) and not _on16(w):
+            self._product_then_activation(a, w, out, "silu")
+        else:
+            self._gemm_gated_silu(_start16(a) if m > 64 or strips else a, w, out)
+
+    @timed("gemm", _gemm_work)
+    def _gemm_gated_silu(self, a, w, out):
+        (m, k), two_n = a.shape, w.shape[0]
         if m <= 64 and self.wide_product(m, two_n // 2, k, "silu") and _on16(a, w):
             _ok(self._lib("gemm").mlr_gemm_wide(_p(a), _p(w), _p(out), _c_int(m), _c_int(two_n // 2), _c_int(k), _c_int(0), _c_int(-2),
                                                 _c_int(1), _stream()), "gemm_gated_silu")

@@ -61,11 +61,12 @@ class SwiGluMlp:
         s = self.spec
         m = x.shape[0]
         act = ctx.workspace.get("act", (m, s.intermediate), x.dtype)
-        if s.activation == "silu" and (ctx.kernels.gated_silu_fused(m, s.hidden) or ctx.kernels.gated_strips(m, s.intermediate, s.hidden)):
+        if s.activation == "silu" and (ctx.kernels.gated_silu_fused(m, s.hidden, self.gate_up) or
+                                       ctx.kernels.gated_strips(m, s.intermediate, s.hidden, self.gate_up)):
             ctx.kernels.gemm_gated_silu(x, self.gate_up, act)      # few rows: the activation rides on the projection
         elif s.activation != "silu" and m <= 64 and ctx.kernels.streams_weight(m, s.hidden):
             ctx.kernels.gemm_gated_act(x, self.gate_up, act, s.activation)
-        elif ctx.kernels.wide_product(m, s.intermediate, s.hidden, s.activation):
+        elif ctx.kernels.wide_product(m, s.intermediate, s.hidden, s.activation, self.gate_up):
             ctx.kernels.gemm_activated(x, self.gate_up, act, s.activation)
         else:
             gate_up = ctx.workspace.get("gate_up", (m, 2 * s.intermediate), x.dtype)
@@ -118,7 +119,7 @@ class ClampedGluMlp:
         act = ctx.workspace.get("act", (m, s.intermediate), x.dtype)
         if k.streams_weight(m, s.hidden):             # few rows: the activation rides on the projection
             k.gemm_gated_clamped(x, self.gate_up, act, float(s.limit), float(s.slope))
-        elif k.wide_product(m, s.intermediate, s.hidden, "clamped"):
+        elif k.wide_product(m, s.intermediate, s.hidden, "clamped", self.gate_up):
             k.gemm_activated(x, self.gate_up, act, "clamped", float(s.limit), float(s.slope))
         else:
             gate_up = ctx.workspace.get("gate_up", (m, 2 * s.intermediate), x.dtype)
@@ -164,7 +165,7 @@ class PlainMlp:
         act = ctx.workspace.get("act", (m, s.intermediate), x.dtype)
         if m <= 64 and k.streams_weight(m, s.hidden):      # few rows: the activation rides on the projection
             k.gemm_act(x, self.up, act, s.activation)
-        elif k.wide_product(m, s.intermediate, s.hidden, s.activation):
+        elif k.wide_product(m, s.intermediate, s.hidden, s.activation, self.up):
             k.gemm_activated(x, self.up, act, s.activation)
         else:
             k.gemm(x, self.up, act)

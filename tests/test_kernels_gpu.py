@@ -438,6 +438,36 @@ def test_gemm_wide_tiles_and_epilogues(mnk):
     assert bool(((out.double() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("dtype,m,n,kk", [(torch.bfloat16, 100, 3000, 512), (torch.bfloat16, 20, 3000, 512), (torch.float32, 8, 1000, 2048)])
+def test_activations_behind_a_weight_off_16_bytes(dtype, m, n, kk):
+    """A weight that is a view off 16 bytes is read where it lies: no call copies it, and the feed-forward's choice of a way looks at
+    it.  The results are the product's and the activation's own launches."""
+    k = kernels(dtype)
+    a, aligned = rnd((m, kk), dtype, 96), rnd((2 * n, kk), dtype, 97, 0.3)
+    w = torch.empty(2 * n * kk + 1, dtype=dtype, device="cuda")[1:].view(2 * n, kk).copy_(aligned)
+    one, want, both = (torch.empty((m, c), dtype=dtype, device="cuda") for c in (n, n, 2 * n))
+    k.gemm(a, w, both)
+    k.silu_mul(both, want)
+    calls = [lambda: k.gemm_gated_silu(a, w, one)] if m > 64 or dtype == torch.float32 else []
+    if dtype == torch.bfloat16:
+        calls.append(lambda: k.gemm_activated(a, w, one, "silu"))
+        assert not k.wide_product(m, n, kk, "silu", w) and k.gated_silu_fused(m, kk, w) == (m <= 64)
+    assert not k.gated_strips(m, n, kk, w)
+    for call in calls:
+        one.fill_(float("nan"))
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        call()
+        assert torch.equal(one, want)
+        assert torch.cuda.max_memory_allocated() - before < w.numel() * w.element_size()
+    if dtype == torch.bfloat16:
+        whole, got = both.clone(), torch.full_like(both, float("nan"))
+        k.plain_act(whole, whole, "gelu_erf")
+        k.gemm_activated(a, w, got, "gelu_erf")
+        assert torch.equal(got, whole)
+
+
 def test_gemm_wide_rows_do_not_depend_on_the_batch():
     """More than 64 rows with an inner size that is a multiple of 64: the tile shape follows the number of
     rows, a row's bits do not."""
