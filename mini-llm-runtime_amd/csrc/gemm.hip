@@ -47,6 +47,7 @@ template <int LEFT> __device__ __forceinline__ void strip_wait() { asm volatile(
 
 // The products of one wavefront: `a` and `w` start at its first row of each, of which there are a_rows and w_rows (more than that
 // are the last one again); lds: [STAGES][G][1 + NT][256] floats of its own.
+constexpr int STRIP_K = 1 << 25;                           // k must be below: a strip's 32 rows then lie within 32 bits of bytes
 template <int NT, int STAGES> constexpr int strip_lds_floats() { return STAGES * 4 * (1 + NT) * 256; }
 template <int NT, int STAGES>
 __device__ __forceinline__ void f32_strip(const float* __restrict__ a, const float* __restrict__ w, int a_rows, int w_rows, int K,
@@ -287,7 +288,7 @@ static int launch_gemm_f32(const float* a, const float* w, float* out, int M, in
     // here).  Two strips a wavefront beyond that, while the rows are few or up to 1024 tiles: 64 rows of 4096 x 1024 14.1 (tiles
     // of 32 16.7), 8 of 151936 x 1024 144 (the weight alone takes 130); 64 rows of 6144 x 1024 (1536 tiles) in tiles of 32 21.3.
     const long long units = (long long)((M + 15) / 16) * ((N + 15) / 16);
-    if (VEC && (M + 15) / 16 <= 65535) {
+    if (VEC && (M + 15) / 16 <= 65535 && K < STRIP_K) {
         if (units <= 768) return units <= 512 ? launch_f32_strip<1, 8>(a, w, out, M, N, K, stream) : launch_f32_strip<1, 5>(a, w, out, M, N, K, stream);
         if (M <= 16 || units <= 1024) return launch_f32_strip<2, 4>(a, w, out, M, N, K, stream);
     }
@@ -324,7 +325,7 @@ extern "C" int mlr_gemm_gated_silu(const void* a, const void* w, void* out, int 
     if (M <= 0 || N <= 0) return 0;
     if (K <= 0) return -1;
     const long long units = (long long)((M + 15) / 16) * ((N + 15) / 16);
-    if (K % 4 != 0 || ((uintptr_t)a | (uintptr_t)w) % 16 != 0 || units > 512) return 1;
+    if (K % 4 != 0 || K >= STRIP_K || ((uintptr_t)a | (uintptr_t)w) % 16 != 0 || units > 512) return 1;
     if (units <= 256) return launch_f32_gated_strip<8>((const float*)a, (const float*)w, (float*)out, M, N, K, stream);
     return launch_f32_gated_strip<4>((const float*)a, (const float*)w, (float*)out, M, N, K, stream);
 }

@@ -466,7 +466,8 @@ class Kernels:
     def gated_strips(self, rows, columns, k, w=None):
         """Whether `gemm_gated_silu` is the float engine's way for `rows` times `columns` gates: tiles of 16 x 16 that are few (and
         the weight `w`, where it is given, starts on 16 bytes)."""
-        return self.dtype == torch.float32 and k % 4 == 0 and -(-rows // 16) * -(-columns // 16) <= 512 and (w is None or _on16(w))
+        return (self.dtype == torch.float32 and k % 4 == 0 and k < 1 << 25 and -(-rows // 16) * -(-columns // 16) <= 512
+                and (w is None or _on16(w)))
 
     def gemm_gated_silu(self, a, w, out):
         """out[M, N] = silu(a . w[:N]^T) * (a . w[N:]^T), w = [gate; up] stacked: up to 64 rows, or any number

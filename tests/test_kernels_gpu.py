@@ -438,6 +438,21 @@ def test_gemm_wide_tiles_and_epilogues(mnk):
     assert bool(((out.double() - want).abs() <= bound).all())
 
 
+def test_gemm_float_of_an_inner_size_beyond_32_bits_of_bytes():
+    """16 rows of 2^26 floats are 2^32 bytes, one more than the few-row kernel's loads reach: the product is the tiles', plain and
+    beside an activation.  (Whole numbers: exact.)"""
+    k, kk = kernels(torch.float32), 1 << 26
+    a, w = torch.zeros((1, kk), device="cuda"), torch.full((2, kk), 3.0, device="cuda")
+    a[0, ::1 << 22] = 1
+    a[0, -1] = 2
+    out, act = torch.full((1, 2), float("nan"), device="cuda"), torch.full((1, 1), float("nan"), device="cuda")
+    k.gemm(a, w, out)
+    assert out.tolist() == [[54.0, 54.0]]
+    assert not k.gated_strips(1, 1, kk)
+    k.silu_mul(out, act)
+    assert abs(act.item() - 54.0 * 54.0) < 1e-3
+
+
 @pytest.mark.parametrize("dtype,m,n,kk", [(torch.bfloat16, 100, 3000, 512), (torch.bfloat16, 20, 3000, 512), (torch.float32, 8, 1000, 2048)])
 def test_activations_behind_a_weight_off_16_bytes(dtype, m, n, kk):
     """A weight that is a view off 16 bytes is read where it lies: no call copies it, and the feed-forward's choice of a way looks at
