@@ -69,8 +69,7 @@ class Runner:
         self.max_length = min(max_length or spec.max_positions, spec.max_positions)
         self.max_batch_tokens = max_batch_tokens or self.max_length
         # library_gemm=False: every product on the hand-written kernels (the vendor library takes none)
-        self.kernels = Kernels(self.dtype, library_gemm=library_gemm)
-        self.kernels.routed = model.routes()
+        self.kernels = Kernels(self.dtype, library_gemm=library_gemm, routed=model.routes())
         self.kernels.prepare(model.libraries())
         for block in model.blocks:                        # sizes that no step could serve are refused now
             for part in block.parts().values():

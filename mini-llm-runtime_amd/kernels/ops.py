@@ -136,14 +136,15 @@ def _tensors_work(*names):
 
 
 class Kernels:
-    routed = False                          # the model chooses among experts: sums keep their order (`wide_product`)
-
-    def __init__(self, dtype, library_gemm=True):
+    def __init__(self, dtype, library_gemm=True, routed=False):
+        """`library_gemm`: the vendor library takes the products that it is the faster way for.  `routed`: the launches are those of
+        a model that chooses among experts, whose products keep the order of their sums (`wide_product`)."""
         _need(dtype in (torch.float32, torch.bfloat16), f"no kernels for element type {dtype}")
         if not torch.cuda.is_available():
             raise KernelError("no GPU is visible: the engine's kernels are HIP only")
         self.dtype = dtype
         self.library_gemm = library_gemm
+        self.routed = routed
         self._library_workspace = None      # scratch memory of the vendor library's products, allocated once
         self._wide_choices = {}             # (rows, columns, inner size, activation) -> `wide_product`
         self._libs = {}

@@ -10,9 +10,9 @@ from mini_llm_runtime_amd.kernels.ops import MAX_KEY_SPLITS, MFMA_MAX_PAGES, Ker
 from mini_llm_runtime_amd.parts.registry import PartError, build_part
 
 
-def kernels_without_gpu(dtype=torch.bfloat16):
+def kernels_without_gpu(dtype=torch.bfloat16, routed=False):
     k = Kernels.__new__(Kernels)              # the size questions need no device
-    k.dtype, k.library_gemm, k._libs = dtype, True, {}
+    k.dtype, k.library_gemm, k.routed, k._libs = dtype, True, routed, {}
     return k
 
 
@@ -240,7 +240,8 @@ def test_products_of_a_model_with_a_router_keep_the_order_of_their_sums(sizes):
     k = kernels_without_gpu()
     k._wide_choices = {sizes + (None,): True, sizes + ("silu",): True}
     assert k.wide_product(*sizes) and k.wide_product(*sizes, "silu")
-    k.routed = True
+    k = kernels_without_gpu(routed=True)
+    k._wide_choices = {sizes + (None,): True, sizes + ("silu",): True}
     assert not k.wide_product(*sizes) and not k.wide_product(*sizes, "silu")
     k._wide_choices[(1777, 6144, 4096, None)] = True
     assert k.wide_product(1777, 6144, 4096)
@@ -267,3 +268,10 @@ def test_rows_that_do_not_start_on_16_bytes_keep_the_attention_that_takes_them(s
     view = type("View", (), dict(page_size=16, block_table=None))
     attend(ctx, rows(16 * 128, shift_q), k_pages, v_pages, view, None, rows(16 * 128, shift_out), 16, 1, 128, 128, 0.1, None, 0)
     assert taken[0] == ("tiles" if shift_q or shift_out else "rows")
+
+
+def test_whether_a_model_routes_is_said_where_its_kernels_are_made(monkeypatch):
+    """No state of the class, and none that is set from outside later."""
+    monkeypatch.setattr(torch.cuda, "is_available", lambda: True)
+    assert not hasattr(Kernels, "routed")
+    assert Kernels(torch.bfloat16, routed=True).routed and not Kernels(torch.bfloat16).routed
