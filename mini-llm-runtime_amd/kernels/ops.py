@@ -390,23 +390,31 @@ class Kernels:
         weight, which must start on 16 bytes."""
         if self.dtype != torch.bfloat16 or rows <= LIBRARY_GEMM_MIN_ROWS or (w is not None and not _on16(w)):
             return False
-        # A choice among experts turns on the last bit.  The library adds in this kernel's order, bit by bit, but where it cuts k
-        # into parts: few outputs or a long k (of 8 row counts and 21 sizes, compared: none of at least 2^19 outputs with k up to
-        # 8448 differs; 333 x 768 x 2048, every 64 x n x 2048 of few columns, 1777 x 4096 x 18432 do, in one output of 2000).
-        if self.routed and (rows <= 64 or (self.library_gemm and (rows * columns < 1 << 19 or k > 8448))):
+        kind = self.WIDE_ACTS[act]
+        weight_rows = columns * (2 if 1 <= kind <= 5 else 1)
+        if self.routed and (rows <= 64 or (self.library_gemm and not self.library_adds_alike(rows * weight_rows, k))):
             return False
         key = (rows, columns, k, act)
         wins = self._wide_choices.get(key)
         if wins is None:
-            kind = self.WIDE_ACTS[act]
             wins = bool(self._lib("gemm").mlr_gemm_wide_wins(_c_int(rows), _c_int(columns), _c_int(k), _c_int(kind)))
             if not self.library_gemm and rows > 64:
-                weight_rows = columns * (2 if 1 <= kind <= 5 else 1)
                 wins = k % 64 == 0 and rows * k < 2 ** 31 and weight_rows * k < 2 ** 31
             if len(self._wide_choices) >= WIDE_CHOICES_KEPT:
                 self._wide_choices.clear()
             self._wide_choices[key] = wins
         return wins
+
+    @staticmethod
+    def library_adds_alike(outputs, k):
+        """Whether the vendor library's first choice for a product of more than 64 rows adds in the many-row kernel's order, one chain
+        over k.  A choice between two experts that lie within rounding turns on the last bit, so a model that routes takes the kernel
+        only where nothing turns.  Compared bit by bit on 36 000 products of 65 to 8192 rows (library of ROCm 7.2): none of 2^18
+        to 2^23 outputs with k up to 8192 differs (16 000), none of up to 2^24 with k up to 2048 (7 000).  Outside, the library
+        cuts k into parts or deals them out to workgroups: few outputs (333 x 768 x 2048), many (from 2^23.1 at k = 2560, 2^23.9 at
+        2112; 1603 x 28736 x 6016), long k (from 8832 with 2^21 outputs, nearly all beyond 16384).  Where the library times its candidates (multiples of
+        64 rows) it may choose one that cuts k, another one in another process: there this kernel's order is the lasting one."""
+        return 1 << 19 <= outputs < (1 << 24 if k <= 2048 else 1 << 23) and k <= 8192
 
     # the epilogues of `gemm_activated` (csrc/gemm.hip, WIDE_*)
     WIDE_ACTS = {None: 0, "silu": 2, "gelu_tanh": 3, "relu": 4, "clamped": 5, "relu_squared": 6, "gelu_erf": 7}

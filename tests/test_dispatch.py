@@ -233,7 +233,7 @@ def test_key_ranges_of_one_width_whatever_the_batch():
     assert keys == 512 and splits == -(-300000 // 512) <= MAX_KEY_SPLITS and chunk == 3
 
 
-@pytest.mark.parametrize("sizes", [(17, 6144, 2048), (64, 12288, 1024), (333, 768, 2048), (1777, 4096, 18432)])
+@pytest.mark.parametrize("sizes", [(17, 6144, 2048), (64, 12288, 1024), (333, 768, 2048), (1777, 4096, 18432), (1603, 28736, 6016), (653, 23648, 2176)])
 def test_products_of_a_model_with_a_router_keep_the_order_of_their_sums(sizes):
     """Where the vendor library may add in another order than the many-row kernel, a model that chooses among experts stays with
     it (asked without a GPU: the answer must not need the kernels' library); other models ask the kernels' own rule."""
@@ -243,8 +243,9 @@ def test_products_of_a_model_with_a_router_keep_the_order_of_their_sums(sizes):
     k = kernels_without_gpu(routed=True)
     k._wide_choices = {sizes + (None,): True, sizes + ("silu",): True}
     assert not k.wide_product(*sizes) and not k.wide_product(*sizes, "silu")
-    k._wide_choices[(1777, 6144, 4096, None)] = True
-    assert k.wide_product(1777, 6144, 4096)
+    k._wide_choices.update({(1777, 4096, 4096, None): True, (1777, 6144, 4096, None): True, (1777, 3000, 2048, "silu"): True, (1777, 6000, 2048, "silu"): True})
+    assert k.wide_product(1777, 4096, 4096) and not k.wide_product(1777, 6144, 4096)
+    assert k.wide_product(1777, 3000, 2048, "silu") and not k.wide_product(1777, 6000, 2048, "silu")     # (a gate's outputs are two)
 
 
 @pytest.mark.parametrize("shift_q,shift_out", [(0, 0), (1, 0), (0, 1)])

@@ -438,6 +438,28 @@ def test_gemm_wide_tiles_and_epilogues(mnk):
     assert bool(((out.double() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("m,n,kk", [(65, 8072, 8192), (67, 16000, 64), (75, 111800, 1984), (99, 80000, 8128), (130, 4040, 4032), (333, 1576, 8000),
+                                    (333, 25000, 8192), (509, 32800, 2048), (701, 760, 7360), (997, 536, 3328), (1001, 8376, 8192), (1499, 11100, 1088),
+                                    (2047, 264, 2048), (2001, 4192, 8192), (2049, 8184, 2048), (4099, 2040, 5056), (8191, 1016, 8192), (8190, 2040, 1920)])
+def test_the_library_adds_alike_where_models_with_a_router_leave_it(m, n, kk):
+    """Products inside and at the edges of `library_adds_alike`: the vendor library's own first choice has the many-row kernel's bits,
+    alone and with the activation behind it in a launch of its own.  (Row counts that the library does not time.)"""
+    from mini_llm_runtime_amd.kernels.ops import _c_int, _p, _stream
+    k = kernels(torch.bfloat16)
+    assert k.library_adds_alike(m * n, kk) and m % 64 != 0
+    a = rnd((m, kk), torch.bfloat16, 98)
+    w = torch.empty((n, kk), dtype=torch.bfloat16, device="cuda").normal_(generator=torch.Generator("cuda").manual_seed(99)).mul_(0.05)
+    out, own = (torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    k.wide_product = lambda *sizes: False
+    k.gemm(a, w, out)
+    assert k._lib("gemm").mlr_gemm_wide(_p(a), _p(w), _p(own), _c_int(m), _c_int(n), _c_int(kk), _c_int(0), _c_int(-1), _c_int(0), _stream()) == 0
+    assert torch.equal(out, own)
+    act, one = (torch.full((m, n // 2), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    k.silu_mul(out, act)
+    k.gemm_activated(a, w, one, "silu")
+    assert torch.equal(act, one)
+
+
 def test_gemm_float_of_an_inner_size_beyond_32_bits_of_bytes():
     """16 rows of 2^26 floats are 2^32 bytes, one more than the few-row kernel's loads reach: the product is the tiles', plain and
     beside an activation.  (Whole numbers: exact.)"""
