@@ -1371,16 +1371,16 @@ static const WideCost WIDE_COSTS[WIDE_SHAPES] = {
 
 
 // The same for 17 to 64 rows, where a workgroup reads its weight once and what counts is the bytes of weight under way and what a
-// turn waits: narrow tiles with up to 19 blocks on their way, two of them a turn.  `row`: what 16 more rows add to a round.  Fitted to
-// 200 products of 17, 32, 40 and 64 rows, inner sizes of 1024 to 8192 and 512 to 51200 rows of weight, weights cold (the predicted
-// tile is 1 % behind the best one on average).  Strips of 16 columns have no gated form.  With one block a turn, a turn of the tiles
-// of 32 x 16 to 64 x 16 took 0.14 to 0.2 us: 32 x 4096 x 1024 5.2 -> 4.7 us, 32 x 2112 x 4096 10.3 -> 9.3, 17 x 2 * 704 x 2048 6.8 ->
-// 5.1; tiles of 64 x 32 and 64 x 64, which two workgroups of a compute unit share, gain nothing by it.
-struct FewCost { int shape, bm, bn, per_unit; float fixed, one, all, row; };
+// turn waits: narrow tiles with up to 19 blocks on their way, two of them a turn.  `turn`: what a round takes whatever k is (its
+// first blocks' way, closing the parts of k, the epilogue); `row`: what 16 more rows add to 1024 k of one.  Fitted to 768 products of
+// 17 to 64 rows, inner sizes drawn from 512 to 9000 and 256 to 36000 rows of weight, weights cold (the predicted tile is 0.5 % behind
+// the best one, geometric mean).  Strips of 16 columns have no gated form.  32 x 4096 x 1024 5.0 us, 32 x 2112 x 4096 9.5,
+// 17 x 2 * 704 x 2048 6.1; tiles of 64 x 32 and 64 x 64, which two workgroups of a compute unit share, gain nothing by two blocks a turn.
+struct FewCost { int shape, bm, bn, per_unit; float fixed, turn, one, all, row; };
 static const FewCost FEW_COSTS[] = {
-    {15, 64, 32, 2, 1.94f, 2.07f, 5.72f, 0.59f}, {16, 64, 64, 2, 1.87f, 3.1f, 10.4f, 0.67f}, {10, 64, 16, 1, 1.38f, 0.f, 1.76f, 0.28f},
-    {11, 64, 96, 1, 2.15f, 0.f, 4.17f, 0.48f},  {12, 32, 16, 1, 2.1f, 0.f, 1.81f, 0.f},    {13, 32, 32, 1, 0.83f, 0.f, 3.04f, 0.f},
-    {14, 32, 64, 1, 0.97f, 0.f, 4.1f, 0.f}};
+    {10, 64, 16, 1, 0.47f, 1.99f, 0.f, 1.42f, 0.253f}, {11, 64, 96, 1, -3.38f, 6.82f, 0.f, 3.83f, 0.461f}, {12, 32, 16, 1, 0.25f, 2.28f, 0.f, 1.51f, 0.f},
+    {13, 32, 32, 1, -0.86f, 3.48f, 0.f, 2.12f, 0.f},   {14, 32, 64, 1, -3.54f, 6.09f, 0.f, 3.32f, 0.f},    {15, 64, 32, 2, 1.83f, 1.25f, 2.05f, 5.37f, 0.465f},
+    {16, 64, 64, 2, 2.20f, 0.93f, 2.60f, 9.16f, 0.711f}};
 
 static int few_shape_for(int M, int N, int K, bool gated) {
     const int units = compute_units() > 0 ? compute_units() : 256, row_tiles = (M + 15) / 16;
@@ -1391,7 +1391,8 @@ static int few_shape_for(int M, int N, int K, bool gated) {
         const int bn = gated ? c.bn / 2 : c.bn, tiles = (N + bn - 1) / bn, slots = units * c.per_unit, left = tiles % slots;
         const bool alone = c.per_unit == 2 && left > 0 && left <= units;
         const float rounds = (float)(tiles / slots + (left > 0 && !alone ? 1 : 0)), more = c.row * (float)row_tiles;
-        const float us = c.fixed + (rounds * (c.all + more) + (alone ? c.one + 0.6f * more : 0.f)) * (float)K * (1.0f / 1024.0f);
+        const float us = c.fixed + (rounds + (alone ? 0.6f : 0.f)) * c.turn +
+                         (rounds * (c.all + more) + (alone ? c.one + 0.6f * more : 0.f)) * (float)K * (1.0f / 1024.0f);
         if (best < 0 || us < time) {
             best = c.shape;
             time = us;
@@ -1455,19 +1456,20 @@ static int wide_shape_for(int M, int N, int K, bool gated, float* time) {
 
 // Whether 17 to 64 rows are the many-row kernel's, instead of the skinny kernels' (which take 64 rows up to k = 1024, 32 up to 2048)
 // and of the vendor library's beyond.  It loses where few workgroups walk a long k -- a turn of 128 k waits for a barrier, 0.14 us
-// and more -- and where the activation's rows, which every strip of columns reads again, outweigh its weight: 1024 columns at
-// k = 4096 (8.0 us of the library for 8.7, 64 rows 9.8 for 12.4), 64 x 4096 x 12288 (34.7 for 40.1), 64 x 2048 x 5632 (13.4 for
-// 18.2); up to 32 rows it holds on to k = 8192 (32 x 4096 x 5632 17.5 -> 15.8, 32 x 5120 x 8192 26.9 -> 26.0).
-// Against those: 24 x 6144 x 1024 8.0 -> 5.5 us, 32 x 6144 x 2048 16.1 -> 8.4, 64 x 6144 x 2048 13.2 -> 10.2, with gate and silu
-// 64 x 2 * 3072 x 1024 11.5 -> 6.4, 64 x 2 * 5632 x 2048 18.2 -> 14.3, 64 x 2 * 12288 x 4096 46.5 -> 40.6 (the library's product
-// and its activation's launch before); over 250 products 0.73 of the time (geometric mean, 0.43 to 1.06).  Above 34000 rows of
-// weight the library streams it faster (64 x 2 * 25600 x 5120: 106, 121).
+// and more -- and where the activation's rows, which every strip of columns reads again, outweigh its weight.  Measured on 768
+// products (the sizes of the tiles' fit above), time against those, geometric mean: up to 32 rows 0.4 to 0.85 up to k = 3072, with more than
+// 1024 columns 0.5 to 0.8 up to 4096 and, of up to 8192 rows of weight, 0.61 to 0.79 up to 8192; beyond 32 rows 0.42 to 0.84 up to 2048 and,
+// gated or of more than 1024 columns, 0.5 to 0.79 up to 3072, and up to 4096 0.64 to 0.93 with a gate and 0.8 to 0.9 without where there are 4096
+// columns.  Not beyond: few columns at long k take up to 1.6 of the library's time (48 x 2 * 464 x 4224 10 us for 7), and weights of
+// more than 32768 rows 1.03 to 1.16, from 24576 on 1.03 to 1.06 without a gate at k above 2048 (64 x 2 * 25600 x 5120: 106, 121).  All that this takes:
+// 0.69 (550 products, 0.37 to 1.24); 24 x 6144 x 1024 8.0 -> 5.8 us, 64 x 6144 x 2048 13.2 -> 10.2, with gate and silu 64 x 2 * 3072 x 1024
+// 11.5 -> 7.0, 64 x 2 * 12288 x 4096 46.5 -> 46.2 (the library's product and its activation's launch before).
 static bool few_wins(int M, int N, int K, bool gated) {
     const long long weight = (long long)N * (gated ? 2 : 1);
-    if (M <= 16 || M > 64 || weight > 34000) return false;
-    if (M <= 32) return K <= 2816 || (N > 1024 && (K <= 4096 || (K <= 8192 && weight <= 8192)));
-    if (K <= 2816) return K <= 2048 || gated || N > 1024;
-    return K <= 4096 && (gated ? N > 1024 && N <= 12288 : N >= 4096);
+    if (M <= 16 || M > 64 || weight > (gated || K <= 2048 ? 32768 : 24576)) return false;
+    if (M <= 32) return K <= 3072 || (N > 1024 && (K <= 4096 || (K <= 8192 && weight <= 8192)));
+    if (K <= 3072) return K <= 2048 || gated || N > 1024;
+    return K <= 4096 && (gated ? N > 1024 : N >= 4096);
 }
 
 // Whether the kernel takes these operands at all: whole blocks of k, 32-bit offsets, rows that start on 16 bytes.
@@ -1526,20 +1528,26 @@ extern "C" int mlr_gemm_heads(const void* a, long lda, long a_head, const void* 
 }
 
 // Whether 17 rows and more are this kernel's beside the vendor library (act: WIDE_*): up to 64 rows as `few_wins` says.  Beyond, the
-// library has the faster way on large products (60 GFLOP and more) on which this kernel's tiles do not come out evenly: below a
-// predicted 1.2 PFLOP/s.  (154 products of 97 to 2048 rows: 12 % less time than the library alone, geometric mean, where the better
-// of both would be 14 %; 0.53 to 1.18 of the library's time on the products that this takes.  2048 x 5120 x 25600: 525 us for the
-// library's 427; 1533 x 5120 x 25600: 345 for 513.)  An activation that would otherwise be a launch of its own, which reads the
-// products and writes its results at 4.5 TB/s, counts for the kernel.
+// library has the faster way
+//   - on large products (60 GFLOP and more) on which this kernel's tiles do not come out evenly: below a predicted 1.3 PFLOP/s;
+//   - on few outputs of a long k, which it cuts (128 x 792 x 11776: 21 us for 38);
+//   - on weights of more than 45000 rows while the rows are few (97 x 48000 x 3000: 0.9 of this kernel's time).
+// An activation makes no difference: in the epilogue it takes what its own launch does (1.4 us and 1.0 us a million outputs beside 2.3
+// and 0.88: an exponential and a division an output; 2048 x 2 * 12288 x 4096: 26 and 24 us).
+// Measured on 1840 products of 65 to 2048 rows (inner sizes drawn from 512 to 12000 and 512 to 60000 rows of weight, and the Qwen3
+// layers at 20 row counts), against the library and the activation's launch, geometric mean: drawn sizes 0.82 plain and 0.84 gated,
+// where the better of both would be 0.81 and 0.82; the Qwen3 layers 0.91 and 1.01 (0.89 and 0.98); of all that this takes 0.38 to 1.32.
+// (A prediction of the library's time from its bytes, flops and k, within 16 %, chose no better.)
 extern "C" int mlr_gemm_wide_wins(int M, int N, int K, int act) {
     const bool gated = act >= WIDE_SILU && act <= WIDE_CLAMPED;
     if (M <= 16 || N <= 0 || K <= 0 || !wide_takes(nullptr, nullptr, M, N, K, gated)) return 0;
     if (M <= 64) return few_wins(M, N, K, gated) ? 1 : 0;
+    const long long weight = (long long)N * (gated ? 2 : 1);
+    if ((K > 8192 && M * weight < (1 << 17)) || (M <= 128 && weight > 45000)) return 0;
     float time = 0.f;
     wide_shape_for(M, N, K, gated, &time);
-    const float gflop = 2e-9f * (float)M * (float)N * (float)K * (gated ? 2.f : 1.f);
-    const float launch = act == WIDE_PLAIN ? 0.f : 3.0f + 1e-6f * (float)M * (float)N * (gated ? 6.f : 4.f) / 4.5f;
-    return gflop < 60.f || time <= gflop / 1.2f + launch ? 1 : 0;
+    const float gflop = 2e-9f * (float)M * (float)weight * (float)K;
+    return gflop < 60.f || time <= gflop / 1.3f ? 1 : 0;
 }
 
 // out[M, N] = act of the products, act one of WIDE_SILU_ROUNDED .. (gated: w is [2N, K] = [gate; up]; limit and slope are
