@@ -410,11 +410,11 @@ class Kernels:
         """Whether the vendor library's first choice for a product of more than 64 rows adds in the many-row kernel's order, one chain
         over k.  A choice between two experts that lie within rounding turns on the last bit, so a model that routes takes the kernel
         only where nothing turns.  Compared bit by bit on 36 000 products of 65 to 8192 rows (library of ROCm 7.2): none of 2^18
-        to 2^23 outputs with k up to 8192 differs (16 000), none of up to 2^24 with k up to 2048 (7 000).  Outside, the library
+        to 2^23 outputs with k up to 8704 differs (17 000), none of up to 2^24 with k up to 2048 (7 000).  Outside, the library
         cuts k into parts or deals them out to workgroups: few outputs (333 x 768 x 2048), many (from 2^23.1 at k = 2560, 2^23.9 at
         2112; 1603 x 28736 x 6016), long k (from 8832 with 2^21 outputs, nearly all beyond 16384).  Where the library times its candidates (multiples of
         64 rows) it may choose one that cuts k, another one in another process: there this kernel's order is the lasting one."""
-        return 1 << 19 <= outputs < (1 << 24 if k <= 2048 else 1 << 23) and k <= 8192
+        return 1 << 19 <= outputs < (1 << 24 if k <= 2048 else 1 << 23) and k <= 8704
 
     # the epilogues of `gemm_activated` (csrc/gemm.hip, WIDE_*)
     WIDE_ACTS = {None: 0, "silu": 2, "gelu_tanh": 3, "relu": 4, "clamped": 5, "relu_squared": 6, "gelu_erf": 7}

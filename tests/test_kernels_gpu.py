@@ -439,7 +439,7 @@ def test_gemm_wide_tiles_and_epilogues(mnk):
 
 
 @pytest.mark.parametrize("m,n,kk", [(65, 8072, 8192), (67, 16000, 64), (75, 111800, 1984), (99, 80000, 8128), (130, 4040, 4032), (333, 1576, 8000),
-                                    (333, 25000, 8192), (509, 32800, 2048), (701, 760, 7360), (997, 536, 3328), (1001, 8376, 8192), (1499, 11100, 1088),
+                                    (333, 25000, 8192), (509, 32800, 2048), (701, 760, 7360), (997, 536, 3328), (1001, 8376, 8704), (70, 34944, 8704), (1499, 11100, 1088),
                                     (2047, 264, 2048), (2001, 4192, 8192), (2049, 8184, 2048), (4099, 2040, 5056), (8191, 1016, 8192), (8190, 2040, 1920)])
 def test_the_library_adds_alike_where_models_with_a_router_leave_it(m, n, kk):
     """Products inside and at the edges of `library_adds_alike`: the vendor library's own first choice has the many-row kernel's bits,
