@@ -37,7 +37,10 @@
 // exceeds it by more than 2^8 (probabilities then stay below 256, far from overflow; the quotient at the
 // end does not depend on the reference): raising it means rescaling 64 accumulators, and with 32 columns
 // in a wavefront some column would need it in nearly every tile otherwise.  The decision is taken per
-// column from the column's own scores, so a column's arithmetic does not depend on its neighbours.
+// column from the column's own scores, so a column's arithmetic does not depend on its neighbours.  It does depend on the
+// workgroup's width where that is two ways over the keys: with head size 128 a column of 128 has one reference and one chain for both
+// halves of its blocks, a column of 64 two that are merged, so the two round their probabilities otherwise (as key ranges do, below;
+// both are the step's choice, by its number of rows).
 // The sum of a column's probabilities is taken over their bfloat16 roundings, the values that the second
 // product multiplies.
 //

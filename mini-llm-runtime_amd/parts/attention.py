@@ -228,7 +228,8 @@ class GqaAttention:
                                                 split_keys=ctx.split_keys)
             # workgroups of 128 columns (half the loads a column of those of 64) when the batch fills the compute units with
             # them: one each, or two where they have four wavefronts (head size 128: 2048 tokens behind 8192 keys 295 us for
-            # 323 with 32 heads, two of 128 a unit; 237 for 204 with 16, one a unit); else of 64
+            # 323 with 32 heads, two of 128 a unit; 237 for 204 with 16, one a unit); else of 64.  (A token's result turns on this
+            # choice, as on that of key ranges, by the rounding of its probabilities: both follow the step's number of rows.)
             columns = 128 if m * s.q_heads >= (256 if s.head_dim == 128 else 128) * ctx.compute_units else 64
             big_factor = (columns // 16 if tiles
                           else 4 if k.prefill_attention_supported(*sizes, ctx.max_context) else 0)

@@ -834,6 +834,7 @@ def test_prompt_portions_of_head_size_128(hq, hkv, page, before, n, window, spli
         want[:, head], size[:, head] = w @ values[:, head // g].double(), w @ values[:, head // g].double().abs()
     # a probability is rounded to bfloat16 (2^-9 of itself, in numerator and denominator) and its score is a 32-bit sum; so is the result
     bound = (2.0 ** -8 + 1e-4) * size + 2.0 ** -8 * want.abs()
+    widths = []
     for columns in (128, 64):
         for cap in {columns // g, max(1, columns // g - 3)}:
             first = list(range(0, n, cap))
@@ -848,6 +849,13 @@ def test_prompt_portions_of_head_size_128(hq, hkv, page, before, n, window, spli
                 assert bool(((out.double().view(n, hq, d) - want).abs() <= bound).all()), (columns, cap)
                 assert before_out is None or torch.equal(out, before_out), (columns, cap)
                 before_out = out
+        widths.append(before_out.double().view(n, hq, d))
+    # the two widths round the same probabilities beside other references, each by at most 2^-9 of itself, and the sums of
+    # their roundings; the results to bfloat16
+    assert bool(((widths[0] - widths[1]).abs() <= (2.0 ** -7 + 2e-4) * size + 2.0 ** -8 * widths[0].abs()).all())
+    # over all results the two errors are about as large: one width is no less exact than the other
+    errors = [float((w - want).norm() / want.norm()) for w in widths]
+    assert max(errors) <= 1.1 * min(errors), errors
 
 
 @pytest.mark.parametrize("d", [128, 64])
