@@ -465,14 +465,6 @@ struct SkinnyEpilogue {
     float glu_slope;          //        y = g sigmoid(slope g) (u + 1); 0: y = silu(gate) up; -1: gelu_tanh(gate) up; -2: relu(gate) up
     int plain_act;            // a plain product's activation: 0 none, 1 relu(x)^2, 2 the exact gelu x Phi(x)
 };
-__device__ __forceinline__ float plain_activation(float x, int act) {
-    if (act == 1) {
-        x = fmaxf(x, 0.f);
-        return x * x;
-    }
-    return 0.5f * x * (1.0f + erff(x * 0.70710678118654752440f));
-}
-
 // PAIR: a workgroup owns `cols` (17..32) output columns, two strips side by side, the second one partly
 // used: for a number of columns that deals strips of 16 unevenly to the compute units (384 strips on 256
 // units take as long as 512), 24 columns a workgroup give every unit the same work.  The second strip
@@ -698,23 +690,13 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const __
             }
             float y = v[0];
             if (GATED) {
-                if (epi.glu_limit > 0.f) {
-                    const float gg = fminf(v[0], epi.glu_limit);
-                    const float uu = fminf(fmaxf(v[NW - 1], -epi.glu_limit), epi.glu_limit);
-                    y = (gg / (1.0f + expf(-epi.glu_slope * gg))) * (uu + 1.0f);
-                } else if (epi.glu_limit < -1.5f) {
-                    y = fmaxf(v[0], 0.f) * v[NW - 1];
-                } else if (epi.glu_limit < 0.f) {
-                    const float gg = v[0];
-                    y = 0.5f * gg * (1.0f + tanhf(0.7978845608028654f * (gg + 0.044715f * gg * gg * gg))) * v[NW - 1];
-                } else {
-                    y = (v[0] / (1.0f + expf(-v[0]))) * v[NW - 1];
-                }
+                if (epi.glu_limit > 0.f) y = clamped_glu(v[0], v[NW - 1], epi.glu_limit, epi.glu_slope);
+                else y = (epi.glu_limit < -1.5f ? gate_act<2>(v[0]) : epi.glu_limit < 0.f ? gate_act<1>(v[0]) : gate_act<0>(v[0])) * v[NW - 1];
             }
             if constexpr (!GATED && !OUT_FLOAT && EPI == EPI_NONE) {
                 if (epi.plain_act) {
-                    y = plain_activation(y, epi.plain_act);
-                    if constexpr (PAIR) v[1] = plain_activation(v[1], epi.plain_act);
+                    y = epi.plain_act == 1 ? plain_act<0>(y) : plain_act<1>(y);
+                    if constexpr (PAIR) v[1] = epi.plain_act == 1 ? plain_act<0>(v[1]) : plain_act<1>(v[1]);
                 }
             }
             y4[i][r] = y;

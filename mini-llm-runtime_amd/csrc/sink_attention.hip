@@ -763,9 +763,6 @@ __device__ __forceinline__ void load_to_lds(intx4 rsrc, uint32_t at, const __bf1
     const uint32_t lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)to);
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(at), "s"(rsrc) : "memory", "m0");
 }
-template <int LEFT> __device__ __forceinline__ void sink_arrive() {      // (the compiler does not follow loads that go to LDS)
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LEFT) : "memory");
-}
 
 template <int NKF, int NVT, bool SHARED, int STAGES>
 __global__ __launch_bounds__(512, 2) void sink_attention_rows_kernel(SinkArgs a, const int32_t* __restrict__ group_first,
@@ -938,8 +935,8 @@ __global__ __launch_bounds__(512, 2) void sink_attention_rows_kernel(SinkArgs a,
     int stage = 0;
     for (int i = 0; i < i_end; ++i) {
         // this wavefront's part of the tile is there, and behind the barrier everyone's; everyone is done with the tile before
-        if (i + STAGES - 2 < i_end) sink_arrive<S::LOADS * (STAGES - 2)>();
-        else sink_arrive<0>();
+        if (i + STAGES - 2 < i_end) wide_arrive<S::LOADS * (STAGES - 2)>();
+        else wide_arrive<0>();
         if (i + STAGES - 1 < i_end) ask(i + STAGES - 1, stage == 0 ? STAGES - 1 : stage - 1);
         clear(i, stage);
         if (wave * 16 < count * head_block) tile(tile_at(i), stage);      // (a wavefront without columns only brings rows)
