@@ -1511,14 +1511,16 @@ extern "C" int mlr_gemm_heads(const void* a, long lda, long a_head, const void* 
 
 // Whether 17 rows and more are this kernel's beside the vendor library (act: WIDE_*): up to 64 rows as `few_wins` says.  Beyond, the
 // library has the faster way
-//   - on large products (60 GFLOP and more) on which this kernel's tiles do not come out evenly: below a predicted 1.3 PFLOP/s;
+//   - on large products: of row counts whose plan it times (multiples of 64: the fastest of up to 32) from 40 GFLOP on -- up to 30 this
+//     kernel takes 0.88 of its time, to 60 1.00, to 120 1.06, beyond 1.11 --, of others from 60 on where this kernel's tiles do not come out
+//     evenly, below a predicted 1.3 PFLOP/s (it is 0.84, 0.94, 0.99 and 1.02 of the library's there; 1533 x 5120 x 25600 355 us for 518);
 //   - on few outputs of a long k, which it cuts (128 x 792 x 11776: 21 us for 38);
 //   - on weights of more than 45000 rows while the rows are few (97 x 48000 x 3000: 0.9 of this kernel's time).
 // An activation makes no difference: in the epilogue it takes what its own launch does (1.4 us and 1.0 us a million outputs beside 2.3
 // and 0.88: an exponential and a division an output; 2048 x 2 * 12288 x 4096: 26 and 24 us).
 // Measured on 1840 products of 65 to 2048 rows (inner sizes drawn from 512 to 12000 and 512 to 60000 rows of weight, and the Qwen3
 // layers at 20 row counts), against the library and the activation's launch, geometric mean: drawn sizes 0.82 plain and 0.84 gated,
-// where the better of both would be 0.81 and 0.82; the Qwen3 layers 0.91 and 1.01 (0.89 and 0.98); of all that this takes 0.38 to 1.32.
+// where the better of both would be 0.81 and 0.82; the Qwen3 layers 0.91 and 1.00 (0.89 and 0.98); of all that this takes 0.38 to 1.32.
 // (A prediction of the library's time from its bytes, flops and k, within 16 %, chose no better.)
 extern "C" int mlr_gemm_wide_wins(int M, int N, int K, int act) {
     const bool gated = act >= WIDE_SILU && act <= WIDE_CLAMPED;
@@ -1526,9 +1528,10 @@ extern "C" int mlr_gemm_wide_wins(int M, int N, int K, int act) {
     if (M <= 64) return few_wins(M, N, K, gated) ? 1 : 0;
     const long long weight = (long long)N * (gated ? 2 : 1);
     if ((K > 8192 && M * weight < (1 << 17)) || (M <= 128 && weight > 45000)) return 0;
+    const float gflop = 2e-9f * (float)M * (float)weight * (float)K;
+    if (M % 64 == 0) return gflop < 40.f ? 1 : 0;
     float time = 0.f;
     wide_shape_for(M, N, K, gated, &time);
-    const float gflop = 2e-9f * (float)M * (float)weight * (float)K;
     return gflop < 60.f || time <= gflop / 1.3f ? 1 : 0;
 }
 
