@@ -1522,14 +1522,15 @@ extern "C" int mlr_gemm_heads(const void* a, long lda, long a_head, const void* 
 // layers at 20 row counts), against the library and the activation's launch, geometric mean: drawn sizes 0.82 plain and 0.84 gated,
 // where the better of both would be 0.81 and 0.82; the Qwen3 layers 0.91 and 1.00 (0.89 and 0.98); of all that this takes 0.38 to 1.32.
 // (A prediction of the library's time from its bytes, flops and k, within 16 %, chose no better.)
-extern "C" int mlr_gemm_wide_wins(int M, int N, int K, int act) {
+// one_order: the sums must not turn on which plan the library's timing picks: timed row counts are judged as the others.
+extern "C" int mlr_gemm_wide_wins(int M, int N, int K, int act, int one_order) {
     const bool gated = act >= WIDE_SILU && act <= WIDE_CLAMPED;
     if (M <= 16 || N <= 0 || K <= 0 || !wide_takes(nullptr, nullptr, M, N, K, gated)) return 0;
     if (M <= 64) return few_wins(M, N, K, gated) ? 1 : 0;
     const long long weight = (long long)N * (gated ? 2 : 1);
     if ((K > 8192 && M * weight < (1 << 17)) || (M <= 128 && weight > 45000)) return 0;
     const float gflop = 2e-9f * (float)M * (float)weight * (float)K;
-    if (M % 64 == 0) return gflop < 40.f ? 1 : 0;
+    if (M % 64 == 0 && !one_order) return gflop < 40.f ? 1 : 0;
     float time = 0.f;
     wide_shape_for(M, N, K, gated, &time);
     return gflop < 60.f || time <= gflop / 1.3f ? 1 : 0;

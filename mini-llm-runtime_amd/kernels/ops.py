@@ -397,7 +397,8 @@ class Kernels:
         key = (rows, columns, k, act)
         wins = self._wide_choices.get(key)
         if wins is None:
-            wins = bool(self._lib("gemm").mlr_gemm_wide_wins(_c_int(rows), _c_int(columns), _c_int(k), _c_int(kind)))
+            wins = bool(self._lib("gemm").mlr_gemm_wide_wins(_c_int(rows), _c_int(columns), _c_int(k), _c_int(kind),
+                                                                   _c_int(1 if self.routed else 0)))
             if not self.library_gemm and rows > 64:
                 wins = k % 64 == 0 and rows * k < 2 ** 31 and weight_rows * k < 2 ** 31
             if len(self._wide_choices) >= WIDE_CHOICES_KEPT:
@@ -413,7 +414,8 @@ class Kernels:
         to 2^23 outputs with k up to 8704 differs (17 000), none of up to 2^24 with k up to 2048 (7 000).  Outside, the library
         cuts k into parts or deals them out to workgroups: few outputs (333 x 768 x 2048), many (from 2^23.1 at k = 2560, 2^23.9 at
         2112; 1603 x 28736 x 6016), long k (from 8832 with 2^21 outputs, nearly all beyond 16384).  Where the library times its candidates (multiples of
-        64 rows) it may choose one that cuts k, another one in another process: there this kernel's order is the lasting one."""
+        64 rows) it may choose one that cuts k, another one in another process: there this kernel's order is the lasting one, and a
+        model that routes takes it by the rule for other row counts."""
         return 1 << 19 <= outputs < (1 << 24 if k <= 2048 else 1 << 23) and k <= 8704
 
     # the epilogues of `gemm_activated` (csrc/gemm.hip, WIDE_*)

@@ -1609,3 +1609,14 @@ def test_a_position_beyond_the_block_table_has_no_page(dtype, rows):
         if p < inside:
             assert torch.equal(v_pages[int(table[s, p // page]), :, :, p % page].cpu(),
                                qkv[i, (hq + hkv) * d:].view(hkv, d).cpu())
+
+
+def test_models_with_a_router_do_not_turn_on_timed_plans():
+    """A large product of a row count whose library plan is chosen by timing: the library's for a model without a router, and by the rule
+    of any other row count, so in one order of sums, for a model with one."""
+    from mini_llm_runtime_amd.kernels import Kernels
+    plain, routed = Kernels(torch.bfloat16), Kernels(torch.bfloat16, routed=True)
+    for n, kk in [(2048, 8448), (4000, 4096), (8000, 2048)]:
+        assert not plain.wide_product(2048, n, kk)
+        assert routed.wide_product(2048, n, kk) == routed.wide_product(2047, n, kk)
+    assert plain.wide_product(2048, 2048, 2048) and routed.wide_product(2048, 2048, 2048)
