@@ -1620,3 +1620,15 @@ def test_models_with_a_router_do_not_turn_on_timed_plans():
         assert not plain.wide_product(2048, n, kk)
         assert routed.wide_product(2048, n, kk) == routed.wide_product(2047, n, kk)
     assert plain.wide_product(2048, 2048, 2048) and routed.wide_product(2048, 2048, 2048)
+
+
+@pytest.mark.parametrize("m,n,kk,act,taken", [
+    # (time of the many-row kernel over the library's and the activation's launch, where both were measured)
+    (900, 25600, 5120, "silu", False), (777, 12288, 4096, "silu", False),        # 1.19 and 1.27 while the epilogue's time was a gain
+    (2048, 12288, 4096, "silu", False), (2048, 4096, 12288, None, False), (512, 5120, 8192, None, False),    # 1.08, 1.15 and 1.22: plans that were timed
+    (128, 792, 11776, None, False), (97, 48000, 3008, None, False),              # 1.85 and 1.11: few outputs of a long k, a long weight
+    (64, 31368, 2176, None, False), (40, 29528, 3328, None, False), (24, 36000, 576, None, False),           # 1.06, 1.04: long weights beside few rows
+    (2048, 1024, 3072, None, True), (2048, 3072, 1024, "silu", True), (1533, 5120, 25600, None, True),       # 0.92, 0.90 and 0.69
+    (32, 12288, 1024, "silu", True), (64, 6144, 2048, None, True), (32, 4096, 8192, None, True)])
+def test_the_rule_between_the_kernel_and_the_library_follows_its_measurements(m, n, kk, act, taken):
+    assert kernels(torch.bfloat16).wide_product(m, n, kk, act) == taken
