@@ -9,7 +9,7 @@
 // Head size 128 (four wavefronts, two workgroups a compute unit): the blocks go to LDS by loads that do not pass registers, and
 // the loop over the blocks that a wavefront sees whole has nothing to check.  What bounds it is what a SIMD can issue for a tile
 // and how long a tile's chain is (first product, softmax, second product), not memory: per tile 16 matrix instructions (512
-// cycles), 58 vector and some 25 scalar ones; counters at 10 000 keys of context (kernel of 237 us): matrix cores 42 % of the
+// cycles), 49 vector and some 25 scalar ones; counters at 10 000 keys of context (kernel of 237 us): matrix cores 42 % of the
 // cycles, LDS 22 %, no bank conflicts.  Measured (16 query heads over 8, pages of 16; the kernel that staged through registers,
 // eight wavefronts of 128 columns, in brackets): 2048 tokens 32.7 us with 64 columns (42.5), behind 10 240 keys 201 (232);
 // 32 query heads over 8, 2048 tokens behind 8192 keys 292 us with 128 columns (332), 64 over 8, 1501 tokens 56.5 (77); 4096 tokens
@@ -33,10 +33,12 @@
 // is the key with bits 2 and 3 swapped, and the registers are neighbouring keys.  Either way one 16-byte read gives the
 // matching A operand.
 //
-// Softmax in the base-2 domain, 32-bit.  A column's reference maximum is only raised when a tile's maximum
-// exceeds it by more than 2^8 (probabilities then stay below 256, far from overflow; the quotient at the
+// Softmax in the base-2 domain, 32-bit.  A column's reference is the maximum of one of its tiles and is only raised when the
+// probabilities that a lane makes of a tile sum up to more than 2^8 (each then stays below that, far from overflow; the quotient at the
 // end does not depend on the reference): raising it means rescaling 64 accumulators, and with 32 columns
-// in a wavefront some column would need it in nearly every tile otherwise.  The decision is taken per
+// in a wavefront some column would need it in nearly every tile otherwise.  The sum is there anyway, so most tiles never take a
+// maximum: 49 vector instructions a tile for 58, and the exponentials need not wait for it (12 321 tokens of 16 heads in portions of
+// 2048: 0.6 % of the whole prompt, which the card's power bounds).  The decision is taken per
 // column from the column's own scores, so a column's arithmetic does not depend on its neighbours.  It does depend on the
 // workgroup's width where that is two ways over the keys: with head size 128 a column of 128 has one reference and one chain for both
 // halves of its blocks, a column of 64 two that are merged, so the two round their probabilities otherwise (as key ranges do, below;
@@ -65,7 +67,7 @@ typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 #define TILE_KEYS 32
 #define PAGE_IDS 2048
 #define VPITCH (BLOCK_KEYS + 8)        // elements per channel row of a staged block of values
-#define RAISE_BY 8.0f                  // base-2 exponent by which a tile must exceed the reference
+#define RAISE_AT 256.0f                // sum of a lane's probabilities in a tile from which the reference may be raised
 
 struct TileArgs {
     const __bf16* q;             // [M, q_heads, head_dim]
@@ -106,14 +108,6 @@ struct TileShape {
     static constexpr size_t merge_bytes = NQ * (size_t)NO * 64 * sizeof(float);
     static constexpr size_t lds_bytes = PAGE_IDS * sizeof(int32_t) + (kv_bytes > merge_bytes ? kv_bytes : merge_bytes);
 };
-
-// max(a, b, c) in one instruction (the compiler puts a canonicalising instruction before every fmaxf of a
-// matrix-core result; NaN never gets here: masked scores are -inf, others finite)
-__device__ __forceinline__ float max3(float a, float b, float c) {
-    float r;
-    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
 
 // This wavefront's loads to LDS and its LDS reads are done, and so are every other wavefront's (the compiler does not follow
 // loads that go to LDS).
@@ -207,29 +201,37 @@ __device__ __forceinline__ void tile_group(const TileArgs& a, int grp, int kvh, 
                     sc[t][i] = (key >= kbegin_c && key < kend_c) ? sc[t][i] : -INFINITY;
                 }
         }
-        // (the compiler does not count an asm among the readers of a matrix instruction's result, which must wait: eight passes,
-        // twelve slots; behind the mask it has seen to it)
-        if (interior) {
+        // (the sum is taken over the probabilities as the second product sees them, rounded to bfloat16, two
+        // at a time: v_dot2c_f32_bf16 with a pair of ones, half the instructions of single additions)
+        const bf16x2 ones = {(__bf16)1.0f, (__bf16)1.0f};
+        float psum;
+        auto probabilities = [&]() {
+            float sum[2] = {0.f, 0.f};                        // (two chains: each addition waits for the one before it)
 #pragma unroll
-            for (int t = 0; t < T; ++t) {
-                if (t == 0) asm volatile("s_nop 11" : "+v"(sc[t]));
-                else asm volatile("" : "+v"(sc[t]));
-            }
-        }
-        float mx = max3(sc[0][0], sc[0][1], sc[0][2]);
+            for (int t = 0; t < T; ++t)
 #pragma unroll
-        for (int t = 0; t < T; ++t) {
+                for (int m = 0; m < 2; ++m) {
 #pragma unroll
-            for (int i = t == 0 ? 3 : 0; i + 6 <= (t == 0 ? 15 : 12); i += 6)
-                mx = max3(mx, max3(sc[t][i], sc[t][i + 1], sc[t][i + 2]), max3(sc[t][i + 3], sc[t][i + 4], sc[t][i + 5]));
-            if (t == 0) mx = max3(mx, sc[t][15], sc[t][15]);
-            else mx = max3(mx, max3(sc[t][12], sc[t][13], sc[t][14]), sc[t][15]);
-        }
-        if (__builtin_amdgcn_ballot_w64(mx > raise_at) != 0) {
-            const float both = fmaxf(mx, __shfl_xor(mx, 32, 64)), full = both * c2;      // the column's maximum in this tile (c2 > 0)
-            // (the same in both lanes of a column, and the vote's own comparison: a column is raised by its own scores, not where a
-            // neighbour's vote lets a comparison that rounds otherwise pass; full alone may be -inf)
-            if (both > raise_at && full > m_ref) {
+                    for (int e = 0; e < 8; ++e) pf[t][m][e] = (__bf16)__builtin_amdgcn_exp2f(fmaf(sc[t][8 * m + e], c2, m_neg));
+#pragma unroll
+                    for (int e = 0; e < 8; e += 2)
+                        sum[m] = __builtin_amdgcn_fdot2_f32_bf16(bf16x2{pf[t][m][e], pf[t][m][e + 1]}, ones, sum[m], false);
+                }
+            psum = sum[0] + sum[1];
+        };
+        probabilities();
+        // A lane's sum beyond RAISE_AT says that some score may lie too far above the reference: only then the maximum is taken (in
+        // every tile it would be nine instructions, a wait for the first product's last result before anything else can begin, and a
+        // branch in front of the exponentials).  Both lanes of a column see both sums, so a column is raised by its own scores.
+        if (__builtin_amdgcn_ballot_w64(psum > RAISE_AT) != 0) {
+            const float most = fmaxf(psum, __shfl_xor(psum, 32, 64));
+            float mx = sc[0][0];
+#pragma unroll
+            for (int t = 0; t < T; ++t)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sc[t][i]);
+            const float full = fmaxf(mx, __shfl_xor(mx, 32, 64)) * c2;        // the column's maximum in this tile (c2 > 0)
+            if (most > RAISE_AT && full > m_ref) {
                 const float corr = __builtin_amdgcn_exp2f(m_ref - full);      // -inf - finite: 0
                 l_run *= corr;
 #pragma unroll
@@ -238,23 +240,9 @@ __device__ __forceinline__ void tile_group(const TileArgs& a, int grp, int kvh, 
                     for (int i = 0; i < 16; ++i) o[db][i] *= corr;
                 m_ref = full;
                 m_neg = -fmaxf(full, -1e30f);
-                raise_at = (full + RAISE_BY) / c2;
             }
+            probabilities();
         }
-        // (the sum is taken over the probabilities as the second product sees them, rounded to bfloat16, two
-        // at a time: v_dot2c_f32_bf16 with a pair of ones, half the instructions of single additions)
-        const bf16x2 ones = {(__bf16)1.0f, (__bf16)1.0f};
-        float psum = 0.f;
-#pragma unroll
-        for (int t = 0; t < T; ++t)
-#pragma unroll
-            for (int m = 0; m < 2; ++m) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) pf[t][m][e] = (__bf16)__builtin_amdgcn_exp2f(fmaf(sc[t][8 * m + e], c2, m_neg));
-#pragma unroll
-                for (int e = 0; e < 8; e += 2)
-                    psum = __builtin_amdgcn_fdot2_f32_bf16(bf16x2{pf[t][m][e], pf[t][m][e + 1]}, ones, psum, false);
-            }
         l_run += psum;
     };
 
