@@ -925,8 +925,38 @@ struct WideArgs {
     int lda, ldo, a_head, out_head;       // of the form with a product a head: row pitches of activation and output, and from head to head
 };
 
+#define QKV_HEAD 128              // channels of a head
+
+// The LDS of that form: the finished tile in the blocks' place, head by head, then every row's position, page and place in it, and
+// which eights of rows lie side by side in a page.
+template <class S>
+struct QkvTile {
+    static constexpr int PITCH = QKV_HEAD + 8, VPITCH = S::BM + 8;                 // of a row of a head; of a channel of a head of values
+    static constexpr int HEADS = S::BN / QKV_HEAD, PASSES = S::BM * HEADS * 8 / (64 * S::WAVES);
+    static constexpr int HEAD = S::BM * PITCH;                                      // elements of a head
+    static constexpr size_t tile_bytes = (size_t)HEADS * HEAD * sizeof(__bf16);
+    static constexpr size_t rows_at = tile_bytes > S::lds_bytes ? tile_bytes : S::lds_bytes;
+    static constexpr size_t lds_bytes = rows_at + (S::BM * 3 + S::BM / 8) * sizeof(int32_t);
+};
+
+// What the form with the heads' epilogue needs besides (QKV): w = [q heads; k heads; v heads] of 128 rows each.
+struct QkvArgs : WideArgs {
+    __bf16* q_out;                // [M, q_heads, 128]
+    __bf16* k_pages;              // [pages][kv_heads][page_size][128]
+    __bf16* v_pages;              // [pages][kv_heads][128][page_size]
+    const int32_t* block_table; const int32_t* slots; const int32_t* positions;
+    const float* q_norm_w; const float* k_norm_w; const float* rope;      // rope [positions][128]: cosines, sines; the others null: no norm
+    float eps;
+    int max_blocks, q_heads, kv_heads, page_size, write_cache;
+};
+
 // HEADS: head h multiplies its columns of wider rows by a weight of its own, out[m][h] = a[m][h] . w[h]^T; the tiles are counted
 // head by head.
+// QKV: the product of attention's q, k and v with what `qk_norm_rope_kv_vec_kernel` (rope_kv.hip) makes of it, the same bits: a tile
+// holds whole heads, so once it lies in LDS, rounded to bfloat16, eight lanes take a row of a head, norm and turn it and write the
+// queries to their matrix and the keys to their page; heads of values go to LDS transposed, so that eight rows of a channel are one
+// read and one store into their page.
+// The q/k/v matrix itself is never written: 2048 x 4096 x 1024 22.2 us for the 28.0 of the two launches, 19.1 of them the product.
 // FEW (17 to 64 rows): the sums of `gemm_skinny_kernel`, bit by bit, so that a row's results do not turn on whether 16 rows or 64
 // are computed with it: eight parts of k, of whole blocks, each one sum and added in ascending order, and 16 consecutive bytes of
 // every 32 of a row an instruction.  (The parts are also the more exact sum: worked out with normal operands, a
@@ -935,9 +965,11 @@ struct WideArgs {
 // for closing the parts, 0.4 for a gate), and 0.69 of the time of the kernels that took these rows before.
 // PAIRED: a turn is two blocks, and its operands are in registers before it begins: a small tile has few products a block, and
 // what its turns cost is the wait for the LDS and for the other wavefronts.
-template <int WM, int WN, int TM, int TN, int NS, bool OUT_FLOAT, bool GATED, bool HEADS = false, bool FEW = false, bool PAIRED = false>
-__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const WideArgs args) {
+template <int WM, int WN, int TM, int TN, int NS, bool OUT_FLOAT, bool GATED, bool HEADS = false, bool FEW = false, bool PAIRED = false, bool QKV = false>
+__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const std::conditional_t<QKV, QkvArgs, WideArgs> args) {
     using S = WideShape<WM, WN, TM, TN, NS>;
+    using Q = QkvTile<S>;
+    static_assert(!QKV || (!OUT_FLOAT && !GATED && !HEADS && !FEW && S::BN % QKV_HEAD == 0), "whole heads");
     constexpr int BM = S::BM, BN = S::BN, LOADS = S::LOADS;
     static_assert(!GATED || TN % 2 == 0, "gate and up tiles come in pairs");
     static_assert((!PAIRED || FEW) && (!FEW || !HEADS), "forms for 17 to 64 rows");
@@ -1070,6 +1102,23 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const WideAr
         __builtin_amdgcn_s_setprio(0);
     };
 
+    // QKV: thread t looks up where row m0 + t of the tile lies in the cache, behind the first loads of operands
+    int row_pos = 0, row_slot = 0, row_page = -1;
+    if constexpr (QKV) {
+        const int m = min(m0 + t, M - 1);
+        row_pos = args.positions[m];
+        row_slot = args.slots[m];
+    }
+    int32_t* row_lds = reinterpret_cast<int32_t*>(reinterpret_cast<unsigned char*>(wide_lds) + (QKV ? Q::rows_at : 0));   // [BM] positions, pages, places
+    auto find_page = [&]() {
+        if constexpr (QKV) {
+            if (t < BM) row_lds[t] = row_pos;                     // (the loop's barriers lie before its readers)
+            const int block = row_pos / args.page_size;
+            const int id = args.block_table[(size_t)row_slot * args.max_blocks + min(args.write_cache ? block : 0, args.max_blocks - 1)];
+            row_page = args.write_cache && block < args.max_blocks && m0 + t < M ? id : -1;
+        }
+    };
+
     if constexpr (PAIRED) {
         constexpr int PAIRS = NS / 2, LOADS_PAIR = 2 * LOADS;
         static_assert(NS % 2 == 0 && PAIRS >= 2, "whole pairs of blocks");
@@ -1163,6 +1212,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const WideAr
         for (int s = 0; s < NS; ++s)
 #pragma unroll
             for (int i = 0; i < LOADS; ++i) load(i, s, s);
+        find_page();
         wide_arrive<LOADS * (NS - 1)>();
         read_all(H0, 0);
         int stage = 0;
@@ -1198,6 +1248,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const WideAr
         for (int s = 0; s < blocks; ++s)
 #pragma unroll
             for (int i = 0; i < LOADS; ++i) load(i, s, s);
+        find_page();
         wide_arrive<0>();
         for (int s = 0; s < blocks; ++s) {
             read_all(H0, s);
@@ -1228,6 +1279,139 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const WideAr
                 else
 #pragma unroll
                     for (int r = 0; r < 4; ++r) if (n + r < N) o[r] = acc[i][j][r];
+            }
+        }
+        return;
+    }
+    if constexpr (QKV) {
+        // What counts here is the path for requests (16 bytes a lane take it 16 cycles a wavefront) and the instructions: the norm's
+        // weights are asked for once a thread, which stays with one head of the tile, and the rotation of its rows before the tile is
+        // put into LDS.
+        constexpr int LANES = 8, THREADS = 64 * S::WAVES, AHEAD = Q::PASSES < 4 ? Q::PASSES : 4;
+        constexpr int ROWS = THREADS / LANES / Q::HEADS;          // of a pass
+        static_assert(THREADS / LANES % Q::HEADS == 0 && Q::PASSES % AHEAD == 0, "a thread stays with one head");
+        typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4_t;
+        const int head0 = n0 / QKV_HEAD, all_heads = args.q_heads + 2 * args.kv_heads, turned = args.q_heads + args.kv_heads;
+        const int P = args.page_size, c = t % LANES, at = t / LANES % Q::HEADS, my_row = t / LANES / Q::HEADS, head = head0 + at;
+        const bool is_q = head < args.q_heads;
+        floatx4 co[AHEAD][2], si[AHEAD][2], wl[2], wh[2];
+        auto ask = [&](int pass0) {
+#pragma unroll
+            for (int p = 0; p < AHEAD; ++p) {
+                const float* cs = args.rope + (size_t)row_lds[my_row + (pass0 + p) * ROWS] * QKV_HEAD + 8 * c;
+#pragma unroll
+                for (int x = 0; x < 2; ++x) {
+                    co[p][x] = *reinterpret_cast<const floatx4*>(cs + 4 * x);
+                    si[p][x] = *reinterpret_cast<const floatx4*>(cs + 64 + 4 * x);
+                }
+            }
+        };
+        const float* w = is_q ? args.q_norm_w : args.k_norm_w;
+        const bool normed = w != nullptr;
+        if (head0 < turned) {
+            ask(0);
+            if (normed) {
+#pragma unroll
+                for (int x = 0; x < 2; ++x) {
+                    wl[x] = *reinterpret_cast<const floatx4*>(w + 8 * c + 4 * x);
+                    wh[x] = *reinterpret_cast<const floatx4*>(w + 64 + 8 * c + 4 * x);
+                }
+            }
+        }
+        // (the last operands are there since the last turn but one: behind the barrier everyone has read them)
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (t < BM) {                                             // (whole wavefronts)
+            const int place = row_pos % P;
+            row_lds[BM + t] = row_page;
+            row_lds[2 * BM + t] = place;
+            const int page_before = __shfl_up(row_page, 1, MLR_WAVE), place_before = __shfl_up(place, 1, MLR_WAVE);       // (by all lanes)
+            const bool follows = lane % 8 == 0 ? place % 8 == 0 && row_page >= 0 : page_before == row_page && place_before + 1 == place;
+            const uint64_t all = __builtin_amdgcn_ballot_w64(follows);
+            if (lane % 8 == 0) row_lds[3 * BM + t / 8] = (all >> lane & 0xff) == 0xff;
+        }
+        const int wave_head = wn * TN * 16 / QKV_HEAD, in_head = wn * TN * 16 % QKV_HEAD;         // a wavefront's columns are of one head
+        static_assert(QKV_HEAD % (TN * 16) == 0 && QKV_HEAD * Q::VPITCH <= Q::HEAD, "a wavefront's columns are of one head, whose values take its place");
+        __bf16* tile = wide_lds + wave_head * Q::HEAD;
+        typedef __attribute__((__vector_size__(2 * sizeof(uint32_t)))) uint32_t uint2_t;
+        const bool of_values = head0 + wave_head >= turned;
+        const uint32_t pick = lane & 1 ? 0x03020706u : 0x05040100u;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const bf16x4_t four = {(__bf16)acc[i][j][0], (__bf16)acc[i][j][1], (__bf16)acc[i][j][2], (__bf16)acc[i][j][3]};
+                if (!of_values) {
+                    *reinterpret_cast<bf16x4_t*>(tile + ((wm * TM + i) * 16 + li) * Q::PITCH + in_head + j * 16 + 4 * g) = four;
+                    continue;
+                }
+                // four channels of one row a lane become four rows of one channel, between the four lanes of a quad: halves with the
+                // lane two places away, then quarters with its neighbour
+                const uint2_t own = __builtin_bit_cast(uint2_t, four);
+                const uint32_t other = __builtin_amdgcn_mov_dpp(lane & 2 ? own[0] : own[1], 0x4e, 0xf, 0xf, true);
+                const uint32_t lo = lane & 2 ? other : own[0], hi = lane & 2 ? own[1] : other;
+                const uint2_t rows = {__builtin_amdgcn_perm(__builtin_amdgcn_mov_dpp(lo, 0xb1, 0xf, 0xf, true), lo, pick),
+                                      __builtin_amdgcn_perm(__builtin_amdgcn_mov_dpp(hi, 0xb1, 0xf, 0xf, true), hi, pick)};
+                *reinterpret_cast<uint2_t*>(tile + (in_head + j * 16 + 4 * g + (lane & 3)) * Q::VPITCH + (wm * TM + i) * 16 + (li & ~3)) = rows;
+            }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (head0 < turned) {                                     // queries and keys: eight lanes a row of a head
+#pragma unroll
+            for (int pass0 = 0; pass0 < Q::PASSES; pass0 += AHEAD) {
+                if (pass0 > 0) ask(pass0);
+#pragma unroll
+                for (int p = 0; p < AHEAD; ++p) {
+                    const int row = my_row + (pass0 + p) * ROWS;
+                    const __bf16* from = wide_lds + at * Q::HEAD + row * Q::PITCH + 8 * c;
+                    const bf16x8 lo = *reinterpret_cast<const bf16x8*>(from), hi = *reinterpret_cast<const bf16x8*>(from + 64);
+                    const int page = row_lds[BM + row], place = row_lds[2 * BM + row];
+                    float a[8], b[8], sum = 0.f;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        a[e] = (float)lo[e];
+                        b[e] = (float)hi[e];
+                        sum += squares(a[e], b[e]);
+                    }
+#pragma unroll
+                    for (int off = 1; off < LANES; off <<= 1) sum += __shfl_xor(sum, off, MLR_WAVE);
+                    if (normed) {
+                        const float scale = 1.0f / sqrtf(sum / (float)QKV_HEAD + args.eps);
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) {
+                            a[e] = (a[e] * scale) * wl[e / 4][e % 4];
+                            b[e] = (b[e] * scale) * wh[e / 4][e % 4];
+                        }
+                    }
+                    bf16x8 x8, y8;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        x8[e] = (__bf16)turn_x(a[e], b[e], co[p][e / 4][e % 4], si[p][e / 4][e % 4]);
+                        y8[e] = (__bf16)turn_y(a[e], b[e], co[p][e / 4][e % 4], si[p][e / 4][e % 4]);
+                    }
+                    if (m0 + row >= M || head >= turned || (!is_q && page < 0)) continue;
+                    __bf16* dst = is_q ? args.q_out + ((size_t)(m0 + row) * args.q_heads + head) * QKV_HEAD
+                                       : args.k_pages + (((size_t)page * args.kv_heads + head - args.q_heads) * P + place) * QKV_HEAD;
+                    *reinterpret_cast<bf16x8*>(dst + 8 * c) = x8;
+                    *reinterpret_cast<bf16x8*>(dst + 64 + 8 * c) = y8;
+                }
+            }
+        }
+        // values: a thread takes eight rows of a channel, one store where they are eight neighbouring places of a page (two eights of
+        // a channel side by side: with pages of sixteen, lanes that follow each other write bytes that do)
+        for (int v = max(turned - head0, 0); v < Q::HEADS && head0 + v < all_heads; ++v) {
+            __bf16* pages = args.v_pages + (size_t)(head0 + v - turned) * QKV_HEAD * P;
+            const size_t page_elems = (size_t)args.kv_heads * QKV_HEAD * P;
+#pragma unroll 2
+            for (int item = t; item < BM / 8 * QKV_HEAD; item += THREADS) {
+                const int d = (item >> 1) % QKV_HEAD, r0 = (item / (2 * QKV_HEAD) * 2 + (item & 1)) * 8;
+                const bf16x8 rows = *reinterpret_cast<const bf16x8*>(wide_lds + v * Q::HEAD + d * Q::VPITCH + r0);
+                const int page = row_lds[BM + r0], place = row_lds[2 * BM + r0];
+                if (row_lds[3 * BM + r0 / 8]) {
+                    *reinterpret_cast<bf16x8*>(pages + page * page_elems + (size_t)d * P + place) = rows;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (row_lds[BM + r0 + e] >= 0) pages[row_lds[BM + r0 + e] * page_elems + (size_t)d * P + row_lds[2 * BM + r0 + e]] = rows[e];
+                }
             }
         }
         return;
@@ -1416,18 +1600,23 @@ static int launch_wide_shape(int shape, WideArgs& args, bool out_float, bool gat
     }
 }
 
-// The shape with the least predicted time, and that time in microseconds.
-static int wide_shape_for(int M, int N, int K, bool gated, float* time) {
+// The predicted time of a shape in microseconds.
+static float wide_time(int shape, int M, int N, int K, bool gated) {
     const int units = compute_units() > 0 ? compute_units() : 256;
+    const WideCost& c = WIDE_COSTS[shape];
+    const int bn = gated ? c.bn / 2 : c.bn;
+    const long long tiles = (long long)((M + c.bm - 1) / c.bm) * ((N + bn - 1) / bn), slots = (long long)units * c.per_unit;
+    const long long left = tiles % slots;
+    const bool alone = c.per_unit == 2 && left > 0 && left <= units;          // the last tiles have a compute unit each
+    const float rounds = (float)(tiles / slots + (left > 0 && !alone ? 1 : 0));
+    return c.fixed + (rounds * c.all + (alone ? c.one : 0.f)) * (float)K * (1.0f / 1024.0f);
+}
+
+// The shape with the least predicted time, and that time.
+static int wide_shape_for(int M, int N, int K, bool gated, float* time) {
     int best = 0;
     for (int s = 0; s < WIDE_SHAPES; ++s) {
-        const WideCost& c = WIDE_COSTS[s];
-        const int bn = gated ? c.bn / 2 : c.bn;
-        const long long tiles = (long long)((M + c.bm - 1) / c.bm) * ((N + bn - 1) / bn), slots = (long long)units * c.per_unit;
-        const long long left = tiles % slots;
-        const bool alone = c.per_unit == 2 && left > 0 && left <= units;      // the last tiles have a compute unit each
-        const float rounds = (float)(tiles / slots + (left > 0 && !alone ? 1 : 0));
-        const float us = c.fixed + (rounds * c.all + (alone ? c.one : 0.f)) * (float)K * (1.0f / 1024.0f);
+        const float us = wide_time(s, M, N, K, gated);
         if (s == 0 || us < *time) {
             best = s;
             *time = us;
@@ -1534,6 +1723,99 @@ extern "C" int mlr_gemm_wide_wins(int M, int N, int K, int act, int one_order) {
     float time = 0.f;
     wide_shape_for(M, N, K, gated, &time);
     return gflop < 60.f || time <= gflop / 1.3f ? 1 : 0;
+}
+
+template <int WM, int WN, int TM, int TN, int NS>
+static int launch_qkv(QkvArgs& args, hipStream_t stream) {
+    using S = WideShape<WM, WN, TM, TN, NS>;
+    using Q = QkvTile<S>;
+    static_assert(Q::lds_bytes <= 160 * 1024, "the tile and its rows' places must fit the LDS");
+    static_assert(S::BM <= 64 * S::WAVES && S::BM * Q::HEADS * 8 % (64 * S::WAVES) == 0, "a thread a row, whole passes");
+    args.tiles_m = (args.M + S::BM - 1) / S::BM;
+    args.tiles_n = (args.N + S::BN - 1) / S::BN;
+    if ((long long)args.tiles_m * args.tiles_n > 0x7fffffffLL / 8) return -2;
+    auto* kernel = gemm_wide_kernel<WM, WN, TM, TN, NS, false, false, false, false, false, true>;
+    static const hipError_t allowed = hipFuncSetAttribute(
+        reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)Q::lds_bytes);
+    if (allowed != hipSuccess) return (int)allowed;
+    kernel<<<dim3(args.tiles_m * args.tiles_n), 64 * S::WAVES, Q::lds_bytes, stream>>>(args);
+    return (int)hipGetLastError();
+}
+
+// The tiles that hold whole heads: the one with the least predicted time, the heads' epilogue with it (3 us a tile of 256 x 128).
+static int qkv_shape_for(int M, int N, int K, float* time) {
+    const int units = compute_units() > 0 ? compute_units() : 256;
+    int best = -1;
+    for (const int s : {4, 5, 7, 9}) {
+        const WideCost& c = WIDE_COSTS[s];
+        const long long tiles = (long long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+        const float us = wide_time(s, M, N, K, false) + 3.f / (256 * 128) * (float)((tiles + units - 1) / units * c.bm * c.bn);
+        if (best < 0 || us < *time) {
+            best = s;
+            *time = us;
+        }
+    }
+    return best;
+}
+
+// Whether `mlr_gemm_qkv` is the way for these sizes: where the product is this kernel's anyway, and the tile of whole heads with its
+// epilogue takes no longer than the best tile and the other launch, 3 us and 0.6 a million outputs.  Measured (product + launch, one
+// launch): 2048 x 4096 x 1024 28.0, 22.2 us; 1024 x 4096 x 1024 19.7, 13.4; 333 x 6144 x 4096 38.9, 36.2; 700 x 6144 x 4096 50.4, 45.8;
+// 333 x 10240 x 5120 56.8, 52.5.  Not where narrower tiles win by more: 256 x 6144 x 4096 32.8, 39.7; 160 x 4096 x 1024 11, 11.
+extern "C" int mlr_gemm_qkv_wins(int M, int q_heads, int kv_heads, int K, int one_order) {
+    const int N = (q_heads + 2 * kv_heads) * QKV_HEAD;
+    if (M <= 64 || !mlr_gemm_wide_wins(M, N, K, WIDE_PLAIN, one_order)) return 0;
+    float time = 0.f, any = 0.f;
+    qkv_shape_for(M, N, K, &time);
+    wide_shape_for(M, N, K, false, &any);
+    return time <= any + 3.f + 0.6e-6f * (float)M * (float)N ? 1 : 0;
+}
+
+// attention's q, k and v = a . w^T, w [(q_heads + 2 kv_heads) * 128, K], of more than 64 rows, with the heads' norms (weights null: none),
+// the rotation of whole heads in split-half pairs by `rope` [positions][128] and the writes of keys and values into their pages:
+// the bits of `mlr_gemm_wide` followed by `mlr_qk_norm_rope_kv`.  shape: 4, 5, 7, 9, or -1 for the one with the least predicted time.
+// Returns -1 for sizes and operands that it does not take.
+extern "C" int mlr_gemm_qkv(const void* a, const void* w, int M, int K, void* q_out, void* k_pages, void* v_pages,
+                            const int32_t* block_table, int max_blocks, const int32_t* slots, const int32_t* positions,
+                            const float* q_norm_w, const float* k_norm_w, float eps, const float* rope, int q_heads, int kv_heads,
+                            int page_size, int write_cache, int shape, hipStream_t stream) {
+    if (M <= 0) return 0;
+    const uintptr_t starts = reinterpret_cast<uintptr_t>(q_out) | reinterpret_cast<uintptr_t>(k_pages) | reinterpret_cast<uintptr_t>(v_pages) |
+                             reinterpret_cast<uintptr_t>(q_norm_w) | reinterpret_cast<uintptr_t>(k_norm_w) | reinterpret_cast<uintptr_t>(rope);
+    if (q_heads <= 0 || kv_heads <= 0 || page_size <= 0 || max_blocks <= 0 || rope == nullptr || (q_norm_w == nullptr) != (k_norm_w == nullptr) ||
+        (starts & 15) != 0 || (page_size % 8 != 0) || K <= 0)
+        return -1;
+    const int N = (q_heads + 2 * kv_heads) * QKV_HEAD;
+    if (!wide_takes(a, w, M, N, K, false)) return -1;
+    QkvArgs args{};
+    args.a = (const __bf16*)a;
+    args.w = (const __bf16*)w;
+    args.M = M;
+    args.N = N;
+    args.K = K;
+    args.q_out = (__bf16*)q_out;
+    args.k_pages = (__bf16*)k_pages;
+    args.v_pages = (__bf16*)v_pages;
+    args.block_table = block_table;
+    args.slots = slots;
+    args.positions = positions;
+    args.q_norm_w = q_norm_w;
+    args.k_norm_w = k_norm_w;
+    args.rope = rope;
+    args.eps = eps;
+    args.max_blocks = max_blocks;
+    args.q_heads = q_heads;
+    args.kv_heads = kv_heads;
+    args.page_size = page_size;
+    args.write_cache = write_cache;
+    float time = 0.f;
+    switch (shape < 0 ? qkv_shape_for(M, N, K, &time) : shape) {
+        case 4: return launch_qkv<2, 4, 4, 2, 4>(args, stream);
+        case 5: return launch_qkv<4, 2, 3, 4, 3>(args, stream);
+        case 7: return launch_qkv<4, 2, 4, 4, 3>(args, stream);
+        case 9: return launch_qkv<2, 4, 8, 4, 2>(args, stream);
+        default: return -1;
+    }
 }
 
 // out[M, N] = act of the products, act one of WIDE_SILU_ROUNDED .. (gated: w is [2N, K] = [gate; up]; limit and slope are

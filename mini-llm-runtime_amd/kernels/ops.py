@@ -101,6 +101,10 @@ def _gemm_work(self, a, w, out, *rest, **kw):
     return _size(a) + _size(w) + _size(out), 2 * a.shape[0] * w.shape[0] * w.shape[1]
 
 
+def _gemm_qkv_work(self, a, w, q_out, *rest, **kw):
+    return _size(a) + _size(w) + a.shape[0] * w.shape[0] * a.element_size(), 2 * a.shape[0] * w.shape[0] * w.shape[1]
+
+
 def _rows_prenorm_work(self, h, delta, weight, out, ss):
     return 2 * _size(h) + _size(delta) + _size(out), 0
 
@@ -406,6 +410,23 @@ class Kernels:
             self._wide_choices[key] = wins
         return wins
 
+    def qkv_product(self, rows, q_heads, kv_heads, head_dim, k, page_size, *operands):
+        """Whether `gemm_qkv` is the way from a norm's output to queries and a cache of these sizes: heads of 128 channels, pages of
+        whole eights, a product that is the many-row kernel's anyway (`wide_product`) in a tile that holds whole heads, without
+        losing more by that tile than the launch it saves.  `operands`: tensors that must start on 16 bytes."""
+        if self.dtype != torch.bfloat16 or rows <= 64 or head_dim != 128 or page_size % 8 != 0 or not _on16(*operands):
+            return False
+        n = (q_heads + 2 * kv_heads) * head_dim
+        if not self.wide_product(rows, n, k):
+            return False
+        key = (rows, q_heads, kv_heads, k, "qkv")
+        wins = self._wide_choices.get(key)
+        if wins is None:
+            wins = bool(self._lib("gemm").mlr_gemm_qkv_wins(_c_int(rows), _c_int(q_heads), _c_int(kv_heads), _c_int(k),
+                                                            _c_int(1 if self.routed else 0))) or not self.library_gemm
+            self._wide_choices[key] = wins
+        return wins
+
     @staticmethod
     def library_adds_alike(outputs, k):
         """Whether the vendor library's first choice for a product of more than 64 rows adds in the many-row kernel's order, one chain
@@ -660,6 +681,32 @@ class Kernels:
                _c_float(eps), _p(rope), _c_int(m), _c_int(q_heads), _c_int(kv_heads), _c_int(head_dim),
                _c_int(page_size), _c_int(1 if write_cache else 0), _c_int(rot_dim), _c_int(1 if interleaved else 0),
                _stream()), "qk_norm_rope_kv")
+
+    @timed("gemm", _gemm_qkv_work)
+    def gemm_qkv(self, a, w, q_out, k_pages, v_pages, block_table, slots, positions, q_norm_w, k_norm_w, eps, rope, q_heads,
+                 kv_heads, head_dim, page_size, write_cache=True, shape=-1):
+        """`gemm` of attention's stacked q, k and v and `qk_norm_rope_kv` of the result in one launch, the same bits: heads of 128
+        channels turned whole in split-half pairs, for the sizes of `qkv_product`.  `shape`: the kernel's tile (4, 5, 7 or 9;
+        -1: the one with the least predicted time)."""
+        _need(self.dtype == torch.bfloat16 and head_dim == 128, "gemm_qkv: bfloat16, heads of 128 channels")
+        _tensor(a, "a", self.dtype, ndim=2)
+        m, k = a.shape
+        _tensor(w, "w", self.dtype, ((q_heads + 2 * kv_heads) * head_dim, k))
+        _tensor(q_out, "q_out", self.dtype, (m, q_heads * head_dim))
+        self._check_cache(k_pages, v_pages, kv_heads, head_dim, page_size)
+        _tensor(block_table, "block_table", torch.int32, ndim=2)
+        _tensor(slots, "slots", torch.int32, (m,))
+        _tensor(positions, "positions", torch.int32, (m,))
+        _need((q_norm_w is None) == (k_norm_w is None), "gemm_qkv: both norms or neither")
+        if q_norm_w is not None:
+            _tensor(q_norm_w, "q_norm_w", torch.float32, (head_dim,))
+            _tensor(k_norm_w, "k_norm_w", torch.float32, (head_dim,))
+        _tensor(rope, "rope", torch.float32, ndim=2)
+        _need(rope.shape[1] == head_dim, "gemm_qkv: the rotation must turn the whole head")
+        _ok(self._lib("gemm").mlr_gemm_qkv(
+            _p(a), _p(w), _c_int(m), _c_int(k), _p(q_out), _p(k_pages), _p(v_pages), _p(block_table), _c_int(block_table.shape[1]),
+            _p(slots), _p(positions), _p(q_norm_w), _p(k_norm_w), _c_float(eps), _p(rope), _c_int(q_heads), _c_int(kv_heads),
+            _c_int(page_size), _c_int(1 if write_cache else 0), _c_int(shape), _stream()), "gemm_qkv")
 
     @staticmethod
     def attention_partial_numel(rows, q_heads, head_dim, max_splits):

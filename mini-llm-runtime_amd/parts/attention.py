@@ -142,9 +142,7 @@ class GqaAttention:
     def forward(self, ctx, x, cache_id, write_cache=True):
         s = self.spec
         m = x.shape[0]
-        qkv = ctx.workspace.get("qkv", (m, (s.q_heads + 2 * s.kv_heads) * s.head_dim), x.dtype)
-        ctx.kernels.gemm(x, self.qkv, qkv)
-        attn = self._attend(ctx, qkv, cache_id, write_cache)
+        attn = self._project_and_attend(ctx, x, cache_id, write_cache)
         out = ctx.workspace.get("mixer_out", (m, s.hidden), x.dtype)
         ctx.kernels.gemm(attn, self.o, out)
         return out
@@ -169,23 +167,51 @@ class GqaAttention:
             kernels.profiler.next_work(*self._work)
             self._work = None
 
+    def _rotation(self, ctx, device):
+        s = self.spec
+        rotation = self.position.rotation(ctx.max_positions, device) if self.position is not None else None
+        if rotation is not None and not (2 <= rotation.dim <= s.head_dim and rotation.dim % 2 == 0
+                                         and rotation.table.shape[1] == rotation.dim):
+            raise PartError(f"the position part turns {rotation.dim} channels of a head of {s.head_dim}: must be "
+                            "even, at most the head, and as wide as its table")
+        return rotation
+
+    def _project_and_attend(self, ctx, x, cache_id, write_cache):
+        """The fused projection of x and what `_attend` makes of it; many rows in one launch up to the attention itself."""
+        s = self.spec
+        k = ctx.kernels
+        m = x.shape[0]
+        view = ctx.cache.kv_view(cache_id)
+        rotation = self._rotation(ctx, x.device)
+        norms = (self.q_norm.weight, self.k_norm.weight) if self.q_norm is not None else (None, None)
+        decode = ctx.single_tokens and write_cache and k.decode_fusion_supported(s.q_heads, s.kv_heads, s.head_dim, view.page_size)
+        if (not decode and rotation is not None and rotation.dim == s.head_dim and not rotation.interleaved
+                and k.qkv_product(m, s.q_heads, s.kv_heads, s.head_dim, x.shape[1], view.page_size, x, self.qkv, rotation.table,
+                                  *(w for w in norms if w is not None))):
+            self._start_work(ctx, x.element_size())
+            q = ctx.workspace.get("q", (m, s.q_heads * s.head_dim), x.dtype)
+            k.gemm_qkv(x, self.qkv, q, view.k_pages, view.v_pages, view.block_table, ctx.slots, ctx.positions, *norms,
+                       self.q_norm.eps if self.q_norm is not None else 0.0, rotation.table, s.q_heads, s.kv_heads, s.head_dim,
+                       view.page_size, write_cache)
+            return self._attend_cached(ctx, q, view)
+        qkv = ctx.workspace.get("qkv", (m, (s.q_heads + 2 * s.kv_heads) * s.head_dim), x.dtype)
+        k.gemm(x, self.qkv, qkv)
+        return self._attend(ctx, qkv, cache_id, write_cache)
+
+    def _start_work(self, ctx, element_size):
+        k = ctx.kernels
+        self._work = self._attention_work(ctx, element_size) if k.profiler is not None and not ctx.fixed_groups else None
+
     def _attend(self, ctx, qkv, cache_id, write_cache):
         """Norm of q and k, rotation, cache write and attention on the fused projection's output; the heads'
         outputs [B, q_heads * head_dim] (before the output projection)."""
         s = self.spec
         k = ctx.kernels
-        if k.profiler is not None and not ctx.fixed_groups:
-            self._work = self._attention_work(ctx, qkv.element_size())
-        else:
-            self._work = None
+        self._start_work(ctx, qkv.element_size())
         x = qkv
         m = qkv.shape[0]
         view = ctx.cache.kv_view(cache_id)
-        rotation = self.position.rotation(ctx.max_positions, x.device) if self.position is not None else None
-        if rotation is not None and not (2 <= rotation.dim <= s.head_dim and rotation.dim % 2 == 0
-                                         and rotation.table.shape[1] == rotation.dim):
-            raise PartError(f"the position part turns {rotation.dim} channels of a head of {s.head_dim}: must be "
-                            "even, at most the head, and as wide as its table")
+        rotation = self._rotation(ctx, x.device)
         rope = rotation.table if rotation is not None else None
         interleaved = rotation is not None and rotation.interleaved
         whole_split_half = rotation is None or (rotation.dim == s.head_dim and not rotation.interleaved)
@@ -215,7 +241,14 @@ class GqaAttention:
             self.k_norm.weight if self.k_norm is not None else None,
             self.q_norm.eps if self.q_norm is not None else 0.0, rope,
             s.q_heads, s.kv_heads, s.head_dim, view.page_size, write_cache, interleaved=interleaved)
-        attn = ctx.workspace.get("attn", (m, s.q_heads * s.head_dim), x.dtype)
+        return self._attend_cached(ctx, q, view)
+
+    def _attend_cached(self, ctx, q, view):
+        """Attention of queries that are normed and turned, over keys and values that are in their pages."""
+        s = self.spec
+        k = ctx.kernels
+        m = q.shape[0]
+        attn = ctx.workspace.get("attn", (m, s.q_heads * s.head_dim), q.dtype)
         if k.mfma_attention_supported(s.q_heads, s.kv_heads, s.head_dim, view.page_size):
             # prompt portions go to one of the LDS-staged kernels (the 32x32-tile one where it takes the
             # sizes), single tokens and short portions to the one that can split a token's keys over
