@@ -93,6 +93,7 @@ def _as_paged(spec):
 class StateSpec:
     shape: Tuple[int, ...]
     dtype: torch.dtype = torch.float32
+    paired: bool = False              # two rows a slot that take turns being the live one (`CacheManager.state_pairs`)
 
 
 @dataclass
@@ -270,7 +271,7 @@ class CacheManager:
         """(bytes of pages, of block tables, of state slabs) that a manager with these sizes allocates:
         per group of equal specs every tensor of the spec as [entries, pages + 1, *shape within a page]
         and a table [max_slots + 1, ceil(max_length / page size)] of int32; per `StateSpec` two slabs
-        [max_slots + 1, *shape] (live and staged)."""
+        [max_slots + 1, *shape] (live and staged), or one of pairs of rows."""
         groups = {}
         state = 0
         for spec in entry_specs:
@@ -363,9 +364,15 @@ class CacheManager:
         # State of fixed size: a live slab, which mixers read, and a staged one, into which they write the
         # state their step leads to; the staged rows of a step's requests become live when every layer has
         # run (`commit_state`), so a step that fails on the way leaves the live state as it was.
-        self._states, self._staged = {}, {}
+        # A paired entry has two rows a slot in one slab instead: a step reads the live one and writes the
+        # other, and a step that has run turns its requests' pairs round (`retire`) -- here, where the next
+        # step's rows are named, so that nothing is copied.
+        self._states, self._staged, self._pairs = {}, {}, {}
+        self._live_row = 2 * np.arange(max_slots + 1, dtype=np.int32)
         for cid, spec in enumerate(self.entry_specs):
-            if isinstance(spec, StateSpec):
+            if isinstance(spec, StateSpec) and spec.paired:
+                self._pairs[cid] = torch.zeros((2 * (max_slots + 1), *spec.shape), dtype=spec.dtype, device=self.device)
+            elif isinstance(spec, StateSpec):
                 self._states[cid] = torch.zeros((max_slots + 1, *spec.shape), dtype=spec.dtype, device=self.device)
                 self._staged[cid] = torch.zeros_like(self._states[cid])
         self._state_rows = [t[0].numel() * t.element_size() for t in self._states.values()]
@@ -398,6 +405,20 @@ class CacheManager:
         """[max_slots + 1, *shape]: where a mixer leaves the state that its step leads to, in the rows of the
         step's slots (every slot of the step, in every step that writes the entry)."""
         return self._staged[cache_id]
+
+    def state_pairs(self, cache_id):
+        """[2 (max_slots + 1), *shape]: a paired entry's rows.  A step finds the state of a request in the row that
+        `state_rows` names and leaves the state it leads to in the other row of the pair, row ^ 1 (every request of
+        the step, in every step that writes the entry)."""
+        return self._pairs[cache_id]
+
+    def state_rows(self, slots):
+        """The live rows of the slots (an int32 vector, the same for every paired entry).  The scratch request's is
+        never written and stays zero."""
+        return self._live_row[slots]
+
+    def has_pairs(self):
+        return bool(self._pairs)
 
     def has_state(self):
         return bool(self._states)
@@ -442,13 +463,15 @@ class CacheManager:
         return sum(t.numel() * t.element_size() for t in self._tables)
 
     def state_bytes(self):
-        return sum(t.numel() * t.element_size() for t in list(self._states.values()) + list(self._staged.values()))
+        return sum(t.numel() * t.element_size() for t in (*self._states.values(), *self._staged.values(), *self._pairs.values()))
 
     # -- requests --------------------------------------------------------------------------------
     def acquire_slot(self):
         slot = self.book.acquire_slot()
         for state in self._states.values():
             state[slot].zero_()
+        for pairs in self._pairs.values():
+            pairs[self._live_row[slot]].zero_()
         return slot
 
     def release_slot(self, slot):
@@ -473,9 +496,12 @@ class CacheManager:
         return first
 
     def retire(self, slots):
-        """After a step: give back what windows have passed.  The device tables are brought up
-        to date before the next step (commit)."""
-        return self.book.retire(slots)
+        """After a step: what it wrote becomes the requests' state (paired entries), and what windows have passed is
+        given back.  The device tables are brought up to date before the next step (commit)."""
+        passed = self.book.retire(slots)
+        if self._pairs:
+            self._live_row[slots] ^= 1
+        return passed
 
     def sync_tables(self):
         """Changed rows of the block tables go to the device through a pinned staging copy of the table, with

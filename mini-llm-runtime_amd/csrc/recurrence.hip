@@ -5,7 +5,9 @@
 // portions and single tokens; a request's tokens are consecutive rows of the batch (`seg_first`, `seg_count`,
 // one entry a request of the step).  The live state of a request is read from `live + slot * stride`, the
 // state that the step leads to is written to `stage + slot * stride` (the engine makes it live when every
-// layer has run).  Every sum is taken in an order that depends on the token's own data only, so a token's
+// layer has run).  Where both are one slab, its rows come in pairs: `slots` names the live row of a pair and the other one, slot ^ 1,
+// is written, so that making it live is a matter of which row the next step names (a copy of every state otherwise: 48 requests of
+// eight layers of 1 MB, 133 us of a step of 1730).  Every sum is taken in an order that depends on the token's own data only, so a token's
 // result does not depend on how its request was cut into steps or on what else the batch holds.
 //
 // The delta rule (`delta_rule_kernel`) is the same walk with a write that first takes back what the state already
@@ -34,6 +36,7 @@ struct ConvArgs {
     const float* live; float* stage; long state_stride;
     const int32_t* slots; const int32_t* positions;
     int rows, channels, taps, silu, write_state;
+    int pair;                                  // a slot's written row is slot ^ pair
 };
 
 #define CONV_MAX_TAPS 8
@@ -64,7 +67,7 @@ __global__ __launch_bounds__(256) void causal_conv_kernel(ConvArgs a) {
     if (last && a.write_state) {
 #pragma unroll
         for (int d = 0; d < CONV_MAX_TAPS - 1; ++d) {
-            if (d < before) a.stage[(size_t)slot * a.state_stride + (size_t)(before - 1 - d) * a.channels + c] = in[d];
+            if (d < before) a.stage[(size_t)(slot ^ a.pair) * a.state_stride + (size_t)(before - 1 - d) * a.channels + c] = in[d];
         }
     }
 }
@@ -113,7 +116,7 @@ __global__ __launch_bounds__(256) void causal_conv_rows_kernel(ConvArgs a) {
             for (int d = 0; d < before; ++d)
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
-                    a.stage[(size_t)slot * a.state_stride + (size_t)(before - 1 - d) * a.channels + c + e] = in[d][e];
+                    a.stage[(size_t)(slot ^ a.pair) * a.state_stride + (size_t)(before - 1 - d) * a.channels + c + e] = in[d][e];
         }
     }
 }
@@ -163,6 +166,7 @@ struct ScanArgs {
     const float* rope; const int32_t* positions; int rot_dim;
     float* piece_state;                        // [pieces][heads][N][V]: L_c after the first pass, S_c after the second
     float* piece_decay;                        // [pieces][heads][N]: A_c
+    int pair;                                  // a slot's written row is slot ^ pair
 };
 
 #define SCAN_COLS 64
@@ -191,7 +195,7 @@ __global__ __launch_bounds__(256) void linear_recurrence_kernel(ScanArgs a) {
     const int col = col0 + j;
     const int N = a.N, V = a.V;
     const int qk_head = head / a.heads_per_group;
-    const size_t state_at = (size_t)slot * a.state_stride + (size_t)head * N * V;
+    const size_t state_at = (size_t)slot * a.state_stride + (size_t)head * N * V, stage_at = (size_t)(slot ^ a.pair) * a.state_stride + (size_t)head * N * V;
     const size_t piece_at = ((size_t)seg * a.heads + head) * N * V;
     float S[NR], A[NR];
 #pragma unroll
@@ -273,7 +277,7 @@ __global__ __launch_bounds__(256) void linear_recurrence_kernel(ScanArgs a) {
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
             const int i = part * NR + r;
-            if (i < N) a.stage[state_at + (size_t)i * V + col] = S[r];
+            if (i < N) a.stage[stage_at + (size_t)i * V + col] = S[r];
         }
     }
     if (MODE == 1) {
@@ -301,7 +305,7 @@ __global__ void piece_states_kernel(ScanArgs a, int pieces) {
         const float last = a.piece_state[(size_t)c * per + e];
         a.piece_state[(size_t)c * per + e] = S;
         S = a.piece_decay[(size_t)c * a.heads * a.N + hi] * S + last;
-        if (a.write_state && (c + 1 == pieces || a.slots[a.seg_first[c + 1]] != slot)) a.stage[(size_t)slot * a.state_stride + e] = S;
+        if (a.write_state && (c + 1 == pieces || a.slots[a.seg_first[c + 1]] != slot)) a.stage[(size_t)(slot ^ a.pair) * a.state_stride + e] = S;
     }
 }
 
@@ -332,6 +336,7 @@ struct DeltaArgs {
     int heads, heads_per_group, N, V, write_state, unit_norm;
     float q_scale, unit_eps;
     int decay_per_head;                        // one decay for all key channels of a head
+    int pair;                                  // a slot's written row is slot ^ pair
 };
 
 // Where the log decay of (row, head, key channel i) lies.
@@ -363,7 +368,7 @@ __global__ __launch_bounds__(64) void delta_rule_kernel(DeltaArgs a) {
     const int col = col0 + j;
     const int N = a.N, V = a.V;
     const int qk_head = head / a.heads_per_group;
-    const size_t state_at = (size_t)slot * a.state_stride + (size_t)head * N * V;
+    const size_t state_at = (size_t)slot * a.state_stride + (size_t)head * N * V, stage_at = (size_t)(slot ^ a.pair) * a.state_stride + (size_t)head * N * V;
     float S[NR];
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
@@ -435,7 +440,7 @@ __global__ __launch_bounds__(64) void delta_rule_kernel(DeltaArgs a) {
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
             const int i = part * NR + r;
-            if (i < N) a.stage[state_at + (size_t)i * V + col] = S[r];
+            if (i < N) a.stage[stage_at + (size_t)i * V + col] = S[r];
         }
     }
 }
@@ -720,7 +725,7 @@ __global__ __launch_bounds__(256, AHEAD ? 1 : 3) void delta_chunk_scan_kernel(De
     int chunk0 = 0;
     for (int s = 0; s < seg; ++s) chunk0 += (a.seg_count[s] + C - 1) / C;
     const size_t step = (size_t)a.heads * delta_chunk_floats(N, V);
-    const size_t state_at = (size_t)slot * a.state_stride + (size_t)head * N * V;
+    const size_t state_at = (size_t)slot * a.state_stride + (size_t)head * N * V, stage_at = (size_t)(slot ^ a.pair) * a.state_stride + (size_t)head * N * V;
     const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
     floatx4 S[NT];
     bool mine[NT];
@@ -852,7 +857,7 @@ __global__ __launch_bounds__(256, AHEAD ? 1 : 3) void delta_chunk_scan_kernel(De
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int ch = (wave + 4 * j) * 16 + b4 + i;
-                if (ch < N) a.stage[state_at + (size_t)ch * V + col] = S[j][i];
+                if (ch < N) a.stage[stage_at + (size_t)ch * V + col] = S[j][i];
             }
 }
 
@@ -902,7 +907,7 @@ int mlr_causal_conv(const void* x, long x_stride, const float* w, const float* b
     if (rows <= 0 || channels <= 0) return 0;
     if (taps < 1 || taps > CONV_MAX_TAPS) return -1;
     ConvArgs a{(const elem_t*)x, x_stride, w, b, (elem_t*)out, out_stride, live, stage, state_stride, slots, positions,
-               rows, channels, taps, silu, write_state};
+               rows, channels, taps, silu, write_state, live == stage};
 #if MLR_BF16
     const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     // A walk of CONV_ROWS rows takes 11 us however few they are.  The line lies where one value a thread takes as long: 256
@@ -947,7 +952,7 @@ int mlr_linear_recurrence(const void* q, long q_stride, const void* k, long k_st
     ScanArgs a{(const elem_t*)q, q_stride, (const elem_t*)k, k_stride, (const elem_t*)v, v_stride, log_decay, decay_stride,
                v_scale, v_scale_stride, skip, out, live, stage, state_stride, seg_first, seg_count, slots, heads,
                heads_per_group, n_keys, n_values, decay_per_channel, write_state, q_scale, silu, rope, positions, rot_dim, piece_state,
-               piece_decay};
+               piece_decay, live == stage};
     if ((piece_state == nullptr) != (piece_decay == nullptr)) return -2;
     const int nr = (n_keys + SCAN_PARTS - 1) / SCAN_PARTS;
     if (nr <= 8) return launch_scan<8, 16>(a, segments, rows == segments, stream);
@@ -981,7 +986,7 @@ int mlr_delta_rule(const void* q, long q_stride, const void* k, long k_stride, c
         return -1;
     DeltaArgs a{(const elem_t*)q, q_stride, (const elem_t*)k, k_stride, (const elem_t*)v, v_stride, log_decay, beta_raw,
                 beta_stride, out, live, stage, state_stride, seg_first, seg_count, slots, heads, heads_per_group, n_keys,
-                n_values, write_state, unit_norm, q_scale, unit_eps, decay_per_head};
+                n_values, write_state, unit_norm, q_scale, unit_eps, decay_per_head, live == stage};
     int parts = n_keys > 128 ? 4 : n_keys > 64 ? 2 : 1;
     if (n_values <= 16 && parts < 4) parts = 4;
     else if (n_values <= 32 && parts < 2) parts = 2;
@@ -1018,7 +1023,7 @@ int mlr_delta_rule_chunked(const void* q, long q_stride, const void* k, long k_s
         return -1;
     DeltaChunkArgs g{{(const elem_t*)q, q_stride, (const elem_t*)k, k_stride, (const elem_t*)v, v_stride, log_decay, beta_raw,
                       beta_stride, out, live, stage, state_stride, seg_first, seg_count, slots, heads, heads_per_group, n_keys,
-                      n_values, write_state, unit_norm, q_scale, unit_eps, decay_per_head},
+                      n_values, write_state, unit_norm, q_scale, unit_eps, decay_per_head, live == stage},
                      chunk_first, chunk_count, scratch};
     if ((reinterpret_cast<uintptr_t>(scratch) & 15) != 0) return -1;
     const int C = DELTA_CHUNK, Np = delta_padded(n_keys);

@@ -40,6 +40,7 @@ struct ChunkArgs {
     const float* rope; const int32_t* positions;
     int rot_dim, chunk, heads, heads_per_group, N, V, write_state, silu;
     float q_scale;
+    int pair;                                  // a slot's written row is slot ^ pair (1 where live and stage are one slab of pairs of rows)
 };
 
 #define LOG2E 1.4426950408889634f
@@ -223,7 +224,7 @@ __global__ __launch_bounds__(256) void chunk_states_kernel(ChunkArgs a) {
             }
         }
     }
-    if (a.write_state) a.stage[at] = S;
+    if (a.write_state) a.stage[(size_t)(slot ^ a.pair) * a.state_stride + ((size_t)head * a.N + n) * a.V + v] = S;
 }
 
 // Outputs: one workgroup per 64 rows of a chunk, head and VB value channels.  The rows' queries lie in LDS; the state's
@@ -434,7 +435,7 @@ int mlr_decayed_recurrence_chunks(const void* q, long q_stride, const void* k, l
         return -1;
     ChunkArgs a{(const __bf16*)q, q_stride, (const __bf16*)k, k_stride, (const __bf16*)v, v_stride, log_decay, out, live, stage,
                 state_stride, slots, seg_first, seg_count, chunk_first, chunk_count, chunk_state, rope, positions, rot_dim, chunk,
-                heads, heads_per_group, n_keys, n_values, write_state, silu, q_scale};
+                heads, heads_per_group, n_keys, n_values, write_state, silu, q_scale, live == stage};
     return silu ? launch_chunks<3>(a, segments, chunks, stream) : launch_chunks<1>(a, segments, chunks, stream);
 }
 

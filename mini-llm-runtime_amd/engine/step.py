@@ -86,7 +86,7 @@ class Runner:
         plan = lambda workspace, pages: MemoryPlan(
             weights=model.arena.planned if model.arena is not None else model.weight_bytes(),
             kv_pages=pages[0], block_tables=pages[1], state=pages[2], workspace=Workspace.plan_bytes(workspace),
-            metadata=5 * 4 * self.max_batch_tokens + 8, library_scratch=LIBRARY_GEMM_WORKSPACE if uses_library else 0)
+            metadata=6 * 4 * self.max_batch_tokens + 8, library_scratch=LIBRARY_GEMM_WORKSPACE if uses_library else 0)
         auto = max_tokens is None
         if auto and device_budget_bytes is None:
             device_budget_bytes = 0
@@ -138,10 +138,11 @@ class Runner:
         # split attention keeps its partial results within what was planned for them
         self.ctx.partial_budget = workspace_plan.get(("attn_partial", torch.float32))
         self.ctx.status = self._status if self.check_finite else None
-        # one vector a step: token ids, positions, slots (a value a token), wanted rows, and -- for a model that
-        # keeps state per request -- one slot per entry
-        self._upload = Uploader(5 * self.max_batch_tokens, self.device)
-        self._meta = torch.empty(5 * self.max_batch_tokens, dtype=torch.int32, device=self.device)
+        # one vector a step: token ids, positions, slots and, for a model with paired state, the requests' live rows of
+        # it (a value a token), wanted rows, and -- for a model that keeps other state per request -- one slot per entry
+        self._lanes = 4 if self.cache.has_pairs() else 3
+        self._upload = Uploader(6 * self.max_batch_tokens, self.device)
+        self._meta = torch.empty(6 * self.max_batch_tokens, dtype=torch.int32, device=self.device)
         self.poisoned = False
         self.steps = 0
         # steps of few tokens are launch-bound: after a first eager run a step's shape is captured once
@@ -258,13 +259,13 @@ class Runner:
             for n, want in shape:
                 rows.extend(base + w for w in want)
                 base += n
-            # ids | positions | slots | one slot per entry (these change from step to step) | wanted rows (fixed)
-            n_seg = len(shape)
-            meta = torch.empty(3 * total + n_seg + max(len(rows), 1), dtype=torch.int32, device=self.device)
+            # ids | positions | slots (| live rows) | one slot per entry (these change from step to step) | wanted rows (fixed)
+            n_seg, per_token = len(shape), self._lanes * total
+            meta = torch.empty(per_token + n_seg + max(len(rows), 1), dtype=torch.int32, device=self.device)
             if rows:
-                meta[3 * total + n_seg:3 * total + n_seg + len(rows)] = torch.tensor(rows, dtype=torch.int32,
+                meta[per_token + n_seg:per_token + n_seg + len(rows)] = torch.tensor(rows, dtype=torch.int32,
                                                                                       device=self.device)
-            state = dict(meta=meta, upload=Uploader(3 * total + n_seg, self.device), graph=None, logits=None, runs=0,
+            state = dict(meta=meta, upload=Uploader(per_token + n_seg, self.device), graph=None, logits=None, runs=0,
                          rows=len(rows), groups={}, keep=None, eager=False)
             self._graphs[sig] = state
             while len(self._graphs) > self.max_graphs:
@@ -273,7 +274,7 @@ class Runner:
             self._graphs[sig] = self._graphs.pop(sig)        # most recently used last
         meta = state["meta"]
         rows_of, segments = self._rows(entries, arrays, first, fill, fill_first)
-        n_seg = len(segments)
+        n_seg, per_token = len(segments), self._lanes * total
         state["upload"].send(np.concatenate([rows_of.ravel(), np.fromiter((seg[0] for seg in segments), np.int32, n_seg)]),
                              meta)
         if state["graph"] is not None:
@@ -283,11 +284,12 @@ class Runner:
         ctx.begin_step()
         ctx.n_tokens = total
         ctx.token_ids, ctx.positions, ctx.slots = meta[0:total], meta[total:2 * total], meta[2 * total:3 * total]
-        ctx.segment_slots = meta[3 * total:3 * total + n_seg]
+        ctx.state_rows = meta[3 * total:per_token] if self._lanes == 4 else None
+        ctx.segment_slots = meta[per_token:per_token + n_seg]
         ctx.segments = segments
         ctx.single_tokens = total == len(segments)
         r = state["rows"]
-        want_rows = meta[3 * total + n_seg:3 * total + n_seg + r] if r else None
+        want_rows = meta[per_token + n_seg:per_token + n_seg + r] if r else None
         if state["eager"]:                                # a shape whose capture did not hold
             ctx.max_context = max(p0 + n for (_, _, n, p0) in segments)
             return self.model.forward(ctx, want_rows)
@@ -297,7 +299,8 @@ class Runner:
         if state["runs"] == 1:                            # first time: eager, sizes the scratch buffers
             return self.model.forward(ctx, want_rows)
         # The capture runs the step more than once: eagerly (the reference), then twice as a replay of the
-        # fresh graph.  Running a step again writes the same keys and values into the same pages; state of
+        # fresh graph.  Running a step again writes the same keys and values into the same pages, and the same rows of
+        # paired state from the same live ones; other state of
         # fixed size, which a step ADVANCES, is put back to where the step found it before every further run,
         # so that it has advanced exactly once when this returns.
         before = self.cache.snapshot_state()
@@ -316,7 +319,7 @@ class Runner:
             self.graph_failures += 1
             ctx.fixed_groups = None
             ctx.begin_step()
-            ctx.segment_slots = meta[3 * total:3 * total + n_seg]
+            ctx.segment_slots = meta[per_token:per_token + n_seg]
             ctx.max_context = max(p0 + n for (_, _, n, p0) in segments)
             self.cache.restore_state(before)
             return self.model.forward(ctx, want_rows)
@@ -451,8 +454,9 @@ class Runner:
         return ids.astype(np.int32)
 
     def _rows(self, entries, arrays, first, fill=0, fill_first=False):
-        """(token ids | positions | slots of the step's rows as int32 [3, rows], the segments (slot, first row,
-        tokens, first position)); `fill` rows of the scratch request (token 0 at position 0) in front or behind."""
+        """(token ids | positions | slots of the step's rows as int32 [3, rows], or with the live rows of paired state [4, rows],
+        the segments (slot, first row, tokens, first position)); `fill` rows of the scratch request (token 0 at position 0) in
+        front or behind."""
         total = sum(len(a) for a in arrays) + fill
         scratch = self.cache.scratch_slot
         if total <= 4 * (len(entries) + fill):
@@ -471,8 +475,9 @@ class Runner:
             if fill and not fill_first:
                 segments += [(scratch, len(ids) + i, 1, 0) for i in range(fill)]
                 ids, pos, slot_of = ids + [0] * fill, pos + [0] * fill, slot_of + [scratch] * fill
-            return np.array([ids, pos, slot_of], dtype=np.int32), segments
-        rows = np.empty((3, total), dtype=np.int32)
+            lanes = [ids, pos, slot_of] if self._lanes == 3 else [ids, pos, slot_of, self.cache.state_rows(slot_of)]
+            return np.array(lanes, dtype=np.int32), segments
+        rows = np.empty((self._lanes, total), dtype=np.int32)
         segments, at = [], 0
         if fill and fill_first:
             rows[0:2, :fill], rows[2, :fill] = 0, scratch
@@ -488,6 +493,8 @@ class Runner:
         if fill and not fill_first:
             rows[0:2, at:], rows[2, at:] = 0, scratch
             segments += [(scratch, at + i, 1, 0) for i in range(fill)]
+        if self._lanes == 4:
+            rows[3] = self.cache.state_rows(rows[2])
         return rows, segments
 
     def step(self, entries: List[Entry]):
@@ -533,8 +540,10 @@ class Runner:
             ctx.segments = segments
             ctx.single_tokens = total == len(entries)
             ctx.max_context = max(p0 + n for (_, _, n, p0) in segments)
-            want_rows = self._meta[3 * total:3 * total + r] if r else None
-            ctx.segment_slots = self._meta[3 * total + r:3 * total + r + len(segments)] if stateful else None
+            per_token = self._lanes * total
+            ctx.state_rows = self._meta[3 * total:per_token] if self._lanes == 4 else None
+            want_rows = self._meta[per_token:per_token + r] if r else None
+            ctx.segment_slots = self._meta[per_token + r:per_token + r + len(segments)] if stateful else None
             logits = self.model.forward(ctx, want_rows)
             self.cache.retire(slots)
             self.steps += 1

@@ -1069,6 +1069,9 @@ class Kernels:
 
     @staticmethod
     def _check_state(live, stage, offset, count):
+        """States that are read from row slots[r] of `live` and written to that row of `stage`; where both are one slab, its rows
+        come in pairs: `slots` names the live row of a pair and the other one, slot ^ 1, is written."""
+        _need(live.data_ptr() != stage.data_ptr() or live.shape[0] % 2 == 0, "a slab of pairs of rows has an even number of them")
         for name, t in (("live", live), ("stage", stage)):
             _need(isinstance(t, torch.Tensor) and t.is_cuda and t.dtype is torch.float32 and t.dim() == 2
                   and t.is_contiguous(), f"{name}: the state must be float32 [slots, floats] on the GPU")

@@ -5,8 +5,8 @@ recurrence per head,
 token by token from the state that earlier steps left (`Kernels.linear_recurrence`); they differ in where q, k,
 v and the decay a come from and in what happens to o.  The delta rule's write first takes back what the state
 holds for the token's key (`Kernels.delta_rule`).  The state of a request lives in the cache manager's
-slots (`StateSpec`): read from the live rows, written to the staged ones, which become live when every layer of
-the step has run."""
+slots (a paired `StateSpec`): read from the live row of a slot's pair, written to the other one, which becomes live when every
+layer of the step has run."""
 from __future__ import annotations
 
 import torch
@@ -92,7 +92,7 @@ class GatedLinearAttention:
 
     def cache_spec(self):
         s = self.spec
-        return StateSpec((s.heads * s.head_dim * s.value_dim,), torch.float32)
+        return StateSpec((s.heads * s.head_dim * s.value_dim,), torch.float32, paired=True)
 
     def libraries(self):
         return ["gemm", "recurrence", "elementwise"]
@@ -122,9 +122,9 @@ class GatedLinearAttention:
         a, b = self.qk_width, 2 * self.qk_width
         c = b + self.v_width
         o = ws.get("recurrent_out", (m, self.v_width), torch.float32)
+        state = ctx.cache.state_pairs(cache_id)
         _recurrence(ctx, s.heads * s.head_dim * s.value_dim, s.heads, s.head_dim,
-                    proj[:, :a], proj[:, a:b], proj[:, b:c], log_decay, o, ctx.cache.state_view(cache_id),
-                    ctx.cache.state_stage(cache_id), 0, ctx.slots, s.heads, s.head_dim,
+                    proj[:, :a], proj[:, a:b], proj[:, b:c], log_decay, o, state, state, 0, ctx.state_rows, s.heads, s.head_dim,
                     s.value_dim, q_scale=float(s.head_dim) ** -0.5, write_state=write_cache)
         y = ws.get("recurrent_normed", (m, self.v_width), x.dtype)
         k.gated_part_norm(o, proj[:, c:], self.norm, y, s.value_dim, float(s.eps), gate_first=False, gate_kind="silu")
@@ -174,7 +174,7 @@ class Mamba2:
         self.norm, self.o = weights["norm"], weights["o"]
 
     def cache_spec(self):
-        return StateSpec((self.state_floats + (self.spec.conv_taps - 1) * self.channels,), torch.float32)
+        return StateSpec((self.state_floats + (self.spec.conv_taps - 1) * self.channels,), torch.float32, paired=True)
 
     def libraries(self):
         return ["gemm", "recurrence", "elementwise"]
@@ -196,17 +196,17 @@ class Mamba2:
         k.gemm(x, self.w_in, proj)
         inner, bc = self.inner, self.bc
         z, xbc, raw = proj[:, :inner], proj[:, inner:inner + self.channels], proj[:, inner + self.channels:]
-        live, stage = ctx.cache.state_view(cache_id), ctx.cache.state_stage(cache_id)
+        pairs = ctx.cache.state_pairs(cache_id)
         conv = ws.get("mamba_conv", (m, self.channels), x.dtype)
-        k.causal_conv(xbc, self.conv, self.conv_bias, conv, live, stage, self.state_floats, ctx.slots, ctx.positions,
+        k.causal_conv(xbc, self.conv, self.conv_bias, conv, pairs, pairs, self.state_floats, ctx.state_rows, ctx.positions,
                       silu=True, write_state=write_cache)
         dt = ws.get("mamba_dt", (m, s.heads), torch.float32)
         log_decay = ws.get("log_decay", (m, s.heads), torch.float32)
         k.mamba_step(raw, self.dt_bias, self.a_log, dt, log_decay)
         y = ws.get("recurrent_out", (m, inner), torch.float32)
         _recurrence(ctx, self.state_floats, s.heads, s.state,
-                    conv[:, inner + bc:], conv[:, inner:inner + bc], conv[:, :inner], log_decay, y, live, stage, 0,
-                    ctx.slots, s.heads, s.state, s.value_dim, heads_per_group=s.heads // s.groups,
+                    conv[:, inner + bc:], conv[:, inner:inner + bc], conv[:, :inner], log_decay, y, pairs, pairs, 0,
+                    ctx.state_rows, s.heads, s.state, s.value_dim, heads_per_group=s.heads // s.groups,
                     v_scale=dt, skip=self.skip, write_state=write_cache)
         normed = ws.get("recurrent_normed", (m, inner), x.dtype)
         k.gated_part_norm(y, z, self.norm, normed, inner // s.norm_groups, float(s.eps), gate_first=True, gate_kind="silu")
@@ -256,7 +256,7 @@ class DecayedLinearAttention:
 
     def cache_spec(self):
         s = self.spec
-        return StateSpec((s.heads * s.head_dim * s.value_dim,), torch.float32)
+        return StateSpec((s.heads * s.head_dim * s.value_dim,), torch.float32, paired=True)
 
     def libraries(self):
         chunks = ["recurrence_chunks"] if self.proj is not None and self.proj.dtype == torch.bfloat16 else []
@@ -294,7 +294,7 @@ class DecayedLinearAttention:
         c = b + self.v_width
         o = ws.get("recurrent_out", (m, self.v_width), torch.float32)
         q, kk, v = proj[:, :a], proj[:, a:b], proj[:, b:c]
-        live, stage = ctx.cache.state_view(cache_id), ctx.cache.state_stage(cache_id)
+        pairs = ctx.cache.state_pairs(cache_id)
         turns = self._turns(ctx, x.device)
         more = dict(q_scale=float(s.k_scale), write_state=write_cache, activation=s.activation, **turns)
         state = s.heads * s.head_dim * s.value_dim
@@ -304,13 +304,13 @@ class DecayedLinearAttention:
             few, (c_first, c_count, c_n), _ = ctx.token_groups(SHORT, PIECE // SHORT)
             _, (first, count, n), _ = ctx.token_groups(SHORT, WHOLE // SHORT)
             if n:
-                k.decayed_recurrence_chunks(q, kk, v, self._log_decay, o, live, stage, 0, first, count, n, ctx.slots, c_first, c_count,
+                k.decayed_recurrence_chunks(q, kk, v, self._log_decay, o, pairs, pairs, 0, first, count, n, ctx.state_rows, c_first, c_count,
                                             c_n, PIECE, ws.get("recurrent_pieces", (c_n * state,), torch.float32), s.heads,
                                             s.head_dim, s.value_dim, **more)
             if few[2]:
-                k.linear_recurrence(q, kk, v, self._log_decay, o, live, stage, 0, *few, ctx.slots, s.heads, s.head_dim, s.value_dim, **more)
+                k.linear_recurrence(q, kk, v, self._log_decay, o, pairs, pairs, 0, *few, ctx.state_rows, s.heads, s.head_dim, s.value_dim, **more)
         else:
-            _recurrence(ctx, state, s.heads, s.head_dim, q, kk, v, self._log_decay, o, live, stage, 0, ctx.slots, s.heads, s.head_dim,
+            _recurrence(ctx, state, s.heads, s.head_dim, q, kk, v, self._log_decay, o, pairs, pairs, 0, ctx.state_rows, s.heads, s.head_dim,
                         s.value_dim, **more)
         y = ws.get("recurrent_normed", (m, self.v_width), x.dtype)
         k.gated_part_norm(o, proj[:, c:], self.norm, y, self.v_width if s.norm == "row" else s.value_dim, float(s.eps),
@@ -413,7 +413,7 @@ class DeltaRule:
         self.dt_bias, self.a_log, self.norm, self.o = weights["dt_bias"], weights["A_log"], weights["norm"], weights["o"]
 
     def cache_spec(self):
-        return StateSpec((self.state_floats + (self.spec.conv_taps - 1) * self.channels,), torch.float32)
+        return StateSpec((self.state_floats + (self.spec.conv_taps - 1) * self.channels,), torch.float32, paired=True)
 
     def libraries(self):
         return ["gemm", "recurrence", "elementwise"]
@@ -449,9 +449,9 @@ class DeltaRule:
         ws = ctx.workspace
         proj = ws.get("delta_proj", (m, self.proj.shape[0]), x.dtype)
         k.gemm(x, self.proj, proj)
-        live, stage = ctx.cache.state_view(cache_id), ctx.cache.state_stage(cache_id)
+        pairs = ctx.cache.state_pairs(cache_id)
         conv = ws.get("delta_conv", (m, self.channels), x.dtype)
-        k.causal_conv(proj[:, :self.channels], self.conv, None, conv, live, stage, self.state_floats, ctx.slots, ctx.positions,
+        k.causal_conv(proj[:, :self.channels], self.conv, None, conv, pairs, pairs, self.state_floats, ctx.state_rows, ctx.positions,
                       silu=True, write_state=write_cache)
         # the decays: 32-bit sums of a projection (one a head, or a low-rank pair's second product a key channel), then
         # softplus and the head's rate
@@ -485,10 +485,10 @@ class DeltaRule:
             # a request's chunks in their order; the float engine stays with one order of sums a token
             (c_first, c_count, c_n), _, _ = ctx.token_groups(DELTA_CHUNK, 0)
             scratch = ws.get("delta_chunks", (k.delta_chunk_floats(c_n, s.heads, s.head_dim, s.value_dim),), torch.float32)
-            k.delta_rule_chunked(conv[:, :a], conv[:, a:b], conv[:, b:], log_decay, beta, o, live, stage, 0, first, count, n,
-                                 ctx.slots, c_first, c_count, c_n, scratch, s.heads, s.head_dim, s.value_dim, **more)
+            k.delta_rule_chunked(conv[:, :a], conv[:, a:b], conv[:, b:], log_decay, beta, o, pairs, pairs, 0, first, count, n,
+                                 ctx.state_rows, c_first, c_count, c_n, scratch, s.heads, s.head_dim, s.value_dim, **more)
         else:
-            k.delta_rule(conv[:, :a], conv[:, a:b], conv[:, b:], log_decay, beta, o, live, stage, 0, first, count, n, ctx.slots,
+            k.delta_rule(conv[:, :a], conv[:, a:b], conv[:, b:], log_decay, beta, o, pairs, pairs, 0, first, count, n, ctx.state_rows,
                          s.heads, s.head_dim, s.value_dim, **more)
         y = ws.get("recurrent_normed", (m, self.v_width), x.dtype)
         k.gated_part_norm(o, gate, self.norm, y, s.value_dim, float(s.eps), gate_first=False,

@@ -45,7 +45,9 @@ A mixer with state of fixed size (cache_spec() -> StateSpec) reads a request's l
 ctx.cache.state_view(cache_id)[slot] and leaves the state its step leads to in
 ctx.cache.state_stage(cache_id)[slot], for every slot of the step (when write_cache).  The staged rows become
 live when every layer of the step has run, so a step that fails on the way leaves the live state as it was.
-ctx.segment_slots holds the step's slots as a device vector (one a segment).
+ctx.segment_slots holds the step's slots as a device vector (one a segment).  A StateSpec(.., paired=True) keeps two rows a
+slot in ctx.cache.state_pairs(cache_id) instead: a token's request has its live state in row ctx.state_rows[token] (device int32), the
+mixer leaves the state its step leads to in row ^ 1, and nothing is copied to make it live.
 
 A part may set the class attribute `graph_safe = True` when what it launches depends only on the step's
 SHAPE -- how many tokens each entry brings (ctx.n_tokens, the lengths in ctx.segments, ctx.single_tokens,
