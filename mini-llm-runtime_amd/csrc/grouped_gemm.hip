@@ -266,7 +266,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(GroupedArgs g) {
     }
 }
 
-// Experts with many rows each (inner sizes in multiples of 64): 32 x 32 tiles of v_mfma_f32_32x32x16_bf16 out of LDS blocks
+// Experts (inner sizes in multiples of 64): 32 x 32 tiles of v_mfma_f32_32x32x16_bf16 out of LDS blocks
 // of 64 k, NS of them, brought by loads that do not pass through registers (`buffer_load_dwordx4 .. lds`).  A workgroup of
 // WM x WN wavefronts, each TM x TN tiles, owns 32 WM TM sorted rows of one expert and 32 WN TN of its weight's rows.  The weight
 // is the instruction's first operand, so a lane ends up with four consecutive columns of one row (lane = 32 h + i: row i of
@@ -360,7 +360,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void experts_wide_kernel(GroupedAr
     // The products of k step ks; between them, when READ, the reads of the next step out of block `from` and, when LOAD, the loads
     // of block kb into `into`.  The scheduling barriers keep it so.
     auto products = [&](int ks, bool do_read, int from, bool do_load, int kb, int into) {
-        constexpr int OPERANDS = TM + TN, STEPS = TN * TM, PER = (OPERANDS + STEPS - 2) / (STEPS - 1), PER_L = (LOADS + STEPS - 1) / STEPS;
+        constexpr int OPERANDS = TM + TN, STEPS = TN * TM, PER = STEPS == 1 ? OPERANDS : (OPERANDS + STEPS - 2) / (STEPS > 1 ? STEPS - 1 : 1), PER_L = (LOADS + STEPS - 1) / STEPS;
         __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int s = 0; s < STEPS; ++s) {
@@ -499,7 +499,14 @@ static int launch_experts_wide(const GroupedArgs& g, hipStream_t stream) {
 struct ExpertsCost { int bm, bn; float round, all; };
 static const ExpertsCost EXPERTS_COSTS[] = {{128, 128, 5.32f, 9.03f}, {128, 192, 6.74f, 12.02f}, {128, 256, 7.25f, 14.68f}, {192, 256, 9.80f, 21.20f}};
 
+// Fewer rows an expert than fill such tiles half: what counts is the weight's way from memory, so narrow tiles, two workgroups on a
+// compute unit, and five or six blocks on their way: 32 x 64 while an expert's rows fit 32, 64 x 64 while they fit 64.  Measured on
+// 126 products of 8 to 64 experts with 1 to 127 rows each (uneven; 704 to 6144 k, 768 to 12288 rows of weight out of memory) against the
+// kernel that stages through registers, which took all of them before: up to 20 rows 0.83 of its time, to 55 0.81, beyond, in the
+// tiles above, 0.60 (the bits are the same).  16 experts, 192 rows: 1408 x 2048 gated 27.4 -> 23.4 us, 2048 x 704 15.8 -> 12.0 (the
+// weights alone 19 and 10); 8 experts of 64 rows, 2816 x 2048 gated 44.7 -> 28.0.
 static int experts_shape_for(int M, int N, int K, int groups) {
+    if ((long)M < 56L * groups) return (long)M <= 20L * groups ? 4 : 5;
     const int units = compute_units() > 0 ? compute_units() : 256;
     int best = 0;
     float least = 0.f;
@@ -529,6 +536,8 @@ static int run_experts_wide(int shape, const GroupedArgs& g, hipStream_t stream)
         case 1: return launch_experts_wide<4, 2, 1, 3, 3>(g, stream);
         case 2: return launch_experts_wide<2, 4, 2, 2, 3>(g, stream);
         case 3: return launch_experts_wide<2, 4, 3, 2, 2>(g, stream);
+        case 4: return launch_experts_wide<1, 2, 1, 1, 6>(g, stream);
+        case 5: return launch_experts_wide<2, 2, 1, 1, 5>(g, stream);
         default: return -1;
     }
 }
@@ -748,9 +757,8 @@ int mlr_grouped_gemm(const void* a, long lda, long a_group, const void* w, long 
     GroupedArgs g{(const elem_t*)a, lda, a_group, (const elem_t*)w, w_group, out, ldo, out_group, offsets, gather,
                   M, N, K, groups, act, out_float, limit, slope};
 #if MLR_BF16
-    // experts with many rows each: the large tiles (below 128 rows an expert most of a tile would be padding; the products a
-    // head, with inner sizes of 128 to 512, are faster on the small one)
-    if ((long)M >= 128L * groups && experts_wide_takes(g, a_rows)) return run_experts_wide(experts_shape_for(M, N, K, groups), g, stream);
+    // rows by expert (the products a head, with inner sizes of 128 to 512, are faster on the small tile below)
+    if (experts_wide_takes(g, a_rows)) return run_experts_wide(experts_shape_for(M, N, K, groups), g, stream);
     if (offsets != nullptr && (long)M >= 256L * groups && N >= 128) {
         const int row_tiles = (M + 127) / 128 + (offsets ? groups : 0);
         if (row_tiles > 65535 || groups > 65535) return -2;
@@ -769,7 +777,7 @@ int mlr_grouped_gemm(const void* a, long lda, long a_group, const void* w, long 
     return (int)hipGetLastError();
 }
 
-// For tests and measurements: the products of experts with many rows in a given shape (0 .. 3).
+// For tests and measurements: the products of experts in a given shape (0 .. 5).
 int mlr_experts_wide(const void* a, const void* w, void* out, const int32_t* offsets, const int32_t* gather, int M, int N, int K,
                      int groups, int act, int shape, long a_rows, hipStream_t stream) {
 #if MLR_BF16
