@@ -13,19 +13,15 @@
 // `head_mix_attention_kernel`: one workgroup a token, any sizes, both engines; tiles of 64 keys at absolute multiples
 // of 64, so a token's sums and their order follow from its own position alone.
 //
-// On the matrix cores (bfloat16), four query heads a kv head, 1, 2 or 4 of those, keys and values of 128 channels: `head_mix_walk_kernel`, one
-// walk over the keys; `head_mix_walk_finish_kernel` where the keys are dealt out in ranges.
-//
-// Other sizes on the matrix cores, three launches over groups of up to NQ consecutive tokens of a request:
+// On the matrix cores (bfloat16), three launches over groups of up to NQ consecutive tokens of a request:
 //   `head_scores_kernel`   e = exp(s) of every (token, key, head) into scratch, and the sums of e;
 //   `head_mix_values_kernel`  weights e / sum, mixed over the heads by one product with `mix`, times the values;
 //   `head_mix_finish_kernel`  the shares of the key ranges added, turned back, gated.
-// A mixed weight needs the finished sums of ALL heads, so the weights cannot be mixed on the first walk over the keys; the
-// one-walk form keeps every head's sums over every kv head's values instead, kv_heads times the work of the second
-// product.  Scores are bounded by the cap, so exp(s) is taken without a running maximum (caps up to 60: exp(60) times
+// A mixed weight needs the finished sums of ALL heads, so the weights cannot be mixed on the first walk over the keys
+// (a walk that keeps every head's sums over every kv head's values instead does kv_heads times the work of the second
+// product).  Scores are bounded by the cap, so exp(s) is taken without a running maximum (caps up to 60: exp(60) times
 // 2^24 keys fits 32 bits) and nothing is ever rescaled.
 #include "common.h"
-#include <type_traits>
 
 struct HeadMixArgs {
     const elem_t* q; long q_stride;            // q[m * q_stride + head * key_dim + d]
@@ -589,430 +585,6 @@ __global__ __launch_bounds__(256) void head_mix_finish_kernel(HeadMixArgs a, Til
     }
 }
 
-// ---- one walk over the keys -----------------------------------------------------------------------------------
-//   O[h, g](i) = sum_j exp(s_h(i, j)) v_g(j)   for every head h and every kv head g,
-//   o_h(i)     = sum_h' mix[h, h'] / (sum_j exp(s_h'(i, j)) + exp(sink)) O[h', kv(h)](i)
-// The exponentials never leave the workgroup, are rounded to bfloat16 once, and the heads are mixed in 32-bit at the end.  One
-// workgroup of eight wavefronts: a group of NQ tokens (4, or a single one) x a range of keys, in blocks of BK keys.
-//   The scores of a block as D[key][row], row = (head, token) of one kv head's tile of 16 (a single token: all heads, of which the
-//   columns of a key's own kv head are kept): a lane has four keys of one row, which go to LDS as one access.
-//   Then O as D[row][channel] += P[row][key] V[key][channel], a wavefront 16 KV of the KV 128 value channels: register r of
-//   lane block b is head r of a kv head, of token b (a single token: of kv head b), so all heads of a token lie in one lane
-//   and mixing them needs no exchange.
-// Values come straight from the pages (a load is 8 lines of the cache); keys, of which an operand's load would touch 16 half lines, go
-// to LDS past the registers, each wavefront's own: a load is four whole rows, piece p of row r at place p ^ r.  What bounds it is
-// the path of a compute unit for requests, 64 bytes a cycle: 128 KB for a block of 64 keys of four kv heads; that is why four tokens
-// share it.  Measured (16 heads over 4 of 128 channels, pages of 16; the other matrix-core form in brackets): a prompt of 700 tokens 28.6 us
-// (48.1), 1400 49.2 (81.9), 2500 122 (119), 40 tokens behind 2400 keys 23 (43), 512 behind 8000 143 (143); 700 tokens beside 32 single
-// ones of 100 to 1500 keys 39 us in its two launches (87 in six).  With the keys' operands straight from the pages 35 for the 28.6.
-struct WalkArgs {
-    const int32_t* group_first; const int32_t* group_count;
-    float* partial;                            // [groups][ranges][rows][kv_heads * 128], ranges > 1
-    float* sums;                               // [groups][ranges][rows]
-    int groups, ranges, range_keys, page_log;
-    uint32_t cache_bytes;                      // of the keys, and of the values
-};
-
-template <int KV, int NQ>
-struct WalkShape {
-    static constexpr int H = 4 * KV, RT = NQ == 4 ? KV : 1, ROWS = 16 * RT, BK = NQ == 4 ? 64 : 128, KT = BK / 16, KS = BK / 32;
-    static constexpr int PITCH = BK + 8, TPW = NQ == 4 ? (KV * KT + 7) / 8 : 1, KG = NQ == 4 ? 1 : KV;   // score tiles of a wavefront, kv heads of one
-    static constexpr int OUT_PITCH = 128 + 4, WIDTH = KV * 128;
-    static constexpr size_t p_bytes = (NQ == 4 ? 2 : 1) * (size_t)ROWS * PITCH * sizeof(__bf16), out_bytes = (size_t)NQ * H * OUT_PITCH * sizeof(float);
-    static constexpr int SETS = NQ == 4 ? 2 : 1;                                     // blocks of keys in LDS, of values in registers
-    static constexpr size_t sums_at = p_bytes, keys_at = (sums_at + 8 * 16 * sizeof(float) + 1023) / 1024 * 1024;
-    static constexpr size_t key_bytes = (size_t)SETS * 8 * TPW * KG * 4096, lds_bytes = keys_at + key_bytes;
-    // behind the walk, in the keys' place: the factors of the sums and the mixed outputs
-    static constexpr size_t coef_at = keys_at, out_at = coef_at + (size_t)NQ * H * H * sizeof(float);
-    static_assert(out_at + out_bytes <= lds_bytes, "the outputs must fit the keys' place");
-    static_assert(lds_bytes <= 160 * 1024, "the blocks of keys must fit the LDS");
-    // the row of token t's head h
-    static __device__ __forceinline__ int row(int t, int h) { return NQ == 4 ? (h >> 2) * 16 + t * 4 + (h & 3) : h; }
-};
-
-// a pair of channels of one head's output, turned back (cosine and sine of minus the angle), gated and stored
-__device__ __forceinline__ void store_pair(const HeadMixArgs& a, int m, int h, int j, float u, float v, float co, float si, float gate) {
-    const int c0 = a.v_interleaved ? 2 * j : j, c1 = a.v_interleaved ? 2 * j + 1 : j + 64;
-    if (a.v_rope) {
-        const float x = turn_x(u, v, co, si);
-        v = turn_y(u, v, co, si);
-        u = x;
-    }
-    if (a.gate != nullptr) {
-        const float f = 1.0f / (1.0f + expf(-gate));
-        u *= f;
-        v *= f;
-    }
-    __bf16* dst = a.out + (size_t)m * a.out_stride + (size_t)h * 128;
-    dst[c0] = (__bf16)u;
-    dst[c1] = (__bf16)v;
-}
-
-// group g of t, range z of its keys
-template <int KV, int NQ>
-__device__ __forceinline__ void walk_group(const HeadMixArgs& a, const WalkArgs& t, int g, int z, unsigned char* lds_raw) {
-    using S = WalkShape<KV, NQ>;
-    constexpr int H = S::H, RT = S::RT, BK = S::BK, KT = S::KT, KS = S::KS, TPW = S::TPW, KG = S::KG, PITCH = S::PITCH, NKF = 4;
-    __bf16* p_lds = reinterpret_cast<__bf16*>(lds_raw);                              // [SETS][ROWS][PITCH]
-    float* out_lds = reinterpret_cast<float*>(lds_raw + S::out_at);                  // [NQ][H][OUT_PITCH]
-    float* coef = reinterpret_cast<float*>(lds_raw + S::coef_at);                    // [NQ][H][H]
-    float* sum_lds = reinterpret_cast<float*>(lds_raw + S::sums_at);                 // [8][16]
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i16 = lane & 15, b = lane >> 4;
-    const int first = t.group_first[g], count = t.group_count[g];
-    const int p0 = a.positions[first], kend = p0 + count;
-    const int k_begin = z * t.range_keys, k_end = min(kend, k_begin + t.range_keys);
-    if (k_begin >= k_end) return;
-    const int32_t* table = a.block_table + (size_t)a.slots[first] * a.max_blocks;
-    const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
-
-    // scores: this wavefront's tiles of 16 keys, of kv head gq (a single token: of all of them)
-    // (with one kv head half of the wavefronts have none)
-    const bool scoring = NQ == 1 || wave * TPW < KV * KT;
-    const int tile0 = scoring ? wave * TPW : 0, gq = NQ == 4 ? tile0 / KT : 0, kt0 = NQ == 4 ? tile0 % KT : wave;
-    const int tok = NQ == 4 ? i16 >> 2 : 0, head = NQ == 4 ? gq * 4 + (i16 & 3) : i16;
-    const bool row_ok = scoring && tok < count && head < H;
-    bf16x8 qf[NKF];
-    {
-        const __bf16* src = a.q + (size_t)(first + (row_ok ? tok : 0)) * a.q_stride + (size_t)(row_ok ? head : 0) * 128;
-#pragma unroll
-        for (int kf = 0; kf < NKF; ++kf) {
-            const bf16x8 v = *reinterpret_cast<const bf16x8*>(src + kf * 32 + b * 8);
-            qf[kf] = row_ok ? v : zero8;
-        }
-    }
-    // values: this wavefront's 16 KV channels, of kv head gv
-    const int gv = wave * KV / 8, chan0 = wave * 16 * KV % 128;
-    // (a block's instructions are what a group of four costs: 700 a wavefront with an address of its own for every load, 2 us a block;
-    // so pages of 2^k keys and caches below 4 GB, a load's place being 32 bits and a constant)
-    const int log = t.page_log, PS = 1 << log, place_mask = PS - 1;
-    const uint32_t page_bytes = (uint32_t)KV * PS * 256u, value_step = 16u * PS * 2u;
-    const auto k_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)a.k_pages, 0, (int)t.cache_bytes, 0x00027000);
-    const auto v_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)a.v_pages, 0, (int)t.cache_bytes, 0x00027000);
-    const uint32_t k_at = (uint32_t)gq * PS * 256u, v_at = (uint32_t)(gv * 128 + chan0 + i16) * PS * 2u;
-    // (groups of four: the next block's values on their way too; single tokens have a block or two, all of it asked for at once)
-    constexpr int SETS = S::SETS;
-    bf16x8 vreg[SETS][KS][KV];
-    int kid[TPW], vid[KS];
-    // (clamped: loads behind no branch; four keys, and eight values of a lane, lie in one page; a page that is missing reads as page 0)
-    auto ask = [&](int k0) {
-#pragma unroll
-        for (int x = 0; x < TPW; ++x) kid[x] = table[min(k0 + (kt0 + x) * 16 + (i16 & ~3), (kend - 1) & ~3) >> log];
-    };
-    auto ask_values = [&](int k0) {
-#pragma unroll
-        for (int s = 0; s < KS; ++s) vid[s] = table[min(k0 + s * 32 + 8 * b, (kend - 1) & ~7) >> log];
-    };
-    unsigned char* keys_lds = lds_raw + S::keys_at + (size_t)wave * (SETS * TPW * KG * 4096);
-    uint32_t key_piece[4];                     // which bytes of four rows a lane asks for: of row b of rows 4 j .. 4 j + 3
-#pragma unroll
-    for (int j = 0; j < 4; ++j) key_piece[j] = 256u * b + 16u * (i16 ^ (4 * j + b));
-    auto fetch = [&](int k0, int set) {
-#pragma unroll
-        for (int x = 0; x < TPW; ++x)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int key = min(k0 + (kt0 + x) * 16 + 4 * j, (kend - 1) & ~3);                         // (the same in every lane)
-                const uint32_t at = (uint32_t)max(__builtin_amdgcn_readlane(kid[x], 4 * j), 0) * page_bytes + k_at + (uint32_t)(key & place_mask) * 256u;
-#pragma unroll
-                for (int y = 0; y < KG; ++y)
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds(k_rsrc, (__attribute__((address_space(3))) void*)(keys_lds + ((set * TPW + x) * KG + y) * 4096 + j * 1024),
-                                                             16, (int)key_piece[j], (int)(at + (uint32_t)(y * PS) * 256u), 0, 0);
-            }
-    };
-    auto fetch_values = [&](int k0, auto set_) {
-        constexpr int set = decltype(set_)::value;
-#pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            const uint32_t at = (uint32_t)max(vid[s], 0) * page_bytes + v_at + (uint32_t)(min(k0 + s * 32 + 8 * b, (kend - 1) & ~7) & place_mask) * 2u;
-#pragma unroll
-            for (int v = 0; v < KV; ++v)
-                vreg[set][s][v] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(v_rsrc, (int)at, (int)(v * value_step), 0));
-        }
-    };
-    floatx4 acc[RT][KV];
-#pragma unroll
-    for (int c = 0; c < RT; ++c)
-#pragma unroll
-        for (int v = 0; v < KV; ++v) acc[c][v] = floatx4{0.f, 0.f, 0.f, 0.f};
-    float sum = 0.f;
-    // exp(cap tanh(x scale / cap)) = 2^(c1 - 2 c1 / (1 + 2^(x k))), c1 = cap log2(e), k = 2 log2(e) scale / cap
-    const float c1 = a.softcap * 1.4426950408889634f, c2 = -2.0f * c1, kx = 2.0f * 1.4426950408889634f * (a.scale / a.softcap);
-    constexpr std::integral_constant<int, 0> SET0{};
-    constexpr std::integral_constant<int, SETS - 1> SET1{};
-    ask(k_begin);
-    ask_values(k_begin);
-    fetch(k_begin, 0);
-    if (NQ == 4) ask(k_begin + BK);
-    asm volatile("" ::: "memory");             // (the order of these is counted on)
-    __builtin_amdgcn_sched_barrier(0);
-    fetch_values(k_begin, SET0);
-    if (NQ == 4) ask_values(k_begin + BK);
-    auto block = [&](int k0, auto set_) {
-        constexpr int set = decltype(set_)::value, buf = set;
-        const bool more = NQ == 4 || k0 + BK < k_end;
-        // this wavefront's keys are there (the compiler does not follow loads that go to LDS); all that it asked for behind them is a
-        // single token's values
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NQ == 4 ? 0 : KS * KV) : "memory");
-        bf16x8 kreg[TPW][KG][NKF];
-#pragma unroll
-        for (int x = 0; x < TPW; ++x)
-#pragma unroll
-            for (int y = 0; y < KG; ++y)
-#pragma unroll
-                for (int kf = 0; kf < NKF; ++kf)
-                    kreg[x][y][kf] = *reinterpret_cast<const bf16x8*>(keys_lds + ((set * TPW + x) * KG + y) * 4096 + i16 * 256 + 16 * ((4 * kf + b) ^ i16));
-        if (NQ == 4) {
-            fetch_values(k0 + BK, std::integral_constant<int, SETS - 1 - set>{});
-            ask_values(k0 + 2 * BK);
-        } else if (more) {
-            ask(k0 + BK);
-            ask_values(k0 + BK);
-        }
-        floatx4 sc[TPW];
-        if (scoring) {
-#pragma unroll
-            for (int x = 0; x < TPW; ++x) {
-#pragma unroll
-                for (int y = 0; y < KG; ++y) {
-                    floatx4 d = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                    for (int kf = 0; kf < NKF; ++kf) d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kreg[x][y][kf], qf[kf], d, 0, 0, 0);
-                    if (y == 0) sc[x] = d;
-                    else
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) sc[x][r] = i16 >> 2 == y ? d[r] : sc[x][r];
-                }
-            }
-        }
-        if (more) {
-            // (single tokens: into the place that this wavefront has just read)
-            if (SETS == 1) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            fetch(k0 + BK, SETS - 1 - set);
-            if (NQ == 4) ask(k0 + 2 * BK);
-        }
-        if (scoring) {
-            const bool plain = k0 + BK - 1 <= p0 && count == NQ && (NQ == 4 || KV == 4);       // every row sees every key
-            __bf16* to = p_lds + (buf * S::ROWS + (NQ == 4 ? gq * 16 : 0) + i16) * PITCH + 4 * b;
-#pragma unroll
-            for (int x = 0; x < TPW; ++x) {
-                float e[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float w = __builtin_amdgcn_exp2f(kx * sc[x][r]);
-                    e[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(c2, __builtin_amdgcn_rcpf(1.0f + w), c1));
-                }
-                if (!plain) {
-                    const int key = k0 + (kt0 + x) * 16 + 4 * b - p0;
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) e[r] = __uint_as_float(__float_as_uint(e[r]) & (row_ok && key + r <= tok ? 0xffffffffu : 0u));
-                }
-                bf16x4 e4;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    sum += e[r];
-                    e4[r] = (__bf16)e[r];
-                }
-                *reinterpret_cast<bf16x4*>(to + (kt0 + x) * 16) = e4;
-            }
-        }
-        __syncthreads();
-        if (k0 + BK > kend) {                  // (places behind the last key hold anything)
-#pragma unroll
-            for (int s = 0; s < KS; ++s)
-#pragma unroll
-                for (int v = 0; v < KV; ++v)
-#pragma unroll
-                    for (int j = 0; j < 8; ++j)
-                        if (k0 + s * 32 + 8 * b + j >= kend) vreg[set][s][v][j] = (__bf16)0.f;
-        }
-#pragma unroll
-        for (int s = 0; s < KS; ++s)
-#pragma unroll
-            for (int c = 0; c < RT; ++c) {
-                const bf16x8 pf = *reinterpret_cast<const bf16x8*>(p_lds + (buf * S::ROWS + c * 16 + i16) * PITCH + s * 32 + 8 * b);
-#pragma unroll
-                for (int v = 0; v < KV; ++v) acc[c][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf, vreg[set][s][v], acc[c][v], 0, 0, 0);
-            }
-        if (SETS == 1 && more) {
-            fetch_values(k0 + BK, set_);
-            __syncthreads();                   // (one buffer: everyone has read it)
-        }
-    };
-    for (int k0 = k_begin; k0 < k_end; k0 += SETS * BK) {
-        block(k0, SET0);
-        if (SETS == 1) continue;
-        if (k0 + BK >= k_end) break;
-        block(k0 + BK, SET1);
-    }
-    // what turning back and gating the outputs takes, asked for before the heads are mixed: output n of a thread is pair `lane` of
-    // token and head (wave + 8 n)
-    constexpr int OUTS = (NQ * H + 7) / 8;
-    float co[OUTS], si[OUTS], gate[OUTS];
-    if (t.ranges == 1) {
-#pragma unroll
-        for (int n = 0; n < OUTS; ++n) {
-            const int ti = min((wave + 8 * n) / H, count - 1), h = (wave + 8 * n) % H;
-            const float* cs = a.v_rope ? a.v_rope + (size_t)(p0 + ti) * 128 : nullptr;
-            co[n] = cs ? cs[lane] : 1.f;
-            si[n] = cs ? -cs[64 + lane] : 0.f;
-            gate[n] = a.gate ? to_float(a.gate[(size_t)(first + ti) * a.gate_stride + h]) : 0.f;
-        }
-    }
-    sum += __shfl_xor(sum, 16, MLR_WAVE);
-    sum += __shfl_xor(sum, 32, MLR_WAVE);
-    if (b == 0) sum_lds[wave * 16 + i16] = sum;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // (keys asked for beyond the last block: their place is used again)
-    __syncthreads();
-    // a row's sum over the wavefronts that scored it, in their order
-    auto row_sum = [&](int row) {
-        constexpr int WAVES = NQ == 4 ? KT / TPW : 8;
-        float total = 0.f;
-#pragma unroll
-        for (int w = 0; w < WAVES; ++w) total += sum_lds[((NQ == 4 ? (row >> 4) * WAVES : 0) + w) * 16 + (row & 15)];
-        return total;
-    };
-    if (t.ranges > 1) {
-        const size_t at = ((size_t)g * t.ranges + z) * S::ROWS;
-        if (tid < S::ROWS) t.sums[at + tid] = row_sum(tid);
-#pragma unroll
-        for (int c = 0; c < RT; ++c)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-                for (int v = 0; v < KV; ++v) t.partial[(at + c * 16 + 4 * b + r) * S::WIDTH + wave * 16 * KV + v * 16 + i16] = acc[c][v][r];
-        return;
-    }
-    for (int i = tid; i < NQ * H * H; i += 512) {
-        const int hs = i % H, ho = i / H % H, ti = i / (H * H);
-        const float den = row_sum(S::row(ti, hs)) + (a.sink_kind ? expf(sink_term(a, hs)) : 0.f);
-        coef[i] = a.mix[ho * H + hs] * (den > 0.f ? 1.0f / den : 0.f);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int hh = 0; hh < 4; ++hh) {
-        float o[KV];
-#pragma unroll
-        for (int v = 0; v < KV; ++v) o[v] = 0.f;
-#pragma unroll
-        for (int c = 0; c < RT; ++c) {
-            floatx4 f = {0.f, 0.f, 0.f, 0.f};
-            if (NQ == 4 || b < KV) f = *reinterpret_cast<const floatx4*>(coef + ((NQ == 4 ? b * H : 0) + gv * 4 + hh) * H + (NQ == 4 ? c : b) * 4);
-#pragma unroll
-            for (int v = 0; v < KV; ++v)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) o[v] = __builtin_fmaf(f[r], acc[c][v][r], o[v]);
-        }
-#pragma unroll
-        for (int v = 0; v < KV; ++v) {
-            if (NQ == 1) {
-                o[v] += __shfl_xor(o[v], 16, MLR_WAVE);
-                o[v] += __shfl_xor(o[v], 32, MLR_WAVE);
-            }
-            if (NQ == 4 || b == 0) out_lds[((NQ == 4 ? b * H : 0) + gv * 4 + hh) * S::OUT_PITCH + chan0 + v * 16 + i16] = o[v];
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int n = 0; n < OUTS; ++n) {
-        const int ti = (wave + 8 * n) / H, h = (wave + 8 * n) % H;
-        if (ti >= count) continue;
-        const float* row = out_lds + (ti * H + h) * S::OUT_PITCH;
-        store_pair(a, first + ti, h, lane, row[a.v_interleaved ? 2 * lane : lane], row[a.v_interleaved ? 2 * lane + 1 : lane + 64], co[n], si[n], gate[n]);
-    }
-}
-
-// A step's groups of four tokens and its single tokens in one launch: those wait for their own chain of blocks, these for memory.
-// (A prompt's last groups have the most keys: first.)
-template <int KV>
-__global__ __launch_bounds__(512, 2) void head_mix_walk_kernel(HeadMixArgs a, WalkArgs fours, WalkArgs ones) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
-    const int n = fours.groups * fours.ranges, i = blockIdx.x;
-    if (i < n) walk_group<KV, 4>(a, fours, fours.groups - 1 - i % fours.groups, i / fours.groups, lds_raw);
-    else walk_group<KV, 1>(a, ones, (i - n) % ones.groups, (i - n) / ones.groups, lds_raw);
-}
-
-// The ranges' shares added in ascending order, the heads mixed: a workgroup takes the heads of one kv head of a token, its four
-// wavefronts the source heads of a kv head each, a lane a pair of channels.
-template <int KV, int NQ>
-__device__ __forceinline__ void walk_finish(const HeadMixArgs& a, const WalkArgs& t, int g, int ti, float (&part)[4][4][2][64]) {
-    using S = WalkShape<KV, NQ>;
-    const int gv = blockIdx.y, j = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (ti >= t.group_count[g]) return;
-    const int first = t.group_first[g], m = first + ti, p0 = a.positions[first];
-    const int used = min(t.ranges, (p0 + t.group_count[g] - 1) / t.range_keys + 1);      // ranges that hold a key
-    const int c0 = gv * 128 + (a.v_interleaved ? 2 * j : j), c1 = gv * 128 + (a.v_interleaved ? 2 * j + 1 : j + 64);
-    const size_t base = (size_t)g * t.ranges * S::ROWS;
-    const int hh = wave;                       // the head that this wavefront finishes
-    const float* cs = a.v_rope ? a.v_rope + (size_t)(p0 + ti) * 128 : nullptr;
-    const float co = cs ? cs[j] : 1.f, si = cs ? -cs[64 + j] : 0.f;
-    const float gate = a.gate ? to_float(a.gate[(size_t)m * a.gate_stride + gv * 4 + hh]) : 0.f;
-    float u[4] = {0.f, 0.f, 0.f, 0.f}, v[4] = {0.f, 0.f, 0.f, 0.f};
-    if (wave < KV) {
-        float x[4], y[4], den[4], f[4][4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            x[r] = y[r] = 0.f;
-            den[r] = a.sink_kind ? expf(sink_term(a, wave * 4 + r)) : 0.f;
-#pragma unroll
-            for (int h = 0; h < 4; ++h) f[h][r] = a.mix[(gv * 4 + h) * S::H + wave * 4 + r];
-        }
-#pragma unroll 4
-        for (int z = 0; z < used; ++z)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const size_t row = base + (size_t)z * S::ROWS + S::row(ti, wave * 4 + r);
-                den[r] += t.sums[row];
-                x[r] += t.partial[row * S::WIDTH + c0];
-                y[r] += t.partial[row * S::WIDTH + c1];
-            }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const float inv = den[r] > 0.f ? 1.0f / den[r] : 0.f;
-#pragma unroll
-            for (int h = 0; h < 4; ++h) {
-                u[h] = __builtin_fmaf(f[h][r] * inv, x[r], u[h]);
-                v[h] = __builtin_fmaf(f[h][r] * inv, y[r], v[h]);
-            }
-        }
-    }
-#pragma unroll
-    for (int h = 0; h < 4; ++h) {
-        part[wave][h][0][j] = u[h];
-        part[wave][h][1][j] = v[h];
-    }
-    __syncthreads();
-    float su = 0.f, sv = 0.f;
-#pragma unroll
-    for (int w = 0; w < KV; ++w) {
-        su += part[w][hh][0][j];
-        sv += part[w][hh][1][j];
-    }
-    store_pair(a, m, gv * 4 + hh, j, su, sv, co, si, gate);
-}
-
-template <int KV>
-__global__ __launch_bounds__(256) void head_mix_walk_finish_kernel(HeadMixArgs a, WalkArgs fours, WalkArgs ones) {
-    __shared__ float part[4][4][2][64];
-    const int n = fours.ranges > 1 ? 4 * fours.groups : 0, i = blockIdx.x;
-    if (i < n) walk_finish<KV, 4>(a, fours, i / 4, i % 4, part);
-    else walk_finish<KV, 1>(a, ones, i - n, 0, part);
-}
-
-template <int KV>
-static int launch_walk(const HeadMixArgs& a, const WalkArgs& fours, const WalkArgs& ones, hipStream_t stream) {
-    constexpr size_t four = WalkShape<KV, 4>::lds_bytes, one = WalkShape<KV, 1>::lds_bytes, most = four > one ? four : one;
-    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&head_mix_walk_kernel<KV>),
-                                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)most);
-    if (allowed != hipSuccess) return (int)allowed;
-    const long blocks = (long)fours.groups * fours.ranges + (long)ones.groups * ones.ranges;
-    if (blocks > 0x7fffffffL) return -2;
-    head_mix_walk_kernel<KV><<<dim3((unsigned)blocks), 512, fours.groups ? ones.groups ? most : four : one, stream>>>(a, fours, ones);
-    const int rc = (int)hipGetLastError(), tokens = (fours.ranges > 1 ? 4 * fours.groups : 0) + (ones.ranges > 1 ? ones.groups : 0);
-    if (rc != 0 || tokens == 0) return rc;
-    head_mix_walk_finish_kernel<KV><<<dim3(tokens, KV), 256, 0, stream>>>(a, fours, ones);
-    return (int)hipGetLastError();
-}
-
 template <int HK, int CT, int VT, int NQ>
 static int launch_mix(const HeadMixArgs& a, const TileArgs& t, int kv_block, hipStream_t stream) {
     const int hp = 1 << t.hp_log, units = NQ == 16 ? 16 : 8;
@@ -1082,44 +654,6 @@ int mlr_head_mix_attention(const void* q, long q_stride, const void* k_pages, co
                   out_stride, max_blocks, q_heads, kv_heads, key_dim, value_dim, page_size, scale, softcap};
     head_mix_attention_kernel<<<rows, 256, lds, stream>>>(a);
     return (int)hipGetLastError();
-}
-
-// The form that walks the keys once, over `fours` groups of up to four consecutive tokens of a request each and `ones` single tokens
-// (either may be 0): q_heads = 4 kv_heads, kv_heads 1, 2 or 4, keys and values of 128 channels, pages of 2^k keys from 8 on, caches
-// below 4 GB.  `.._ranges` ranges of `.._keys` keys (a multiple of 128) together hold the longest context; where they are more than
-// one, .._partial holds groups * ranges * rows * kv_heads * 128 floats and .._sums groups * ranges * rows, rows = 16 kv_heads for groups
-// of four and 16 for single tokens.  Returns 1 when the sizes are not this form's.
-int mlr_head_mix_walk(const void* q, long q_stride, const void* k_pages, const void* v_pages, const int32_t* block_table,
-                      int max_blocks, const int32_t* slots, const int32_t* positions, const float* mix, const float* sink,
-                      float sink_value, int sink_kind, const float* v_rope, int v_interleaved, const void* gate,
-                      long gate_stride, void* out, long out_stride, const int32_t* fours_first, const int32_t* fours_count, int fours,
-                      int fours_keys, int fours_ranges, float* fours_sums, float* fours_partial, const int32_t* ones_first,
-                      const int32_t* ones_count, int ones, int ones_keys, int ones_ranges, float* ones_sums, float* ones_partial,
-                      int q_heads, int kv_heads, int key_dim, int value_dim, int page_size, int num_pages, float scale, float softcap,
-                      hipStream_t stream) {
-#if MLR_BF16
-    if (fours < 0 || ones < 0) return -1;
-    if (fours + ones == 0) return 0;
-    const unsigned long long bytes = (unsigned long long)(num_pages > 0 ? num_pages : 0) * kv_heads * page_size * 256;
-    if (q_heads != 4 * kv_heads || (kv_heads != 1 && kv_heads != 2 && kv_heads != 4) || value_dim != 128 || key_dim != 128 ||
-        page_size < 8 || (page_size & (page_size - 1)) != 0 || bytes >= (1ull << 32) || q_stride % 8 != 0 ||
-        !(softcap > 0.f && softcap <= 60.f))
-        return 1;
-    int page_log = 0;
-    while ((1 << page_log) < page_size) ++page_log;
-    const WalkArgs f{fours_first, fours_count, fours_partial, fours_sums, fours, fours ? fours_ranges : 1, fours ? fours_keys : 128, page_log, (uint32_t)bytes};
-    const WalkArgs o{ones_first, ones_count, ones_partial, ones_sums, ones, ones ? ones_ranges : 1, ones ? ones_keys : 128, page_log, (uint32_t)bytes};
-    for (const WalkArgs* t : {&f, &o})
-        if (t->ranges < 1 || t->range_keys <= 0 || t->range_keys % 128 != 0 || (t->ranges > 1 && (t->sums == nullptr || t->partial == nullptr)))
-            return -1;
-    if (sink_kind < 0 || sink_kind > 2 || (sink_kind == 2 && sink == nullptr)) return -1;
-    HeadMixArgs a{(const elem_t*)q, q_stride, (const elem_t*)k_pages, (const elem_t*)v_pages, block_table, slots, positions,
-                  mix, sink, sink_value, sink_kind, v_rope, v_interleaved, (const elem_t*)gate, gate_stride, (elem_t*)out,
-                  out_stride, max_blocks, q_heads, kv_heads, key_dim, value_dim, page_size, scale, softcap};
-    return kv_heads == 4 ? launch_walk<4>(a, f, o, stream) : kv_heads == 2 ? launch_walk<2>(a, f, o, stream) : launch_walk<1>(a, f, o, stream);
-#else
-    return 1;
-#endif
 }
 
 // The matrix-core form over `groups` groups of up to `group_tokens` (16 or 1) consecutive tokens of a request each.

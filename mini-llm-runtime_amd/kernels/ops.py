@@ -2044,45 +2044,6 @@ class Kernels:
                 return pad, inner, block
         return None
 
-    def head_mix_walk_supported(self, q_heads, kv_heads, key_dim, value_dim, page_size, softcap, num_pages=0):
-        """Whether the form that walks the keys once takes these sizes (else `head_mix_tiles` where it does): four query heads for
-        each of 1, 2 or 4 kv heads, keys and values of 128 channels, pages of 2^k keys from 8 on, caches below 4 GB, capped scores."""
-        return (self.dtype == torch.bfloat16 and kv_heads in (1, 2, 4) and q_heads == 4 * kv_heads and value_dim == key_dim == 128
-                and page_size >= 8 and page_size & (page_size - 1) == 0 and num_pages * kv_heads * page_size * 256 < 1 << 32
-                and softcap is not None and 0 < softcap <= self.HEAD_MIX_MAX_CAP)
-
-    @staticmethod
-    def head_mix_walk_rows(kv_heads, group_tokens):
-        """Rows of a group in `head_mix_walk`'s scratch memory, kv_heads * 128 floats and one sum each."""
-        return 16 * kv_heads if group_tokens == 4 else 16
-
-    @timed("attention")
-    def head_mix_walk(self, q, k_pages, v_pages, block_table, slots, positions, mix, sink, v_rope, gate, out, fours, ones, q_heads,
-                      kv_heads, key_dim, value_dim, page_size, scale, softcap):
-        """`head_mix_attention` in one walk over the keys, for groups of up to four consecutive tokens of a request each (`fours`) and
-        single tokens (`ones`); either None or (first rows, tokens, groups, keys of a range, ranges, sums, partial): ranges of a
-        multiple of 128 keys hold every context of the groups, and where they are more than one, `sums` and `partial` hold groups *
-        ranges * `head_mix_walk_rows` sums and as many rows of kv_heads * 128 floats."""
-        _need(self.head_mix_walk_supported(q_heads, kv_heads, key_dim, value_dim, page_size, softcap, k_pages.shape[0]),
-              "head_mix_walk: sizes that this form does not take")
-        args = self._head_mix_operands(q, k_pages, v_pages, block_table, slots, positions, mix, sink, v_rope, gate, out,
-                                       q_heads, kv_heads, key_dim, value_dim, page_size)
-        for some, tokens in ((fours, 4), (ones, 1)):
-            first, count, groups, keys, ranges, sums, partial = some or (None, None, 0, 128, 1, None, None)
-            if groups:
-                _tensor(first, "first", torch.int32, (groups,))
-                _tensor(count, "count", torch.int32, (groups,))
-                _need(ranges >= 1 and keys > 0 and keys % 128 == 0, "head_mix_walk: launch shape")
-            if ranges > 1:
-                rows = groups * ranges * self.head_mix_walk_rows(kv_heads, tokens)
-                _tensor(sums, "sums", torch.float32, ndim=1)
-                _tensor(partial, "partial", torch.float32, ndim=1)
-                _need(sums.numel() >= rows and partial.numel() >= rows * kv_heads * 128, "head_mix_walk: scratch too small")
-            args += (_p(first), _p(count), _c_int(groups), _c_int(keys), _c_int(ranges), _p(sums), _p(partial))
-        _ok(self._lib("head_mix_attention").mlr_head_mix_walk(
-            *args, _c_int(q_heads), _c_int(kv_heads), _c_int(key_dim), _c_int(value_dim), _c_int(page_size), _c_int(k_pages.shape[0]),
-            _c_float(scale), _c_float(softcap), _stream()), "head_mix_walk")
-
     def head_mix_tiles_supported(self, q_heads, kv_heads, key_dim, value_dim, page_size, softcap):
         """Whether the matrix-core form takes these sizes: the bfloat16 engine, keys in multiples of 8 channels up to 256,
         values in multiples of 16, pages in multiples of 8 places, capped scores, up to 32 query heads a kv head and 128

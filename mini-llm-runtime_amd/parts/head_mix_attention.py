@@ -7,9 +7,8 @@ head's output is turned back by the query's position --, and one sigmoid gate a 
 Per token the cache keeps the turned keys [kv_heads, head_dim] and the turned values [kv_heads, value_dim], the values
 transposed within a page.
 
-The bfloat16 engine runs the attention on the matrix cores where they take the sizes: in one walk over the keys
-(`Kernels.head_mix_walk`: up to four kv heads of four query heads each), or through scratch memory (`Kernels.head_mix_tiles`: the
-exponentials of all scores, bounded by taking a step's tokens in portions); else, and in the
+The bfloat16 engine runs the attention on the matrix cores where they take the sizes (`Kernels.head_mix_tiles`: the
+exponentials of all scores go through scratch memory, bounded by taking a step's tokens in portions); else, and in the
 float engine, one workgroup a token, whose sums follow from the token's position alone.
 """
 from __future__ import annotations
@@ -28,8 +27,6 @@ SUMS_CAP = 4 << 20            # floats of the sums
 MOST_RANGES = 64
 RANGE = 256                   # the narrowest range of keys of a workgroup
 WIDE_RANGE = 1024             # and the one that costs nothing
-WALK_RANGE = 128              # keys of a block of single tokens in the form that walks the keys once
-WALK_GROUP = 4                # tokens of a group of a prompt portion in the form that walks the keys once
 
 
 def _up(n, unit):
@@ -70,21 +67,6 @@ class LaunchShape:
         rows = self.groups * tokens
         self.e_numel, self.sums_numel = rows * row_e, rows * inner * self.score_ranges
         self.partial_numel = rows * row_o * self.value_ranges
-
-
-def walk_shape(kv_heads, groups, tokens, context, target):
-    """(keys of a range, ranges, groups a launch, rows of scratch memory a group and range) of `groups` groups of `tokens` tokens over
-    contexts up to `context` keys in one walk: ranges of one block for single tokens, whose workgroups wait for memory, and as many as
-    fill the GPU for groups of four; what the scratch memory does not hold at once goes through several launches."""
-    from ..kernels.ops import Kernels
-    rows = Kernels.head_mix_walk_rows(kv_heads, tokens)
-    room = max(1, min(PARTIAL_CAP // (rows * kv_heads * 128), SUMS_CAP // rows))          # ranges of groups that fit
-    ranges = max(1, min(MOST_RANGES, -(-context // (RANGE if tokens > 1 else WALK_RANGE)), room))
-    if tokens > 1:
-        ranges = max(1, min(ranges, target // groups, room // groups))
-    keys = _up(-(-context // ranges), 128)
-    ranges = -(-context // keys)
-    return keys, ranges, groups if ranges == 1 else max(1, min(groups, room // ranges)), rows
 
 
 @register_part("mixer", "head_mix_attention")
@@ -168,7 +150,6 @@ class HeadMixAttention:
         layout = self._layout()
         if dtype == torch.bfloat16 and layout is not None and s.softcap is not None:
             inner = layout[1]
-            plan[(f"token_groups_1_{WALK_GROUP}", torch.int32)] = 2 * rows + 2
             keys = _up(int((limits or {}).get("max_length") or 1), 32)
             plan[(f"token_groups_1_{GROUP}", torch.int32)] = 2 * rows + 2
             # (a portion of two tokens takes a whole group of scratch rows)
@@ -207,9 +188,6 @@ class HeadMixAttention:
             k.head_mix_attention(q, k_pages, v_pages, view.block_table, ctx.slots, ctx.positions, self.mix, self.sink, v_rope,
                                  gate, attn, *sizes, float(s.scale), s.softcap)
             return
-        if k.head_mix_walk_supported(*sizes, s.softcap, k_pages.shape[0]):
-            self._walk(ctx, q, k_pages, v_pages, view, v_rope, gate, attn, sizes)
-            return
         small, big, _ = ctx.token_groups(1, GROUP)
         for (first, count, n), tokens in ((big, GROUP), (small, 1)):
             if n == 0:
@@ -224,35 +202,3 @@ class HeadMixAttention:
                                  gate, attn, first[at:at + some], count[at:at + some], some, tokens, *sizes, float(s.scale),
                                  float(s.softcap), e, sums, partial, shape.ktiles, shape.score_keys, shape.score_ranges,
                                  shape.value_keys, shape.value_ranges, shape.kv_block)
-
-    def _walk(self, ctx, q, k_pages, v_pages, view, v_rope, gate, attn, sizes):
-        """Groups of four and single tokens in one launch where the scratch memory holds what both leave, else in several."""
-        s = self.spec
-        small, big, _ = ctx.token_groups(1, WALK_GROUP)
-        parts = []
-        for (first, count, n), tokens in ((big, WALK_GROUP), (small, 1)):
-            keys, ranges, some, rows = walk_shape(s.kv_heads, max(1, n), tokens, ctx.max_context, ctx.target_workgroups // 2)
-            parts.append((first, count, n, keys, ranges, some, some * ranges * rows if n and ranges > 1 else 0))
-        need = [p[6] for p in parts]
-        together = all(n == some for _, _, n, _, _, some, _ in parts if n) and sum(need) <= SUMS_CAP and \
-            sum(need) * s.kv_heads * 128 <= PARTIAL_CAP
-        rows = sum(need) if together else max(need)
-        width = s.kv_heads * 128
-        sums = ctx.workspace.get("mix_sums", (rows,), torch.float32) if rows else None
-        partial = ctx.workspace.get("mix_partial", (rows * width,), torch.float32) if rows else None
-
-        def part(i, at=0, scratch=0):
-            first, count, n, keys, ranges, some, use = parts[i]
-            now = min(some, n - at)
-            if now <= 0:
-                return None
-            return (first[at:at + now], count[at:at + now], now, keys, ranges, sums[scratch:scratch + use] if use else None,
-                    partial[scratch * width:(scratch + use) * width] if use else None)
-        if together:
-            launches = [(part(0), part(1, scratch=need[0]))]
-        else:
-            launches = [(part(0, at), None) for at in range(0, parts[0][2], parts[0][5])] + \
-                       [(None, part(1, at)) for at in range(0, parts[1][2], parts[1][5])]
-        for fours, ones in launches:
-            ctx.kernels.head_mix_walk(q, k_pages, v_pages, view.block_table, ctx.slots, ctx.positions, self.mix, self.sink, v_rope, gate,
-                                      attn, fours, ones, *sizes, float(s.scale), float(s.softcap))
