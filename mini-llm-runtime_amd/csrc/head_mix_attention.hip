@@ -208,12 +208,10 @@ struct PageOf {
 // are on their way while a tile's exponentials are taken, and the ids of the pages after that.
 // HPL: log2 of the places a kv head's heads take, 2 for all from four on (a lane's four rows are then one token's).
 template <int NKF, int RT, int HPL>
-__global__ __launch_bounds__(256) void head_scores_kernel(HeadMixArgs a, TileArgs t) {
+__device__ __forceinline__ void head_scores(const HeadMixArgs& a, const TileArgs& t, int g, int block_y, int block_z, float (&sum_lds)[4][RT * 16]) {
     constexpr int TOKENS = HPL == 0 ? 4 : HPL == 1 ? 2 : 1, PER = 4 / TOKENS;      // tokens of a lane's four rows; rows a token
-    __shared__ float sum_lds[4][RT * 16];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i16 = lane & 15, b = lane >> 4;
-    const int g = (int)gridDim.x - 1 - (int)blockIdx.x;        // (a prompt's last groups have the most keys: first)
-    const int kvh = blockIdx.y % t.kv_pad, row0 = (blockIdx.y / t.kv_pad) * RT * 16;
+    const int kvh = block_y % t.kv_pad, row0 = (block_y / t.kv_pad) * RT * 16;
     const int first = t.group_first[g], count = t.group_count[g];
     const int hp_log = HPL < 2 ? HPL : t.hp_log, hp = 1 << hp_log, hg = a.q_heads / a.kv_heads, D = a.key_dim;
     const PageOf pages{a.page_size, t.page_log};
@@ -236,8 +234,8 @@ __global__ __launch_bounds__(256) void head_scores_kernel(HeadMixArgs a, TileArg
         }
     }
     const int kt_step = t.score_keys / TK;
-    const int kt_end = min((kend + TK - 1) / TK, ((int)blockIdx.z + 1) * kt_step);
-    int kt = (int)blockIdx.z * kt_step + wave;
+    const int kt_end = min((kend + TK - 1) / TK, (block_z + 1) * kt_step);
+    int kt = block_z * kt_step + wave;
     const int te = TK * t.head_k, half = t.head_k == 16 ? 256 : 512;       // elements of a tile, of its half (one step of heads)
     // where the lane's rows go (tokens beyond the group's have no scratch; padded heads store their zeros)
     __bf16* dst[RT][TOKENS];
@@ -351,8 +349,30 @@ __global__ __launch_bounds__(256) void head_scores_kernel(HeadMixArgs a, TileArg
     for (int r = tid; r < RT * 16; r += 256) {
         const int row = row0 + r, ti = row >> hp_log, hh = row & (hp - 1);
         if (ti < count)
-            t.sums[(((size_t)g * t.group_tokens + ti) * t.head_k + kvh * hp + hh) * t.score_ranges + blockIdx.z] =
+            t.sums[(((size_t)g * t.group_tokens + ti) * t.head_k + kvh * hp + hh) * t.score_ranges + block_z] =
                 (sum_lds[0][r] + sum_lds[1][r]) + (sum_lds[2][r] + sum_lds[3][r]);
+    }
+}
+
+// (A prompt's last groups have the most keys: first.)
+template <int NKF, int RT, int HPL>
+__global__ __launch_bounds__(256) void head_scores_kernel(HeadMixArgs a, TileArgs t) {
+    __shared__ float sum_lds[4][RT * 16];
+    head_scores<NKF, RT, HPL>(a, t, (int)gridDim.x - 1 - (int)blockIdx.x, blockIdx.y, blockIdx.z, sum_lds);
+}
+
+// A step's groups (t, its grid counted along x) and its single tokens behind them in one launch: the groups' workgroups are few and
+// walk chains of tiles, the single tokens' wait for memory.  A layer of 16 heads over 4, a portion of 700 tokens and 32 single ones of 100
+// to 1500 keys: scores 24.8 us for 21.3 and 14.9, values 28.0 for 23.3 and 17.1, finish 7.1 for twice 4.9.
+template <int NKF, int RT, int HPL>
+__global__ __launch_bounds__(256) void head_scores_both_kernel(HeadMixArgs a, TileArgs t, TileArgs s, int ty, int sy) {
+    __shared__ float sum_lds[4][RT * 16], one_lds[4][16];
+    const int n = t.groups * ty * t.score_ranges, i = blockIdx.x;
+    if (i < n) {
+        head_scores<NKF, RT, HPL>(a, t, t.groups - 1 - i % t.groups, i / t.groups % ty, i / (t.groups * ty), sum_lds);
+    } else {
+        const int j = i - n;
+        head_scores<NKF, 1, HPL>(a, s, s.groups - 1 - j % s.groups, j / s.groups % sy, j / (s.groups * sy), one_lds);
     }
 }
 
@@ -365,11 +385,10 @@ __global__ __launch_bounds__(256) void head_scores_kernel(HeadMixArgs a, TileArg
 // Two LDS buffers: one barrier a turn.  HK: 16, 32 (one step of the mixing product, its operands in registers) or 0
 // (any multiple of 32: `mix` and the inverse sums in LDS).
 template <int HK, int CT, int VT, int NQ>
-__global__ __launch_bounds__(512) void head_mix_values_kernel(HeadMixArgs a, TileArgs t, int kv_block) {
+__device__ __forceinline__ void head_mix_values(const HeadMixArgs& a, const TileArgs& t, int kv_block, int g, int block_y, int block_z, unsigned char* lds_raw) {
     constexpr int UNITS = NQ == 16 ? 16 : 8, UPW = UNITS / 8, KSUB = NQ == 16 ? 1 : 8;
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i16 = lane & 15, b = lane >> 4;
-    const int g = (int)gridDim.x - 1 - (int)blockIdx.x, kv0 = blockIdx.y * kv_block;
+    const int kv0 = block_y * kv_block;
     const int first = t.group_first[g], count = t.group_count[g];
     const int hp = 1 << t.hp_log, hg = a.q_heads / a.kv_heads, V = a.value_dim, PS = a.page_size, H = a.q_heads;
     const int p0 = a.positions[first], kend = p0 + count;
@@ -422,7 +441,7 @@ __global__ __launch_bounds__(512) void head_mix_values_kernel(HeadMixArgs a, Til
     for (int c = 0; c < CT; ++c)
 #pragma unroll
         for (int v = 0; v < VT; ++v) acc[c][v] = floatx4{0.f, 0.f, 0.f, 0.f};
-    const int kt_first = (int)blockIdx.z * (t.value_keys / TK);
+    const int kt_first = block_z * (t.value_keys / TK);
     const int kt_end = min((kend + TK - 1) / TK, kt_first + t.value_keys / TK);
     const size_t te = (size_t)TK * head_k;
     const __bf16* e_group = t.e + (size_t)g * t.group_tokens * t.ktiles * te;
@@ -540,7 +559,7 @@ __global__ __launch_bounds__(512) void head_mix_values_kernel(HeadMixArgs a, Til
     for (int c = 0; c < CT; ++c) {
         const int col = c * 16 + i16, ti = NQ == 16 ? col >> t.hp_log : 0, hh = NQ == 16 ? col & (hp - 1) : col;
         if (ti >= count || hh >= hg) continue;
-        float* dst = t.partial + ((((size_t)g * t.group_tokens + ti) * H + kvh * hg + hh) * t.value_ranges + blockIdx.z) * V;
+        float* dst = t.partial + ((((size_t)g * t.group_tokens + ti) * H + kvh * hg + hh) * t.value_ranges + block_z) * V;
 #pragma unroll
         for (int v = 0; v < VT; ++v) {
             const int ch = (vpart + vs * v) * 16 + 4 * b;
@@ -549,16 +568,38 @@ __global__ __launch_bounds__(512) void head_mix_values_kernel(HeadMixArgs a, Til
     }
 }
 
+template <int HK, int CT, int VT, int NQ>
+__global__ __launch_bounds__(512) void head_mix_values_kernel(HeadMixArgs a, TileArgs t, int kv_block) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+    head_mix_values<HK, CT, VT, NQ>(a, t, kv_block, (int)gridDim.x - 1 - (int)blockIdx.x, blockIdx.y, blockIdx.z, lds_raw);
+}
+
+template <int HK, int CT, int VT, int ONE_VT>
+__global__ __launch_bounds__(512) void head_mix_values_both_kernel(HeadMixArgs a, TileArgs t, TileArgs s, int kv_block, int one_block) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+    const int ty = (a.kv_heads + kv_block - 1) / kv_block, sy = (a.kv_heads + one_block - 1) / one_block, n = t.groups * ty * t.value_ranges;
+    const int i = blockIdx.x;
+    if (i < n) {
+        head_mix_values<HK, CT, VT, 16>(a, t, kv_block, t.groups - 1 - i % t.groups, i / t.groups % ty, i / (t.groups * ty), lds_raw);
+    } else {
+        const int j = i - n;
+        head_mix_values<HK, 1, ONE_VT, 1>(a, s, one_block, s.groups - 1 - j % s.groups, j / s.groups % sy, j / (s.groups * sy), lds_raw);
+    }
+}
+
 // The ranges' shares added in ascending order, turned back, gated: a workgroup takes 256 channel pairs of a token of a
 // group.
-__global__ __launch_bounds__(256) void head_mix_finish_kernel(HeadMixArgs a, TileArgs t) {
-    const int g = blockIdx.x, ti = blockIdx.y, V = a.value_dim, half = V >> 1;
+// (Behind t's tokens those of s, single ones, where the step has both.)
+__global__ __launch_bounds__(256) void head_mix_finish_kernel(HeadMixArgs a, TileArgs both, TileArgs s) {
+    const int n = both.groups * both.group_tokens, i = blockIdx.x;
+    const TileArgs& t = i < n ? both : s;
+    const int g = i < n ? i / both.group_tokens : i - n, ti = i < n ? i % both.group_tokens : 0, V = a.value_dim, half = V >> 1;
     if (ti >= t.group_count[g]) return;
     const int m = t.group_first[g] + ti;
     const float* base = t.partial + ((size_t)g * t.group_tokens + ti) * a.q_heads * t.value_ranges * V;
     const int used = min(t.value_ranges, (a.positions[m] + t.value_keys) / t.value_keys);      // ranges that hold a key
     const float* cs = a.v_rope ? a.v_rope + (size_t)a.positions[m] * V : nullptr;
-    const int o = blockIdx.z * 256 + threadIdx.x;
+    const int o = blockIdx.y * 256 + threadIdx.x;
     if (o < a.q_heads * half) {
         const int h = o / half, j = o % half;
         const int c0 = a.v_interleaved ? 2 * j : j, c1 = a.v_interleaved ? 2 * j + 1 : j + half;
@@ -608,6 +649,55 @@ static int launch_mix_heads(const HeadMixArgs& a, const TileArgs& t, int kv_bloc
     if (t.head_k == 16) return launch_mix<16, CT, VT, NQ>(a, t, kv_block, stream);
     if (t.head_k == 32) return launch_mix<32, CT, VT, NQ>(a, t, kv_block, stream);
     return launch_mix<0, CT, VT, NQ>(a, t, kv_block, stream);
+}
+
+template <int HK, int VT, int ONE_VT>
+static int launch_mix_both_as(const HeadMixArgs& a, const TileArgs& t, const TileArgs& s, int kv_block, int one_block, hipStream_t stream) {
+    const size_t group = (size_t)2 * kv_block * (16 * 4 + 1) * TK * sizeof(__bf16), one = (size_t)2 * one_block * (8 * 4 + 1) * TK * sizeof(__bf16);
+    const size_t lds = group > one ? group : one;                 // (kv blocks of up to 8 heads' places: at most 66 KB)
+    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&head_mix_values_both_kernel<HK, 4, VT, ONE_VT>),
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
+    if (allowed != hipSuccess) return (int)allowed;
+    const long blocks = (long)t.groups * ((a.kv_heads + kv_block - 1) / kv_block) * t.value_ranges +
+                        (long)s.groups * ((a.kv_heads + one_block - 1) / one_block) * s.value_ranges;
+    if (blocks > 0x7fffffffL) return -2;
+    head_mix_values_both_kernel<HK, 4, VT, ONE_VT><<<(unsigned)blocks, 512, lds, stream>>>(a, t, s, kv_block, one_block);
+    return (int)hipGetLastError();
+}
+
+template <int HK>
+static int launch_mix_both(const HeadMixArgs& a, const TileArgs& t, const TileArgs& s, int kv_block, int one_block, hipStream_t stream) {
+    const auto two = [&](int block) { return (a.value_dim / 16 + 8 / block - 1) / (8 / block) <= 2; };
+    if (two(kv_block)) return two(one_block) ? launch_mix_both_as<HK, 2, 2>(a, t, s, kv_block, one_block, stream) : launch_mix_both_as<HK, 2, 4>(a, t, s, kv_block, one_block, stream);
+    return two(one_block) ? launch_mix_both_as<HK, 4, 2>(a, t, s, kv_block, one_block, stream) : launch_mix_both_as<HK, 4, 4>(a, t, s, kv_block, one_block, stream);
+}
+
+// One launch's shape and scratch memory, checked: 0, 1 for sizes that are not this form's, or -1.
+static int tile_args(const HeadMixArgs& a, const int32_t* group_first, const int32_t* group_count, int groups, int group_tokens, void* e,
+                     float* sums, float* partial, int ktiles, int head_pad, int head_k, int score_keys, int score_ranges, int value_keys,
+                     int value_ranges, int kv_block, TileArgs& t) {
+    int hp_log = 0;
+    while ((1 << hp_log) < head_pad) ++hp_log;
+    const int hg = a.kv_heads > 0 ? a.q_heads / a.kv_heads : 0;
+    if (a.kv_heads <= 0 || a.q_heads % a.kv_heads != 0 || (1 << hp_log) != head_pad || hg > head_pad || head_pad > 32) return -1;
+    if (a.key_dim % 8 != 0 || a.key_dim > 256 || a.value_dim % 16 != 0 || a.page_size % 8 != 0 || a.q_stride % 8 != 0 ||
+        !(a.softcap > 0.f && a.softcap <= 60.f))
+        return 1;
+    if ((group_tokens != 16 && group_tokens != 1) || (head_k != 16 && head_k % 32 != 0) || head_k > 128 ||
+        head_k % head_pad != 0 || head_k < a.kv_heads * head_pad || a.sink_kind < 0 || a.sink_kind > 2 ||
+        (a.sink_kind == 2 && a.sink == nullptr))
+        return -1;
+    if (score_keys % TK != 0 || value_keys % (group_tokens == 1 ? 8 * TK : TK) != 0 || score_ranges < 1 || value_ranges < 1 ||
+        score_keys <= 0 || value_keys <= 0 || (long)score_keys * score_ranges < (long)ktiles * TK ||
+        (long)value_keys * value_ranges < (long)ktiles * TK || value_ranges > 65535)
+        return -1;
+    if ((kv_block != 1 && kv_block != 2 && kv_block != 4 && kv_block != 8) || kv_block * head_pad > 32) return -1;
+    int page_log = 0;
+    while ((1 << page_log) < a.page_size) ++page_log;
+    if ((1 << page_log) != a.page_size) page_log = -1;
+    t = TileArgs{group_first, group_count, groups, group_tokens, (__bf16*)e, sums, partial, ktiles, hp_log, head_k,
+                 head_k / head_pad, page_log, score_keys, score_ranges, value_keys, value_ranges};
+    return 0;
 }
 
 template <int NKF>
@@ -672,39 +762,22 @@ int mlr_head_mix_tiles(const void* q, long q_stride, const void* k_pages, const 
                        int value_ranges, int kv_block, hipStream_t stream) {
 #if MLR_BF16
     if (groups <= 0) return 0;
-    int hp_log = 0;
-    while ((1 << hp_log) < head_pad) ++hp_log;
-    const int hg = kv_heads > 0 ? q_heads / kv_heads : 0;
-    if (kv_heads <= 0 || q_heads % kv_heads != 0 || (1 << hp_log) != head_pad || hg > head_pad || head_pad > 32) return -1;
-    if (key_dim % 8 != 0 || key_dim > 256 || value_dim % 16 != 0 || page_size % 8 != 0 || q_stride % 8 != 0 ||
-        !(softcap > 0.f && softcap <= 60.f))
-        return 1;
-    if ((group_tokens != 16 && group_tokens != 1) || (head_k != 16 && head_k % 32 != 0) || head_k > 128 ||
-        head_k % head_pad != 0 || head_k < kv_heads * head_pad || sink_kind < 0 || sink_kind > 2 ||
-        (sink_kind == 2 && sink == nullptr))
-        return -1;
-    if (score_keys % TK != 0 || value_keys % (group_tokens == 1 ? 8 * TK : TK) != 0 || score_ranges < 1 || value_ranges < 1 ||
-        score_keys <= 0 || value_keys <= 0 || (long)score_keys * score_ranges < (long)ktiles * TK ||
-        (long)value_keys * value_ranges < (long)ktiles * TK || value_ranges > 65535)
-        return -1;
-    if ((kv_block != 1 && kv_block != 2 && kv_block != 4 && kv_block != 8) || kv_block * head_pad > 32) return -1;
-    HeadMixArgs a{(const elem_t*)q, q_stride, (const elem_t*)k_pages, (const elem_t*)v_pages, block_table, slots, positions,
-                  mix, sink, sink_value, sink_kind, v_rope, v_interleaved, (const elem_t*)gate, gate_stride, (elem_t*)out,
-                  out_stride, max_blocks, q_heads, kv_heads, key_dim, value_dim, page_size, scale, softcap};
-    int page_log = 0;
-    while ((1 << page_log) < page_size) ++page_log;
-    if ((1 << page_log) != page_size) page_log = -1;
-    TileArgs t{group_first, group_count, groups, group_tokens, (__bf16*)e, sums, partial, ktiles, hp_log, head_k,
-               head_k / head_pad, page_log, score_keys, score_ranges, value_keys, value_ranges};
+    const HeadMixArgs args{(const elem_t*)q, q_stride, (const elem_t*)k_pages, (const elem_t*)v_pages, block_table, slots, positions,
+                           mix, sink, sink_value, sink_kind, v_rope, v_interleaved, (const elem_t*)gate, gate_stride, (elem_t*)out,
+                           out_stride, max_blocks, q_heads, kv_heads, key_dim, value_dim, page_size, scale, softcap};
+    TileArgs t;
+    int rc = tile_args(args, group_first, group_count, groups, group_tokens, e, sums, partial, ktiles, head_pad, head_k, score_keys,
+                       score_ranges, value_keys, value_ranges, kv_block, t);
+    if (rc != 0) return rc;
     const int ct = group_tokens == 16 ? head_pad : (head_pad + 15) / 16;
     const int vt = (value_dim / 16 + 8 / kv_block - 1) / (8 / kv_block);
     if (ct * vt > 32 || vt > 8) return 1;
     const int nkf = (key_dim + 31) / 32;
-    int rc = nkf <= 2 ? launch_scores<2>(a, t, stream) : nkf <= 4 ? launch_scores<4>(a, t, stream) : launch_scores<8>(a, t, stream);
+    rc = nkf <= 2 ? launch_scores<2>(args, t, stream) : nkf <= 4 ? launch_scores<4>(args, t, stream) : launch_scores<8>(args, t, stream);
     if (rc != 0) return rc;
     rc = 1;
 #define MLR_MIX_CLASS(NQ, CT, VT)                                                     \
-    if (rc == 1 && group_tokens == NQ && ct == CT && vt <= VT) rc = launch_mix_heads<CT, VT, NQ>(a, t, kv_block, stream);
+    if (rc == 1 && group_tokens == NQ && ct == CT && vt <= VT) rc = launch_mix_heads<CT, VT, NQ>(args, t, kv_block, stream);
     MLR_MIX_CLASS(16, 1, 2) MLR_MIX_CLASS(16, 1, 4) MLR_MIX_CLASS(16, 1, 8)
     MLR_MIX_CLASS(16, 2, 2) MLR_MIX_CLASS(16, 2, 4) MLR_MIX_CLASS(16, 2, 8)
     MLR_MIX_CLASS(16, 4, 1) MLR_MIX_CLASS(16, 4, 2) MLR_MIX_CLASS(16, 4, 4)
@@ -712,7 +785,50 @@ int mlr_head_mix_tiles(const void* q, long q_stride, const void* k_pages, const 
     MLR_MIX_CLASS(1, 1, 1) MLR_MIX_CLASS(1, 1, 2) MLR_MIX_CLASS(1, 1, 4) MLR_MIX_CLASS(1, 1, 8) MLR_MIX_CLASS(1, 2, 2) MLR_MIX_CLASS(1, 2, 8)
 #undef MLR_MIX_CLASS
     if (rc != 0) return rc;
-    head_mix_finish_kernel<<<dim3(groups, group_tokens, (q_heads * (value_dim / 2) + 255) / 256), 256, 0, stream>>>(a, t);
+    head_mix_finish_kernel<<<dim3(groups * group_tokens, (q_heads * (value_dim / 2) + 255) / 256), 256, 0, stream>>>(args, t, t);
+    return (int)hipGetLastError();
+#else
+    return 1;
+#endif
+}
+
+// Groups of up to 16 tokens and single tokens (`ones` groups) in the three launches of one of them, for heads in places of four, up to
+// eight kv heads, keys of up to 128 channels: the same workgroups and so the same bits.  shape and one_shape: ktiles, score_keys,
+// score_ranges, value_keys, value_ranges, kv_block as above, with scratch memory of each one's own.  Returns 1 when the sizes are not
+// this form's.
+int mlr_head_mix_tiles_both(const void* q, long q_stride, const void* k_pages, const void* v_pages, const int32_t* block_table,
+                            int max_blocks, const int32_t* slots, const int32_t* positions, const float* mix, const float* sink,
+                            float sink_value, int sink_kind, const float* v_rope, int v_interleaved, const void* gate,
+                            long gate_stride, void* out, long out_stride, const int32_t* group_first, const int32_t* group_count,
+                            int groups, void* e, float* sums, float* partial, const int* shape, const int32_t* one_first,
+                            const int32_t* one_count, int ones, void* one_e, float* one_sums, float* one_partial, const int* one_shape,
+                            int q_heads, int kv_heads, int key_dim, int value_dim, int page_size, float scale, float softcap,
+                            int head_pad, int head_k, hipStream_t stream) {
+#if MLR_BF16
+    if (groups <= 0 || ones <= 0) return -1;
+    const HeadMixArgs args{(const elem_t*)q, q_stride, (const elem_t*)k_pages, (const elem_t*)v_pages, block_table, slots, positions,
+                           mix, sink, sink_value, sink_kind, v_rope, v_interleaved, (const elem_t*)gate, gate_stride, (elem_t*)out,
+                           out_stride, max_blocks, q_heads, kv_heads, key_dim, value_dim, page_size, scale, softcap};
+    if (head_pad != 4 || key_dim > 128 || (head_k != 16 && head_k != 32)) return 1;
+    TileArgs t, s;
+    int rc = tile_args(args, group_first, group_count, groups, 16, e, sums, partial, shape[0], head_pad, head_k, shape[1], shape[2],
+                       shape[3], shape[4], shape[5], t);
+    if (rc == 0)
+        rc = tile_args(args, one_first, one_count, ones, 1, one_e, one_sums, one_partial, one_shape[0], head_pad, head_k, one_shape[1],
+                       one_shape[2], one_shape[3], one_shape[4], one_shape[5], s);
+    if (rc != 0) return rc;
+    const auto tiles = [&](int block) { return (value_dim / 16 + 8 / block - 1) / (8 / block); };
+    if (tiles(shape[5]) > 4 || tiles(one_shape[5]) > 4) return 1;
+    const long score_blocks = (long)t.kv_pad * ((long)groups * t.score_ranges + (long)ones * s.score_ranges);
+    if (score_blocks > 0x7fffffffL) return -2;
+    // (a group's 64 rows are one workgroup's four tiles, a token's four rows one)
+    if (key_dim <= 64) head_scores_both_kernel<2, 4, 2><<<(unsigned)score_blocks, 256, 0, stream>>>(args, t, s, t.kv_pad, s.kv_pad);
+    else head_scores_both_kernel<4, 4, 2><<<(unsigned)score_blocks, 256, 0, stream>>>(args, t, s, t.kv_pad, s.kv_pad);
+    rc = (int)hipGetLastError();
+    if (rc != 0) return rc;
+    rc = head_k == 16 ? launch_mix_both<16>(args, t, s, shape[5], one_shape[5], stream) : launch_mix_both<32>(args, t, s, shape[5], one_shape[5], stream);
+    if (rc != 0) return rc;
+    head_mix_finish_kernel<<<dim3(groups * 16 + ones, (q_heads * (value_dim / 2) + 255) / 256), 256, 0, stream>>>(args, t, s);
     return (int)hipGetLastError();
 #else
     return 1;

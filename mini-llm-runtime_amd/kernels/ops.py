@@ -2065,7 +2065,19 @@ class Kernels:
               "head_mix_tiles: sizes that the matrix-core form does not take")
         args = self._head_mix_operands(q, k_pages, v_pages, block_table, slots, positions, mix, sink, v_rope, gate, out,
                                        q_heads, kv_heads, key_dim, value_dim, page_size)
-        pad, inner, most = self.head_mix_layout(q_heads, kv_heads, value_dim)
+        pad, inner, _ = self.head_mix_layout(q_heads, kv_heads, value_dim)
+        self._head_mix_launch(group_first, group_count, groups, group_tokens, q_heads, kv_heads, value_dim, e, sums, partial, ktiles,
+                              score_keys, score_ranges, value_keys, value_ranges, kv_block)
+        _ok(self._lib("head_mix_attention").mlr_head_mix_tiles(
+            *args, _p(group_first), _p(group_count), _c_int(groups), _c_int(group_tokens), _c_int(q_heads), _c_int(kv_heads),
+            _c_int(key_dim), _c_int(value_dim), _c_int(page_size), _c_float(scale), _c_float(softcap), _p(e), _p(sums),
+            _p(partial), _c_int(ktiles), _c_int(pad), _c_int(inner), _c_int(score_keys), _c_int(score_ranges),
+            _c_int(value_keys), _c_int(value_ranges), _c_int(kv_block), _stream()), "head_mix_tiles")
+
+    def _head_mix_launch(self, group_first, group_count, groups, group_tokens, q_heads, kv_heads, value_dim, e, sums, partial, ktiles,
+                         score_keys, score_ranges, value_keys, value_ranges, kv_block):
+        """One launch's groups, key ranges and scratch memory, checked."""
+        _, inner, most = self.head_mix_layout(q_heads, kv_heads, value_dim)
         _tensor(group_first, "group_first", torch.int32, ndim=1)
         _tensor(group_count, "group_count", torch.int32, ndim=1)
         _need(group_first.numel() >= groups and group_count.numel() >= groups, "group vectors too short")
@@ -2079,11 +2091,31 @@ class Kernels:
         _tensor(partial, "partial", torch.float32, ndim=1)
         _need(e.numel() >= rows * keys * inner and sums.numel() >= rows * inner * score_ranges
               and partial.numel() >= rows * q_heads * value_ranges * value_dim, "head_mix_tiles: scratch too small")
-        _ok(self._lib("head_mix_attention").mlr_head_mix_tiles(
-            *args, _p(group_first), _p(group_count), _c_int(groups), _c_int(group_tokens), _c_int(q_heads), _c_int(kv_heads),
-            _c_int(key_dim), _c_int(value_dim), _c_int(page_size), _c_float(scale), _c_float(softcap), _p(e), _p(sums),
-            _p(partial), _c_int(ktiles), _c_int(pad), _c_int(inner), _c_int(score_keys), _c_int(score_ranges),
-            _c_int(value_keys), _c_int(value_ranges), _c_int(kv_block), _stream()), "head_mix_tiles")
+
+    def head_mix_both_supported(self, q_heads, kv_heads, key_dim, value_dim, page_size, softcap):
+        """Whether `head_mix_tiles_both` takes these sizes: those of `head_mix_tiles` with three or four query heads a kv head, up to
+        eight kv heads, keys of up to 128 channels and values of up to 256."""
+        layout = self.head_mix_layout(q_heads, kv_heads, value_dim)
+        return (self.head_mix_tiles_supported(q_heads, kv_heads, key_dim, value_dim, page_size, softcap) and layout[0] == 4 and layout[1] <= 32
+                and key_dim <= 128 and value_dim <= 256)
+
+    @timed("attention")
+    def head_mix_tiles_both(self, q, k_pages, v_pages, block_table, slots, positions, mix, sink, v_rope, gate, out, big, ones, q_heads,
+                            kv_heads, key_dim, value_dim, page_size, scale, softcap):
+        """`head_mix_tiles` for groups of up to 16 tokens (`big`) and for single tokens (`ones`) in the launches of one of them, the same
+        bits.  Either: (first rows, tokens, groups, e, sums, partial, ktiles, score_keys, score_ranges, value_keys, value_ranges,
+        kv_block), with scratch memory of its own."""
+        _need(self.head_mix_both_supported(q_heads, kv_heads, key_dim, value_dim, page_size, softcap),
+              "head_mix_tiles_both: sizes that this form does not take")
+        args = self._head_mix_operands(q, k_pages, v_pages, block_table, slots, positions, mix, sink, v_rope, gate, out,
+                                       q_heads, kv_heads, key_dim, value_dim, page_size)
+        pad, inner, _ = self.head_mix_layout(q_heads, kv_heads, value_dim)
+        for (first, count, groups, e, sums, partial, *shape), tokens in ((big, 16), (ones, 1)):
+            self._head_mix_launch(first, count, groups, tokens, q_heads, kv_heads, value_dim, e, sums, partial, *shape)
+            args += (_p(first), _p(count), _c_int(groups), _p(e), _p(sums), _p(partial), (ctypes.c_int * 6)(*shape))
+        _ok(self._lib("head_mix_attention").mlr_head_mix_tiles_both(
+            *args, _c_int(q_heads), _c_int(kv_heads), _c_int(key_dim), _c_int(value_dim), _c_int(page_size), _c_float(scale),
+            _c_float(softcap), _c_int(pad), _c_int(inner), _stream()), "head_mix_tiles_both")
 
     # -- many small products, routing ----------------------------------------------------------
     GROUPED_ACTS = {None: 0, "relu_squared": 1, "gated_silu": 2, "gated_gelu_tanh": 3, "gated_clamped": 4, "gelu_erf": 5}

@@ -68,6 +68,9 @@ class LaunchShape:
         self.e_numel, self.sums_numel = rows * row_e, rows * inner * self.score_ranges
         self.partial_numel = rows * row_o * self.value_ranges
 
+    def launch(self):
+        return self.ktiles, self.score_keys, self.score_ranges, self.value_keys, self.value_ranges, self.kv_block
+
 
 @register_part("mixer", "head_mix_attention")
 class HeadMixAttention:
@@ -189,16 +192,28 @@ class HeadMixAttention:
                                  gate, attn, *sizes, float(s.scale), s.softcap)
             return
         small, big, _ = ctx.token_groups(1, GROUP)
-        for (first, count, n), tokens in ((big, GROUP), (small, 1)):
-            if n == 0:
-                continue
-            shape = LaunchShape(s, self._layout(), n, tokens, ctx.max_context, ctx.target_workgroups // 2)
-            e = ctx.workspace.get("mix_e", (shape.e_numel,), q.dtype)
-            sums = ctx.workspace.get("mix_sums", (shape.sums_numel,), torch.float32)
-            partial = ctx.workspace.get("mix_partial", (shape.partial_numel,), torch.float32)
+        parts = [(part, tokens, LaunchShape(s, self._layout(), part[2], tokens, ctx.max_context, ctx.target_workgroups // 2))
+                 for part, tokens in ((big, GROUP), (small, 1)) if part[2]]
+        shapes = [shape for _, _, shape in parts]
+        total = lambda what: sum(getattr(shape, what) for shape in shapes)
+        together = (len(parts) == 2 and all(part[2] == shape.groups for part, _, shape in parts) and total("e_numel") <= SCRATCH_CAP
+                    and total("sums_numel") <= SUMS_CAP and total("partial_numel") <= PARTIAL_CAP
+                    and k.head_mix_both_supported(*sizes, s.softcap))
+        most = total if together else lambda what: max(getattr(shape, what) for shape in shapes)
+        e = ctx.workspace.get("mix_e", (most("e_numel"),), q.dtype)
+        sums = ctx.workspace.get("mix_sums", (most("sums_numel"),), torch.float32)
+        partial = ctx.workspace.get("mix_partial", (most("partial_numel"),), torch.float32)
+        before = (q, k_pages, v_pages, view.block_table, ctx.slots, ctx.positions, self.mix, self.sink, v_rope, gate, attn)
+        if together:
+            launch, at = [], (0, 0, 0)
+            for (first, count, n), _, shape in parts:
+                ends = (at[0] + shape.e_numel, at[1] + shape.sums_numel, at[2] + shape.partial_numel)
+                launch.append((first, count, n, e[at[0]:ends[0]], sums[at[1]:ends[1]], partial[at[2]:ends[2]], *shape.launch()))
+                at = ends
+            k.head_mix_tiles_both(*before, *launch, *sizes, float(s.scale), float(s.softcap))
+            return
+        for (first, count, n), tokens, shape in parts:
             for at in range(0, n, shape.groups):
                 some = min(shape.groups, n - at)
-                k.head_mix_tiles(q, k_pages, v_pages, view.block_table, ctx.slots, ctx.positions, self.mix, self.sink, v_rope,
-                                 gate, attn, first[at:at + some], count[at:at + some], some, tokens, *sizes, float(s.scale),
-                                 float(s.softcap), e, sums, partial, shape.ktiles, shape.score_keys, shape.score_ranges,
-                                 shape.value_keys, shape.value_ranges, shape.kv_block)
+                k.head_mix_tiles(*before, first[at:at + some], count[at:at + some], some, tokens, *sizes, float(s.scale),
+                                 float(s.softcap), e, sums, partial, *shape.launch())
