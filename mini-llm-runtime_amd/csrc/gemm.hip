@@ -1711,12 +1711,15 @@ extern "C" int mlr_gemm_heads(const void* a, long lda, long a_head, const void* 
 // layers at 20 row counts), against the library and the activation's launch, geometric mean: drawn sizes 0.82 plain and 0.84 gated,
 // where the better of both would be 0.81 and 0.82; the Qwen3 layers 0.91 and 1.00 (0.89 and 0.98); of all that this takes 0.38 to 1.32.
 // (A prediction of the library's time from its bytes, flops and k, within 16 %, chose no better.)
-// one_order: the sums must not turn on which plan the library's timing picks: timed row counts are judged as the others.
+// one_order: the sums must not turn on which plan the library's timing picks: timed row counts are judged as the others; and up to 64
+// rows the question is the tiles of one sum over k, as the library adds, up to 16384 rows of weight: 0.39 to 0.95 of the library's time and the
+// activation's launch at the sizes below it (105 products from 5632 rows of weight and k from 1024 to 4096 on, weights cold, but 1.00 for
+// 64 x 9216 x 3072: 48 x 8192 x 2048 13.8 -> 9.8 us, 48 x 5632 x 2048 13.2 -> 9.3, 24 x 12288 x 4096 26.1 -> 21.8), 0.82 to 1.16 beyond.
 extern "C" int mlr_gemm_wide_wins(int M, int N, int K, int act, int one_order) {
     const bool gated = act >= WIDE_SILU && act <= WIDE_CLAMPED;
     if (M <= 16 || N <= 0 || K <= 0 || !wide_takes(nullptr, nullptr, M, N, K, gated)) return 0;
-    if (M <= 64) return few_wins(M, N, K, gated) ? 1 : 0;
     const long long weight = (long long)N * (gated ? 2 : 1);
+    if (M <= 64) return (one_order ? weight <= 16384 : few_wins(M, N, K, gated)) ? 1 : 0;
     if ((K > 8192 && M * weight < (1 << 17)) || (M <= 128 && weight > 45000)) return 0;
     const float gflop = 2e-9f * (float)M * (float)weight * (float)K;
     if (M % 64 == 0 && !one_order) return gflop < 40.f ? 1 : 0;
@@ -1819,13 +1822,13 @@ extern "C" int mlr_gemm_qkv(const void* a, const void* w, int M, int K, void* q_
 }
 
 // out[M, N] = act of the products, act one of WIDE_SILU_ROUNDED .. (gated: w is [2N, K] = [gate; up]; limit and slope are
-// WIDE_CLAMPED's): the bits of the product followed by the activation's own kernel.
+// WIDE_CLAMPED's): the bits of the product followed by the activation's own kernel.  one_order: up to 64 rows, too, one sum over k.
 extern "C" int mlr_gemm_activated(const void* a, const void* w, void* out, int M, int N, int K, int act, float limit, float slope,
-                                  hipStream_t stream) {
+                                  int one_order, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
     if (K <= 0 || act < WIDE_SILU_ROUNDED || act > WIDE_GELU_ERF || (act == WIDE_CLAMPED && !(limit > 0.f))) return -1;
     if (!wide_takes(a, w, M, N, K, act <= WIDE_CLAMPED)) return -2;
-    return run_wide(M <= 64 ? WIDE_FEW : WIDE_MANY, a, w, out, M, N, K, false, act, limit, slope, stream);
+    return run_wide(M <= 64 && !one_order ? WIDE_FEW : WIDE_MANY, a, w, out, M, N, K, false, act, limit, slope, stream);
 }
 
 template <int WM, int WN, int TM, int TN>

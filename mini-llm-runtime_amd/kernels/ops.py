@@ -350,9 +350,9 @@ class Kernels:
         _need(k == k2, lambda: f"gemm: inner sizes differ ({k} and {k2})")
         _need(out.dtype in (self.dtype, torch.float32), lambda: f"gemm: output type {out.dtype} not supported")
         _tensor(out, "out", out.dtype, (m, n))
-        if m <= 64 and out.dtype == torch.bfloat16 and self.wide_product(m, n, k) and _on16(a, w):
-            _ok(self._lib("gemm").mlr_gemm_wide(_p(a), _p(w), _p(out), _c_int(m), _c_int(n), _c_int(k), _c_int(0), _c_int(-2), _c_int(0),
-                                                _stream()), "gemm")
+        if m <= 64 and out.dtype == torch.bfloat16 and (self.few_product(m, n, k) or self.wide_product(m, n, k)) and _on16(a, w):
+            _ok(self._lib("gemm").mlr_gemm_wide(_p(a), _p(w), _p(out), _c_int(m), _c_int(n), _c_int(k), _c_int(0),
+                                                _c_int(-1 if self.one_sum(m, k) else -2), _c_int(0), _stream()), "gemm")
             return
         if library and self.library_gemm and self.dtype == torch.bfloat16 and m > LIBRARY_GEMM_MIN_ROWS and \
                 (out.dtype == torch.float32 or not (self.streams_weight(m, k) or (self.wide_product(m, n, k) and _on16(a, w)))):
@@ -396,8 +396,12 @@ class Kernels:
             return False
         kind = self.WIDE_ACTS[act]
         weight_rows = columns * (2 if 1 <= kind <= 5 else 1)
-        if self.routed and (rows <= 64 or (self.library_gemm and not self.library_adds_alike(rows * weight_rows, k))):
-            return False
+        if self.routed:
+            if rows <= 64:
+                if self.streams_weight(rows, k) or not self.library_adds_few_alike(rows, weight_rows, k):
+                    return False
+            elif self.library_gemm and not self.library_adds_alike(rows * weight_rows, k):
+                return False
         key = (rows, columns, k, act)
         wins = self._wide_choices.get(key)
         if wins is None:
@@ -405,6 +409,27 @@ class Kernels:
                                                                    _c_int(1 if self.routed else 0)))
             if not self.library_gemm and rows > 64:
                 wins = k % 64 == 0 and rows * k < 2 ** 31 and weight_rows * k < 2 ** 31
+            if len(self._wide_choices) >= WIDE_CHOICES_KEPT:
+                self._wide_choices.clear()
+            self._wide_choices[key] = wins
+        return wins
+
+    def one_sum(self, rows, k):
+        """Whether the many-row kernel adds in one chain over k: the library's order, which a model that routes keeps.  Up to 64 rows it
+        otherwise adds as the kernels that stream the weight do."""
+        return rows > 64 or (self.routed and not self.streams_weight(rows, k))
+
+    def few_product(self, rows, columns, k, act=None):
+        """Whether the many-row kernel's narrow tiles take 17 to 64 rows in place of the kernels that stream the weight: with their
+        bits, so for a model that routes as well, which `wide_product` keeps with the library where these are not the ones to replace."""
+        if not self.routed:
+            return rows <= 64 and self.wide_product(rows, columns, k, act)
+        if not LIBRARY_GEMM_MIN_ROWS < rows <= 64 or not self.streams_weight(rows, k):
+            return False
+        key = (rows, columns, k, act, "few")
+        wins = self._wide_choices.get(key)
+        if wins is None:
+            wins = bool(self._lib("gemm").mlr_gemm_wide_wins(_c_int(rows), _c_int(columns), _c_int(k), _c_int(self.WIDE_ACTS[act]), _c_int(0)))
             if len(self._wide_choices) >= WIDE_CHOICES_KEPT:
                 self._wide_choices.clear()
             self._wide_choices[key] = wins
@@ -438,6 +463,13 @@ class Kernels:
         64 rows) it may choose one that cuts k, another one in another process: there this kernel's order is the lasting one, and a
         model that routes takes it by the rule for other row counts."""
         return 1 << 19 <= outputs < (1 << 24 if k <= 2048 else 1 << 23) and k <= 8704
+
+    @staticmethod
+    def library_adds_few_alike(rows, weight_rows, k):
+        """The same for 17 to 64 rows, where the library cuts k as long as the rows of weight are few: compared bit by bit on 30 000
+        products of k from 1024 to 4096 and weights of up to 2^26 elements, none differs from 5632 rows of weight on (beyond 32 rows; the last
+        that does has 5440) and from 8448 on (17 to 32; the last has 8192)."""
+        return (8448 if rows <= 32 else 5632) <= weight_rows and 1024 <= k <= 4096 and weight_rows * k <= 1 << 26
 
     # the epilogues of `gemm_activated` (csrc/gemm.hip, WIDE_*)
     WIDE_ACTS = {None: 0, "silu": 2, "gelu_tanh": 3, "relu": 4, "clamped": 5, "relu_squared": 6, "gelu_erf": 7}
@@ -482,7 +514,8 @@ class Kernels:
     def _gemm_activated(self, a, w, out, kind, limit, slope):
         (m, k), n = a.shape, out.shape[1]
         _ok(self._lib("gemm").mlr_gemm_activated(_p(a), _p(w), _p(out), _c_int(m), _c_int(n), _c_int(k), _c_int(self.WIDE_ACTS[kind]),
-                                                 _c_float(limit), _c_float(slope), _stream()), "gemm_activated")
+                                                 _c_float(limit), _c_float(slope), _c_int(1 if self.one_sum(m, k) else 0), _stream()),
+            "gemm_activated")
 
     def gated_silu_fused(self, rows, k=None, w=None):
         """Whether `gemm_gated_silu` is the path for this many rows and inner size: the bfloat16 engine, where
@@ -524,7 +557,7 @@ class Kernels:
     @timed("gemm", _gemm_work)
     def _gemm_gated_silu(self, a, w, out):
         (m, k), two_n = a.shape, w.shape[0]
-        if m <= 64 and self.wide_product(m, two_n // 2, k, "silu") and _on16(a, w):
+        if self.few_product(m, two_n // 2, k, "silu") and _on16(a, w):
             _ok(self._lib("gemm").mlr_gemm_wide(_p(a), _p(w), _p(out), _c_int(m), _c_int(two_n // 2), _c_int(k), _c_int(0), _c_int(-2),
                                                 _c_int(1), _stream()), "gemm_gated_silu")
             return

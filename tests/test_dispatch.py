@@ -248,6 +248,19 @@ def test_products_of_a_model_with_a_router_keep_the_order_of_their_sums(sizes):
     assert k.wide_product(1777, 3000, 2048, "silu") and not k.wide_product(1777, 6000, 2048, "silu")     # (a gate's outputs are two)
 
 
+@pytest.mark.parametrize("m,n,kk,act,taken,one_sum,few", [
+    (33, 5632, 2112, None, True, True, False), (64, 8192, 4096, "silu", True, True, False), (32, 8448, 2112, None, True, True, False),
+    (33, 5624, 2112, None, False, True, False), (32, 8192, 2112, None, False, True, False), (64, 16448, 4096, None, False, True, False),
+    (64, 5632, 4160, None, False, True, False), (33, 2816, 2112, "silu", True, True, False), (33, 5632, 2112, "gelu_erf", True, True, False),
+    (32, 8448, 2048, None, False, False, True), (64, 8448, 1024, "silu", False, False, True), (16, 8448, 2048, None, False, False, False)])
+def test_up_to_64_rows_of_a_model_with_a_router(m, n, kk, act, taken, one_sum, few):
+    """In place of the library tiles of one sum over k, where it adds so; in place of the kernels that stream the weight the narrow
+    tiles, whose sums are theirs.  (Asked with the kernels' own rule always answering yes.)"""
+    k = kernels_without_gpu(routed=True)
+    k._wide_choices = {(m, n, kk, act): True, (m, n, kk, act, "few"): True}
+    assert (k.wide_product(m, n, kk, act), k.one_sum(m, kk), k.few_product(m, n, kk, act)) == (taken, one_sum, few)
+
+
 @pytest.mark.parametrize("shift_q,shift_out", [(0, 0), (1, 0), (0, 1)])
 def test_rows_that_do_not_start_on_16_bytes_keep_the_attention_that_takes_them(shift_q, shift_out):
     """Queries or results that are views off 16 bytes: the prompt portions' kernel for whole rows does not take them, the general one

@@ -460,6 +460,43 @@ def test_the_library_adds_alike_where_models_with_a_router_leave_it(m, n, kk):
     assert torch.equal(act, one)
 
 
+@pytest.mark.parametrize("m,n,kk", [(33, 5632, 1408), (33, 5632, 4096), (47, 5640, 2048), (48, 8192, 2048), (63, 16384, 4096), (50, 11264, 1088), (17, 8448, 2112),
+                                    (25, 8456, 4096), (32, 16384, 3072)])
+def test_up_to_64_rows_add_as_the_library_does_in_a_model_with_a_router(m, n, kk):
+    """Inside and at the edges of `library_adds_few_alike`: the library's bits, plain and with the activation behind it."""
+    from mini_llm_runtime_amd.kernels import Kernels
+    k, library = Kernels(torch.bfloat16, routed=True), Kernels(torch.bfloat16, routed=True)
+    assert k.wide_product(m, n, kk) and k.wide_product(m, n // 2, kk, "silu") and k.one_sum(m, kk)
+    library.wide_product = lambda *sizes: False
+    a, w = rnd((m, kk), torch.bfloat16, 41), rnd((n, kk), torch.bfloat16, 42, 0.05)
+    out, own = (torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    library.gemm(a, w, out)
+    k.gemm(a, w, own)
+    assert torch.equal(out, own)
+    act, one = (torch.full((m, n // 2), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    for kind in ("silu", "relu", "clamped"):
+        k._product_then_activation(a, w, act, kind, 7.0, 1.702)
+        k.gemm_activated(a, w, one, kind, 7.0, 1.702)
+        assert torch.equal(act, one), kind
+
+
+@pytest.mark.parametrize("m,n,kk", [(17, 6144, 2048), (32, 2816, 2048), (33, 512, 1024), (64, 12288, 1024), (24, 8448, 1984), (48, 30, 704)])
+def test_the_narrow_tiles_of_a_model_with_a_router_have_the_streamed_kernels_bits(m, n, kk):
+    from mini_llm_runtime_amd.kernels import Kernels
+    k, streamed = Kernels(torch.bfloat16, routed=True), Kernels(torch.bfloat16, routed=True)
+    assert k.few_product(m, n, kk) and not k.wide_product(m, n, kk)
+    streamed.few_product = lambda *sizes: False
+    a, w = rnd((m, kk), torch.bfloat16, 43), rnd((n, kk), torch.bfloat16, 44, 0.05)
+    out, own = (torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    streamed.gemm(a, w, out)
+    k.gemm(a, w, own)
+    assert torch.equal(out, own)
+    act, one = (torch.full((m, n // 2), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    streamed.gemm_gated_silu(a, w, act)
+    k.gemm_gated_silu(a, w, one)
+    assert torch.equal(act, one)
+
+
 def test_gemm_float_of_an_inner_size_beyond_32_bits_of_bytes():
     """16 rows of 2^26 floats are 2^32 bytes, one more than the few-row kernel's loads reach: the product is the tiles', plain and
     beside an activation.  (Whole numbers: exact.)"""
