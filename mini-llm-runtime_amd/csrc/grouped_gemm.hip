@@ -544,125 +544,138 @@ static int run_experts_wide(int shape, const GroupedArgs& g, hipStream_t stream)
 #endif
 
 // ---------------------------------------------------------------------------------------------------------
-#define MAX_EXPERTS 256         // 64 lanes x EXPERT_REGS
-#define EXPERT_REGS 4
+#define MAX_EXPERTS 256
 
-// The largest value among the lanes' candidates and, among equals, the lowest index; every lane gets both.
-__device__ __forceinline__ void wave_best(float& value, int& index) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const float ov = __shfl_xor(value, off, MLR_WAVE);
-        const int oi = __shfl_xor(index, off, MLR_WAVE);
-        if (ov > value || (ov == value && oi < index)) {
-            value = ov;
-            index = oi;
-        }
-    }
-}
+struct Routing {
+    int experts, top, group_count, group_keep, renorm, softmax, group_best;
+    const float* correction;
+    float out_scale;
+};
 
-// One wavefront a token.  s = sigmoid(z), or softmax(z) over all experts (`softmax`), z[m * ld ..] the token's router
+// A token a workgroup, an expert a thread.  s = sigmoid(z), or softmax(z) over all experts (`softmax`), z[m * ld ..] the token's router
 // logits (float: a product of the framework's own, 32-bit sums).  The experts form `group_count`
 // equal groups of neighbours; a group's score is the sum of its two largest s (of its only one, when a group is
 // one expert), or its largest (`group_best`); only experts of the `group_keep` best groups stand; of
 // those the `top` largest s are chosen (ties: the lower index), ids[m][i] in descending order of s with weights[m][i] = s itself.
 // With `correction` [experts] the choice (of groups and of experts) goes by s + correction while the weights stay
 // the plain s; with `renorm` the chosen weights are divided by their sum (+ 1e-20); `out_scale` multiplies them.
-__global__ __launch_bounds__(64) void router_topk_kernel(const float* __restrict__ z, long ld, int32_t* __restrict__ ids,
-                                                         float* __restrict__ weights, int experts, int top,
-                                                         int group_count, int group_keep,
-                                                         const float* __restrict__ correction, int renorm, float out_scale,
-                                                         int softmax, int group_best) {
-    __shared__ float s_lds[MAX_EXPERTS];      // what the choice goes by
-    __shared__ float w_lds[MAX_EXPERTS];      // the plain scores
-    __shared__ float g_lds[MAX_EXPERTS];
-    const int m = blockIdx.x, lane = threadIdx.x;
-    const float* zr = z + (size_t)m * ld;
-    float z_max = 0.f, z_sum = 1.f;
-    if (softmax) {
+//
+// Bound by its chain of dependent steps, not by work: so a place in the order is counted, by every thread for its own expert against
+// all others, where one choice after the other took six exchanges between lanes each, and one group for all needs no rounds.
+// 48 tokens, 4 of 20 experts: 7.8 -> 3.4 us; 8 of 64 in 4 of 8 groups 11.6 -> 4.6, of 256 14.7 -> 10.4; 1777 tokens, 4 of 16: 8.7 -> 3.6.
+// (The choice and the sort below in one launch of one workgroup, three tokens a wavefront: 10.7 us for 3.4 and 2.0.)
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void router_topk_kernel(const float* __restrict__ z, long ld, Routing r,
+                                                                 int32_t* __restrict__ ids, float* __restrict__ weights) {
+    __shared__ __attribute__((aligned(16))) int keys[64 * WAVES];
+    __shared__ float by[64 * WAVES];                                       // what the choice goes by
+    __shared__ float plain[64 * WAVES];                                    // the plain scores
+    __shared__ float group[64 * WAVES];
+    __shared__ int choice[64 * WAVES];
+    const int e = threadIdx.x, experts = r.experts, lane = e % 64;
+    const float* zr = z + (size_t)blockIdx.x * ld;
+    const bool expert = e < experts;
+    const float logit = expert ? zr[e] : 0.f;
+    float z_max = 0.f, z_sum = 1.f, cand = -INFINITY;
+    if (r.softmax) {                                                       // (each wavefront by itself)
         z_max = -INFINITY;
-        for (int e = lane; e < experts; e += 64) z_max = fmaxf(z_max, zr[e]);
+        for (int o = lane; o < experts; o += 64) z_max = fmaxf(z_max, zr[o]);
         z_max = wave_max(z_max);
         z_sum = 0.f;
-        for (int e = lane; e < experts; e += 64) z_sum += expf(zr[e] - z_max);
+        for (int o = lane; o < experts; o += 64) z_sum += expf(zr[o] - z_max);
         z_sum = wave_sum(z_sum);
     }
-    for (int e = lane; e < experts; e += 64) {
-        const float sc = softmax ? expf(zr[e] - z_max) / z_sum : 1.0f / (1.0f + expf(-zr[e]));
-        w_lds[e] = sc;
-        s_lds[e] = correction != nullptr ? sc + correction[e] : sc;
+    if (expert) {
+        const float sc = r.softmax ? expf(logit - z_max) / z_sum : 1.0f / (1.0f + expf(-logit));
+        plain[e] = sc;
+        cand = r.correction != nullptr ? sc + r.correction[e] : sc;
     }
+    if (e < r.top) choice[e] = 0;                                          // (fewer candidates than `top`: refused on the host)
+    const int per = experts / r.group_count;
+    if (r.group_count == 1) {
+        // the group stands if its score is more than -inf: two of its values (or one) are
+        const int there = WAVES == 1 ? __popcll(__ballot(cand > -INFINITY)) : __syncthreads_count(cand > -INFINITY);
+        if (there < (per >= 2 && !r.group_best ? 2 : 1)) cand = -INFINITY;
+    } else {
+        by[e] = cand;
+        __syncthreads();
+        if (e < r.group_count) {
+            float first = -INFINITY, second = -INFINITY;
+            for (int i = 0; i < per; ++i) {
+                const float v = by[e * per + i];
+                if (v > first) {
+                    second = first;
+                    first = v;
+                } else if (v > second) {
+                    second = v;
+                }
+            }
+            group[e] = per >= 2 && !r.group_best ? first + second : first;
+        }
+        __syncthreads();
+        if (expert) {
+            const int mine = e / per;
+            const float score = group[mine];
+            int before = 0;
+            for (int g = 0; g < r.group_count; ++g) {
+                const float v = group[g];
+                before += v > score || (v == score && g < mine) ? 1 : 0;
+            }
+            if (!(score > -INFINITY && before < r.group_keep)) cand = -INFINITY;
+        }
+    }
+    // As whole numbers in the order of the floats (no candidate: the lowest), so that among equals the lower index is the larger by one
+    // subtraction: four operations a pair, none of them on masks.
+    constexpr int NONE = -0x7fffffff - 1;
+    const int bits = __float_as_int(cand + 0.0f);                          // (0 for -0)
+    const int key = cand > -INFINITY ? bits ^ ((bits >> 31) & 0x7fffffff) : NONE;
+    keys[e] = key;
     __syncthreads();
-    const int per = experts / group_count;
-    for (int gidx = lane; gidx < group_count; gidx += 64) {
-        float first = -INFINITY, second = -INFINITY;
-        for (int i = 0; i < per; ++i) {
-            const float v = s_lds[gidx * per + i];
-            if (v > first) {
-                second = first;
-                first = v;
-            } else if (v > second) {
-                second = v;
-            }
+    int before = 0;
+    for (int j = 0; j < experts; j += 16) {                                // (16 at once: their reads are under way together)
+        int4 v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = *reinterpret_cast<const int4*>(&keys[j + 4 * q]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int at = j + 4 * q;
+            before += v[q].x > key - (at < e ? 1 : 0) ? 1 : 0;
+            before += v[q].y > key - (at + 1 < e ? 1 : 0) ? 1 : 0;
+            before += v[q].z > key - (at + 2 < e ? 1 : 0) ? 1 : 0;
+            before += v[q].w > key - (at + 3 < e ? 1 : 0) ? 1 : 0;
         }
-        g_lds[gidx] = per >= 2 && !group_best ? first + second : first;
     }
+    if (key != NONE && before < r.top) choice[before] = e;
     __syncthreads();
-    // the groups that stand: group_keep times the best of those left; their experts become candidates
-    float cand[EXPERT_REGS];
-#pragma unroll
-    for (int i = 0; i < EXPERT_REGS; ++i) cand[i] = -INFINITY;
-    for (int round = 0; round < group_keep; ++round) {
-        float best = -INFINITY;
-        int which = 0x7fffffff;
-        for (int gidx = lane; gidx < group_count; gidx += 64) {
-            const float v = g_lds[gidx];
-            if (v > best) {                    // (ascending indices: the lowest among equals stays)
-                best = v;
-                which = gidx;
-            }
-        }
-        wave_best(best, which);
-        if (which == 0x7fffffff) break;
-        __syncthreads();
-        if (lane == 0) g_lds[which] = -INFINITY;
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < EXPERT_REGS; ++i) {
-            const int e = lane + 64 * i;
-            if (e < experts && e / per == which) cand[i] = s_lds[e];
-        }
+    if (e >= r.top) return;
+    const int which = choice[e];
+    float w = plain[which];
+    if (r.renorm) {
+        float sum = 0.f;
+        for (int c = 0; c < r.top; ++c) sum += plain[choice[c]];           // (in the order of the choices)
+        w = w / (sum + 1e-20f);
     }
-    float chosen_sum = 0.f;
-    for (int round = 0; round < top; ++round) {
-        float best = -INFINITY;
-        int which = 0x7fffffff;
+    ids[(size_t)blockIdx.x * r.top + e] = which;
+    weights[(size_t)blockIdx.x * r.top + e] = r.renorm || r.out_scale != 1.0f ? w * r.out_scale : w;
+}
+
+// Where the experts' rows of the sorted list start: start[e] the sum of count[0 .. e - 1], offsets[experts] of all; one wavefront
+// (one thread from expert to expert: 256 of them, 4.6 us of the sort below for 3.0).
+__device__ __forceinline__ void expert_starts(const int* count, int experts, int* start, int32_t* __restrict__ offsets) {
+    const int lane = threadIdx.x % 64;
+    int before = 0;
+    for (int e0 = 0; e0 < experts; e0 += 64) {
+        const int own = e0 + lane < experts ? count[e0 + lane] : 0;
+        int sum = own;
 #pragma unroll
-        for (int i = 0; i < EXPERT_REGS; ++i) {
-            const int e = lane + 64 * i;
-            if (e < experts && cand[i] > best) {
-                best = cand[i];
-                which = e;
-            }
+        for (int off = 1; off < 64; off *= 2) {
+            const int other = __shfl_up(sum, off, MLR_WAVE);
+            if (lane >= off) sum += other;
         }
-        wave_best(best, which);
-        if (which == 0x7fffffff) which = 0, best = 0.f;      // (fewer candidates than `top`: refused on the host)
-#pragma unroll
-        for (int i = 0; i < EXPERT_REGS; ++i)
-            if (lane + 64 * i == which) cand[i] = -INFINITY;
-        chosen_sum += w_lds[which];                           // (the same on every lane, in the order of the choices)
-        if (lane == 0) {
-            ids[(size_t)m * top + round] = which;
-            weights[(size_t)m * top + round] = w_lds[which];
-        }
+        if (e0 + lane < experts) offsets[e0 + lane] = start[e0 + lane] = before + sum - own;
+        before += __shfl(sum, 63, MLR_WAVE);
     }
-    if (renorm || out_scale != 1.0f) {
-        __syncthreads();
-        for (int r = lane; r < top; r += 64) {
-            float w = weights[(size_t)m * top + r];
-            if (renorm) w = w / (chosen_sum + 1e-20f);
-            weights[(size_t)m * top + r] = w * out_scale;
-        }
-    }
+    if (lane == 0) offsets[experts] = before;
 }
 
 // The `pairs` chosen (token, expert) pairs sorted by expert, by ONE workgroup: offsets[e] .. offsets[e + 1] are
@@ -671,23 +684,14 @@ __global__ __launch_bounds__(64) void router_topk_kernel(const float* __restrict
 __global__ __launch_bounds__(1024) void route_sort_kernel(const int32_t* __restrict__ ids, int pairs, int top,
                                                           int experts, int32_t* __restrict__ offsets,
                                                           int32_t* __restrict__ token_of, int32_t* __restrict__ row_of) {
-    __shared__ int count[MAX_EXPERTS + 1];
+    __shared__ int count[MAX_EXPERTS];
     __shared__ int cursor[MAX_EXPERTS];
     const int t = threadIdx.x;
-    for (int e = t; e <= experts; e += blockDim.x) count[e] = 0;
+    for (int e = t; e < experts; e += blockDim.x) count[e] = 0;
     __syncthreads();
     for (int i = t; i < pairs; i += blockDim.x) atomicAdd(&count[ids[i]], 1);
     __syncthreads();
-    if (t == 0) {
-        int at = 0;
-        for (int e = 0; e < experts; ++e) {
-            const int n = count[e];
-            cursor[e] = at;
-            offsets[e] = at;
-            at += n;
-        }
-        offsets[experts] = at;
-    }
+    if (t < 64) expert_starts(count, experts, cursor, offsets);
     __syncthreads();
     for (int i = t; i < pairs; i += blockDim.x) {
         const int row = atomicAdd(&cursor[ids[i]], 1);
@@ -798,8 +802,9 @@ int mlr_router_topk(const float* z, long ld, int32_t* ids, float* weights, int r
     if (ld < experts || experts < 1 || experts > MAX_EXPERTS || group_count < 1 || experts % group_count != 0 || group_keep < 1 ||
         group_keep > group_count || top < 1 || top > group_keep * (experts / group_count))
         return -1;
-    router_topk_kernel<<<rows, 64, 0, stream>>>(z, ld, ids, weights, experts, top, group_count, group_keep, correction, renorm,
-                                                out_scale, softmax, group_best);
+    const Routing r{experts, top, group_count, group_keep, renorm, softmax, group_best, correction, out_scale};
+    if (experts <= 64) router_topk_kernel<1><<<rows, 64, 0, stream>>>(z, ld, r, ids, weights);
+    else router_topk_kernel<4><<<rows, 256, 0, stream>>>(z, ld, r, ids, weights);
     return (int)hipGetLastError();
 }
 
