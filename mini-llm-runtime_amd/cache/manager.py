@@ -29,6 +29,7 @@ import numpy as np
 import torch
 
 from ..kernels import build
+from ..kernels.ops import PinnedCopy
 
 
 class CacheError(RuntimeError):
@@ -158,6 +159,8 @@ class PageBook:
             raise CacheError("max_slots and max_length must be positive")
         self.max_slots, self.max_length = max_slots, max_length
         self.groups = []                  # (page_size, num_pages, window)
+        self._commit_into = None
+        self._dirty = (ctypes.c_int32 * max_slots)()
 
     def __del__(self):
         h, self._h = getattr(self, "_h", None), None
@@ -245,6 +248,19 @@ class PageBook:
             self._raise(rc, -1, (0, 0))
         return first.tolist()
 
+    def commit_into(self, slots, counts, first, at=None):
+        """`commit_first` on int32 numpy vectors, the positions written into `first`; `at`: pointers to (anything, the counts, the slots,
+        the positions), where the caller has them."""
+        fn = self._commit_into
+        if fn is None:
+            fn = self._commit_into = self._lib["mlr_cache_commit_first"]
+            fn.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p]
+        _, counts_at, slots_at, first_at = at if at is not None else (None, counts.ctypes.data, slots.ctypes.data, first.ctypes.data)
+        rc = fn(self._h, slots_at, counts_at, len(slots), first_at)
+        if rc != 0:
+            self.prepare(slots, counts)           # raises the precise error
+            self._raise(rc, -1, (0, 0))
+
     def retire(self, slots):
         s, sp = _i32(slots)
         rc = self._lib.mlr_cache_retire(self._h, sp, len(s))
@@ -253,9 +269,9 @@ class PageBook:
         return rc
 
     def take_dirty(self, group=0):
-        out = np.empty(self.max_slots, dtype=np.int32)
-        n = self._lib.mlr_cache_take_dirty(self._h, group, out.ctypes.data_as(ctypes.POINTER(ctypes.c_int32)))
-        return out[:n].tolist()
+        out = self._dirty
+        n = self._lib.mlr_cache_take_dirty(self._h, group, out)
+        return out[:n]
 
     def check(self):
         rc = self._lib.mlr_cache_check(self._h)
@@ -360,7 +376,7 @@ class CacheManager:
             table = torch.full((max_slots + 1, self.book.max_blocks(g)), -1, dtype=torch.int32, device=self.device)
             table[max_slots, 0] = pages
             self._tables.append(table)
-        self._stages = {}                # group -> [pinned copy of its table, event of the last upload, in use]
+        self._stages = {}                # group -> (copies of its table, the pinned memory they leave, as a numpy array, the table)
         # State of fixed size: a live slab, which mixers read, and a staged one, into which they write the
         # state their step leads to; the staged rows of a step's requests become live when every layer has
         # run (`commit_state`), so a step that fails on the way leaves the live state as it was.
@@ -495,6 +511,10 @@ class CacheManager:
         self.sync_tables()
         return first
 
+    def commit_into(self, slots, counts, first, at=None):
+        self.book.commit_into(slots, counts, first, at)
+        self.sync_tables()
+
     def retire(self, slots):
         """After a step: what it wrote becomes the requests' state (paired entries), and what windows have passed is
         given back.  The device tables are brought up to date before the next step (commit)."""
@@ -511,26 +531,25 @@ class CacheManager:
             rows = self.book.take_dirty(g)
             if not rows:
                 continue
-            host = torch.from_numpy(self.book.table(g))
             if dev.device.type != "cuda":
-                dev[:self.max_slots].copy_(host)
+                dev[:self.max_slots].copy_(torch.from_numpy(self.book.table(g)))
                 continue
             stage = self._stages.get(g)
             if stage is None:
-                stage = self._stages[g] = [torch.empty(tuple(host.shape), dtype=torch.int32).pin_memory(),
-                                           torch.cuda.Event(), False]
-            pinned, event, busy = stage
-            if busy:
-                event.synchronize()
-            if len(rows) * 4 >= self.max_slots:
-                pinned.copy_(host)
-                dev[:self.max_slots].copy_(pinned, non_blocking=True)
-            else:
-                for s in rows:
-                    pinned[s].copy_(host[s])
-                    dev[s].copy_(pinned[s], non_blocking=True)
-            event.record()
-            stage[2] = True
+                host = self.book.table(g)
+                pinned = torch.empty(host.shape, dtype=torch.int32).pin_memory()
+                stage = self._stages[g] = (PinnedCopy(), pinned, pinned.numpy(), host)
+            copy, pinned, view, host = stage
+            copy.wait()
+            row = 4 * host.shape[1]
+            # one copy of the rows between the first and the last that changed, as long as that is not much more than the rows: a copy
+            # takes as long as 64 KB of one
+            spans = [(rows[0], rows[-1] + 1)]
+            if (rows[-1] + 1 - rows[0]) * row > 65536 * len(rows):
+                spans = [(s, s + 1) for s in rows]
+            for low, high in spans:
+                view[low:high] = host[low:high]
+                copy.copy(dev, pinned.data_ptr() + low * row, (high - low) * row, low * row)
 
     def check(self):
         self.book.check()

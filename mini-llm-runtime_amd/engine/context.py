@@ -1,8 +1,11 @@
 """What a part may see of the running step, and the scratch memory it may use."""
 from __future__ import annotations
 
-import numpy as np
+import ctypes
+
 import torch
+
+from ..kernels.ops import PinnedCopy
 
 
 class Workspace:
@@ -81,27 +84,30 @@ class Uploader:
 
     def __init__(self, capacity, device):
         self.device = torch.device(device)
+        self._copy = PinnedCopy()
+        self._reserve(capacity)
+
+    def _reserve(self, capacity):
         self._host = torch.empty(capacity, dtype=torch.int32).pin_memory()
-        self._event = torch.cuda.Event()
-        self._busy = False
+        self._view = self._host.numpy()
+        self.address = ctypes.c_void_p(self._host.data_ptr())
+
+    def stage(self, n):
+        """The buffer's first n values as an int32 numpy vector, free to be written."""
+        self._copy.wait()
+        if n > self._view.size:
+            self._reserve(max(n, 2 * self._view.size))
+        return self._view[:n]
+
+    def upload(self, n, dst):
+        """The first n values to the device int32 vector dst, which holds at least that many."""
+        self._copy.copy(dst, self.address, 4 * n)
 
     def send(self, values, dst):
         """values: a list of ints or an int32 numpy vector; dst: device int32 vector of at least that many elements."""
         n = len(values)
-        if n > self._host.numel():
-            if self._busy:
-                self._event.synchronize()
-                self._busy = False
-            self._host = torch.empty(max(n, 2 * self._host.numel()), dtype=torch.int32).pin_memory()
-        if self._busy:
-            self._event.synchronize()
-        if isinstance(values, np.ndarray):
-            self._host.numpy()[:n] = values               # (a view of the pinned buffer: one copy, no tensor made)
-        else:
-            self._host[:n] = torch.tensor(values, dtype=torch.int32)
-        dst[:n].copy_(self._host[:n], non_blocking=True)
-        self._event.record()
-        self._busy = True
+        self.stage(n)[:] = values
+        self.upload(n, dst)
 
 
 # Single tokens that fill the GPU without a split, one workgroup a token and kv head: the longest context of the batch would

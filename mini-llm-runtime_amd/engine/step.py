@@ -7,6 +7,7 @@ windows have passed.  Generation, trace replay and the benchmark all go through 
 """
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass, field
 from typing import List, Sequence
 
@@ -14,7 +15,7 @@ import numpy as np
 import torch
 
 from ..cache.manager import CacheManager
-from ..kernels import Kernels
+from ..kernels import Kernels, build
 from ..kernels.ops import LIBRARY_GEMM_WORKSPACE
 from ..kernels.profile import Profiler
 from .context import StepContext, Uploader, Workspace
@@ -34,6 +35,20 @@ class Entry:
     slot: int
     tokens: Sequence[int]
     want: Sequence[int] = field(default_factory=list)     # places among `tokens` whose logits are asked for
+
+
+@dataclass
+class _Batch:
+    """A checked batch: int32 vectors over its entries (numbers of tokens, slots, first positions once the pages are taken) and
+    over its tokens and wanted rows."""
+    total: int
+    ids: np.ndarray
+    counts: np.ndarray
+    slots: np.ndarray
+    want_rows: np.ndarray
+    single: bool                      # every entry is one token that wants its logits
+    first: np.ndarray
+    at: tuple                         # where ids, counts, slots and first lie
 
 
 def _kv_dtype(name, engine_dtype):
@@ -142,6 +157,14 @@ class Runner:
         # it (a value a token), wanted rows, and -- for a model that keeps other state per request -- one slot per entry
         self._lanes = 4 if self.cache.has_pairs() else 3
         self._upload = Uploader(6 * self.max_batch_tokens, self.device)
+        self._inputs = build.load("step_inputs")
+        # (ids, counts, slots, numbers of wanted places, first positions: a value a token; wanted rows; totals)
+        self._plain = [np.empty(self.max_batch_tokens, np.int32) for _ in range(5)] + [np.empty(max(self.max_logits_rows, 1), np.int32),
+                                                                                       np.empty(4, np.int32)]
+        ids, counts, slots, places, first, rows, totals = (ctypes.c_void_p(v.ctypes.data) for v in self._plain)
+        self._plain_at = (ids, counts, slots, first)
+        self._plain_args = (ctypes.c_long(model.spec.vocab_size), self.max_batch_tokens, self.max_logits_rows, ids, counts, slots, places,
+                            rows, totals)
         self._meta = torch.empty(6 * self.max_batch_tokens, dtype=torch.int32, device=self.device)
         self.poisoned = False
         self.steps = 0
@@ -178,7 +201,7 @@ class Runner:
         """What a captured step is fixed to: how many tokens every entry brings and where it wants logits."""
         return tuple((len(e.tokens), tuple(int(w) for w in e.want)) for e in entries)
 
-    def _decode_fill(self, entries):
+    def _decode_fill(self, entries, single=False):
         """(rows of the scratch request, where they go) that fill the single tokens of a batch (each wanting
         its logits) up to a number that comes again: every number up to 8, even ones up to 16, multiples of 4
         up to 64, of 8 beyond.  So that a server whose requests come and go captures a few dozen graphs, not
@@ -187,7 +210,7 @@ class Runner:
         gets them in front, so that the wanted logits stay one block of rows."""
         if self.cache.scratch_slot is None or not self.use_graphs:
             return 0, False
-        n = 0
+        n = len(entries) if single else 0              # (`single`: every entry is such a token)
         while n < len(entries) and len(entries[n].tokens) == 1 and list(entries[n].want) == [0]:
             n += 1
         mixed = n < len(entries)
@@ -195,8 +218,9 @@ class Runner:
             return 0, False
         step = 1 if n <= 8 else 2 if n <= 16 else 4 if n <= 64 else 8
         fill = -(-n // step) * step - n
-        total = sum(len(e.tokens) for e in entries) + fill
-        wanted = sum(len(e.want) for e in entries) + fill       # (the scratch rows' logits are computed and dropped)
+        # (the scratch rows' logits are computed and dropped)
+        total = n + fill if single else sum(len(e.tokens) for e in entries) + fill
+        wanted = n + fill if single else sum(len(e.want) for e in entries) + fill
         if (n + fill > self.graph_max_batch or total > min(self.graph_max_tokens, self.max_batch_tokens)
                 or wanted > self.max_logits_rows):
             return 0, False
@@ -212,7 +236,7 @@ class Runner:
             bucket *= 2
         return min(bucket, self.max_length)
 
-    def _graph_wanted(self, entries, total, sig):
+    def _graph_wanted(self, single, total, sig):
         """Steps are launch-bound unless they bring many tokens.  Steps of single tokens with logits for
         each (decoding) are captured the second time they come, others (portions beside decoded tokens)
         once their shape has come `graph_after` times: a prompt's last portion rarely comes again."""
@@ -221,7 +245,7 @@ class Runner:
         if sig in self._graphs:
             return True
         shape = sig[0]
-        if total == len(shape) and all(w == (0,) for _, w in shape):
+        if single or (total == len(shape) and all(w == (0,) for _, w in shape)):
             return total <= self.graph_max_batch
         seen = self._seen.get(sig, 0) + 1
         self._seen[sig] = seen
@@ -244,7 +268,7 @@ class Runner:
                 return False
         return True
 
-    def _graph_step(self, entries, arrays, first, total, sig, fill=0, fill_first=False):
+    def _graph_step(self, batch, total, sig, fill=0, fill_first=False):
         """The same kernels as any step, launched from a captured graph.  The graph's buffers are fixed:
         token ids, positions and slots live in a vector of their own per shape (the wanted rows and the
         token groups, which depend on the shape only, are written there once), key splits are laid out
@@ -273,13 +297,17 @@ class Runner:
         else:
             self._graphs[sig] = self._graphs.pop(sig)        # most recently used last
         meta = state["meta"]
-        rows_of, segments = self._rows(entries, arrays, first, fill, fill_first)
-        n_seg, per_token = len(segments), self._lanes * total
-        state["upload"].send(np.concatenate([rows_of.ravel(), np.fromiter((seg[0] for seg in segments), np.int32, n_seg)]),
-                             meta)
+        n_seg, per_token = len(shape), self._lanes * total
+        vector = state["upload"].stage(per_token + n_seg)
+        self._put_rows(batch, state["upload"], vector, fill, fill_first)
+        at = per_token + (fill if fill_first else 0)
+        vector[per_token:] = self.cache.scratch_slot or 0
+        vector[at:at + len(batch.slots)] = batch.slots
+        state["upload"].upload(per_token + n_seg, meta)
         if state["graph"] is not None:
             state["graph"].replay()
             return state["logits"]
+        segments = self._segments(batch, fill, fill_first)
         ctx = self.ctx
         ctx.begin_step()
         ctx.n_tokens = total
@@ -387,9 +415,25 @@ class Runner:
         return sum(1 for st in self._graphs.values() if st["graph"] is not None) - before
 
     # -- the step ------------------------------------------------------------------------------
-    def _validate(self, entries):
+    def _gather(self, entries):
+        """The batch of `entries`: a plain one in one native pass, any other, and what must be refused, entry by entry."""
         if self.poisoned:
             raise StepError("an earlier step failed after it had started; build a new runner")
+        ids, counts, slots, _, first, rows, totals = self._plain
+        if self._inputs.mlr_step_entries(ctypes.py_object(entries), *self._plain_args) == 0:
+            n, total, r, single = totals.tolist()
+            return _Batch(total, ids[:total], counts[:n], slots[:n], rows[:r], bool(single), first[:n], self._plain_at)
+        total, arrays, wanted = self._validate(entries)
+        counts = np.array([len(a) for a in arrays], dtype=np.int32)
+        base = np.cumsum(counts) - counts
+        ids = np.concatenate([np.asarray(a, dtype=np.int32) for a in arrays])
+        slots = np.array([e.slot for e in entries], dtype=np.int32)
+        rows = np.concatenate([b + np.asarray(w, dtype=np.int64) for b, w in zip(base, wanted)]).astype(np.int32)
+        first = np.empty(len(entries), dtype=np.int32)
+        return _Batch(total, ids, counts, slots, rows, False, first,
+                      tuple(ctypes.c_void_p(v.ctypes.data) for v in (ids, counts, slots, first)))
+
+    def _validate(self, entries):
         if not entries:
             raise StepError("empty batch")
         vocab = self.model.spec.vocab_size
@@ -439,7 +483,7 @@ class Runner:
                 if not inside:
                     raise StepError(f"token id {t} is outside the vocabulary [0, {vocab})" if isinstance(t, (int, np.integer))
                                     else "token ids must be whole numbers")
-            return tokens                                 # (as they came: `_rows` puts them into its vector)
+            return tokens                                 # (as they came: `_gather` puts them into its vector)
         ids = np.asarray(tokens)
         if ids.ndim != 1 or ids.dtype.kind not in "iub":
             try:                                          # (numbers too large for a machine word, or no numbers)
@@ -453,97 +497,72 @@ class Runner:
             raise StepError(f"token id {ids[outside][0]} is outside the vocabulary [0, {vocab})")
         return ids.astype(np.int32)
 
-    def _rows(self, entries, arrays, first, fill=0, fill_first=False):
-        """(token ids | positions | slots of the step's rows as int32 [3, rows], or with the live rows of paired state [4, rows],
-        the segments (slot, first row, tokens, first position)); `fill` rows of the scratch request (token 0 at position 0) in
-        front or behind."""
-        total = sum(len(a) for a in arrays) + fill
-        scratch = self.cache.scratch_slot
-        if total <= 4 * (len(entries) + fill):
-            # mostly single tokens (a decoding step): three short lists and one conversion cost less than
-            # a few vector operations for every entry
-            ids, pos, slot_of, segments = [], [], [], []
-            if fill and fill_first:
-                segments = [(scratch, i, 1, 0) for i in range(fill)]
-                ids, pos, slot_of = [0] * fill, [0] * fill, [scratch] * fill
-            for e, tokens, p0 in zip(entries, arrays, first):
-                n = len(tokens)
-                segments.append((e.slot, len(ids), n, p0))
-                ids.extend(tokens)
-                pos.extend(range(p0, p0 + n))
-                slot_of.extend([e.slot] * n)
-            if fill and not fill_first:
-                segments += [(scratch, len(ids) + i, 1, 0) for i in range(fill)]
-                ids, pos, slot_of = ids + [0] * fill, pos + [0] * fill, slot_of + [scratch] * fill
-            lanes = [ids, pos, slot_of] if self._lanes == 3 else [ids, pos, slot_of, self.cache.state_rows(slot_of)]
-            return np.array(lanes, dtype=np.int32), segments
-        rows = np.empty((self._lanes, total), dtype=np.int32)
-        segments, at = [], 0
-        if fill and fill_first:
-            rows[0:2, :fill], rows[2, :fill] = 0, scratch
-            segments += [(scratch, i, 1, 0) for i in range(fill)]
-            at = fill
-        for e, ids, p0 in zip(entries, arrays, first):
-            n = len(ids)
-            rows[0, at:at + n] = ids
-            rows[1, at:at + n] = np.arange(p0, p0 + n, dtype=np.int32)
-            rows[2, at:at + n] = e.slot
-            segments.append((e.slot, at, n, p0))
+    def _put_rows(self, batch, upload, out, fill=0, fill_first=False):
+        """Token ids | positions | slots of the step's rows, and with paired state the live rows of it, into `out`, the vector that
+        `upload` gave; `fill` rows of the scratch request (token 0 at position 0) in front or behind."""
+        rows = batch.total + fill
+        self._inputs.mlr_step_rows(len(batch.counts), batch.total, *batch.at, fill, 1 if fill_first else 0, self.cache.scratch_slot or 0,
+                                   upload.address)
+        if self._lanes == 4:
+            out[3 * rows:4 * rows] = self.cache.state_rows(out[2 * rows:3 * rows])
+
+    def _segments(self, batch, fill=0, fill_first=False):
+        """(slot, first row, tokens, first position) of every entry, those of the scratch request among them."""
+        counts, segments, at = batch.counts.tolist(), [], 0
+        if fill_first:
+            segments, at = [(self.cache.scratch_slot, i, 1, 0) for i in range(fill)], fill
+        for slot, n, p0 in zip(batch.slots.tolist(), counts, batch.first.tolist()):
+            segments.append((slot, at, n, p0))
             at += n
         if fill and not fill_first:
-            rows[0:2, at:], rows[2, at:] = 0, scratch
-            segments += [(scratch, at + i, 1, 0) for i in range(fill)]
-        if self._lanes == 4:
-            rows[3] = self.cache.state_rows(rows[2])
-        return rows, segments
+            segments += [(self.cache.scratch_slot, at + i, 1, 0) for i in range(fill)]
+        return segments
 
     def step(self, entries: List[Entry]):
         """Returns float logits [R, V] on the device (R = wanted places, in the order of the
         entries and of their `want`), or None when nothing is wanted."""
-        total, arrays, wanted = self._validate(entries)
-        slots = [e.slot for e in entries]
-        counts = [len(e.tokens) for e in entries]
-        first = self.cache.commit_first(slots, counts)    # raises with nothing changed, else takes the pages
+        batch = self._gather(entries)
+        total, slots = batch.total, batch.slots
+        self.cache.commit_into(slots, batch.counts, batch.first, batch.at)      # raises with nothing changed, else takes the pages
         try:
-            sig = self._signature(entries) if self.use_graphs and total <= self.graph_max_tokens else None
-            fill, fill_first = self._decode_fill(entries) if sig is not None else (0, False)
+            longest = int((batch.first + batch.counts).max())
+            sig = None
+            if self.use_graphs and total <= self.graph_max_tokens:
+                sig = ((1, (0,)),) * total if batch.single else self._signature(entries)
+            fill, fill_first = self._decode_fill(entries, batch.single) if sig is not None else (0, False)
             if fill:
                 sig = ((1, (0,)),) * fill + sig if fill_first else sig + ((1, (0,)),) * fill
             if sig is not None:                           # a captured step is keyed by its shape and its context bucket
-                sig = (sig, self._context_bucket(max(p0 + n for p0, n in zip(first, counts))))
-            if sig is not None and self._graph_wanted(entries, total + fill, sig):
-                logits = self._graph_step(entries, arrays, first, total + fill, sig, fill, fill_first)
+                sig = (sig, self._context_bucket(longest))
+            if sig is not None and self._graph_wanted(batch.single, total + fill, sig):
+                logits = self._graph_step(batch, total + fill, sig, fill, fill_first)
                 self.cache.retire(slots)
                 self.steps += 1
                 self._raise_if_not_finite()
                 if fill and logits is not None:           # the scratch rows' logits are dropped
                     return logits[fill:] if fill_first else logits[:len(entries)]
                 return logits
-            rows_of, segments = self._rows(entries, arrays, first)
-            if all(type(w) is list for w in wanted):       # (few places each: one short list)
-                rows = np.array([seg[1] + w for seg, places in zip(segments, wanted) for w in places], dtype=np.int32)
-            else:
-                rows = np.concatenate([seg[1] + np.asarray(w, dtype=np.int64) for seg, w in zip(segments, wanted)]
-                                      ).astype(np.int32)
-            r = rows.size
+            n, r = len(slots), len(batch.want_rows)
             stateful = self.cache.has_state()
-            parts = [rows_of.ravel(), rows]
+            per_token = self._lanes * total
+            vector = self._upload.stage(per_token + r + (n if stateful else 0))
+            self._put_rows(batch, self._upload, vector)
+            vector[per_token:per_token + r] = batch.want_rows
             if stateful:
-                parts.append(np.fromiter((seg[0] for seg in segments), np.int32, len(segments)))
-            self._upload.send(np.concatenate(parts), self._meta)
+                vector[per_token + r:] = slots
+            self._upload.upload(len(vector), self._meta)
             ctx = self.ctx
             ctx.begin_step()
             ctx.n_tokens = total
             ctx.token_ids = self._meta[0:total]
             ctx.positions = self._meta[total:2 * total]
             ctx.slots = self._meta[2 * total:3 * total]
-            ctx.segments = segments
-            ctx.single_tokens = total == len(entries)
-            ctx.max_context = max(p0 + n for (_, _, n, p0) in segments)
-            per_token = self._lanes * total
+            ctx.segments = self._segments(batch)
+            ctx.single_tokens = total == n
+            ctx.max_context = longest
             ctx.state_rows = self._meta[3 * total:per_token] if self._lanes == 4 else None
             want_rows = self._meta[per_token:per_token + r] if r else None
-            ctx.segment_slots = self._meta[per_token + r:per_token + r + len(segments)] if stateful else None
+            ctx.segment_slots = self._meta[per_token + r:per_token + r + n] if stateful else None
             logits = self.model.forward(ctx, want_rows)
             self.cache.retire(slots)
             self.steps += 1

@@ -16,6 +16,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 import threading
 import time
@@ -51,11 +52,14 @@ HIP_LIBRARIES = {
     "portion_attention": (["portion_attention.hip"], ["common.h"], False),      # likewise
     "recurrence_chunks": (["recurrence_chunks.hip"], ["common.h"], False),      # likewise
     "sampling": (["sampling.hip"], ["no_alloc.h"], False),
+    "upload": (["upload.hip"], [], False),
     "library_gemm": (["library_gemm.hip"], [], False, ["-lhipblaslt"]),      # host code around hipBLASLt
 }
 HOST_LIBRARIES = {
     "host": (["host/cache_manager.cpp", "host/scheduler.cpp"], []),
+    "step_inputs": (["host/step_inputs.cpp"], []),
 }
+PYTHON_LIBRARIES = {"step_inputs"}       # they read Python objects: compiled with the interpreter's headers, called with its lock held
 
 _loaded = {}
 _lock = threading.Lock()
@@ -110,6 +114,8 @@ def _plan(name, tag):
     if name in HOST_LIBRARIES:
         sources, headers = HOST_LIBRARIES[name]
         flags = HOST_SANITIZE_FLAGS if host_sanitized() else HOST_FLAGS
+        if name in PYTHON_LIBRARIES:
+            flags = [*flags, "-I" + sysconfig.get_paths()["include"]]
         out = os.path.join(_lib_dir(), f"libmlr_{name}{'_sanitized' if host_sanitized() else ''}.so")
         cmd = [_find_cxx(), *flags, "-o", out] + [os.path.join(CSRC, s) for s in sources]
     else:
@@ -206,7 +212,7 @@ def load(name, dtype=None):
     ensure_built([name], dtype if typed else None)
     out, _, _ = _plan(name, tag)
     try:
-        lib = ctypes.CDLL(out)
+        lib = (ctypes.PyDLL if name in PYTHON_LIBRARIES else ctypes.CDLL)(out)
     except OSError as err:
         raise BuildError(f"cannot load {out}: {err}") from None
     _loaded[key] = lib

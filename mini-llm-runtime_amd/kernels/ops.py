@@ -57,6 +57,43 @@ def _stream():
     return _ptr(torch.cuda.current_stream().cuda_stream)
 
 
+class PinnedCopy:
+    """Asynchronous copies from pinned memory on the current stream, and the wait until they have left it."""
+
+    def __init__(self):
+        self._handle = None
+
+    def _open(self):
+        lib = build.load("upload")
+        if not getattr(lib, "_mlr_typed", False):
+            lib.mlr_upload_create.restype = ctypes.c_void_p
+            lib.mlr_upload_create.argtypes = []
+            lib.mlr_upload_wait.argtypes = lib.mlr_upload_destroy.argtypes = [ctypes.c_void_p]
+            lib.mlr_upload_destroy.restype = None
+            lib.mlr_upload_copy.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
+            lib._mlr_typed = True
+        self._lib, self._handle = lib, lib.mlr_upload_create()
+        if not self._handle:
+            raise MemoryError("upload")
+
+    def wait(self):
+        if self._handle is not None:
+            _ok(self._lib.mlr_upload_wait(self._handle), "upload")
+
+    def copy(self, dst, address, size, offset=0):
+        """`size` bytes from pinned memory at `address` into the device tensor `dst`, `offset` bytes into it."""
+        _need(dst.is_cuda and dst.is_contiguous() and 0 <= offset and offset + size <= dst.numel() * dst.element_size(),
+              "upload: a contiguous device tensor that holds the bytes")
+        if self._handle is None:
+            self._open()
+        _ok(self._lib.mlr_upload_copy(self._handle, dst.data_ptr() + offset, address, size, _stream()), "upload")
+
+    def __del__(self):
+        handle, self._handle = getattr(self, "_handle", None), None
+        if handle:
+            self._lib.mlr_upload_destroy(handle)
+
+
 def _need(cond, message):
     """`message` is a string or, where building it costs time, a function that returns one."""
     if not cond:

@@ -1,0 +1,94 @@
+"""A step's inputs: the native pass over a batch's entries, the vectors for the device, and the block tables' way there."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from mini_llm_runtime_amd.engine import Entry
+from mini_llm_runtime_amd.kernels import build
+
+VOCAB, TOKENS, ROWS = 1000, 64, 12
+
+
+def gathered(entries, vocab=VOCAB):
+    """What the native pass makes of the entries, or None where it leaves them to the caller."""
+    ids, counts, slots, places, rows, totals = (np.full(max(n, 1), -7, np.int32) for n in (TOKENS, TOKENS, TOKENS, TOKENS, ROWS, 4))
+    rc = build.load("step_inputs").mlr_step_entries(ctypes.py_object(entries), ctypes.c_long(vocab), TOKENS, ROWS,
+                                                    *(ctypes.c_void_p(v.ctypes.data) for v in (ids, counts, slots, places, rows, totals)))
+    assert rc in (0, 1)
+    if rc:
+        return None
+    n, total, r, single = totals.tolist()
+    return ids[:total].tolist(), counts[:n].tolist(), slots[:n].tolist(), places[:n].tolist(), rows[:r].tolist(), bool(single)
+
+
+@pytest.mark.parametrize("batch,single", [
+    ([(3, [5], [0])], True), ([(0, [0], [0]), (7, [VOCAB - 1], [0])], True), ([(1, (4, 5, 6), (0, 2)), (2, [9], [])], False),
+    ([(1, [1] * TOKENS, list(range(ROWS)))], False), ([(4, [8], [])], False), ([(i, [i], [0]) for i in range(ROWS)], True)])
+def test_a_plain_batch_is_read_in_one_pass(batch, single):
+    entries = [Entry(*e) for e in batch]
+    starts = np.cumsum([0] + [len(e.tokens) for e in entries])
+    assert gathered(entries) == ([t for e in entries for t in e.tokens], [len(e.tokens) for e in entries], [e.slot for e in entries],
+                                 [len(e.want) for e in entries], [int(s) + w for s, e in zip(starts, entries) for w in e.want], single)
+
+
+@pytest.mark.parametrize("entries", [
+    [], (Entry(0, [1], []),), [Entry(0, [], [])], [Entry(0, [VOCAB], [])], [Entry(0, [-1], [])], [Entry(0, [1 << 70], [])], [Entry(0, [1.0], [])],
+    [Entry(0, [True], [])], [Entry(0, np.array([1, 2]), [])], [Entry(0, ["1"], [])], [Entry(0, [1], [1])], [Entry(0, [1], [-1])],
+    [Entry(0, [1, 2], [1, 0])], [Entry(0, [1, 2], [1, 1])], [Entry(0, [1], range(1))], [Entry(-1, [1], [0])], [Entry(None, [1], [0])],
+    [Entry(0, [1] * (TOKENS + 1), [])], [Entry(0, [1] * 40, list(range(ROWS + 1)))], [object()], [Entry(0, [1] * 40, []), Entry(1, [1] * 25, [])],
+    [Entry(np.int64(0), [1], [0])], [Entry(0, None, [])]])
+def test_any_other_batch_is_left_to_the_caller(entries):
+    """Refusals with their messages, and the forms that are taken element by element (numpy vectors, places in any order)."""
+    assert gathered(entries) is None
+
+
+def test_entries_that_are_more_than_tuples_of_values():
+    """Attributes that are code: one that raises, one that empties the list it is read from."""
+    class Odd:
+        want, tokens = [0], [3]
+
+        def __init__(self, act):
+            self.act = act
+
+        @property
+        def slot(self):
+            return self.act()
+
+    def fails():
+        raise RuntimeError("no slot")
+    assert gathered([Odd(fails)]) is None
+    entries = []
+    entries += [Odd(lambda: (entries.clear(), 5)[1]), Odd(lambda: 6)]
+    assert gathered(entries) == ([3], [1], [5], [1], [0], True)
+
+
+@pytest.mark.parametrize("fill,fill_first", [(0, False), (3, False), (2, True)])
+def test_the_rows_of_a_step(fill, fill_first):
+    counts, slots, first = (np.array(v, np.int32) for v in ([1, 4, 2], [5, 0, 9], [17, 0, 300]))
+    ids = np.arange(100, 107, dtype=np.int32)
+    out = np.full((3, 7 + fill), -1, np.int32)
+    build.load("step_inputs").mlr_step_rows(3, 7, *(ctypes.c_void_p(v.ctypes.data) for v in (ids, counts, slots, first)), fill, int(fill_first), 11,
+                                            ctypes.c_void_p(out.ctypes.data))
+    rows = [ids.tolist(), [17, 0, 1, 2, 3, 300, 301], [5, 0, 0, 0, 0, 9, 9]]
+    extra = [[0] * fill, [0] * fill, [11] * fill]
+    assert out.tolist() == [e + r if fill_first else r + e for r, e in zip(rows, extra)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("slots,length", [(40, 40960), (40, 512), (1, 128)])
+def test_changed_rows_of_the_block_tables_reach_the_device(slots, length):
+    """Rows far apart in a large table go one by one, in a small one as one piece with what lies between."""
+    from mini_llm_runtime_amd.cache.manager import CacheManager, KvSpec
+    cache = CacheManager([KvSpec(1, 16)], torch.float32, torch.device("cuda:0"), 16, 4096, slots, length)
+    for _ in range(slots):
+        cache.acquire_slot()
+    table = cache._tables[0]
+    for step in ([0, slots - 1], [slots // 2], list(range(0, slots, 3)), [slots - 1]):
+        step = sorted(set(step))
+        first = np.full(len(step), -1, np.int32)
+        lengths = [cache.length(s) for s in step]
+        cache.commit_into(np.array(step, np.int32), np.full(len(step), 17, np.int32), first)
+        assert first.tolist() == lengths
+        assert np.array_equal(table[:slots].cpu().numpy(), cache.book.table(0))
