@@ -51,8 +51,9 @@ class Sampler:
         self.max_rows = rows
         self._params = torch.empty((2, rows), dtype=torch.float32, device=self.device)
         self._host = torch.empty((2, rows), dtype=torch.float32).pin_memory()
-        self._tokens = torch.empty(rows, dtype=torch.int32, device=self.device)
-        self._status = torch.zeros(2, dtype=torch.int32, device=self.device)
+        self._result = torch.zeros(2 + rows, dtype=torch.int32, device=self.device)      # status | tokens: one copy back
+        self._result_host = torch.empty(2 + rows, dtype=torch.int32).pin_memory()
+        self._status, self._tokens = self._result[:2], self._result[2:]
         need_f, need_i = self.kernels.sample_scratch(rows)
         self._scratch_f = torch.empty(need_f, dtype=torch.float32, device=self.device)
         self._scratch_i = torch.empty(need_i, dtype=torch.int32, device=self.device)
@@ -73,7 +74,10 @@ class Sampler:
         tokens = self._tokens[:rows]
         self.kernels.sample(logits, temp, uni, tokens, self._status, self._scratch_f, self._scratch_i,
                             any_sampling=any(t > 0 for t in temperatures))
-        out = torch.cat([tokens, self._status]).cpu().tolist()     # one copy back, one sync
-        if out[rows] != 0:
-            raise NonFiniteLogits(f"row {out[rows + 1]} of the logits holds a value that is not finite")
-        return out[:rows]
+        out = self._result_host[:2 + rows]
+        out.copy_(self._result[:2 + rows], non_blocking=True)
+        torch.cuda.current_stream(self.device).synchronize()
+        bad, row, *picked = out.tolist()
+        if bad != 0:
+            raise NonFiniteLogits(f"row {row} of the logits holds a value that is not finite")
+        return picked
