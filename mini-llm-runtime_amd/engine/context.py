@@ -210,14 +210,16 @@ class StepContext:
         workgroup per (token group, kv head); a small batch over long contexts does not, so there the
         keys of a token are split over several workgroups, in ranges [s * split_keys, (s + 1) *
         split_keys) of absolute key positions, and merged in ascending order.  split_keys is the
-        largest of base, 2 base, 4 base, ... that still gives `target_workgroups`; what a token's
+        largest of base, 2 base, 4 base, ... that still gives `target_workgroups`, or where base is too wide for that narrower
+        (`narrowed`; not in a model that routes, whose choices turn on the last bit); what a token's
         result is does not depend on the choice beyond rounding.  `rows` tokens take part; the partial
         results are indexed by batch row, of which there are `batch_rows`.  `longest`: the most keys a
         workgroup of the kernel can walk without a split; a longer context is split whatever the batch."""
         forced = longest is not None and self.max_context > longest
         if rows > self.split_max_tokens and not forced:
             return 0, 1, None
-        return self._split(max(1, rows * kv_heads), self.target_workgroups, batch_rows, q_heads, head_dim, longest, LONG_RANGE)
+        return self._split(max(1, rows * kv_heads), self.target_workgroups, batch_rows, q_heads, head_dim, longest, LONG_RANGE,
+                           narrow=not self.routed)
 
     def group_split(self, groups, batch_rows, kv_heads, q_heads, head_dim, longest=None):
         """As `attention_split` for `groups` groups of many tokens each (prompt portions), which give
@@ -244,6 +246,21 @@ class StepContext:
         return keys, max_splits, chunk, self.workspace.get("attn_partial", (chunk * per_row,), torch.float32)
 
     @staticmethod
+    def narrowed(base, walk, units, enough, ranges):
+        """The width of a key range where ranges of `base` keys leave the chip idle, `units` workgroups a range, for contexts of up to
+        `walk` keys: halved, to 64 keys at least, while that gives no more than `enough` workgroups and `ranges` ranges.  A
+        workgroup's time is a chain of tiles, the merge's a chain of ranges, sixteen of which it asks for at once.
+
+        Plain attention, weights cold: one request of the 0.6B sizes behind 200, 700, 1100 and 1500 tokens 1173, 1175, 1175 and 1182 us a
+        step with ranges of 256, now 1088, 1098, 1128 and 1140; three of four 8B layers behind 700 to 1200 669 -> 647.  Behind 3900 tokens
+        32 ranges would cost 6 %; four requests of 1000 to 1900 tokens on 512 workgroups, two a compute unit, 5 % (400: as before).
+        Differential attention, where half a workgroup works, gains up to 512 and 32 ranges: 8 requests of 1000 to 1700 tokens 714 -> 683."""
+        keys = base
+        while keys % 128 == 0 and -(-walk // (keys // 2)) <= ranges and units * -(-walk // (keys // 2)) <= enough:
+            keys //= 2
+        return keys
+
+    @staticmethod
     def forced_splits(max_length, base, longest):
         """Key splits that a context of `max_length` needs at least when one workgroup walks at most `longest`
         keys: ranges of the largest of base, 2 base, 4 base, ... that `longest` holds (1: no split needed)."""
@@ -254,7 +271,7 @@ class StepContext:
             keys *= 2
         return -(-max_length // keys)
 
-    def _split(self, units, enough, batch_rows, q_heads, head_dim, longest=None, widest=None):
+    def _split(self, units, enough, batch_rows, q_heads, head_dim, longest=None, widest=None, narrow=False):
         """`units` workgroups without a split; no split when they are `enough`, but for contexts beyond `widest` keys.  The partial results never take
         more than `partial_budget` floats (when one is set: the runner's memory plan): key ranges are doubled
         until they fit, which a forced split allows up to `longest`."""
@@ -262,7 +279,7 @@ class StepContext:
         forced = longest is not None and self.max_context > longest
         if base <= 0 or (self.max_context <= base and not forced):
             return 0, 1, None
-        keys = base
+        keys = self.narrowed(base, self.max_context, units, 3 * self.compute_units // 2, 20) if narrow else base
         while keys * 2 < self.max_context and units * (-(-self.max_context // (keys * 2))) >= self.target_workgroups:
             keys *= 2
         if forced:

@@ -107,11 +107,12 @@ class DiffAttention:
             plan[(f"token_groups_{SMALL_GROUP}_{factor}", torch.int32)] = 2 * rows + 2
         return plan
 
-    def _tile_splits(self, ctx, units, places, budget):
+    def _tile_splits(self, ctx, units, places, budget, short=False):
         """(width of a key range, number of ranges) for a launch of the matrix-core kernel that has `units`
         workgroups without ranges and `places` rows of partial results: no ranges where the batch fills the GPU or
         the context is short; else the widest ranges that still give `target_workgroups`, widened further until
-        the partial results fit `budget` floats."""
+        the partial results fit `budget` floats; `short`: groups of single tokens and short portions, whose ranges may be
+        narrower than the setting (`StepContext.narrowed`)."""
         s = self.spec
         base, longest = ctx.split_keys, ctx.max_context
         # keys that one workgroup walks without ranges: every earlier key, or behind a mask its tokens' window or block
@@ -123,7 +124,8 @@ class DiffAttention:
             raise PartError(f"a context of {longest} tokens needs key ranges (split_keys > 0): one workgroup walks {reach} keys")
         if base <= 0 or walk <= base or (units >= ctx.target_workgroups and not forced):
             return 0, 1
-        keys = base
+        # (a model that routes keeps the sums that it has: a choice between experts turns on the last bit)
+        keys = base if ctx.routed or not short else ctx.narrowed(base, walk, units, ctx.target_workgroups, 32)
         while keys * 2 < walk and keys * 2 <= reach and (units * (-(-walk // (keys * 2))) >= ctx.target_workgroups or
                                                           (forced and units >= ctx.target_workgroups)):
             keys *= 2
@@ -148,7 +150,7 @@ class DiffAttention:
         for (first, count, n), group_tokens in ((big, tokens), (small, SMALL_GROUP)):
             if n == 0:
                 continue
-            split_keys, splits = self._tile_splits(ctx, n * per_group, n * group_tokens, partial.numel())
+            split_keys, splits = self._tile_splits(ctx, n * per_group, n * group_tokens, partial.numel(), group_tokens == SMALL_GROUP)
             # (single tokens and short portions always leave partial results, where their room allows: the two maps
             # of a head then run side by side and the merge kernel finishes the head)
             through = splits > 1 or (group_tokens == SMALL_GROUP and

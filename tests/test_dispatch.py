@@ -233,6 +233,22 @@ def test_key_ranges_of_one_width_whatever_the_batch():
     assert keys == 512 and splits == -(-300000 // 512) <= MAX_KEY_SPLITS and chunk == 3
 
 
+@pytest.mark.parametrize("rows,max_context,keys", [
+    (1, 512, 64), (1, 257, 64), (1, 1280, 64), (1, 1281, 128), (1, 2560, 128), (1, 2561, 256), (6, 512, 64), (7, 512, 128), (12, 512, 128),
+    (13, 512, 256), (3, 2048, 128), (4, 2048, 256), (8, 4096, 512), (1, 256, 0)])
+def test_few_workgroups_take_narrower_key_ranges(rows, max_context, keys):
+    """Half the setting's width while that is no more than three workgroups to two compute units and twenty ranges; a model that routes, a setting that has no half
+    and one that is narrow already stay with the setting."""
+    def split(base, routed=False):
+        ctx = context(max_context, split_keys=base)
+        ctx.compute_units, ctx.routed = 256, routed
+        return ctx.attention_split(rows, rows, 8, 16, 128, longest=65504)[:2]
+    assert split(256) == ((keys, -(-max_context // keys)) if keys else (0, 1))
+    assert split(256, routed=True)[0] == (0 if max_context <= 256 else max(256, keys))
+    assert max_context <= 320 or rows * 8 * -(-max_context // 320) >= 512 or split(320)[0] == 320
+    assert max_context > 512 or split(64)[0] in (64, 128)
+
+
 @pytest.mark.parametrize("sizes", [(17, 6144, 2048), (64, 12288, 1024), (333, 768, 2048), (1777, 4096, 18432), (1603, 28736, 6016), (653, 23648, 2176)])
 def test_products_of_a_model_with_a_router_keep_the_order_of_their_sums(sizes):
     """Where the vendor library may add in another order than the many-row kernel, a model that chooses among experts stays with
