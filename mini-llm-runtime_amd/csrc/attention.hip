@@ -242,8 +242,9 @@ __global__ __launch_bounds__(64) void attention_combine_kernel(AttnArgs a) {
 // in its order, so the same bits.  A workgroup serves 16 columns -- consecutive tokens of one request times the query heads of
 // one kv head -- which share what it reads of keys and values; the kernel above, one token a workgroup, fetches every value of a
 // channel from a cache line of its own (16 heads on 8 of 128 channels, pages of 16: 111 us for eight tokens behind 400 keys, 306
-// behind 4000, 0.68 ms for a prompt of 400 and 16.7 for one of 2048; here 27, 76, 62 us and 0.69 ms, and with tiles of 16 keys,
-// whose sums are other ones, 17, 62, 53 us and 0.59 ms).  Groups are found by the kernel: a row leads one when it is a multiple
+// behind 4000, 0.68 ms for a prompt of 400 and 16.7 for one of 2048; here 19, 63, 50 us and 0.57 ms).  A tile is a chain of products,
+// exchanges and waits, so no wait may stand for more than it needs: with branches around loads, LDS reads and products, page ids and
+// sums exchanged through LDS and every tile's values waited for before its scores, the four took 26, 77, 61 us and 0.69 ms.  Groups are found by the kernel: a row leads one when it is a multiple
 // of the tokens a group holds or does not continue the row before it.
 //
 // Keys are walked in tiles of 64 at absolute multiples of 64.  Per tile: wavefront w takes the scores of keys 16 w ..,
@@ -253,6 +254,12 @@ __global__ __launch_bounds__(64) void attention_combine_kernel(AttnArgs a) {
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 
 #define F32_PITCH 68           // floats between columns of the scores in LDS: 64 lanes' reads meet every bank once
+
+// A value of the 16 lanes around this one, D lanes on (a tree over them: 8, 4, then 2 and 1, each lane with the one D away); no LDS.
+template <int D> __device__ __forceinline__ float row16_other(float v) {
+    constexpr int CTRL = D == 8 ? 0x128 : D == 4 ? 0x124 : D == 2 ? 0x4E : 0xB1;     // (rotations by 8 and by 4, the latter of what
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));      // repeats; swaps in fours)
+}
 
 template <int NC, bool EXACT>
 __global__ __launch_bounds__(256, NC <= 8 ? 2 : 1) void attention_f32_kernel(AttnArgs a, int rows) {
@@ -275,7 +282,7 @@ __global__ __launch_bounds__(256, NC <= 8 ? 2 : 1) void attention_f32_kernel(Att
         hi = min(hi, (split + 1) * a.split_keys);
         if (lo >= hi) return;                                                // (no token of the group reads this part)
     }
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, b4 = (lane >> 4) * 4;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, b4 = (lane >> 4) * 4;
     const int tok = min(c / g, ntok - 1), head = kvh * g + c % g;
     // the column and the places of a tile (j, j + 16, j + 32, j + 48) that this thread takes part in the softmax with
     const int col = threadIdx.x >> 4, j = threadIdx.x & 15, pos = pos0 + min(col / g, ntok - 1);
@@ -287,16 +294,19 @@ __global__ __launch_bounds__(256, NC <= 8 ? 2 : 1) void attention_f32_kernel(Att
     for (int i = 0; i < NC; ++i) q[i] = EXACT || i < nc ? turned(*reinterpret_cast<const floatx4*>(qr + i * 16)) : floatx4{0.f, 0.f, 0.f, 0.f};
 
     constexpr int NV = (NC + 3) / 4;                                         // blocks of 16 channels of a wavefront
+    constexpr bool ALL = EXACT && NC % 4 == 0;                               // .. all of which there are
     const int t_first = lo / 64, t_end = (hi + 63) / 64;
     const int32_t* table = a.block_table + (size_t)slot * a.max_blocks;
     int pages = -1;                                                          // lane i: page of the i-th 16 keys of the next 16 tiles
     auto load_pages = [&](int t) {
         const int block = (t * 64 + lane * 16) / P;
         pages = t * 64 + lane * 16 < hi && block < a.max_blocks ? table[block] : -1;
+        asm volatile("" : "+v"(pages));              // (waited for here, once in 16 tiles, and not wherever it is read)
     };
+    auto page_of = [&](int i) { return __builtin_amdgcn_readlane(pages, i); };
     floatx4 k[NC], v[NV][4];
     auto load_k = [&](int t) {
-        const int page = __shfl(pages, ((t - t_first) & 15) * 4 + wave), at = (t * 64 + wave * 16) % P;
+        const int page = page_of(((t - t_first) & 15) * 4 + wave), at = (t * 64 + wave * 16) % P;
         const float* kr = a.k_pages + ((long long)max(page, 0) * a.kv_heads + kvh) * P * D + (size_t)(at + c) * D + b4;
 #pragma unroll
         for (int i = 0; i < NC; ++i)
@@ -305,11 +315,11 @@ __global__ __launch_bounds__(256, NC <= 8 ? 2 : 1) void attention_f32_kernel(Att
     auto load_v = [&](int t) {
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-            const int page = __shfl(pages, ((t - t_first) & 15) * 4 + s), at = (t * 64 + s * 16) % P;
+            const int page = page_of(((t - t_first) & 15) * 4 + s), at = (t * 64 + s * 16) % P;
             const float* vr = a.v_pages + ((long long)max(page, 0) * a.kv_heads + kvh) * P * D + (size_t)c * P + at + b4;
 #pragma unroll
             for (int i = 0; i < NV; ++i)
-                if (wave + 4 * i < nc) v[i][s] = *reinterpret_cast<const floatx4*>(vr + (size_t)(wave + 4 * i) * 16 * P);
+                if (ALL || wave + 4 * i < nc) v[i][s] = *reinterpret_cast<const floatx4*>(vr + (size_t)(wave + 4 * i) * 16 * P);
         }
     };
     float run_max = -INFINITY, run_sum = 0.f;
@@ -318,7 +328,9 @@ __global__ __launch_bounds__(256, NC <= 8 ? 2 : 1) void attention_f32_kernel(Att
     for (int i = 0; i < NV; ++i) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
     load_pages(t_first);
     load_k(t_first);
+    __builtin_amdgcn_sched_barrier(0);               // (keys first, as in the loop: its wait for them need not wait for the values)
     load_v(t_first);
+    __builtin_amdgcn_sched_barrier(0);
     for (int t = t_first; t < t_end; ++t) {
         const int buf = t & 1, nth = ((t - t_first) & 15) * 4;
         floatx4 score = {0.f, 0.f, 0.f, 0.f};
@@ -338,23 +350,27 @@ __global__ __launch_bounds__(256, NC <= 8 ? 2 : 1) void attention_f32_kernel(Att
         *reinterpret_cast<floatx4*>(&p_lds[buf][c * F32_PITCH + wave * 16 + b4]) = score;
         int seen_page[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) seen_page[i] = __shfl(pages, nth + i);
+        for (int i = 0; i < 4; ++i) seen_page[i] = page_of(nth + i);
         // (the next tile's keys are on their way from here on, its values from the end of this turn on: each into the
-        // registers that are free then)
-        const bool more = t + 1 < t_end;
-        if (more && nth == 60) load_pages(t + 1);
-        if (more) load_k(t + 1);
+        // registers that are free then; behind the last tile that one again, since a branch around a load would have every wait
+        // count on the loads that it skips)
+        const int ahead = min(t + 1, t_end - 1);
+        if (ahead > t && nth == 60) load_pages(ahead);
+        load_k(ahead);
         __syncthreads();
         float p[4], top = -INFINITY;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int key = t * 64 + 16 * i + j;
             const bool seen = seen_page[i] >= 0 && key >= from && key < until;
-            p[i] = seen ? p_lds[buf][col * F32_PITCH + 16 * i + j] * a.scale : -INFINITY;
+            const float score = p_lds[buf][col * F32_PITCH + 16 * i + j] * a.scale;      // (read whether seen or not: no branch)
+            p[i] = seen ? score : -INFINITY;
             top = fmaxf(top, p[i]);
         }
-#pragma unroll
-        for (int d = 8; d > 0; d >>= 1) top = fmaxf(top, __shfl_xor(top, d));
+        top = fmaxf(top, row16_other<8>(top));
+        top = fmaxf(top, row16_other<4>(top));
+        top = fmaxf(top, row16_other<2>(top));
+        top = fmaxf(top, row16_other<1>(top));
         const float new_max = fmaxf(run_max, top);
         const float corr = new_max > -INFINITY ? expf(run_max - new_max) : 1.f;
 #pragma unroll
@@ -362,8 +378,10 @@ __global__ __launch_bounds__(256, NC <= 8 ? 2 : 1) void attention_f32_kernel(Att
             // (a score that is not a number stays one where nothing else sets the maximum: pages that nobody wrote show)
             p[i] = p[i] != p[i] ? p[i] : new_max > -INFINITY ? expf(p[i] - new_max) : 0.f;
         float sum = (p[0] + p[2]) + (p[1] + p[3]);
-#pragma unroll
-        for (int d = 8; d > 0; d >>= 1) sum += __shfl_xor(sum, d);
+        sum += row16_other<8>(sum);
+        sum += row16_other<4>(sum);
+        sum += row16_other<2>(sum);
+        sum += row16_other<1>(sum);
         run_sum = run_sum * corr + sum;
         run_max = new_max;
 #pragma unroll
@@ -373,42 +391,49 @@ __global__ __launch_bounds__(256, NC <= 8 ? 2 : 1) void attention_f32_kernel(Att
         // Every token of the group sees the whole tile, or values that a token must not see would meet its probability
         // of zero: places that were never written are cleared, and where a value is not finite the tokens go one by one.
         const float scale_by = corr_lds[buf][c];
+        const float* pr = &p_lds[buf][c * F32_PITCH + (lane >> 4)];
+        float prob[16];                                                      // (asked for together)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) prob[i] = pr[4 * i];
         bool mapped = true;
 #pragma unroll
         for (int s = 0; s < 4; ++s) mapped = mapped && seen_page[s] >= 0;
         const bool inner = mapped && t * 64 >= lo && t * 64 + 63 <= pos0 && (a.window <= 0 || t * 64 > pos0 + ntok - 1 - a.window);
         bool odd = false;
+        if (!inner) {
 #pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            acc[i] *= scale_by;
-            if (wave + 4 * i >= nc) continue;
+            for (int i = 0; i < NV; ++i) {
+                if (!ALL && wave + 4 * i >= nc) continue;
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                if (!inner) {
+                for (int s = 0; s < 4; ++s)
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const int key = t * 64 + s * 16 + b4 + e;
                         if (seen_page[s] < 0 || key < lo || key >= hi) v[i][s][e] = 0.f;
                         odd |= !(fabsf(v[i][s][e]) <= 3.402823466e38f);
                     }
-                }
-                v[i][s] = turned(v[i][s]);                                   // element e: the key 16 s + 4 e + lane / 16
             }
         }
-        const float* pr = &p_lds[buf][c * F32_PITCH + (lane >> 4)];
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            acc[i] *= scale_by;
+            if (!ALL && wave + 4 * i >= nc) continue;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) v[i][s] = turned(v[i][s]);           // element e: the key 16 s + 4 e + lane / 16
+        }
         if (__builtin_expect(__any(odd), 0)) {
             for (int other = 0; other < ntok; ++other) {
                 const int own = pos0 + other, own_from = a.window > 0 ? max(0, own - a.window + 1) : 0;
 #pragma unroll
                 for (int i = 0; i < NV; ++i) {
-                    if (wave + 4 * i >= nc) continue;
+                    if (!ALL && wave + 4 * i >= nc) continue;
                     floatx4 next = acc[i];
 #pragma unroll
                     for (int s = 0; s < 4; ++s)
 #pragma unroll
                         for (int e = 0; e < 4; ++e) {
                             const int key = t * 64 + 16 * s + 4 * e + (lane >> 4);
-                            next = __builtin_amdgcn_mfma_f32_16x16x4f32(key >= own_from && key <= own ? v[i][s][e] : 0.f, pr[16 * s + 4 * e], next, 0, 0, 0);
+                            next = __builtin_amdgcn_mfma_f32_16x16x4f32(key >= own_from && key <= own ? v[i][s][e] : 0.f, prob[4 * s + e], next, 0, 0, 0);
                         }
                     if (tok == other) acc[i] = next;
                 }
@@ -418,13 +443,13 @@ __global__ __launch_bounds__(256, NC <= 8 ? 2 : 1) void attention_f32_kernel(Att
             for (int s = 0; s < 4; ++s)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const float prob = pr[16 * s + 4 * e];
 #pragma unroll
                     for (int i = 0; i < NV; ++i)
-                        if (wave + 4 * i < nc) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i][s][e], prob, acc[i], 0, 0, 0);
+                        if (ALL || wave + 4 * i < nc) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i][s][e], prob[4 * s + e], acc[i], 0, 0, 0);
                 }
         }
-        if (more) load_v(t + 1);
+        load_v(ahead);
+        __builtin_amdgcn_sched_barrier(0);           // (asked for here: left alone they sink behind the next tile's scores)
     }
     if (j == 0) sum_lds[col] = run_sum;
     const bool split_up = a.max_splits > 1;
@@ -439,7 +464,7 @@ __global__ __launch_bounds__(256, NC <= 8 ? 2 : 1) void attention_f32_kernel(Att
     const float den = sum_lds[c];
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-        if (wave + 4 * i >= nc) continue;
+        if (!ALL && wave + 4 * i >= nc) continue;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int d = (wave + 4 * i) * 16 + b4 + e;
