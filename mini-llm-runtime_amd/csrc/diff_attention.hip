@@ -47,6 +47,7 @@ struct DiffArgs {
     // group_first[group] + i while i < group_count[group] (partial results are indexed by blockIdx.x)
     const int32_t* group_first; const int32_t* group_count; int group_tokens;
     int mask_kind, mask_size;                  // 0: every earlier key; 1: the last mask_size positions; 2: the query's block
+    unsigned page_magic;                       // ceil(2^32 / page_size): the high word of a product with it divides by the page size
 };
 
 #define MASK_NONE 0
@@ -234,13 +235,14 @@ __global__ __launch_bounds__(64) void diff_attention_partial_kernel(DiffArgs a) 
 }
 
 // Two wavefronts per (token, head), a map each, merged over their key ranges, then the head's epilogue by the first.  Bound by
-// its chain of loads: a range's values are asked for eight ranges at a time, the first eight before the weights are known
-// (8 tokens of 16 heads in 11 ranges: 13.8 us with one wavefront, range by range, now 5.5).
+// its chain of loads: a range's values are asked for AHEAD ranges at a time, the first of them before the weights are known
+// (8 tokens of 16 heads in 11 ranges: 13.8 us with one wavefront, range by range, 5.5 eight at a time; in 8 to 14 ranges of 128
+// keys 6.8, and with sixteen at a time and no condition on a load 5.4).  VR: value channels a lane, value_dim <= 64 VR.
+template <int VR, int AHEAD>
 __global__ __launch_bounds__(128) void diff_attention_combine_kernel(DiffArgs a) {
-    constexpr int AHEAD = 8;
     __shared__ float w_lds[2][COMBINE_MAX_SPLITS];
     __shared__ float l_lds[2][COMBINE_MAX_SPLITS];
-    __shared__ float second[64 * MAX_V_REGS];
+    __shared__ float second[64 * VR];
     const int m = diff_row(a), head = blockIdx.y, lane = threadIdx.x & 63, map = threadIdx.x >> 6;
     if (m < 0) return;
     const int V = a.value_dim;
@@ -249,19 +251,19 @@ __global__ __launch_bounds__(128) void diff_attention_combine_kernel(DiffArgs a)
     const int s0 = a.max_splits > 1 ? min(a.max_splits - 1, first_key(a, pos) / a.split_keys) : 0;
     const int n = (a.max_splits > 1 ? min(a.max_splits - 1, pos / a.split_keys) + 1 : 1) - s0;
     const float* base = a.partial + (((size_t)blockIdx.x * a.q_heads * 2 + head * 2 + map) * a.max_splits + s0) * (V + 2);
-    float part[AHEAD][MAX_V_REGS], gate[MAX_V_REGS];
+    float part[AHEAD][VR], gate[VR];
     auto fetch = [&](int s) {
 #pragma unroll
         for (int u = 0; u < AHEAD; ++u)
 #pragma unroll
-            for (int i = 0; i < MAX_V_REGS; ++i) {
-                const int c = lane + 64 * i;
-                part[u][i] = s + u < n && c < V ? base[(size_t)(s + u) * (V + 2) + c] : 0.f;
+            for (int i = 0; i < VR; ++i) {
+                const int c = min(lane + 64 * i, V - 1);      // (clamped: no branch around a load; what is read twice is not used)
+                part[u][i] = base[(size_t)min(s + u, n - 1) * (V + 2) + c];
             }
     };
     fetch(0);
 #pragma unroll
-    for (int i = 0; i < MAX_V_REGS; ++i) {
+    for (int i = 0; i < VR; ++i) {
         const int c = lane + 64 * i;
         gate[i] = a.gate && c < V ? to_float(a.gate[(size_t)m * a.gate_stride + (size_t)head * V + c]) : 0.f;
     }
@@ -278,9 +280,9 @@ __global__ __launch_bounds__(128) void diff_attention_combine_kernel(DiffArgs a)
         w_lds[map][s] = smax > -INFINITY ? expf(smax - gmax) : 0.f;
     }
     __syncthreads();
-    float den = 0.f, num[MAX_V_REGS];
+    float den = 0.f, num[VR];
 #pragma unroll
-    for (int i = 0; i < MAX_V_REGS; ++i) num[i] = 0.f;
+    for (int i = 0; i < VR; ++i) num[i] = 0.f;
     for (int s = 0; s < n; s += AHEAD) {
         if (s > 0) fetch(s);
 #pragma unroll
@@ -289,19 +291,19 @@ __global__ __launch_bounds__(128) void diff_attention_combine_kernel(DiffArgs a)
             const float w = w_lds[map][s + u];
             den += w * l_lds[map][s + u];
 #pragma unroll
-            for (int i = 0; i < MAX_V_REGS; ++i) num[i] += w * part[u][i];
+            for (int i = 0; i < VR; ++i) num[i] += w * part[u][i];
         }
     }
 #pragma unroll
-    for (int i = 0; i < MAX_V_REGS; ++i) {
+    for (int i = 0; i < VR; ++i) {
         num[i] = den != 0.f ? num[i] / den : 0.f;
         if (map == 1) second[lane + 64 * i] = num[i];
     }
     __syncthreads();
     if (map == 1) return;
-    float o[MAX_V_REGS], ss = 0.f;
+    float o[VR], ss = 0.f;
 #pragma unroll
-    for (int i = 0; i < MAX_V_REGS; ++i) {
+    for (int i = 0; i < VR; ++i) {
         const int c = lane + 64 * i;
         o[i] = c < V ? num[i] - a.lam * second[c] : 0.f;
         ss += o[i] * o[i];
@@ -309,13 +311,18 @@ __global__ __launch_bounds__(128) void diff_attention_combine_kernel(DiffArgs a)
     ss = wave_sum(ss);
     const float unit = a.out_scale / sqrtf(ss / (float)V + a.eps);
 #pragma unroll
-    for (int i = 0; i < MAX_V_REGS; ++i) {
+    for (int i = 0; i < VR; ++i) {
         const int c = lane + 64 * i;
         if (c >= V) continue;
         float y = o[i] * unit;
         if (a.gate) y *= 1.0f / (1.0f + expf(-gate[i]));
         a.out[((size_t)m * a.q_heads + head) * V + c] = from_float<elem_t>(y);
     }
+}
+
+static void launch_combine(const DiffArgs& a, int rows, hipStream_t stream) {
+    if (a.value_dim <= 128) diff_attention_combine_kernel<2, 16><<<dim3(rows, a.q_heads), 128, 0, stream>>>(a);
+    else diff_attention_combine_kernel<MAX_V_REGS, 8><<<dim3(rows, a.q_heads), 128, 0, stream>>>(a);
 }
 
 #if MLR_BF16
@@ -327,14 +334,17 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 
 // NCH: ceil(head_dim / 32) chunks of 32 channels a map; NDB: blocks of 16 value channels (value_dim <= 16 NDB).
 // head_dim and value_dim multiples of 16, the page size a multiple of 8.
-template <int NCH, int NDB>
+// FULL: a head's channels fill the chunks and blocks (head_dim = 32 NCH, value_dim = 16 NDB), so that nothing in a tile hangs on a
+// branch.  A tile is a chain of exchanges, and its time was the branches': around every product, LDS read and load (whose page id was
+// divided for behind one more), each waiting for what was under way.  8 tokens behind 1000 to 1700 keys in ranges of 128: 16.2 -> 12.6 us.
+template <int NCH, int NDB, bool FULL>
 __device__ __forceinline__ void diff_tiles_group(const DiffArgs& a, const int32_t* __restrict__ group_row0,
                                                  const int32_t* __restrict__ group_ntok, int col_heads, int wave_heads,
                                                  int token_blocks, int map_split, int grp, __bf16* k_lds, __bf16* v_lds,
                                                  int32_t* page_lds) {
     constexpr int KPITCH = 2 * 32 * NCH + 8;          // elements per key row in LDS (both maps)
     constexpr int VPITCH = TKEYS + 4;                 // elements per value channel row in LDS
-    const int D = a.head_dim, V = a.value_dim, P = a.page_size;
+    const int D = FULL ? 32 * NCH : a.head_dim, V = FULL ? 16 * NDB : a.value_dim, P = a.page_size;
     const int g = a.q_heads / a.kv_heads;
     // The 16 columns of a wavefront: `col_heads` query heads of the kv head side by side for each of 16 / col_heads
     // tokens (prompt portions: one head, 16 tokens; single tokens and short portions: up to four heads of each
@@ -344,8 +354,8 @@ __device__ __forceinline__ void diff_tiles_group(const DiffArgs& a, const int32_
     const int heads_per_wg = col_heads * wave_heads;
     const int head_sets = (g + heads_per_wg - 1) / heads_per_wg;
     const int kvh = blockIdx.y / head_sets, head_set = blockIdx.y % head_sets;
-    const int lane = threadIdx.x & 63, wave = map_split ? (int)((threadIdx.x >> 6) & 1) : (int)(threadIdx.x >> 6);
-    const int my_map = threadIdx.x >> 7;              // (map_split only)
+    const int lane = threadIdx.x & 63, nth_wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave = map_split ? nth_wave & 1 : nth_wave;
+    const int my_map = nth_wave >> 1;                 // (map_split only)
     const int col = lane & 15, b = lane >> 4;
     const int row0 = group_row0[grp], ntok = group_ntok[grp];
     const int slot = a.slots[row0], pos0 = a.positions[row0];
@@ -380,7 +390,7 @@ __device__ __forceinline__ void diff_tiles_group(const DiffArgs& a, const int32_
         for (int c = 0; c < NCH; ++c) {
             const int d0 = 32 * c + 8 * b;
             qf[map][c] = zero8;
-            if (col_valid && d0 < D)
+            if (col_valid && (FULL || d0 < D))
                 qf[map][c] = *reinterpret_cast<const bf16x8*>(q + (size_t)(row0 + tok) * a.q_stride + (size_t)(head * 2 + map) * D + d0);
         }
     // scores in the base-2 domain; the cap as cap * tanh(x / cap) with tanh(y) = 1 - 2 / (exp(2 y) + 1)
@@ -414,10 +424,9 @@ __device__ __forceinline__ void diff_tiles_group(const DiffArgs& a, const int32_
     }
     // (no load from the block table here: a global load behind a branch makes the compiler wait for every load in
     // flight, one tile's loads would then go out one after the other; the host keeps a range within the cache)
-    const bool pow2 = (P & (P - 1)) == 0;
-    const int pshift = __ffs(P) - 1;
-    auto block_of = [&](int kp) { return pow2 ? kp >> pshift : kp / P; };
-    auto within = [&](int kp) { return pow2 ? kp & (P - 1) : kp % P; };
+    // (no branch between sizes that are powers of two and others: exact below 2^32 / P keys, and always for the former)
+    auto block_of = [&](int kp) { return (int)__umulhi((unsigned)kp, a.page_magic); };
+    auto within = [&](int kp) { return kp - block_of(kp) * P; };
     auto page_of = [&](int kp) {
         const int page = page_lds[min(max(block_of(kp) - first_page, 0), TILES_PAGE_CACHE - 1)];
         return kp < k_hi ? page : -1;
@@ -428,7 +437,7 @@ __device__ __forceinline__ void diff_tiles_group(const DiffArgs& a, const int32_
     bool k_mine[KST], v_mine[VST];
 #pragma unroll
     for (int i = 0; i < KST; ++i) {
-        k_mine[i] = (int)threadIdx.x + 256 * i < k_chunks;
+        k_mine[i] = FULL || (int)threadIdx.x + 256 * i < k_chunks;
         const int ci = min((int)threadIdx.x + 256 * i, k_chunks - 1);
         const int key = ci / (2 * D / 8), ch = 8 * (ci % (2 * D / 8)), map = ch >= D ? 1 : 0;
         k_key[i] = key;
@@ -438,7 +447,7 @@ __device__ __forceinline__ void diff_tiles_group(const DiffArgs& a, const int32_
     }
 #pragma unroll
     for (int i = 0; i < VST; ++i) {
-        v_mine[i] = (int)threadIdx.x + 256 * i < v_chunks;
+        v_mine[i] = (FULL && NDB % 4 == 0) || (int)threadIdx.x + 256 * i < v_chunks;
         const int ci = min((int)threadIdx.x + 256 * i, v_chunks - 1);
         v_ch[i] = ci >> 2;
         v_key[i] = 8 * (ci & 3);
@@ -501,7 +510,7 @@ __device__ __forceinline__ void diff_tiles_group(const DiffArgs& a, const int32_
 #pragma unroll
                 for (int c = 0; c < NCH; ++c) {
                     bf16x8 kf = zero8;                // (channels at and beyond head_dim were never staged)
-                    if (32 * c + 8 * b < D)
+                    if (FULL || 32 * c + 8 * b < D)
                         kf = *reinterpret_cast<const bf16x8*>(&k_lds[(16 * j + col) * KPITCH + map * 32 * NCH + 32 * c + 8 * b]);
                     s[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[map][c], s[j], 0, 0, 0);
                 }
@@ -511,14 +520,26 @@ __device__ __forceinline__ void diff_tiles_group(const DiffArgs& a, const int32_
             for (int j = 0; j < 2; ++j)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    float x = s[j][r] * pre;
-                    if (capped) {
-                        const float e = __builtin_amdgcn_exp2f(x);                    // exp(2 s / cap)
-                        x = cap2 - 2.0f * cap2 * __builtin_amdgcn_rcpf(e + 1.0f);
-                    }
-                    const int key = tb + 16 * j + 4 * b + r;
-                    sv[j][r] = (interior || (key < kend_c && key >= kbeg_c)) ? x : -INFINITY;
+                    sv[j][r] = s[j][r] * pre;
                 }
+            if (capped) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float e = __builtin_amdgcn_exp2f(sv[j][r]);             // exp(2 s / cap)
+                        sv[j][r] = cap2 - 2.0f * cap2 * __builtin_amdgcn_rcpf(e + 1.0f);
+                    }
+            }
+            if (!interior) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int key = tb + 16 * j + 4 * b + r;
+                        if (!(key < kend_c && key >= kbeg_c)) sv[j][r] = -INFINITY;
+                    }
+            }
             float tile_max = fmaxf(fmaxf(fmaxf(sv[0][0], sv[0][1]), fmaxf(sv[0][2], sv[0][3])),
                                    fmaxf(fmaxf(sv[1][0], sv[1][1]), fmaxf(sv[1][2], sv[1][3])));
             tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16, MLR_WAVE));
@@ -546,7 +567,7 @@ __device__ __forceinline__ void diff_tiles_group(const DiffArgs& a, const int32_
             l_run[map] += psum;
 #pragma unroll
             for (int db = 0; db < NDB; ++db) {
-                if (16 * db >= V) break;
+                if (!FULL && 16 * db >= V) break;
                 const __bf16* vrow = &v_lds[(16 * db + col) * VPITCH];
                 const bf16x4 v0 = *reinterpret_cast<const bf16x4*>(vrow + 4 * b);
                 const bf16x4 v1 = *reinterpret_cast<const bf16x4*>(vrow + 16 + 4 * b);
@@ -560,7 +581,9 @@ __device__ __forceinline__ void diff_tiles_group(const DiffArgs& a, const int32_
     const int tb_last = k_lo + ((k_hi - k_lo - 1) / TKEYS) * TKEYS;
     Staged sa, sb;
     fetch(k_lo, sa);
+    __builtin_amdgcn_sched_barrier(0);                // (in this order, as in the loop: its waits count on it)
     fetch(min(k_lo + TKEYS, tb_last), sb);
+    __builtin_amdgcn_sched_barrier(0);
     for (int tb = k_lo; tb < k_hi; tb += 2 * TKEYS) {
         __syncthreads();                              // the tile before has been read
         stash(sa);
@@ -589,7 +612,7 @@ __device__ __forceinline__ void diff_tiles_group(const DiffArgs& a, const int32_
             float* dst = a.partial + ((place * a.q_heads * 2 + head * 2 + map) * a.max_splits + split) * (V + 2);
 #pragma unroll
             for (int db = 0; db < NDB; ++db) {
-                if (16 * db >= V) break;
+                if (!FULL && 16 * db >= V) break;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) dst[16 * db + 4 * b + r] = o[map][db][r];
             }
@@ -605,7 +628,7 @@ __device__ __forceinline__ void diff_tiles_group(const DiffArgs& a, const int32_
     float ss = 0.f;
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
-        if (16 * db >= V) break;
+        if (!FULL && 16 * db >= V) break;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const float d = o[0][db][r] * inv1 - a.lam * (o[1][db][r] * inv2);
@@ -621,7 +644,7 @@ __device__ __forceinline__ void diff_tiles_group(const DiffArgs& a, const int32_
     const __bf16* gate = a.gate ? reinterpret_cast<const __bf16*>(a.gate) + (size_t)(row0 + tok) * a.gate_stride + (size_t)head * V : nullptr;
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
-        if (16 * db >= V) break;
+        if (!FULL && 16 * db >= V) break;
         bf16x4 w4;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -633,7 +656,7 @@ __device__ __forceinline__ void diff_tiles_group(const DiffArgs& a, const int32_
     }
 }
 
-template <int NCH, int NDB>
+template <int NCH, int NDB, bool FULL>
 __global__ __launch_bounds__(256) void diff_attention_tiles_kernel(DiffArgs a, const int32_t* __restrict__ group_row0,
                                                                    const int32_t* __restrict__ group_ntok, int groups,
                                                                    int col_heads, int wave_heads, int token_blocks,
@@ -642,8 +665,17 @@ __global__ __launch_bounds__(256) void diff_attention_tiles_kernel(DiffArgs a, c
     __shared__ __attribute__((aligned(16))) __bf16 v_lds[16 * NDB * (TKEYS + 4)];
     __shared__ int32_t page_lds[TILES_PAGE_CACHE];
     // (the longest groups of a prompt first: the workgroups that start last are the short ones)
-    diff_tiles_group<NCH, NDB>(a, group_row0, group_ntok, col_heads, wave_heads, token_blocks, map_split,
+    diff_tiles_group<NCH, NDB, FULL>(a, group_row0, group_ntok, col_heads, wave_heads, token_blocks, map_split,
                                groups - 1 - (int)blockIdx.x, k_lds, v_lds, page_lds);
+}
+
+template <int NCH, int NDB>
+static void launch_tiles_as(const DiffArgs& a, const int32_t* row0, const int32_t* ntok, int groups, dim3 grid, int ch, int wh, int tbw,
+                            int ms, hipStream_t stream) {
+    if (a.head_dim == 32 * NCH && a.value_dim == 16 * NDB)
+        diff_attention_tiles_kernel<NCH, NDB, true><<<grid, 256, 0, stream>>>(a, row0, ntok, groups, ch, wh, tbw, ms);
+    else
+        diff_attention_tiles_kernel<NCH, NDB, false><<<grid, 256, 0, stream>>>(a, row0, ntok, groups, ch, wh, tbw, ms);
 }
 
 template <int NCH>
@@ -652,9 +684,9 @@ static int launch_tiles(const DiffArgs& a, const int32_t* row0, const int32_t* n
     const int g = a.q_heads / a.kv_heads;
     dim3 grid(groups, a.kv_heads * ((g + ch * wh - 1) / (ch * wh)), a.max_splits);
     const int ndb = (a.value_dim + 15) / 16;
-    if (ndb <= 2) diff_attention_tiles_kernel<NCH, 2><<<grid, 256, 0, stream>>>(a, row0, ntok, groups, ch, wh, tbw, ms);
-    else if (ndb <= 4) diff_attention_tiles_kernel<NCH, 4><<<grid, 256, 0, stream>>>(a, row0, ntok, groups, ch, wh, tbw, ms);
-    else diff_attention_tiles_kernel<NCH, 8><<<grid, 256, 0, stream>>>(a, row0, ntok, groups, ch, wh, tbw, ms);
+    if (ndb <= 2) launch_tiles_as<NCH, 2>(a, row0, ntok, groups, grid, ch, wh, tbw, ms, stream);
+    else if (ndb <= 4) launch_tiles_as<NCH, 4>(a, row0, ntok, groups, grid, ch, wh, tbw, ms, stream);
+    else launch_tiles_as<NCH, 8>(a, row0, ntok, groups, grid, ch, wh, tbw, ms, stream);
     return (int)hipGetLastError();
 }
 #endif
@@ -702,11 +734,11 @@ int mlr_diff_attention(const void* q, long q_stride, const void* k_pages, const 
     DiffArgs a{(const elem_t*)q, q_stride, (const elem_t*)k_pages, (const elem_t*)v_pages, block_table, slots, positions,
                (const elem_t*)gate, gate_stride, (elem_t*)out, partial, max_blocks, q_heads, kv_heads, head_dim, value_dim,
                page_size, split_keys, max_splits, scale, softcap, temp_coef, temp_every, lam, out_scale, eps,
-               group_first, group_count, group_tokens, mask_kind, mask_size};
+               group_first, group_count, group_tokens, mask_kind, mask_size, 0};
     diff_attention_partial_kernel<<<dim3(rows, q_heads * 2, max_splits), 64, 0, stream>>>(a);
     int err = (int)hipGetLastError();
     if (err != 0) return err;
-    diff_attention_combine_kernel<<<dim3(rows, q_heads), 128, 0, stream>>>(a);
+    launch_combine(a, rows, stream);
     return (int)hipGetLastError();
 }
 
@@ -751,14 +783,15 @@ int mlr_diff_attention_tiles(const void* q, long q_stride, const void* k_pages, 
     DiffArgs a{(const elem_t*)q, q_stride, (const elem_t*)k_pages, (const elem_t*)v_pages, block_table, slots, positions,
                (const elem_t*)gate, gate_stride, (elem_t*)out, partial, max_blocks, q_heads, kv_heads, head_dim, value_dim,
                page_size, split_keys, max_splits, scale, softcap, temp_coef, temp_every, lam, out_scale, eps,
-               group_row0, group_ntok, group_tokens, mask_kind, mask_size};
+               group_row0, group_ntok, group_tokens, mask_kind, mask_size,
+               (unsigned)(((1ull << 32) + (unsigned)page_size - 1) / (unsigned)page_size)};
     const int nch = (head_dim + 31) / 32;
     int err;
     if (nch == 1) err = launch_tiles<1>(a, group_row0, group_ntok, groups, ch, wh, tbw, ms, stream);
     else if (nch == 2) err = launch_tiles<2>(a, group_row0, group_ntok, groups, ch, wh, tbw, ms, stream);
     else err = launch_tiles<4>(a, group_row0, group_ntok, groups, ch, wh, tbw, ms, stream);
     if (err != 0 || partial == nullptr) return err;
-    diff_attention_combine_kernel<<<dim3(groups * group_tokens, q_heads), 128, 0, stream>>>(a);
+    launch_combine(a, groups * group_tokens, stream);
     return (int)hipGetLastError();
 #else
     return -10;
