@@ -509,8 +509,8 @@ __device__ __forceinline__ floatx4 mma4_lower(const floatx4& a, const floatx4& b
 // thread takes one pair (120 a half); between the halves e^{c_t - c_s} = e^{c_t - c_15} e^{c_15 - c_s}, neither above 1, and
 // the sums are a matrix product.  T = (I + A)^-1 by halves too: two triangles of 16 a lane column by column, and
 // -T22 A21 T11 between them.  A thread for each of 1024 pairs, half of them idle, T row by row over 32 rows, and the two
-// products with T one element a thread took 199 us for 2048 tokens of 16 heads of 128 x 128 channels; this one 98, of
-// which the exponentials are the most.
+// products with T one element a thread took 199 us for 2048 tokens of 16 heads of 128 x 128 channels; this one 104 while a
+// thread waited for its elements of q, k and the decays one after the other, now 87, of which the exponentials are the most.
 __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(DeltaChunkArgs g) {
     constexpr int C = DELTA_CHUNK, CS = DELTA_CHUNK + 4;
     const DeltaArgs& a = g.d;
@@ -535,20 +535,37 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(DeltaChunkArgs
     float* Y = Kt + (size_t)C * Np;
     float* B = Y + (size_t)C * V;
     float* G = B + C * C;
-    for (int idx = tid; idx < C * Np; idx += 256) {
-        const int t = idx / Np, i = idx % Np;
-        float dq = 0.f, dk = 0.f, dc = 0.f;
-        if (t < n && i < N) {
-            const size_t row = (size_t)(r0 + t);
-            dq = to_float(a.q[row * a.q_stride + qk_head * N + i]);
-            dk = to_float(a.k[row * a.k_stride + qk_head * N + i]);
-            dc = a.log_decay[decay_at(a, row, head, i)];
+    // (eight elements of each asked for at once, clamped and without a branch: one after the other a thread waited for memory
+    // sixteen times, and once more for every beta)
+    const float beta_raw = a.beta_raw[(size_t)(r0 + min(tid, n - 1)) * a.beta_stride + head];
+    constexpr int EACH = 8;
+    for (int at = tid; at < C * Np; at += 256 * EACH) {
+        elem_t dq[EACH], dk[EACH];
+        float dc[EACH];
+        int t[EACH], i[EACH];
+#pragma unroll
+        for (int e = 0; e < EACH; ++e) {
+            t[e] = (at + 256 * e) / Np;
+            i[e] = (at + 256 * e) % Np;
+            const size_t row = (size_t)(r0 + min(t[e], n - 1));
+            const int ch = min(i[e], N - 1);
+            dq[e] = a.q[row * a.q_stride + qk_head * N + ch];
+            dk[e] = a.k[row * a.k_stride + qk_head * N + ch];
+            dc[e] = a.log_decay[decay_at(a, row, head, ch)];
         }
-        q_l[t * NS + i] = dq; k_l[t * NS + i] = dk; c_l[t * NS + i] = dc;
+#pragma unroll
+        for (int e = 0; e < EACH; ++e) {
+            if (at + 256 * e >= C * Np) break;
+            const bool there = t[e] < n && i[e] < N;
+            q_l[t[e] * NS + i[e]] = there ? to_float(dq[e]) : 0.f;
+            k_l[t[e] * NS + i[e]] = there ? to_float(dk[e]) : 0.f;
+            c_l[t[e] * NS + i[e]] = there ? dc[e] : 0.f;
+        }
     }
+    if (tid < C) beta_l[tid] = tid < n ? sigmoid_f(beta_raw) : 0.f;
     for (int p = tid; p < C * CS; p += 256) A_l[p] = B_l[p] = T_l[p] = 0.f;
     __syncthreads();
-    for (int t = wave; t < C; t += 4) {                     // unit vectors, q scaled; beta
+    for (int t = wave; t < C; t += 4) {                     // unit vectors, q scaled
         float qq = 0.f, kk = 0.f;
         for (int i = lane; i < N; i += 64) {
             const float dq = q_l[t * NS + i], dk = k_l[t * NS + i];
@@ -561,7 +578,6 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(DeltaChunkArgs
             fk = 1.0f / sqrtf(wave_sum(kk) + a.unit_eps);
         }
         for (int i = lane; i < N; i += 64) { q_l[t * NS + i] *= fq; k_l[t * NS + i] *= fk; }
-        if (lane == 0) beta_l[t] = t < n ? sigmoid_f(a.beta_raw[(size_t)(r0 + t) * a.beta_stride + head]) : 0.f;
     }
     for (int i = tid; i < Np; i += 256) {                   // c_t: the running sum of the log decays (rows past n add 0)
         float sum = 0.f;
