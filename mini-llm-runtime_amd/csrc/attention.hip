@@ -244,8 +244,8 @@ __global__ __launch_bounds__(64) void attention_combine_kernel(AttnArgs a) {
 // channel from a cache line of its own (16 heads on 8 of 128 channels, pages of 16: 111 us for eight tokens behind 400 keys, 306
 // behind 4000, 0.68 ms for a prompt of 400 and 16.7 for one of 2048; here 19, 63, 50 us and 0.57 ms).  A tile is a chain of products,
 // exchanges and waits, so no wait may stand for more than it needs: with branches around loads, LDS reads and products, page ids and
-// sums exchanged through LDS and every tile's values waited for before its scores, the four took 26, 77, 61 us and 0.69 ms.  Groups are found by the kernel: a row leads one when it is a multiple
-// of the tokens a group holds or does not continue the row before it.
+// sums exchanged through LDS and every tile's values waited for before its scores, the four took 26, 77, 61 us and 0.69 ms.
+// Groups are found by the kernel: a row leads one when it is a multiple of the tokens a group holds or does not continue the row before it.
 //
 // Keys are walked in tiles of 64 at absolute multiples of 64.  Per tile: wavefront w takes the scores of keys 16 w ..,
 // scores^T = K . Q^T, a chain over up to 128 channels a time; they meet in LDS, where 16 threads a column take the running

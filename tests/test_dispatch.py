@@ -249,6 +249,20 @@ def test_few_workgroups_take_narrower_key_ranges(rows, max_context, keys):
     assert max_context > 512 or split(64)[0] in (64, 128)
 
 
+@pytest.mark.parametrize("units,max_context,short,routed,keys", [
+    (32, 2048, True, False, 128), (32, 2724, True, False, 256), (16, 2724, True, False, 128), (4, 2048, True, False, 64), (4, 4096, True, False, 128),
+    (4, 4097, True, False, 256), (32, 2048, False, False, 256), (32, 2048, True, True, 256), (64, 512, True, False, 64), (128, 512, True, False, 128),
+    (512, 2048, True, False, 0), (4, 256, True, False, 0)])
+def test_differential_attention_of_few_short_groups_takes_narrower_key_ranges(units, max_context, short, routed, keys):
+    from mini_llm_runtime_amd.parts.diff_attention import DiffAttention
+    part = object.__new__(DiffAttention)
+    part.spec, part.mask, part._page_size = type("Spec", (), dict(q_heads=16, value_dim=128)), None, 16
+    ctx = context(max_context)
+    ctx.routed = routed
+    found = part._tile_splits(ctx, units, 4 * units, 1 << 40, short)
+    assert found == ((keys, -(-max_context // keys)) if keys else (0, 1))
+
+
 @pytest.mark.parametrize("sizes", [(17, 6144, 2048), (64, 12288, 1024), (333, 768, 2048), (1777, 4096, 18432), (1603, 28736, 6016), (653, 23648, 2176)])
 def test_products_of_a_model_with_a_router_keep_the_order_of_their_sums(sizes):
     """Where the vendor library may add in another order than the many-row kernel, a model that chooses among experts stays with
