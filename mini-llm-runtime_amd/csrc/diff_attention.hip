@@ -28,6 +28,7 @@
 // both maps.  Keys and values are staged once per workgroup through LDS in tiles of 32 keys and serve both maps of
 // all its heads; the head's epilogue (difference, norm, gate) runs in registers.
 #include "common.h"
+#include "pages.h"
 
 #define TILE_KEYS 64
 #define DIM_CHUNK 64
@@ -47,7 +48,7 @@ struct DiffArgs {
     // group_first[group] + i while i < group_count[group] (partial results are indexed by blockIdx.x)
     const int32_t* group_first; const int32_t* group_count; int group_tokens;
     int mask_kind, mask_size;                  // 0: every earlier key; 1: the last mask_size positions; 2: the query's block
-    unsigned page_magic;                       // ceil(2^32 / page_size): the high word of a product with it divides by the page size
+    PageDivisor pages;                         // (of the matrix-core kernel)
 };
 
 #define MASK_NONE 0
@@ -424,8 +425,8 @@ __device__ __forceinline__ void diff_tiles_group(const DiffArgs& a, const int32_
     }
     // (no load from the block table here: a global load behind a branch makes the compiler wait for every load in
     // flight, one tile's loads would then go out one after the other; the host keeps a range within the cache)
-    // (no branch between sizes that are powers of two and others: exact below 2^32 / P keys, and always for the former)
-    auto block_of = [&](int kp) { return (int)__umulhi((unsigned)kp, a.page_magic); };
+    // (no branch between sizes that are powers of two and others)
+    auto block_of = [&](int kp) { return page_of_key(a.pages, kp); };
     auto within = [&](int kp) { return kp - block_of(kp) * P; };
     auto page_of = [&](int kp) {
         const int page = page_lds[min(max(block_of(kp) - first_page, 0), TILES_PAGE_CACHE - 1)];
@@ -734,13 +735,16 @@ int mlr_diff_attention(const void* q, long q_stride, const void* k_pages, const 
     DiffArgs a{(const elem_t*)q, q_stride, (const elem_t*)k_pages, (const elem_t*)v_pages, block_table, slots, positions,
                (const elem_t*)gate, gate_stride, (elem_t*)out, partial, max_blocks, q_heads, kv_heads, head_dim, value_dim,
                page_size, split_keys, max_splits, scale, softcap, temp_coef, temp_every, lam, out_scale, eps,
-               group_first, group_count, group_tokens, mask_kind, mask_size, 0};
+               group_first, group_count, group_tokens, mask_kind, mask_size, {}};
     diff_attention_partial_kernel<<<dim3(rows, q_heads * 2, max_splits), 64, 0, stream>>>(a);
     int err = (int)hipGetLastError();
     if (err != 0) return err;
     launch_combine(a, rows, stream);
     return (int)hipGetLastError();
 }
+
+// For tests: the page of a key as the matrix-core kernels work it out (pages.h).
+int mlr_page_of_key(int page_size, int key) { return page_of_key(page_divisor(page_size), key); }
 
 // Groups of consecutive tokens of one request on the matrix cores (bfloat16): prompt portions in groups of up to
 // 16 * (4 / min(4, q_heads / kv_heads)) tokens, single tokens and short portions in smaller ones.  `group_tokens`:
@@ -783,8 +787,7 @@ int mlr_diff_attention_tiles(const void* q, long q_stride, const void* k_pages, 
     DiffArgs a{(const elem_t*)q, q_stride, (const elem_t*)k_pages, (const elem_t*)v_pages, block_table, slots, positions,
                (const elem_t*)gate, gate_stride, (elem_t*)out, partial, max_blocks, q_heads, kv_heads, head_dim, value_dim,
                page_size, split_keys, max_splits, scale, softcap, temp_coef, temp_every, lam, out_scale, eps,
-               group_row0, group_ntok, group_tokens, mask_kind, mask_size,
-               (unsigned)(((1ull << 32) + (unsigned)page_size - 1) / (unsigned)page_size)};
+               group_row0, group_ntok, group_tokens, mask_kind, mask_size, page_divisor(page_size)};
     const int nch = (head_dim + 31) / 32;
     int err;
     if (nch == 1) err = launch_tiles<1>(a, group_row0, group_ntok, groups, ch, wh, tbw, ms, stream);

@@ -22,6 +22,7 @@
 // engine's for sizes that the matrix-core kernel does not take.
 // `sink_attention_tiles_kernel` (bfloat16): the same on the matrix cores, see there.
 #include "common.h"
+#include "pages.h"
 
 #define MASK_ALL 0
 #define MASK_WINDOW 1
@@ -45,6 +46,7 @@ struct SinkArgs {
     // the group's first tile on and leaves (unnormalised values, maximum, sum) in partial[((g * tokens + i) * q_heads +
     // head) * splits + z][value_dim + 4] for token i of group g; null: one workgroup walks every key and writes out
     float* partial; int split_keys, splits, group_tokens;
+    PageDivisor pages;                         // (of `sink_attention_tiles_kernel`)
 };
 
 __device__ __forceinline__ int first_seen(int pos, int kind, int size) {
@@ -614,13 +616,11 @@ __global__ __launch_bounds__(256) void sink_attention_tiles_kernel(SinkArgs a, c
     bf16x8 kreg_a[NSK], vreg_a[NSV];
     bool have_a = false;
     const int my_key = tid & 31, my_chunk = tid >> 5;
-    // (a key's page by the high word of a product with ceil(2^32 / page size): exact below 2^32 / page size keys)
-    const unsigned magic = 0xffffffffu / (unsigned)a.page_size + 1u;
     auto fetch = [&](int t0, bf16x8 (&kreg)[NSK], bf16x8 (&vreg)[NSV], bool& have) {
         const int kp = t0 + my_key;
         const bool lead = t0 < lead_end;
         const bool inside = (kp >= kbegin || kp < a.keep_first) && kp < (lead ? lead_end : main_end);
-        const int kb = a.page_size > 1 ? (int)__umulhi((unsigned)kp, magic) : kp;
+        const int kb = page_of_key(a.pages, kp);
         const int rel = inside ? kb - (lead ? lead0 : block0) : -1, blk = lead ? rel : n_lead + rel;
         const int listed = page_lds[min(max(blk, 0), max(n_blocks - 1, 0))];
         const int page = (rel >= 0 && blk < n_blocks) ? listed : -1;
@@ -1064,7 +1064,7 @@ int mlr_sink_attention(const void* q, long q_stride, const void* k_pages, long k
         return -1;
     SinkArgs a{(const elem_t*)q, q_stride, (const elem_t*)k_pages, k_row, (const elem_t*)v_pages, v_row, block_table,
                slots, positions, sink, (elem_t*)out, out_stride, max_blocks, q_heads, kv_heads, key_dim, value_dim,
-               page_size, mask_kind, mask_size, keep_first, scale, softcap, nullptr, 0, 1, 1};
+               page_size, mask_kind, mask_size, keep_first, scale, softcap, nullptr, 0, 1, 1, {}};
     sink_attention_kernel<<<dim3(rows, q_heads), 64, 0, stream>>>(a);
     return (int)hipGetLastError();
 }
@@ -1151,7 +1151,7 @@ int mlr_sink_attention_tiles(const void* q, long q_stride, const void* k_pages, 
     SinkArgs a{(const elem_t*)q, q_stride, (const elem_t*)k_pages, k_row, (const elem_t*)v_pages, v_row, block_table,
                slots, positions, sink, (elem_t*)out, out_stride, max_blocks, q_heads, kv_heads, key_dim, value_dim,
                page_size, mask_kind, mask_size, keep_first, scale, softcap, splits > 1 ? partial : nullptr, split_keys, splits > 1 ? splits : 1,
-               (split_values ? 16 : 64) / head_block};
+               (split_values ? 16 : 64) / head_block, page_divisor(page_size)};
     if (splits > 1 && (partial == nullptr || split_keys <= 0 || split_keys % TK != 0 || splits > 65535 || a.group_tokens > 65535))
         return -1;
     const int nkf = (key_dim + 31) / 32, nvt = value_dim / 16;
@@ -1195,7 +1195,7 @@ int mlr_sink_attention_rows(const void* q, long q_stride, const void* k_pages, l
     if ((long)kv_heads * head_blocks > 65535) return -2;
     SinkArgs a{(const elem_t*)q, q_stride, (const elem_t*)k_pages, k_row, (const elem_t*)v_pages, v_row, block_table,
                slots, positions, sink, (elem_t*)out, out_stride, max_blocks, q_heads, kv_heads, key_dim, value_dim,
-               page_size, mask_kind, mask_size, keep_first, scale, softcap, nullptr, 0, 1, 128 / head_block};
+               page_size, mask_kind, mask_size, keep_first, scale, softcap, nullptr, 0, 1, 128 / head_block, {}};
     if (key_dim == 576 && value_dim == 512 && k_pages == v_pages && k_row == v_row)
         return launch_sink_rows<18, 32, true, 4>(a, group_first, group_count, groups, head_block, head_blocks, stream);
     if (key_dim == 128 && value_dim == 128 && k_pages != v_pages)

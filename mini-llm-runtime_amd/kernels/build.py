@@ -44,8 +44,8 @@ HIP_LIBRARIES = {
     "attention": (["attention.hip"], ["common.h"], True),
     "gemm": (["gemm.hip"], ["common.h"], True),
     "recurrence": (["recurrence.hip"], ["common.h"], True),
-    "diff_attention": (["diff_attention.hip"], ["common.h"], True),
-    "sink_attention": (["sink_attention.hip"], ["common.h"], True),
+    "diff_attention": (["diff_attention.hip"], ["common.h", "pages.h"], True),
+    "sink_attention": (["sink_attention.hip"], ["common.h", "pages.h"], True),
     "head_mix_attention": (["head_mix_attention.hip"], ["common.h"], True),
     "grouped_gemm": (["grouped_gemm.hip"], ["common.h"], True),
     "attention_tiles": (["attention_tiles.hip"], [], False),      # bfloat16 only by nature
