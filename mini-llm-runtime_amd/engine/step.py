@@ -472,7 +472,7 @@ class Runner:
 
     @staticmethod
     def _token_ids(tokens, vocab):
-        """An entry's tokens, checked (as they came when they are few, else as an int32 vector); refused when they
+        """An entry's tokens, checked (as a list when they are few, else as an int32 vector); refused when they
         are no whole numbers of the vocabulary."""
         if len(tokens) <= 16:                             # (few tokens: plain comparisons cost less than vectors)
             for t in tokens:
@@ -483,7 +483,7 @@ class Runner:
                 if not inside:
                     raise StepError(f"token id {t} is outside the vocabulary [0, {vocab})" if isinstance(t, (int, np.integer))
                                     else "token ids must be whole numbers")
-            return tokens                                 # (as they came: `_gather` puts them into its vector)
+            return [int(t) for t in tokens]               # (bytes and sets, too, hold whole numbers, and are no vectors)
         ids = np.asarray(tokens)
         if ids.ndim != 1 or ids.dtype.kind not in "iub":
             try:                                          # (numbers too large for a machine word, or no numbers)

@@ -64,6 +64,25 @@ def test_entries_that_are_more_than_tuples_of_values():
     assert gathered(entries) == ([3], [1], [5], [1], [0], True)
 
 
+@pytest.mark.parametrize("tokens", [b"\x05", bytearray(b"\x03\x04"), {7}, {9: "a"}, range(3), np.array([5, 6]), [np.int64(4)], (True,), [4.0], torch.tensor([8, 2]),
+                                    b"\x01" * 17, range(20)])
+def test_odd_forms_of_tokens_become_the_same_batch(tokens):
+    """What the native pass leaves to the Python one is taken as any list of the same numbers is."""
+    from types import SimpleNamespace
+    from mini_llm_runtime_amd.engine.step import Runner
+    r = object.__new__(Runner)
+    r.poisoned, r.max_batch_tokens, r.max_logits_rows, r.model = False, TOKENS, ROWS, SimpleNamespace(spec=SimpleNamespace(vocab_size=VOCAB))
+    ids, counts, slots, places, rows, totals = (np.full(n, -7, np.int32) for n in (TOKENS, TOKENS, TOKENS, TOKENS, ROWS, 4))
+    r._plain, r._plain_at, r._inputs = [ids, counts, slots, places, np.empty(TOKENS, np.int32), rows, totals], None, build.load("step_inputs")
+    r._plain_args = (ctypes.c_long(VOCAB), TOKENS, ROWS, *(ctypes.c_void_p(v.ctypes.data) for v in (ids, counts, slots, places, rows, totals)))
+    numbers = [int(t) for t in tokens]
+    for first in ([Entry(1, [3, 4], [1])], []):
+        want = r._gather([*first, Entry(2, numbers, [0])])
+        want = [v.tolist() for v in (want.ids, want.counts, want.slots, want.want_rows)]
+        got = r._gather([*first, Entry(2, tokens, [0])])
+        assert [v.tolist() for v in (got.ids, got.counts, got.slots, got.want_rows)] == want and got.ids.dtype == np.int32
+
+
 @pytest.mark.parametrize("fill,fill_first", [(0, False), (3, False), (2, True)])
 def test_the_rows_of_a_step(fill, fill_first):
     counts, slots, first = (np.array(v, np.int32) for v in ([1, 4, 2], [5, 0, 9], [17, 0, 300]))
