@@ -1127,7 +1127,7 @@ class Kernels:
         if bias is not None:
             _tensor(bias, "bias", torch.float32, (channels,))
         os_ = self._columns(out, "out", self.dtype, rows, channels)
-        self._check_state(live, stage, state_offset, (taps - 1) * channels)
+        self._check_state(live, stage, state_offset, (taps - 1) * channels, write_state)
         _tensor(slots, "slots", torch.int32, (rows,))
         _tensor(positions, "positions", torch.int32, (rows,))
         fn = self._lib("recurrence").mlr_causal_conv
@@ -1138,10 +1138,10 @@ class Kernels:
             "causal_conv")
 
     @staticmethod
-    def _check_state(live, stage, offset, count):
+    def _check_state(live, stage, offset, count, write_state):
         """States that are read from row slots[r] of `live` and written to that row of `stage`; where both are one slab, its rows
         come in pairs: `slots` names the live row of a pair and the other one, slot ^ 1, is written."""
-        _need(live.data_ptr() != stage.data_ptr() or live.shape[0] % 2 == 0, "a slab of pairs of rows has an even number of them")
+        _need(live.data_ptr() != stage.data_ptr() or not write_state or live.shape[0] % 2 == 0, "a slab of pairs of rows has an even number of them")
         for name, t in (("live", live), ("stage", stage)):
             _need(isinstance(t, torch.Tensor) and t.is_cuda and t.dtype is torch.float32 and t.dim() == 2
                   and t.is_contiguous(), f"{name}: the state must be float32 [slots, floats] on the GPU")
@@ -1212,7 +1212,7 @@ class Kernels:
         if skip is not None:
             _tensor(skip, "skip", torch.float32, (heads,))
         _tensor(out, "out", torch.float32, (rows, heads * n_values))
-        self._check_state(live, stage, state_offset, heads * n_keys * n_values)
+        self._check_state(live, stage, state_offset, heads * n_keys * n_values, write_state)
         _tensor(seg_first, "seg_first", torch.int32, (segments,))
         _tensor(seg_count, "seg_count", torch.int32, (segments,))
         _tensor(slots, "slots", torch.int32, (rows,))
@@ -1264,7 +1264,7 @@ class Kernels:
               "and no more requests and heads than the grid takes")
         _tensor(log_decay, "log_decay", torch.float32, (heads,))
         _tensor(out, "out", torch.float32, (rows, heads * n_values))
-        self._check_state(live, stage, state_offset, heads * n_keys * n_values)
+        self._check_state(live, stage, state_offset, heads * n_keys * n_values, write_state)
         for name, t, n in (("seg_first", seg_first, segments), ("seg_count", seg_count, segments), ("chunk_first", chunk_first, chunks),
                            ("chunk_count", chunk_count, chunks)):
             _tensor(t, name, torch.int32, (n,))
@@ -1326,7 +1326,7 @@ class Kernels:
         _tensor(log_decay, "log_decay", torch.float32, (rows, heads if decay_per_head else heads * n_keys))
         bs = self._columns(beta_raw, "beta_raw", torch.float32, rows, heads)
         _tensor(out, "out", torch.float32, (rows, heads * n_values))
-        self._check_state(live, stage, state_offset, heads * n_keys * n_values)
+        self._check_state(live, stage, state_offset, heads * n_keys * n_values, write_state)
         _tensor(seg_first, "seg_first", torch.int32, (segments,))
         _tensor(seg_count, "seg_count", torch.int32, (segments,))
         _tensor(slots, "slots", torch.int32, (rows,))
@@ -1370,7 +1370,7 @@ class Kernels:
         _tensor(log_decay, "log_decay", torch.float32, (rows, heads if decay_per_head else heads * n_keys))
         bs = self._columns(beta_raw, "beta_raw", torch.float32, rows, heads)
         _tensor(out, "out", torch.float32, (rows, heads * n_values))
-        self._check_state(live, stage, state_offset, heads * n_keys * n_values)
+        self._check_state(live, stage, state_offset, heads * n_keys * n_values, write_state)
         _tensor(seg_first, "seg_first", torch.int32, (segments,))
         _tensor(seg_count, "seg_count", torch.int32, (segments,))
         _tensor(chunk_first, "chunk_first", torch.int32, (chunks,))

@@ -98,3 +98,19 @@ def test_one_slab_of_pairs_gives_what_two_slabs_give(dtype):
             else:                                            # (what the kernel does not write of a row stays 3)
                 changed = written != 3.0
                 assert changed.any() and torch.equal(written[changed], stage[s][changed]) and torch.equal(stage[s][~changed], live[s][~changed]), i
+
+
+@pytest.mark.gpu
+def test_a_slab_that_is_only_read_need_not_come_in_pairs():
+    from mini_llm_runtime_amd.kernels import KernelError, Kernels
+    k = Kernels(torch.float32)
+    ints = lambda *x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    q, decay, slab = torch.randn(1, 8, device="cuda"), -torch.rand(1, 8, device="cuda"), torch.randn(3, 64, device="cuda")
+    before, outs = slab.clone(), []
+    for stage in (slab, slab.clone()):
+        out = torch.full((1, 8), float("nan"), device="cuda")
+        k.linear_recurrence(q, q, q, decay, out, slab, stage, 0, ints(0), ints(1), 1, ints(2), 1, 8, 8, write_state=False)
+        outs.append(out)
+    assert torch.equal(*outs) and torch.equal(slab, before)
+    with pytest.raises(KernelError, match="pairs"):
+        k.linear_recurrence(q, q, q, decay, outs[0], slab, slab, 0, ints(0), ints(1), 1, ints(2), 1, 8, 8)
