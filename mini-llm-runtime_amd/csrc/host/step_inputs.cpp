@@ -1,10 +1,11 @@
 // A step's inputs out of its batch entries: the tokens, counts, slots and wanted places of a plain batch read from the Python
-// objects in one pass, and the vectors that go to the device.  All of it is before the GPU has anything to do: entry by entry in Python
-// a step of 64 single tokens took 53 us for the first and 19 for the second, 198 from its call to the captured graph's launch; here
-// 5 and 2, and with the block tables' rows in one copy (../upload.hip) 48.
+// objects in one pass; step_rows.cpp lays them out for the device.  All of it is before the GPU has anything to do: entry by entry in
+// Python a step of 64 single tokens took 53 us for the first and 19 for the second, 198 from its call to the captured graph's launch;
+// here 5 and 2, and with the block tables' rows in one copy (../upload.hip) 48.
 //
 // Called through ctypes.PyDLL, so with the interpreter's lock held.  Raises nothing: what is not a plain batch is left to the
-// caller, which refuses it with the precise error or takes its odd forms.
+// caller, which refuses it with the precise error or takes its odd forms; it also takes every batch where this file could not be
+// compiled for want of the interpreter's headers.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -100,29 +101,6 @@ int mlr_step_entries(PyObject* entries, long vocab, int max_tokens, int max_rows
     totals[2] = rows;
     totals[3] = single ? 1 : 0;
     return 0;
-}
-
-// out: token ids | positions | slots of the step's rows, `total` rows of n entries and `fill` rows of the scratch request (token 0 at
-// position 0) in front of them or behind.
-void mlr_step_rows(int n, int total, const int32_t* ids, const int32_t* counts, const int32_t* slots, const int32_t* first, int fill,
-                   int fill_first, int scratch, int32_t* out) {
-    const int rows = total + fill;
-    int32_t *token = out, *position = out + rows, *slot = out + 2 * (int64_t)rows;
-    int at = 0;
-    const auto scratch_rows = [&]() {
-        for (int i = 0; i < fill; ++i, ++at) {
-            token[at] = position[at] = 0;
-            slot[at] = scratch;
-        }
-    };
-    if (fill_first) scratch_rows();
-    for (int e = 0, k = 0; e < n; ++e)
-        for (int i = 0; i < counts[e]; ++i, ++at, ++k) {
-            token[at] = ids[k];
-            position[at] = first[e] + i;
-            slot[at] = slots[e];
-        }
-    if (!fill_first) scratch_rows();
 }
 
 }  // extern "C"

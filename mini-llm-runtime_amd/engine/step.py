@@ -157,7 +157,8 @@ class Runner:
         # it (a value a token), wanted rows, and -- for a model that keeps other state per request -- one slot per entry
         self._lanes = 4 if self.cache.has_pairs() else 3
         self._upload = Uploader(6 * self.max_batch_tokens, self.device)
-        self._inputs = build.load("step_inputs")
+        self._host = build.load("host")
+        self._inputs = build.load("step_inputs") if build.available("step_inputs") else None
         # (ids, counts, slots, numbers of wanted places, first positions: a value a token; wanted rows; totals)
         self._plain = [np.empty(self.max_batch_tokens, np.int32) for _ in range(5)] + [np.empty(max(self.max_logits_rows, 1), np.int32),
                                                                                        np.empty(4, np.int32)]
@@ -416,11 +417,12 @@ class Runner:
 
     # -- the step ------------------------------------------------------------------------------
     def _gather(self, entries):
-        """The batch of `entries`: a plain one in one native pass, any other, and what must be refused, entry by entry."""
+        """The batch of `entries`: a plain one in one native pass (where it could be compiled), any other, and what must be refused,
+        entry by entry."""
         if self.poisoned:
             raise StepError("an earlier step failed after it had started; build a new runner")
         ids, counts, slots, _, first, rows, totals = self._plain
-        if self._inputs.mlr_step_entries(ctypes.py_object(entries), *self._plain_args) == 0:
+        if self._inputs is not None and self._inputs.mlr_step_entries(ctypes.py_object(entries), *self._plain_args) == 0:
             n, total, r, single = totals.tolist()
             return _Batch(total, ids[:total], counts[:n], slots[:n], rows[:r], bool(single), first[:n], self._plain_at)
         total, arrays, wanted = self._validate(entries)
@@ -501,7 +503,7 @@ class Runner:
         """Token ids | positions | slots of the step's rows, and with paired state the live rows of it, into `out`, the vector that
         `upload` gave; `fill` rows of the scratch request (token 0 at position 0) in front or behind."""
         rows = batch.total + fill
-        self._inputs.mlr_step_rows(len(batch.counts), batch.total, *batch.at, fill, 1 if fill_first else 0, self.cache.scratch_slot or 0,
+        self._host.mlr_step_rows(len(batch.counts), batch.total, *batch.at, fill, 1 if fill_first else 0, self.cache.scratch_slot or 0,
                                    upload.address)
         if self._lanes == 4:
             out[3 * rows:4 * rows] = self.cache.state_rows(out[2 * rows:3 * rows])

@@ -56,10 +56,12 @@ HIP_LIBRARIES = {
     "library_gemm": (["library_gemm.hip"], [], False, ["-lhipblaslt"]),      # host code around hipBLASLt
 }
 HOST_LIBRARIES = {
-    "host": (["host/cache_manager.cpp", "host/scheduler.cpp"], []),
-    "step_inputs": (["host/step_inputs.cpp"], []),
+    "host": (["host/cache_manager.cpp", "host/scheduler.cpp", "host/step_rows.cpp"], []),
+    "step_inputs": (["host/step_inputs.cpp", "host/step_rows.cpp"], []),
 }
-PYTHON_LIBRARIES = {"step_inputs"}       # they read Python objects: compiled with the interpreter's headers, called with its lock held
+# They read Python objects: compiled with the interpreter's headers, called with its lock held.  An interpreter may come without
+# its headers, so whoever uses one has a way without it (`available`).
+PYTHON_LIBRARIES = {"step_inputs"}
 
 _loaded = {}
 _lock = threading.Lock()
@@ -109,13 +111,25 @@ def _find_cxx():
     raise BuildError("no C++ compiler found for the host library")
 
 
+def _python_include():
+    return sysconfig.get_paths()["include"]
+
+
+def available(name):
+    """Whether a library is built or can be: one that reads Python objects needs the interpreter's headers."""
+    if name not in PYTHON_LIBRARIES or os.path.isfile(os.path.join(_python_include(), "Python.h")):
+        return True
+    out, _, digest = _plan(name, None)
+    return _is_current(out, digest)
+
+
 def _plan(name, tag):
     """(output path, command, digest of everything the output depends on)."""
     if name in HOST_LIBRARIES:
         sources, headers = HOST_LIBRARIES[name]
         flags = HOST_SANITIZE_FLAGS if host_sanitized() else HOST_FLAGS
         if name in PYTHON_LIBRARIES:
-            flags = [*flags, "-I" + sysconfig.get_paths()["include"]]
+            flags = [*flags, "-I" + _python_include()]
         out = os.path.join(_lib_dir(), f"libmlr_{name}{'_sanitized' if host_sanitized() else ''}.so")
         cmd = [_find_cxx(), *flags, "-o", out] + [os.path.join(CSRC, s) for s in sources]
     else:
@@ -166,6 +180,8 @@ def ensure_built(names, dtype=None, force=False, verbose=True):
             raise BuildError(f"library {name} needs an element type")
         out, cmd, digest = _plan(name, tag)
         if force or not _is_current(out, digest):
+            if not available(name):
+                raise BuildError(f"library {name} needs the Python interpreter's C headers, and {_python_include()} has no Python.h")
             todo.append((name, out, cmd, digest))
     if not todo:
         return
@@ -223,7 +239,7 @@ def load(name, dtype=None):
 def build_all(force=True, verbose=True):
     """Every library for both element types (the build check)."""
     import torch
-    ensure_built(list(HOST_LIBRARIES), force=force, verbose=verbose)
+    ensure_built([n for n in HOST_LIBRARIES if available(n)], force=force, verbose=verbose)
     untyped = [n for n, v in HIP_LIBRARIES.items() if not v[2]]
     typed = [n for n, v in HIP_LIBRARIES.items() if v[2]]
     ensure_built(untyped, force=force, verbose=verbose)

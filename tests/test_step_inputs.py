@@ -83,6 +83,48 @@ def test_odd_forms_of_tokens_become_the_same_batch(tokens):
         assert [v.tolist() for v in (got.ids, got.counts, got.slots, got.want_rows)] == want and got.ids.dtype == np.int32
 
 
+def test_without_the_interpreters_headers_every_batch_is_read_entry_by_entry(tmp_path, monkeypatch):
+    """The library that reads Python objects cannot be compiled there (and says what is missing); all others are."""
+    made = []
+    monkeypatch.setattr(build, "_python_include", lambda: str(tmp_path))
+    monkeypatch.setattr(build, "_lib_dir", lambda: str(tmp_path))
+    monkeypatch.setattr(build, "_compile", lambda out, cmd, digest: made.append(out))
+    assert not build.available("step_inputs") and build.available("host")
+    with pytest.raises(build.BuildError, match="Python.h"):
+        build.ensure_built(["step_inputs"], verbose=False)
+    build.build_all(verbose=False)
+    assert len(made) == len(build.HOST_LIBRARIES) - 1 + sum(2 if v[2] else 1 for v in build.HIP_LIBRARIES.values())
+    assert not any("step_inputs" in out for out in made)
+    out, _, digest = build._plan("step_inputs", None)
+    (tmp_path / "Python.h").touch()
+    assert build.available("step_inputs")
+    (tmp_path / "Python.h").unlink()
+    with open(out, "w"), open(out + ".stamp", "w") as stamp:
+        stamp.write(digest)
+    assert build.available("step_inputs")                   # (built elsewhere)
+
+
+@pytest.mark.gpu
+def test_a_runner_without_the_native_pass(model_folders, monkeypatch):
+    """The same logits to the bit: whole prompts, portions beside single tokens, captured steps with rows of the scratch request."""
+    from conftest import PAGE_SIZE, TINY
+    from helpers import last_one_by_one, make_requests, mixed, run_steps, whole
+    from mini_llm_runtime_amd.engine import Runner
+    from mini_llm_runtime_amd.parts import DecoderModel
+    model = DecoderModel.load(model_folders["A"], torch.float32)
+    reqs = make_requests(TINY["A"]["vocab_size"], [40, 13, 70, 2, 29], seed=3)
+    got = []
+    for there in (True, False):
+        monkeypatch.setattr(build, "available", lambda name: there or name != "step_inputs")
+        r = Runner(model, max_tokens=640, max_slots=6, max_length=160, max_batch_tokens=160, page_size=PAGE_SIZE["A"])
+        assert (r._inputs is not None) == there
+        got.append([run_steps(r, steps) for steps in (whole(reqs), mixed(reqs, seed=2)[0], last_one_by_one(reqs, tail=8))])
+    for with_it, without in zip(*got):
+        assert with_it.keys() == without.keys()
+        for i in with_it:
+            assert np.array_equal(with_it[i], without[i], equal_nan=True)
+
+
 @pytest.mark.parametrize("fill,fill_first", [(0, False), (3, False), (2, True)])
 def test_the_rows_of_a_step(fill, fill_first):
     counts, slots, first = (np.array(v, np.int32) for v in ([1, 4, 2], [5, 0, 9], [17, 0, 300]))
