@@ -124,8 +124,9 @@ class DiffAttention:
             raise PartError(f"a context of {longest} tokens needs key ranges (split_keys > 0): one workgroup walks {reach} keys")
         if base <= 0 or walk <= base or (units >= ctx.target_workgroups and not forced):
             return 0, 1
-        # (a model that routes keeps the sums that it has: a choice between experts turns on the last bit)
-        keys = base if ctx.routed or not short else ctx.narrowed(base, walk, units, ctx.target_workgroups, 32)
+        # (a model that routes keeps the sums that it has: a choice between experts turns on the last bit.  Ranges are launched and
+        # have their places for every key of the context, behind a mask too)
+        keys = base if ctx.routed or not short else ctx.narrowed(base, longest, units, ctx.target_workgroups, 32)
         while keys * 2 < walk and keys * 2 <= reach and (units * (-(-walk // (keys * 2))) >= ctx.target_workgroups or
                                                           (forced and units >= ctx.target_workgroups)):
             keys *= 2

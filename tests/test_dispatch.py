@@ -278,6 +278,25 @@ def test_products_of_a_model_with_a_router_keep_the_order_of_their_sums(sizes):
     assert k.wide_product(1777, 3000, 2048, "silu") and not k.wide_product(1777, 6000, 2048, "silu")     # (a gate's outputs are two)
 
 
+@pytest.mark.parametrize("mask,size", [("window", 512), ("chunk", 1), ("window", 100000), (None, 0)])
+@pytest.mark.parametrize("units", [1, 4, 16, 32, 200])
+def test_narrower_key_ranges_of_differential_attention_are_few_behind_a_mask_too(units, mask, size):
+    """Ranges are launched for the whole context, whatever part of it a mask lets a workgroup walk: what narrowing adds stays within its
+    32 ranges and its number of workgroups, and a long context behind a short window has the ranges of the setting."""
+    from mini_llm_runtime_amd.parts.diff_attention import DiffAttention
+    part = object.__new__(DiffAttention)
+    part.spec, part.mask, part.mask_size, part._page_size = type("Spec", (), dict(q_heads=16, value_dim=128)), mask, size, 16
+    for max_context in (200, 600, 1100, 2048, 4096, 4097, 8192, 8193, 32768):
+        ctx = context(max_context)
+        ctx.routed = False
+        keys, splits = part._tile_splits(ctx, units, 4 * units, 1 << 40, True)
+        if splits == 1:
+            continue
+        wide = part._tile_splits(ctx, units, 4 * units, 1 << 40, False)
+        assert splits == -(-max_context // keys)
+        assert (keys, splits) == wide or (keys < 256 and splits <= 32 and units * splits <= ctx.target_workgroups)
+
+
 @pytest.mark.parametrize("m,n,kk,act,taken,one_sum,few", [
     (33, 5632, 2112, None, True, True, False), (64, 8192, 4096, "silu", True, True, False), (32, 8448, 2112, None, True, True, False),
     (33, 5624, 2112, None, False, True, False), (32, 8192, 2112, None, False, True, False), (64, 16448, 4096, None, False, True, False),
