@@ -163,8 +163,8 @@ __device__ __forceinline__ void tile_group(const TileArgs& a, int grp, int kvh, 
         }
     }
     float m_ref = -INFINITY, l_run = 0.f;
-    float m_neg = 1e30f, raise_at = -INFINITY;       // -m_ref as it is added (a column with no key yet: exp2(-inf + finite) = 0, not NaN);
-                                                     // the score above which it is raised
+    float m_neg = 1e30f;             // -m_ref as it is added (a column with no key yet: exp2(-inf + finite) = 0, not NaN; the first key
+                                     // that it sees gets exp2(1e30) = inf, a sum beyond RAISE_AT, which sets the reference)
     floatx16 o[DB];
 #pragma unroll
     for (int db = 0; db < DB; ++db)

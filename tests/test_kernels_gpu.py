@@ -895,33 +895,43 @@ def test_prompt_portions_of_head_size_128(hq, hkv, page, before, n, window, spli
     assert max(errors) <= 1.1 * min(errors), errors
 
 
-@pytest.mark.parametrize("d", [128, 64])
-def test_prompt_portions_columns_do_not_depend_on_their_neighbours(d):
-    """A column's reference is raised by its own scores alone.  The second block's maximum is the rounded threshold itself, which
-    times the scale exceeds reference + 8 by a rounding: with neighbours that raise theirs in the same tile and with ones that
-    do not, the column's results are the same bits.  (Scores are sums of three factors of eight bits: exact.  The other keys of
-    the block lie at the edges of a probability's rounding to bfloat16, each with a channel of its own, so a raised reference shows.)"""
+@pytest.mark.parametrize("d,columns", [(128, 64), (128, 128), (64, 64), (64, 128)])
+def test_prompt_portions_columns_do_not_depend_on_their_neighbours(d, columns):
+    """A column's reference is raised by its own probabilities alone: where one of its two lanes' sums over a tile exceeds 256.  The first
+    block sets the reference, the second holds probabilities of 6 to 20 times that: with lanes' sums just below 256 and of exactly 256 (not
+    raised), just above, and above in one lane of the two (raised).  With neighbours that raise theirs in the same tile and with ones
+    that do not, the column's results are the same bits; and they are the softmax's, which they would not be if its lanes disagreed.
+    (Scores are sums of three factors of eight bits: exact.  The probabilities of the second block lie at the edges of the rounding to
+    bfloat16, each with a channel of its own, and the largest is no power of two: a raised reference shows.)"""
     k = kernels(torch.bfloat16)
     f32, scale, page = np.float32, d ** -0.5, 64
     c2 = f32(scale) * f32(1.44269504088896340736)
-    edges = []
-    for s0 in np.arange(20, 110, 2.0 ** -5).astype(f32):
-        m0 = f32(s0 * c2)
-        s1 = f32(f32(m0 + f32(8)) / c2)
-        if f32(s1 * c2) > f32(m0 + f32(8)) and 64 <= s1 < 128:
-            edges.append((s0, m0, s1))
-    edges = edges[:4]
-    assert len(edges) == 4
+    # a lane's sum is over 16 keys of a tile of 32, and over both tiles of a block where one wavefront takes them together
+    tiles = 2 if d == 128 and columns == 128 else 1
+    lane_of = (np.arange(32) >> (3 if d == 128 else 2)) & 1
+
+    def lane(total):
+        """Sixteen probabilities of about total / tiles together, each halfway between two bfloat16 numbers."""
+        p = total / tiles / 16 * (1 + (np.arange(16) - 7.5) / 32)
+        ulp = 2.0 ** (np.floor(np.log2(p)) - 7)
+        return (np.floor(p / ulp) + 0.5) * ulp
+    # halfway, too, eight on either side of a power of two; one is put above its edge, the next below: exactly 256
+    even = (16 + np.concatenate([-np.arange(31, 74, 6) / 32, np.arange(5, 48, 6) / 16])) / tiles
+    kinds = [(lane(254.5), lane(254.5)), (even, even), (lane(258), lane(258)), (lane(258), lane(100))]
+    spread = [[tiles * 2.0 ** (np.floor(np.log2(p)) - 8) for p in pair] for pair in kinds]        # whichever way an edge goes
+    lows, highs = ([[tiles * p.sum() + sign * u.sum() for p, u in zip(*two)] for two in zip(kinds, spread)] for sign in (-1, 1))
+    assert max(highs[0]) < 256 < min(lows[2]) and lows[3][0] > 256 > highs[3][1]
+    assert tiles * even.sum() == 256 and (even[:8] < 16 / tiles).all() and (even[8:] > 16 / tiles).all()
     keys, values = np.zeros((160, 4, d), f32), np.zeros((160, 4, d), f32)
-    for head, (s0, m0, s1) in enumerate(edges):
+    for head, lanes in enumerate(kinds):
         scores = np.zeros(128, f32)
-        scores[[0, 32]] = s0                                 # (both halves of a block: either may have a reference of its own)
+        scores[[0, 32]] = s0 = f32(60 + head)                # (both halves of a block: either may have a reference of its own)
         for half in (64, 96):
-            scores[half] = s1
-            for i in range(1, 32):
-                middle = (2 * ((i - 1) // 7) + 1) * 2.0 ** -8 + 1         # between two neighbours in bfloat16, times 2^4
-                x = f32((float(m0) + 4 + math.log2(middle)) / float(c2))
-                scores[half + i] = x + f32((i - 1) % 7 - 3) * np.spacing(x)
+            for side in (0, 1):
+                x = ((float(f32(s0 * c2)) + np.log2(lanes[side])) / float(c2)).astype(f32)
+                off = np.where(np.arange(16) % 2 == 0, 6, -6) if head == 1 else np.arange(16) % 7 - 3
+                x = x + off.astype(f32) * np.spacing(x)
+                scores[half + np.flatnonzero(lane_of == side)] = x
         rest = scores.copy()
         for part in range(3):                                # eight bits each
             digit = torch.tensor(rest).view(torch.int32).bitwise_and(-65536).view(torch.float32).numpy()
@@ -937,16 +947,22 @@ def test_prompt_portions_columns_do_not_depend_on_their_neighbours(d):
     table = torch.tensor([[0, 1, 2]], dtype=torch.int32, device="cuda")
     slots, pos = torch.zeros(32, dtype=torch.int32, device="cuda"), torch.arange(128, 160, dtype=torch.int32, device="cuda")
     first, count = torch.tensor([0], dtype=torch.int32, device="cuda"), torch.tensor([32], dtype=torch.int32, device="cuda")
-    for columns in (64, 128):
-        got = []
-        for neighbours in (0.0, 2.0):
-            q = torch.zeros((32, 4, d))
-            q[0, :, :3], q[1:, :, :3] = 1, neighbours
-            out = torch.full((32, 4 * d), float("nan"), dtype=torch.bfloat16, device="cuda")
-            k.attention_tiles(q.view(32, -1).to(torch.bfloat16).cuda(), k_pages, v_pages, table, slots, pos, out, first, count, 1, 4, 4, d, page, scale,
-                              columns=columns)
-            got.append(out[0])
-        assert bool((got[0].view(4, d)[:, 1:32] > 0).all()) and torch.equal(got[0], got[1]), columns
+    got = []
+    for neighbours in (0.0, 2.0):
+        q = torch.zeros((32, 4, d))
+        q[0, :, :3], q[1:, :, :3] = 1, neighbours
+        out = torch.full((32, 4 * d), float("nan"), dtype=torch.bfloat16, device="cuda")
+        k.attention_tiles(q.view(32, -1).to(torch.bfloat16).cuda(), k_pages, v_pages, table, slots, pos, out, first, count, 1, 4, 4, d, page, scale,
+                          columns=columns)
+        got.append(out.view(32, 4, d))
+        score = (q.double().transpose(0, 1) @ torch.tensor(keys).double().permute(1, 2, 0)) * scale               # [4, 32, 160]
+        seen = torch.arange(160)[None] <= torch.arange(128, 160)[:, None]
+        want = (torch.softmax(score.masked_fill(~seen, -math.inf), -1) @ torch.tensor(values).double().transpose(0, 1)).transpose(0, 1)
+        # a probability is rounded to bfloat16 (2^-9 of itself, in numerator and denominator) and its score is a 32-bit sum; so is the result
+        error = (out.view(32, 4, d).double().cpu() - want).abs()
+        assert bool((error <= (2.0 ** -7 + 1e-4) * want).all()), (neighbours, float((error / want.clamp_min(1e-30)).max()))
+    for head in range(4):
+        assert bool((got[0][0, head, :64] > 0).all()) and torch.equal(got[0][0, head], got[1][0, head]), head
 
 
 @pytest.mark.parametrize("hq,hkv,d,page,window,split_keys", [(4, 2, 128, 16, None, 0), (4, 2, 128, 16, None, 64), (6, 2, 64, 32, 20, 0),
