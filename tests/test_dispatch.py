@@ -233,20 +233,22 @@ def test_key_ranges_of_one_width_whatever_the_batch():
     assert keys == 512 and splits == -(-300000 // 512) <= MAX_KEY_SPLITS and chunk == 3
 
 
-@pytest.mark.parametrize("rows,max_context,keys", [
-    (1, 512, 64), (1, 257, 64), (1, 1280, 64), (1, 1281, 128), (1, 2560, 128), (1, 2561, 256), (6, 512, 64), (7, 512, 128), (12, 512, 128),
-    (13, 512, 256), (3, 2048, 128), (4, 2048, 256), (8, 4096, 512), (1, 256, 0)])
-def test_few_workgroups_take_narrower_key_ranges(rows, max_context, keys):
-    """Half the setting's width while that is no more than three workgroups to two compute units and twenty ranges; a model that routes, a setting that has no half
-    and one that is narrow already stay with the setting."""
+@pytest.mark.parametrize("rows,max_context,keys,wide,of_64,of_320", [
+    (1, 512, 64, 256, 64, 320), (1, 257, 64, 256, 64, 0), (1, 1280, 64, 256, 64, 320), (1, 1281, 128, 256, 64, 320), (1, 2560, 128, 256, 64, 320),
+    (1, 2561, 256, 256, 64, 320), (6, 512, 64, 256, 64, 320), (7, 512, 128, 256, 64, 320), (12, 512, 128, 256, 64, 320), (13, 512, 256, 256, 64, 320),
+    (3, 2048, 128, 256, 64, 320), (4, 2048, 256, 256, 128, 320), (8, 4096, 512, 512, 512, 320), (1, 256, 0, 0, 64, 0)])
+def test_few_workgroups_take_narrower_key_ranges(rows, max_context, keys, wide, of_64, of_320):
+    """Half the setting's width (256) while that is no more than three workgroups to two compute units and twenty ranges.  A model that
+    routes (`wide`), a setting whose half is no multiple of 64 (320) and one that is narrow already (64) are never narrowed: their ranges
+    are the setting's, or wider ones where those still fill the GPU.  (0: one workgroup walks every key.)"""
     def split(base, routed=False):
         ctx = context(max_context, split_keys=base)
         ctx.compute_units, ctx.routed = 256, routed
         return ctx.attention_split(rows, rows, 8, 16, 128, longest=65504)[:2]
-    assert split(256) == ((keys, -(-max_context // keys)) if keys else (0, 1))
-    assert split(256, routed=True)[0] == (0 if max_context <= 256 else max(256, keys))
-    assert max_context <= 320 or rows * 8 * -(-max_context // 320) >= 512 or split(320)[0] == 320
-    assert max_context > 512 or split(64)[0] in (64, 128)
+    ranges = lambda width: (width, -(-max_context // width) if width else 1)  # noqa: E731
+    assert split(256) == ranges(keys) and split(256, routed=True) == ranges(wide)
+    assert split(64) == split(64, routed=True) == ranges(of_64)
+    assert split(320) == split(320, routed=True) == ranges(of_320)
 
 
 @pytest.mark.parametrize("units,max_context,short,routed,keys", [
