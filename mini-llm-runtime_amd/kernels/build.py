@@ -26,8 +26,8 @@ ARCH = "gfx950"
 HIP_FLAGS = ["-O3", "-std=c++17", "-shared", "-fPIC", f"--offload-arch={ARCH}",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 HOST_FLAGS = ["-O2", "-std=c++17", "-shared", "-fPIC"]
-# MLR_HOST_SANITIZE=1 in the environment: the host library (page bookkeeping, batch forming) is built with the
-# address and undefined-behaviour sanitizers, as its own file, and loaded instead of the plain one.  The
+# MLR_HOST_SANITIZE=1 in the environment: the host libraries (page bookkeeping, batch forming, a step's inputs) are built with the
+# address and undefined-behaviour sanitizers, as files of their own, and loaded instead of the plain ones.  The
 # process must then have the sanitizer's runtime loaded first (LD_PRELOAD=$(gcc -print-file-name=libasan.so)).
 # The reference runs its host tests the same way in CI (.github/workflows/ci.yml:60-71).  CPU code only.
 HOST_SANITIZE_FLAGS = ["-O1", "-g", "-fno-omit-frame-pointer", "-std=c++17", "-shared", "-fPIC",
