@@ -500,14 +500,27 @@ struct ExpertsCost { int bm, bn; float round, all; };
 static const ExpertsCost EXPERTS_COSTS[] = {{128, 128, 5.32f, 9.03f}, {128, 192, 6.74f, 12.02f}, {128, 256, 7.25f, 14.68f}, {192, 256, 9.80f, 21.20f}};
 
 // Fewer rows an expert than fill such tiles half: what counts is the weight's way from memory, so narrow tiles, two workgroups on a
-// compute unit, and five or six blocks on their way: 32 x 64 while an expert's rows fit 32, 64 x 64 while they fit 64.  Measured on
-// 126 products of 8 to 64 experts with 1 to 127 rows each (uneven; 704 to 6144 k, 768 to 12288 rows of weight out of memory) against the
-// kernel that stages through registers, which took all of them before: up to 20 rows 0.83 of its time, to 55 0.81, beyond, in the
-// tiles above, 0.60 (the bits are the same).  16 experts, 192 rows: 1408 x 2048 gated 27.4 -> 23.4 us, 2048 x 704 15.8 -> 12.0 (the
-// weights alone 19 and 10); 8 experts of 64 rows, 2816 x 2048 gated 44.7 -> 28.0.
+// compute unit, and five or six blocks on their way: 32 x 64 while an expert's rows fit 32, 64 x 64 while they fit 64, or up to 128
+// rows while such tiles are no more than compute units (2 experts, 176 x 1088 x 256: 5.7 us, in a tile of 128 x 128 7.9; 4 of 392 x
+// 4096 x 1152 15.5, 18.6).  Measured on 126 products of 8 to 64 experts with 1 to 127 rows each (uneven; 704 to 6144 k, 768 to 12288
+// rows of weight out of memory) against the kernel that stages through registers, which took all of them before: up to 20 rows 0.83
+// of its time, to 55 0.81, beyond, in the tiles above, 0.60 (the bits are the same).  16 experts, 192 rows: 1408 x 2048 gated 27.4 ->
+// 23.4 us, 2048 x 704 15.8 -> 12.0 (the weights alone 19 and 10); 8 experts of 64 rows, 2816 x 2048 gated 44.7 -> 28.0.
+// Of up to 32 experts the products with a short k are that kernel's (-1): it asks for 128 k at a time and has four workgroups on a
+// compute unit, so its whole k is under way at once, while a workgroup here sets out a pipeline of five blocks first, and 512 to 1024
+// tiles are one round there and two here.  On 1100 products of 2 to 256 experts (64 to 1152 k, weights out of memory) these tiles took
+// below 448 k 0.65 to 1.41 of its time, 0.97 in the mean (32 experts, 79 rows, 4064 x 256 gated: 19.0 us, here 26.7), below 704 with
+// more than two tiles a unit 0.69 to 1.17 and 0.93 (16 experts, 39 rows, 3744 x 640 gated: 16.8, 19.6), beyond either line 0.52 to 1.15
+// and 0.79.  Of more experts they took 0.11 to 1.08 whatever k: that kernel looks for its expert one after the other.
 static int experts_shape_for(int M, int N, int K, int groups) {
-    if ((long)M < 56L * groups) return (long)M <= 20L * groups ? 4 : 5;
     const int units = compute_units() > 0 ? compute_units() : 256;
+    if ((long)M < 128L * groups) {
+        const long tiles = (long)groups * ((N + 63) / 64);
+        const bool one_round = (long)M >= 56L * groups && tiles <= units;
+        if (groups <= 32 && !one_round && K < (tiles <= 2 * units ? 448 : 704)) return -1;
+        if ((long)M < 56L * groups) return (long)M <= 20L * groups ? 4 : 5;
+        if (one_round) return 5;
+    }
     int best = 0;
     float least = 0.f;
     for (int s = 0; s < 4; ++s) {
@@ -762,7 +775,8 @@ int mlr_grouped_gemm(const void* a, long lda, long a_group, const void* w, long 
                   M, N, K, groups, act, out_float, limit, slope};
 #if MLR_BF16
     // rows by expert (the products a head, with inner sizes of 128 to 512, are faster on the small tile below)
-    if (experts_wide_takes(g, a_rows)) return run_experts_wide(experts_shape_for(M, N, K, groups), g, stream);
+    const int shape = experts_wide_takes(g, a_rows) ? experts_shape_for(M, N, K, groups) : -1;
+    if (shape >= 0) return run_experts_wide(shape, g, stream);
     if (offsets != nullptr && (long)M >= 256L * groups && N >= 128) {
         const int row_tiles = (M + 127) / 128 + (offsets ? groups : 0);
         if (row_tiles > 65535 || groups > 65535) return -2;
@@ -779,6 +793,15 @@ int mlr_grouped_gemm(const void* a, long lda, long a_group, const void* w, long 
     grouped_gemm_kernel<<<grid, 256, 0, stream>>>(g);
 #endif
     return (int)hipGetLastError();
+}
+
+// For tests: the shape that the products of experts take, -1 for the kernel that stages through registers.
+int mlr_experts_shape(int M, int N, int K, int groups) {
+#if MLR_BF16
+    return N >= 128 && K % EB_K == 0 ? experts_shape_for(M, N, K, groups) : -1;
+#else
+    return -1;
+#endif
 }
 
 // For tests and measurements: the products of experts in a given shape (0 .. 5).

@@ -340,3 +340,13 @@ def test_whether_a_model_routes_is_said_where_its_kernels_are_made(monkeypatch):
     monkeypatch.setattr(torch.cuda, "is_available", lambda: True)
     assert not hasattr(Kernels, "routed")
     assert Kernels(torch.bfloat16, routed=True).routed and not Kernels(torch.bfloat16).routed
+
+
+@pytest.mark.parametrize("rows,n,k,experts,shape", [
+    (160, 4096, 448, 8, 4), (160, 4096, 384, 8, -1), (161, 4096, 448, 8, 5), (447, 4096, 384, 8, -1), (320, 2048, 448, 16, 4), (320, 2112, 448, 16, -1),
+    (320, 2112, 640, 16, -1), (320, 2112, 704, 16, 4), (640, 4096, 640, 32, -1), (640, 4096, 64, 33, 4), (8, 128, 64, 256, 4), (448, 2048, 64, 8, 5),
+    (1023, 2048, 64, 8, 5), (447, 2048, 64, 8, -1), (448, 2112, 64, 8, -1), (448, 128, 64, 2, 0), (64, 100, 1024, 2, -1), (64, 128, 1000, 2, -1)])
+def test_products_of_experts_with_few_rows(rows, n, k, experts, shape):
+    """Both sides of every line: a short k of up to 32 experts, the rows a tile holds, tiles that are no more than compute units."""
+    from mini_llm_runtime_amd.kernels import build
+    assert build.load("grouped_gemm", torch.bfloat16).mlr_experts_shape(rows, n, k, experts) == shape
