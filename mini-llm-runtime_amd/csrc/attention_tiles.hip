@@ -34,11 +34,14 @@
 // matching A operand.
 //
 // Softmax in the base-2 domain, 32-bit.  A column's reference is the maximum of one of its tiles and is only raised when the
-// probabilities that a lane makes of a tile sum up to more than 2^8 (each then stays below that, far from overflow; the quotient at the
-// end does not depend on the reference): raising it means rescaling 64 accumulators, and with 32 columns
-// in a wavefront some column would need it in nearly every tile otherwise.  The sum is there anyway, so most tiles never take a
-// maximum: 49 vector instructions a tile for 58, and the exponentials need not wait for it (12 321 tokens of 16 heads in portions of
-// 2048: 0.6 % of the whole prompt, which the card's power bounds).  The decision is taken per
+// probabilities that a lane makes of a tile sum up to more than 2^20 (each then stays below that, as far from overflow as a value below
+// 2^107 leaves it; a probability has its eight bits at any size, and the quotient at the end does not depend on the reference): raising
+// it means taking the tile's exponentials again and rescaling 64 accumulators for all 32 columns of a wavefront, of which some one
+// would need it in many tiles otherwise.  From 2^8 on, scores that vary little gain as much but scores of a standard deviation
+// of 4 (before the base-2 scale) lose: against a maximum taken in every tile, 16 heads of 64 channels, 1000 tokens 17.6 us at a deviation
+// of 1, 19.3 at 4; with 2^8 17.7 and 22.3, now 17.7 and 17.8; heads of 128 behind 4000 keys 47.0 and 54.4, 45.1 and 59.7, now 44.9 and 45.2.
+// The sum is there anyway, so most tiles never take a maximum: 49 vector instructions a tile for 58, and the exponentials need not
+// wait for it (12 321 tokens of 16 heads in portions of 2048: 0.6 % of the whole prompt).  The decision is taken per
 // column from the column's own scores, so a column's arithmetic does not depend on its neighbours.  It does depend on the
 // workgroup's width where that is two ways over the keys: with head size 128 a column of 128 has one reference and one chain for both
 // halves of its blocks, a column of 64 two that are merged, so the two round their probabilities otherwise (as key ranges do, below;
@@ -67,7 +70,7 @@ typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 #define TILE_KEYS 32
 #define PAGE_IDS 2048
 #define VPITCH (BLOCK_KEYS + 8)        // elements per channel row of a staged block of values
-#define RAISE_AT 256.0f                // sum of a lane's probabilities in a tile from which the reference may be raised
+#define RAISE_AT 1048576.0f            // sum of a lane's probabilities in a tile from which the reference may be raised
 
 struct TileArgs {
     const __bf16* q;             // [M, q_heads, head_dim]

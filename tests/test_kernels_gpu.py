@@ -897,31 +897,31 @@ def test_prompt_portions_of_head_size_128(hq, hkv, page, before, n, window, spli
 
 @pytest.mark.parametrize("d,columns", [(128, 64), (128, 128), (64, 64), (64, 128)])
 def test_prompt_portions_columns_do_not_depend_on_their_neighbours(d, columns):
-    """A column's reference is raised by its own probabilities alone: where one of its two lanes' sums over a tile exceeds 256.  The first
-    block sets the reference, the second holds probabilities of 6 to 20 times that: with lanes' sums just below 256 and of exactly 256 (not
-    raised), just above, and above in one lane of the two (raised).  With neighbours that raise theirs in the same tile and with ones
+    """A column's reference is raised by its own probabilities alone: where one of its two lanes' sums over a tile exceeds 2^20.  The first
+    block sets the reference, the second holds probabilities of some 2^16 times that: with lanes' sums just below 2^20 and of exactly 2^20
+    (not raised), just above, and above in one lane of the two (raised).  With neighbours that raise theirs in the same tile and with ones
     that do not, the column's results are the same bits; and they are the softmax's, which they would not be if its lanes disagreed.
     (Scores are sums of three factors of eight bits: exact.  The probabilities of the second block lie at the edges of the rounding to
     bfloat16, each with a channel of its own, and the largest is no power of two: a raised reference shows.)"""
     k = kernels(torch.bfloat16)
-    f32, scale, page = np.float32, d ** -0.5, 64
+    f32, scale, page, bound = np.float32, d ** -0.5, 64, 2.0 ** 20
     c2 = f32(scale) * f32(1.44269504088896340736)
     # a lane's sum is over 16 keys of a tile of 32, and over both tiles of a block where one wavefront takes them together
     tiles = 2 if d == 128 and columns == 128 else 1
     lane_of = (np.arange(32) >> (3 if d == 128 else 2)) & 1
 
     def lane(total):
-        """Sixteen probabilities of about total / tiles together, each halfway between two bfloat16 numbers."""
-        p = total / tiles / 16 * (1 + (np.arange(16) - 7.5) / 32)
+        """Sixteen probabilities of about total / tiles of the bound together, each halfway between two bfloat16 numbers."""
+        p = total * bound / tiles / 16 * (1 + (np.arange(16) - 7.5) / 32)
         ulp = 2.0 ** (np.floor(np.log2(p)) - 7)
         return (np.floor(p / ulp) + 0.5) * ulp
-    # halfway, too, eight on either side of a power of two; one is put above its edge, the next below: exactly 256
-    even = (16 + np.concatenate([-np.arange(31, 74, 6) / 32, np.arange(5, 48, 6) / 16])) / tiles
-    kinds = [(lane(254.5), lane(254.5)), (even, even), (lane(258), lane(258)), (lane(258), lane(100))]
+    # halfway, too, eight on either side of a power of two; one is put above its edge, the next below: exactly the bound
+    even = (16 + np.concatenate([-np.arange(31, 74, 6) / 32, np.arange(5, 48, 6) / 16])) * (bound / 256 / tiles)
+    kinds = [(lane(0.994), lane(0.994)), (even, even), (lane(1.008), lane(1.008)), (lane(1.008), lane(0.4))]
     spread = [[tiles * 2.0 ** (np.floor(np.log2(p)) - 8) for p in pair] for pair in kinds]        # whichever way an edge goes
     lows, highs = ([[tiles * p.sum() + sign * u.sum() for p, u in zip(*two)] for two in zip(kinds, spread)] for sign in (-1, 1))
-    assert max(highs[0]) < 256 < min(lows[2]) and lows[3][0] > 256 > highs[3][1]
-    assert tiles * even.sum() == 256 and (even[:8] < 16 / tiles).all() and (even[8:] > 16 / tiles).all()
+    assert max(highs[0]) < bound < min(lows[2]) and lows[3][0] > bound > highs[3][1]
+    assert tiles * even.sum() == bound and (even[:8] < bound / 16 / tiles).all() and (even[8:] > bound / 16 / tiles).all()
     keys, values = np.zeros((160, 4, d), f32), np.zeros((160, 4, d), f32)
     for head, lanes in enumerate(kinds):
         scores = np.zeros(128, f32)
@@ -963,6 +963,15 @@ def test_prompt_portions_columns_do_not_depend_on_their_neighbours(d, columns):
         assert bool((error <= (2.0 ** -7 + 1e-4) * want).all()), (neighbours, float((error / want.clamp_min(1e-30)).max()))
     for head in range(4):
         assert bool((got[0][0, head, :64] > 0).all()) and torch.equal(got[0][0, head], got[1][0, head]), head
+    # the bound lies no lower: the probabilities at it were rounded beside the first reference (a raise to their maximum would change 40
+    # of the 64 results; a result at an edge of its own rounding may go either way)
+    kept = even + np.where(np.arange(16) % 2 == 0, 0.5, -0.5) * 2.0 ** (np.floor(np.log2(even)) - 7)
+    share = torch.zeros(64, dtype=torch.float64)
+    for side in (0, 1):
+        for half in (0, 32):
+            share[half + np.flatnonzero(lane_of == side)] = torch.tensor(kept)
+    total = share.sum() + 2 + float((63 + 1) * 2.0 ** -float(f32(f32(61) * c2)))                   # (and the other keys, with scores of zero)
+    assert int((got[0][0, 1, :64].cpu() == (share / total).to(torch.bfloat16)).sum()) >= 60
 
 
 @pytest.mark.parametrize("hq,hkv,d,page,window,split_keys", [(4, 2, 128, 16, None, 0), (4, 2, 128, 16, None, 64), (6, 2, 64, 32, 20, 0),
