@@ -557,7 +557,8 @@ static int run_experts_wide(int shape, const GroupedArgs& g, hipStream_t stream)
 #endif
 
 // ---------------------------------------------------------------------------------------------------------
-#define MAX_EXPERTS 256
+#define MAX_EXPERTS 256         // 64 lanes x EXPERT_REGS
+#define EXPERT_REGS 4
 
 struct Routing {
     int experts, top, group_count, group_keep, renorm, softmax, group_best;
@@ -670,6 +671,129 @@ __global__ __launch_bounds__(64 * WAVES) void router_topk_kernel(const float* __
     }
     ids[(size_t)blockIdx.x * r.top + e] = which;
     weights[(size_t)blockIdx.x * r.top + e] = r.renorm || r.out_scale != 1.0f ? w * r.out_scale : w;
+}
+
+// The same, one choice after the other, a wavefront a token: a round is six exchanges between the lanes' best.
+// The largest value among the lanes' candidates and, among equals, the lowest index; every lane gets both.
+__device__ __forceinline__ void wave_best(float& value, int& index) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const float ov = __shfl_xor(value, off, MLR_WAVE);
+        const int oi = __shfl_xor(index, off, MLR_WAVE);
+        if (ov > value || (ov == value && oi < index)) {
+            value = ov;
+            index = oi;
+        }
+    }
+}
+
+__global__ __launch_bounds__(64) void router_rounds_kernel(const float* __restrict__ z, long ld, Routing r,
+                                                           int32_t* __restrict__ ids, float* __restrict__ weights) {
+    __shared__ float s_lds[MAX_EXPERTS];      // what the choice goes by
+    __shared__ float w_lds[MAX_EXPERTS];      // the plain scores
+    __shared__ float g_lds[MAX_EXPERTS];
+    const int m = blockIdx.x, lane = threadIdx.x, experts = r.experts, top = r.top, group_count = r.group_count;
+    const float* zr = z + (size_t)m * ld;
+    float z_max = 0.f, z_sum = 1.f;
+    if (r.softmax) {
+        z_max = -INFINITY;
+        for (int e = lane; e < experts; e += 64) z_max = fmaxf(z_max, zr[e]);
+        z_max = wave_max(z_max);
+        z_sum = 0.f;
+        for (int e = lane; e < experts; e += 64) z_sum += expf(zr[e] - z_max);
+        z_sum = wave_sum(z_sum);
+    }
+    for (int e = lane; e < experts; e += 64) {
+        const float sc = r.softmax ? expf(zr[e] - z_max) / z_sum : 1.0f / (1.0f + expf(-zr[e]));
+        w_lds[e] = sc;
+        s_lds[e] = r.correction != nullptr ? sc + r.correction[e] : sc;
+    }
+    __syncthreads();
+    const int per = experts / group_count;
+    for (int gidx = lane; gidx < group_count; gidx += 64) {
+        float first = -INFINITY, second = -INFINITY;
+        for (int i = 0; i < per; ++i) {
+            const float v = s_lds[gidx * per + i];
+            if (v > first) {
+                second = first;
+                first = v;
+            } else if (v > second) {
+                second = v;
+            }
+        }
+        g_lds[gidx] = per >= 2 && !r.group_best ? first + second : first;
+    }
+    __syncthreads();
+    // the groups that stand: r.group_keep times the best of those left; their experts become candidates
+    float cand[EXPERT_REGS];
+#pragma unroll
+    for (int i = 0; i < EXPERT_REGS; ++i) cand[i] = -INFINITY;
+    for (int round = 0; round < r.group_keep; ++round) {
+        float best = -INFINITY;
+        int which = 0x7fffffff;
+        for (int gidx = lane; gidx < group_count; gidx += 64) {
+            const float v = g_lds[gidx];
+            if (v > best) {                    // (ascending indices: the lowest among equals stays)
+                best = v;
+                which = gidx;
+            }
+        }
+        wave_best(best, which);
+        if (which == 0x7fffffff) break;
+        __syncthreads();
+        if (lane == 0) g_lds[which] = -INFINITY;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < EXPERT_REGS; ++i) {
+            const int e = lane + 64 * i;
+            if (e < experts && e / per == which) cand[i] = s_lds[e];
+        }
+    }
+    float chosen_sum = 0.f;
+    for (int round = 0; round < top; ++round) {
+        float best = -INFINITY;
+        int which = 0x7fffffff;
+#pragma unroll
+        for (int i = 0; i < EXPERT_REGS; ++i) {
+            const int e = lane + 64 * i;
+            if (e < experts && cand[i] > best) {
+                best = cand[i];
+                which = e;
+            }
+        }
+        wave_best(best, which);
+        if (which == 0x7fffffff) which = 0, best = 0.f;      // (fewer candidates than `top`: refused on the host)
+#pragma unroll
+        for (int i = 0; i < EXPERT_REGS; ++i)
+            if (lane + 64 * i == which) cand[i] = -INFINITY;
+        chosen_sum += w_lds[which];                           // (the same on every lane, in the order of the choices)
+        if (lane == 0) {
+            ids[(size_t)m * top + round] = which;
+            weights[(size_t)m * top + round] = w_lds[which];
+        }
+    }
+    if (r.renorm || r.out_scale != 1.0f) {
+        __syncthreads();
+        for (int c = lane; c < top; c += 64) {
+            float w = weights[(size_t)m * top + c];
+            if (r.renorm) w = w / (chosen_sum + 1e-20f);
+            weights[(size_t)m * top + c] = w * r.out_scale;
+        }
+    }
+}
+
+// Which of the two a step takes, by their predicted times (us).  Counting is a comparison of every expert with every other in four
+// wavefronts, so it is bound by that work once the tokens are many; the rounds' time is their number, and one lane's walk over the
+// scores of a group.  Up to 64 experts counting is the faster one always (0.23 to 0.97 of the rounds' time).  Measured, rounds and
+// counting: 8 of 256 in 4 of 8 groups 13.0 and 9.3 for one token, 15.6 and 21.9 for 2048; 6 of 160 16.7 and 5.7, 2048 tokens 21.3 and
+// 13.5, 4096 20.9 and 23.0; 1 of 256 in 1 of 8 groups 6.3 and 9.2.  (By this line 72 to 256 experts, 1 to 4096 tokens, 1 to 12 chosen
+// took 0.27 to 1.01 of the rounds' time.)
+static bool choose_in_rounds(const Routing& r, int rows) {
+    if (r.experts <= 64) return false;
+    const float per = (float)(r.experts / r.group_count), m = (float)rows, e = (float)r.experts;
+    const float rounds = 2.6f + 0.06f * per + 0.67f * (float)(r.group_keep + r.top) + 0.0007f * m;
+    const float counting = 2.4f + 0.018f * e + (r.group_count > 1 ? 0.5f + 0.055f * per : 0.f) + m * (0.0008f + 2.26e-5f * e);
+    return rounds < counting;
 }
 
 // Where the experts' rows of the sorted list start: start[e] the sum of count[0 .. e - 1], offsets[experts] of all; one wavefront
@@ -826,7 +950,8 @@ int mlr_router_topk(const float* z, long ld, int32_t* ids, float* weights, int r
         group_keep > group_count || top < 1 || top > group_keep * (experts / group_count))
         return -1;
     const Routing r{experts, top, group_count, group_keep, renorm, softmax, group_best, correction, out_scale};
-    if (experts <= 64) router_topk_kernel<1><<<rows, 64, 0, stream>>>(z, ld, r, ids, weights);
+    if (choose_in_rounds(r, rows)) router_rounds_kernel<<<rows, 64, 0, stream>>>(z, ld, r, ids, weights);
+    else if (experts <= 64) router_topk_kernel<1><<<rows, 64, 0, stream>>>(z, ld, r, ids, weights);
     else router_topk_kernel<4><<<rows, 256, 0, stream>>>(z, ld, r, ids, weights);
     return (int)hipGetLastError();
 }

@@ -43,9 +43,10 @@ def chosen_in_rounds(scores, top, count, keep, best_alone):
 
 @pytest.mark.parametrize("best_alone", [False, True])
 @pytest.mark.parametrize("rows,experts,top,count,keep", [(1, 1, 1, 1, 1), (1, 64, 64, 1, 1), (16, 20, 4, 1, 1), (17, 21, 4, 7, 2), (64, 64, 8, 8, 3), (64, 60, 5, 60, 9),
-                                                         (65, 16, 4, 4, 4), (33, 65, 6, 5, 2), (40, 256, 8, 8, 4), (130, 128, 3, 1, 1)])
+                                                         (65, 16, 4, 4, 4), (33, 65, 6, 5, 2), (40, 256, 8, 8, 4), (130, 128, 3, 1, 1),
+                                                         (40, 160, 2, 8, 1), (5, 256, 1, 8, 1), (33, 128, 2, 128, 2), (900, 256, 3, 8, 2), (17, 65, 13, 5, 1)])
 def test_a_place_in_the_order_is_the_choice_round_after_round(rows, experts, top, count, keep, best_alone):
-    """Scores that tie in plenty, rows of infinities and NaN among them, with and without a correction."""
+    """Scores that tie in plenty, rows of infinities and NaN among them, with and without a correction; sizes of either kernel."""
     from mini_llm_runtime_amd.kernels import Kernels
     k = Kernels(torch.float32)
     rng = np.random.default_rng(rows * 1000 + experts)
