@@ -205,13 +205,13 @@ class StepContext:
         self._groups[key] = hit
         return hit
 
-    def attention_split(self, rows, batch_rows, kv_heads, q_heads, head_dim, longest=None):
+    def attention_split(self, rows, batch_rows, kv_heads, q_heads, head_dim, longest=None, narrow=True):
         """(split_keys, max_splits, partial buffer).  A batch of many tokens fills the GPU with one
         workgroup per (token group, kv head); a small batch over long contexts does not, so there the
         keys of a token are split over several workgroups, in ranges [s * split_keys, (s + 1) *
         split_keys) of absolute key positions, and merged in ascending order.  split_keys is the
         largest of base, 2 base, 4 base, ... that still gives `target_workgroups`, or where base is too wide for that narrower
-        (`narrowed`; not in a model that routes, whose choices turn on the last bit); what a token's
+        (`narrowed`; not in a model that routes, whose choices turn on the last bit, nor where `narrow` says no); what a token's
         result is does not depend on the choice beyond rounding.  `rows` tokens take part; the partial
         results are indexed by batch row, of which there are `batch_rows`.  `longest`: the most keys a
         workgroup of the kernel can walk without a split; a longer context is split whatever the batch."""
@@ -219,7 +219,7 @@ class StepContext:
         if rows > self.split_max_tokens and not forced:
             return 0, 1, None
         return self._split(max(1, rows * kv_heads), self.target_workgroups, batch_rows, q_heads, head_dim, longest, LONG_RANGE,
-                           narrow=not self.routed)
+                           narrow=narrow and not self.routed)
 
     def group_split(self, groups, batch_rows, kv_heads, q_heads, head_dim, longest=None):
         """As `attention_split` for `groups` groups of many tokens each (prompt portions), which give

@@ -283,8 +283,12 @@ class GqaAttention:
             if small[2]:
                 # (partial results are indexed by batch row: they reach as far as the last row of a small group,
                 # which in the scheduler's batches -- single tokens first -- is the number of single tokens)
+                # Ranges narrower than the setting are for chains of tiles; a portion of several tokens is several groups and rows
+                # to merge already (a step by layer of the 0.6B sizes with ranges of 256 and of 64 keys: 5 tokens behind 300 56.7 and 61.3
+                # us, with 256 and 128 4 behind 600 56.5 and 58.8, but two tokens behind 1300 54.3 and 51.4)
                 split_keys, max_splits, partial = ctx.attention_split(
-                    small_rows, small_end, s.kv_heads, s.q_heads, s.head_dim, longest=k.mfma_longest_context(view.page_size))
+                    small_rows, small_end, s.kv_heads, s.q_heads, s.head_dim, longest=k.mfma_longest_context(view.page_size),
+                    narrow=small_rows <= 2)
                 self._hint(k)
                 k.attention_mfma(q, view.k_pages, view.v_pages, view.block_table, ctx.slots, ctx.positions, attn,
                                  small[0], small[1], small[2], s.q_heads, s.kv_heads, s.head_dim, view.page_size,

@@ -251,6 +251,25 @@ def test_few_workgroups_take_narrower_key_ranges(rows, max_context, keys, wide, 
     assert split(320) == split(320, routed=True) == ranges(of_320)
 
 
+@pytest.mark.parametrize("lengths,keys", [([1], 64), ([2], 64), ([1, 1], 64), ([3], 256), ([2, 1], 256), ([5], 256), ([1] * 6, 256), ([400, 2], 64), ([400, 3], 256)])
+def test_short_portions_keep_the_settings_key_ranges(lengths, keys):
+    """What single tokens alone gain by (they have a kernel of their own) costs portions of several tokens."""
+    part, ctx = attention_part(), context(512)
+    ctx.workspace.reserve({("token_groups_8_4", torch.int32): 4000})
+    ctx._group_upload, ctx.n_tokens, ctx.routed, ctx.compute_units = HostUpload(), sum(lengths), False, 256
+    ctx.segments = [(i, sum(lengths[:i]), n, 0) for i, n in enumerate(lengths)]
+    ctx.slots = ctx.positions = torch.zeros(sum(lengths), dtype=torch.int32)
+    taken = []
+    ctx.kernels.profiler = None
+    ctx.kernels.attention_mfma = lambda *a, **kw: taken.append((kw["split_keys"], kw["max_splits"]))
+    ctx.kernels.attention_tiles = lambda *a, **kw: None
+    part._work = None
+    pages = torch.empty((70, 8, 16, 128), dtype=torch.bfloat16)
+    view = type("View", (), dict(k_pages=pages, v_pages=pages, block_table=None, page_size=16))
+    part._attend_cached(ctx, torch.empty((sum(lengths), 16 * 128), dtype=torch.bfloat16), view)
+    assert taken == [(keys, 512 // keys)]
+
+
 @pytest.mark.parametrize("units,max_context,short,routed,keys", [
     (32, 2048, True, False, 128), (32, 2724, True, False, 256), (16, 2724, True, False, 128), (4, 2048, True, False, 64), (4, 4096, True, False, 128),
     (4, 4097, True, False, 256), (32, 2048, False, False, 256), (32, 2048, True, True, 256), (64, 512, True, False, 64), (128, 512, True, False, 128),
