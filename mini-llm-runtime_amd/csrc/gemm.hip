@@ -1761,13 +1761,13 @@ static int qkv_shape_for(int M, int N, int K, float* time) {
     return best;
 }
 
-// Whether `mlr_gemm_qkv` is the way for these sizes: where the product is this kernel's anyway, and the tile of whole heads with its
+// Whether `mlr_gemm_qkv` is the way for a product of these sizes that is this kernel's anyway: the tile of whole heads with its
 // epilogue takes no longer than the best tile and the other launch, 3 us and 0.6 a million outputs.  Measured (product + launch, one
 // launch): 2048 x 4096 x 1024 28.0, 22.2 us; 1024 x 4096 x 1024 19.7, 13.4; 333 x 6144 x 4096 38.9, 36.2; 700 x 6144 x 4096 50.4, 45.8;
 // 333 x 10240 x 5120 56.8, 52.5.  Not where narrower tiles win by more: 256 x 6144 x 4096 32.8, 39.7; 160 x 4096 x 1024 11, 11.
-extern "C" int mlr_gemm_qkv_wins(int M, int q_heads, int kv_heads, int K, int one_order) {
+extern "C" int mlr_gemm_qkv_wins(int M, int q_heads, int kv_heads, int K) {
     const int N = (q_heads + 2 * kv_heads) * QKV_HEAD;
-    if (M <= 64 || !mlr_gemm_wide_wins(M, N, K, WIDE_PLAIN, one_order)) return 0;
+    if (M <= 64 || q_heads <= 0 || kv_heads <= 0 || K <= 0 || !wide_takes(nullptr, nullptr, M, N, K, false)) return 0;
     float time = 0.f, any = 0.f;
     qkv_shape_for(M, N, K, &time);
     wide_shape_for(M, N, K, false, &any);

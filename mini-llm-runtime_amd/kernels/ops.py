@@ -484,8 +484,7 @@ class Kernels:
         key = (rows, q_heads, kv_heads, k, "qkv")
         wins = self._wide_choices.get(key)
         if wins is None:
-            wins = bool(self._lib("gemm").mlr_gemm_qkv_wins(_c_int(rows), _c_int(q_heads), _c_int(kv_heads), _c_int(k),
-                                                            _c_int(1 if self.routed else 0))) or not self.library_gemm
+            wins = bool(self._lib("gemm").mlr_gemm_qkv_wins(_c_int(rows), _c_int(q_heads), _c_int(kv_heads), _c_int(k)))
             self._wide_choices[key] = wins
         return wins
 

@@ -361,6 +361,16 @@ def test_whether_a_model_routes_is_said_where_its_kernels_are_made(monkeypatch):
     assert Kernels(torch.bfloat16, routed=True).routed and not Kernels(torch.bfloat16).routed
 
 
+@pytest.mark.parametrize("library", [True, False])
+def test_heads_in_the_products_epilogue_only_where_their_tile_is_worth_it(library):
+    """Narrow products leave most of the chip idle in tiles of whole heads: they keep the best tile and the launch behind it, whether the
+    vendor library stands beside the kernel or not."""
+    k = kernels_without_gpu()
+    k.library_gemm, k._wide_choices = library, {}
+    assert all(k.qkv_product(m, q, kv, 128, inner, 16) for m, q, kv, inner in ((2048, 16, 8, 1024), (1024, 16, 8, 1024), (333, 32, 8, 4096)))
+    assert not any(k.qkv_product(m, q, kv, 128, inner, 16) for m, q, kv, inner in ((83, 7, 1, 5120), (256, 32, 8, 4096), (99, 16, 2, 5120), (128, 24, 8, 2560)))
+
+
 @pytest.mark.parametrize("rows,n,k,experts,shape", [
     (160, 4096, 448, 8, 4), (160, 4096, 384, 8, -1), (161, 4096, 448, 8, 5), (447, 4096, 384, 8, -1), (320, 2048, 448, 16, 4), (320, 2112, 448, 16, -1),
     (320, 2112, 640, 16, -1), (320, 2112, 704, 16, 4), (640, 4096, 640, 32, -1), (640, 4096, 64, 33, 4), (8, 128, 64, 256, 4), (448, 2048, 64, 8, 5),
