@@ -426,14 +426,23 @@ class Runner:
             n, total, r, single = totals.tolist()
             return _Batch(total, ids[:total], counts[:n], slots[:n], rows[:r], bool(single), first[:n], self._plain_at)
         total, arrays, wanted = self._validate(entries)
-        counts = np.array([len(a) for a in arrays], dtype=np.int32)
-        base = np.cumsum(counts) - counts
-        ids = np.concatenate([np.asarray(a, dtype=np.int32) for a in arrays])
-        slots = np.array([e.slot for e in entries], dtype=np.int32)
-        rows = np.concatenate([b + np.asarray(w, dtype=np.int64) for b, w in zip(base, wanted)]).astype(np.int32)
-        first = np.empty(len(entries), dtype=np.int32)
-        return _Batch(total, ids, counts, slots, rows, False, first,
-                      tuple(ctypes.c_void_p(v.ctypes.data) for v in (ids, counts, slots, first)))
+        n = len(entries)
+        slots[:n] = np.array([e.slot for e in entries], dtype=np.int32)
+        counts[:n] = lengths = [len(a) for a in arrays]
+        # (mostly single tokens, a decoding step: short lists cost less than a vector for every entry)
+        ids[:total] = [t for a in arrays for t in a] if total <= 4 * n else np.concatenate(arrays)
+        if all(type(w) is list for w in wanted):
+            places, at = [], 0
+            for length, want in zip(lengths, wanted):
+                places.extend([at + w for w in want])
+                at += length
+        else:
+            base = np.cumsum(lengths) - lengths
+            places = np.concatenate([b + np.asarray(w, dtype=np.int64) for b, w in zip(base, wanted)])
+        r = len(places)
+        rows[:r] = places
+        single = total == n == r and all(len(w) == 1 for w in wanted)
+        return _Batch(total, ids[:total], counts[:n], slots[:n], rows[:r], single, first[:n], self._plain_at)
 
     def _validate(self, entries):
         if not entries:

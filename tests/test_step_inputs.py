@@ -76,11 +76,13 @@ def test_odd_forms_of_tokens_become_the_same_batch(tokens):
     r._plain, r._plain_at, r._inputs = [ids, counts, slots, places, np.empty(TOKENS, np.int32), rows, totals], None, build.load("step_inputs")
     r._plain_args = (ctypes.c_long(VOCAB), TOKENS, ROWS, *(ctypes.c_void_p(v.ctypes.data) for v in (ids, counts, slots, places, rows, totals)))
     numbers = [int(t) for t in tokens]
-    for first in ([Entry(1, [3, 4], [1])], []):
-        want = r._gather([*first, Entry(2, numbers, [0])])
-        want = [v.tolist() for v in (want.ids, want.counts, want.slots, want.want_rows)]
-        got = r._gather([*first, Entry(2, tokens, [0])])
-        assert [v.tolist() for v in (got.ids, got.counts, got.slots, got.want_rows)] == want and got.ids.dtype == np.int32
+    def made(batch):
+        assert len(batch.first) == len(batch.slots) and batch.ids.dtype == np.int32
+        return [v.tolist() for v in (batch.ids, batch.counts, batch.slots, batch.want_rows)] + [batch.total, batch.single]
+    for first in ([Entry(1, [3, 4], [1])], [], [Entry(3, [8], [0])]):
+        want = made(r._gather([*first, Entry(2, numbers, [0])]))
+        assert made(r._gather([*first, Entry(2, tokens, [0])])) == want
+        assert made(r._gather([*first, Entry(np.int64(2), numbers, np.array([0]))])) == want
 
 
 def test_without_the_interpreters_headers_every_batch_is_read_entry_by_entry(tmp_path, monkeypatch):
