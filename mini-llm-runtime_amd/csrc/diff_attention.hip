@@ -744,7 +744,7 @@ int mlr_diff_attention(const void* q, long q_stride, const void* k_pages, const 
 }
 
 // For tests: the page of a key as the matrix-core kernels work it out (pages.h).
-int mlr_page_of_key(int page_size, int key) { return page_of_key(page_divisor(page_size), key); }
+int mlr_page_of_key(int page_size, int key) { return page_size > 1 ? page_of_key(page_divisor(page_size), key) : key; }
 
 // Groups of consecutive tokens of one request on the matrix cores (bfloat16): prompt portions in groups of up to
 // 16 * (4 / min(4, q_heads / kv_heads)) tokens, single tokens and short portions in smaller ones.  `group_tokens`:

@@ -620,7 +620,7 @@ __global__ __launch_bounds__(256) void sink_attention_tiles_kernel(SinkArgs a, c
         const int kp = t0 + my_key;
         const bool lead = t0 < lead_end;
         const bool inside = (kp >= kbegin || kp < a.keep_first) && kp < (lead ? lead_end : main_end);
-        const int kb = page_of_key(a.pages, kp);
+        const int kb = a.page_size > 1 ? page_of_key(a.pages, kp) : kp;
         const int rel = inside ? kb - (lead ? lead0 : block0) : -1, blk = lead ? rel : n_lead + rel;
         const int listed = page_lds[min(max(blk, 0), max(n_blocks - 1, 0))];
         const int page = (rel >= 0 && blk < n_blocks) ? listed : -1;
