@@ -562,30 +562,227 @@ struct KvTile {
 
 #define DECODE_PAGE_CACHE 4096
 
-// Decoding (every group is one new token of a request) without a kernel of its own for the per-head norm,
-// the rotation and the cache write: the attention kernel takes the raw projection, norms and rotates its
-// queries itself and walks the keys that are cached already (positions below the token's own); the merge
-// kernel, which follows anyway, norms and rotates the token's own key, adds the token's own score and
-// value as one more summand, and writes key and value into their pages for the steps to come.
+// Decoding (every group is one new token of a request) in one launch: the attention kernel takes the raw projection, norms and
+// rotates its queries itself and walks the keys that are cached already (positions below the token's own); whoever merges the
+// key ranges norms and rotates the token's own key, adds the token's own score and value as one more summand, and writes key and
+// value into their pages for the steps to come (`DecodeMerge`).  The last workgroup of a (token, kv head) to be done merges: each
+// leaves its sums with write-through stores, waits until they have arrived, and adds one to the counter of its token and kv head;
+// the one that finds the others counted reads all of them past the caches.  Nobody waits for anybody, and the order of the sums
+// is that of the ranges, whoever merges.  (No fence: a release at device scope writes the XCD's L2 back.)
 // Needs head_dim % 64 == 0 (a lane of the attention kernel then holds both channels of a rotation pair).
 struct DecodeFusion {
     const __bf16* qkv;          // [M, ld]: q heads, k heads, v heads of every row
     const float* q_norm_w;      // [head_dim] or null
     const float* k_norm_w;
     const float* rope;          // [positions, head_dim]: cosines | sines, or null
+    int32_t* arrivals;          // [M, kv_heads] workgroups that have left their sums; zero before and after a launch
     int ld;
     float eps;
+    int workgroups;             // 0: key ranges at absolute multiples of split_keys, else see `even_ranges`
 };
 
-template <int NCH, bool FUSED>   // NCH: ceil(head_dim / 32)
+// Key ranges of one token of `units` (tokens times kv heads) behind `walk` keys: its share of `workgroups`, or of twice, three times
+// as many where a range would be wide (`wide` keys to a share of the first); none of less than 64 keys, and none of less than 256
+// beyond sixteen.  A token's own keys decide, not the longest context that the step (or its graph) was laid out for: evenly wide
+// ranges keep the compute units evenly busy, and one workgroup a unit, or two, is what they take best -- a few more than that cost
+// the step a second round (`StepContext.even_split` has the figures).
+__host__ __device__ inline int even_ranges(int walk, int workgroups, int units, int wide) {
+    const int rounds = (walk + wide - 1) / wide, n = (int)((long long)workgroups * rounds / units);
+    const int least = walk / 256 > 16 ? walk / 256 : 16, pieces = (walk + 63) / 64;
+    const int most = least < pieces ? least : pieces;
+    return n < 1 ? 1 : n < most ? n : most;
+}
+
+// What workgroups of other compute units leave and read during a launch: stores that go through to memory, loads that do not stop
+// at a cache of the reader's.
+__device__ __forceinline__ void store_through(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ float load_through(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ void wavefront_sync() {               // LDS accesses of a wavefront's own, in order
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+
+// The merge for `DecodeFusion`, by one wavefront for one (token, head): the splits' partial results, the token's own key and value
+// besides; the first head of every kv head writes those into the cache.  A lane takes the rotation pairs lane and lane + 64 and
+// the ND channels lane + 64 i.  Loads are asked for as early as their addresses are known: `ask` the raw q, k, v, norm weights,
+// rotation row and page, `own` makes the token's own score of them, both before it is known who merges.
+// Bound by three trips past the caches, one after the other (sums out, the count, sums in): 4.2 us behind the attention of one
+// token of 16 heads in nine ranges, where a launch of its own took 5.3 (both together 12.8 us for 13.9; 8 tokens behind 3600 keys
+// 31.3 for 32.2).  Where one workgroup has all of a token's keys its sums stay in LDS (64 tokens of 32 heads 75 us for 77).
+template <int ND>
+struct DecodeMerge {
+    static constexpr int D = 64 * ND, HALF = 32 * ND, NP = (ND + 1) / 2;        // a lane's rotation pairs
+    float qa[NP], qb[NP], ka[NP], kb[NP], qwa[NP], qwb[NP], kwa[NP], kwb[NP], vv[ND], co[NP], si[NP];
+    __bf16 k_lo[NP], k_hi[NP];
+    float s_own, den, num[ND], gmax;
+    int page;
+
+    __device__ __forceinline__ void ask(const AttnArgs& a, const DecodeFusion& f, int m, int head, int kvh, int pos, int slot, int lane) {
+        const int P = a.page_size;
+        const __bf16* row = f.qkv + (size_t)m * f.ld;
+        const __bf16* qs = row + (size_t)head * D;
+        const __bf16* ks = row + (size_t)(a.q_heads + kvh) * D;
+        const __bf16* vs = row + (size_t)(a.q_heads + a.kv_heads + kvh) * D;
+        const bool normed = f.q_norm_w != nullptr, rotated = f.rope != nullptr;
+        const float* qw = normed ? f.q_norm_w : reinterpret_cast<const float*>(row);      // (any readable address)
+        const float* kw = normed ? f.k_norm_w : reinterpret_cast<const float*>(row);
+        const float* cs = (rotated ? f.rope : reinterpret_cast<const float*>(a.positions)) + (rotated ? (size_t)pos * D : 0);
+        const int page_read = a.block_table[(size_t)slot * a.max_blocks + min(pos / P, a.max_blocks - 1)];
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            const int j = min(lane + 64 * i, HALF - 1), jr = rotated ? j : 0;
+            qa[i] = (float)qs[j];
+            qb[i] = (float)qs[j + HALF];
+            ka[i] = (float)ks[j];
+            kb[i] = (float)ks[j + HALF];
+            qwa[i] = qw[j];
+            qwb[i] = qw[j + HALF];
+            kwa[i] = kw[j];
+            kwb[i] = kw[j + HALF];
+            co[i] = cs[jr];
+            si[i] = cs[rotated ? jr + HALF : 0];
+        }
+#pragma unroll
+        for (int i = 0; i < ND; ++i) vv[i] = (float)vs[lane + 64 * i];
+        page = pos / P < a.max_blocks ? page_read : -1;          // (beyond the request's row of the table: no page)
+    }
+
+    // query and key of this token: norm, rotation, rounded to bfloat16 (what the cache holds), and their product
+    __device__ __forceinline__ void own(const AttnArgs& a, const DecodeFusion& f, int lane) {
+        float qsum = 0.f, ksum = 0.f;
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            if (lane + 64 * i >= HALF) qa[i] = qb[i] = ka[i] = kb[i] = 0.f;
+            qsum += squares(qa[i], qb[i]);
+            ksum += squares(ka[i], kb[i]);
+        }
+        if (f.q_norm_w != nullptr) {
+            qsum = wave_sum(qsum);
+            ksum = wave_sum(ksum);
+            const float qscale = 1.0f / sqrtf(qsum / (float)D + f.eps), kscale = 1.0f / sqrtf(ksum / (float)D + f.eps);
+#pragma unroll
+            for (int i = 0; i < NP; ++i) {
+                qa[i] = (qa[i] * qscale) * qwa[i];
+                qb[i] = (qb[i] * qscale) * qwb[i];
+                ka[i] = (ka[i] * kscale) * kwa[i];
+                kb[i] = (kb[i] * kscale) * kwb[i];
+            }
+        }
+        float dot = 0.f;
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            float qx = qa[i], qy = qb[i], kx = ka[i], ky = kb[i];
+            if (f.rope != nullptr) {
+                qx = turn_x(qa[i], qb[i], co[i], si[i]);
+                qy = turn_y(qa[i], qb[i], co[i], si[i]);
+                kx = turn_x(ka[i], kb[i], co[i], si[i]);
+                ky = turn_y(ka[i], kb[i], co[i], si[i]);
+            }
+            k_lo[i] = (__bf16)kx;
+            k_hi[i] = (__bf16)ky;
+            if (lane + 64 * i < HALF)
+                dot += (float)(__bf16)qx * (float)k_lo[i] + (float)(__bf16)qy * (float)k_hi[i];
+        }
+        s_own = wave_sum(dot) * (a.scale * 1.44269504088896340736f);       // base-2 domain, as the partial maxima
+    }
+
+    // The sums of n partial results from `base` on (sums [D], maximum, sum of probabilities each), in ascending order; maxima are
+    // base-2 exponents.  weights: COMBINE_MAX_SPLITS floats of LDS.
+    __device__ __forceinline__ void gather(const float* base, int n, float* weights, int lane) {
+        constexpr int AHEAD = 16;
+        const float* mine = base + (size_t)min(lane, n - 1) * (D + 2) + D;
+        const float smax = load_through(mine), ssum = load_through(mine + 1);
+        gmax = s_own;
+        den = 0.f;
+#pragma unroll
+        for (int i = 0; i < ND; ++i) num[i] = 0.f;
+#pragma unroll 1
+        for (int s0 = 0; s0 < n; s0 += AHEAD) {
+            float part[AHEAD][ND];
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u)                       // (clamped: no branch around a load)
+#pragma unroll
+                for (int i = 0; i < ND; ++i) part[u][i] = load_through(base + (size_t)min(s0 + u, n - 1) * (D + 2) + lane + 64 * i);
+            if (s0 == 0) {                                        // the splits' weights and the denominator
+                float top = lane < n ? smax : -INFINITY;
+#pragma unroll 1
+                for (int s = lane + 64; s < n; s += 64) top = fmaxf(top, load_through(base + (size_t)s * (D + 2) + D));
+                gmax = fmaxf(wave_max(top), gmax);
+                const float w = smax > -INFINITY ? __builtin_amdgcn_exp2f(smax - gmax) : 0.f;
+                if (lane < n) {
+                    weights[lane] = w;
+                    den = w * ssum;
+                }
+#pragma unroll 1
+                for (int s = lane + 64; s < n; s += 64) {
+                    const float* p = base + (size_t)s * (D + 2) + D;
+                    const float m = load_through(p), x = m > -INFINITY ? __builtin_amdgcn_exp2f(m - gmax) : 0.f;
+                    weights[s] = x;
+                    den += x * load_through(p + 1);
+                }
+                wavefront_sync();
+            }
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) {
+                if (s0 + u >= n) break;
+                const float w = weights[s0 + u];
+#pragma unroll
+                for (int i = 0; i < ND; ++i) num[i] += w * part[u][i];
+            }
+        }
+        den = wave_sum(den);
+    }
+
+    // The same of the one result of a token whose keys one workgroup had, in LDS.
+    __device__ __forceinline__ void gather_own(const float* whole, int lane) {
+        gmax = fmaxf(whole[D], s_own);
+        const float w = whole[D] > -INFINITY ? __builtin_amdgcn_exp2f(whole[D] - gmax) : 0.f;
+        den = w * whole[D + 1];
+#pragma unroll
+        for (int i = 0; i < ND; ++i) num[i] = w * whole[lane + 64 * i];
+    }
+
+    // The token's own summand, the head's output and, once per kv head, key and value into their pages.
+    __device__ __forceinline__ void finish(const AttnArgs& a, int m, int head, int kvh, bool writes, int pos, int lane) {
+        const float w_own = __builtin_amdgcn_exp2f(s_own - gmax);
+        den += w_own;
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+            a.out[((size_t)m * a.q_heads + head) * D + lane + 64 * i] = from_float<elem_t>((num[i] + w_own * vv[i]) / den);
+        if (!writes || page < 0) return;
+        const int P = a.page_size;
+        const size_t pk = (size_t)page * a.kv_heads + kvh;
+        __bf16* kdst = reinterpret_cast<__bf16*>(const_cast<elem_t*>(a.k_pages)) + (pk * P + pos % P) * D;
+        __bf16* vdst = reinterpret_cast<__bf16*>(const_cast<elem_t*>(a.v_pages)) + pk * D * P + pos % P;
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            const int j = lane + 64 * i;
+            if (j < HALF) {
+                kdst[j] = k_lo[i];
+                kdst[j + HALF] = k_hi[i];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < ND; ++i) vdst[(size_t)(lane + 64 * i) * P] = (__bf16)vv[i];
+    }
+};
+
+// NCH: ceil(head_dim / 32); PAGE: keys of a page, 0 for any multiple of 16.  A decoding step waits for the address of its first keys,
+// and a short workgroup's time is instructions: with the head size and the usual page known, page ids of a wavefront in scalar
+// registers and a merge of a third less code a step of the 0.6B sizes behind 1100 keys takes 1046 us for 1120, 8 tokens behind 3600
+// 1623 for 1715.
+template <int NCH, bool FUSED, int PAGE = 0>
 __global__ __launch_bounds__(256, (NCH <= 4 ? 2 : 1)) void attention_mfma_kernel(AttnArgs a, const int32_t* __restrict__ group_row0,
                                                              const int32_t* __restrict__ group_ntok, DecodeFusion f) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     __shared__ int32_t page_lds[DECODE_PAGE_CACHE];    // the request's page ids for this workgroup's key range
-    const int D = a.head_dim, P = a.page_size;
+    __shared__ int32_t arrived;                        // FUSED: workgroups of this token and kv head that were done before this one
+    const int D = FUSED ? 32 * NCH : a.head_dim, P = PAGE > 0 ? PAGE : a.page_size;
     const int g = a.q_heads / a.kv_heads;
     const int grp = blockIdx.x, kvh = blockIdx.y, split = blockIdx.z;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15, b = lane >> 4;
     // (FUSED: group i is the one token in batch row i; no need to wait for the group vectors)
     const int row0 = FUSED ? grp : group_row0[grp], ntok = FUSED ? 1 : group_ntok[grp];
@@ -597,11 +794,23 @@ __global__ __launch_bounds__(256, (NCH <= 4 ? 2 : 1)) void attention_mfma_kernel
     const int kend_c = FUSED ? max(kend_full - 1, 0) : kend_full;     // FUSED: the token's own key is not cached yet
     const int glo = a.window > 0 ? max(0, pos0 + 1 - a.window) : 0;   // the group's key range [glo, ke)
     const int ke = pos0 + ntok - (FUSED ? 1 : 0);                      // keys below ke are written
-    int lo = glo, hi = ke;
-    if (a.max_splits > 1) {
-        const int first_split = glo / a.split_keys;
-        const int last_split = min(a.max_splits - 1, max(ke - 1, 0) / a.split_keys);
-        if (split < first_split || split > last_split) return;          // no keys here: the whole workgroup leaves
+    int lo = glo, hi = ke, first_split = 0, splits = 1;                // the key ranges that hold keys
+    if (FUSED && f.workgroups > 0) {
+        const int from = glo / MFMA_TILE_KEYS * MFMA_TILE_KEYS, walk = max(ke - from, 1), pieces = (walk + 63) / 64;
+        const int n = min(a.max_splits, even_ranges(walk, f.workgroups, gridDim.x * gridDim.y, a.split_keys));
+        const int width = (pieces + n - 1) / n * 64;                    // whole 64 keys, from the tile of the first one on
+        splits = (walk + width - 1) / width;
+        if (split >= splits) return;
+        lo = max(lo, from + split * width);
+        hi = min(hi, from + (split + 1) * width);
+    } else if (a.max_splits > 1) {
+        first_split = glo / a.split_keys;
+        splits = min(a.max_splits - 1, max(ke - 1, 0) / a.split_keys) + 1 - first_split;
+        if (FUSED) {                                                     // (a window of the token's own key: one workgroup all the same)
+            first_split = min(first_split, a.max_splits - 1);
+            splits = max(splits, 1);
+        }
+        if (split < first_split || split >= first_split + splits) return;          // no keys here: the whole workgroup leaves
         lo = max(lo, split * a.split_keys);
         hi = min(hi, (split + 1) * a.split_keys);
     }
@@ -724,7 +933,7 @@ __global__ __launch_bounds__(256, (NCH <= 4 ? 2 : 1)) void attention_mfma_kernel
         for (int j = 0; j < 2; ++j) {
             const int key0 = T.tb + 16 * j;
             const int idx = min(max(key0 / P - first_page, 0), DECODE_PAGE_CACHE - 1);
-            const int page = key0 < hi ? page_lds[idx] : -1;
+            const int page = __builtin_amdgcn_readfirstlane(key0 < hi ? page_lds[idx] : -1);
             T.ok |= (page >= 0 ? 1 : 0) << j;
             const size_t pk = (size_t)max(page, 0) * a.kv_heads + kvh;
             const __bf16* kptr = kp_base + (pk * P + key0 % P) * D + k_lane;
@@ -832,6 +1041,86 @@ __global__ __launch_bounds__(256, (NCH <= 4 ? 2 : 1)) void attention_mfma_kernel
     l_run += __shfl_xor(l_run, 16, MLR_WAVE);
     l_run += __shfl_xor(l_run, 32, MLR_WAVE);
 
+    if constexpr (FUSED) {
+        // every wavefront parks the sums of the g columns in LDS and all threads add them in the order 0..3, a channel each
+        constexpr int ND = NCH / 2;
+        const int pitch = D + 4;
+        float* ml = lds + 4 * g * pitch;                   // [4][g] maxima and sums of probabilities
+        float* whole = ml + 8 * g;                         // [g][D + 2] the result where no other workgroup has a part in it
+        if (col_valid) {
+#pragma unroll
+            for (int db = 0; db < 2 * NCH; ++db) *reinterpret_cast<floatx4*>(lds + (wave * g + col) * pitch + 16 * db + 4 * b) = o[db];
+            if (b == 0) {
+                ml[2 * (wave * g + col)] = m_run;
+                ml[2 * (wave * g + col) + 1] = l_run;
+            }
+        }
+        DecodeMerge<ND> merge;
+        if (wave < g) merge.ask(a, f, row0, kvh * g + wave, kvh, pos0, slot, lane);
+        __syncthreads();
+        for (int u = threadIdx.x; u < g * D; u += 256) {
+            const int c = u / D, d = u % D;
+            float mw[4], lw[4], m_tot = -INFINITY;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                mw[w] = ml[2 * (w * g + c)];
+                lw[w] = ml[2 * (w * g + c) + 1];
+                m_tot = fmaxf(m_tot, mw[w]);
+            }
+            float l_tot = 0.f, sum = 0.f;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                // (a wavefront that saw no key has sum 0 and is passed over; one whose keys were all NaN -- a page
+                // that nobody wrote -- has maximum -inf too, but a NaN sum, and must not be: 0 x NaN stays NaN)
+                const float share = mw[w] > -INFINITY ? __builtin_amdgcn_exp2f(mw[w] - m_tot) : 0.f;
+                const float part = lds[(w * g + c) * pitch + d];
+                l_tot += lw[w] == 0.f ? 0.f : lw[w] * share;
+                sum += lw[w] == 0.f ? 0.f : part * share;
+            }
+            if (splits == 1) {
+                whole[c * (D + 2) + d] = sum;
+                if (d == 0) {
+                    whole[c * (D + 2) + D] = m_tot;
+                    whole[c * (D + 2) + D + 1] = l_tot;
+                }
+                continue;
+            }
+            float* dst = a.partial + (((size_t)row0 * a.q_heads + kvh * g + c) * a.max_splits + split) * (D + 2);
+            store_through(dst + d, sum);
+            if (d == 0) {
+                store_through(dst + D, m_tot);
+                store_through(dst + D + 1, l_tot);
+            }
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wavefront's sums have arrived, and behind the barrier the others'
+        __syncthreads();
+        int32_t* counter = f.arrivals + (size_t)row0 * a.kv_heads + kvh;
+        int32_t before = 0;
+        const bool counts = threadIdx.x == 192;            // (of the wavefront that has no head to prepare where there are few)
+        if (splits > 1 && counts) before = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (wave < g) merge.own(a, f, lane);
+        if (counts) arrived = before;
+        __syncthreads();
+        if (splits > 1) {
+            if (arrived != splits - 1) return;
+            if (counts) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);    // for the next launch
+        }
+        asm volatile("" ::: "memory");
+#pragma unroll 1
+        for (int h = wave; h < g; h += 4) {
+            const int head = kvh * g + h;
+            if (h != wave) {
+                merge.ask(a, f, row0, head, kvh, pos0, slot, lane);
+                merge.own(a, f, lane);
+            }
+            if (splits == 1) merge.gather_own(whole + h * (D + 2), lane);
+            else merge.gather(a.partial + (((size_t)row0 * a.q_heads + head) * a.max_splits + first_split) * (D + 2), splits,
+                              reinterpret_cast<float*>(page_lds) + wave * COMBINE_MAX_SPLITS, lane);
+            merge.finish(a, row0, head, kvh, h == 0, pos0, lane);
+            wavefront_sync();
+        }
+        return;
+    }
     // merge the wavefronts: 1..3 park their state in LDS, 0 merges in ascending order
     const int stride = 16 * D + 32;                        // floats per wavefront: the sums [D / 4][16 columns][4], max[16], sum[16]
     if (wave > 0) {
@@ -873,7 +1162,7 @@ __global__ __launch_bounds__(256, (NCH <= 4 ? 2 : 1)) void attention_mfma_kernel
             }
         }
         if (col_valid) {
-            if (a.max_splits > 1 || FUSED) {                   // (FUSED: the merge kernel always follows)
+            if (a.max_splits > 1) {
                 float* dst = a.partial + (out_row * a.max_splits + split) * (D + 2);
 #pragma unroll
                 for (int db = 0; db < 2 * NCH; ++db) {
@@ -1215,215 +1504,51 @@ __global__ __launch_bounds__(64) void attention_combine_groups_kernel(AttnArgs a
     }
 }
 
-// The merge for `DecodeFusion`: one wavefront per (token, head).  Besides the splits' partial results it adds
-// the token's own key and value (see `DecodeFusion`), and the first head of every kv head writes them
-// into the cache.  A lane takes the rotation pairs lane and lane + 64 and the ND channels lane + 64 i.
-// Bound by its chain of loads: 6.2 us for one token of 16 heads of 128 channels in 5 splits and 6.9 for 8 tokens in 8 while
-// the splits' values were asked for behind their weights, then 5.1; with sixteen of them asked for at once instead of
-// eight a step of 28 layers behind 1980 tokens, 16 splits, takes 1140 us for 1201.
-template <int ND>
-__global__ __launch_bounds__(64) void attention_combine_fused_kernel(AttnArgs a, DecodeFusion f) {
-    // (group i is batch row i here.)  Loads are asked for as early as their addresses are known: the row's
-    // position and slot, its raw q, k, v and the norm weights at once; then what needs the position (the
-    // rotation row, the page id, the splits' maxima and sums, the values of the first sixteen splits); then the others',
-    // sixteen at a time.
-    __shared__ float w_lds[COMBINE_MAX_SPLITS];
-    const int m = blockIdx.x, head = blockIdx.y;
-    const int D = a.head_dim, P = a.page_size, half = D >> 1;
-    const int g = a.q_heads / a.kv_heads, kvh = head / g;
-    const int lane = threadIdx.x;
-    const int pos = a.positions[m], slot = a.slots[m];
-    const __bf16* row = f.qkv + (size_t)m * f.ld;
-    const __bf16* qs = row + (size_t)head * D;
-    const __bf16* ks = row + (size_t)(a.q_heads + kvh) * D;
-    const __bf16* vs = row + (size_t)(a.q_heads + a.kv_heads + kvh) * D;
-    const bool normed = f.q_norm_w != nullptr, rotated = f.rope != nullptr;
-    const float* qw = normed ? f.q_norm_w : reinterpret_cast<const float*>(row);      // (any readable address)
-    const float* kw = normed ? f.k_norm_w : reinterpret_cast<const float*>(row);
-    float qa[2], qb[2], ka[2], kb[2], qwa[2], qwb[2], kwa[2], kwb[2], vv[ND];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int j = min(lane + 64 * i, half - 1);
-        qa[i] = (float)qs[j];
-        qb[i] = (float)qs[j + half];
-        ka[i] = (float)ks[j];
-        kb[i] = (float)ks[j + half];
-        qwa[i] = qw[j];
-        qwb[i] = qw[j + half];
-        kwa[i] = kw[j];
-        kwb[i] = kw[j + half];
-    }
-#pragma unroll
-    for (int i = 0; i < ND; ++i) vv[i] = (float)vs[min(lane + 64 * i, D - 1)];
-    // second round: everything that needs the position
-    const float* cs = (rotated ? f.rope : reinterpret_cast<const float*>(a.positions)) + (rotated ? (size_t)pos * D : 0);
-    float co[2], si[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int j = rotated ? min(lane + 64 * i, half - 1) : 0;
-        co[i] = cs[j];
-        si[i] = cs[rotated ? j + half : 0];
-    }
-    const int page_read = a.block_table[(size_t)slot * a.max_blocks + min(pos / P, a.max_blocks - 1)];
-    const int page = pos / P < a.max_blocks ? page_read : -1;    // (beyond the request's row of the table: no page)
-    const int glo = a.window > 0 ? max(0, pos + 1 - a.window) : 0;
-    const int first = a.max_splits > 1 ? glo / a.split_keys : 0;
-    const int last = a.max_splits > 1 ? min(a.max_splits - 1, max(pos - 1, 0) / a.split_keys) : 0;
-    const int n = last - first + 1;                     // the same range of splits that the attention kernel served
-    const float* base = a.partial + (((size_t)m * a.q_heads + head) * a.max_splits + first) * (D + 2);
-    constexpr int AHEAD = 16;
-    float part[AHEAD][ND];
-    auto fetch = [&](int s0) {                          // (clamped: no branch around a load)
-#pragma unroll
-        for (int u = 0; u < AHEAD; ++u)
-#pragma unroll
-            for (int i = 0; i < ND; ++i) part[u][i] = base[(size_t)min(s0 + u, n - 1) * (D + 2) + lane + 64 * i];
-    };
-    fetch(0);
-    float smax[COMBINE_MAX_SPLITS / 64], ssum[COMBINE_MAX_SPLITS / 64];
-    float gmax = -INFINITY;
-#pragma unroll
-    for (int r = 0; r < COMBINE_MAX_SPLITS / 64; ++r) {
-        const int s = lane + 64 * r;
-        if (64 * r >= n) break;
-        const float* p = base + (size_t)min(s, n - 1) * (D + 2);
-        smax[r] = s < n ? p[D] : -INFINITY;
-        ssum[r] = p[D + 1];
-        gmax = fmaxf(gmax, smax[r]);
-    }
+extern "C" int mlr_attention_even_ranges(int walk, int workgroups, int units, int wide) { return even_ranges(walk, workgroups, units, wide); }
 
-    // query and key of this token: norm, rotation, rounded to bfloat16 (what the cache holds)
-    float qsum = 0.f, ksum = 0.f;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        if (lane + 64 * i >= half) qa[i] = qb[i] = ka[i] = kb[i] = 0.f;
-        qsum += squares(qa[i], qb[i]);
-        ksum += squares(ka[i], kb[i]);
-    }
-    if (normed) {
-        qsum = wave_sum(qsum);
-        ksum = wave_sum(ksum);
-        const float qscale = 1.0f / sqrtf(qsum / (float)D + f.eps), kscale = 1.0f / sqrtf(ksum / (float)D + f.eps);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            qa[i] = (qa[i] * qscale) * qwa[i];
-            qb[i] = (qb[i] * qscale) * qwb[i];
-            ka[i] = (ka[i] * kscale) * kwa[i];
-            kb[i] = (kb[i] * kscale) * kwb[i];
-        }
-    }
-    float dot = 0.f;
-    __bf16 k_lo[2], k_hi[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        float qx = qa[i], qy = qb[i], kx = ka[i], ky = kb[i];
-        if (rotated) {
-            qx = turn_x(qa[i], qb[i], co[i], si[i]);
-            qy = turn_y(qa[i], qb[i], co[i], si[i]);
-            kx = turn_x(ka[i], kb[i], co[i], si[i]);
-            ky = turn_y(ka[i], kb[i], co[i], si[i]);
-        }
-        k_lo[i] = (__bf16)kx;
-        k_hi[i] = (__bf16)ky;
-        if (lane + 64 * i < half)
-            dot += (float)(__bf16)qx * (float)k_lo[i] + (float)(__bf16)qy * (float)k_hi[i];
-    }
-    const float s_own = wave_sum(dot) * (a.scale * 1.44269504088896340736f);     // base-2 domain, as the partial maxima
-    gmax = fmaxf(wave_max(gmax), s_own);
-    // the splits' weights (maxima are base-2 exponents) and the denominator, summed in ascending order
-#pragma unroll
-    for (int r = 0; r < COMBINE_MAX_SPLITS / 64; ++r) {
-        const int s = lane + 64 * r;
-        if (64 * r >= n) break;
-        if (s < n) w_lds[s] = smax[r] > -INFINITY ? __builtin_amdgcn_exp2f(smax[r] - gmax) * 1.0f : 0.f;
-    }
-    __syncthreads();
-    float den = 0.f;
-#pragma unroll
-    for (int r = 0; r < COMBINE_MAX_SPLITS / 64; ++r) {
-        const int s = lane + 64 * r;
-        if (64 * r >= n) break;
-        den += s < n ? w_lds[s] * ssum[r] : 0.f;
-    }
-    den = wave_sum(den);
-    float num[ND];
-#pragma unroll
-    for (int i = 0; i < ND; ++i) num[i] = 0.f;
-    for (int s0 = 0; s0 < n; s0 += AHEAD) {
-        if (s0 > 0) fetch(s0);
-#pragma unroll
-        for (int u = 0; u < AHEAD; ++u) {
-            if (s0 + u >= n) break;
-            const float w = w_lds[s0 + u];
-#pragma unroll
-            for (int i = 0; i < ND; ++i) num[i] += w * part[u][i];
-        }
-    }
-    const float w_own = __builtin_amdgcn_exp2f(s_own - gmax);
-    den += w_own;
-#pragma unroll
-    for (int i = 0; i < ND; ++i) {
-        const int d = lane + 64 * i;
-        if (d < D) a.out[((size_t)m * a.q_heads + head) * D + d] = from_float<elem_t>((num[i] + w_own * vv[i]) / den);
-    }
-    // key and value into their pages, once per kv head
-    if (head != kvh * g || page < 0) return;
-    const size_t pk = (size_t)page * a.kv_heads + kvh;
-    __bf16* kdst = reinterpret_cast<__bf16*>(const_cast<elem_t*>(a.k_pages)) + (pk * P + pos % P) * D;
-    __bf16* vdst = reinterpret_cast<__bf16*>(const_cast<elem_t*>(a.v_pages)) + pk * D * P + pos % P;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int j = lane + 64 * i;
-        if (j < half) {
-            kdst[j] = k_lo[i];
-            kdst[j + half] = k_hi[i];
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < ND; ++i) {
-        const int d = lane + 64 * i;
-        if (d < D) vdst[(size_t)d * P] = (__bf16)vv[i];
-    }
+template <int NCH, int PAGE>
+static int launch_decode_fused(dim3 grid, const AttnArgs& a, const int32_t* group_row0, const int32_t* group_ntok, const DecodeFusion& f,
+                               hipStream_t stream) {
+    auto* kernel = attention_mfma_kernel<NCH, true, PAGE>;
+    const auto lds_bytes = [](int g) { return sizeof(float) * (size_t)g * (4 * (32 * NCH + 6) + 32 * NCH + 2); };      // four wavefronts' and the workgroup's
+    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes(16));
+    if (allowed != hipSuccess) return (int)allowed;
+    kernel<<<grid, 256, lds_bytes(a.q_heads / a.kv_heads), stream>>>(a, group_row0, group_ntok, f);
+    return (int)hipGetLastError();
 }
 
 // Decoding with `DecodeFusion`: group i is the one token in batch row i (group_row0[i] = i, group_ntok[i] = 1);
 // qkv holds the raw projections
 // [rows, ld].  Key and value of every token are written into the cache.  `partial` holds at least
-// rows * q_heads * max(max_splits, 1) * (head_dim + 2) floats, also without splits.
+// rows * q_heads * max(max_splits, 1) * (head_dim + 2) floats, also without splits; `arrivals` rows * kv_heads zeros, which are
+// zeros again when the launch is done.
 // Needs what `mlr_attention_mfma` needs and head_dim % 64 == 0.
 extern "C" int mlr_attention_decode_fused(
     const void* qkv, int ld, const void* k_pages, const void* v_pages, const int32_t* block_table, int max_blocks,
     const int32_t* slots, const int32_t* positions, void* out, float* partial, const int32_t* group_row0,
     const int32_t* group_ntok, int groups, int q_heads, int kv_heads, int head_dim, int page_size, int window,
-    float scale, int split_keys, int max_splits, const float* q_norm_w, const float* k_norm_w, float eps,
-    const float* rope, hipStream_t stream) {
+    float scale, int split_keys, int max_splits, int workgroups, const float* q_norm_w, const float* k_norm_w, float eps,
+    const float* rope, int32_t* arrivals, hipStream_t stream) {
     if (groups <= 0) return 0;
     if (head_dim % 64 != 0 || head_dim > 256 || page_size % 16 != 0 || q_heads % kv_heads != 0 ||
-        q_heads / kv_heads > 16 || partial == nullptr || (q_norm_w == nullptr) != (k_norm_w == nullptr)) return -1;
+        q_heads / kv_heads > 16 || partial == nullptr || arrivals == nullptr || (q_norm_w == nullptr) != (k_norm_w == nullptr)) return -1;
     if (max_splits < 1) max_splits = 1;
-    if (max_splits > 1 && (split_keys <= 0 || split_keys % MFMA_TILE_KEYS != 0 || max_splits > COMBINE_MAX_SPLITS)) return -2;
-    if ((max_splits > 1 ? split_keys / page_size + 2 : max_blocks) > DECODE_PAGE_CACHE) return -3;
+    if ((max_splits > 1 || workgroups > 0) && (split_keys <= 0 || split_keys % MFMA_TILE_KEYS != 0 || max_splits > COMBINE_MAX_SPLITS)) return -2;
+    if (workgroups == 0 && (max_splits > 1 ? split_keys / page_size + 2 : max_blocks) > DECODE_PAGE_CACHE) return -3;
+    // (an even range is less than twice a share's keys)
+    if (workgroups > 0 && (2ll * split_keys * groups * kv_heads / workgroups + 128) / page_size + 2 > DECODE_PAGE_CACHE) return -3;
     AttnArgs a{nullptr, (const elem_t*)k_pages, (const elem_t*)v_pages, block_table, slots,
                positions, (elem_t*)out, partial, max_blocks, q_heads, kv_heads, head_dim, page_size,
                window, split_keys, max_splits, scale};
-    DecodeFusion f{(const __bf16*)qkv, q_norm_w, k_norm_w, rope, ld, eps};
+    DecodeFusion f{(const __bf16*)qkv, q_norm_w, k_norm_w, rope, arrivals, ld, eps, workgroups};
     dim3 grid(groups, kv_heads, max_splits);
-    const size_t lds = sizeof(float) * 3 * (16 * (size_t)head_dim + 32);
     switch (head_dim / 32) {
-        case 2: attention_mfma_kernel<2, true><<<grid, 256, lds, stream>>>(a, group_row0, group_ntok, f); break;
-        case 4: attention_mfma_kernel<4, true><<<grid, 256, lds, stream>>>(a, group_row0, group_ntok, f); break;
-        case 6: attention_mfma_kernel<6, true><<<grid, 256, lds, stream>>>(a, group_row0, group_ntok, f); break;
-        default: attention_mfma_kernel<8, true><<<grid, 256, lds, stream>>>(a, group_row0, group_ntok, f); break;
+        case 2: return page_size == 16 ? launch_decode_fused<2, 16>(grid, a, group_row0, group_ntok, f, stream) : launch_decode_fused<2, 0>(grid, a, group_row0, group_ntok, f, stream);
+        case 4: return page_size == 16 ? launch_decode_fused<4, 16>(grid, a, group_row0, group_ntok, f, stream) : launch_decode_fused<4, 0>(grid, a, group_row0, group_ntok, f, stream);
+        case 6: return launch_decode_fused<6, 0>(grid, a, group_row0, group_ntok, f, stream);
+        default: return launch_decode_fused<8, 0>(grid, a, group_row0, group_ntok, f, stream);
     }
-    int err = (int)hipGetLastError();
-    if (err != 0) return err;
-    switch (head_dim / 64) {
-        case 1: attention_combine_fused_kernel<1><<<dim3(groups, q_heads), 64, 0, stream>>>(a, f); break;
-        case 2: attention_combine_fused_kernel<2><<<dim3(groups, q_heads), 64, 0, stream>>>(a, f); break;
-        case 3: attention_combine_fused_kernel<3><<<dim3(groups, q_heads), 64, 0, stream>>>(a, f); break;
-        default: attention_combine_fused_kernel<4><<<dim3(groups, q_heads), 64, 0, stream>>>(a, f); break;
-    }
-    return (int)hipGetLastError();
 }
 
 // Groups: group_row0[i] = first batch row of group i, group_ntok[i] = its tokens (consecutive rows of one

@@ -12,7 +12,10 @@ class Workspace:
     """Named scratch buffers that live as long as the runner.  `reserve` carves every buffer that the
     parts have named for the largest step out of ONE allocation; a name that was not planned (a part
     without a plan), or a size beyond its plan, is allocated when it is first asked for and grows only
-    when a larger size is asked, so steady steps allocate nothing either way."""
+    when a larger size is asked, so steady steps allocate nothing either way.  The buffers of COUNTERS hold zeros when they are
+    made; whoever counts in one leaves zeros behind."""
+
+    COUNTERS = ("arrivals",)
 
     def __init__(self, device):
         self.device = torch.device(device)
@@ -36,6 +39,8 @@ class Workspace:
         for (name, dtype), count in plan.items():
             size = count * torch.empty((), dtype=dtype).element_size()
             self._buffers[(name, dtype)] = self._arena[at:at + size].view(dtype)
+            if name in self.COUNTERS:
+                self._buffers[(name, dtype)].zero_()
             at += -(-size // 256) * 256
 
     def unplanned_bytes(self):
@@ -53,7 +58,7 @@ class Workspace:
         key = (name, dtype)
         buf = self._buffers.get(key)
         if buf is None or buf.numel() < count:
-            buf = torch.empty(max(count, 1), dtype=dtype, device=self.device)
+            buf = (torch.zeros if name in self.COUNTERS else torch.empty)(max(count, 1), dtype=dtype, device=self.device)
             self._buffers[key] = buf
             self._unplanned[key] = buf.numel() * buf.element_size()
             for stale in [k for k in self._views if k[0] == name and k[1] == dtype]:
@@ -220,6 +225,34 @@ class StepContext:
             return 0, 1, None
         return self._split(max(1, rows * kv_heads), self.target_workgroups, batch_rows, q_heads, head_dim, longest, LONG_RANGE,
                            narrow=narrow and not self.routed)
+
+    def even_split(self, rows, kv_heads, q_heads, head_dim):
+        """(workgroups, wide, max_splits, partial buffer) for single tokens whose key ranges are merged in the launch that makes them
+        (`attention_decode_fused`): every token's keys in ranges of its own, evenly wide (`even_ranges`); None where `attention_split`
+        has to say: no splits wanted, a model that routes, partial results that would not fit, so many tokens that one has not two units.
+
+        One workgroup a compute unit takes the keys as fast as two, each more is another partial result that the merge waits for, and a
+        few more than fill the units cost a second round.  Measured with 1 to 64 tokens of 16 query and 8 kv heads of 128 channels behind
+        400 to 8000 keys, pages cold, us a layer, ranges as `attention_split` cuts them and even ones: 1 token behind 1100 keys 12.6, 12.2;
+        behind 3800 15.1, 15.3; 2 behind 1100 15.9, 12.9; 6 behind 2000 21.4, 20.1; 8 behind 4600 to 4900 43.2, 40.1; 12 behind 2000
+        30.9, 28.0; 16 behind up to 3800 38.8, 37.4.  Not beyond half the units: 24 behind 2000 50.7, 45.0, but 24 behind 300 to 3800 48.5,
+        59.2, where a long context's one range keeps the step waiting, and 64 behind 129 to 3000, whose second ranges are dealt out when
+        the first are done, 76.3, 84.6."""
+        units, workgroups = rows * kv_heads, min(self.compute_units, self.target_workgroups)
+        if rows > self.split_max_tokens or self.split_keys <= 0 or self.routed or 2 * units > workgroups:
+            return None
+        wide = -(-LONG_RANGE * workgroups // units // 64) * 64
+        max_splits = self.even_ranges(self.max_context, workgroups, units, wide)
+        numel = self.kernels.attention_partial_numel(rows, q_heads, head_dim, max_splits)
+        if max_splits > 1024 or (self.partial_budget is not None and numel > self.partial_budget):
+            return None
+        return workgroups, wide, max_splits, self.workspace.get("attn_partial", (numel,), torch.float32)
+
+    @staticmethod
+    def even_ranges(walk, workgroups, units, wide):
+        """The kernel's rule (`even_ranges` in attention.hip) for one token behind `walk` keys: it never gives a shorter context more
+        ranges than a longer one."""
+        return max(1, min(workgroups * -(-walk // wide) // units, max(16, walk // 256), -(-walk // 64)))
 
     def group_split(self, groups, batch_rows, kv_heads, q_heads, head_dim, longest=None):
         """As `attention_split` for `groups` groups of many tokens each (prompt portions), which give

@@ -114,6 +114,8 @@ class GqaAttention:
         plan = {("qkv", dtype): rows * (width + 2 * s.kv_heads * s.head_dim), ("q", dtype): rows * width,
                 ("attn", dtype): rows * width, ("mixer_out", dtype): rows * s.hidden,
                 ("attn_partial", torch.float32): partial}
+        if dtype == torch.bfloat16:
+            plan[("arrivals", torch.int32)] = rows * s.kv_heads
         for big_factor in (0, 4, 8):
             plan[(f"token_groups_{tq}_{big_factor}", torch.int32)] = 2 * rows + 2
         return plan
@@ -217,11 +219,16 @@ class GqaAttention:
         whole_split_half = rotation is None or (rotation.dim == s.head_dim and not rotation.interleaved)
         if (ctx.single_tokens and write_cache and x.dtype == torch.bfloat16 and whole_split_half
                 and k.decode_fusion_supported(s.q_heads, s.kv_heads, s.head_dim, view.page_size)):
-            # decoding: norm, rotation and cache write ride in the attention's two launches
+            # decoding: norm, rotation and cache write ride in the attention's launch
             attn = ctx.workspace.get("attn", (m, s.q_heads * s.head_dim), x.dtype)
             groups, _, _ = ctx.token_groups(max(1, 16 // (s.q_heads // s.kv_heads)), 0)
-            split_keys, max_splits, partial = ctx.attention_split(m, m, s.kv_heads, s.q_heads, s.head_dim,
-                                                                  longest=k.mfma_longest_context(view.page_size))
+            even = ctx.even_split(m, s.kv_heads, s.q_heads, s.head_dim)
+            if even is not None:
+                workgroups, split_keys, max_splits, partial = even
+            else:
+                workgroups = 0
+                split_keys, max_splits, partial = ctx.attention_split(m, m, s.kv_heads, s.q_heads, s.head_dim,
+                                                                      longest=k.mfma_longest_context(view.page_size))
             if partial is None:
                 partial = ctx.workspace.get("attn_partial", (k.attention_partial_numel(m, s.q_heads, s.head_dim, 1),),
                                             torch.float32)
@@ -232,7 +239,8 @@ class GqaAttention:
                 self.q_norm.weight if self.q_norm is not None else None,
                 self.k_norm.weight if self.k_norm is not None else None,
                 self.q_norm.eps if self.q_norm is not None else 0.0, rope, partial,
-                window=s.window, split_keys=split_keys, max_splits=max_splits)
+                window=s.window, split_keys=split_keys, max_splits=max_splits,
+                workgroups=workgroups, arrivals=ctx.workspace.get("arrivals", (m * s.kv_heads,), torch.int32))
             return attn
         q = ctx.workspace.get("q", (m, s.q_heads * s.head_dim), x.dtype)
         k.qk_norm_rope_kv(
