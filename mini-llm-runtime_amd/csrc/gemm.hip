@@ -482,7 +482,7 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const __
     __shared__ float part[SKINNY_WAVES - 1][NW][MT][64][4];
     __shared__ float ss_lds[SKINNY_WAVES][16];
     extern __shared__ __attribute__((aligned(16))) char staged[];   // [SKINNY_WAVES][M][pitch] when STAGE
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r16 = lane & 15, b = lane >> 4;
     const int cols = PAIR ? epi.cols : 16;
     const int n0 = blockIdx.x * cols;
@@ -496,20 +496,25 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const __
     // What the epilogue needs from memory is asked for here, before the weight, by every wavefront alike
     // (no branch around a load); only wavefront 0 uses it.
     float ss_mine = 0.f;                                   // EPI_SCALE: this lane's share of the row's partial sums
+    float4 ss4[EPI == EPI_SCALE ? 4 : 1];                  // ... which are added when the weight is multiplied, where these hold them all
+    const int ss_quads = epi.ss_parts >> 2, ss_run = (ss_quads + 4 * SKINNY_WAVES - 1) / (4 * SKINNY_WAVES);
+    const bool ss_later = EPI == EPI_SCALE && epi.ss_vec && ss_run <= 4;
     float4 h4 = make_float4(0.f, 0.f, 0.f, 0.f), nw4 = h4;  // EPI_RESIDUAL: h and the next norm's weights at (row r16, columns n0 + 4 b ..)
     float4 h4b = h4, nw4b = h4;                            // ... and, PAIR, at the second strip's columns n0 + 16 + 4 b ..
     if constexpr (EPI == EPI_SCALE) {
         // the row's partial sums are dealt out to the 32 (wavefront, lane block) pairs in runs of q; a run is
         // added in ascending order (four sums that lie side by side as (0 + 1) + (2 + 3) first, when their number
         // allows 16-byte loads), the four runs of a wavefront as (0 + 1) + (2 + 3), the wavefronts in the order
-        // 0..7: an order that depends on nothing but the number of partial sums.  Four loads are asked for before
-        // the first is used: a load a turn of the loop would cost a trip to the cache each, one after the other,
-        // before the workgroup has asked for any of its weight.
+        // 0..7: an order that depends on nothing but the number of partial sums.  Up to 512 of them a lane's four loads are asked
+        // for here and used behind the products: used here, they cost a trip to the cache before the workgroup has asked for any of
+        // its weight (0.6B sizes, one token: 1046 us a step, so 1034; eight 1623, 1606).  Of more, four are asked for before the first is used.
         const float* row = epi.ss + (size_t)min(r16, M - 1) * epi.ss_parts;
         const int pair = wave * 4 + b;
-        if (epi.ss_vec) {
-            const int quads = epi.ss_parts >> 2;
-            const int q = (quads + 4 * SKINNY_WAVES - 1) / (4 * SKINNY_WAVES);
+        if (ss_later) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) ss4[j] = reinterpret_cast<const float4*>(row)[min(pair * ss_run + j, ss_quads - 1)];
+        } else if (epi.ss_vec) {
+            const int quads = ss_quads, q = ss_run;
             const float4* row4 = reinterpret_cast<const float4*>(row);
             for (int j0 = 0; j0 < q; j0 += 4) {
                 float4 v[4];
@@ -662,6 +667,12 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const __
                 for (int r = 0; r < 4; ++r) part[wave - 1][g][i][lane][r] = acc[g][i][r];
     }
     if constexpr (EPI == EPI_SCALE) {
+        if (ss_later) {
+            const int pair = wave * 4 + b;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                ss_mine += j < ss_run && pair * ss_run + j < ss_quads ? (ss4[j].x + ss4[j].y) + (ss4[j].z + ss4[j].w) : 0.f;
+        }
         ss_mine += __shfl_xor(ss_mine, 16, MLR_WAVE);
         ss_mine += __shfl_xor(ss_mine, 32, MLR_WAVE);
         if (b == 0) ss_lds[wave][r16] = ss_mine;
@@ -786,9 +797,19 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const __
         }
         return;
     }
+    // (whole groups of four columns on 8 or 16 bytes: one store a lane)
+    const bool whole = (N & 3) == 0 && (reinterpret_cast<size_t>(out_raw) & (OUT_FLOAT ? 15 : 7)) == 0;
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
         const int m = 16 * i + r16;
+        if (whole) {
+            const size_t at = (size_t)m * N + n0 + 4 * b;
+            typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4_t;
+            if (m >= M || n0 + 4 * b >= N) continue;
+            if (OUT_FLOAT) *reinterpret_cast<float4*>((float*)out_raw + at) = make_float4(y4[i][0], y4[i][1], y4[i][2], y4[i][3]);
+            else *reinterpret_cast<bf16x4_t*>((__bf16*)out_raw + at) = bf16x4_t{(__bf16)y4[i][0], (__bf16)y4[i][1], (__bf16)y4[i][2], (__bf16)y4[i][3]};
+            continue;
+        }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int n = n0 + 4 * b + r;
