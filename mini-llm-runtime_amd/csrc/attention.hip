@@ -36,6 +36,7 @@ struct AttnArgs {
     float* partial;             // [M, q_heads, max_splits, head_dim + 2] when max_splits > 1
     int max_blocks, q_heads, kv_heads, head_dim, page_size, window, split_keys, max_splits;
     float scale;
+    int heads_per_kv;           // q_heads / kv_heads (of the matrix-core kernels)
 };
 
 __global__ __launch_bounds__(256) void paged_attention_kernel(AttnArgs a) {
@@ -579,7 +580,14 @@ struct DecodeFusion {
     int ld;
     float eps;
     int workgroups;             // 0: key ranges at absolute multiples of split_keys, else see `even_ranges`
+    int share;                  // workgroups / (tokens times kv heads)
 };
+
+// x / n rounded down, for 0 <= x < 2^20: the reciprocal is off by less than the half that keeps a quotient from a whole number.
+__device__ __forceinline__ int quotient(int x, int n) {
+    return __builtin_amdgcn_readfirstlane((int)(((float)x + 0.5f) * __builtin_amdgcn_rcpf((float)n)));
+}
+
 
 // Key ranges of one token of `units` (tokens times kv heads) behind `walk` keys: its share of `workgroups`, or of twice, three times
 // as many where a range would be wide (`wide` keys to a share of the first); none of less than 64 keys, and none of less than 256
@@ -587,7 +595,7 @@ struct DecodeFusion {
 // ranges keep the compute units evenly busy, and one workgroup a unit, or two, is what they take best -- a few more than that cost
 // the step a second round (`StepContext.even_split` has the figures).
 __host__ __device__ inline int even_ranges(int walk, int workgroups, int units, int wide) {
-    const int rounds = (walk + wide - 1) / wide, n = (int)((long long)workgroups * rounds / units);
+    const int rounds = (walk + wide - 1) / wide, n = workgroups * rounds / units;
     const int least = walk / 256 > 16 ? walk / 256 : 16, pieces = (walk + 63) / 64;
     const int most = least < pieces ? least : pieces;
     return n < 1 ? 1 : n < most ? n : most;
@@ -780,14 +788,15 @@ __global__ __launch_bounds__(256, (NCH <= 4 ? 2 : 1)) void attention_mfma_kernel
     __shared__ int32_t page_lds[DECODE_PAGE_CACHE];    // the request's page ids for this workgroup's key range
     __shared__ int32_t arrived;                        // FUSED: workgroups of this token and kv head that were done before this one
     const int D = FUSED ? 32 * NCH : a.head_dim, P = PAGE > 0 ? PAGE : a.page_size;
-    const int g = a.q_heads / a.kv_heads;
+    const int g = a.heads_per_kv;
     const int grp = blockIdx.x, kvh = blockIdx.y, split = blockIdx.z;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15, b = lane >> 4;
     // (FUSED: group i is the one token in batch row i; no need to wait for the group vectors)
     const int row0 = FUSED ? grp : group_row0[grp], ntok = FUSED ? 1 : group_ntok[grp];
-    const int slot = a.slots[row0], pos0 = a.positions[row0];
-    const int tok = col / g, hh = col % g;
+    int slot = a.slots[row0], pos0 = a.positions[row0];
+    asm volatile("" : "+s"(slot), "+s"(pos0));                         // (asked for together)
+    const int tok = FUSED ? col >= g : col / g, hh = FUSED ? col : col % g;       // (FUSED: of columns beyond the heads, never used)
     const bool col_valid = tok < ntok;
     const int kend_full = col_valid ? pos0 + tok + 1 : 0;
     int kbegin_c = a.window > 0 ? max(0, kend_full - a.window) : 0;
@@ -796,13 +805,14 @@ __global__ __launch_bounds__(256, (NCH <= 4 ? 2 : 1)) void attention_mfma_kernel
     const int ke = pos0 + ntok - (FUSED ? 1 : 0);                      // keys below ke are written
     int lo = glo, hi = ke, first_split = 0, splits = 1;                // the key ranges that hold keys
     if (FUSED && f.workgroups > 0) {
-        const int from = glo / MFMA_TILE_KEYS * MFMA_TILE_KEYS, walk = max(ke - from, 1), pieces = (walk + 63) / 64;
-        const int n = min(a.max_splits, even_ranges(walk, f.workgroups, gridDim.x * gridDim.y, a.split_keys));
-        const int width = (pieces + n - 1) / n * 64;                    // whole 64 keys, from the tile of the first one on
-        splits = (walk + width - 1) / width;
+        const int from = glo & -MFMA_TILE_KEYS, walk = max(ke - from, 1), pieces = (walk + 63) >> 6;
+        const int n = min(a.max_splits, walk <= a.split_keys ? min(f.share, min(max(walk >> 8, 16), pieces))
+                                                             : even_ranges(walk, f.workgroups, gridDim.x * gridDim.y, a.split_keys));
+        const int width = quotient(pieces + n - 1, n);                  // in 64 keys, from the tile of the first one on
+        splits = quotient(pieces + width - 1, width);
         if (split >= splits) return;
-        lo = max(lo, from + split * width);
-        hi = min(hi, from + (split + 1) * width);
+        lo = max(lo, from + split * width * 64);
+        hi = min(hi, from + (split + 1) * width * 64);
     } else if (a.max_splits > 1) {
         first_split = glo / a.split_keys;
         splits = min(a.max_splits - 1, max(ke - 1, 0) / a.split_keys) + 1 - first_split;
@@ -825,9 +835,11 @@ __global__ __launch_bounds__(256, (NCH <= 4 ? 2 : 1)) void attention_mfma_kernel
     const int32_t* table = a.block_table + (size_t)slot * a.max_blocks;
 
     // page ids first, into LDS: a tile's loads then never wait on a load of the block table
+    // (a page of sixteen keys: a tile's two ids, neighbours in the table, come straight into scalar registers, a tile ahead)
+    constexpr bool SCALAR_PAGES = FUSED && PAGE == 16;
     const int t_begin = lo / MFMA_TILE_KEYS, t_end = (hi + MFMA_TILE_KEYS - 1) / MFMA_TILE_KEYS;
-    const int first_page = t_begin * MFMA_TILE_KEYS / P;
-    {
+    const int first_page = SCALAR_PAGES ? 0 : t_begin * MFMA_TILE_KEYS / P;
+    if constexpr (!SCALAR_PAGES) {
         const int n_pages = min(DECODE_PAGE_CACHE, (hi + P - 1) / P - first_page);
         // (an entry beyond the request's row of the table is no page, like an entry of -1)
         for (int i = threadIdx.x; i < n_pages; i += 256)
@@ -862,7 +874,7 @@ __global__ __launch_bounds__(256, (NCH <= 4 ? 2 : 1)) void attention_mfma_kernel
                 qf[c] = *reinterpret_cast<const bf16x8*>(q + ((size_t)(row0 + tok) * a.q_heads + kvh * g + hh) * D + d0);
         }
     }
-    __syncthreads();
+    if constexpr (!SCALAR_PAGES) __syncthreads();
     auto finish_queries = [&]() {
         // per-head norm, rotation (a lane holds channels 32 c + 8 b .. of every chunk c, so with head_dim =
         // 32 NCH, NCH even, the partner d + head_dim / 2 of a channel is in chunk c + NCH / 2 of the same
@@ -926,14 +938,28 @@ __global__ __launch_bounds__(256, (NCH <= 4 ? 2 : 1)) void attention_mfma_kernel
     // No branch around a load: a load behind a branch makes the compiler wait for every load in flight.
     // A missing page reads page 0 instead, channels beyond head_dim read channel block 0; both are
     // discarded when the tile is used.
-    auto load = [&](int t, KvTile<NCH>& T) {
+    struct Ids { int at[2]; };
+    auto ids = [&](int t) {
+        Ids r{{-1, -1}};
+        if constexpr (SCALAR_PAGES) {
+            typedef const __attribute__((address_space(4))) int32_t* scalar_ptr;
+            const scalar_ptr scalars = (scalar_ptr)table;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int id = scalars[min(max(2 * t + j, 0), a.max_blocks - 1)];
+                r.at[j] = t * MFMA_TILE_KEYS + 16 * j < hi && 2 * t + j < a.max_blocks ? id : -1;
+            }
+        }
+        return r;
+    };
+    auto load = [&](int t, KvTile<NCH>& T, const Ids& known) {
         T.tb = t * MFMA_TILE_KEYS;
         T.ok = 0;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const int key0 = T.tb + 16 * j;
             const int idx = min(max(key0 / P - first_page, 0), DECODE_PAGE_CACHE - 1);
-            const int page = __builtin_amdgcn_readfirstlane(key0 < hi ? page_lds[idx] : -1);
+            const int page = SCALAR_PAGES ? known.at[j] : __builtin_amdgcn_readfirstlane(key0 < hi ? page_lds[idx] : -1);
             T.ok |= (page >= 0 ? 1 : 0) << j;
             const size_t pk = (size_t)max(page, 0) * a.kv_heads + kvh;
             const __bf16* kptr = kp_base + (pk * P + key0 % P) * D + k_lane;
@@ -965,14 +991,21 @@ __global__ __launch_bounds__(256, (NCH <= 4 ? 2 : 1)) void attention_mfma_kernel
         }
         // this lane: keys tb + 16 j + 4 b + r of column `col`
         float sv[2][4];
+        if (FUSED && T.ok == 3 && T.tb >= lo && T.tb + MFMA_TILE_KEYS <= hi) {       // (one token: its keys are every column's)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+            for (int j = 0; j < 2; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int key = T.tb + 16 * j + 4 * b + r;
-                const bool ok = ((T.ok >> j) & 1) && key >= kbegin_c && key < kstop_c;
-                sv[j][r] = ok ? s[j][r] * c2 : -INFINITY;
-            }
+                for (int r = 0; r < 4; ++r) sv[j][r] = s[j][r] * c2;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int key = T.tb + 16 * j + 4 * b + r;
+                    const bool ok = ((T.ok >> j) & 1) && key >= kbegin_c && key < kstop_c;
+                    sv[j][r] = ok ? s[j][r] * c2 : -INFINITY;
+                }
+        }
         float tile_max = fmaxf(fmaxf(fmaxf(sv[0][0], sv[0][1]), fmaxf(sv[0][2], sv[0][3])),
                                fmaxf(fmaxf(sv[1][0], sv[1][1]), fmaxf(sv[1][2], sv[1][3])));
         tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16, MLR_WAVE));
@@ -1023,14 +1056,17 @@ __global__ __launch_bounds__(256, (NCH <= 4 ? 2 : 1)) void attention_mfma_kernel
         KvTile<NCH> ta, tb2;
         int t = t_begin + wave;
         const int t_last = t + ((t_end - 1 - t) / 4) * 4;
-        if (t < t_end) load(t, ta);
+        Ids next = ids(min(t + 4, t_last));
+        if (t < t_end) load(t, ta, ids(t));
         if (FUSED) finish_queries();
         if (t < t_end) {
             for (;;) {
-                load(min(t + 4, t_last), tb2);
+                load(min(t + 4, t_last), tb2, next);
+                next = ids(min(t + 8, t_last));
                 compute(ta);
                 if (t + 4 >= t_end) break;
-                load(min(t + 8, t_last), ta);
+                load(min(t + 8, t_last), ta, next);
+                next = ids(min(t + 12, t_last));
                 compute(tb2);
                 if (t + 8 >= t_end) break;
                 t += 8;
@@ -1536,12 +1572,13 @@ extern "C" int mlr_attention_decode_fused(
     if (max_splits < 1) max_splits = 1;
     if ((max_splits > 1 || workgroups > 0) && (split_keys <= 0 || split_keys % MFMA_TILE_KEYS != 0 || max_splits > COMBINE_MAX_SPLITS)) return -2;
     if (workgroups == 0 && (max_splits > 1 ? split_keys / page_size + 2 : max_blocks) > DECODE_PAGE_CACHE) return -3;
-    // (an even range is less than twice a share's keys)
+    // (an even range is less than twice a share's keys; `quotient`)
+    if (workgroups > 0 && (long long)max_blocks * page_size >= 1ll << 25) return -2;
     if (workgroups > 0 && (2ll * split_keys * groups * kv_heads / workgroups + 128) / page_size + 2 > DECODE_PAGE_CACHE) return -3;
     AttnArgs a{nullptr, (const elem_t*)k_pages, (const elem_t*)v_pages, block_table, slots,
                positions, (elem_t*)out, partial, max_blocks, q_heads, kv_heads, head_dim, page_size,
-               window, split_keys, max_splits, scale};
-    DecodeFusion f{(const __bf16*)qkv, q_norm_w, k_norm_w, rope, arrivals, ld, eps, workgroups};
+               window, split_keys, max_splits, scale, q_heads / kv_heads};
+    DecodeFusion f{(const __bf16*)qkv, q_norm_w, k_norm_w, rope, arrivals, ld, eps, workgroups, workgroups > groups * kv_heads ? workgroups / (groups * kv_heads) : 1};
     dim3 grid(groups, kv_heads, max_splits);
     switch (head_dim / 32) {
         case 2: return page_size == 16 ? launch_decode_fused<2, 16>(grid, a, group_row0, group_ntok, f, stream) : launch_decode_fused<2, 0>(grid, a, group_row0, group_ntok, f, stream);
@@ -1569,7 +1606,7 @@ extern "C" int mlr_attention_mfma(
     if ((max_splits > 1 ? split_keys / page_size + 2 : max_blocks) > DECODE_PAGE_CACHE) return -3;
     AttnArgs a{(const elem_t*)q, (const elem_t*)k_pages, (const elem_t*)v_pages, block_table, slots,
                positions, (elem_t*)out, partial, max_blocks, q_heads, kv_heads, head_dim, page_size,
-               window, split_keys, max_splits < 1 ? 1 : max_splits, scale};
+               window, split_keys, max_splits < 1 ? 1 : max_splits, scale, q_heads / kv_heads};
     dim3 grid(groups, kv_heads, a.max_splits);
     const size_t lds = sizeof(float) * 3 * (16 * (size_t)head_dim + 32);
     const int nch = (head_dim + 31) / 32;
