@@ -888,8 +888,8 @@ __global__ __launch_bounds__(256, (NCH <= 4 ? 2 : 1)) void attention_mfma_kernel
                 x[c][e] = (float)q_raw[c][e];
                 sq += x[c][e] * x[c][e];
             }
-        sq += __shfl_xor(sq, 16, MLR_WAVE);
-        sq += __shfl_xor(sq, 32, MLR_WAVE);
+        sq = xor_sum<16>(sq);
+        sq = xor_sum<32>(sq);
         if (f.q_norm_w) {
             const float scale = 1.0f / sqrtf(sq / (float)D + f.eps);
 #pragma unroll
@@ -1008,8 +1008,8 @@ __global__ __launch_bounds__(256, (NCH <= 4 ? 2 : 1)) void attention_mfma_kernel
         }
         float tile_max = fmaxf(fmaxf(fmaxf(sv[0][0], sv[0][1]), fmaxf(sv[0][2], sv[0][3])),
                                fmaxf(fmaxf(sv[1][0], sv[1][1]), fmaxf(sv[1][2], sv[1][3])));
-        tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16, MLR_WAVE));
-        tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, MLR_WAVE));
+        tile_max = xor_max<16>(tile_max);
+        tile_max = xor_max<32>(tile_max);
         // the running maximum rarely moves after the first tiles: rescale only when it does, for any column
         if (__builtin_amdgcn_ballot_w64(tile_max > m_run) != 0) {
             const float m_new = fmaxf(m_run, tile_max);
@@ -1074,8 +1074,8 @@ __global__ __launch_bounds__(256, (NCH <= 4 ? 2 : 1)) void attention_mfma_kernel
         }
     }
     // per column: the four lane blocks hold partial sums of the same column
-    l_run += __shfl_xor(l_run, 16, MLR_WAVE);
-    l_run += __shfl_xor(l_run, 32, MLR_WAVE);
+    l_run = xor_sum<16>(l_run);
+    l_run = xor_sum<32>(l_run);
 
     if constexpr (FUSED) {
         // every wavefront parks the sums of the g columns in LDS and all threads add them in the order 0..3, a channel each
@@ -1393,8 +1393,8 @@ __device__ __forceinline__ void prefill_group(const AttnArgs& a, const int32_t* 
         }
         float tile_max = fmaxf(fmaxf(fmaxf(sv[0][0], sv[0][1]), fmaxf(sv[0][2], sv[0][3])),
                                fmaxf(fmaxf(sv[1][0], sv[1][1]), fmaxf(sv[1][2], sv[1][3])));
-        tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16, MLR_WAVE));
-        tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, MLR_WAVE));
+        tile_max = xor_max<16>(tile_max);
+        tile_max = xor_max<32>(tile_max);
         // the running maximum rarely moves after the first tiles: rescale only when it does, for any column
         if (__builtin_amdgcn_ballot_w64(tile_max > m_run) != 0) {
             const float m_new = fmaxf(m_run, tile_max);
@@ -1457,8 +1457,8 @@ __device__ __forceinline__ void prefill_group(const AttnArgs& a, const int32_t* 
         compute(t + 2, buf);
         buf ^= 1;
     }
-    l_run += __shfl_xor(l_run, 16, MLR_WAVE);
-    l_run += __shfl_xor(l_run, 32, MLR_WAVE);
+    l_run = xor_sum<16>(l_run);
+    l_run = xor_sum<32>(l_run);
     if (!col_valid) return;
     __bf16* dst = reinterpret_cast<__bf16*>(a.out) + ((size_t)(row0 + tok) * a.q_heads + kvh * g + hh) * D;
 #pragma unroll

@@ -84,15 +84,57 @@ template <typename V> __device__ __forceinline__ V turned(const V& v) {
     return V{__uint_as_float(r[0]), __uint_as_float(r[1]), __uint_as_float(r[2]), __uint_as_float(r[3])};
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, MLR_WAVE);
+// Values of other lanes without a trip through LDS, which a `__shfl_xor` is (a sum over a wavefront is a chain of six; one token of
+// the 0.6B sizes 1019 -> 1000 us a step, the float engine through the scheduler 32.3 -> 32.05 ms, Pamunex 2.55 -> 2.515):
+// the lane i ^ OFF within 16 lanes by DPP; across rows of 16 both operands of a swap, of which one is the lane's own value and the
+// other its partner's -- which is which does not matter to a sum or a maximum.  All lanes of the wavefront take part.
+template <int OFF> __device__ __forceinline__ float row_xor(float v) {
+    static_assert(OFF == 1 || OFF == 2 || OFF == 4 || OFF == 8, "within 16 lanes");
+    const int x = __float_as_int(v);
+    if (OFF == 4) {                                       // lanes 0-3 and 8-11 from four up, the others from four down
+        const int up = __builtin_amdgcn_update_dpp(x, x, 0x104, 0xf, 0x5, false);
+        return __int_as_float(__builtin_amdgcn_update_dpp(up, x, 0x114, 0xf, 0xa, false));
+    }
+    constexpr int CTRL = OFF == 1 ? 0xb1 : OFF == 2 ? 0x4e : 0x128;         // quad_perm [1, 0, 3, 2], [2, 3, 0, 1], row_ror:8
+    return __int_as_float(__builtin_amdgcn_update_dpp(x, x, CTRL, 0xf, 0xf, false));
+}
+struct lane_pair { float a, b; };
+template <int OFF> __device__ __forceinline__ lane_pair xor_pair(float v) {
+    const unsigned x = __float_as_uint(v);
+    if constexpr (OFF == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+        return {__uint_as_float(r[0]), __uint_as_float(r[1])};
+    } else if constexpr (OFF == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+        return {__uint_as_float(r[0]), __uint_as_float(r[1])};
+    } else {
+        return {v, row_xor<OFF>(v)};
+    }
+}
+template <int OFF> __device__ __forceinline__ float xor_sum(float v) { const lane_pair p = xor_pair<OFF>(v); return p.a + p.b; }
+template <int OFF> __device__ __forceinline__ float xor_max(float v) { const lane_pair p = xor_pair<OFF>(v); return fmaxf(p.a, p.b); }
+// The sum of groups of `lanes` (a power of two) neighbouring lanes, added from the nearest partner to the farthest.
+__device__ __forceinline__ float group_sum(float v, int lanes) {
+    if (lanes > 1) v = xor_sum<1>(v);
+    if (lanes > 2) v = xor_sum<2>(v);
+    if (lanes > 4) v = xor_sum<4>(v);
+    if (lanes > 8) v = xor_sum<8>(v);
+    if (lanes > 16) v = xor_sum<16>(v);
+    if (lanes > 32) v = xor_sum<32>(v);
     return v;
 }
+
+// The sum of the lanes FROM, 2 FROM, .. apart, likewise.
+template <int FROM> __device__ __forceinline__ float far_sum(float v) {
+    if constexpr (FROM < 64) return far_sum<2 * FROM>(xor_sum<FROM>(v));
+    else return v;
+}
+
+__device__ __forceinline__ float wave_sum(float v) {
+    return xor_sum<1>(xor_sum<2>(xor_sum<4>(xor_sum<8>(xor_sum<16>(xor_sum<32>(v))))));
+}
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, MLR_WAVE));
-    return v;
+    return xor_max<1>(xor_max<2>(xor_max<4>(xor_max<8>(xor_max<16>(xor_max<32>(v))))));
 }
 
 // Sum over a workgroup of up to 1024 threads (a multiple of 64); every thread gets the

@@ -543,8 +543,8 @@ __device__ __forceinline__ void diff_tiles_group(const DiffArgs& a, const int32_
             }
             float tile_max = fmaxf(fmaxf(fmaxf(sv[0][0], sv[0][1]), fmaxf(sv[0][2], sv[0][3])),
                                    fmaxf(fmaxf(sv[1][0], sv[1][1]), fmaxf(sv[1][2], sv[1][3])));
-            tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16, MLR_WAVE));
-            tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, MLR_WAVE));
+            tile_max = xor_max<16>(tile_max);
+            tile_max = xor_max<32>(tile_max);
             // (the running maximum rarely moves after the first tiles: rescale only when it does, for any column)
             if (__builtin_amdgcn_ballot_w64(tile_max > m_run[map]) != 0) {
                 const float m_new = fmaxf(m_run[map], tile_max);
@@ -600,8 +600,8 @@ __device__ __forceinline__ void diff_tiles_group(const DiffArgs& a, const int32_
     }
 #pragma unroll
     for (int map = 0; map < 2; ++map) {
-        l_run[map] += __shfl_xor(l_run[map], 16, MLR_WAVE);
-        l_run[map] += __shfl_xor(l_run[map], 32, MLR_WAVE);
+        l_run[map] = xor_sum<16>(l_run[map]);
+        l_run[map] = xor_sum<32>(l_run[map]);
     }
     if (a.partial != nullptr) {
         // (max, sum, weighted values) of this key range, the maximum back in the natural domain
@@ -637,8 +637,8 @@ __device__ __forceinline__ void diff_tiles_group(const DiffArgs& a, const int32_
             ss += d * d;
         }
     }
-    ss += __shfl_xor(ss, 16, MLR_WAVE);
-    ss += __shfl_xor(ss, 32, MLR_WAVE);
+    ss = xor_sum<16>(ss);
+    ss = xor_sum<32>(ss);
     if (!col_valid) return;
     const float unit = a.out_scale / sqrtf(ss / (float)V + a.eps);
     __bf16* dst = reinterpret_cast<__bf16*>(a.out) + ((size_t)(row0 + tok) * a.q_heads + head) * V;

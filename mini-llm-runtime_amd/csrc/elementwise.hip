@@ -795,7 +795,7 @@ __global__ __launch_bounds__(256) void gated_part_norm_reg_kernel(const float* _
         }
     }
     if (BLOCK) sum = block_sum(sum, scratch);
-    else for (int d = 1; d < group; d <<= 1) sum += __shfl_xor(sum, d, MLR_WAVE);
+    else sum = group_sum(sum, group);
     const float scale = 1.0f / sqrtf(sum / (float)part + eps);
 #pragma unroll
     for (int i = 0; i < PART_CHUNKS; ++i) {

@@ -673,8 +673,8 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const __
             for (int j = 0; j < 4; ++j)
                 ss_mine += j < ss_run && pair * ss_run + j < ss_quads ? (ss4[j].x + ss4[j].y) + (ss4[j].z + ss4[j].w) : 0.f;
         }
-        ss_mine += __shfl_xor(ss_mine, 16, MLR_WAVE);
-        ss_mine += __shfl_xor(ss_mine, 32, MLR_WAVE);
+        ss_mine = xor_sum<16>(ss_mine);
+        ss_mine = xor_sum<32>(ss_mine);
         if (b == 0) ss_lds[wave][r16] = ss_mine;
     }
     __syncthreads();
@@ -777,10 +777,10 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const __
                 }
             }
             if (epi.next_w) {
-                sq += __shfl_xor(sq, 16, MLR_WAVE);
-                sq += __shfl_xor(sq, 32, MLR_WAVE);
-                sq2 += __shfl_xor(sq2, 16, MLR_WAVE);
-                sq2 += __shfl_xor(sq2, 32, MLR_WAVE);
+                sq = xor_sum<16>(sq);
+                sq = xor_sum<32>(sq);
+                sq2 = xor_sum<16>(sq2);
+                sq2 = xor_sum<32>(sq2);
                 if (b == 0 && row_ok) {
                     // a workgroup a part; the parts beyond the workgroups, up to the buffer's capacity, are zero
                     float* parts = epi.ss_out + (size_t)r16 * epi.ss_stride;
@@ -791,8 +791,8 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const __
             return;
         }
         if (epi.next_w) {
-            sq += __shfl_xor(sq, 16, MLR_WAVE);            // (0 + 1) + (2 + 3) over the lane blocks: the strip's 16 columns
-            sq += __shfl_xor(sq, 32, MLR_WAVE);
+            sq = xor_sum<16>(sq);            // (0 + 1) + (2 + 3) over the lane blocks: the strip's 16 columns
+            sq = xor_sum<32>(sq);
             if (b == 0 && row_ok) epi.ss_out[(size_t)r16 * gridDim.x + blockIdx.x] = sq;
         }
         return;
@@ -1392,8 +1392,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const std::c
                         b[e] = (float)hi[e];
                         sum += squares(a[e], b[e]);
                     }
-#pragma unroll
-                    for (int off = 1; off < LANES; off <<= 1) sum += __shfl_xor(sum, off, MLR_WAVE);
+                    sum = group_sum(sum, LANES);
                     if (normed) {
                         const float scale = 1.0f / sqrtf(sum / (float)QKV_HEAD + args.eps);
 #pragma unroll

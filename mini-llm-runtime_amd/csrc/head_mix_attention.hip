@@ -341,8 +341,7 @@ __device__ __forceinline__ void head_scores(const HeadMixArgs& a, const TileArgs
 #pragma unroll
         for (int x = 0; x < 4; ++x) {
             float v = sums[r][x];
-#pragma unroll
-            for (int off = 1; off < 16; off <<= 1) v += __shfl_xor(v, off, MLR_WAVE);
+            v = group_sum(v, 16);
             if (i16 == 0) sum_lds[wave][r * 16 + 4 * b + x] = v;
         }
     __syncthreads();

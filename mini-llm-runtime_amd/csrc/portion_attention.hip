@@ -256,7 +256,7 @@ __global__ __launch_bounds__(128 * NQ, ND > 8 && NQ == 2 ? 1 : 2) void portion_a
         mx = max3(mx, max3(sc[9], sc[10], sc[11]), max3(sc[12], sc[13], sc[14]));
         mx = fmaxf(mx, sc[15]) * c2;                                   // c2 > 0
         if (__builtin_amdgcn_ballot_w64(mx > m_ref + RAISE_BY) != 0) {
-            const float full = fmaxf(mx, __shfl_xor(mx, 32, 64));     // the column's maximum in this tile
+            const float full = xor_max<32>(mx);     // the column's maximum in this tile
             if (full > m_ref + RAISE_BY) {
                 const float corr = __builtin_amdgcn_exp2f(m_ref - full);      // -inf - finite: 0
                 l_run *= corr;
@@ -298,7 +298,7 @@ __global__ __launch_bounds__(128 * NQ, ND > 8 && NQ == 2 ? 1 : 2) void portion_a
     }
 
     // the two key parities; the sink; the division
-    l_run += __shfl_xor(l_run, 32, 64);
+    l_run = xor_sum<32>(l_run);
     __syncthreads();
     float* mine = merge_lds + (size_t)cq * S::NO * 64 + lane;
     if (kp == 1) {

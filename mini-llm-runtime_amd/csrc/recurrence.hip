@@ -425,11 +425,8 @@ __global__ __launch_bounds__(64) void delta_rule_kernel(DeltaArgs a) {
                 sk += kt[r] * S[r];
                 sq += qt[r] * S[r];
             }
-#pragma unroll
-            for (int off = COLS; off < 64; off <<= 1) {   // the parts of a column lie COLS lanes apart
-                sk += __shfl_xor(sk, off, 64);
-                sq += __shfl_xor(sq, off, 64);
-            }
+            sk = far_sum<COLS>(sk);                       // the parts of a column lie COLS lanes apart
+            sq = far_sum<COLS>(sq);
             const float u = beta_lds[t] * (v_lds[t * COLS + j] - sk);
 #pragma unroll
             for (int r = 0; r < NR; ++r) S[r] += kt[r] * u;

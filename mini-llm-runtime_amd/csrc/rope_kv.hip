@@ -255,7 +255,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kv_vec_kernel(
         b[e] = (float)hi8[e];
         sum += squares(a[e], b[e]);
     }
-    for (int off = 1; off < lph; off <<= 1) sum += __shfl_xor(sum, off, MLR_WAVE);
+    sum = group_sum(sum, lph);
     if (!active) return;
     const bool cache_ok = write_cache && page >= 0;
     const size_t cache_page = (size_t)(page < 0 ? 0 : page) * kv_heads;

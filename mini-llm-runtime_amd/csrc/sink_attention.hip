@@ -354,7 +354,7 @@ __global__ __launch_bounds__(256) void sink_qkv_prep_vec_kernel(
         float sum = 0.f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) sum += x[e] * x[e];
-        for (int d = 1; d < lanes; d <<= 1) sum += __shfl_xor(sum, d, MLR_WAVE);
+        sum = group_sum(sum, lanes);
         const float r = 1.0f / sqrtf(sum / (float)key_dim + eps);
         const float* w = unit < q_heads ? q_norm_w : k_norm_w;
         float f[8] = {1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f};
@@ -371,7 +371,7 @@ __global__ __launch_bounds__(256) void sink_qkv_prep_vec_kernel(
         float sum = 0.f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) sum += x[e] * x[e];
-        for (int d = 1; d < lanes; d <<= 1) sum += __shfl_xor(sum, d, MLR_WAVE);
+        sum = group_sum(sum, lanes);
         const float r = 1.0f / sqrtf(sum / (float)key_dim + eps);
         const float* w = unit < q_heads ? q_norm_w : k_norm_w;
         float f[8] = {1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f};
@@ -510,8 +510,8 @@ struct SinkColumn {
         float tile_max = -INFINITY;
 #pragma unroll
         for (int e = 0; e < 8; ++e) tile_max = fmaxf(tile_max, sc[e]);
-        tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16, MLR_WAVE));
-        tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, MLR_WAVE));
+        tile_max = xor_max<16>(tile_max);
+        tile_max = xor_max<32>(tile_max);
         const float new_max = fmaxf(run_max, tile_max);
         // (the raw exponential instruction: its arguments are at most 0, and what underflows may be 0)
         const float corr = new_max > -INFINITY ? __builtin_amdgcn_exp2f(run_max - new_max) : 1.f;
@@ -522,8 +522,8 @@ struct SinkColumn {
             part += p;
             pf[e] = (__bf16)p;
         }
-        part += __shfl_xor(part, 16, MLR_WAVE);
-        part += __shfl_xor(part, 32, MLR_WAVE);
+        part = xor_sum<16>(part);
+        part = xor_sum<32>(part);
         run_sum = run_sum * corr + part;
         run_max = new_max;
         return corr;
