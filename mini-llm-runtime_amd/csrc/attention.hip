@@ -795,7 +795,10 @@ __global__ __launch_bounds__(256, (NCH <= 4 ? 2 : 1)) void attention_mfma_kernel
     // (FUSED: group i is the one token in batch row i; no need to wait for the group vectors)
     const int row0 = FUSED ? grp : group_row0[grp], ntok = FUSED ? 1 : group_ntok[grp];
     int slot = a.slots[row0], pos0 = a.positions[row0];
-    asm volatile("" : "+s"(slot), "+s"(pos0));                         // (asked for together)
+    // (asked for together, the other arguments with them and not as each is first needed)
+    if constexpr (FUSED)
+        asm volatile("" : "+s"(slot), "+s"(pos0) : "s"(a.block_table), "s"(a.max_blocks), "s"(a.kv_heads), "s"(f.qkv), "s"(f.q_norm_w), "s"(f.rope), "s"(f.ld), "s"(f.share));
+    else asm volatile("" : "+s"(slot), "+s"(pos0));
     const int tok = FUSED ? col >= g : col / g, hh = FUSED ? col : col % g;       // (FUSED: of columns beyond the heads, never used)
     const bool col_valid = tok < ntok;
     const int kend_full = col_valid ? pos0 + tok + 1 : 0;
@@ -880,14 +883,15 @@ __global__ __launch_bounds__(256, (NCH <= 4 ? 2 : 1)) void attention_mfma_kernel
         // 32 NCH, NCH even, the partner d + head_dim / 2 of a channel is in chunk c + NCH / 2 of the same
         // lane), rounded to bfloat16 as the cache's keys are
         float x[NCH][8];
-        float sq = 0.f;
+        float sqs[4] = {0.f, 0.f, 0.f, 0.f};                      // (four short chains instead of one)
 #pragma unroll
         for (int c = 0; c < NCH; ++c)
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 x[c][e] = (float)q_raw[c][e];
-                sq += x[c][e] * x[c][e];
+                sqs[e % 4] += x[c][e] * x[c][e];
             }
+        float sq = (sqs[0] + sqs[1]) + (sqs[2] + sqs[3]);
         sq = xor_sum<16>(sq);
         sq = xor_sum<32>(sq);
         if (f.q_norm_w) {
@@ -946,8 +950,9 @@ __global__ __launch_bounds__(256, (NCH <= 4 ? 2 : 1)) void attention_mfma_kernel
             const scalar_ptr scalars = (scalar_ptr)table;
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                const int id = scalars[min(max(2 * t + j, 0), a.max_blocks - 1)];
-                r.at[j] = t * MFMA_TILE_KEYS + 16 * j < hi && 2 * t + j < a.max_blocks ? id : -1;
+                int none = __builtin_amdgcn_readfirstlane(t * MFMA_TILE_KEYS + 16 * j < hi && 2 * t + j < a.max_blocks ? 0 : -1);
+                asm("" : "+s"(none));                             // (else the load comes behind a branch, and its answer before the next one's)
+                r.at[j] = scalars[min(max(2 * t + j, 0), a.max_blocks - 1)] | none;
             }
         }
         return r;
@@ -1056,8 +1061,9 @@ __global__ __launch_bounds__(256, (NCH <= 4 ? 2 : 1)) void attention_mfma_kernel
         KvTile<NCH> ta, tb2;
         int t = t_begin + wave;
         const int t_last = t + ((t_end - 1 - t) / 4) * 4;
+        const Ids first = ids(t);
         Ids next = ids(min(t + 4, t_last));
-        if (t < t_end) load(t, ta, ids(t));
+        if (t < t_end) load(t, ta, first);
         if (FUSED) finish_queries();
         if (t < t_end) {
             for (;;) {
