@@ -578,16 +578,24 @@ struct Routing {
 // all others, where one choice after the other took six exchanges between lanes each, and one group for all needs no rounds.
 // 48 tokens, 4 of 20 experts: 7.8 -> 3.4 us; 8 of 64 in 4 of 8 groups 11.6 -> 4.6, of 256 14.7 -> 10.4; 1777 tokens, 4 of 16: 8.7 -> 3.6.
 // (The choice and the sort below in one launch of one workgroup, three tokens a wavefront: 10.7 us for 3.4 and 2.0.)
+// zr: the token's logits; one wavefront (WAVES 1) needs no other one of its workgroup.
 template <int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void router_topk_kernel(const float* __restrict__ z, long ld, Routing r,
-                                                                 int32_t* __restrict__ ids, float* __restrict__ weights) {
+__device__ __forceinline__ void choose_experts(const float* zr, const Routing& r, int32_t* __restrict__ ids, float* __restrict__ weights) {
+    auto sync = []() {
+        if (WAVES > 1) {
+            __syncthreads();
+        } else {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+    };
     __shared__ __attribute__((aligned(16))) int keys[64 * WAVES];
     __shared__ float by[64 * WAVES];                                       // what the choice goes by
     __shared__ float plain[64 * WAVES];                                    // the plain scores
     __shared__ float group[64 * WAVES];
     __shared__ int choice[64 * WAVES];
     const int e = threadIdx.x, experts = r.experts, lane = e % 64;
-    const float* zr = z + (size_t)blockIdx.x * ld;
     const bool expert = e < experts;
     const float logit = expert ? zr[e] : 0.f;
     float z_max = 0.f, z_sum = 1.f, cand = -INFINITY;
@@ -612,7 +620,7 @@ __global__ __launch_bounds__(64 * WAVES) void router_topk_kernel(const float* __
         if (there < (per >= 2 && !r.group_best ? 2 : 1)) cand = -INFINITY;
     } else {
         by[e] = cand;
-        __syncthreads();
+        sync();
         if (e < r.group_count) {
             float first = -INFINITY, second = -INFINITY;
             for (int i = 0; i < per; ++i) {
@@ -626,7 +634,7 @@ __global__ __launch_bounds__(64 * WAVES) void router_topk_kernel(const float* __
             }
             group[e] = per >= 2 && !r.group_best ? first + second : first;
         }
-        __syncthreads();
+        sync();
         if (expert) {
             const int mine = e / per;
             const float score = group[mine];
@@ -644,7 +652,7 @@ __global__ __launch_bounds__(64 * WAVES) void router_topk_kernel(const float* __
     const int bits = __float_as_int(cand + 0.0f);                          // (0 for -0)
     const int key = cand > -INFINITY ? bits ^ ((bits >> 31) & 0x7fffffff) : NONE;
     keys[e] = key;
-    __syncthreads();
+    sync();
     int before = 0;
     for (int j = 0; j < experts; j += 16) {                                // (16 at once: their reads are under way together)
         int4 v[4];
@@ -660,7 +668,7 @@ __global__ __launch_bounds__(64 * WAVES) void router_topk_kernel(const float* __
         }
     }
     if (key != NONE && before < r.top) choice[before] = e;
-    __syncthreads();
+    sync();
     if (e >= r.top) return;
     const int which = choice[e];
     float w = plain[which];
@@ -672,6 +680,71 @@ __global__ __launch_bounds__(64 * WAVES) void router_topk_kernel(const float* __
     ids[(size_t)blockIdx.x * r.top + e] = which;
     weights[(size_t)blockIdx.x * r.top + e] = r.renorm || r.out_scale != 1.0f ? w * r.out_scale : w;
 }
+
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void router_topk_kernel(const float* __restrict__ z, long ld, Routing r,
+                                                                 int32_t* __restrict__ ids, float* __restrict__ weights) {
+    choose_experts<WAVES>(z + (size_t)blockIdx.x * ld, r, ids, weights);
+}
+
+#if MLR_BF16
+// The router's product with the choice behind it: a token a workgroup, z[e] = x . w[e] for all `outputs` rows of w (the experts, and
+// beyond them a shared expert's gate) in 32-bit, written to z and chosen from.  Eight wavefronts take every eighth row, a lane eight
+// neighbouring channels of every 512, in the order of the channels, and the lanes' sums by halves (`wave_sum`): a token's logits do
+// not depend on the others.
+// Bound by its chain of trips -- row and weights, the lanes' sums, the choice -- where the product alone was a launch of two or three
+// workgroups.  48 tokens, 20 outputs of 2048 channels 7.6 -> 4.3 us, 732 tokens, 8 outputs 8.9 -> 5.1, 1777 tokens 9.0 -> 7.0 (in a
+// model, where the product finds its operands elsewhere, 12.4, 15.9 and 15.6 before).
+#define ROUTER_OUTPUTS 128
+#define ROUTER_WAVES 8
+template <int AT_ONCE>          // rows of w a wavefront takes side by side
+__global__ __launch_bounds__(64 * ROUTER_WAVES) void router_kernel(const __bf16* __restrict__ x, const __bf16* __restrict__ w,
+                                                                   float* __restrict__ z, long ld, int width, int outputs, Routing r,
+                                                                   int32_t* __restrict__ ids, float* __restrict__ weights) {
+    typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
+    struct eight { bf16x2 pair[4]; };
+    __shared__ float z_lds[ROUTER_OUTPUTS];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const __bf16* row = x + (size_t)blockIdx.x * width;
+    constexpr int AHEAD = 4;
+    for (int e0 = wave; e0 < outputs; e0 += ROUTER_WAVES * AT_ONCE) {
+        float sum[AT_ONCE] = {};
+        for (int c0 = 0; c0 < width; c0 += 512 * AHEAD) {
+            vec16 v[AHEAD], u[AT_ONCE][AHEAD];
+#pragma unroll
+            for (int q = 0; q < AHEAD; ++q) {                              // (clamped: no branch around a load)
+                const int at = min(c0 + 512 * q + 8 * lane, width - 8);
+                v[q] = *reinterpret_cast<const vec16*>(row + at);
+#pragma unroll
+                for (int j = 0; j < AT_ONCE; ++j)
+                    u[j][q] = *reinterpret_cast<const vec16*>(w + (size_t)min(e0 + ROUTER_WAVES * j, outputs - 1) * width + at);
+            }
+#pragma unroll
+            for (int q = 0; q < AHEAD; ++q) {
+                if (c0 + 512 * q + 8 * lane >= width) v[q] = vec16{{0, 0, 0, 0}};
+                const eight a = __builtin_bit_cast(eight, v[q]);
+#pragma unroll
+                for (int j = 0; j < AT_ONCE; ++j) {
+                    // (an expert that is not finite does not reach a token through channels that are not there)
+                    if (c0 + 512 * q + 8 * lane >= width) u[j][q] = vec16{{0, 0, 0, 0}};
+                    const eight b = __builtin_bit_cast(eight, u[j][q]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) sum[j] = __builtin_amdgcn_fdot2_f32_bf16(a.pair[e], b.pair[e], sum[j], false);
+                }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < AT_ONCE; ++j) {
+            const float total = wave_sum(sum[j]);
+            if (lane == 0 && e0 + ROUTER_WAVES * j < outputs) z_lds[e0 + ROUTER_WAVES * j] = total;
+        }
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    for (int e = lane; e < outputs; e += 64) z[(size_t)blockIdx.x * ld + e] = z_lds[e];
+    choose_experts<1>(z_lds, r, ids, weights);
+}
+#endif
 
 // The same, one choice after the other, a wavefront a token: a round is six exchanges between the lanes' best.
 // The largest value among the lanes' candidates and, among equals, the lowest index; every lane gets both.
@@ -954,6 +1027,28 @@ int mlr_router_topk(const float* z, long ld, int32_t* ids, float* weights, int r
     else if (experts <= 64) router_topk_kernel<1><<<rows, 64, 0, stream>>>(z, ld, r, ids, weights);
     else router_topk_kernel<4><<<rows, 256, 0, stream>>>(z, ld, r, ids, weights);
     return (int)hipGetLastError();
+}
+
+// z = x . w^T (bfloat16, `outputs` rows of w, float sums) and the choice of `mlr_router_topk` from its first `experts` columns, in one
+// launch; 1 where it does not take the sizes (more than 64 experts, rows that do not come in 16 bytes): nothing was launched.
+int mlr_router(const void* x, const void* w, float* z, long ld, int32_t* ids, float* weights, int rows, int width, int outputs, int experts,
+               int top, int group_count, int group_keep, const float* correction, int renorm, float out_scale, int softmax, int group_best,
+               hipStream_t stream) {
+#if MLR_BF16
+    if (rows <= 0) return 0;
+    if (outputs < experts || ld < outputs || experts < 1 || group_count < 1 || experts % group_count != 0 || group_keep < 1 ||
+        group_keep > group_count || top < 1 || top > group_keep * (experts / group_count))
+        return -1;
+    if (experts > 64 || outputs > ROUTER_OUTPUTS || width < 8 || width % 8 != 0 ||
+        ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) != 0)
+        return 1;
+    const Routing r{experts, top, group_count, group_keep, renorm, softmax, group_best, correction, out_scale};
+    auto* kernel = outputs <= ROUTER_WAVES ? router_kernel<1> : outputs <= 2 * ROUTER_WAVES ? router_kernel<2> : router_kernel<3>;
+    kernel<<<rows, 64 * ROUTER_WAVES, 0, stream>>>((const __bf16*)x, (const __bf16*)w, z, ld, width, outputs, r, ids, weights);
+    return (int)hipGetLastError();
+#else
+    return 1;
+#endif
 }
 
 int mlr_route_sort(const int32_t* ids, int pairs, int top, int experts, int32_t* offsets, int32_t* token_of,

@@ -2287,6 +2287,44 @@ class Kernels:
             _c_int(group_count), _c_int(group_keep), _p(correction), _c_int(1 if renormalize else 0), _c_float(scale),
             _c_int(self.ROUTER_SCORES[score]), _c_int(self.ROUTER_GROUPS[group_score]), _stream()), "router_topk")
 
+    # rows x outputs x channels, and outputs x channels (every token reads the weight again): one launch and two, us, 1777 tokens of 8 x
+    # 2048 7.0, 9.0, of 8 x 4096 10.4, 9.9; 2048 of 16 x 2048 9.0, 7.9; 48 of 64 x 2048 7.2, 8.2, of 64 x 4096 10.2, 9.8
+    ROUTER_FUSED_WORK, ROUTER_FUSED_WEIGHT = 1 << 25, 1 << 17
+
+    def router(self, x, w, logits, ids, weights, group_count=1, group_keep=1, correction=None, renormalize=False, scale=1.0,
+               score="sigmoid", group_score="best_two", experts=None):
+        """logits = x . w^T in 32-bit sums and the choice of `router_topk` from its first `experts` columns: one launch while the
+        product is small (`ROUTER_FUSED_WORK`, `ROUTER_FUSED_WEIGHT`), two otherwise."""
+        rows, width = x.shape
+        outputs = logits.shape[1]
+        experts = outputs if experts is None else experts
+        top = ids.shape[1]
+        if self.dtype == torch.bfloat16 and rows * outputs * width <= self.ROUTER_FUSED_WORK and outputs * width <= self.ROUTER_FUSED_WEIGHT and experts <= 64 and outputs <= 128 and \
+                width % 8 == 0 and _on16(x, w):
+            _tensor(x, "x", self.dtype, ndim=2)
+            _tensor(w, "w", self.dtype, (outputs, width))
+            _tensor(logits, "logits", torch.float32, (rows, outputs))
+            _need(score in self.ROUTER_SCORES and group_score in self.ROUTER_GROUPS, f"router: {score!r}, {group_score!r}")
+            if correction is not None:
+                _tensor(correction, "correction", torch.float32, (experts,))
+            _tensor(ids, "ids", torch.int32, (rows, top))
+            _tensor(weights, "weights", torch.float32, (rows, top))
+            self._router_launch(x, w, logits, ids, weights, experts, group_count, group_keep, correction, renormalize, scale,
+                                self.ROUTER_SCORES[score], self.ROUTER_GROUPS[group_score])
+            return
+        self.gemm(x, w, logits)
+        self.router_topk(logits, ids, weights, group_count, group_keep, correction=correction, renormalize=renormalize, scale=scale,
+                         score=score, group_score=group_score, experts=experts)
+
+    @timed("gemm")
+    def _router_launch(self, x, w, logits, ids, weights, experts, group_count, group_keep, correction, renormalize, scale, score, group_score):
+        rows, width = x.shape
+        outputs, top = logits.shape[1], ids.shape[1]
+        _ok(self._lib("grouped_gemm").mlr_router(
+            _p(x), _p(w), _p(logits), ctypes.c_long(outputs), _p(ids), _p(weights), _c_int(rows), _c_int(width), _c_int(outputs), _c_int(experts),
+            _c_int(top), _c_int(group_count), _c_int(group_keep), _p(correction), _c_int(1 if renormalize else 0), _c_float(scale),
+            _c_int(score), _c_int(group_score), _stream()), "router")
+
     @timed("gemm")
     def route_sort(self, ids, experts, offsets, token_of, row_of):
         """The (token, choice) pairs of ids [rows, top] sorted by expert: offsets int32 [experts + 1], token_of

@@ -129,10 +129,9 @@ class RoutedMlp:
         token_of = ws.get("route_token", (pairs,), torch.int32)
         row_of = ws.get("route_row", (pairs,), torch.int32)
         logits = ws.get("route_logits", (m, self.router.shape[0]), torch.float32)
-        k.gemm(x, self.router, logits)                   # 32-bit sums of the engine's element type's products
-        k.router_topk(logits, ids, weights, s.group_count, s.group_keep, correction=self.correction,
-                      renormalize=bool(s.renormalize), scale=float(getattr(s, "route_scale", 1.0)), score=s.score,
-                      group_score=s.group_score, experts=self.choices)
+        k.router(x, self.router, logits, ids, weights, s.group_count, s.group_keep, correction=self.correction,
+                 renormalize=bool(s.renormalize), scale=float(getattr(s, "route_scale", 1.0)), score=s.score,
+                 group_score=s.group_score, experts=self.choices)      # (32-bit sums of the engine's element type's products)
         k.route_sort(ids, self.choices, offsets, token_of, row_of)
         offsets = offsets[:s.experts + 1]                # (the pairs of experts without tensors lie behind the others')
         act = ws.get("route_act", (pairs, s.intermediate), x.dtype)
