@@ -631,6 +631,8 @@ __device__ __forceinline__ void tile_group(const TileArgs& a, int grp, int kvh, 
 // The merge of key splits: one wavefront per (group, head, token of the group), four a workgroup; a lane takes
 // the channels lane and lane + 64.  Splits are added in ascending order.  A token whose keys lay in one split
 // was finished by that split's workgroup.
+// Bound by its chain of loads: with one split after the other, its values asked for behind its weight, the merge of 33 tokens in 49
+// splits of 16 heads took 17.7 us, now 7.5.
 __global__ __launch_bounds__(256) void tiles_combine_kernel(TileArgs a) {
     const int grp = blockIdx.x, head = blockIdx.y, j = blockIdx.z * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
@@ -648,14 +650,31 @@ __global__ __launch_bounds__(256) void tiles_combine_kernel(TileArgs a) {
     for (int off = 32; off > 0; off >>= 1) gmax = fmaxf(gmax, __shfl_xor(gmax, off, 64));
     const int d0 = min(lane, D - 1), d1 = min(lane + 64, D - 1);
     float den = 0.f, n0 = 0.f, n1 = 0.f;
-    for (int s = first; s <= last; ++s) {
-        const float* p = base + (size_t)s * (D + 4);
-        const float sm = p[D];
-        const float w = sm > -INFINITY ? __builtin_amdgcn_exp2f(sm - gmax) : 0.f;   // maxima are base-2 exponents
-        den += w * p[D + 1];
-        n0 += w * p[d0];
-        n1 += w * p[d1];
+    constexpr int AHEAD = 8;
+    for (int s0 = first; s0 <= last; s0 += 64) {         // a lane a split's weight, and eight splits' values under way
+        const float* mine = base + (size_t)min(s0 + lane, last) * (D + 4) + D;
+        const float sm = mine[0], sum = mine[1];
+        const float w = s0 + lane <= last && sm > -INFINITY ? __builtin_amdgcn_exp2f(sm - gmax) : 0.f;   // maxima are base-2 exponents
+        den += s0 + lane <= last ? w * sum : 0.f;
+        const int n = min(64, last + 1 - s0);
+        for (int u0 = 0; u0 < n; u0 += AHEAD) {
+            float v0[AHEAD], v1[AHEAD];
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) {            // (clamped: no branch around a load)
+                const float* p = base + (size_t)min(s0 + u0 + u, last) * (D + 4);
+                v0[u] = p[d0];
+                v1[u] = p[d1];
+            }
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) {
+                const float of = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), u0 + u));
+                n0 += of * v0[u];
+                n1 += of * v1[u];
+            }
+        }
     }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) den += __shfl_xor(den, off, 64);
     const float inv = den != 0.f ? 1.f / den : 0.f;
     __bf16* dst = a.out + ((size_t)m * a.q_heads + head) * D;
     if (lane < D) dst[lane] = (__bf16)(n0 * inv);
