@@ -49,6 +49,9 @@ struct DiffArgs {
     const int32_t* group_first; const int32_t* group_count; int group_tokens;
     int mask_kind, mask_size;                  // 0: every earlier key; 1: the last mask_size positions; 2: the query's block
     PageDivisor pages;                         // (of the matrix-core kernel)
+    // groups of ONE new token each, whose key and value are in no page yet (else null): rows of a projection, written by the launch
+    const elem_t* own_k; long own_k_stride;    // own_k[row * own_k_stride + kv_head * 2 * head_dim + d]
+    const elem_t* own_v; long own_v_stride;
 };
 
 #define MASK_NONE 0
@@ -416,22 +419,6 @@ __device__ __forceinline__ void diff_tiles_group(const DiffArgs& a, const int32_
     const int k_lo = a.max_splits > 1 ? max(split * a.split_keys, group_lo) : group_lo;
     const int k_hi = a.max_splits > 1 ? min(ke, (split + 1) * a.split_keys) : ke;
     if (k_lo >= k_hi) return;                         // (a range beyond the group's keys: the merge does not read it)
-    // page ids of the range first, so that a tile's loads do not wait for a load of the block table
-    const int first_page = k_lo / P;                  // (the page that holds key k_lo)
-    {
-        const int n_pages = min(TILES_PAGE_CACHE, (k_hi + P - 1) / P - first_page);
-        for (int i = threadIdx.x; i < n_pages; i += 256) page_lds[i] = first_page + i < a.max_blocks ? table[first_page + i] : -1;
-        __syncthreads();
-    }
-    // (no load from the block table here: a global load behind a branch makes the compiler wait for every load in
-    // flight, one tile's loads would then go out one after the other; the host keeps a range within the cache)
-    // (no branch between sizes that are powers of two and others)
-    auto block_of = [&](int kp) { return page_of_key(a.pages, kp); };
-    auto within = [&](int kp) { return kp - block_of(kp) * P; };
-    auto page_of = [&](int kp) {
-        const int page = page_lds[min(max(block_of(kp) - first_page, 0), TILES_PAGE_CACHE - 1)];
-        return kp < k_hi ? page : -1;
-    };
     // what a thread stages does not change from tile to tile
     constexpr int KST = NCH, VST = (NDB + 3) / 4;     // 16-byte chunks a thread stages per tile
     int k_key[KST], k_goff[KST], k_loff[KST], v_ch[VST], v_key[VST], v_loff[VST];
@@ -454,6 +441,36 @@ __device__ __forceinline__ void diff_tiles_group(const DiffArgs& a, const int32_
         v_key[i] = 8 * (ci & 3);
         v_loff[i] = (ci >> 2) * VPITCH + 8 * (ci & 3);
     }
+    // A new token's own key and value take their places on the way to LDS, whatever the pages hold there, and one workgroup a kv
+    // head writes them into the pages: a launch less a layer than with a kernel for that (4.7 us).  Asked for here, with the
+    // queries, and written at the end: between the fetches of the tiles either made them wait.
+    const bool own = a.own_k != nullptr && k_lo <= pos0 && pos0 < k_hi;
+    const __bf16* from_k = reinterpret_cast<const __bf16*>(a.own_k) + (size_t)row0 * a.own_k_stride + (size_t)kvh * (2 * D);
+    const __bf16* from_v = reinterpret_cast<const __bf16*>(a.own_v) + (size_t)row0 * a.own_v_stride + (size_t)kvh * V;
+    bf16x8 own_k[KST];
+    __bf16 own_v[VST];
+    if (own) {
+#pragma unroll
+        for (int i = 0; i < KST; ++i) own_k[i] = *reinterpret_cast<const bf16x8*>(from_k + k_goff[i]);
+#pragma unroll
+        for (int i = 0; i < VST; ++i) own_v[i] = from_v[v_ch[i]];
+    }
+    // page ids of the range first, so that a tile's loads do not wait for a load of the block table
+    const int first_page = k_lo / P;                  // (the page that holds key k_lo)
+    {
+        const int n_pages = min(TILES_PAGE_CACHE, (k_hi + P - 1) / P - first_page);
+        for (int i = threadIdx.x; i < n_pages; i += 256) page_lds[i] = first_page + i < a.max_blocks ? table[first_page + i] : -1;
+        __syncthreads();
+    }
+    // (no load from the block table here: a global load behind a branch makes the compiler wait for every load in
+    // flight, one tile's loads would then go out one after the other; the host keeps a range within the cache)
+    // (no branch between sizes that are powers of two and others)
+    auto block_of = [&](int kp) { return page_of_key(a.pages, kp); };
+    auto within = [&](int kp) { return kp - block_of(kp) * P; };
+    auto page_of = [&](int kp) {
+        const int page = page_lds[min(max(block_of(kp) - first_page, 0), TILES_PAGE_CACHE - 1)];
+        return kp < k_hi ? page : -1;
+    };
     struct Staged {                                   // one tile on its way: registers between memory and LDS
         bf16x8 k[KST], v[VST];
         int tb, ok;                                   // bit i: chunk i of the keys, bit 16 + i: of the values, is there
@@ -482,17 +499,20 @@ __device__ __forceinline__ void diff_tiles_group(const DiffArgs& a, const int32_
 #pragma unroll
         for (int i = 0; i < KST; ++i) {
             if (!k_mine[i]) continue;
-            *reinterpret_cast<bf16x8*>(&k_lds[k_loff[i]]) = ((st.ok >> i) & 1) ? st.k[i] : zero8;
+            const bf16x8 k = own && st.tb + k_key[i] == pos0 ? own_k[i] : st.k[i];
+            *reinterpret_cast<bf16x8*>(&k_lds[k_loff[i]]) = ((st.ok >> i) & 1) ? k : zero8;
         }
 #pragma unroll
         for (int i = 0; i < VST; ++i) {
             if (!v_mine[i]) continue;
             bf16x8 v = ((st.ok >> (16 + i)) & 1) ? st.v[i] : zero8;
             const int key0 = st.tb + v_key[i];
-            if (key0 + 8 > k_hi) {
+            if (key0 + 8 > k_hi || (own && key0 + 8 > pos0)) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e)           // keys that are not written yet count as zero
+                for (int e = 0; e < 8; ++e) {         // keys that are not written yet count as zero
+                    if (own && key0 + e == pos0 && ((st.ok >> (16 + i)) & 1)) v[e] = own_v[i];
                     if (key0 + e >= k_hi) v[e] = (__bf16)0.f;
+                }
             }
             *reinterpret_cast<bf16x4*>(&v_lds[v_loff[i]]) = bf16x4{v[0], v[1], v[2], v[3]};
             *reinterpret_cast<bf16x4*>(&v_lds[v_loff[i] + 4]) = bf16x4{v[4], v[5], v[6], v[7]};
@@ -597,6 +617,19 @@ __device__ __forceinline__ void diff_tiles_group(const DiffArgs& a, const int32_
         __syncthreads();
         fetch(min(tb + 3 * TKEYS, tb_last), sb);
         compute(tb + TKEYS);
+    }
+    if (own && head_set == 0) {
+        const int page = page_of(pos0), at = within(pos0);
+        if (page >= 0) {
+            __bf16* k_to = const_cast<__bf16*>(kp_base) + (((size_t)page * a.kv_heads + kvh) * P + at) * (2 * D);
+            __bf16* v_to = const_cast<__bf16*>(vp_base) + ((size_t)page * a.kv_heads + kvh) * V * P + at;
+#pragma unroll
+            for (int i = 0; i < KST; ++i)             // (the threads that stage a tile's first key, and its first keys' values)
+                if (k_mine[i] && k_key[i] == 0) *reinterpret_cast<bf16x8*>(k_to + k_goff[i]) = own_k[i];
+#pragma unroll
+            for (int i = 0; i < VST; ++i)
+                if (v_mine[i] && v_key[i] == 0) v_to[(size_t)v_ch[i] * P] = own_v[i];
+        }
     }
 #pragma unroll
     for (int map = 0; map < 2; ++map) {
@@ -735,7 +768,7 @@ int mlr_diff_attention(const void* q, long q_stride, const void* k_pages, const 
     DiffArgs a{(const elem_t*)q, q_stride, (const elem_t*)k_pages, (const elem_t*)v_pages, block_table, slots, positions,
                (const elem_t*)gate, gate_stride, (elem_t*)out, partial, max_blocks, q_heads, kv_heads, head_dim, value_dim,
                page_size, split_keys, max_splits, scale, softcap, temp_coef, temp_every, lam, out_scale, eps,
-               group_first, group_count, group_tokens, mask_kind, mask_size, {}};
+               group_first, group_count, group_tokens, mask_kind, mask_size, {}, nullptr, 0, nullptr, 0};
     diff_attention_partial_kernel<<<dim3(rows, q_heads * 2, max_splits), 64, 0, stream>>>(a);
     int err = (int)hipGetLastError();
     if (err != 0) return err;
@@ -750,7 +783,8 @@ int mlr_page_of_key(int page_size, int key) { return page_size > 1 ? page_of_key
 // 16 * (4 / min(4, q_heads / kv_heads)) tokens, single tokens and short portions in smaller ones.  `group_tokens`:
 // the most tokens of a group.  With max_splits > 1 every group's keys are cut into ranges of split_keys (a
 // multiple of 64) whose partial results [groups * group_tokens, q_heads * 2, max_splits, value_dim + 2] are merged
-// by the kernel that also serves the scalar path.  `max_context`: no token of the step lies at or beyond it.
+// by the kernel that also serves the scalar path.  own_k, own_v (or null): every group is one new token of a request, whose key and
+// value (rows of a projection, 16-byte aligned keys) are written into their pages here.  `max_context`: no token of the step lies at or beyond it.
 // Returns -10 where the sizes are not taken.
 int mlr_diff_attention_tiles(const void* q, long q_stride, const void* k_pages, const void* v_pages,
                              const int32_t* block_table, int max_blocks, const int32_t* slots, const int32_t* positions,
@@ -758,9 +792,11 @@ int mlr_diff_attention_tiles(const void* q, long q_stride, const void* k_pages, 
                              const int32_t* group_ntok, int groups, int group_tokens, int q_heads, int kv_heads,
                              int head_dim, int value_dim, int page_size, float scale, float softcap, float temp_coef,
                              float temp_every, float lam, float out_scale, float eps, int split_keys, int max_splits,
-                             int max_context, int mask_kind, int mask_size, hipStream_t stream) {
+                             int max_context, int mask_kind, int mask_size, const void* own_k, long own_k_stride, const void* own_v,
+                             long own_v_stride, hipStream_t stream) {
 #if MLR_BF16
     if (groups <= 0) return 0;
+    if ((own_k == nullptr) != (own_v == nullptr) || (reinterpret_cast<uintptr_t>(own_k) & 15) != 0 || own_k_stride % 8 != 0) return -6;
     if (mask_kind < MASK_NONE || mask_kind > MASK_CHUNK || (mask_kind != MASK_NONE && mask_size < 1)) return -5;
     // (behind a mask a workgroup walks the keys of its tokens' window or block only)
     if (mask_kind != MASK_NONE && mask_size + group_tokens + 2 * TILE_KEYS < max_context)
@@ -787,7 +823,8 @@ int mlr_diff_attention_tiles(const void* q, long q_stride, const void* k_pages, 
     DiffArgs a{(const elem_t*)q, q_stride, (const elem_t*)k_pages, (const elem_t*)v_pages, block_table, slots, positions,
                (const elem_t*)gate, gate_stride, (elem_t*)out, partial, max_blocks, q_heads, kv_heads, head_dim, value_dim,
                page_size, split_keys, max_splits, scale, softcap, temp_coef, temp_every, lam, out_scale, eps,
-               group_row0, group_ntok, group_tokens, mask_kind, mask_size, page_divisor(page_size)};
+               group_row0, group_ntok, group_tokens, mask_kind, mask_size, page_divisor(page_size),
+               (const elem_t*)own_k, own_k_stride, (const elem_t*)own_v, own_v_stride};
     const int nch = (head_dim + 31) / 32;
     int err;
     if (nch == 1) err = launch_tiles<1>(a, group_row0, group_ntok, groups, ch, wh, tbw, ms, stream);

@@ -1513,11 +1513,13 @@ class Kernels:
     def diff_attention_tiles(self, q, k_pages, v_pages, block_table, slots, positions, gate, out, partial, group_row0,
                              group_ntok, groups, group_tokens, q_heads, kv_heads, head_dim, value_dim, page_size, scale, lam,
                              out_scale, eps, softcap=None, temp_coef=0.0, temp_every=1.0, split_keys=0, max_splits=1,
-                             max_context=None, mask=None, mask_size=0):
+                             max_context=None, mask=None, mask_size=0, own=None):
         """As `diff_attention` for the rows of `groups` groups of consecutive tokens of one request each (first row,
         number of tokens: device int32 vectors; at most `group_tokens` tokens a group), on the matrix cores.
         `max_context`: a bound on the step's positions + 1 (default: what the block table can hold); the keys that one
-        workgroup walks -- a key range, or all of them -- must lie in `DIFF_TILES_PAGES` pages at most."""
+        workgroup walks -- a key range, or all of them -- must lie in `DIFF_TILES_PAGES` pages at most.
+        `own`: (keys, values) of the step, as `diff_kv_write` takes them, when every group is ONE new token of a request (the
+        caller vouches for that): they are written into their pages here."""
         rows = q.shape[0]
         qs = self._columns(q, "q", self.dtype, rows, q_heads * 2 * head_dim)
         gs = self._columns(gate, "gate", self.dtype, rows, q_heads * value_dim) if gate is not None else 0
@@ -1550,13 +1552,20 @@ class Kernels:
         walk = max_context if mask is None else min(max_context, mask_size + group_tokens + 2 * ATTENTION_TILE_KEYS)
         _need(self.diff_tiles_reach(page_size) >= (split_keys if max_splits > 1 else walk),
               "diff_attention_tiles: one workgroup would walk more pages than it keeps ids of; cut the keys into ranges")
+        own_k, own_v, ks, vs = None, None, 0, 0
+        if own is not None:
+            own_k, own_v = own
+            ks = self._columns(own_k, "own keys", self.dtype, rows, kv_heads * 2 * head_dim)
+            vs = self._columns(own_v, "own values", self.dtype, rows, kv_heads * value_dim)
+            _need(ks % 8 == 0 and own_k.data_ptr() % 16 == 0, "diff_attention_tiles: unaligned keys")
         fn = self._lib("diff_attention").mlr_diff_attention_tiles
         _ok(fn(_p(q), ctypes.c_long(qs), _p(k_pages), _p(v_pages), _p(block_table), _c_int(block_table.shape[1]), _p(slots),
                _p(positions), _p(gate), ctypes.c_long(gs), _p(out), _p(partial if through_partial else None), _p(group_row0),
                _p(group_ntok), _c_int(groups), _c_int(group_tokens), _c_int(q_heads), _c_int(kv_heads), _c_int(head_dim),
                _c_int(value_dim), _c_int(page_size), _c_float(scale), _c_float(softcap or 0.0), _c_float(temp_coef),
                _c_float(temp_every), _c_float(lam), _c_float(out_scale), _c_float(eps), _c_int(split_keys),
-               _c_int(max_splits), _c_int(max_context), _c_int(self.MASK_KINDS[mask]), _c_int(mask_size), _stream()),
+               _c_int(max_splits), _c_int(max_context), _c_int(self.MASK_KINDS[mask]), _c_int(mask_size), _p(own_k), ctypes.c_long(ks),
+               _p(own_v), ctypes.c_long(vs), _stream()),
             "diff_attention_tiles")
 
     # -- layer norm, plain activations ---------------------------------------------------------

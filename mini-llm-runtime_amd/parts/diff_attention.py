@@ -136,7 +136,7 @@ class DiffAttention:
         splits = -(-longest // keys)
         return (keys, splits) if splits > 1 else (0, 1)
 
-    def _attend_tiles(self, ctx, q, gate, view, attn):
+    def _attend_tiles(self, ctx, q, gate, view, attn, own=None):
         """The bfloat16 engine on the matrix cores: prompt portions in groups of 16 to 64 tokens, single tokens and
         portions of up to SMALL_GROUP tokens in groups of their own."""
         s = self.spec
@@ -161,7 +161,7 @@ class DiffAttention:
                                    s.value_dim, view.page_size, float(s.scale), self.lam, float(s.out_scale), float(s.eps),
                                    softcap=s.softcap, temp_coef=temp.coef if temp else 0.0,
                                    temp_every=temp.every if temp else 1.0, split_keys=split_keys, max_splits=splits,
-                                   max_context=ctx.max_context, mask=self.mask, mask_size=self.mask_size)
+                                   max_context=ctx.max_context, mask=self.mask, mask_size=self.mask_size, own=own)
 
     def forward(self, ctx, x, cache_id, write_cache=True):
         s = self.spec
@@ -180,13 +180,16 @@ class DiffAttention:
             rope, interleaved = _rope_table(self.position, ctx, x.device, s.head_dim)
             k.diff_qkv_prep(q, keys, values, k_pages, v_pages, view.block_table, ctx.slots, ctx.positions, rope, s.q_heads,
                             s.kv_heads, s.head_dim, s.value_dim, view.page_size, write_cache, interleaved=interleaved)
-        elif write_cache:
+        tiles = k.diff_tiles_supported(s.q_heads, s.kv_heads, s.head_dim, s.value_dim, view.page_size, proj.stride(0), proj.stride(0)) \
+            and a % 8 == 0 and c % 4 == 0
+        # (single tokens as they are projected: the attention's launch writes them)
+        own = (keys, values) if self.position is None and write_cache and tiles and ctx.single_tokens and proj.stride(0) % 8 == 0 else None
+        if self.position is None and write_cache and own is None:
             k.diff_kv_write(keys, values, k_pages, v_pages, view.block_table, ctx.slots, ctx.positions, s.kv_heads,
                             s.head_dim, s.value_dim, view.page_size)
         attn = ctx.workspace.get("attn", (m, self.o_width), x.dtype)
-        if k.diff_tiles_supported(s.q_heads, s.kv_heads, s.head_dim, s.value_dim, view.page_size, proj.stride(0), proj.stride(0)) \
-                and a % 8 == 0 and c % 4 == 0:
-            self._attend_tiles(ctx, q, gate, view, attn)
+        if tiles:
+            self._attend_tiles(ctx, q, gate, view, attn, own)
             out = ctx.workspace.get("mixer_out", (m, s.hidden), x.dtype)
             k.gemm(attn, self.o, out)
             return out
