@@ -469,10 +469,13 @@ struct DeltaChunkArgs {
     float* scratch;                                              // [chunks][heads][delta_chunk_floats(N, V)]
 };
 
-// W [DC][Np], Qhat [DC][Np], Kbar^T [Np][DC], Y [DC][V], B [DC][DC], G [Np]; Np: N up to a multiple of 16, zeros there
+// W, Qhat, Kbar [DC x Np], Y [DC x Vp], B [DC x DC], G [Np]; Np, Vp: N and V up to a multiple of 16, zeros there.  All but G lie as
+// the scan's wavefronts read them, 16 x 16 elements in one run of 1 KB: block (column / 16, row / 16), in it lane, element as a
+// product takes them -- W, Qhat and B: lane = 16 (column % 16 / 4) + row % 16, element = column % 4; Kbar (rows are tokens) and Y:
+// lane = 16 (row % 16 / 4) + column % 16, element = row % 4.  (As rows, a load of the scan touched 16 lines of which it used a half.)
 __host__ __device__ inline int delta_padded(int N) { return (N + 15) / 16 * 16; }
 __host__ __device__ inline size_t delta_chunk_floats(int N, int V) {
-    return (size_t)DELTA_CHUNK * (3 * delta_padded(N) + V + DELTA_CHUNK) + delta_padded(N);
+    return (size_t)DELTA_CHUNK * (3 * delta_padded(N) + delta_padded(V) + DELTA_CHUNK) + delta_padded(N);
 }
 
 __device__ __forceinline__ floatx4 mma4(const floatx4& a, const floatx4& b, floatx4 c) {
@@ -490,6 +493,7 @@ __device__ __forceinline__ floatx4 mma4_lower(const floatx4& a, const floatx4& b
     if (__builtin_expect(!__any(odd), 1)) return mma4(a, b, c);
     const int first = ((threadIdx.x & 63) >> 4) * 4;
     floatx4 out = c;
+#pragma unroll 1
     for (int t = 0; t < 16; ++t) {
         floatx4 seen;
 #pragma unroll
@@ -507,7 +511,8 @@ __device__ __forceinline__ floatx4 mma4_lower(const floatx4& a, const floatx4& b
 // the sums are a matrix product.  T = (I + A)^-1 by halves too: two triangles of 16 a lane column by column, and
 // -T22 A21 T11 between them.  A thread for each of 1024 pairs, half of them idle, T row by row over 32 rows, and the two
 // products with T one element a thread took 199 us for 2048 tokens of 16 heads of 128 x 128 channels; this one 104 while a
-// thread waited for its elements of q, k and the decays one after the other, now 87, of which the exponentials are the most.
+// thread waited for its elements of q, k and the decays one after the other, 87 until the loops that leave the results stopped
+// dividing for their places and taking e^{c_t} twice, now 75, of which the exponentials are the most.
 __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(DeltaChunkArgs g) {
     constexpr int C = DELTA_CHUNK, CS = DELTA_CHUNK + 4;
     const DeltaArgs& a = g.d;
@@ -530,7 +535,7 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(DeltaChunkArgs
     float* Qh = W + (size_t)C * Np;
     float* Kt = Qh + (size_t)C * Np;
     float* Y = Kt + (size_t)C * Np;
-    float* B = Y + (size_t)C * V;
+    float* B = Y + (size_t)C * delta_padded(V);
     float* G = B + C * C;
     // (eight elements of each asked for at once, clamped and without a branch: one after the other a thread waited for memory
     // sixteen times, and once more for every beta)
@@ -629,14 +634,30 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(DeltaChunkArgs
         *reinterpret_cast<floatx4*>(part_l + (wave * 2) * 256 + lane * 4) = sa;
         *reinterpret_cast<floatx4*>(part_l + (wave * 2 + 1) * 256 + lane * 4) = sb;
     }
-    for (int idx = tid; idx < C * Np; idx += 256) {         // Qhat and G (they read what the loops above read)
-        const int t = idx / Np, i = idx % Np;
-        Qh[idx] = q_l[t * NS + i] * expf(c_l[t * NS + i]);
-        if (t == 0) G[i] = expf(c_l[(C - 1) * NS + i]);
-    }
-    for (int idx = tid; idx < C * Np; idx += 256) {         // Kbar, a channel's tokens side by side
-        const int i = idx / C, t = idx % C;
-        Kt[idx] = k_l[t * NS + i] * expf(c_l[(C - 1) * NS + i] - c_l[t * NS + i]);
+    floatx4 e_c[4];                                         // e^{c_t}, of the elements that this thread leaves in Qhat
+    {                                                       // Qhat, Kbar and G (they read what the loops above read)
+        const int rt = wave & 1, t = 16 * rt + c;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int i0 = 16 * ((wave >> 1) + 2 * u), i = i0 + b4;
+            if (i0 >= Np) break;
+            const floatx4 ct = four(c_l + t * NS + i);
+            floatx4 x = four(q_l + t * NS + i);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                e_c[u][e] = expf(ct[e]);
+                x[e] *= e_c[u][e];
+            }
+            *reinterpret_cast<floatx4*>(Qh + (size_t)(i0 / 16 * 2 + rt) * 256 + lane * 4) = x;
+            const float last = c_l[(C - 1) * NS + i0 + c];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int at = (16 * rt + b4 + e) * NS + i0 + c;
+                x[e] = k_l[at] * expf(last - c_l[at]);
+            }
+            *reinterpret_cast<floatx4*>(Kt + (size_t)(i0 / 16 * 2 + rt) * 256 + lane * 4) = x;
+        }
+        if (tid < Np) G[tid] = expf(c_l[(C - 1) * NS + tid]);
     }
     __syncthreads();
     {
@@ -650,9 +671,18 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(DeltaChunkArgs
         A_l[t * CS + s] = beta_l[t] * sa;
         B_l[t * CS + s] = sb;
     }
-    for (int idx = tid; idx < C * Np; idx += 256) {         // beta Khat in q's place
-        const int t = idx / Np, i = idx % Np;
-        q_l[t * NS + i] = beta_l[t] * k_l[t * NS + i] * expf(c_l[t * NS + i]);
+    {                                                       // beta Khat in q's place
+        const int t = 16 * (wave & 1) + c;
+        const float beta = beta_l[t];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int i0 = 16 * ((wave >> 1) + 2 * u), i = i0 + b4;
+            if (i0 >= Np) break;
+            floatx4 x = four(k_l + t * NS + i);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = beta * x[e] * e_c[u][e];
+            *reinterpret_cast<floatx4*>(q_l + t * NS + i) = x;
+        }
     }
     if (tid < 32) {                                         // the inverses of the two triangles, a column a lane, row after row
         const int j = tid & 15, h0 = tid & 16;
@@ -676,22 +706,19 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(DeltaChunkArgs
 #pragma unroll
         for (int i = 0; i < 4; ++i) T_l[(16 + b4 + i) * CS + c] = -p[i];
     }
-    for (int p = tid; p < C * C; p += 256) B[p] = B_l[(p / C) * CS + p % C];
+    {
+        const int rt = wave & 1, st = wave >> 1;
+        *reinterpret_cast<floatx4*>(B + wave * 256 + lane * 4) = four(B_l + (16 * rt + c) * CS + 16 * st + b4);
+    }
     __syncthreads();
     floatx4 tf[2][2];                                       // T's rows 16 rt + c, columns 16 st + b4 ..
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
         for (int st = 0; st < 2; ++st) tf[rt][st] = four(T_l + (16 * rt + c) * CS + 16 * st + b4);
-    auto product = [&](const floatx4 (&x)[2], float* dst, int width, int col, bool ok) {      // T x, 16 columns
-        floatx4 top = mma4_lower(tf[0][0], x[0], floatx4{0.f, 0.f, 0.f, 0.f});
-        floatx4 low = mma4_lower(tf[1][1], x[1], mma4(tf[1][0], x[0], floatx4{0.f, 0.f, 0.f, 0.f}));
-        if (!ok) return;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            dst[(size_t)(b4 + i) * width + col] = top[i];
-            dst[(size_t)(16 + b4 + i) * width + col] = low[i];
-        }
+    auto product = [&](const floatx4 (&x)[2], floatx4& top, floatx4& low) {                   // T x, 16 columns
+        top = mma4_lower(tf[0][0], x[0], floatx4{0.f, 0.f, 0.f, 0.f});
+        low = mma4_lower(tf[1][1], x[1], mma4(tf[1][0], x[0], floatx4{0.f, 0.f, 0.f, 0.f}));
     };
     for (int i0 = wave * 16; i0 < Np; i0 += 64) {
         floatx4 x[2];
@@ -699,7 +726,14 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(DeltaChunkArgs
         for (int st = 0; st < 2; ++st)
 #pragma unroll
             for (int i = 0; i < 4; ++i) x[st][i] = q_l[(16 * st + b4 + i) * NS + i0 + c];
-        product(x, W, Np, i0 + c, true);
+        floatx4 top, low;
+        product(x, top, low);
+        float* dst = W + (size_t)(i0 / 16 * 2) * 256 + (c >> 2) * 64 + (c & 3);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            dst[(b4 + i) * 4] = top[i];
+            dst[256 + (b4 + i) * 4] = low[i];
+        }
     }
     for (int j0 = wave * 16; j0 < V; j0 += 64) {
         const int j = j0 + c;
@@ -711,7 +745,11 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(DeltaChunkArgs
                 const int t = 16 * st + b4 + i;
                 x[st][i] = t < n && j < V ? beta_l[t] * to_float(a.v[(size_t)(r0 + t) * a.v_stride + head * V + j]) : 0.f;
             }
-        product(x, Y, V, j, j < V);
+        floatx4 top, low;
+        product(x, top, low);
+        float* dst = Y + (size_t)(j0 / 16 * 2) * 256 + lane * 4;
+        *reinterpret_cast<floatx4*>(dst) = top;
+        *reinterpret_cast<floatx4*>(dst + 256) = low;
     }
 }
 
@@ -719,9 +757,10 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(DeltaChunkArgs
 // and keeps their part of the state in registers.  A chunk: every wavefront's share of W S0 goes through LDS (the one barrier
 // a chunk), all add them up to U, and update their part of the state; the shares of O meet in LDS likewise and are added a
 // chunk later.  A chunk's operands are on their way while the chunk before is worked on.  Scalar sums out of tiles staged in
-// LDS took 598 us for 2048 tokens of 16 heads of 128 x 128 channels (64 chunks, 128 workgroups); this one 153, 2.4 us a
+// LDS took 598 us for 2048 tokens of 16 heads of 128 x 128 channels (64 chunks, 128 workgroups); this one 102, 1.6 us a
 // chunk, of which 0.7 are its 52 matrix instructions a wavefront and the rest the chain between them: it is bound by the
-// walk's length, not by memory (with one chunk of operands under way instead of two 166 us).  Without AHEAD, for more workgroups
+// walk's length, not by memory.  (149 us with the operands as rows, a load's 64 lanes in 16 lines of which it used a half; 111 with
+// a loop that waited for every load in its head and with Qhat S0 wholly before the barrier.)  Without AHEAD, for more workgroups
 // than compute units, a chunk's operands are asked for as it begins, and three workgroups share a unit.
 template <int NT, bool AHEAD>
 __global__ __launch_bounds__(256, AHEAD ? 1 : 3) void delta_chunk_scan_kernel(DeltaChunkArgs g) {
@@ -760,34 +799,36 @@ __global__ __launch_bounds__(256, AHEAD ? 1 : 3) void delta_chunk_scan_kernel(De
         const float* Qh = from + (size_t)C * Np;
         const float* Kt = Qh + (size_t)C * Np;
         const float* Y = Kt + (size_t)C * Np;
-        const float* B = Y + (size_t)C * V;
+        const float* B = Y + (size_t)C * delta_padded(V);
         const float* G = B + C * C;
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-            const int n0 = mine[j] ? (wave + 4 * j) * 16 : 0;                  // (for a tile that is not there: its state stays zero)
+            const int tile = mine[j] ? wave + 4 * j : 0;                       // (for a tile that is not there: its state stays zero)
 #pragma unroll
             for (int rt = 0; rt < 2; ++rt) {
-                x.w[rt][j] = *reinterpret_cast<const floatx4*>(from + (16 * rt + c) * Np + n0 + b4);
-                x.q[rt][j] = *reinterpret_cast<const floatx4*>(Qh + (16 * rt + c) * Np + n0 + b4);
-                x.k[j][rt] = *reinterpret_cast<const floatx4*>(Kt + (n0 + c) * C + 16 * rt + b4);
+                const int at = (tile * 2 + rt) * 256 + lane * 4;
+                x.w[rt][j] = *reinterpret_cast<const floatx4*>(from + at);
+                x.q[rt][j] = *reinterpret_cast<const floatx4*>(Qh + at);
+                x.k[j][rt] = *reinterpret_cast<const floatx4*>(Kt + at);
             }
-            x.gate[j] = *reinterpret_cast<const floatx4*>(G + n0 + b4);
+            x.gate[j] = *reinterpret_cast<const floatx4*>(G + tile * 16 + b4);
         }
-        x.b = *reinterpret_cast<const floatx4*>(B + (16 * b_row + c) * C + 16 * b_col + b4);
+        x.b = *reinterpret_cast<const floatx4*>(B + wave * 256 + lane * 4);
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) x.y[rt][i] = Y[(size_t)(16 * rt + b4 + i) * V + (col_ok ? col : 0)];
+        for (int rt = 0; rt < 2; ++rt) x.y[rt] = *reinterpret_cast<const floatx4*>(Y + ((int)blockIdx.z * 2 + rt) * 256 + lane * 4);
     };
     auto put_out = [&](int buf, int c0) {                   // the shares of a chunk's O, added up: two of a lane's elements a thread
-        const int rt = wave >> 1, e0 = (wave & 1) * 2;
+        const int rt = wave >> 1, e0 = (wave & 1) * 2, t = 16 * rt + b4 + e0;
+        float2 o = *reinterpret_cast<const float2*>(&o_l[buf][0][rt][lane * 4 + e0]);
 #pragma unroll
-        for (int e = e0; e < e0 + 2; ++e) {
-            const int t = 16 * rt + b4 + e;
-            const float o = ((o_l[buf][0][rt][lane * 4 + e] + o_l[buf][1][rt][lane * 4 + e]) + o_l[buf][2][rt][lane * 4 + e]) +
-                            o_l[buf][3][rt][lane * 4 + e];
-            if (c0 + t < n && col_ok) a.out[(size_t)(r0 + c0 + t) * ((size_t)a.heads * V) + head * V + col] = o;
+        for (int w = 1; w < 4; ++w) {
+            const float2 more = *reinterpret_cast<const float2*>(&o_l[buf][w][rt][lane * 4 + e0]);
+            o.x += more.x;
+            o.y += more.y;
         }
+        float* dst = a.out + (size_t)(r0 + c0 + t) * ((size_t)a.heads * V) + head * V + col;
+        if (c0 + t < n && col_ok) dst[0] = o.x;
+        if (c0 + t + 1 < n && col_ok) dst[(size_t)a.heads * V] = o.y;
     };
     const float* base = g.scratch + (size_t)chunk0 * step + (size_t)head * delta_chunk_floats(N, V);
     auto work = [&](const Chunk& now, int c0, int buf) {
@@ -800,19 +841,28 @@ __global__ __launch_bounds__(256, AHEAD ? 1 : 3) void delta_chunk_scan_kernel(De
                 for (int rt = 0; rt < 2; ++rt) part[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.w[rt][j][i], S[j][i], part[rt], 0, 0, 0);
 #pragma unroll
         for (int rt = 0; rt < 2; ++rt) *reinterpret_cast<floatx4*>(&u_l[buf][wave][rt][lane * 4]) = part[rt];
+        // (Qhat S0, not on the way to U: half of it while the shares go into LDS, half while they come out)
+        auto start_out = [&](int from, int to) {
 #pragma unroll
-        for (int j = 0; j < NT; ++j)
+            for (int e = from; e < to; ++e)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int rt = 0; rt < 2; ++rt) o[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.q[rt][j][i], S[j][i], o[rt], 0, 0, 0);
+                for (int rt = 0; rt < 2; ++rt) o[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.q[rt][e >> 2][e & 3], S[e >> 2][e & 3], o[rt], 0, 0, 0);
+        };
+        start_out(0, 2 * NT);
         __syncthreads();
-        floatx4 u[2];
+        floatx4 u[2], share[2][4];
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+            for (int w = 0; w < 4; ++w) share[rt][w] = *reinterpret_cast<const floatx4*>(&u_l[buf][w][rt][lane * 4]);
+        __builtin_amdgcn_sched_barrier(0);
+        start_out(2 * NT, 4 * NT);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int rt = 0; rt < 2; ++rt) {
-            floatx4 sum = *reinterpret_cast<const floatx4*>(&u_l[buf][0][rt][lane * 4]);
+            floatx4 sum = share[rt][0];
 #pragma unroll
-            for (int w = 1; w < 4; ++w) sum += *reinterpret_cast<const floatx4*>(&u_l[buf][w][rt][lane * 4]);
+            for (int w = 1; w < 4; ++w) sum += share[rt][w];
             u[rt] = now.y[rt] - sum;
         }
 #pragma unroll
@@ -839,19 +889,29 @@ __global__ __launch_bounds__(256, AHEAD ? 1 : 3) void delta_chunk_scan_kernel(De
         Chunk ring[3];                                      // the chunk at work and the two behind it
         const float* last = base + (size_t)((n - 1) / C) * step;
         fetch(base, ring[0]);
+        __builtin_amdgcn_sched_barrier(0);                  // (in this order, as in the loop: its waits count on it)
         fetch(base + step <= last ? base + step : last, ring[1]);
+        __builtin_amdgcn_sched_barrier(0);
         auto turn = [&](const Chunk& now, Chunk& ahead, int c0) {
             fetch(base + 2 * step <= last ? base + 2 * step : last, ahead);    // (never behind a branch)
             base += step;
             work(now, c0, buf);
             buf ^= 1;
         };
-        for (int c0 = 0; c0 < n; c0 += 3 * C) {
+        // (no way out of the loop's middle: where such paths meet, its head waits for every load that is under way)
+        int c0 = 0;
+        for (; c0 + 2 * C < n; c0 += 3 * C) {
             turn(ring[0], ring[2], c0);
-            if (c0 + C >= n) break;
             turn(ring[1], ring[0], c0 + C);
-            if (c0 + 2 * C >= n) break;
             turn(ring[2], ring[1], c0 + 2 * C);
+        }
+        if (c0 < n) {
+            work(ring[0], c0, buf);
+            buf ^= 1;
+        }
+        if (c0 + C < n) {
+            work(ring[1], c0 + C, buf);
+            buf ^= 1;
         }
     } else {
         for (int c0 = 0; c0 < n; c0 += C) {
@@ -1049,8 +1109,8 @@ int mlr_delta_rule_chunked(const void* q, long q_stride, const void* k, long k_s
     if (err != 0) return err;
     const dim3 grid(segments, heads, (n_values + 15) / 16);
     // (two chunks of operands on their way while one is at work while no compute unit has a second workgroup, which the registers
-    // would keep out: one request of 2048 tokens of 16 heads of 128 x 128 244 us, without 271; but four of 512 181 and 158, 64 of
-    // 32 404 and 218, 64 of 9 380 and 194)
+    // would keep out: both kernels, one request of 2048 tokens of 16 heads of 128 x 128 172 us, without 194; but three of 700 165
+    // and 148, four of 512 128 and 115, 64 of 32 245 and 178, 64 of 9 238 and 169)
     const bool ahead = (long)segments * heads * ((n_values + 15) / 16) <= 256;
     if (Np <= 64) {
         if (ahead) delta_chunk_scan_kernel<1, true><<<grid, 256, 0, stream>>>(g);

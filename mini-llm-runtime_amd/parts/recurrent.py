@@ -436,8 +436,8 @@ class DeltaRule:
         s = self.spec
         if dtype != torch.bfloat16 or rows < CHUNKS_FROM or s.head_dim > 128:
             return {}
-        keys = -(-s.head_dim // 16) * 16                 # (the kernels pad a head's key channels: `Kernels.delta_chunk_floats`)
-        per = DELTA_CHUNK * (3 * keys + s.value_dim + DELTA_CHUNK) + keys
+        keys, values = (-(-n // 16) * 16 for n in (s.head_dim, s.value_dim))     # (as the kernels pad a head: `Kernels.delta_chunk_floats`)
+        per = DELTA_CHUNK * (3 * keys + values + DELTA_CHUNK) + keys
         chunks = rows // DELTA_CHUNK + min(rows, int((limits or {}).get("max_slots") or rows))
         return {("delta_chunks", torch.float32): min(chunks, max(1, PIECE_FLOATS // (per * s.heads))) * per * s.heads,
                 (f"token_groups_{DELTA_CHUNK}_0", torch.int32): 2 * chunks + 2}
