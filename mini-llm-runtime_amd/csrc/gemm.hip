@@ -944,6 +944,8 @@ struct WideArgs {
     float limit, slope;   // of WIDE_CLAMPED
     int vector_out;       // rows of the output start on 16 bytes
     int lda, ldo, a_head, out_head;       // of the form with a product a head: row pitches of activation and output, and from head to head
+    float* partial;                       // SPLIT: the parts' sums, 8 - 8 / SPLIT + 1 tiles of floats a tile of the output
+    int32_t* arrivals;                    // SPLIT: [tiles] workgroups that have left theirs; zero before and after a launch
 };
 
 #define QKV_HEAD 128              // channels of a head
@@ -986,14 +988,18 @@ struct QkvArgs : WideArgs {
 // for closing the parts, 0.4 for a gate), and 0.69 of the time of the kernels that took these rows before.
 // PAIRED: a turn is two blocks, and its operands are in registers before it begins: a small tile has few products a block, and
 // what its turns cost is the wait for the LDS and for the other wavefronts.
-template <int WM, int WN, int TM, int TN, int NS, bool OUT_FLOAT, bool GATED, bool HEADS = false, bool FEW = false, bool PAIRED = false, bool QKV = false>
+// SPLIT (FEW): SPLIT workgroups a tile, each with 8 / SPLIT of the parts; the one that arrives last adds all parts up in their order,
+// the same bits (3 us of a launch: its reads of them).  What a product of few rows is bound by is what its compute units read out of the L2 (12 TB/s of all of them): strips
+// narrow enough for every unit to have one each read the rows again, so wide tiles that share them, and the units that those leave
+// idle given parts of k.
+template <int WM, int WN, int TM, int TN, int NS, bool OUT_FLOAT, bool GATED, bool HEADS = false, bool FEW = false, bool PAIRED = false, bool QKV = false, int SPLIT = 1>
 __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const std::conditional_t<QKV, QkvArgs, WideArgs> args) {
     using S = WideShape<WM, WN, TM, TN, NS>;
     using Q = QkvTile<S>;
     static_assert(!QKV || (!OUT_FLOAT && !GATED && !HEADS && !FEW && S::BN % QKV_HEAD == 0), "whole heads");
     constexpr int BM = S::BM, BN = S::BN, LOADS = S::LOADS;
     static_assert(!GATED || TN % 2 == 0, "gate and up tiles come in pairs");
-    static_assert((!PAIRED || FEW) && (!FEW || !HEADS), "forms for 17 to 64 rows");
+    static_assert((!PAIRED || FEW) && (!FEW || !HEADS) && (SPLIT == 1 || (FEW && SKINNY_WAVES % SPLIT == 0)), "forms for 17 to 64 rows");
     extern __shared__ __attribute__((aligned(16))) __bf16 wide_lds[];
     const int M = args.M, N = args.N, K = args.K;
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -1002,10 +1008,14 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const std::c
     // Workgroups go to the 8 XCDs in turn; each XCD gets a contiguous range of tiles, and in it eight tiles of rows beside
     // each other for every tile of columns, so that an L2 holds what its tiles share.
     constexpr int GROUP = 8;
-    int tm, tn, head = 0;
+    int tm, tn, head = 0, share = 0;                              // share: of the parts of k (SPLIT)
     {
-        const int one = args.tiles_m * args.tiles_n, total = HEADS ? (int)gridDim.x : one, xcd = blockIdx.x % 8;
+        const int one = args.tiles_m * args.tiles_n, total = HEADS || SPLIT > 1 ? (int)gridDim.x : one, xcd = blockIdx.x % 8;
         int tile = xcd * (total / 8) + min(xcd, total % 8) + blockIdx.x / 8;
+        if (SPLIT > 1) {                                          // (a tile's workgroups side by side, on one XCD but for the last of them)
+            share = tile % SPLIT;
+            tile /= SPLIT;
+        }
         if (HEADS) {
             head = tile / one;
             tile -= head * one;
@@ -1043,10 +1053,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const std::c
                                                           (int)((uint32_t)N * (GATED ? 2u : 1u) * (uint32_t)K * 2u), 0x00027000);
     const auto a_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(args.a + (HEADS ? (size_t)head * args.a_head : 0)), 0,
                                                           (int)((HEADS ? (uint32_t)(M - 1) * (uint32_t)args.lda + (uint32_t)K : (uint32_t)M * (uint32_t)K) * 2u), 0x00027000);
+    constexpr int PER = SKINNY_WAVES / SPLIT;                     // parts of k that a workgroup has
+    const int all_blocks = K / WIDE_BK, part_blocks = (all_blocks + SKINNY_WAVES - 1) / SKINNY_WAVES;
+    const int first_block = SPLIT > 1 ? share * PER * part_blocks : 0;
     auto load = [&](int i, int kb, int stage) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds((wave * LOADS + i) * 8 < BN ? w_rsrc : a_rsrc,
                                                  (__attribute__((address_space(3))) void*)(wide_lds + stage * S::STAGE + (wave * LOADS + i) * 512),
-                                                 16, (int)src[i], kb * (WIDE_BK * 2), 0, 0);
+                                                 16, (int)src[i], (first_block + kb) * (WIDE_BK * 2), 0, 0);
     };
 
     floatx4 acc[TM][TN];
@@ -1054,17 +1067,35 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const std::c
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-    const int blocks = K / WIDE_BK, part_blocks = (blocks + SKINNY_WAVES - 1) / SKINNY_WAVES;
+    const int blocks = SPLIT > 1 ? min(all_blocks - first_block, PER * part_blocks) : all_blocks;
     floatx4 sum[FEW ? TM : 1][FEW ? TN : 1];                      // FEW: the parts of k that are done
-    int part_left = part_blocks;
+    floatx4 part[SPLIT > 1 ? PER : 1][FEW ? TM : 1][FEW ? TN : 1];           // SPLIT: each by itself, but the first share's (in `sum`)
+    int part_left = part_blocks, closed = 0;
     if constexpr (FEW) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j) sum[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < TN; ++j) {
+                sum[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int q = 0; q < (SPLIT > 1 ? PER : 1); ++q) part[q][i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+            }
     }
     auto close_part = [&]() {
-        if constexpr (FEW) {
+        if (SPLIT > 1 && share > 0) {
+#pragma unroll
+            for (int q = 0; q < (SPLIT > 1 ? PER : 1); ++q)
+                if (closed == q) {                                // (the same in every lane)
+#pragma unroll
+                    for (int i = 0; i < TM; ++i)
+#pragma unroll
+                        for (int j = 0; j < TN; ++j) {
+                            part[q][i][j] = acc[i][j];
+                            acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+                        }
+                }
+            ++closed;
+        } else if constexpr (FEW) {
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -1279,8 +1310,46 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const std::c
             block_done();
         }
     }
-    if constexpr (FEW) {
-        close_part();                                             // (the last part, where it is a shorter one)
+    if constexpr (FEW) close_part();                              // (the last part, where it is a shorter one)
+    if constexpr (SPLIT > 1) {
+        // The shares' sums pass the L2s (coherent at the device), whatever XCD the last workgroup runs on: they are there once the
+        // stores are through, and only then is the arrival counted.
+        constexpr int VALUES = SKINNY_WAVES - PER + 1, LANE = 4 * 64 * WM * WN, AROUND = 0x10;     // (AROUND: sc1)
+        const int tile = tm * args.tiles_n + tn;
+        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(args.partial + (size_t)tile * VALUES * TM * TN * LANE), 0, VALUES * TM * TN * LANE * 4, 0x00027000);
+        auto at = [&](int v, int i, int j) { return ((v * TM + i) * TN + j) * LANE * 4; };
+        typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                if (share == 0) {
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, sum[i][j]), rsrc, t * 16, at(0, i, j), AROUND);
+                } else {
+#pragma unroll
+                    for (int q = 0; q < PER; ++q)
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, part[q][i][j]), rsrc, t * 16, at(1 + (share - 1) * PER + q, i, j), AROUND);
+                }
+            }
+        wide_arrive<0>();
+        int32_t* meet = reinterpret_cast<int32_t*>(wide_lds);
+        if (t == 0) *meet = __hip_atomic_fetch_add(args.arrivals + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (*meet != SPLIT - 1) return;
+        if (t == 0) __hip_atomic_store(args.arrivals + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                u32x4_t got[VALUES];
+#pragma unroll
+                for (int v = 0; v < VALUES; ++v) got[v] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, t * 16, at(v, i, j), AROUND);
+                acc[i][j] = __builtin_bit_cast(floatx4, got[0]);
+#pragma unroll
+                for (int v = 1; v < VALUES; ++v) acc[i][j] += __builtin_bit_cast(floatx4, got[v]);
+            }
+    } else if constexpr (FEW) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -1597,6 +1666,66 @@ static int launch_few(WideArgs& args, bool out_float, bool gated, hipStream_t st
     return -1;
 }
 
+// The forms with several workgroups a tile (SPLIT), and what they cost: as above, a round's time by 1024 k of a share, `row` by 16 rows;
+// `half`: the same of a last round whose workgroups have a compute unit each.  Fitted to 560 products of 17 to 64 rows (200 of up to 32),
+// inner sizes drawn from 1500 to 26000 and 512 to 16384 rows of weight, weights cold (rms 6 to 14 %; the predicted form is 0.7 %
+// behind the best one, geometric mean).
+struct SplitCost { int shape, splits, bm, bn, per_unit; float fixed, turn, all, row, half_turn, half_all, half_row; };
+static const SplitCost SPLIT_COSTS[] = {
+    {0, 2, 32, 64, 1, -2.16f, 6.78f, 0.76f, 1.53f, 0.f, 0.f, 0.f},  {1, 2, 64, 64, 2, 5.14f, 4.57f, 7.40f, 0.94f, 0.56f, 3.02f, 0.43f},
+    {2, 4, 32, 32, 1, 1.61f, 3.19f, 0.48f, 0.97f, 0.f, 0.f, 0.f},   {3, 4, 32, 64, 1, 0.03f, 4.88f, 0.80f, 1.61f, 0.f, 0.f, 0.f},
+    {4, 4, 64, 64, 2, 1.00f, 7.20f, 9.18f, 0.65f, 4.71f, 3.03f, 0.48f}, {5, 4, 64, 128, 1, -2.00f, 9.44f, 5.99f, 0.52f, 0.f, 0.f, 0.f},
+    {6, 4, 64, 32, 2, 2.07f, 3.93f, 3.92f, 0.90f, 2.80f, 2.45f, 0.24f}};
+
+static int split_shape_for(int M, int N, int K) {
+    const int units = compute_units() > 0 ? compute_units() : 256;
+    const float row_tiles = (float)((M + 15) / 16);
+    int best = -1;
+    float time = 0.f;
+    for (const SplitCost& c : SPLIT_COSTS) {
+        if (M > c.bm) continue;
+        const int workgroups = (N + c.bn - 1) / c.bn * c.splits, slots = units * c.per_unit, left = workgroups % slots;
+        const bool half = c.per_unit == 2 && left > 0 && left <= units;
+        const float rounds = (float)(workgroups / slots + (left > 0 && !half ? 1 : 0)), k = (float)(K / c.splits) * (1.0f / 1024.0f);
+        const float us = c.fixed + rounds * (c.turn + (c.all + c.row * row_tiles) * k) + (half ? c.half_turn + (c.half_all + c.half_row * row_tiles) * k : 0.f);
+        if (best < 0 || us < time) {
+            best = c.shape;
+            time = us;
+        }
+    }
+    return best;
+}
+
+template <int SPLIT, bool PAIRED, int WM, int WN, int TM, int TN, int NS>
+static int launch_split(WideArgs& args, long floats, int counters, hipStream_t stream) {
+    using S = WideShape<WM, WN, TM, TN, NS>;
+    constexpr int PER = SKINNY_WAVES / SPLIT;
+    args.tiles_m = (args.M + S::BM - 1) / S::BM;
+    args.tiles_n = (args.N + S::BN - 1) / S::BN;
+    const long tiles = (long)args.tiles_m * args.tiles_n, blocks = args.K / WIDE_BK, part_blocks = (blocks + SKINNY_WAVES - 1) / SKINNY_WAVES;
+    // (every workgroup has something to multiply; the last one's blocks are those that are left)
+    if (args.tiles_m != 1 || tiles > counters || tiles * (SKINNY_WAVES - PER + 1) * S::BM * S::BN > floats || blocks <= (SPLIT - 1) * PER * part_blocks) return -1;
+    auto* kernel = gemm_wide_kernel<WM, WN, TM, TN, NS, false, false, false, true, PAIRED, false, SPLIT>;
+    static const hipError_t allowed = hipFuncSetAttribute(
+        reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds_bytes);
+    if (allowed != hipSuccess) return (int)allowed;
+    kernel<<<dim3((unsigned)(tiles * SPLIT)), 64 * S::WAVES, S::lds_bytes, stream>>>(args);
+    return (int)hipGetLastError();
+}
+
+static int launch_split_shape(int shape, WideArgs& args, long floats, int counters, hipStream_t stream) {
+    switch (shape) {
+        case 0: return launch_split<2, true, 2, 2, 1, 2, 12>(args, floats, counters, stream);
+        case 1: return launch_split<2, false, 2, 2, 2, 2, 5>(args, floats, counters, stream);
+        case 2: return launch_split<4, true, 2, 1, 1, 2, 14>(args, floats, counters, stream);
+        case 3: return launch_split<4, true, 2, 2, 1, 2, 12>(args, floats, counters, stream);
+        case 4: return launch_split<4, false, 2, 2, 2, 2, 5>(args, floats, counters, stream);
+        case 5: return launch_split<4, false, 2, 2, 2, 4, 6>(args, floats, counters, stream);
+        case 6: return launch_split<4, false, 2, 2, 2, 1, 6>(args, floats, counters, stream);
+        default: return -1;
+    }
+}
+
 static int launch_wide_shape(int shape, WideArgs& args, bool out_float, bool gated, hipStream_t stream) {
     switch (shape) {
         case 0: return launch_wide<2, 2, 2, 1, 6, 4, 1, 1, 2>(args, out_float, gated, stream);
@@ -1673,7 +1802,7 @@ enum { WIDE_MANY = -1, WIDE_FEW = -2 };      // the tile with the least predicte
 static int run_wide(int shape, const void* a, const void* w, void* out, int M, int N, int K, bool out_float, int act, float limit,
                     float slope, hipStream_t stream) {
     const bool gated = act >= WIDE_SILU && act <= WIDE_CLAMPED;
-    WideArgs args{(const __bf16*)a, (const __bf16*)w, out, M, N, K, 0, 0, act, limit, slope, 0, 0, 0, 0, 0};
+    WideArgs args{(const __bf16*)a, (const __bf16*)w, out, M, N, K, 0, 0, act, limit, slope, 0, 0, 0, 0, 0, nullptr, nullptr};
     const uintptr_t row_bytes = (uintptr_t)N * (out_float ? 4 : 2);
     args.vector_out = ((reinterpret_cast<uintptr_t>(out) | row_bytes) & 15) == 0 ? 1 : 0;
     float time = 0.f;
@@ -1689,6 +1818,36 @@ extern "C" int mlr_gemm_wide(const void* a, const void* w, void* out, int M, int
     if (M <= 0 || N <= 0) return 0;
     if (K <= 0 || (gated && out_float) || !wide_takes(a, w, M, N, K, gated != 0)) return -1;
     return run_wide(shape, a, w, out, M, N, K, out_float != 0, gated ? WIDE_SILU : WIDE_PLAIN, 0.f, 0.f, stream);
+}
+
+// Whether 17 to 64 rows are the forms' with several workgroups a tile, instead of those above and the vendor library.  Measured on the
+// products of the forms' fit against what took them before, geometric mean: the 310 that this takes 0.63 (0.34 to 1.02; of those
+// where the library has a plan that cuts k itself, a row count and sizes in whole 16s, 0.7 to 1); below these inner sizes 1.04 to 1.4,
+// beyond these rows of weight 0.9 to 1.3.  64 x 4096 x 12288 34.0 -> 26.0 us, 48 x 5120 x 25600 84.7 -> 62.1, 32 x 2048 x 5632
+// 12.4 -> 9.2, 64 x 4096 x 4096 14.4 -> 12.4, 20 x 3000 x 8960 19.4 -> 15.1.
+static bool split_wins(int M, int N, int K) {
+    if (M <= 16 || M > 64) return false;
+    if (K >= 14336) return N <= 16384;
+    if (K >= 9216) return N <= 8192;
+    if (K >= 6144) return N <= 6144;
+    if (K >= 4224) return N <= 4096;
+    if (K >= 3136) return N <= (M > 32 ? 4096 : 2048);
+    return K >= 2560 && M > 32 && N > 1024 && N <= 2048;
+}
+extern "C" int mlr_gemm_split_wins(int M, int N, int K) {
+    return N > 0 && K > 0 && wide_takes(nullptr, nullptr, M, N, K, false) && split_wins(M, N, K) ? 1 : 0;
+}
+
+// The product of 17 to 64 rows with several workgroups a tile, the bits of `mlr_gemm_wide` with -2; `partial`: `floats` floats on 16
+// bytes, `arrivals`: `counters` zeros, which are zero again behind it; one launch at a time may use them.  shape: 0 .. 6, or -1 for
+// the form with the least predicted time.  -1: sizes or room that it does not take, nothing was launched.
+extern "C" int mlr_gemm_split(const void* a, const void* w, void* out, int M, int N, int K, float* partial, long floats, int32_t* arrivals,
+                              int counters, int shape, hipStream_t stream) {
+    if (M <= 16 || M > 64 || N <= 0 || K <= 0 || partial == nullptr || arrivals == nullptr || (reinterpret_cast<uintptr_t>(partial) & 15) != 0 ||
+        !wide_takes(a, w, M, N, K, false)) return -1;
+    WideArgs args{(const __bf16*)a, (const __bf16*)w, out, M, N, K, 0, 0, WIDE_PLAIN, 0.f, 0.f, 0, 0, 0, 0, 0, partial, arrivals};
+    args.vector_out = ((reinterpret_cast<uintptr_t>(out) | (uintptr_t)N * 2) & 15) == 0 ? 1 : 0;
+    return launch_split_shape(shape < 0 ? split_shape_for(M, N, K) : shape, args, floats, counters, stream);
 }
 
 // out[m][h] = a[m][h] . w[h]^T of many rows: out and a with rows of `ldo` and `lda` elements, heads `out_head` and `a_head` apart,
@@ -1709,7 +1868,7 @@ extern "C" int mlr_gemm_heads(const void* a, long lda, long a_head, const void* 
     if ((long long)tiles_m * tiles_n * heads > 0x7fffffffLL / 8) return -3;
     const int vector_out = (reinterpret_cast<uintptr_t>(out) & 15) == 0 && ldo % 8 == 0 && out_head % 8 == 0 ? 1 : 0;
     const WideArgs args{(const __bf16*)a, (const __bf16*)w, out, M, N, K, tiles_m, tiles_n, WIDE_PLAIN, 0.f, 0.f, vector_out,
-                        (int)lda, (int)ldo, (int)a_head, (int)out_head};
+                        (int)lda, (int)ldo, (int)a_head, (int)out_head, nullptr, nullptr};
     auto* kernel = gemm_wide_kernel<4, 2, 2, 2, 2, false, false, true>;
     static const hipError_t allowed = hipFuncSetAttribute(
         reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds_bytes);

@@ -140,7 +140,7 @@ class Runner:
         self.workspace = Workspace(self.device)
         self.workspace.reserve(workspace_plan)
         if uses_library:
-            self.kernels.reserve_library_workspace(self.device)
+            self.kernels.reserve_split_workspace(self.device)
         self.check_finite = bool(check_finite)
         self._status = torch.zeros(2, dtype=torch.int32, device=self.device)
         if profile:

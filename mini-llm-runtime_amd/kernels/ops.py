@@ -25,6 +25,8 @@ ATTENTION_TILE_KEYS = 64
 LIBRARY_GEMM_MIN_ROWS = 16    # above this many rows the bfloat16 engine's projections may go to the library
 WIDE_CHOICES_KEPT = 4096      # products whose way (our kernel or the library) is remembered
 LIBRARY_GEMM_WORKSPACE = 128 << 20   # bytes of scratch memory that the library may use
+SPLIT_COUNTERS = 1024          # places at its end that count a tile's workgroups (512 tiles at most: 16384 columns in tiles of 32)
+SPLIT_PARTIAL_BYTES = 32 << 20 # of it for the parts of a product that several workgroups a tile share (64 rows of 16384 columns: 28 MB)
 PREFILL_MAX_PAGES = 2048      # page ids of one group that the prompt-portion attention kernel keeps in LDS
 TILES_MAX_HEAD_DIM = 128      # the 32x32-tile kernel for prompt portions keeps two sets of accumulators per lane
 TILES_COLUMNS = (128, 64)     # (token, head) columns of one of its workgroups: the usual and the small one
@@ -187,6 +189,7 @@ class Kernels:
         self.library_gemm = library_gemm
         self.routed = routed
         self._library_workspace = None      # scratch memory of the vendor library's products, allocated once
+        self._split = None                  # in it: room for the parts of a product and the counters of who has left them
         self._wide_choices = {}             # (rows, columns, inner size, activation) -> `wide_product`
         self._libs = {}
         self.profiler = None                # a `Profiler`: every launch is then bracketed by events
@@ -387,6 +390,11 @@ class Kernels:
         _need(k == k2, lambda: f"gemm: inner sizes differ ({k} and {k2})")
         _need(out.dtype in (self.dtype, torch.float32), lambda: f"gemm: output type {out.dtype} not supported")
         _tensor(out, "out", out.dtype, (m, n))
+        if m <= 64 and out.dtype == torch.bfloat16 and self._split is not None and self.split_product(m, n, k) and _on16(a, w):
+            partial, arrivals = self._split
+            _ok(self._lib("gemm").mlr_gemm_split(_p(a), _p(w), _p(out), _c_int(m), _c_int(n), _c_int(k), _p(partial),
+                                                 ctypes.c_long(partial.numel()), _p(arrivals), _c_int(arrivals.numel()), _c_int(-1), _stream()), "gemm")
+            return
         if m <= 64 and out.dtype == torch.bfloat16 and (self.few_product(m, n, k) or self.wide_product(m, n, k)) and _on16(a, w):
             _ok(self._lib("gemm").mlr_gemm_wide(_p(a), _p(w), _p(out), _c_int(m), _c_int(n), _c_int(k), _c_int(0),
                                                 _c_int(-1 if self.one_sum(m, k) else -2), _c_int(0), _stream()), "gemm")
@@ -399,7 +407,7 @@ class Kernels:
             ws = self.reserve_library_workspace(a.device)
             _ok(self._lib("library_gemm").mlr_library_gemm(_p(a), _p(w), _p(out), _c_int(m), _c_int(n), _c_int(k),
                                                            _c_int(1 if out.dtype == torch.float32 else 0),
-                                                           _p(ws), _c_size_t(ws.numel()), _stream()), "library_gemm")
+                                                           _p(ws), _c_size_t(ws.numel() - SPLIT_COUNTERS * 4), _stream()), "library_gemm")
             return
         fn = self._lib("gemm").mlr_gemm
         _ok(fn(_p(a), _p(w), _p(out), _c_int(m), _c_int(n), _c_int(k),
@@ -410,6 +418,30 @@ class Kernels:
         if self._library_workspace is None:
             self._library_workspace = torch.empty(LIBRARY_GEMM_WORKSPACE, dtype=torch.uint8, device=device)
         return self._library_workspace
+
+    def reserve_split_workspace(self, device):
+        """From here on products of few rows may share a tile out to several workgroups (`split_product`): their parts meet in the
+        scratch memory of the library's products, so one launch of either at a time, as a runner's steps make them; the end of it,
+        which the library is not given, counts the workgroups that have left theirs."""
+        ws = self.reserve_library_workspace(device)
+        if self._split is None:
+            arrivals = ws[ws.numel() - SPLIT_COUNTERS * 4:].view(torch.int32)
+            arrivals.zero_()
+            self._split = (ws[:SPLIT_PARTIAL_BYTES].view(torch.float32), arrivals)
+
+    def split_product(self, rows, columns, k):
+        """Whether a product of 17 to 64 rows is taken by several workgroups a tile: the sums of `few_product`, bit by bit, so not for a
+        model that routes, which keeps the library's where this would replace them."""
+        if self.dtype != torch.bfloat16 or self.routed or not LIBRARY_GEMM_MIN_ROWS < rows <= 64:
+            return False
+        key = (rows, columns, k, "split")
+        wins = self._wide_choices.get(key)
+        if wins is None:
+            wins = bool(self._lib("gemm").mlr_gemm_split_wins(_c_int(rows), _c_int(columns), _c_int(k)))
+            if len(self._wide_choices) >= WIDE_CHOICES_KEPT:
+                self._wide_choices.clear()
+            self._wide_choices[key] = wins
+        return wins
 
     def library_workspace_bytes(self):
         return 0 if self._library_workspace is None else self._library_workspace.numel()

@@ -1,0 +1,82 @@
+"""Products of 17 to 64 rows whose tiles several workgroups share: when they are taken, and their bits."""
+import ctypes
+
+import pytest
+import torch
+
+from mini_llm_runtime_amd.kernels import Kernels
+from mini_llm_runtime_amd.kernels import ops
+
+
+def without_gpu(routed=False):
+    k = object.__new__(Kernels)
+    k.dtype, k.library_gemm, k.routed, k.profiler = torch.bfloat16, True, routed, None
+    k._libs, k._wide_choices, k._split = {}, {}, None
+    return k
+
+
+@pytest.mark.parametrize("rows,columns,inner,taken", [
+    (16, 4096, 12288, False), (17, 4096, 12288, True), (64, 4096, 12288, True), (65, 4096, 12288, False), (64, 4096, 2048, False),
+    (64, 2048, 2560, True), (32, 2048, 2560, False), (64, 1024, 2560, False), (32, 2048, 3136, True), (32, 2049, 3136, False),
+    (33, 4096, 3136, True), (20, 4097, 4224, False), (64, 6144, 6144, True), (64, 8192, 9216, True), (64, 16384, 14336, True),
+    (64, 16385, 14336, False), (64, 4096, 12289, False)])
+def test_long_inner_sizes_of_few_rows_are_shared_out(rows, columns, inner, taken):
+    assert without_gpu().split_product(rows, columns, inner) == taken
+    assert not without_gpu(routed=True).split_product(rows, columns, inner)
+
+
+# (inner sizes whose last share is one block, a part's last block missing, as many as parts; columns in whole tiles, ragged, odd)
+@pytest.mark.gpu
+@pytest.mark.parametrize("inner", [512, 448, 64 * 25, 64 * 49, 4096, 64 * 67])
+@pytest.mark.parametrize("rows,columns", [(17, 16), (32, 64), (31, 1000), (33, 129), (64, 128), (50, 2047), (64, 4096)])
+def test_a_shared_tile_has_the_bits_of_one_workgroups(rows, columns, inner):
+    k = Kernels(torch.bfloat16)
+    gen = torch.Generator().manual_seed(rows + columns + inner)
+    draw = lambda *shape: torch.randn(*shape, generator=gen).to(torch.bfloat16).cuda()
+    a, w = draw(rows, inner), draw(columns, inner)
+    want = torch.empty(rows, columns, dtype=torch.bfloat16, device="cuda")
+    number, place = ctypes.c_int, lambda t: ctypes.c_void_p(t.data_ptr())
+    lib, stream = k._lib("gemm"), ops._stream()
+    sizes = (number(rows), number(columns), number(inner))
+    assert lib.mlr_gemm_wide(place(a), place(w), place(want), *sizes, number(0), number(-2), number(0), stream) == 0
+    partial = torch.full((1 << 23,), float("nan"), device="cuda")
+    arrivals = torch.zeros(ops.SPLIT_COUNTERS, dtype=torch.int32, device="cuda")
+    taken = 0
+    for shape in range(-1, 7):
+        for _ in range(2):                               # (the counters are what they were)
+            got = torch.full_like(want, float("nan"))
+            code = lib.mlr_gemm_split(place(a), place(w), place(got), *sizes, place(partial), ctypes.c_long(partial.numel()), place(arrivals),
+                                      number(arrivals.numel()), number(shape), stream)
+            if code == -1:
+                assert torch.isnan(got).all()            # (too few blocks of k for the shares: nothing was launched)
+                continue
+            assert code == 0 and torch.equal(got.view(torch.int16), want.view(torch.int16)), shape
+            taken += 1
+        assert not arrivals.any()
+    assert taken >= (0 if inner < 512 else 8)
+    # no room, no launch
+    code = lib.mlr_gemm_split(place(a), place(w), place(got), *sizes, place(partial), ctypes.c_long(64), place(arrivals),
+                              number(arrivals.numel()), number(-1), stream)
+    assert code == -1
+
+
+@pytest.mark.gpu
+def test_the_runners_kernels_share_products_out_and_others_do_not():
+    k, other = Kernels(torch.bfloat16), Kernels(torch.bfloat16)
+    k.reserve_split_workspace("cuda")
+    a, w = torch.randn(40, 4160, device="cuda").bfloat16(), torch.randn(1500, 4160, device="cuda").bfloat16()
+    out, again = (torch.empty(40, 1500, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    k.gemm(a, w, out)
+    few = torch.empty_like(out)
+    assert k._lib("gemm").mlr_gemm_wide(*(ctypes.c_void_p(t.data_ptr()) for t in (a, w, few)), *(ctypes.c_int(n) for n in (40, 1500, 4160, 0, -2, 0)),
+                                        ops._stream()) == 0
+    assert torch.equal(out.view(torch.int16), few.view(torch.int16)) and other._split is None
+    other.gemm(a, w, again)
+    want = a.float() @ w.float().T
+    for got in (out, again):                             # (one rounding to bfloat16 of sums whose terms are about 1)
+        torch.testing.assert_close(got.float(), want, rtol=2 ** -8, atol=2 ** -8)
+    # between a product of the library, which has the rest of the scratch memory, and another
+    k.gemm(torch.randn(64, 2048, device="cuda").bfloat16(), torch.randn(4096, 2048, device="cuda").bfloat16(),
+           torch.empty(64, 4096, device="cuda"))
+    k.gemm(a, w, again)
+    assert torch.equal(out.view(torch.int16), again.view(torch.int16))
