@@ -980,7 +980,7 @@ struct QkvArgs : WideArgs {
 // queries to their matrix and the keys to their page; heads of values go to LDS transposed, so that eight rows of a channel are one
 // read and one store into their page.
 // The q/k/v matrix itself is never written: 2048 x 4096 x 1024 22.2 us for the 28.0 of the two launches, 19.1 of them the product.
-// FEW (17 to 64 rows): the sums of `gemm_skinny_kernel`, bit by bit, so that a row's results do not turn on whether 16 rows or 64
+// FEW (up to 64 rows): the sums of `gemm_skinny_kernel`, bit by bit, so that a row's results do not turn on whether 16 rows or 64
 // are computed with it: eight parts of k, of whole blocks, each one sum and added in ascending order, and 16 consecutive bytes of
 // every 32 of a row an instruction.  (The parts are also the more exact sum: worked out with normal operands, a
 // rounding an instruction, its rms error is 0.63, 0.54 and 0.45 of one chain's at k = 1024, 2048 and 4096.)
@@ -1675,7 +1675,10 @@ static const SplitCost SPLIT_COSTS[] = {
     {0, 2, 32, 64, 1, -2.16f, 6.78f, 0.76f, 1.53f, 0.f, 0.f, 0.f},  {1, 2, 64, 64, 2, 5.14f, 4.57f, 7.40f, 0.94f, 0.56f, 3.02f, 0.43f},
     {2, 4, 32, 32, 1, 1.61f, 3.19f, 0.48f, 0.97f, 0.f, 0.f, 0.f},   {3, 4, 32, 64, 1, 0.03f, 4.88f, 0.80f, 1.61f, 0.f, 0.f, 0.f},
     {4, 4, 64, 64, 2, 1.00f, 7.20f, 9.18f, 0.65f, 4.71f, 3.03f, 0.48f}, {5, 4, 64, 128, 1, -2.00f, 9.44f, 5.99f, 0.52f, 0.f, 0.f, 0.f},
-    {6, 4, 64, 32, 2, 2.07f, 3.93f, 3.92f, 0.90f, 2.80f, 2.45f, 0.24f}};
+    {6, 4, 64, 32, 2, 2.07f, 3.93f, 3.92f, 0.90f, 2.80f, 2.45f, 0.24f},
+    // up to 16 rows: fitted to 250 products of them, inner sizes from 2000 to 26000 (rms 6, 11 and 14 %; 1.3 % behind the best form)
+    {7, 4, 16, 32, 2, 2.11f, 2.73f, 4.85f, 0.f, 2.39f, 2.45f, 0.f}, {8, 4, 16, 64, 2, 0.52f, 4.32f, 9.20f, 0.f, 3.92f, 3.47f, 0.f},
+    {9, 2, 16, 64, 1, -4.12f, 8.15f, 3.26f, 0.f, 0.f, 0.f, 0.f}};
 
 static int split_shape_for(int M, int N, int K) {
     const int units = compute_units() > 0 ? compute_units() : 256;
@@ -1683,7 +1686,7 @@ static int split_shape_for(int M, int N, int K) {
     int best = -1;
     float time = 0.f;
     for (const SplitCost& c : SPLIT_COSTS) {
-        if (M > c.bm) continue;
+        if (M > c.bm || (M <= 16) != (c.bm == 16)) continue;
         const int workgroups = (N + c.bn - 1) / c.bn * c.splits, slots = units * c.per_unit, left = workgroups % slots;
         const bool half = c.per_unit == 2 && left > 0 && left <= units;
         const float rounds = (float)(workgroups / slots + (left > 0 && !half ? 1 : 0)), k = (float)(K / c.splits) * (1.0f / 1024.0f);
@@ -1722,6 +1725,9 @@ static int launch_split_shape(int shape, WideArgs& args, long floats, int counte
         case 4: return launch_split<4, false, 2, 2, 2, 2, 5>(args, floats, counters, stream);
         case 5: return launch_split<4, false, 2, 2, 2, 4, 6>(args, floats, counters, stream);
         case 6: return launch_split<4, false, 2, 2, 2, 1, 6>(args, floats, counters, stream);
+        case 7: return launch_split<4, false, 1, 2, 1, 1, 12>(args, floats, counters, stream);
+        case 8: return launch_split<4, false, 1, 2, 1, 2, 8>(args, floats, counters, stream);
+        case 9: return launch_split<2, true, 1, 2, 1, 2, 12>(args, floats, counters, stream);
         default: return -1;
     }
 }
@@ -1820,13 +1826,20 @@ extern "C" int mlr_gemm_wide(const void* a, const void* w, void* out, int M, int
     return run_wide(shape, a, w, out, M, N, K, out_float != 0, gated ? WIDE_SILU : WIDE_PLAIN, 0.f, 0.f, stream);
 }
 
-// Whether 17 to 64 rows are the forms' with several workgroups a tile, instead of those above and the vendor library.  Measured on the
+// Whether up to 64 rows are the forms' with several workgroups a tile, instead of the kernels above and the vendor library.  Up to 16
+// rows, against `gemm_skinny_kernel` on 250 products, geometric mean: 0.75 of those that this takes (0.49 to 1.06); below these inner sizes 0.86 to
+// 1.15, and where a strip of 16 columns a compute unit comes out even (193 to 256 strips) 0.97 (to 1.07) up to 5120.  8 x 2048 x 5632
+// 10.8 -> 8.7 us, 1 x 2048 x 8448 14.6 -> 10.4, 16 x 4096 x 12288 27.1 -> 20.6, 8 x 3000 x 8960 17.3 -> 13.3.  From 17 on: measured on the
 // products of the forms' fit against what took them before, geometric mean: the 310 that this takes 0.63 (0.34 to 1.02; of those
 // where the library has a plan that cuts k itself, a row count and sizes in whole 16s, 0.7 to 1); below these inner sizes 1.04 to 1.4,
 // beyond these rows of weight 0.9 to 1.3.  64 x 4096 x 12288 34.0 -> 26.0 us, 48 x 5120 x 25600 84.7 -> 62.1, 32 x 2048 x 5632
 // 12.4 -> 9.2, 64 x 4096 x 4096 14.4 -> 12.4, 20 x 3000 x 8960 19.4 -> 15.1.
 static bool split_wins(int M, int N, int K) {
-    if (M <= 16 || M > 64) return false;
+    if (M <= 0 || M > 64) return false;
+    if (M <= 16) {
+        const int units = compute_units() > 0 ? compute_units() : 256, strips = (N + 15) / 16;
+        return N <= 8192 && (K >= 5120 || (K >= 3584 && !(4 * strips > 3 * units && strips <= units)));
+    }
     if (K >= 14336) return N <= 16384;
     if (K >= 9216) return N <= 8192;
     if (K >= 6144) return N <= 6144;
@@ -1838,12 +1851,12 @@ extern "C" int mlr_gemm_split_wins(int M, int N, int K) {
     return N > 0 && K > 0 && wide_takes(nullptr, nullptr, M, N, K, false) && split_wins(M, N, K) ? 1 : 0;
 }
 
-// The product of 17 to 64 rows with several workgroups a tile, the bits of `mlr_gemm_wide` with -2; `partial`: `floats` floats on 16
-// bytes, `arrivals`: `counters` zeros, which are zero again behind it; one launch at a time may use them.  shape: 0 .. 6, or -1 for
+// The product of up to 64 rows with several workgroups a tile, the bits of the other kernels of few rows; `partial`: `floats` floats on 16
+// bytes, `arrivals`: `counters` zeros, which are zero again behind it; one launch at a time may use them.  shape: 0 .. 9, or -1 for
 // the form with the least predicted time.  -1: sizes or room that it does not take, nothing was launched.
 extern "C" int mlr_gemm_split(const void* a, const void* w, void* out, int M, int N, int K, float* partial, long floats, int32_t* arrivals,
                               int counters, int shape, hipStream_t stream) {
-    if (M <= 16 || M > 64 || N <= 0 || K <= 0 || partial == nullptr || arrivals == nullptr || (reinterpret_cast<uintptr_t>(partial) & 15) != 0 ||
+    if (M <= 0 || M > 64 || N <= 0 || K <= 0 || partial == nullptr || arrivals == nullptr || (reinterpret_cast<uintptr_t>(partial) & 15) != 0 ||
         !wide_takes(a, w, M, N, K, false)) return -1;
     WideArgs args{(const __bf16*)a, (const __bf16*)w, out, M, N, K, 0, 0, WIDE_PLAIN, 0.f, 0.f, 0, 0, 0, 0, 0, partial, arrivals};
     args.vector_out = ((reinterpret_cast<uintptr_t>(out) | (uintptr_t)N * 2) & 15) == 0 ? 1 : 0;

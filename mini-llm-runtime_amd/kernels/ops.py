@@ -430,9 +430,9 @@ class Kernels:
             self._split = (ws[:SPLIT_PARTIAL_BYTES].view(torch.float32), arrivals)
 
     def split_product(self, rows, columns, k):
-        """Whether a product of 17 to 64 rows is taken by several workgroups a tile: the sums of `few_product`, bit by bit, so not for a
-        model that routes, which keeps the library's where this would replace them."""
-        if self.dtype != torch.bfloat16 or self.routed or not LIBRARY_GEMM_MIN_ROWS < rows <= 64:
+        """Whether a product of up to 64 rows is taken by several workgroups a tile: the sums of the other kernels of few rows, bit by
+        bit, so from 17 rows on not for a model that routes, which keeps the library's where this would replace them."""
+        if self.dtype != torch.bfloat16 or rows > (LIBRARY_GEMM_MIN_ROWS if self.routed else 64):
             return False
         key = (rows, columns, k, "split")
         wins = self._wide_choices.get(key)

@@ -1,4 +1,4 @@
-"""Products of 17 to 64 rows whose tiles several workgroups share: when they are taken, and their bits."""
+"""Products of up to 64 rows whose tiles several workgroups share: when they are taken, and their bits."""
 import ctypes
 
 import pytest
@@ -16,19 +16,20 @@ def without_gpu(routed=False):
 
 
 @pytest.mark.parametrize("rows,columns,inner,taken", [
-    (16, 4096, 12288, False), (17, 4096, 12288, True), (64, 4096, 12288, True), (65, 4096, 12288, False), (64, 4096, 2048, False),
+    (1, 2048, 5632, True), (16, 2048, 3584, True), (16, 2048, 3520, False), (8, 4096, 4096, False), (8, 4096, 5120, True), (8, 8192, 3584, True),
+    (8, 8193, 9216, False), (16, 4096, 12288, True), (17, 4096, 12288, True), (64, 4096, 12288, True), (65, 4096, 12288, False), (64, 4096, 2048, False),
     (64, 2048, 2560, True), (32, 2048, 2560, False), (64, 1024, 2560, False), (32, 2048, 3136, True), (32, 2049, 3136, False),
     (33, 4096, 3136, True), (20, 4097, 4224, False), (64, 6144, 6144, True), (64, 8192, 9216, True), (64, 16384, 14336, True),
     (64, 16385, 14336, False), (64, 4096, 12289, False)])
 def test_long_inner_sizes_of_few_rows_are_shared_out(rows, columns, inner, taken):
     assert without_gpu().split_product(rows, columns, inner) == taken
-    assert not without_gpu(routed=True).split_product(rows, columns, inner)
+    assert without_gpu(routed=True).split_product(rows, columns, inner) == (taken and rows <= 16)
 
 
 # (inner sizes whose last share is one block, a part's last block missing, as many as parts; columns in whole tiles, ragged, odd)
 @pytest.mark.gpu
 @pytest.mark.parametrize("inner", [512, 448, 64 * 25, 64 * 49, 4096, 64 * 67])
-@pytest.mark.parametrize("rows,columns", [(17, 16), (32, 64), (31, 1000), (33, 129), (64, 128), (50, 2047), (64, 4096)])
+@pytest.mark.parametrize("rows,columns", [(1, 64), (5, 40), (16, 1000), (16, 2050), (17, 16), (32, 64), (31, 1000), (33, 129), (64, 128), (50, 2047), (64, 4096)])
 def test_a_shared_tile_has_the_bits_of_one_workgroups(rows, columns, inner):
     k = Kernels(torch.bfloat16)
     gen = torch.Generator().manual_seed(rows + columns + inner)
@@ -38,11 +39,14 @@ def test_a_shared_tile_has_the_bits_of_one_workgroups(rows, columns, inner):
     number, place = ctypes.c_int, lambda t: ctypes.c_void_p(t.data_ptr())
     lib, stream = k._lib("gemm"), ops._stream()
     sizes = (number(rows), number(columns), number(inner))
-    assert lib.mlr_gemm_wide(place(a), place(w), place(want), *sizes, number(0), number(-2), number(0), stream) == 0
+    if rows > 16:
+        assert lib.mlr_gemm_wide(place(a), place(w), place(want), *sizes, number(0), number(-2), number(0), stream) == 0
+    else:
+        assert lib.mlr_gemm(place(a), place(w), place(want), *sizes, number(0), stream) == 0
     partial = torch.full((1 << 23,), float("nan"), device="cuda")
     arrivals = torch.zeros(ops.SPLIT_COUNTERS, dtype=torch.int32, device="cuda")
     taken = 0
-    for shape in range(-1, 7):
+    for shape in range(-1, 10):
         for _ in range(2):                               # (the counters are what they were)
             got = torch.full_like(want, float("nan"))
             code = lib.mlr_gemm_split(place(a), place(w), place(got), *sizes, place(partial), ctypes.c_long(partial.numel()), place(arrivals),
