@@ -28,8 +28,7 @@ template <> __device__ __forceinline__ __bf16 from_float<__bf16>(float x) { retu
 struct alignas(16) vec16 { uint32_t w[4]; };
 
 // Load MLR_VEC consecutive elements (16 bytes, 16-byte aligned) as floats.
-__device__ __forceinline__ void load_vec(const elem_t* p, float* out) {
-    vec16 v = *reinterpret_cast<const vec16*>(p);
+__device__ __forceinline__ void vec_values(const vec16& v, float* out) {
 #if MLR_BF16
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -41,6 +40,8 @@ __device__ __forceinline__ void load_vec(const elem_t* p, float* out) {
     for (int i = 0; i < 4; ++i) out[i] = __uint_as_float(v.w[i]);
 #endif
 }
+
+__device__ __forceinline__ void load_vec(const elem_t* p, float* out) { vec_values(*reinterpret_cast<const vec16*>(p), out); }
 
 __device__ __forceinline__ void store_vec(elem_t* p, const float* in) {
     alignas(16) elem_t tmp[MLR_VEC];

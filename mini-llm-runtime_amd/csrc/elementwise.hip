@@ -168,8 +168,95 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(float* __restrict__ h,
     }
 }
 
-// One workgroup per row as above, 16 bytes per thread and access (width a multiple of MLR_VEC): for few
-// rows of the bfloat16 engine, where the scalar kernel's latency would show.
+// A row of at most REGS MLR_VEC values a thread (64 threads with WAVE, else 256), 16 bytes an access: everything that it needs is asked
+// for at once -- clamped into the row, no load behind a condition -- and stays in registers.  What bounds it is trips to memory, of
+// which there were two and more: the row's pieces one behind the other, the weight (and the row again) behind the sum.  48 rows of
+// 2048 3.1 -> 2.5 us, 64 of 4096 3.9 -> 2.9, 1533 of 5120 18.6 -> 15.9, 2000 of 1024 5.5 -> 5.4; so too the kernels below: 48 x 2048
+// as the sum of two branches 3.3 -> 2.5, with a layer norm 4.9 -> 3.3, in parts with a gate 3.4 -> 3.0 (a Sagopel decoding step of
+// 48 requests 1300 -> 1277).
+template <int REGS, bool WAVE>
+__device__ __forceinline__ void norm_row_kept(float* __restrict__ hrow, const RowAddend more, const float* __restrict__ weight,
+                                              elem_t* __restrict__ orow, int width, float eps, int write_h, float* scratch) {
+    constexpr int QUADS = MLR_VEC / 4;
+    const int t = WAVE ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
+    constexpr int STEP = (WAVE ? 64 : 256) * MLR_VEC;
+    float4 h4[REGS][QUADS], w4[REGS][QUADS], v4[REGS][QUADS];
+    vec16 d[REGS];
+    auto quads = [&](const float* from, float4 (&to)[REGS][QUADS]) {
+#pragma unroll
+        for (int i = 0; i < REGS; ++i)
+#pragma unroll
+            for (int q = 0; q < QUADS; ++q) to[i][q] = *reinterpret_cast<const float4*>(from + min(t * MLR_VEC + STEP * i, width - MLR_VEC) + 4 * q);
+    };
+    constexpr bool EARLY = !WAVE || REGS <= 2;             // (wider rows of many: the registers are worth more)
+    quads(hrow, h4);
+    if (EARLY) quads(weight, w4);
+    if (more.delta) {
+#pragma unroll
+        for (int i = 0; i < REGS; ++i) d[i] = *reinterpret_cast<const vec16*>(more.delta + min(t * MLR_VEC + STEP * i, width - MLR_VEC));
+    }
+    if (more.vector) quads(more.vector, v4);
+    float x[REGS][MLR_VEC], sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < REGS; ++i) {
+#pragma unroll
+        for (int q = 0; q < QUADS; ++q) {
+            x[i][4 * q] = h4[i][q].x; x[i][4 * q + 1] = h4[i][q].y; x[i][4 * q + 2] = h4[i][q].z; x[i][4 * q + 3] = h4[i][q].w;
+        }
+        if (more.delta) {
+            float dv[MLR_VEC];
+            vec_values(d[i], dv);
+#pragma unroll
+            for (int e = 0; e < MLR_VEC; ++e) x[i][e] = fmaf(more.factor, dv[e], x[i][e]);
+        }
+        if (more.vector) {
+#pragma unroll
+            for (int q = 0; q < QUADS; ++q) {
+                x[i][4 * q] += v4[i][q].x; x[i][4 * q + 1] += v4[i][q].y; x[i][4 * q + 2] += v4[i][q].z; x[i][4 * q + 3] += v4[i][q].w;
+            }
+        }
+        if (t * MLR_VEC + STEP * i < width) {
+#pragma unroll
+            for (int e = 0; e < MLR_VEC; ++e) {                // (the fused operations written out: which they are is part of the result)
+                if (WAVE && i == 0 && e < 2) sum = squares(x[0][0], x[0][1]);
+                else sum = __builtin_fmaf(x[i][e], x[i][e], sum);
+            }
+        }
+    }
+    if (write_h && more.any()) {
+#pragma unroll
+        for (int i = 0; i < REGS; ++i)
+            if (t * MLR_VEC + STEP * i < width) {
+#pragma unroll
+                for (int e = 0; e < MLR_VEC; e += 4)
+                    *reinterpret_cast<float4*>(hrow + t * MLR_VEC + STEP * i + e) = make_float4(x[i][e], x[i][e + 1], x[i][e + 2], x[i][e + 3]);
+            }
+    }
+    sum = WAVE ? wave_sum(sum) : block_sum(sum, scratch);
+    if (!isfinite(sum)) {                      // (the same in every thread that serves the row)
+        norm_row_rescaled<WAVE>(hrow, write_h ? RowAddend{nullptr, 1.f, nullptr} : more, weight, orow, width, eps, scratch);
+        return;
+    }
+    const float scale = 1.0f / sqrtf(sum / (float)width + eps);
+    if (!EARLY) quads(weight, w4);
+#pragma unroll
+    for (int i = 0; i < REGS; ++i) {
+        if (t * MLR_VEC + STEP * i >= width) continue;
+        float y[MLR_VEC];
+#pragma unroll
+        for (int q = 0; q < QUADS; ++q) {
+            y[4 * q] = (x[i][4 * q] * scale) * w4[i][q].x;
+            y[4 * q + 1] = (x[i][4 * q + 1] * scale) * w4[i][q].y;
+            y[4 * q + 2] = (x[i][4 * q + 2] * scale) * w4[i][q].z;
+            y[4 * q + 3] = (x[i][4 * q + 3] * scale) * w4[i][q].w;
+        }
+        store_vec(orow + t * MLR_VEC + STEP * i, y);
+    }
+}
+
+// One workgroup per row, 16 bytes per thread and access (width a multiple of MLR_VEC): for few
+// rows of the bfloat16 engine, where the scalar kernel's latency would show.  REGS 0: rows too wide to be kept.
+template <int REGS>
 __global__ __launch_bounds__(256) void add_rmsnorm_row_vec_kernel(float* __restrict__ h, const RowAddend addend,
                                                                   const float* __restrict__ weight,
                                                                   elem_t* __restrict__ out, const int32_t* __restrict__ rows,
@@ -179,6 +266,11 @@ __global__ __launch_bounds__(256) void add_rmsnorm_row_vec_kernel(float* __restr
     const size_t src = rows ? (size_t)rows[r] : (size_t)r;
     float* hrow = h + src * width;
     const RowAddend more = addend.of_row(src, width);
+    elem_t* orow = out + (size_t)r * width;
+    if constexpr (REGS > 0) {
+        norm_row_kept<REGS, false>(hrow, more, weight, orow, width, eps, write_h, scratch);
+        return;
+    }
     float sum = 0.f;
     for (int c = threadIdx.x * MLR_VEC; c < width; c += 256 * MLR_VEC) {
         float x[MLR_VEC];
@@ -199,7 +291,6 @@ __global__ __launch_bounds__(256) void add_rmsnorm_row_vec_kernel(float* __restr
         for (int e = 0; e < MLR_VEC; ++e) sum += x[e] * x[e];
     }
     sum = block_sum(sum, scratch);
-    elem_t* orow = out + (size_t)r * width;
     if (!isfinite(sum)) {
         norm_row_rescaled<false>(hrow, write_h ? RowAddend{nullptr, 1.f, nullptr} : more, weight, orow, width, eps, scratch);
         return;
@@ -225,66 +316,17 @@ __global__ __launch_bounds__(256) void add_rmsnorm_row_vec_kernel(float* __restr
     }
 }
 
-// The same for widths that are a multiple of 8 (bfloat16) or 4 (float), 16 bytes per lane and access:
-// one wavefront per row, four rows per workgroup, the row kept in registers between the two passes
-// when it fits (width <= 64 * MLR_VEC * ROW_REGS), else re-read.
+// The same for many rows of at most 64 * MLR_VEC * ROW_REGS values: one wavefront per row, four rows per workgroup.
 #define ROW_REGS 4
+template <int REGS>
 __global__ __launch_bounds__(256) void add_rmsnorm_vec_kernel(float* __restrict__ h, const RowAddend addend,
                                                               const float* __restrict__ weight,
                                                               elem_t* __restrict__ out, const int32_t* __restrict__ rows,
                                                               int n_out, int width, float eps, int write_h) {
-    const int lane = threadIdx.x & 63;
     const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (r >= n_out) return;
     const size_t src = rows ? (size_t)rows[r] : (size_t)r;
-    float* hrow = h + src * width;
-    const RowAddend more = addend.of_row(src, width);
-    float x[ROW_REGS][MLR_VEC];
-    float sum = 0.f;
-#pragma unroll
-    for (int i = 0; i < ROW_REGS; ++i) {
-        const int c = (lane + 64 * i) * MLR_VEC;
-        if (c < width) {
-#pragma unroll
-            for (int e = 0; e < MLR_VEC; e += 4) {
-                const float4 v = *reinterpret_cast<const float4*>(hrow + c + e);
-                x[i][e] = v.x; x[i][e + 1] = v.y; x[i][e + 2] = v.z; x[i][e + 3] = v.w;
-            }
-            if (more.any()) {
-                more.to_vec(x[i], c);
-                if (write_h) {
-#pragma unroll
-                    for (int e = 0; e < MLR_VEC; e += 4)
-                        *reinterpret_cast<float4*>(hrow + c + e) = make_float4(x[i][e], x[i][e + 1], x[i][e + 2], x[i][e + 3]);
-                }
-            }
-#pragma unroll
-            for (int e = 0; e < MLR_VEC; ++e) sum += x[i][e] * x[i][e];
-        }
-    }
-    sum = wave_sum(sum);
-    elem_t* orow = out + (size_t)r * width;
-    if (!isfinite(sum)) {                      // (the same in every lane of the wavefront, which serves this row alone)
-        norm_row_rescaled<true>(hrow, write_h ? RowAddend{nullptr, 1.f, nullptr} : more, weight, orow, width, eps, nullptr);
-        return;
-    }
-    const float scale = 1.0f / sqrtf(sum / (float)width + eps);
-#pragma unroll
-    for (int i = 0; i < ROW_REGS; ++i) {
-        const int c = (lane + 64 * i) * MLR_VEC;
-        if (c < width) {
-            float y[MLR_VEC];
-#pragma unroll
-            for (int e = 0; e < MLR_VEC; e += 4) {
-                const float4 w = *reinterpret_cast<const float4*>(weight + c + e);
-                y[e] = (x[i][e] * scale) * w.x;
-                y[e + 1] = (x[i][e + 1] * scale) * w.y;
-                y[e + 2] = (x[i][e + 2] * scale) * w.z;
-                y[e + 3] = (x[i][e + 3] * scale) * w.w;
-            }
-            store_vec(orow + c, y);
-        }
-    }
+    norm_row_kept<REGS, true>(h + src * width, addend.of_row(src, width), weight, out + (size_t)r * width, width, eps, write_h, nullptr);
 }
 
 // h[m, :] += factor * delta[m, :] + vector (the last residual sum when nothing is normed afterwards).
@@ -630,6 +672,8 @@ __global__ __launch_bounds__(256) void gated_part_norm_kernel(const float* __res
 
 #if MLR_BF16
 // The same three kernels with 16 bytes per lane and access (bfloat16 engine, widths in multiples of 8).
+// REGS > 0: rows of at most 256 REGS 8 values, asked for at once with everything else and kept (see `norm_row_kept`).
+template <int REGS>
 __global__ __launch_bounds__(256) void add2_rmsnorm2_vec_kernel(float* __restrict__ h, const elem_t* __restrict__ d1,
                                                                 const elem_t* __restrict__ d2, const float* __restrict__ w1,
                                                                 const float* __restrict__ w2, elem_t* __restrict__ out1,
@@ -637,44 +681,89 @@ __global__ __launch_bounds__(256) void add2_rmsnorm2_vec_kernel(float* __restric
     __shared__ float scratch[16];
     const size_t r = blockIdx.x;
     float* hrow = h + r * width;
+    constexpr int KEPT = REGS > 0 ? REGS : 1;
+    float4 lo[KEPT], hi[KEPT];
+    vec16 a4[KEPT], b4[KEPT];
+    float g1[KEPT][8], g2[KEPT][8], kept[KEPT][8];
     float sum = 0.f;
-    for (int c = threadIdx.x * 8; c < width; c += 256 * 8) {
-        float x[8], a[8];
-        const float4 lo = *reinterpret_cast<const float4*>(hrow + c), hi = *reinterpret_cast<const float4*>(hrow + c + 4);
-        x[0] = lo.x; x[1] = lo.y; x[2] = lo.z; x[3] = lo.w; x[4] = hi.x; x[5] = hi.y; x[6] = hi.z; x[7] = hi.w;
+    auto add_up = [&](int i, int c, float (&x)[8]) {       // piece i of the row, with what is added to it, written back at c
+        x[0] = lo[i].x; x[1] = lo[i].y; x[2] = lo[i].z; x[3] = lo[i].w; x[4] = hi[i].x; x[5] = hi[i].y; x[6] = hi[i].z; x[7] = hi[i].w;
         if (d1 || d2) {
-            if (d1) load_vec(d1 + r * width + c, a);
+            float a[8];
+            if (d1) vec_values(a4[i], a);
             else {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) a[e] = 0.f;
             }
             if (d2) {
                 float b[8];
-                load_vec(d2 + r * width + c, b);
+                vec_values(b4[i], b);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) a[e] += b[e];
             }
 #pragma unroll
             for (int e = 0; e < 8; ++e) x[e] += a[e];
-            *reinterpret_cast<float4*>(hrow + c) = make_float4(x[0], x[1], x[2], x[3]);
-            *reinterpret_cast<float4*>(hrow + c + 4) = make_float4(x[4], x[5], x[6], x[7]);
+            if (c < width) {
+                *reinterpret_cast<float4*>(hrow + c) = make_float4(x[0], x[1], x[2], x[3]);
+                *reinterpret_cast<float4*>(hrow + c + 4) = make_float4(x[4], x[5], x[6], x[7]);
+            }
         }
+        if (c < width) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) sum += x[e] * x[e];
-    }
-    sum = block_sum(sum, scratch);
-    const float scale = 1.0f / sqrtf(sum / (float)width + eps);
-    for (int c = threadIdx.x * 8; c < width; c += 256 * 8) {       // (this thread wrote these elements of h itself)
-        float x[8], y[8];
-        const float4 lo = *reinterpret_cast<const float4*>(hrow + c), hi = *reinterpret_cast<const float4*>(hrow + c + 4);
-        x[0] = lo.x; x[1] = lo.y; x[2] = lo.z; x[3] = lo.w; x[4] = hi.x; x[5] = hi.y; x[6] = hi.z; x[7] = hi.w;
+            for (int e = 0; e < 8; ++e) sum = __builtin_fmaf(x[e], x[e], sum);
+        }
+    };
+    auto ask = [&](int i, int c) {
+        lo[i] = *reinterpret_cast<const float4*>(hrow + c);
+        hi[i] = *reinterpret_cast<const float4*>(hrow + c + 4);
+        if (d1) a4[i] = *reinterpret_cast<const vec16*>(d1 + r * width + c);
+        if (d2) b4[i] = *reinterpret_cast<const vec16*>(d2 + r * width + c);
+    };
+    auto weights = [&](int i, int c) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) y[e] = (x[e] * scale) * w1[c + e];
+        for (int e = 0; e < 8; ++e) g1[i][e] = w1[c + e];
+        if (out2) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) g2[i][e] = w2[c + e];
+        }
+    };
+    float scale = 0.f;
+    auto finish = [&](int i, int c, const float (&x)[8]) {
+        float y[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[e] = (x[e] * scale) * g1[i][e];
         store_vec(out1 + r * width + c, y);
         if (out2) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) y[e] = (x[e] * scale) * w2[c + e];
+            for (int e = 0; e < 8; ++e) y[e] = (x[e] * scale) * g2[i][e];
             store_vec(out2 + r * width + c, y);
+        }
+    };
+    if constexpr (REGS > 0) {
+#pragma unroll
+        for (int i = 0; i < REGS; ++i) ask(i, min((int)threadIdx.x * 8 + 2048 * i, width - 8));
+#pragma unroll
+        for (int i = 0; i < REGS; ++i) weights(i, min((int)threadIdx.x * 8 + 2048 * i, width - 8));
+#pragma unroll
+        for (int i = 0; i < REGS; ++i) add_up(i, (int)threadIdx.x * 8 + 2048 * i, kept[i]);
+    } else {
+        for (int c = threadIdx.x * 8; c < width; c += 256 * 8) {
+            ask(0, c);
+            add_up(0, c, kept[0]);
+        }
+    }
+    sum = block_sum(sum, scratch);
+    scale = 1.0f / sqrtf(sum / (float)width + eps);
+    if constexpr (REGS > 0) {
+#pragma unroll
+        for (int i = 0; i < REGS; ++i)
+            if ((int)threadIdx.x * 8 + 2048 * i < width) finish(i, (int)threadIdx.x * 8 + 2048 * i, kept[i]);
+    } else {
+        for (int c = threadIdx.x * 8; c < width; c += 256 * 8) {       // (this thread wrote these elements of h itself)
+            const float4 first = *reinterpret_cast<const float4*>(hrow + c), second = *reinterpret_cast<const float4*>(hrow + c + 4);
+            const float x[8] = {first.x, first.y, first.z, first.w, second.x, second.y, second.z, second.w};
+            weights(0, c);
+            finish(0, c, x);
         }
     }
 }
@@ -763,7 +852,7 @@ __global__ __launch_bounds__(256) void gated_part_norm_vec_kernel(const float* _
 // neighbouring lanes (a power of two up to 64) serve a part, or with BLOCK a whole workgroup; a lane takes eight values at
 // a time, at most PART_CHUNKS times.
 #define PART_CHUNKS 4
-template <bool BLOCK>
+template <bool BLOCK, int CHUNKS>
 __global__ __launch_bounds__(256) void gated_part_norm_reg_kernel(const float* __restrict__ y, const elem_t* __restrict__ gate,
                                                                   long gate_stride, const float* __restrict__ weight,
                                                                   elem_t* __restrict__ out, int rows, int width, int part,
@@ -775,37 +864,45 @@ __global__ __launch_bounds__(256) void gated_part_norm_reg_kernel(const float* _
     const bool live = unit < (size_t)rows * parts;
     const size_t m = live ? unit / parts : 0;
     const int c0 = live ? (int)(unit % parts) * part : 0;
-    float v[PART_CHUNKS][8], g[PART_CHUNKS][8];
+    // (everything is asked for at once, clamped into the part, no load behind a condition; see `norm_row_kept`)
+    float v[CHUNKS][8], g[CHUNKS][8], w[CHUNKS][8];
+    float4 lo[CHUNKS], hi[CHUNKS];
+    vec16 gate16[CHUNKS];
     float sum = 0.f;
 #pragma unroll
-    for (int i = 0; i < PART_CHUNKS; ++i) {
-        const int c = (lane + lanes * i) * 8;
-        if (live && c < part) {
-            const float* p = y + m * width + c0 + c;
-            const float4 lo = *reinterpret_cast<const float4*>(p), hi = *reinterpret_cast<const float4*>(p + 4);
-            v[i][0] = lo.x; v[i][1] = lo.y; v[i][2] = lo.z; v[i][3] = lo.w; v[i][4] = hi.x; v[i][5] = hi.y; v[i][6] = hi.z; v[i][7] = hi.w;
-            load_vec(gate + m * gate_stride + c0 + c, g[i]);
+    for (int i = 0; i < CHUNKS; ++i) {
+        const int c = min((lane + lanes * i) * 8, part - 8);
+        const float* p = y + m * width + c0 + c;
+        lo[i] = *reinterpret_cast<const float4*>(p);
+        hi[i] = *reinterpret_cast<const float4*>(p + 4);
+        gate16[i] = *reinterpret_cast<const vec16*>(gate + m * gate_stride + c0 + c);
+    }
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float sg = 1.0f / (1.0f + expf(-g[i][e]));
-                g[i][e] = gate_kind == 0 ? g[i][e] * sg : sg;
-                if (gate_first) v[i][e] *= g[i][e];
-                sum += v[i][e] * v[i][e];
-            }
+    for (int i = 0; i < CHUNKS; ++i) row_weights<8>(weight, (c0 + min((lane + lanes * i) * 8, part - 8)) % period, w[i]);      // (period is a multiple of 8: eight neighbours do not wrap)
+#pragma unroll
+    for (int i = 0; i < CHUNKS; ++i) {
+        const bool in = live && (lane + lanes * i) * 8 < part;
+        v[i][0] = lo[i].x; v[i][1] = lo[i].y; v[i][2] = lo[i].z; v[i][3] = lo[i].w; v[i][4] = hi[i].x; v[i][5] = hi[i].y; v[i][6] = hi[i].z; v[i][7] = hi[i].w;
+        vec_values(gate16[i], g[i]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float sg = 1.0f / (1.0f + expf(-g[i][e]));
+            g[i][e] = gate_kind == 0 ? g[i][e] * sg : sg;
+            if (gate_first) v[i][e] *= g[i][e];
+            if (in && e > 0) sum = i == 0 && e == 1 ? squares(v[0][0], v[0][1]) : __builtin_fmaf(v[i][e], v[i][e], e == 1 ? __builtin_fmaf(v[i][0], v[i][0], sum) : sum);
         }
     }
     if (BLOCK) sum = block_sum(sum, scratch);
     else sum = group_sum(sum, group);
     const float scale = 1.0f / sqrtf(sum / (float)part + eps);
 #pragma unroll
-    for (int i = 0; i < PART_CHUNKS; ++i) {
+    for (int i = 0; i < CHUNKS; ++i) {
         const int c = (lane + lanes * i) * 8;
         if (live && c < part) {
-            float o[8], w[8];
-            row_weights<8>(weight, (c0 + c) % period, w);      // (period is a multiple of 8: eight neighbours do not wrap)
+            float o[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                o[e] = (v[i][e] * scale) * w[e];
+                o[e] = (v[i][e] * scale) * w[i][e];
                 if (!gate_first) o[e] *= g[i][e];
             }
             store_vec(out + m * width + c0 + c, o);
@@ -865,30 +962,46 @@ template <int VEC> __device__ __forceinline__ void store_elems(elem_t* p, const 
 // One workgroup a row, VEC values an access.  Thread t adds up the values t, t + 256, .. of the row, however it was read: a
 // router behind the norm turns on the last bits of it, so the order of the sum is part of the result.  A row of up to LN_ROW
 // values is read once, with VEC 4 through LDS; a longer one is read again for each sum, a value at a time.  1777 rows of 2048
-// values: 12.0 us one value at a time, 9.7 with four.
+// values: 12.0 us one value at a time, 9.7 with four, 8.8 with everything asked for at once.
+// CHUNKS (VEC 4): accesses of a thread, all that the row needs asked for at once, clamped into it, no load behind a condition that
+// differs between threads (see `norm_row_kept`).
 #define LN_ROW 4096
-template <int VEC>
+template <int VEC, int CHUNKS>
 __global__ __launch_bounds__(256) void layernorm_kernel(const elem_t* __restrict__ xe, const float* __restrict__ xf,
                                                         const float* __restrict__ weight, const float* __restrict__ bias,
                                                         const int32_t* __restrict__ rows, float* __restrict__ acc,
                                                         elem_t* __restrict__ cast, elem_t* __restrict__ out, int width,
                                                         float eps, float out_scale) {
     __shared__ float scratch[16];
-    __shared__ __attribute__((aligned(16))) float row[VEC > 1 ? LN_ROW : 1];
-    constexpr int HELD = LN_ROW / 256;
+    __shared__ __attribute__((aligned(16))) float row[VEC > 1 ? CHUNKS * VEC * 256 : 1];
+    constexpr int HELD = CHUNKS * VEC;
     const int r = blockIdx.x;
     const size_t src = rows ? (size_t)rows[r] : (size_t)r;
     const bool kept = width <= LN_ROW;
     float x[HELD / VEC][VEC];                              // the thread's places as it reads and writes them
+    float w[HELD / VEC][VEC], b[HELD / VEC][VEC], h[HELD / VEC][VEC];
     auto read = [&](int c, float* v) {
         if (xe) load_elems<VEC>(xe + src * width + c, v);
         else load_floats<VEC>(xf + src * width + c, v);
     };
-    if (kept) {
+    auto meet = [&](int j) { return min((int)(threadIdx.x + j * 256) * VEC, width - VEC); };
+    if (VEC > 1) {
 #pragma unroll
-        for (int j = 0; j < HELD / VEC; ++j) {
-            const int c = (threadIdx.x + j * 256) * VEC;
-            if (c < width) read(c, x[j]);
+        for (int j = 0; j < CHUNKS; ++j) read(meet(j), x[j]);
+#pragma unroll
+        for (int j = 0; j < CHUNKS; ++j) {
+            load_floats<VEC>(weight + meet(j), w[j]);
+            if (bias) load_floats<VEC>(bias + meet(j), b[j]);
+            if (acc != nullptr) load_floats<VEC>(acc + src * width + meet(j), h[j]);
+        }
+    }
+    if (kept) {
+        if (VEC == 1) {
+#pragma unroll
+            for (int j = 0; j < HELD / VEC; ++j) {
+                const int c = (threadIdx.x + j * 256) * VEC;
+                if (c < width) read(c, x[j]);
+            }
         }
         if (VEC > 1) {
 #pragma unroll
@@ -925,33 +1038,38 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const elem_t* __restrict
         }
     }
     const float inv = 1.0f / sqrtf(block_sum(dev, scratch) / (float)width + eps);
-    auto finish = [&](int c, const float* v) {
-        float y[VEC], w[VEC], b[VEC];
-        load_floats<VEC>(weight + c, w);
-        if (bias) load_floats<VEC>(bias + c, b);
+    auto rest = [&](int c, int j) {                        // (without VEC: a value at a time, as it is needed)
+        load_floats<VEC>(weight + c, w[j]);
+        if (bias) load_floats<VEC>(bias + c, b[j]);
+        if (acc != nullptr) load_floats<VEC>(acc + src * width + c, h[j]);
+    };
+    auto finish = [&](int c, int j) {
+        float y[VEC];
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) y[e] = (((v[e] - mean) * inv) * w[e] + (bias ? b[e] : 0.f)) * out_scale;
+        for (int e = 0; e < VEC; ++e) y[e] = (((x[j][e] - mean) * inv) * w[j][e] + (bias ? b[j][e] : 0.f)) * out_scale;
         if (acc == nullptr) {
             store_elems<VEC>(out + (size_t)r * width + c, y);
             return;
         }
-        float h[VEC];
-        load_floats<VEC>(acc + src * width + c, h);
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) h[e] += y[e];
-        store_floats<VEC>(acc + src * width + c, h);
-        if (cast != nullptr) store_elems<VEC>(cast + src * width + c, h);
+        for (int e = 0; e < VEC; ++e) h[j][e] += y[e];
+        store_floats<VEC>(acc + src * width + c, h[j]);
+        if (cast != nullptr) store_elems<VEC>(cast + src * width + c, h[j]);
     };
     if (kept) {
 #pragma unroll
         for (int j = 0; j < HELD / VEC; ++j) {
             const int c = (threadIdx.x + j * 256) * VEC;
-            if (c < width) finish(c, x[j]);
+            if (c < width) {
+                if (VEC == 1) rest(c, j);
+                finish(c, j);
+            }
         }
     } else {
         for (int c = threadIdx.x * VEC; c < width; c += 256 * VEC) {
             read(c, x[0]);
-            finish(c, x[0]);
+            rest(c, 0);
+            finish(c, 0);
         }
     }
 }
@@ -973,82 +1091,90 @@ __global__ void plain_act_kernel(const elem_t* __restrict__ x, elem_t* __restric
 }
 
 // x = h + (d1 + d2) (each may be null), written back to h when one is given; out = layernorm(x) * weight (+ bias): the two
-// branches of a block and the norm that follows in one pass, the row kept in registers (up to 4 VEC LN2_REGS values a
-// lane's share of the row; wider rows are read again).  One workgroup a row; VEC 4: 16-byte float accesses.
-#define LN2_REGS 8
-template <int VEC>
+// branches of a block and the norm that follows in one pass, the row kept in registers.  One workgroup a row; VEC 4: 16-byte float accesses.
+// REGS: pieces of VEC values that a thread keeps, everything that they need asked for at once (see `norm_row_kept`); 0: wider rows.
+template <int VEC, int REGS>
 __global__ __launch_bounds__(256) void add2_layernorm_kernel(float* __restrict__ h, const elem_t* __restrict__ d1,
                                                              const elem_t* __restrict__ d2, const float* __restrict__ weight,
                                                              const float* __restrict__ bias, elem_t* __restrict__ out,
                                                              int width, float eps) {
     __shared__ float scratch[16];
     const size_t row = (size_t)blockIdx.x * width;
-    const bool kept = width <= LN2_REGS * VEC * 256;
-    float x[LN2_REGS][VEC];
-    auto read = [&](int c, float* v) {
-        load_floats<VEC>(h + row + c, v);
-        float a[VEC], b[VEC];
-        if (d1 != nullptr) load_elems<VEC>(d1 + row + c, a);
-        if (d2 != nullptr) load_elems<VEC>(d2 + row + c, b);
+    constexpr int KEPT = REGS > 0 ? REGS : 1;
+    float x[KEPT][VEC], a[KEPT][VEC], b[KEPT][VEC], w[KEPT][VEC], add[KEPT][VEC];
+    auto ask = [&](int i, int c) {
+        load_floats<VEC>(h + row + c, x[i]);
+        if (d1 != nullptr) load_elems<VEC>(d1 + row + c, a[i]);
+        if (d2 != nullptr) load_elems<VEC>(d2 + row + c, b[i]);
+    };
+    auto weights = [&](int i, int c) {
+        load_floats<VEC>(weight + c, w[i]);
+        if (bias != nullptr) load_floats<VEC>(bias + c, add[i]);
+    };
+    auto place = [&](int i) { return (int)(threadIdx.x + i * 256) * VEC; };
+    float sum = 0.f;
+    auto first = [&](int i, int c) {
 #pragma unroll
         for (int e = 0; e < VEC; ++e)
-            if (d1 != nullptr || d2 != nullptr) v[e] += d2 == nullptr ? a[e] : d1 == nullptr ? b[e] : a[e] + b[e];
-    };
-    float sum = 0.f;
-    auto first = [&](int c, float* v) {
-        read(c, v);
-        if (d1 != nullptr || d2 != nullptr) store_floats<VEC>(h + row + c, v);
+            if (d1 != nullptr || d2 != nullptr) x[i][e] += d2 == nullptr ? a[i][e] : d1 == nullptr ? b[i][e] : a[i][e] + b[i][e];
+        if (c >= width) return;
+        if (d1 != nullptr || d2 != nullptr) store_floats<VEC>(h + row + c, x[i]);
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) sum += v[e];
+        for (int e = 0; e < VEC; ++e) sum += x[i][e];
     };
-    if (kept) {
+    if (REGS > 0) {
 #pragma unroll
-        for (int j = 0; j < LN2_REGS; ++j) {
-            const int c = (threadIdx.x + j * 256) * VEC;
-            if (c < width) first(c, x[j]);
-        }
+        for (int i = 0; i < REGS; ++i) ask(i, min(place(i), width - VEC));
+#pragma unroll
+        for (int i = 0; i < REGS; ++i) weights(i, min(place(i), width - VEC));
+#pragma unroll
+        for (int i = 0; i < REGS; ++i) first(i, place(i));
     } else {
-        for (int c = threadIdx.x * VEC; c < width; c += 256 * VEC) first(c, x[0]);
+        for (int c = threadIdx.x * VEC; c < width; c += 256 * VEC) {
+            ask(0, c);
+            first(0, c);
+        }
     }
     const float mean = block_sum(sum, scratch) / (float)width;
     float dev = 0.f;
-    auto second = [&](const float* v) {
+    auto second = [&](int i) {
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) dev += (v[e] - mean) * (v[e] - mean);
+        for (int e = 0; e < VEC; ++e) {                    // (which operations are fused is part of the result)
+            const float d = x[i][e] - mean;
+            if (VEC > 1 && REGS > 0 && i == 0 && e < 2) dev = squares(x[0][0] - mean, x[0][VEC > 1 ? 1 : 0] - mean);
+            else dev = __builtin_fmaf(d, d, dev);
+        }
     };
-    if (kept) {
+    if (REGS > 0) {
 #pragma unroll
-        for (int j = 0; j < LN2_REGS; ++j)
-            if ((int)(threadIdx.x + j * 256) * VEC < width) second(x[j]);
+        for (int i = 0; i < REGS; ++i)
+            if (place(i) < width) second(i);
     } else {
         for (int c = threadIdx.x * VEC; c < width; c += 256 * VEC) {
             load_floats<VEC>(h + row + c, x[0]);           // (this thread's own values: complete)
-            second(x[0]);
+            second(0);
         }
     }
     const float inv = 1.0f / sqrtf(block_sum(dev, scratch) / (float)width + eps);
-    auto third = [&](int c, const float* v) {
-        float w[VEC], y[VEC];
-        load_floats<VEC>(weight + c, w);
+    auto third = [&](int i, int c) {
+        float y[VEC];
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) y[e] = ((v[e] - mean) * inv) * w[e];
+        for (int e = 0; e < VEC; ++e) y[e] = opaque(((x[i][e] - mean) * inv) * w[i][e]);      // (the bias is added to the rounded product)
         if (bias != nullptr) {
-            load_floats<VEC>(bias + c, w);
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) y[e] += w[e];
+            for (int e = 0; e < VEC; ++e) y[e] += add[i][e];
         }
         store_elems<VEC>(out + row + c, y);
     };
-    if (kept) {
+    if (REGS > 0) {
 #pragma unroll
-        for (int j = 0; j < LN2_REGS; ++j) {
-            const int c = (threadIdx.x + j * 256) * VEC;
-            if (c < width) third(c, x[j]);
-        }
+        for (int i = 0; i < REGS; ++i)
+            if (place(i) < width) third(i, place(i));
     } else {
         for (int c = threadIdx.x * VEC; c < width; c += 256 * VEC) {
             load_floats<VEC>(h + row + c, x[0]);
-            third(c, x[0]);
+            weights(0, c);
+            third(0, c);
         }
     }
 }
@@ -1219,13 +1345,17 @@ int mlr_add_rmsnorm(float* h, const void* delta, float factor, const float* vect
     const RowAddend addend{(const elem_t*)delta, factor, vector};
     // (the float engine keeps its one order of additions for every batch size)
     if (MLR_BF16 && width % MLR_VEC == 0 && width <= 64 * MLR_VEC * ROW_REGS && n_out >= 64) {
-        add_rmsnorm_vec_kernel<<<(n_out + 3) / 4, 256, 0, stream>>>(h, addend, weight, (elem_t*)out,
-                                                                     rows, n_out, width, eps, write_h);
+        const int regs = (width + 64 * MLR_VEC - 1) / (64 * MLR_VEC);
+        auto* kernel = regs == 1 ? add_rmsnorm_vec_kernel<1> : regs == 2 ? add_rmsnorm_vec_kernel<2> : regs == 3 ? add_rmsnorm_vec_kernel<3>
+                                                                                                                : add_rmsnorm_vec_kernel<ROW_REGS>;
+        kernel<<<(n_out + 3) / 4, 256, 0, stream>>>(h, addend, weight, (elem_t*)out, rows, n_out, width, eps, write_h);
         return (int)hipGetLastError();
     }
     if (MLR_BF16 && width % MLR_VEC == 0) {
-        add_rmsnorm_row_vec_kernel<<<n_out, 256, 0, stream>>>(h, addend, weight, (elem_t*)out, rows,
-                                                              width, eps, write_h);
+        const int regs = (width + 256 * MLR_VEC - 1) / (256 * MLR_VEC);
+        auto* kernel = regs == 1 ? add_rmsnorm_row_vec_kernel<1> : regs == 2 ? add_rmsnorm_row_vec_kernel<2> : regs == 3 ? add_rmsnorm_row_vec_kernel<3>
+                                                                                                                        : add_rmsnorm_row_vec_kernel<0>;
+        kernel<<<n_out, 256, 0, stream>>>(h, addend, weight, (elem_t*)out, rows, width, eps, write_h);
         return (int)hipGetLastError();
     }
     if (width <= 256 * 4) add_rmsnorm_kernel<4><<<n_out, 256, 0, stream>>>(h, addend, weight, (elem_t*)out, rows, width, eps, write_h);
@@ -1340,8 +1470,10 @@ int mlr_add2_rmsnorm2(float* h, const void* d1, const void* d2, const float* w1,
     if ((out2 == nullptr) != (w2 == nullptr)) return -1;
 #if MLR_BF16
     if (width % 8 == 0) {
-        add2_rmsnorm2_vec_kernel<<<rows, 256, 0, stream>>>(h, (const elem_t*)d1, (const elem_t*)d2, w1, w2, (elem_t*)out1,
-                                                           (elem_t*)out2, width, eps);
+        // (2048 rows of 2048: 10.9 us, kept 11.2; 2000 of 1024 6.6 and 6.3, 48 of 2048 3.3 and 2.5)
+        const bool kept = width <= 1024 || rows <= 1024;
+        auto* kernel = kept && width <= 2048 ? add2_rmsnorm2_vec_kernel<1> : kept && width <= 4096 ? add2_rmsnorm2_vec_kernel<2> : add2_rmsnorm2_vec_kernel<0>;
+        kernel<<<rows, 256, 0, stream>>>(h, (const elem_t*)d1, (const elem_t*)d2, w1, w2, (elem_t*)out1, (elem_t*)out2, width, eps);
         return (int)hipGetLastError();
     }
 #endif
@@ -1384,12 +1516,11 @@ int mlr_gated_part_norm(const float* y, const void* gate, long gate_stride, cons
             while (group < 64 && group * 8 < part) group *= 2;
             const size_t threads = units * (block ? 256 : group);
             const unsigned grid = (unsigned)((threads + 255) / 256);
-            if (block)
-                gated_part_norm_reg_kernel<true><<<grid, 256, 0, stream>>>(y, (const elem_t*)gate, gate_stride, weight, (elem_t*)out, rows,
-                                                                           width, part, period, eps, gate_first, gate_kind, 256);
-            else
-                gated_part_norm_reg_kernel<false><<<grid, 256, 0, stream>>>(y, (const elem_t*)gate, gate_stride, weight, (elem_t*)out, rows,
-                                                                            width, part, period, eps, gate_first, gate_kind, group);
+            const int chunks = (part + 8 * (block ? 256 : group) - 1) / (8 * (block ? 256 : group));
+            auto* kernel = block ? (chunks == 1 ? gated_part_norm_reg_kernel<true, 1> : chunks == 2 ? gated_part_norm_reg_kernel<true, 2> : gated_part_norm_reg_kernel<true, PART_CHUNKS>)
+                                 : (chunks == 1 ? gated_part_norm_reg_kernel<false, 1> : gated_part_norm_reg_kernel<false, 2>);
+            kernel<<<grid, 256, 0, stream>>>(y, (const elem_t*)gate, gate_stride, weight, (elem_t*)out, rows, width, part, period, eps, gate_first,
+                                             gate_kind, block ? 256 : group);
             return (int)hipGetLastError();
         }
         if (part >= 2048)
@@ -1416,10 +1547,10 @@ int mlr_layernorm(const void* xe, const float* xf, const float* weight, const fl
     if ((xe == nullptr) == (xf == nullptr) || (acc == nullptr && out == nullptr) || (acc != nullptr && rows != nullptr))
         return -1;
     if (width % 4 == 0 && width <= LN_ROW && aligned16(xe, xf, weight, bias, acc, cast, out))
-        layernorm_kernel<4><<<n_out, 256, 0, stream>>>((const elem_t*)xe, xf, weight, bias, rows, acc, (elem_t*)cast,
-                                                       (elem_t*)out, width, eps, out_scale);
+        (width <= 1024 ? layernorm_kernel<4, 1> : width <= 2048 ? layernorm_kernel<4, 2> : layernorm_kernel<4, LN_ROW / 1024>)
+            <<<n_out, 256, 0, stream>>>((const elem_t*)xe, xf, weight, bias, rows, acc, (elem_t*)cast, (elem_t*)out, width, eps, out_scale);
     else
-        layernorm_kernel<1><<<n_out, 256, 0, stream>>>((const elem_t*)xe, xf, weight, bias, rows, acc, (elem_t*)cast,
+        layernorm_kernel<1, LN_ROW / 256><<<n_out, 256, 0, stream>>>((const elem_t*)xe, xf, weight, bias, rows, acc, (elem_t*)cast,
                                                        (elem_t*)out, width, eps, out_scale);
     return (int)hipGetLastError();
 }
@@ -1444,12 +1575,11 @@ int mlr_plain_act(const void* x, void* out, size_t count, int act, hipStream_t s
 int mlr_add2_layernorm(float* h, const void* d1, const void* d2, const float* weight, const float* bias, void* out, int rows,
                        int width, float eps, hipStream_t stream) {
     if (rows <= 0) return 0;
-    if (width % 4 == 0 && aligned16(h, d1, d2, weight, bias, out))
-        add2_layernorm_kernel<4><<<rows, 256, 0, stream>>>(h, (const elem_t*)d1, (const elem_t*)d2, weight, bias,
-                                                           (elem_t*)out, width, eps);
-    else
-        add2_layernorm_kernel<1><<<rows, 256, 0, stream>>>(h, (const elem_t*)d1, (const elem_t*)d2, weight, bias,
-                                                           (elem_t*)out, width, eps);
+    const bool vec = width % 4 == 0 && aligned16(h, d1, d2, weight, bias, out);
+    auto* kernel = vec ? (width <= 1024 ? add2_layernorm_kernel<4, 1> : width <= 2048 ? add2_layernorm_kernel<4, 2> : width <= 4096 ? add2_layernorm_kernel<4, 4>
+                          : width <= 6144 ? add2_layernorm_kernel<4, 6> : width <= 8192 ? add2_layernorm_kernel<4, 8> : add2_layernorm_kernel<4, 0>)
+                       : (width <= 2048 ? add2_layernorm_kernel<1, 8> : add2_layernorm_kernel<1, 0>);
+    kernel<<<rows, 256, 0, stream>>>(h, (const elem_t*)d1, (const elem_t*)d2, weight, bias, (elem_t*)out, width, eps);
     return (int)hipGetLastError();
 }
 
