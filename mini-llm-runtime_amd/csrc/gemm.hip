@@ -1798,10 +1798,24 @@ static bool few_wins(int M, int N, int K, bool gated) {
     return K <= 4096 && (gated ? N > 1024 : N >= 4096);
 }
 
+// Whether up to 16 rows are these tiles' as well, instead of `gemm_skinny_kernel` (the same bits), whose wavefronts make a trip to memory
+// for every 256 k of their part, one behind the other.  Measured on 220 drawn sizes at 1, 8 and 16 rows, weights cold, against it, geometric
+// mean: gated from k = 1024 on 0.85 (0.71 to 1.07; 0.99 to 1.08 below), plain from 1408 on, of more than 4352 columns from 1024 on, 0.90
+// (0.68 to 1.09; 0.97 to 1.12 below).  Not a gate over many columns of a long k (12288 x 4096: 36.3 and 39.5 us), nor beyond the sizes drawn.
+// 8 x 2 * 5632 x 2048 14.8 -> 11.7 us, 8 x 2 * 704 x 2048 7.4 -> 6.0, 8 x 6144 x 2048 8.8 -> 7.3, 8 x 2048 x 2048 5.9 -> 5.3.
+static bool narrow_wins(int M, int N, int K, bool gated) {
+    if (M <= 0 || M > 16 || N < 384 || N > 16384 || K > 6144) return false;
+    return gated ? K >= 1024 && (K <= 3072 || N <= 8192) : K >= 1408 || (K >= 1024 && N > 4352);
+}
+
 // Whether the kernel takes these operands at all: whole blocks of k, 32-bit offsets, rows that start on 16 bytes.
 static bool wide_takes(const void* a, const void* w, int M, int N, int K, bool gated) {
     return K % WIDE_BK == 0 && (unsigned long long)M * K < (1ull << 31) && (unsigned long long)N * (gated ? 2 : 1) * K < (1ull << 31) &&
            ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(w)) & 15) == 0;
+}
+
+extern "C" int mlr_gemm_narrow_wins(int M, int N, int K, int gated) {
+    return N > 0 && K > 0 && wide_takes(nullptr, nullptr, M, N, K, gated != 0) && narrow_wins(M, N, K, gated != 0) ? 1 : 0;
 }
 
 enum { WIDE_MANY = -1, WIDE_FEW = -2 };      // the tile with the least predicted time, of one sum over k or of the forms for 17 to 64 rows

@@ -395,7 +395,8 @@ class Kernels:
             _ok(self._lib("gemm").mlr_gemm_split(_p(a), _p(w), _p(out), _c_int(m), _c_int(n), _c_int(k), _p(partial),
                                                  ctypes.c_long(partial.numel()), _p(arrivals), _c_int(arrivals.numel()), _c_int(-1), _stream()), "gemm")
             return
-        if m <= 64 and out.dtype == torch.bfloat16 and (self.few_product(m, n, k) or self.wide_product(m, n, k)) and _on16(a, w):
+        if m <= 64 and out.dtype == torch.bfloat16 and (self.narrow_product(m, n, k) or self.few_product(m, n, k) or self.wide_product(m, n, k)) \
+                and _on16(a, w):
             _ok(self._lib("gemm").mlr_gemm_wide(_p(a), _p(w), _p(out), _c_int(m), _c_int(n), _c_int(k), _c_int(0),
                                                 _c_int(-1 if self.one_sum(m, k) else -2), _c_int(0), _stream()), "gemm")
             return
@@ -499,6 +500,19 @@ class Kernels:
         wins = self._wide_choices.get(key)
         if wins is None:
             wins = bool(self._lib("gemm").mlr_gemm_wide_wins(_c_int(rows), _c_int(columns), _c_int(k), _c_int(self.WIDE_ACTS[act]), _c_int(0)))
+            if len(self._wide_choices) >= WIDE_CHOICES_KEPT:
+                self._wide_choices.clear()
+            self._wide_choices[key] = wins
+        return wins
+
+    def narrow_product(self, rows, columns, k, gated=False):
+        """Whether the many-row kernel's narrow tiles take up to 16 rows, too, in place of the kernel that streams the weight, with its bits."""
+        if self.dtype != torch.bfloat16 or rows > LIBRARY_GEMM_MIN_ROWS:
+            return False
+        key = (rows, columns, k, gated, "narrow")
+        wins = self._wide_choices.get(key)
+        if wins is None:
+            wins = bool(self._lib("gemm").mlr_gemm_narrow_wins(_c_int(rows), _c_int(columns), _c_int(k), _c_int(1 if gated else 0)))
             if len(self._wide_choices) >= WIDE_CHOICES_KEPT:
                 self._wide_choices.clear()
             self._wide_choices[key] = wins
@@ -625,7 +639,7 @@ class Kernels:
     @timed("gemm", _gemm_work)
     def _gemm_gated_silu(self, a, w, out):
         (m, k), two_n = a.shape, w.shape[0]
-        if self.few_product(m, two_n // 2, k, "silu") and _on16(a, w):
+        if (self.narrow_product(m, two_n // 2, k, gated=True) or self.few_product(m, two_n // 2, k, "silu")) and _on16(a, w):
             _ok(self._lib("gemm").mlr_gemm_wide(_p(a), _p(w), _p(out), _c_int(m), _c_int(two_n // 2), _c_int(k), _c_int(0), _c_int(-2),
                                                 _c_int(1), _stream()), "gemm_gated_silu")
             return
