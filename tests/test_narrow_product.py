@@ -46,3 +46,22 @@ def test_narrow_tiles_have_the_bits_of_the_streaming_kernel(rows, columns, inner
         assert lib.mlr_gemm(place(a), place(w), place(want), *sizes, ctypes.c_int(0), ops._stream()) == 0
         k.gemm(a, w, got)
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+# (columns whose address is not on 16 bytes go to the streaming kernel: its bits)
+@pytest.mark.gpu
+@pytest.mark.parametrize("columns,inner", [(704, 1024), (1000, 1088), (5632, 2048), (3000, 2112)])
+@pytest.mark.parametrize("rows", [1, 7, 16, 17, 32, 64])
+def test_a_clamped_gate_in_narrow_tiles_has_the_bits_of_the_streaming_kernel(columns, inner, rows):
+    k = Kernels(torch.bfloat16)
+    gen = torch.Generator().manual_seed(rows + columns + inner)
+    a = torch.randn(rows, inner, generator=gen).to(torch.bfloat16).cuda()
+    room = torch.empty(2 * columns * inner + 4, dtype=torch.bfloat16, device="cuda")
+    w, off = room[:-4].view(2 * columns, inner), room[4:].view(2 * columns, inner)
+    values = (0.1 * torch.randn(2 * columns, inner, generator=gen)).to(torch.bfloat16).cuda()
+    want, got = (torch.full((rows, columns), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    w.copy_(values)
+    k.gemm_gated_clamped(a, w, got, 2.0, 1.7)
+    off.copy_(values)
+    k.gemm_gated_clamped(a, off, want, 2.0, 1.7)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
