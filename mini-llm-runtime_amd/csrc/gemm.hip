@@ -496,23 +496,25 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const __
     // What the epilogue needs from memory is asked for here, before the weight, by every wavefront alike
     // (no branch around a load); only wavefront 0 uses it.
     float ss_mine = 0.f;                                   // EPI_SCALE: this lane's share of the row's partial sums
-    float4 ss4[EPI == EPI_SCALE ? 4 : 1];                  // ... which are added when the weight is multiplied, where these hold them all
+    constexpr bool SS_LATER = EPI == EPI_SCALE && UMAX <= 2;
+    float4 ss4;                                            // ... which are added when the weight is multiplied, where this holds them all
     const int ss_quads = epi.ss_parts >> 2, ss_run = (ss_quads + 4 * SKINNY_WAVES - 1) / (4 * SKINNY_WAVES);
-    const bool ss_later = EPI == EPI_SCALE && epi.ss_vec && ss_run <= 4;
+    const bool ss_later = SS_LATER && epi.ss_vec && ss_run <= 1;
     float4 h4 = make_float4(0.f, 0.f, 0.f, 0.f), nw4 = h4;  // EPI_RESIDUAL: h and the next norm's weights at (row r16, columns n0 + 4 b ..)
     float4 h4b = h4, nw4b = h4;                            // ... and, PAIR, at the second strip's columns n0 + 16 + 4 b ..
     if constexpr (EPI == EPI_SCALE) {
         // the row's partial sums are dealt out to the 32 (wavefront, lane block) pairs in runs of q; a run is
         // added in ascending order (four sums that lie side by side as (0 + 1) + (2 + 3) first, when their number
         // allows 16-byte loads), the four runs of a wavefront as (0 + 1) + (2 + 3), the wavefronts in the order
-        // 0..7: an order that depends on nothing but the number of partial sums.  Up to 512 of them a lane's four loads are asked
-        // for here and used behind the products: used here, they cost a trip to the cache before the workgroup has asked for any of
-        // its weight (0.6B sizes, one token: 1046 us a step, so 1034; eight 1623, 1606).  Of more, four are asked for before the first is used.
+        // 0..7: an order that depends on nothing but the number of partial sums.  Up to 128 of them (a short k) a lane's one load is
+        // asked for here and used behind the products: used here, it costs a trip to the cache before the workgroup has asked for any of
+        // its weight (0.6B sizes, one token: 1046 us a step, so 1034; eight 1623, 1606).  Of more, four are asked for before the first is
+        // used: kept as well, their registers are what another workgroup on a compute unit needs (10 x 2 * 25600 x 5120 104.7 us, 115.9
+        // with them; 10 x 2 * 12288 x 1024 with four 13.2 and 15.8).
         const float* row = epi.ss + (size_t)min(r16, M - 1) * epi.ss_parts;
         const int pair = wave * 4 + b;
-        if (ss_later) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) ss4[j] = reinterpret_cast<const float4*>(row)[min(pair * ss_run + j, ss_quads - 1)];
+        if (SS_LATER && ss_later) {
+            ss4 = reinterpret_cast<const float4*>(row)[min(pair, ss_quads - 1)];
         } else if (epi.ss_vec) {
             const int quads = ss_quads, q = ss_run;
             const float4* row4 = reinterpret_cast<const float4*>(row);
@@ -667,11 +669,8 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const __
                 for (int r = 0; r < 4; ++r) part[wave - 1][g][i][lane][r] = acc[g][i][r];
     }
     if constexpr (EPI == EPI_SCALE) {
-        if (ss_later) {
-            const int pair = wave * 4 + b;
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                ss_mine += j < ss_run && pair * ss_run + j < ss_quads ? (ss4[j].x + ss4[j].y) + (ss4[j].z + ss4[j].w) : 0.f;
+        if (SS_LATER && ss_later) {
+            ss_mine += wave * 4 + b < ss_quads ? (ss4.x + ss4.y) + (ss4.z + ss4.w) : 0.f;
         }
         ss_mine = xor_sum<16>(ss_mine);
         ss_mine = xor_sum<32>(ss_mine);
