@@ -578,9 +578,12 @@ struct Routing {
 // all others, where one choice after the other took six exchanges between lanes each, and one group for all needs no rounds.
 // 48 tokens, 4 of 20 experts: 7.8 -> 3.4 us; 8 of 64 in 4 of 8 groups 11.6 -> 4.6, of 256 14.7 -> 10.4; 1777 tokens, 4 of 16: 8.7 -> 3.6.
 // (The choice and the sort below in one launch of one workgroup, three tokens a wavefront: 10.7 us for 3.4 and 2.0.)
-// zr: the token's logits; one wavefront (WAVES 1) needs no other one of its workgroup.
-template <int WAVES>
-__device__ __forceinline__ void choose_experts(const float* zr, const Routing& r, int32_t* __restrict__ ids, float* __restrict__ weights) {
+// zr: the token's logits; one wavefront (WAVES 1) needs no other one of its workgroup, of which up to SLOTS choose beside each other,
+// each in a slot of its own.
+template <int WAVES, int SLOTS = 1>
+__device__ __forceinline__ void choose_experts(const float* zr, const Routing& r, int32_t* __restrict__ ids, float* __restrict__ weights, size_t token,
+                                               int slot = 0) {
+    static_assert(WAVES == 1 || SLOTS == 1, "several wavefronts a token: one token a workgroup");
     auto sync = []() {
         if (WAVES > 1) {
             __syncthreads();
@@ -590,12 +593,17 @@ __device__ __forceinline__ void choose_experts(const float* zr, const Routing& r
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
     };
-    __shared__ __attribute__((aligned(16))) int keys[64 * WAVES];
-    __shared__ float by[64 * WAVES];                                       // what the choice goes by
-    __shared__ float plain[64 * WAVES];                                    // the plain scores
-    __shared__ float group[64 * WAVES];
-    __shared__ int choice[64 * WAVES];
-    const int e = threadIdx.x, experts = r.experts, lane = e % 64;
+    __shared__ __attribute__((aligned(16))) int keys_lds[SLOTS][64 * WAVES];
+    __shared__ float by_lds[SLOTS][64 * WAVES];
+    __shared__ float plain_lds[SLOTS][64 * WAVES];
+    __shared__ float group_lds[SLOTS][64 * WAVES];
+    __shared__ int choice_lds[SLOTS][64 * WAVES];
+    int* keys = keys_lds[slot];
+    float* by = by_lds[slot];                                              // what the choice goes by
+    float* plain = plain_lds[slot];                                        // the plain scores
+    float* group = group_lds[slot];
+    int* choice = choice_lds[slot];
+    const int lane = threadIdx.x % 64, e = WAVES == 1 ? lane : (int)threadIdx.x, experts = r.experts;
     const bool expert = e < experts;
     const float logit = expert ? zr[e] : 0.f;
     float z_max = 0.f, z_sum = 1.f, cand = -INFINITY;
@@ -677,72 +685,85 @@ __device__ __forceinline__ void choose_experts(const float* zr, const Routing& r
         for (int c = 0; c < r.top; ++c) sum += plain[choice[c]];           // (in the order of the choices)
         w = w / (sum + 1e-20f);
     }
-    ids[(size_t)blockIdx.x * r.top + e] = which;
-    weights[(size_t)blockIdx.x * r.top + e] = r.renorm || r.out_scale != 1.0f ? w * r.out_scale : w;
+    ids[token * r.top + e] = which;
+    weights[token * r.top + e] = r.renorm || r.out_scale != 1.0f ? w * r.out_scale : w;
 }
 
 template <int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void router_topk_kernel(const float* __restrict__ z, long ld, Routing r,
                                                                  int32_t* __restrict__ ids, float* __restrict__ weights) {
-    choose_experts<WAVES>(z + (size_t)blockIdx.x * ld, r, ids, weights);
+    choose_experts<WAVES>(z + (size_t)blockIdx.x * ld, r, ids, weights, blockIdx.x);
 }
 
 #if MLR_BF16
-// The router's product with the choice behind it: a token a workgroup, z[e] = x . w[e] for all `outputs` rows of w (the experts, and
-// beyond them a shared expert's gate) in 32-bit, written to z and chosen from.  Eight wavefronts take every eighth row, a lane eight
-// neighbouring channels of every 512, in the order of the channels, and the lanes' sums by halves (`wave_sum`): a token's logits do
-// not depend on the others.
-// Bound by its chain of trips -- row and weights, the lanes' sums, the choice -- where the product alone was a launch of two or three
-// workgroups.  48 tokens, 20 outputs of 2048 channels 7.6 -> 4.3 us, 732 tokens, 8 outputs 8.9 -> 5.1, 1777 tokens 9.0 -> 7.0 (in a
-// model, where the product finds its operands elsewhere, 12.4, 15.9 and 15.6 before).
+// The router's product with the choice behind it: TOKENS tokens a workgroup, z[e] = x . w[e] for all `outputs` rows of w (the experts,
+// and beyond them a shared expert's gate) in 32-bit, written to z and chosen from.  Eight wavefronts take every eighth row, a lane eight
+// neighbouring channels of every 512, in the order of the channels, and the lanes' sums by halves (`wave_sum`): a token's logits depend
+// neither on the others nor on how many they are.
+// Few tokens, one a workgroup: bound by its chain of trips -- row and weights, the lanes' sums, the choice -- where the product alone was
+// a launch of two or three workgroups.  48 tokens, 20 outputs of 2048 channels 7.4 -> 5.0 us, 732 tokens, 8 outputs 8.9 -> 5.1.
+// Many, four a workgroup from ROUTER_MANY on: bound by what the workgroups read out of the L2, the whole weight each.  One and four
+// tokens a workgroup, us: 768 x 20 outputs of 2048 channels 7.5, 7.4; 1024 x 8 5.6, 5.2; 2048 x 8 7.7, 6.7; 2048 x 20 12.6, 10.0;
+// 8192 x 20 39.6, 24.0.  (The product by matrix instructions, 16 tokens a workgroup, is slower up to 2048 tokens: 48 x 20 7.9.)
 #define ROUTER_OUTPUTS 128
 #define ROUTER_WAVES 8
-template <int AT_ONCE>          // rows of w a wavefront takes side by side
+#define ROUTER_MANY 768
+template <int TOKENS, int AT_ONCE, int AHEAD>          // AT_ONCE: rows of w a wavefront takes side by side; AHEAD: times 512 channels
 __global__ __launch_bounds__(64 * ROUTER_WAVES) void router_kernel(const __bf16* __restrict__ x, const __bf16* __restrict__ w,
-                                                                   float* __restrict__ z, long ld, int width, int outputs, Routing r,
+                                                                   float* __restrict__ z, long ld, int rows, int width, int outputs, Routing r,
                                                                    int32_t* __restrict__ ids, float* __restrict__ weights) {
     typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
     struct eight { bf16x2 pair[4]; };
-    __shared__ float z_lds[ROUTER_OUTPUTS];
+    static_assert(TOKENS <= ROUTER_WAVES, "a wavefront chooses for one token");
+    __shared__ float z_lds[TOKENS][ROUTER_OUTPUTS];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const __bf16* row = x + (size_t)blockIdx.x * width;
-    constexpr int AHEAD = 4;
+    const int first = blockIdx.x * TOKENS;
     for (int e0 = wave; e0 < outputs; e0 += ROUTER_WAVES * AT_ONCE) {
-        float sum[AT_ONCE] = {};
+        float sum[TOKENS][AT_ONCE] = {};
         for (int c0 = 0; c0 < width; c0 += 512 * AHEAD) {
-            vec16 v[AHEAD], u[AT_ONCE][AHEAD];
+            vec16 v[TOKENS][AHEAD], u[AT_ONCE][AHEAD];
 #pragma unroll
             for (int q = 0; q < AHEAD; ++q) {                              // (clamped: no branch around a load)
                 const int at = min(c0 + 512 * q + 8 * lane, width - 8);
-                v[q] = *reinterpret_cast<const vec16*>(row + at);
+#pragma unroll
+                for (int i = 0; i < TOKENS; ++i) v[i][q] = *reinterpret_cast<const vec16*>(x + (size_t)min(first + i, rows - 1) * width + at);
 #pragma unroll
                 for (int j = 0; j < AT_ONCE; ++j)
                     u[j][q] = *reinterpret_cast<const vec16*>(w + (size_t)min(e0 + ROUTER_WAVES * j, outputs - 1) * width + at);
             }
 #pragma unroll
             for (int q = 0; q < AHEAD; ++q) {
-                if (c0 + 512 * q + 8 * lane >= width) v[q] = vec16{{0, 0, 0, 0}};
-                const eight a = __builtin_bit_cast(eight, v[q]);
+                const bool beyond = c0 + 512 * q + 8 * lane >= width;
+#pragma unroll
+                for (int i = 0; i < TOKENS; ++i)
+                    if (beyond) v[i][q] = vec16{{0, 0, 0, 0}};
 #pragma unroll
                 for (int j = 0; j < AT_ONCE; ++j) {
                     // (an expert that is not finite does not reach a token through channels that are not there)
-                    if (c0 + 512 * q + 8 * lane >= width) u[j][q] = vec16{{0, 0, 0, 0}};
+                    if (beyond) u[j][q] = vec16{{0, 0, 0, 0}};
                     const eight b = __builtin_bit_cast(eight, u[j][q]);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) sum[j] = __builtin_amdgcn_fdot2_f32_bf16(a.pair[e], b.pair[e], sum[j], false);
+                    for (int i = 0; i < TOKENS; ++i) {
+                        const eight a = __builtin_bit_cast(eight, v[i][q]);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) sum[i][j] = __builtin_amdgcn_fdot2_f32_bf16(a.pair[e], b.pair[e], sum[i][j], false);
+                    }
                 }
             }
         }
 #pragma unroll
-        for (int j = 0; j < AT_ONCE; ++j) {
-            const float total = wave_sum(sum[j]);
-            if (lane == 0 && e0 + ROUTER_WAVES * j < outputs) z_lds[e0 + ROUTER_WAVES * j] = total;
-        }
+        for (int i = 0; i < TOKENS; ++i)
+#pragma unroll
+            for (int j = 0; j < AT_ONCE; ++j) {
+                const float total = wave_sum(sum[i][j]);
+                if (lane == 0 && e0 + ROUTER_WAVES * j < outputs) z_lds[i][e0 + ROUTER_WAVES * j] = total;
+            }
     }
     __syncthreads();
-    if (wave != 0) return;
-    for (int e = lane; e < outputs; e += 64) z[(size_t)blockIdx.x * ld + e] = z_lds[e];
-    choose_experts<1>(z_lds, r, ids, weights);
+    const int token = first + wave;
+    if (wave >= TOKENS || token >= rows) return;
+    for (int e = lane; e < outputs; e += 64) z[(size_t)token * ld + e] = z_lds[wave][e];
+    choose_experts<1, TOKENS>(z_lds[wave], r, ids, weights, token, wave);
 }
 #endif
 
@@ -1043,8 +1064,10 @@ int mlr_router(const void* x, const void* w, float* z, long ld, int32_t* ids, fl
         ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) != 0)
         return 1;
     const Routing r{experts, top, group_count, group_keep, renorm, softmax, group_best, correction, out_scale};
-    auto* kernel = outputs <= ROUTER_WAVES ? router_kernel<1> : outputs <= 2 * ROUTER_WAVES ? router_kernel<2> : router_kernel<3>;
-    kernel<<<rows, 64 * ROUTER_WAVES, 0, stream>>>((const __bf16*)x, (const __bf16*)w, z, ld, width, outputs, r, ids, weights);
+    const int step = rows >= ROUTER_MANY ? 4 : 1;
+    auto* kernel = step > 1 ? (outputs <= ROUTER_WAVES ? router_kernel<4, 1, 2> : outputs <= 2 * ROUTER_WAVES ? router_kernel<4, 2, 2> : router_kernel<4, 3, 2>)
+                            : (outputs <= ROUTER_WAVES ? router_kernel<1, 1, 4> : outputs <= 2 * ROUTER_WAVES ? router_kernel<1, 2, 4> : router_kernel<1, 3, 4>);
+    kernel<<<(rows + step - 1) / step, 64 * ROUTER_WAVES, 0, stream>>>((const __bf16*)x, (const __bf16*)w, z, ld, rows, width, outputs, r, ids, weights);
     return (int)hipGetLastError();
 #else
     return 1;

@@ -2342,20 +2342,22 @@ class Kernels:
             _c_int(group_count), _c_int(group_keep), _p(correction), _c_int(1 if renormalize else 0), _c_float(scale),
             _c_int(self.ROUTER_SCORES[score]), _c_int(self.ROUTER_GROUPS[group_score]), _stream()), "router_topk")
 
-    # rows x outputs x channels, and outputs x channels (every token reads the weight again): one launch and two, us, 1777 tokens of 8 x
-    # 2048 7.0, 9.0, of 8 x 4096 10.4, 9.9; 2048 of 16 x 2048 9.0, 7.9; 48 of 64 x 2048 7.2, 8.2, of 64 x 4096 10.2, 9.8
-    ROUTER_FUSED_WORK, ROUTER_FUSED_WEIGHT = 1 << 25, 1 << 17
+    # Outputs x channels up to which the router is one launch, whatever the number of tokens: the order of a token's sums, on whose last
+    # bits a choice may turn, is then the same in every step.  One launch and two, us: 48 tokens of 8 x 2048 3.9, 7.0, of 20 x 2048 5.0, 7.4;
+    # 1024 of 8 x 4096 6.6, 9.1; 2048 of 8 x 2048 6.7, 7.9, of 20 x 2048 10.0, 8.3; 8192 of 8 x 2048 14.2, 10.7, of 20 x 2048 24.0, 12.6.
+    # Not beyond: 2048 of 32 x 2048 14.6, 9.0 (48 of them 6.0, 7.3), of 64 x 2048 29, 9.9.
+    ROUTER_FUSED_WEIGHT = 3 << 14
 
     def router(self, x, w, logits, ids, weights, group_count=1, group_keep=1, correction=None, renormalize=False, scale=1.0,
                score="sigmoid", group_score="best_two", experts=None):
         """logits = x . w^T in 32-bit sums and the choice of `router_topk` from its first `experts` columns: one launch while the
-        product is small (`ROUTER_FUSED_WORK`, `ROUTER_FUSED_WEIGHT`), two otherwise."""
+        weight is small (`ROUTER_FUSED_WEIGHT`), two otherwise."""
         rows, width = x.shape
         outputs = logits.shape[1]
         experts = outputs if experts is None else experts
         top = ids.shape[1]
-        if self.dtype == torch.bfloat16 and rows * outputs * width <= self.ROUTER_FUSED_WORK and outputs * width <= self.ROUTER_FUSED_WEIGHT and experts <= 64 and outputs <= 128 and \
-                width % 8 == 0 and _on16(x, w):
+        if self.dtype == torch.bfloat16 and outputs * width <= self.ROUTER_FUSED_WEIGHT and experts <= 64 and outputs <= 128 and width % 8 == 0 \
+                and _on16(x, w):
             _tensor(x, "x", self.dtype, ndim=2)
             _tensor(w, "w", self.dtype, (outputs, width))
             _tensor(logits, "logits", torch.float32, (rows, outputs))
