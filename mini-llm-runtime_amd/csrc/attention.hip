@@ -1564,23 +1564,26 @@ static int launch_decode_fused(dim3 grid, const AttnArgs& a, const int32_t* grou
 // qkv holds the raw projections
 // [rows, ld].  Key and value of every token are written into the cache.  `partial` holds at least
 // rows * q_heads * max(max_splits, 1) * (head_dim + 2) floats, also without splits; `arrivals` rows * kv_heads zeros, which are
-// zeros again when the launch is done.
-// Needs what `mlr_attention_mfma` needs and head_dim % 64 == 0.
+// zeros again when the launch is done.  `workgroups` > 0: even ranges (`even_ranges`, at most max_splits), no token at or beyond position
+// `max_context`.  Needs what `mlr_attention_mfma` needs and head_dim % 64 == 0.
 extern "C" int mlr_attention_decode_fused(
     const void* qkv, int ld, const void* k_pages, const void* v_pages, const int32_t* block_table, int max_blocks,
     const int32_t* slots, const int32_t* positions, void* out, float* partial, const int32_t* group_row0,
     const int32_t* group_ntok, int groups, int q_heads, int kv_heads, int head_dim, int page_size, int window,
-    float scale, int split_keys, int max_splits, int workgroups, const float* q_norm_w, const float* k_norm_w, float eps,
+    float scale, int split_keys, int max_splits, int workgroups, int max_context, const float* q_norm_w, const float* k_norm_w, float eps,
     const float* rope, int32_t* arrivals, hipStream_t stream) {
     if (groups <= 0) return 0;
+    if (max_splits < 1) max_splits = 1;
     if (head_dim % 64 != 0 || head_dim > 256 || page_size % 16 != 0 || q_heads % kv_heads != 0 ||
         q_heads / kv_heads > 16 || partial == nullptr || arrivals == nullptr || (q_norm_w == nullptr) != (k_norm_w == nullptr)) return -1;
-    if (max_splits < 1) max_splits = 1;
     if ((max_splits > 1 || workgroups > 0) && (split_keys <= 0 || split_keys % MFMA_TILE_KEYS != 0 || max_splits > COMBINE_MAX_SPLITS)) return -2;
     if (workgroups == 0 && (max_splits > 1 ? split_keys / page_size + 2 : max_blocks) > DECODE_PAGE_CACHE) return -3;
-    // (an even range is less than twice a share's keys; `quotient`)
-    if (workgroups > 0 && (long long)max_blocks * page_size >= 1ll << 25) return -2;
-    if (workgroups > 0 && (2ll * split_keys * groups * kv_heads / workgroups + 128) / page_size + 2 > DECODE_PAGE_CACHE) return -3;
+    if (workgroups > 0) {
+        if (max_context <= 0 || max_context >= 1 << 25) return -2;                  // (`quotient`)
+        // an even range is less than twice a share's keys, and where max_splits is what limits their number, its part of the longest walk
+        const long long share = 2ll * split_keys * groups * kv_heads / workgroups + 128, part = ((max_context + 63) / 64 + max_splits - 1) / max_splits * 64ll;
+        if ((share > part ? share : part) / page_size + 2 > DECODE_PAGE_CACHE) return -3;
+    }
     AttnArgs a{nullptr, (const elem_t*)k_pages, (const elem_t*)v_pages, block_table, slots,
                positions, (elem_t*)out, partial, max_blocks, q_heads, kv_heads, head_dim, page_size,
                window, split_keys, max_splits, scale, q_heads / kv_heads};

@@ -925,13 +925,13 @@ class Kernels:
     @timed("attention")
     def attention_decode_fused(self, qkv, k_pages, v_pages, block_table, slots, positions, out, group_row0, group_ntok,
                                groups, q_heads, kv_heads, head_dim, page_size, scale, q_norm_w, k_norm_w, eps, rope,
-                               partial, window=None, split_keys=0, max_splits=1, arrivals=None, workgroups=0):
+                               partial, window=None, split_keys=0, max_splits=1, arrivals=None, workgroups=0, max_context=None):
         """For a batch in which every group is ONE new token of a request (the caller vouches for that):
         per-head RMSNorm of q and k (weights may both be None), rotation by `rope` (may be None), attention
         over the cached keys and the token's own, and the write of the token's key and value into their
-        pages, in one launch.  `qkv` holds the raw projections; `partial` is needed also without splits.  `arrivals`: int32 zeros,
-        a row and kv head each, which count workgroups during the launch and are zeros again behind it (None: made here).
-        `workgroups`: 0, or the key ranges are even ones as `StepContext.even_split` gives them."""
+        pages, in one launch.  `qkv` holds the raw projections; `partial` is needed also without splits.  `arrivals`: int32 zeros, a row and kv head each, which count workgroups during the launch and are zeros again behind it (None:
+        made here).  `workgroups`: 0, or the key ranges are even ones as `StepContext.even_split` gives them, at most `max_splits` of
+        them; then `max_context` is a bound on the positions + 1 (default: what the block table can hold)."""
         _need(self.decode_fusion_supported(q_heads, kv_heads, head_dim, page_size),
               "attention_decode_fused: sizes not supported")
         width = (q_heads + 2 * kv_heads) * head_dim
@@ -960,9 +960,11 @@ class Kernels:
                   lambda: f"split_keys must be a multiple of {ATTENTION_TILE_KEYS}")
         _tensor(partial, "partial", torch.float32, ndim=1)
         _need(partial.numel() >= self.attention_partial_numel(m, q_heads, head_dim, max_splits), "partial buffer too small")
+        max_context = block_table.shape[1] * page_size if max_context is None else max_context
         if workgroups:
             _need(workgroups > 0 and split_keys > 0 and split_keys % ATTENTION_TILE_KEYS == 0, "even key ranges: split_keys is a share's keys")
-            longest = 2 * split_keys * m * kv_heads // workgroups + 128
+            _need(0 < max_context < 1 << 25, "even key ranges: contexts below 2^25 tokens")
+            longest = max(2 * split_keys * m * kv_heads // workgroups + 128, -(-max_context // (64 * max_splits)) * 64)
         _need((longest // page_size + 2 if workgroups else split_keys // page_size + 2 if max_splits > 1 else block_table.shape[1]) <= MFMA_MAX_PAGES,
               "attention_decode_fused: a workgroup's key range spans more than 4096 pages; split the keys")
         if arrivals is None:
@@ -973,7 +975,7 @@ class Kernels:
         _ok(fn(_p(qkv), _c_int(width), _p(k_pages), _p(v_pages), _p(block_table), _c_int(block_table.shape[1]),
                _p(slots), _p(positions), _p(out), _p(partial), _p(group_row0), _p(group_ntok), _c_int(groups),
                _c_int(q_heads), _c_int(kv_heads), _c_int(head_dim), _c_int(page_size), _c_int(window or 0),
-               _c_float(scale), _c_int(split_keys), _c_int(max_splits), _c_int(workgroups), _p(q_norm_w), _p(k_norm_w), _c_float(eps),
+               _c_float(scale), _c_int(split_keys), _c_int(max_splits), _c_int(workgroups), _c_int(max_context), _p(q_norm_w), _p(k_norm_w), _c_float(eps),
                _p(rope), _p(arrivals), _stream()), "attention_decode_fused")
 
     def prefill_attention_supported(self, q_heads, kv_heads, head_dim, page_size, max_context=0):

@@ -240,7 +240,7 @@ class GqaAttention:
                 self.k_norm.weight if self.k_norm is not None else None,
                 self.q_norm.eps if self.q_norm is not None else 0.0, rope, partial,
                 window=s.window, split_keys=split_keys, max_splits=max_splits,
-                workgroups=workgroups, arrivals=ctx.workspace.get("arrivals", (m * s.kv_heads,), torch.int32))
+                workgroups=workgroups, max_context=ctx.max_context, arrivals=ctx.workspace.get("arrivals", (m * s.kv_heads,), torch.int32))
             return attn
         q = ctx.workspace.get("q", (m, s.q_heads * s.head_dim), x.dtype)
         k.qk_norm_rope_kv(

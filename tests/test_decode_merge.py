@@ -31,6 +31,24 @@ def test_counters_are_zeros_when_they_are_made_and_when_they_grow():
     assert ws.get("arrivals", (9000,), torch.int32).eq(0).all()
 
 
+def fused_entry(groups, kv_heads, head_dim, page, split_keys, max_splits, workgroups, max_context):
+    """The kernel's entry with sizes only: for calls that it refuses, which look at no address."""
+    lib, some = build.load("attention", torch.bfloat16), ctypes.c_void_p(256)
+    ints = lambda *values: [ctypes.c_int(v) for v in values]
+    return lib.mlr_attention_decode_fused(some, *ints(3 * kv_heads * head_dim), some, some, some, *ints(1 << 20), some, some, some, some, some, some,
+                                          *ints(groups, kv_heads, kv_heads, head_dim, page, 0), ctypes.c_float(1.0),
+                                          *ints(split_keys, max_splits, workgroups, max_context), None, None, ctypes.c_float(0.0), None, some, None)
+
+
+@pytest.mark.parametrize("max_splits,page,max_context", [(1, 32, 4094 * 32 + 1), (1, 64, 300000), (2, 48, 2 * 4096 * 48 - 64), (7, 16, 1 << 19)])
+def test_fewer_even_ranges_than_the_contexts_need_are_refused(max_splits, page, max_context):
+    # a range of that many keys spans more pages than a workgroup keeps the ids of, whatever the rule's own width is
+    wide = 2048 * 256 // 8
+    assert StepContext.even_ranges(max_context, 256, 8, wide) > max_splits
+    assert fused_entry(1, 8, 128, page, wide, max_splits, 256, max_context) == -3
+    assert fused_entry(1, 8, 128, page, wide, max_splits, 256, 1 << 25) == -2
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("q_heads,kv_heads,d,page,lengths,window", [
     (16, 8, 128, 16, [1, 2, 33, 64, 65, 66, 1000], None),
