@@ -1562,8 +1562,8 @@ static int launch_decode_fused(dim3 grid, const AttnArgs& a, const int32_t* grou
 
 // Decoding with `DecodeFusion`: group i is the one token in batch row i (group_row0[i] = i, group_ntok[i] = 1);
 // qkv holds the raw projections
-// [rows, ld].  Key and value of every token are written into the cache.  `partial` holds at least
-// rows * q_heads * max(max_splits, 1) * (head_dim + 2) floats, also without splits; `arrivals` rows * kv_heads zeros, which are
+// [rows, ld].  Key and value of every token are written into the cache.  With max_splits > 1 `partial` holds at least
+// rows * q_heads * max_splits * (head_dim + 2) floats; `arrivals` rows * kv_heads zeros, which are
 // zeros again when the launch is done.  `workgroups` > 0: even ranges (`even_ranges`, at most max_splits), no token at or beyond position
 // `max_context`.  Needs what `mlr_attention_mfma` needs and head_dim % 64 == 0.
 extern "C" int mlr_attention_decode_fused(
@@ -1575,7 +1575,7 @@ extern "C" int mlr_attention_decode_fused(
     if (groups <= 0) return 0;
     if (max_splits < 1) max_splits = 1;
     if (head_dim % 64 != 0 || head_dim > 256 || page_size % 16 != 0 || q_heads % kv_heads != 0 ||
-        q_heads / kv_heads > 16 || partial == nullptr || arrivals == nullptr || (q_norm_w == nullptr) != (k_norm_w == nullptr)) return -1;
+        q_heads / kv_heads > 16 || (partial == nullptr && max_splits > 1) || arrivals == nullptr || (q_norm_w == nullptr) != (k_norm_w == nullptr)) return -1;
     if ((max_splits > 1 || workgroups > 0) && (split_keys <= 0 || split_keys % MFMA_TILE_KEYS != 0 || max_splits > COMBINE_MAX_SPLITS)) return -2;
     if (workgroups == 0 && (max_splits > 1 ? split_keys / page_size + 2 : max_blocks) > DECODE_PAGE_CACHE) return -3;
     if (workgroups > 0) {

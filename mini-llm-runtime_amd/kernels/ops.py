@@ -929,7 +929,8 @@ class Kernels:
         """For a batch in which every group is ONE new token of a request (the caller vouches for that):
         per-head RMSNorm of q and k (weights may both be None), rotation by `rope` (may be None), attention
         over the cached keys and the token's own, and the write of the token's key and value into their
-        pages, in one launch.  `qkv` holds the raw projections; `partial` is needed also without splits.  `arrivals`: int32 zeros, a row and kv head each, which count workgroups during the launch and are zeros again behind it (None:
+        pages, in one launch.  `qkv` holds the raw projections; `partial`: room for the key ranges' results, None without splits.
+        `arrivals`: int32 zeros, a row and kv head each, which count workgroups during the launch and are zeros again behind it (None:
         made here).  `workgroups`: 0, or the key ranges are even ones as `StepContext.even_split` gives them, at most `max_splits` of
         them; then `max_context` is a bound on the positions + 1 (default: what the block table can hold)."""
         _need(self.decode_fusion_supported(q_heads, kv_heads, head_dim, page_size),
@@ -958,8 +959,8 @@ class Kernels:
         if max_splits > 1:
             _need(split_keys > 0 and split_keys % ATTENTION_TILE_KEYS == 0,
                   lambda: f"split_keys must be a multiple of {ATTENTION_TILE_KEYS}")
-        _tensor(partial, "partial", torch.float32, ndim=1)
-        _need(partial.numel() >= self.attention_partial_numel(m, q_heads, head_dim, max_splits), "partial buffer too small")
+            _tensor(partial, "partial", torch.float32, ndim=1)
+            _need(partial.numel() >= self.attention_partial_numel(m, q_heads, head_dim, max_splits), "partial buffer too small")
         max_context = block_table.shape[1] * page_size if max_context is None else max_context
         if workgroups:
             _need(workgroups > 0 and split_keys > 0 and split_keys % ATTENTION_TILE_KEYS == 0, "even key ranges: split_keys is a share's keys")

@@ -229,9 +229,6 @@ class GqaAttention:
                 workgroups = 0
                 split_keys, max_splits, partial = ctx.attention_split(m, m, s.kv_heads, s.q_heads, s.head_dim,
                                                                       longest=k.mfma_longest_context(view.page_size))
-            if partial is None:
-                partial = ctx.workspace.get("attn_partial", (k.attention_partial_numel(m, s.q_heads, s.head_dim, 1),),
-                                            torch.float32)
             self._hint(k)
             k.attention_decode_fused(
                 qkv, view.k_pages, view.v_pages, view.block_table, ctx.slots, ctx.positions, attn, groups[0], groups[1],

@@ -8,6 +8,7 @@ import torch
 
 from mini_llm_runtime_amd.engine.context import StepContext, Workspace
 from mini_llm_runtime_amd.kernels import build
+from mini_llm_runtime_amd.kernels.ops import KernelError
 
 
 def test_the_hosts_rule_of_even_ranges_is_the_kernels_and_never_falls():
@@ -105,3 +106,26 @@ def test_even_ranges_give_the_plain_attention_on_every_launch(q_heads, kv_heads,
         torch.testing.assert_close(first[s].double().cpu().view(q_heads, d), want, **tol(dtype))
         pg = table[s, (L - 1) // page]
         assert torch.equal(kp[pg, :, (L - 1) % page].cpu(), own_k[s, 0]) and torch.equal(vp[pg, :, :, (L - 1) % page].cpu(), own_v[s, 0])
+
+
+@pytest.mark.gpu
+def test_one_range_a_token_needs_no_room_for_results():
+    # (one workgroup has all of a token's keys: its sums stay in LDS)
+    from test_kernels_gpu import kernels
+    k = kernels(torch.bfloat16)
+    gen = torch.Generator().manual_seed(3)
+    draw = lambda *shape: torch.randn(shape, generator=gen).bfloat16().cuda()
+    table = torch.arange(24, dtype=torch.int32, device="cuda").view(3, 8)
+    pages, qkv = (draw(24, 2, 16, 64), draw(24, 2, 64, 16)), draw(3, 8 * 64)
+    rows, pos = torch.arange(3, dtype=torch.int32, device="cuda"), torch.tensor([0, 40, 127], dtype=torch.int32, device="cuda")
+    outs = []
+    for workgroups, room in ((0, torch.full((k.attention_partial_numel(3, 4, 64, 1),), float("nan"), device="cuda")), (0, None), (6, None)):
+        out = torch.full((3, 256), float("nan"), dtype=torch.bfloat16, device="cuda")
+        k.attention_decode_fused(qkv, pages[0].clone(), pages[1].clone(), table, rows, pos, out, rows, torch.ones_like(rows), 3, 4, 2, 64, 16, 0.125,
+                                 None, None, 0.0, None, room, split_keys=128 if workgroups else 0, workgroups=workgroups)
+        outs.append(out)
+        assert room is None or torch.isnan(room).all()
+    assert torch.isfinite(outs[0]).all() and all(torch.equal(o, outs[0]) for o in outs[1:])
+    with pytest.raises(KernelError):
+        k.attention_decode_fused(qkv, *pages, table, rows, pos, out, rows, torch.ones_like(rows), 3, 4, 2, 64, 16, 0.125, None, None, 0.0, None, None,
+                                 split_keys=64, max_splits=2)
