@@ -58,6 +58,13 @@ def test_fewer_even_ranges_than_the_contexts_need_are_refused(max_splits, page, 
     (5, 1, 128, 64, [2049, 1], 130),
     (16, 1, 256, 16, [300, 65], None),
     (3, 3, 192, 16, [90, 1100], 64),
+    # beyond a share's width: two and three shares of workgroups a token; a window of them
+    (16, 8, 128, 16, [9000, 4097, 4096, 7, 130, 1, 64, 500, 33, 2, 3000, 4161, 90, 17, 250, 8193], None),
+    (8, 8, 64, 32, [9000, 4200, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14], 8200),
+    # more than 64 ranges, and more than 128, which the merge reads in several rounds
+    (16, 1, 64, 32, [20011], None),
+    (5, 1, 128, 16, [40000], None),
+    (5, 1, 64, 64, [36000, 300], None),
 ])
 def test_even_ranges_give_the_plain_attention_on_every_launch(q_heads, kv_heads, d, page, lengths, window):
     from test_kernels_gpu import kernels, plain_attention, tol
