@@ -339,7 +339,9 @@ class Runner:
         expect = probe.clone()
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph):
+            self.kernels.claim_split()                    # (a capture has a stream of its own; nothing runs meanwhile)
             logits = self.model.forward(ctx, want_rows)
+        self.kernels.claim_split()
         state["keep"] = self.workspace.buffers()
         ok = self._replays_match(graph, logits if logits is not None else probe, expect,
                                  lambda: self.cache.restore_state(before))
@@ -534,6 +536,7 @@ class Runner:
         entries and of their `want`), or None when nothing is wanted."""
         batch = self._gather(entries)
         total, slots = batch.total, batch.slots
+        self.kernels.claim_split()                        # (steps follow each other on whatever stream the caller has made current)
         self.cache.commit_into(slots, batch.counts, batch.first, batch.at)      # raises with nothing changed, else takes the pages
         try:
             longest = int((batch.first + batch.counts).max())

@@ -190,6 +190,7 @@ class Kernels:
         self.routed = routed
         self._library_workspace = None      # scratch memory of the vendor library's products, allocated once
         self._split = None                  # in it: room for the parts of a product and the counters of who has left them
+        self._split_stream = None           # the stream whose products may use that room (`claim_split`)
         self._wide_choices = {}             # (rows, columns, inner size, activation) -> `wide_product`
         self._libs = {}
         self.profiler = None                # a `Profiler`: every launch is then bracketed by events
@@ -390,7 +391,7 @@ class Kernels:
         _need(k == k2, lambda: f"gemm: inner sizes differ ({k} and {k2})")
         _need(out.dtype in (self.dtype, torch.float32), lambda: f"gemm: output type {out.dtype} not supported")
         _tensor(out, "out", out.dtype, (m, n))
-        if m <= 64 and out.dtype == torch.bfloat16 and self._split is not None and self.split_product(m, n, k) and _on16(a, w):
+        if m <= 64 and out.dtype == torch.bfloat16 and self.shares_tiles(m, n, k) and _on16(a, w):
             partial, arrivals = self._split
             _ok(self._lib("gemm").mlr_gemm_split(_p(a), _p(w), _p(out), _c_int(m), _c_int(n), _c_int(k), _p(partial),
                                                  ctypes.c_long(partial.numel()), _p(arrivals), _c_int(arrivals.numel()), _c_int(-1), _stream()), "gemm")
@@ -421,14 +422,26 @@ class Kernels:
         return self._library_workspace
 
     def reserve_split_workspace(self, device):
-        """From here on products of few rows may share a tile out to several workgroups (`split_product`): their parts meet in the
-        scratch memory of the library's products, so one launch of either at a time, as a runner's steps make them; the end of it,
-        which the library is not given, counts the workgroups that have left theirs."""
+        """From here on products of few rows on the current stream (`claim_split`) may share a tile out to several workgroups
+        (`split_product`): their parts meet in the scratch memory of the library's products, the end of which, which the library is
+        not given, counts the workgroups that have left theirs."""
         ws = self.reserve_library_workspace(device)
         if self._split is None:
             arrivals = ws[ws.numel() - SPLIT_COUNTERS * 4:].view(torch.int32)
             arrivals.zero_()
             self._split = (ws[:SPLIT_PARTIAL_BYTES].view(torch.float32), arrivals)
+        self.claim_split()
+
+    def claim_split(self):
+        """The room for shared tiles is the current stream's from here on, whose launches come one after the other: two at a time
+        would count each other's workgroups.  A product on another stream takes the kernels that need no room.  (The caller vouches
+        that the stream that had it before has nothing under way in it; a runner claims it for every step.)"""
+        if self._split is not None:
+            self._split_stream = _stream().value or 0
+
+    def shares_tiles(self, rows, columns, k):
+        """Whether a product of these sizes, launched now, is one whose tiles several workgroups share."""
+        return self._split is not None and self.split_product(rows, columns, k) and self._split_stream == (_stream().value or 0)
 
     def split_product(self, rows, columns, k):
         """Whether a product of up to 64 rows is taken by several workgroups a tile: the sums of the other kernels of few rows, bit by

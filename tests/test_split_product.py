@@ -11,7 +11,7 @@ from mini_llm_runtime_amd.kernels import ops
 def without_gpu(routed=False):
     k = object.__new__(Kernels)
     k.dtype, k.library_gemm, k.routed, k.profiler = torch.bfloat16, True, routed, None
-    k._libs, k._wide_choices, k._split = {}, {}, None
+    k._libs, k._wide_choices, k._split, k._split_stream = {}, {}, None, None
     return k
 
 
@@ -24,6 +24,22 @@ def without_gpu(routed=False):
 def test_long_inner_sizes_of_few_rows_are_shared_out(rows, columns, inner, taken):
     assert without_gpu().split_product(rows, columns, inner) == taken
     assert without_gpu(routed=True).split_product(rows, columns, inner) == (taken and rows <= 16)
+
+
+def test_only_the_stream_that_has_the_room_shares_tiles(monkeypatch):
+    k, now = without_gpu(), [0]
+    monkeypatch.setattr(ops, "_stream", lambda: ctypes.c_void_p(now[0]))
+    assert not k.shares_tiles(8, 2048, 5632)               # (no room at all)
+    k.claim_split()
+    k._split = ("room", "counters")
+    assert not k.shares_tiles(8, 2048, 5632)               # (nobody has it yet)
+    for owner in (0, 4096, 0):
+        now[0] = owner
+        k.claim_split()
+        for stream in (0, 4096, 8192):
+            now[0] = stream
+            assert k.shares_tiles(8, 2048, 5632) == (stream == owner)
+            assert not k.shares_tiles(8, 2048, 2048)
 
 
 # (inner sizes whose last share is one block, a part's last block missing, as many as parts; columns in whole tiles, ragged, odd)
@@ -84,3 +100,28 @@ def test_the_runners_kernels_share_products_out_and_others_do_not():
            torch.empty(64, 4096, device="cuda"))
     k.gemm(a, w, again)
     assert torch.equal(out.view(torch.int16), again.view(torch.int16))
+
+
+@pytest.mark.gpu
+def test_products_of_two_streams_at_once_do_not_meet():
+    # a long product on the stream that has the room, short ones beside it on another: their sums stay their own
+    k = Kernels(torch.bfloat16)
+    k.reserve_split_workspace("cuda")
+    gen = torch.Generator().manual_seed(5)
+    draw = lambda *shape: torch.randn(*shape, generator=gen).to(torch.bfloat16).cuda()
+    a, w = [draw(16, 5632) for _ in range(2)], [draw(2048, 5632) for _ in range(2)]
+    want = [torch.empty(16, 2048, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    for i in range(2):
+        k.gemm(a[i], w[i], want[i])
+    outs = [[torch.full_like(want[i], float("nan")) for _ in range(20)] for i in range(2)]
+    other = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for n in range(20):
+        k.gemm(a[0], w[0], outs[0][n])
+        with torch.cuda.stream(other):
+            assert not k.shares_tiles(16, 2048, 5632)
+            k.gemm(a[1], w[1], outs[1][n])
+    torch.cuda.synchronize()
+    for i in range(2):                                     # (up to 16 rows the other kernels' sums, bit by bit)
+        assert all(torch.equal(out.view(torch.int16), want[i].view(torch.int16)) for out in outs[i])
+    assert not k._split[1].any()
