@@ -1799,13 +1799,19 @@ static bool few_wins(int M, int N, int K, bool gated) {
 }
 
 // Whether up to 16 rows are these tiles' as well, instead of `gemm_skinny_kernel` (the same bits), whose wavefronts make a trip to memory
-// for every 256 k of their part, one behind the other.  Measured on 220 drawn sizes at 1, 8 and 16 rows, weights cold, against it, geometric
-// mean: gated from k = 1024 on 0.85 (0.71 to 1.07; 0.99 to 1.08 below), plain from 1408 on, of more than 4352 columns from 1024 on, 0.90
-// (0.68 to 1.09; 0.97 to 1.12 below).  Not a gate over many columns of a long k (12288 x 4096: 36.3 and 39.5 us), nor beyond the sizes drawn.
-// 8 x 2 * 5632 x 2048 14.8 -> 11.7 us, 8 x 2 * 704 x 2048 7.4 -> 6.0, 8 x 6144 x 2048 8.8 -> 7.3, 8 x 2048 x 2048 5.9 -> 5.3.
+// for every 256 k of their part, one behind the other.  Measured at 1 to 16 rows, weights cold, against it: 220 drawn sizes, geometric
+// mean gated from k = 1024 on 0.85 (0.71 to 1.07; 0.99 to 1.08 below), plain from 1408 on, of more than 4352 columns from 1024 on, 0.90
+// (0.68 to 1.09; 0.97 to 1.12 below); and 240 of many columns and whole 256s of k, which have the limits further in.  A gate
+// of more than 6656 columns: up to k = 1536 1.03 to 1.17, where k is a multiple of 2048 (the rows of a tile then lie on the same channels of
+// memory) 1.02 to 1.45, of more than 10240 columns below 8 rows 1.03 to 1.07; the others 0.81 to 1.03.  Plain, of more than 8192
+// columns, up to 8 rows: 0.97 to 1.19 up to 12288, with such k 1.03 to 1.20; the others 0.81 to 1.05.
+// us: 8 x 2 * 5632 x 2048 15.5 -> 13.9, 8 x 2 * 704 x 2048 7.5 -> 6.4, 8 x 6144 x 2048 8.9 -> 7.8, 8 x 2048 x 2048 5.5 -> 5.0; left out:
+// 8 x 2 * 16384 x 2048 30.9, 44.0, 1 x 2 * 12288 x 1024 11.5, 13.5, 1 x 16384 x 4096 26.6, 32.0, 4 x 8448 x 1024 6.9, 7.8.
 static bool narrow_wins(int M, int N, int K, bool gated) {
     if (M <= 0 || M > 16 || N < 384 || N > 16384 || K > 6144) return false;
-    return gated ? K >= 1024 && (K <= 3072 || N <= 8192) : K >= 1408 || (K >= 1024 && N > 4352);
+    if (gated)
+        return K >= 1024 && (N <= 6656 || (K >= 1792 && K % 2048 != 0 && N <= (K > 3072 ? 8192 : M < 8 ? 10240 : 16384)));
+    return (K >= 1408 || (K >= 1024 && N > 4352)) && (N <= 8192 || M > 8 || (N > 12800 && K % 2048 != 0));
 }
 
 // Whether the kernel takes these operands at all: whole blocks of k, 32-bit offsets, rows that start on 16 bytes.
@@ -1840,22 +1846,36 @@ extern "C" int mlr_gemm_wide(const void* a, const void* w, void* out, int M, int
     return run_wide(shape, a, w, out, M, N, K, out_float != 0, gated ? WIDE_SILU : WIDE_PLAIN, 0.f, 0.f, stream);
 }
 
-// Whether up to 64 rows are the forms' with several workgroups a tile, instead of the kernels above and the vendor library.  Up to 16
-// rows, against `gemm_skinny_kernel` on 250 products, geometric mean: 0.75 of those that this takes (0.49 to 1.06); below these inner sizes 0.86 to
-// 1.15, and where a strip of 16 columns a compute unit comes out even (193 to 256 strips) 0.97 (to 1.07) up to 5120.  8 x 2048 x 5632
-// 10.8 -> 8.7 us, 1 x 2048 x 8448 14.6 -> 10.4, 16 x 4096 x 12288 27.1 -> 20.6, 8 x 3000 x 8960 17.3 -> 13.3.  From 17 on: measured on the
-// products of the forms' fit against what took them before, geometric mean: the 310 that this takes 0.63 (0.34 to 1.02; of those
-// where the library has a plan that cuts k itself, a row count and sizes in whole 16s, 0.7 to 1); below these inner sizes 1.04 to 1.4,
-// beyond these rows of weight 0.9 to 1.3.  64 x 4096 x 12288 34.0 -> 26.0 us, 48 x 5120 x 25600 84.7 -> 62.1, 32 x 2048 x 5632
-// 12.4 -> 9.2, 64 x 4096 x 4096 14.4 -> 12.4, 20 x 3000 x 8960 19.4 -> 15.1.
+// Whether up to 64 rows are the forms' with several workgroups a tile, instead of the kernels above and the vendor library.  Measured,
+// weights cold, against what takes them otherwise: drawn products (250 of up to 16 rows, 560 of more; the library is at its
+// worst with such sizes) and 2300 of mostly round ones, whose losses the exceptions leave out.  us, otherwise and so:
+// Up to 16 rows, against `gemm_skinny_kernel`: 8 x 2048 x 5632 10.4 -> 8.7, 1 x 2048 x 8448 14.6 -> 10.4, 16 x 4096 x 12288 26.0 -> 21.5, 8 x 3000
+// x 8960 17.3 -> 13.3; round sizes geometric mean 0.80 (0.48 to 1.04).  Left out: below these inner sizes and where a strip of 16 columns a
+// compute unit comes out even (up to 1.15); k of 8192 and 24576 over many columns (1 x 4096 x 8192 14.8, 18.4), 12288 and 20480 over more
+// than 4096 (8 x 7168 x 12288 35.4, 43.4): rows of weight on the same channels of memory; up to 4 rows of more than 3072 columns (1.00 to 1.06).
+// From 17 rows on: 64 x 4096 x 12288 33.1 -> 27.0, 48 x 5120 x 25600 89.8 -> 71.4, 32 x 2048 x 5632 12.4 -> 9.2, 64 x 4096 x 4096 13.9 -> 12.3,
+// 20 x 3000 x 8960 19.4 -> 15.1; round sizes 0.79 (0.45 to 1.07), of 8208 to 16384 rows of weight 0.94 (0.79 to 1.09).  Left out: below these
+// inner sizes and beyond these rows of weight (up to 1.4), of more than 8192 whole 512s of k (64 x 12288 x 16384 86.0, 106.8; 48 x 16384 x 16384
+// 101.2, 122.4), k in whole 8192s as above (20 x 4096 x 8192 16.2, 19.1; 32 x 6144 x 24576 68.8, 77.7), up to 24 rows of short k (20 x 4096
+// x 5120 11.4, 12.8), few rows of weight that the library cuts k for (48 x 1024 x 5120 8.1, 8.8).
 static bool split_wins(int M, int N, int K) {
     if (M <= 0 || M > 64) return false;
     if (M <= 16) {
         const int units = compute_units() > 0 ? compute_units() : 256, strips = (N + 15) / 16;
+        if (N > 2560 && K % 8192 == 0 && K % 16384 != 0) return false;
+        if (N > 4096 && K > 8192 && K % 4096 == 0 && K % 16384 != 0) return false;
+        if (N > 3072 && M <= 4 && K > 6144 && K < 14336) return false;
         return N <= 8192 && (K >= 5120 || (K >= 3584 && !(4 * strips > 3 * units && strips <= units)));
     }
-    if (K >= 14336) return N <= 16384;
-    if (K >= 9216) return N <= 8192;
+    if (K >= 14336) {
+        if (N > 16384 || (M > 32 && N > 11264 && N <= 12800)) return false;
+        if (N > 8192 && K >= 15360 && (N > 11264 || K % 512 == 0)) return false;
+        return K % 8192 != 0 || (N <= 6144 && (M > 32 || N <= 4096 || K % 16384 == 0));
+    }
+    if (K >= 9216) return N <= (M <= 32 && K % 4096 == 0 ? 6144 : 8192);
+    if (K % 8192 == 0 && N > (M <= 32 ? 3072 : 4096)) return false;
+    if (M <= 24 && (N > 3072 ? K <= 7168 : N > 2048 && K < 5120)) return false;
+    if (M > 32 && N <= 1024 && K <= 6144 && K % 512 == 0) return false;
     if (K >= 6144) return N <= 6144;
     if (K >= 4224) return N <= 4096;
     if (K >= 3136) return N <= (M > 32 ? 4096 : 2048);

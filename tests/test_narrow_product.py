@@ -19,7 +19,12 @@ def without_gpu(routed=False):
     (1, 2048, 2048, False, True), (16, 2048, 1408, False, True), (17, 2048, 2048, False, False), (8, 2048, 1344, False, False),
     (8, 4352, 1024, False, False), (8, 4353, 1024, False, True), (8, 383, 2048, False, False), (8, 384, 2048, False, True),
     (8, 16385, 2048, False, False), (8, 2048, 6144, False, True), (8, 2048, 6208, False, False), (8, 2048, 2050, False, False),
-    (8, 704, 1024, True, True), (8, 704, 960, True, False), (8, 16384, 3072, True, True), (8, 8193, 3136, True, False)])
+    (8, 704, 1024, True, True), (8, 704, 960, True, False), (8, 16384, 3072, True, True), (8, 8193, 3136, True, False),
+    # (many columns: not where the rows of a tile lie on the same channels of memory, nor with a short k or few rows)
+    (8, 6656, 2048, True, True), (8, 6657, 2048, True, False), (8, 16384, 2048, True, False), (16, 8192, 4096, True, False), (1, 7168, 1536, True, False),
+    (1, 7168, 1792, True, True), (7, 10240, 2560, True, True), (7, 10241, 2560, True, False), (8, 10241, 2560, True, True), (8, 8192, 3136, True, True),
+    (8, 8192, 2048, False, True), (8, 8193, 2560, False, False), (9, 8193, 2560, False, True), (1, 12800, 2560, False, False),
+    (1, 12801, 2560, False, True), (1, 16384, 4096, False, False), (9, 16384, 4096, False, True)])
 def test_few_rows_of_a_long_enough_inner_size(rows, columns, inner, gated, taken):
     for routed in (False, True):
         assert without_gpu(routed).narrow_product(rows, columns, inner, gated) == taken

@@ -20,10 +20,27 @@ def without_gpu(routed=False):
     (8, 8193, 9216, False), (16, 4096, 12288, True), (17, 4096, 12288, True), (64, 4096, 12288, True), (65, 4096, 12288, False), (64, 4096, 2048, False),
     (64, 2048, 2560, True), (32, 2048, 2560, False), (64, 1024, 2560, False), (32, 2048, 3136, True), (32, 2049, 3136, False),
     (33, 4096, 3136, True), (20, 4097, 4224, False), (64, 6144, 6144, True), (64, 8192, 9216, True), (64, 16384, 14336, True),
-    (64, 16385, 14336, False), (64, 4096, 12289, False)])
+    (64, 16385, 14336, False), (64, 4096, 12289, False),
+    # (inner sizes that put the rows of weight on the same channels of memory, few rows, round sizes that the library cuts itself)
+    (16, 2560, 8192, True), (16, 2561, 8192, False), (8, 4096, 24576, False), (8, 4096, 16384, True), (16, 4097, 12288, False), (16, 4097, 12352, True),
+    (4, 3073, 8960, False), (5, 3073, 8960, True), (1, 3072, 8960, True), (1, 3073, 14336, True), (20, 3072, 8192, True), (20, 3073, 8192, False),
+    (48, 4096, 8192, True), (48, 4097, 8192, False), (32, 6144, 12288, True), (32, 6145, 12288, False), (48, 8192, 12288, True), (32, 4097, 24576, False),
+    (48, 6144, 24576, True), (64, 8192, 16384, False), (64, 8193, 16384, False), (64, 10240, 15424, True), (64, 10240, 15360, False),
+    (64, 11265, 15424, False), (64, 12288, 14336, False), (32, 12288, 14336, True), (24, 4096, 7168, False), (25, 4096, 7168, True), (24, 3072, 5056, False),
+    (24, 3072, 5120, True), (24, 2048, 4224, True), (33, 1024, 5120, False), (33, 1024, 5184, True), (32, 1024, 5120, True)])
 def test_long_inner_sizes_of_few_rows_are_shared_out(rows, columns, inner, taken):
     assert without_gpu().split_product(rows, columns, inner) == taken
     assert without_gpu(routed=True).split_product(rows, columns, inner) == (taken and rows <= 16)
+
+
+@pytest.mark.parametrize("rows,columns,inner,shared", [
+    (8, 2048, 5632, True), (8, 2560, 5120, True), (8, 2561, 5120, False), (8, 8192, 3584, False), (8, 4096, 6144, False), (8, 5120, 6144, False),
+    (8, 5121, 6144, True), (8, 4096, 6208, True), (17, 2048, 5632, True), (17, 4096, 12288, True), (32, 4096, 5120, True)])
+def test_narrow_tiles_come_before_shared_ones_over_many_columns(monkeypatch, rows, columns, inner, shared):
+    k = without_gpu()
+    monkeypatch.setattr(ops, "_stream", lambda: ctypes.c_void_p(0))
+    k._split, k._split_stream = ("room", "counters"), 0
+    assert k.shares_tiles(rows, columns, inner) == shared
 
 
 def test_only_the_stream_that_has_the_room_shares_tiles(monkeypatch):
