@@ -391,12 +391,13 @@ class Kernels:
         _need(k == k2, lambda: f"gemm: inner sizes differ ({k} and {k2})")
         _need(out.dtype in (self.dtype, torch.float32), lambda: f"gemm: output type {out.dtype} not supported")
         _tensor(out, "out", out.dtype, (m, n))
-        if m <= 64 and out.dtype == torch.bfloat16 and self.shares_tiles(m, n, k) and _on16(a, w):
+        shared = m <= 64 and out.dtype == torch.bfloat16 and self.shares_tiles(m, n, k)
+        if shared and self.has_split() and _on16(a, w):
             partial, arrivals = self._split
             _ok(self._lib("gemm").mlr_gemm_split(_p(a), _p(w), _p(out), _c_int(m), _c_int(n), _c_int(k), _p(partial),
                                                  ctypes.c_long(partial.numel()), _p(arrivals), _c_int(arrivals.numel()), _c_int(-1), _stream()), "gemm")
             return
-        if m <= 64 and out.dtype == torch.bfloat16 and (self.narrow_product(m, n, k) or self.few_product(m, n, k) or self.wide_product(m, n, k)) \
+        if m <= 64 and out.dtype == torch.bfloat16 and (shared or self.narrow_product(m, n, k) or self.few_product(m, n, k) or self.wide_product(m, n, k)) \
                 and _on16(a, w):
             _ok(self._lib("gemm").mlr_gemm_wide(_p(a), _p(w), _p(out), _c_int(m), _c_int(n), _c_int(k), _c_int(0),
                                                 _c_int(-1 if self.one_sum(m, k) else -2), _c_int(0), _stream()), "gemm")
@@ -434,20 +435,22 @@ class Kernels:
 
     def claim_split(self):
         """The room for shared tiles is the current stream's from here on, whose launches come one after the other: two at a time
-        would count each other's workgroups.  A product on another stream takes the kernels that need no room.  (The caller vouches
-        that the stream that had it before has nothing under way in it; a runner claims it for every step.)"""
+        would count each other's workgroups.  A product on another stream takes tiles of one workgroup, with the same bits.  (The caller
+        vouches that the stream that had it before has nothing under way in it; a runner claims it for every step.)"""
         if self._split is not None:
             self._split_stream = _stream().value or 0
 
+    def has_split(self):
+        """Whether the room for shared tiles is the current stream's."""
+        return self._split is not None and self._split_stream == (_stream().value or 0)
+
     def shares_tiles(self, rows, columns, k):
-        """Whether a product of these sizes, launched now, is one whose tiles several workgroups share.  (Up to 16 rows of more than
-        2560 columns the narrow tiles, which have the same bits, are the faster where they take the product, us: 1 x 4096 x 5120 9.9, shared
-        11.7, 16 x 6144 x 4096 12.1, 14.5, 8 x 3072 x 4096 8.2, 8.8; with k = 6144 up to 5120: 5120 15.4, 15.5, 8192 23.2, 21.4.)"""
-        if self._split is None or not self.split_product(rows, columns, k):
-            return False
-        if columns > 2560 and (k < 6144 or columns <= 5120) and self.narrow_product(rows, columns, k):
-            return False
-        return self._split_stream == (_stream().value or 0)
+        """Whether the tiles of a product of these sizes are shared by several workgroups, on the stream that has the room.  (Up to 16
+        rows of more than 2560 columns the narrow tiles, which have the same bits, are the faster where they take the product, us: 1 x
+        4096 x 5120 9.9, shared 11.7, 16 x 6144 x 4096 12.1, 14.5, 8 x 3072 x 4096 8.2, 8.8; with k = 6144 up to 5120: 5120 15.4, 15.5, 8192
+        23.2, 21.4.)"""
+        return self._split is not None and self.split_product(rows, columns, k) and not (
+            columns > 2560 and (k < 6144 or columns <= 5120) and self.narrow_product(rows, columns, k))
 
     def split_product(self, rows, columns, k):
         """Whether a product of up to 64 rows is taken by several workgroups a tile: the sums of the other kernels of few rows, bit by

@@ -46,17 +46,16 @@ def test_narrow_tiles_come_before_shared_ones_over_many_columns(monkeypatch, row
 def test_only_the_stream_that_has_the_room_shares_tiles(monkeypatch):
     k, now = without_gpu(), [0]
     monkeypatch.setattr(ops, "_stream", lambda: ctypes.c_void_p(now[0]))
-    assert not k.shares_tiles(8, 2048, 5632)               # (no room at all)
+    assert not k.shares_tiles(8, 2048, 5632) and not k.has_split()               # (no room at all)
     k.claim_split()
     k._split = ("room", "counters")
-    assert not k.shares_tiles(8, 2048, 5632)               # (nobody has it yet)
+    assert not k.has_split()                               # (nobody has it yet)
     for owner in (0, 4096, 0):
         now[0] = owner
         k.claim_split()
         for stream in (0, 4096, 8192):
             now[0] = stream
-            assert k.shares_tiles(8, 2048, 5632) == (stream == owner)
-            assert not k.shares_tiles(8, 2048, 2048)
+            assert k.shares_tiles(8, 2048, 5632) and k.has_split() == (stream == owner)
 
 
 # (inner sizes whose last share is one block, a part's last block missing, as many as parts; columns in whole tiles, ragged, odd)
@@ -119,26 +118,33 @@ def test_the_runners_kernels_share_products_out_and_others_do_not():
     assert torch.equal(out.view(torch.int16), again.view(torch.int16))
 
 
+# a long product on the stream that has the room, another beside it on a second stream and in a capture of the caller's own: the
+# same bits everywhere, whoever shares
 @pytest.mark.gpu
-def test_products_of_two_streams_at_once_do_not_meet():
-    # a long product on the stream that has the room, short ones beside it on another: their sums stay their own
+@pytest.mark.parametrize("rows", [16, 40])
+def test_products_of_two_streams_at_once_do_not_meet(rows):
     k = Kernels(torch.bfloat16)
     k.reserve_split_workspace("cuda")
     gen = torch.Generator().manual_seed(5)
     draw = lambda *shape: torch.randn(*shape, generator=gen).to(torch.bfloat16).cuda()
-    a, w = [draw(16, 5632) for _ in range(2)], [draw(2048, 5632) for _ in range(2)]
-    want = [torch.empty(16, 2048, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    a, w = [draw(rows, 5632) for _ in range(2)], [draw(2048, 5632) for _ in range(2)]
+    want = [torch.empty(rows, 2048, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    assert k.shares_tiles(rows, 2048, 5632) and k.has_split()
     for i in range(2):
         k.gemm(a[i], w[i], want[i])
     outs = [[torch.full_like(want[i], float("nan")) for _ in range(20)] for i in range(2)]
-    other = torch.cuda.Stream()
+    other, graph, captured = torch.cuda.Stream(), torch.cuda.CUDAGraph(), torch.full_like(want[1], float("nan"))
     torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        assert not k.has_split()
+        k.gemm(a[1], w[1], captured)
     for n in range(20):
         k.gemm(a[0], w[0], outs[0][n])
         with torch.cuda.stream(other):
-            assert not k.shares_tiles(16, 2048, 5632)
+            assert not k.has_split()
             k.gemm(a[1], w[1], outs[1][n])
+            graph.replay()
     torch.cuda.synchronize()
-    for i in range(2):                                     # (up to 16 rows the other kernels' sums, bit by bit)
-        assert all(torch.equal(out.view(torch.int16), want[i].view(torch.int16)) for out in outs[i])
+    same = lambda x, y: torch.equal(x.view(torch.int16), y.view(torch.int16))
+    assert same(captured, want[1]) and all(same(out, want[i]) for i in range(2) for out in outs[i])
     assert not k._split[1].any()
