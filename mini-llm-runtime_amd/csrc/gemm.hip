@@ -496,10 +496,9 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const __
     // What the epilogue needs from memory is asked for here, before the weight, by every wavefront alike
     // (no branch around a load); only wavefront 0 uses it.
     float ss_mine = 0.f;                                   // EPI_SCALE: this lane's share of the row's partial sums
-    constexpr bool SS_LATER = EPI == EPI_SCALE && UMAX <= 2;
-    float4 ss4;                                            // ... which are added when the weight is multiplied, where this holds them all
+    float4 ss4 = make_float4(0.f, 0.f, 0.f, 0.f);          // ... which are added when the weight is multiplied, where this holds them all
     const int ss_quads = epi.ss_parts >> 2, ss_run = (ss_quads + 4 * SKINNY_WAVES - 1) / (4 * SKINNY_WAVES);
-    const bool ss_later = SS_LATER && epi.ss_vec && ss_run <= 1;
+    const bool ss_later = EPI == EPI_SCALE && UMAX <= 2 && epi.ss_vec && ss_run <= 1;
     float4 h4 = make_float4(0.f, 0.f, 0.f, 0.f), nw4 = h4;  // EPI_RESIDUAL: h and the next norm's weights at (row r16, columns n0 + 4 b ..)
     float4 h4b = h4, nw4b = h4;                            // ... and, PAIR, at the second strip's columns n0 + 16 + 4 b ..
     if constexpr (EPI == EPI_SCALE) {
@@ -513,7 +512,7 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const __
         // with them; 10 x 2 * 12288 x 1024 with four 13.2 and 15.8).
         const float* row = epi.ss + (size_t)min(r16, M - 1) * epi.ss_parts;
         const int pair = wave * 4 + b;
-        if (SS_LATER && ss_later) {
+        if (ss_later) {
             ss4 = reinterpret_cast<const float4*>(row)[min(pair, ss_quads - 1)];
         } else if (epi.ss_vec) {
             const int quads = ss_quads, q = ss_run;
@@ -669,9 +668,7 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_skinny_kernel(const __
                 for (int r = 0; r < 4; ++r) part[wave - 1][g][i][lane][r] = acc[g][i][r];
     }
     if constexpr (EPI == EPI_SCALE) {
-        if (SS_LATER && ss_later) {
-            ss_mine += wave * 4 + b < ss_quads ? (ss4.x + ss4.y) + (ss4.z + ss4.w) : 0.f;
-        }
+        if (ss_later && wave * 4 + b < ss_quads) ss_mine += (ss4.x + ss4.y) + (ss4.z + ss4.w);
         ss_mine = xor_sum<16>(ss_mine);
         ss_mine = xor_sum<32>(ss_mine);
         if (b == 0) ss_lds[wave][r16] = ss_mine;
