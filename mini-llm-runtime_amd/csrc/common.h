@@ -86,7 +86,7 @@ template <typename V> __device__ __forceinline__ V turned(const V& v) {
 }
 
 // Values of other lanes without a trip through LDS, which a `__shfl_xor` is (a sum over a wavefront is a chain of six; one token of
-// the 0.6B sizes 1019 -> 1000 us a step, the float engine through the scheduler 32.3 -> 32.05 ms, Pamunex 2.55 -> 2.515):
+// the 0.6B sizes 1019 -> 1000 us a step, Pamunex 2.55 -> 2.515 ms; the float engine, whose time is its products', the same):
 // the lane i ^ OFF within 16 lanes by DPP; across rows of 16 both operands of a swap, of which one is the lane's own value and the
 // other its partner's -- which is which does not matter to a sum or a maximum.  All lanes of the wavefront take part.
 template <int OFF> __device__ __forceinline__ float row_xor(float v) {

@@ -996,7 +996,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_wide_kernel(const std::c
     static_assert(!QKV || (!OUT_FLOAT && !GATED && !HEADS && !FEW && S::BN % QKV_HEAD == 0), "whole heads");
     constexpr int BM = S::BM, BN = S::BN, LOADS = S::LOADS;
     static_assert(!GATED || TN % 2 == 0, "gate and up tiles come in pairs");
-    static_assert((!PAIRED || FEW) && (!FEW || !HEADS) && (SPLIT == 1 || (FEW && SKINNY_WAVES % SPLIT == 0)), "forms for 17 to 64 rows");
+    static_assert((!PAIRED || FEW) && (!FEW || !HEADS) && (SPLIT == 1 || (FEW && SKINNY_WAVES % SPLIT == 0)), "forms for up to 64 rows");
     extern __shared__ __attribute__((aligned(16))) __bf16 wide_lds[];
     const int M = args.M, N = args.N, K = args.K;
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -1786,7 +1786,9 @@ static int wide_shape_for(int M, int N, int K, bool gated, float* time) {
 // columns.  Not beyond: few columns at long k take up to 1.6 of the library's time (48 x 2 * 464 x 4224 10 us for 7), and weights of
 // more than 32768 rows 1.03 to 1.16, from 24576 on 1.03 to 1.06 without a gate at k above 2048 (64 x 2 * 25600 x 5120: 106, 121).  All that this takes:
 // 0.69 (550 products, 0.37 to 1.24); 24 x 6144 x 1024 8.0 -> 5.8 us, 64 x 6144 x 2048 13.2 -> 10.2, with gate and silu 64 x 2 * 3072 x 1024
-// 11.5 -> 7.0, 64 x 2 * 12288 x 4096 46.5 -> 46.2 (the library's product and its activation's launch before).
+// 11.5 -> 7.0, 64 x 2 * 12288 x 4096 46.5 -> 46.2 (the library's product and its activation's launch before).  With the clamped gate, which
+// `gemm_skinny_kernel` took up to 64 rows: 17, 32 and 64 x 2 * 5632 x 2048 18.3, 21.0, 31.1 -> 13.3, 13.9, 17.1, 2 * 704 x 2048 9.6, 10.9, 16.2 ->
+// 6.5, 6.6, 8.4, 2 * 12288 x 4096 49.8, 58.8, 80.9 -> 52.1, 47.7, 49.3.
 static bool few_wins(int M, int N, int K, bool gated) {
     const long long weight = (long long)N * (gated ? 2 : 1);
     if (M <= 16 || M > 64 || weight > (gated || K <= 2048 ? 32768 : 24576)) return false;
@@ -1821,7 +1823,7 @@ extern "C" int mlr_gemm_narrow_wins(int M, int N, int K, int gated) {
     return N > 0 && K > 0 && wide_takes(nullptr, nullptr, M, N, K, gated != 0) && narrow_wins(M, N, K, gated != 0) ? 1 : 0;
 }
 
-enum { WIDE_MANY = -1, WIDE_FEW = -2 };      // the tile with the least predicted time, of one sum over k or of the forms for 17 to 64 rows
+enum { WIDE_MANY = -1, WIDE_FEW = -2 };      // the tile with the least predicted time, of one sum over k or of the forms for up to 64 rows
 static int run_wide(int shape, const void* a, const void* w, void* out, int M, int N, int K, bool out_float, int act, float limit,
                     float slope, hipStream_t stream) {
     const bool gated = (act >= WIDE_SILU && act <= WIDE_CLAMPED) || act == WIDE_CLAMPED_SUMS;
@@ -1835,7 +1837,7 @@ static int run_wide(int shape, const void* a, const void* w, void* out, int M, i
 }
 
 // The kernel in a given shape (0 .. 16, for tests and measurements) or in the one with the least predicted time (-1: of one sum over
-// k; -2: of the forms for 17 to 64 rows, whose sums are those of up to 16 rows), plain or with gate and silu.
+// k; -2: of the forms for up to 64 rows, whose sums are those of `gemm_skinny_kernel`), plain or with gate and silu.
 extern "C" int mlr_gemm_wide(const void* a, const void* w, void* out, int M, int N, int K, int out_float,
                              int shape, int gated, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;

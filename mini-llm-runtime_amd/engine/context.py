@@ -237,7 +237,10 @@ class StepContext:
         behind 3800 15.1, 15.3; 2 behind 1100 15.9, 12.9; 6 behind 2000 21.4, 20.1; 8 behind 4600 to 4900 43.2, 40.1; 12 behind 2000
         30.9, 28.0; 16 behind up to 3800 38.8, 37.4.  Not beyond half the units: 24 behind 2000 50.7, 45.0, but 24 behind 300 to 3800 48.5,
         59.2, where a long context's one range keeps the step waiting, and 64 behind 129 to 3000, whose second ranges are dealt out when
-        the first are done, 76.3, 84.6."""
+        the first are done, 76.3, 84.6.  Longer contexts, where a token has two to four shares of ranges: 1 token behind 16300 24.1, 20.6, behind
+        40000 45.8, 36.6; 4 behind 32768 113.3, 113.8, 40000 138.5, 126.4; 8 behind 16300 100.8, 100.6, 32768 205.3, 198.5, 40000 253.3, 243.5; 16 behind
+        24576 308.6, 293.4, 32768 401.1, 395.1.  (4 behind 8100 31.9, 35.6, where ranges of 1024 keys start on the same channels of memory; 4
+        behind 8300, 1088 keys each, 34.2, 31.6.)"""
         units, workgroups = rows * kv_heads, min(self.compute_units, self.target_workgroups)
         if rows > self.split_max_tokens or self.split_keys <= 0 or self.routed or 2 * units > workgroups:
             return None
