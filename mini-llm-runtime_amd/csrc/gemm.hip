@@ -1801,8 +1801,8 @@ static bool few_wins(int M, int N, int K, bool gated) {
 // for every 256 k of their part, one behind the other.  Measured at 1 to 16 rows, weights cold, against it: 220 drawn sizes, geometric
 // mean gated from k = 1024 on 0.85 (0.71 to 1.07; 0.99 to 1.08 below), plain from 1408 on, of more than 4352 columns from 1024 on, 0.90
 // (0.68 to 1.09; 0.97 to 1.12 below); and 240 of many columns and whole 256s of k, which have the limits further in.  A gate
-// of more than 6656 columns: up to k = 1536 1.03 to 1.17, where k is a multiple of 2048 (the rows of a tile then lie on the same channels of
-// memory) 1.02 to 1.45, of more than 10240 columns below 8 rows 1.03 to 1.07; the others 0.81 to 1.03.  Plain, of more than 8192
+// of more than 6656 columns: up to k = 1536 1.03 to 1.17, where k is a multiple of 2048 (a tile's rows then share channels of memory,
+// it seems) 1.02 to 1.45, of more than 10240 columns below 8 rows 1.03 to 1.07; the others 0.81 to 1.03.  Plain, of more than 8192
 // columns, up to 8 rows: 0.97 to 1.19 up to 12288, with such k 1.03 to 1.20; the others 0.81 to 1.05.
 // us: 8 x 2 * 5632 x 2048 15.5 -> 13.9, 8 x 2 * 704 x 2048 7.5 -> 6.4, 8 x 6144 x 2048 8.9 -> 7.8, 8 x 2048 x 2048 5.5 -> 5.0; left out:
 // 8 x 2 * 16384 x 2048 30.9, 44.0, 1 x 2 * 12288 x 1024 11.5, 13.5, 1 x 16384 x 4096 26.6, 32.0, 4 x 8448 x 1024 6.9, 7.8.
@@ -1851,7 +1851,7 @@ extern "C" int mlr_gemm_wide(const void* a, const void* w, void* out, int M, int
 // Up to 16 rows, against `gemm_skinny_kernel`: 8 x 2048 x 5632 10.4 -> 8.7, 1 x 2048 x 8448 14.6 -> 10.4, 16 x 4096 x 12288 26.0 -> 21.5, 8 x 3000
 // x 8960 17.3 -> 13.3; round sizes geometric mean 0.80 (0.48 to 1.04).  Left out: below these inner sizes and where a strip of 16 columns a
 // compute unit comes out even (up to 1.15); k of 8192 and 24576 over many columns (1 x 4096 x 8192 14.8, 18.4), 12288 and 20480 over more
-// than 4096 (8 x 7168 x 12288 35.4, 43.4): rows of weight on the same channels of memory; up to 4 rows of more than 3072 columns (1.00 to 1.06).
+// than 4096 (8 x 7168 x 12288 35.4, 43.4): as with the narrow tiles; up to 4 rows of more than 3072 columns (1.00 to 1.06).
 // From 17 rows on: 64 x 4096 x 12288 33.1 -> 27.0, 48 x 5120 x 25600 89.8 -> 71.4, 32 x 2048 x 5632 12.4 -> 9.2, 64 x 4096 x 4096 13.9 -> 12.3,
 // 20 x 3000 x 8960 19.4 -> 15.1; round sizes 0.79 (0.45 to 1.07), of 8208 to 16384 rows of weight 0.94 (0.79 to 1.09).  Left out: below these
 // inner sizes and beyond these rows of weight (up to 1.4), of more than 8192 whole 512s of k (64 x 12288 x 16384 86.0, 106.8; 48 x 16384 x 16384

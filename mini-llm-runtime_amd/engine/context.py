@@ -239,7 +239,7 @@ class StepContext:
         59.2, where a long context's one range keeps the step waiting, and 64 behind 129 to 3000, whose second ranges are dealt out when
         the first are done, 76.3, 84.6.  Longer contexts, where a token has two to four shares of ranges: 1 token behind 16300 24.1, 20.6, behind
         40000 45.8, 36.6; 4 behind 32768 113.3, 113.8, 40000 138.5, 126.4; 8 behind 16300 100.8, 100.6, 32768 205.3, 198.5, 40000 253.3, 243.5; 16 behind
-        24576 308.6, 293.4, 32768 401.1, 395.1.  (4 behind 8100 31.9, 35.6, where ranges of 1024 keys start on the same channels of memory; 4
+        24576 308.6, 293.4, 32768 401.1, 395.1.  (4 behind 8100 31.9, 35.6, where ranges lie 1024 keys apart, it seems on the same channels of memory; 4
         behind 8300, 1088 keys each, 34.2, 31.6.)"""
         units, workgroups = rows * kv_heads, min(self.compute_units, self.target_workgroups)
         if rows > self.split_max_tokens or self.split_keys <= 0 or self.routed or 2 * units > workgroups:
